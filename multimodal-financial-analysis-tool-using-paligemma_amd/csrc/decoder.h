@@ -194,7 +194,7 @@ enum RtOut : int {
     RT_SWIGLU = 3,  // activation type, silu(A . W_gate^T) * (A . W_up^T); W = gate rows, then N up rows
 };
 int matmul_rt(hipStream_t s, Act act, const void* A, int lda, const uint16_t* W, int ldw, int M, int N, int K,
-              RtOut mode, const uint16_t* bias, void* out, int ldo, size_t out_bytes, float* scratch);
+              RtOut mode, const uint16_t* bias, void* out, int ldo, size_t out_bytes);
 
 // ---------------------------------------------------------------- selective scan (Mamba)
 // xz rows [x: C | z: C] (activation type); taps state fp32 [slot][K-1][C]
@@ -317,7 +317,7 @@ void wattn_decode(hipStream_t s, Act act, const WAttnDecodeArgs& a);
 enum GemvRtForm : int {
     GF_NONE = 0,    // too many rows: matmul_rt and the step kernels below
     GF_STREAM = 1,  // weight-streaming GEMV; the input may be the streams' next read and norm (as streams_norm)
-    GF_SKINNY = 2,  // MFMA, up to gemv_rt_max_batch() rows of bf16 activations
+    GF_SKINNY = 2,  // MFMA, up to gemv_rt_max_batch() rows
 };
 enum GemvRtMode : int {
     GR_ACT = 0,      // out (activation type) = acc + bias

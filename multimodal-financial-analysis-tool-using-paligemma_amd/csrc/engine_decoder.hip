@@ -403,10 +403,7 @@ int ensure_workspace(pgmi_ctx* x, int rows, int chunks, int gchunks) {
             l2 = std::max(l2, r8(l.width));
             cg = std::max(cg, l.width);
         }
-        if (const int ff = l.experts ? l.shared_ff : l.ff) {
-            l2 = std::max(l2, r8(ff));
-            if (d.act == ACT_F32) l0 = std::max(l0, 2 * ff);  // unfused gate|up
-        }
+        l2 = std::max(l2, r8(l.experts ? l.shared_ff : l.ff));
         if (l.experts) {
             lea = std::max(lea, r8(l.expert_ff));
             top = std::max(top, l.top);
@@ -585,7 +582,7 @@ int forward_body(pgmi_ctx* x, hipStream_t s, const int64_t* ids, int rows, const
         first = false;
     };
     auto out_proj = [&](const Lin& o, const void* in, int ldin, const Sub& sub) {
-        pend.split = matmul_rt(s, d.act, in, ldin, o.w, o.ldw, rows, D, o.k, RT_SLABS, nullptr, d.slabs, D, d.slab_bytes, nullptr);
+        pend.split = matmul_rt(s, d.act, in, ldin, o.w, o.ldw, rows, D, o.k, RT_SLABS, nullptr, d.slabs, D, d.slab_bytes);
         pend.y = d.slabs;
         pend.sub = &sub;
     };
@@ -595,13 +592,13 @@ int forward_body(pgmi_ctx* x, hipStream_t s, const int64_t* ids, int rows, const
         read(i, 0, taps && i ? taps + (long)(i - 1) * rows * D : nullptr);
         if (l.mixer == PGMI_MIXER_MAMBA1) {
             const int C = l.inner, N = l.state, R = l.dt_rank, ldc = r8(C), ldxz = r8(2 * C), ldd = r8(R);
-            matmul_rt(s, d.act, d.h, d.ldh, w.in.w, w.in.ldw, rows, 2 * C, w.in.k, RT_ACT, nullptr, d.p0, ldxz, 0, nullptr);
+            matmul_rt(s, d.act, d.h, d.ldh, w.in.w, w.in.ldw, rows, 2 * C, w.in.k, RT_ACT, nullptr, d.p0, ldxz, 0);
             conv_silu(s, d.act, d.p0, ldxz, C, l.conv, w.conv, w.conv_b, m.seqs, m.nseq, m.scan.p, m.scan.n,
                       at<float>(state, st[i].a), d.p1, ldc);
             const int sp = matmul_rt(s, d.act, d.p1, ldc, w.x.w, w.x.ldw, rows, R + 2 * N, w.x.k, RT_SLABS, nullptr, d.slabs,
-                                     0, d.slab_bytes, nullptr);
+                                     0, d.slab_bytes);
             scan_inputs(s, d.act, d.slabs, sp, rows, R, N, d.dtl, ldd, d.bc);
-            matmul_rt(s, d.act, d.dtl, ldd, w.dt.w, w.dt.ldw, rows, C, w.dt.k, RT_F32, nullptr, d.dt, C, 0, nullptr);
+            matmul_rt(s, d.act, d.dtl, ldd, w.dt.w, w.dt.ldw, rows, C, w.dt.k, RT_F32, nullptr, d.dt, C, 0);
             ScanArgs a{};
             a.dt = d.dt; a.dtb = w.dt_b; a.x = d.p1; a.ldx = ldc; a.z = d.p0 + (size_t)C * d.es; a.ldz = ldxz; a.bc = d.bc;
             a.A_log = w.A_log; a.Dw = w.D; a.state = at<float>(state, st[i].b); a.cstate = d.cstate; a.csum = d.csum;
@@ -613,7 +610,7 @@ int forward_body(pgmi_ctx* x, hipStream_t s, const int64_t* ids, int rows, const
             WAttnArgs a{};
             a.hd = attn_heads(d, l, w); a.sc = attn_score(l, w);
             a.ldqkv = r8(w.in.n); a.ldo = r8(l.heads * l.vdim);
-            matmul_rt(s, d.act, d.h, d.ldh, w.in.w, w.in.ldw, rows, w.in.n, w.in.k, RT_ACT, w.bias, d.p0, a.ldqkv, 0, nullptr);
+            matmul_rt(s, d.act, d.h, d.ldh, w.in.w, w.in.ldw, rows, w.in.n, w.in.k, RT_ACT, w.bias, d.p0, a.ldqkv, 0);
             a.qkv = d.p0; a.q = d.p1; a.kc = at<void>(state, st[i].a); a.vc = at<void>(state, st[i].b);
             a.max_tokens = max_tokens; a.o = d.p2; a.rows = rows; a.seqs = m.seqs; a.nseq = m.nseq; a.row_seq = m.row_seq;
             const auto& t = m.tiles.at(l.heads / l.kv_heads);
@@ -623,7 +620,7 @@ int forward_body(pgmi_ctx* x, hipStream_t s, const int64_t* ids, int rows, const
             out_proj(w.o, d.p2, a.ldo, w.sub[0]);
         } else {
             const int C = l.width, ldz = r8(3 * C), ldc = r8(C);
-            matmul_rt(s, d.act, d.h, d.ldh, w.in.w, w.in.ldw, rows, 3 * C, w.in.k, RT_ACT, w.bias, d.p0, ldz, 0, nullptr);
+            matmul_rt(s, d.act, d.h, d.ldh, w.in.w, w.in.ldw, rows, 3 * C, w.in.k, RT_ACT, w.bias, d.p0, ldz, 0);
             GruArgs a{};
             a.zug = d.p0; a.ld = ldz; a.state = at<float>(state, st[i].a); a.cstate = d.cstate; a.y = d.p2; a.ldy = ldc;
             a.C = C; a.seqs = m.seqs; a.nseq = m.nseq; a.chunks = m.gru.p; a.nchunk = m.gru.n; a.multi = m.gru.multi;
@@ -633,14 +630,13 @@ int forward_body(pgmi_ctx* x, hipStream_t s, const int64_t* ids, int rows, const
         if (has_ff(l)) read(i, 1, nullptr);
         if (l.experts) {
             const int sp = matmul_rt(s, d.act, d.h, d.ldh, w.router.w, w.router.ldw, rows, w.router.n, w.router.k, RT_SLABS,
-                                     nullptr, d.slabs, 0, d.slab_bytes, nullptr);
+                                     nullptr, d.slabs, 0, d.slab_bytes);
             route(s, route_args(d, l, w, rows, sp));
             experts_rt(s, d.act, EX_SWIGLU, expert_args(d, l, w, rows, EX_SWIGLU));
             experts_rt(s, d.act, EX_STORE, expert_args(d, l, w, rows, EX_STORE));
         }
         if (const int ff = l.experts ? l.shared_ff : l.ff) {
-            matmul_rt(s, d.act, d.h, d.ldh, w.gu.w, w.gu.ldw, rows, ff, w.gu.k, RT_SWIGLU, nullptr, d.p2, r8(ff), 0,
-                      reinterpret_cast<float*>(d.p0));
+            matmul_rt(s, d.act, d.h, d.ldh, w.gu.w, w.gu.ldw, rows, ff, w.gu.k, RT_SWIGLU, nullptr, d.p2, r8(ff), 0);
             out_proj(w.down, d.p2, r8(ff), w.sub[1]);
         }
         if (l.experts) pend.mix = expert_mix(d, l);
@@ -680,7 +676,7 @@ int forward_body(pgmi_ctx* x, hipStream_t s, const int64_t* ids, int rows, const
             gemv_rt(s, d.act, GR_F32, g);
         } else {
             matmul_rt(s, d.act, h, d.ldh, d.head.w, d.head.ldw, n_want, d.c.vocab, d.head.k, RT_F32, nullptr, logits,
-                      d.c.vocab, 0, nullptr);
+                      d.c.vocab, 0);
         }
     }
     LAUNCHCHK();
@@ -755,7 +751,7 @@ int decode_body_rt(pgmi_ctx* x, hipStream_t s, const int64_t* ids, int B, void* 
             g.X = d.X; g.S = d.c.streams; g.D = D; g.mix = sub.mix; g.wout = sub.out; g.mult = d.c.residual_mult;
             gemv_rt(s, d.act, GR_STREAMS, g);
         } else {
-            pend.split = matmul_rt(s, d.act, in, ldin, o.w, o.ldw, B, D, o.k, RT_SLABS, nullptr, d.slabs, D, d.slab_bytes, nullptr);
+            pend.split = matmul_rt(s, d.act, in, ldin, o.w, o.ldw, B, D, o.k, RT_SLABS, nullptr, d.slabs, D, d.slab_bytes);
             pend.y = d.slabs;
             pend.sub = &sub;
         }
@@ -777,7 +773,7 @@ int decode_body_rt(pgmi_ctx* x, hipStream_t s, const int64_t* ids, int B, void* 
                 a.z = d.p0; a.ldz = ldc;
             } else {
                 const int ldxz = r8(2 * C);
-                matmul_rt(s, d.act, d.h, d.ldh, w.in.w, w.in.ldw, B, 2 * C, w.in.k, RT_ACT, nullptr, d.p0, ldxz, 0, nullptr);
+                matmul_rt(s, d.act, d.h, d.ldh, w.in.w, w.in.ldw, B, 2 * C, w.in.k, RT_ACT, nullptr, d.p0, ldxz, 0);
                 conv_step(s, d.act, d.p0, ldxz, B, C, l.conv, w.conv, w.conv_b, taps, d.slot, d.pos, d.p1, ldc);
                 a.z = d.p0 + (size_t)C * d.es; a.ldz = ldxz;
             }
@@ -789,7 +785,7 @@ int decode_body_rt(pgmi_ctx* x, hipStream_t s, const int64_t* ids, int B, void* 
                 a.split = g.split;
             } else {
                 a.split = matmul_rt(s, d.act, d.p1, ldc, w.x.w, w.x.ldw, B, w.x.n, w.x.k, RT_SLABS, nullptr, d.slabs, 0,
-                                    d.slab_bytes, nullptr);
+                                    d.slab_bytes);
             }
             a.slabs = d.slabs; a.Wdt = w.dt.w; a.ldwdt = w.dt.ldw; a.dtb = w.dt_b; a.x = d.p1; a.ldx = ldc; a.A_log = w.A_log;
             a.Dw = w.D; a.state = at<float>(state, st[i].b); a.slot = d.slot; a.pos = d.pos; a.y = d.p2; a.ldy = ldc;
@@ -805,7 +801,7 @@ int decode_body_rt(pgmi_ctx* x, hipStream_t s, const int64_t* ids, int B, void* 
                 g.out = d.p0; g.ldo = a.ldqkv; g.bias = w.bias;
                 gemv_rt(s, d.act, GR_ACT, g);
             } else {
-                matmul_rt(s, d.act, d.h, d.ldh, w.in.w, w.in.ldw, B, w.in.n, w.in.k, RT_ACT, w.bias, d.p0, a.ldqkv, 0, nullptr);
+                matmul_rt(s, d.act, d.h, d.ldh, w.in.w, w.in.ldw, B, w.in.n, w.in.k, RT_ACT, w.bias, d.p0, a.ldqkv, 0);
             }
             a.qkv = d.p0; a.kc = at<void>(state, st[i].a); a.vc = at<void>(state, st[i].b); a.max_tokens = max_tokens;
             a.o = d.p2; a.B = B; a.slot = d.slot; a.pos = d.pos; a.part = d.part;
@@ -819,7 +815,7 @@ int decode_body_rt(pgmi_ctx* x, hipStream_t s, const int64_t* ids, int B, void* 
                 g.N = C; g.out = d.p2; g.ldo = ldc; g.bias = w.bias; g.state = at<float>(state, st[i].a);
                 gemv_rt(s, d.act, GR_GRU, g);
             } else {
-                matmul_rt(s, d.act, d.h, d.ldh, w.in.w, w.in.ldw, B, 3 * C, w.in.k, RT_ACT, w.bias, d.p0, r8(3 * C), 0, nullptr);
+                matmul_rt(s, d.act, d.h, d.ldh, w.in.w, w.in.ldw, B, 3 * C, w.in.k, RT_ACT, w.bias, d.p0, r8(3 * C), 0);
                 gru_step(s, d.act, d.p0, r8(3 * C), B, C, at<float>(state, st[i].a), d.slot, d.pos, d.p2, ldc);
             }
             out_proj(w.o, d.p2, ldc, w.sub[0]);
@@ -851,7 +847,7 @@ int decode_body_rt(pgmi_ctx* x, hipStream_t s, const int64_t* ids, int B, void* 
                 gemv_rt(s, d.act, GR_F32, g);
             } else {
                 sp = matmul_rt(s, d.act, d.h, d.ldh, w.router.w, w.router.ldw, B, w.router.n, w.router.k, RT_SLABS, nullptr,
-                               d.slabs, 0, d.slab_bytes, nullptr);
+                               d.slabs, 0, d.slab_bytes);
             }
             route(s, route_args(d, l, w, B, sp));
             experts_rt(s, d.act, EX_SWIGLU, expert_args(d, l, w, B, EX_SWIGLU));
@@ -865,12 +861,11 @@ int decode_body_rt(pgmi_ctx* x, hipStream_t s, const int64_t* ids, int B, void* 
                 g.N = ff; g.out = d.p2; g.ldo = r8(ff);
                 gemv_rt(s, d.act, GR_SWIGLU, g);
             } else {
-                matmul_rt(s, d.act, d.h, d.ldh, w.gu.w, w.gu.ldw, B, ff, w.gu.k, RT_SWIGLU, nullptr, d.p2, r8(ff), 0,
-                          reinterpret_cast<float*>(d.p0));
+                matmul_rt(s, d.act, d.h, d.ldh, w.gu.w, w.gu.ldw, B, ff, w.gu.k, RT_SWIGLU, nullptr, d.p2, r8(ff), 0);
             }
             if (l.experts) {  // the next residual pass scales it by its gate
                 pend.split = matmul_rt(s, d.act, d.p2, r8(ff), w.down.w, w.down.ldw, B, D, w.down.k, RT_SLABS, nullptr, d.slabs, D,
-                                       d.slab_bytes, nullptr);
+                                       d.slab_bytes);
                 pend.y = d.slabs;
             } else {
                 out_proj(w.down, d.p2, r8(ff), w.sub[1]);
@@ -889,7 +884,7 @@ int decode_body_rt(pgmi_ctx* x, hipStream_t s, const int64_t* ids, int B, void* 
         if (!parts) argmax_rows(s, logits, B, V, x->amax_v, x->amax_i, next);
         decode_finish(s, B, d.pmax, d.pidx, parts, next, hist, d.pos);
     } else {
-        matmul_rt(s, d.act, d.h, d.ldh, d.head.w, d.head.ldw, B, V, d.head.k, RT_F32, nullptr, logits, V, 0, nullptr);
+        matmul_rt(s, d.act, d.h, d.ldh, d.head.w, d.head.ldw, B, V, d.head.k, RT_F32, nullptr, logits, V, 0);
         argmax_rows(s, logits, B, V, x->amax_v, x->amax_i, next);
         decode_finish(s, B, nullptr, nullptr, 0, next, hist, d.pos);
     }
@@ -1177,8 +1172,7 @@ int pgmi_op_matmul(pgmi_ctx* x, const void* A, int lda, const void* W, int ldw, 
     if (mode == RT_SWIGLU && act == PGMI_DTYPE_F32 && !scratch) return fail(PGMI_E_ARG, "fp32 gate|up needs scratch");
     const int sp = matmul_rt((hipStream_t)stream, act == PGMI_DTYPE_F32 ? ACT_F32 : ACT_BF16, A, lda,
                              reinterpret_cast<const uint16_t*>(W), ldw, M, N, K, (RtOut)mode,
-                             reinterpret_cast<const uint16_t*>(bias), out, ldo, (size_t)std::max<int64_t>(out_bytes, 0),
-                             reinterpret_cast<float*>(scratch));
+                             reinterpret_cast<const uint16_t*>(bias), out, ldo, (size_t)std::max<int64_t>(out_bytes, 0));
     if (split) *split = sp;
     LAUNCHCHK();
     return 0;

@@ -1,8 +1,8 @@
 // kernels_matmul.hip -- matrix products of the layered decoders: any M and N, K a multiple of 8.
 //
 // bf16 activations run on the prefill GEMM kernels (kernels_gemm.hip: LDS-DMA panel, warp-specialised and 8-phase
-// forms), a few instantiations chosen by shape; fp32 activations on a plain fp32 tile kernel (no reduced-precision
-// matrix mode).  Weights are bf16 [N][ldw] in both.
+// forms), a few instantiations chosen by shape; fp32 activations on tile_f32.h's exact split over the same matrix units.
+// Weights are bf16 [N][ldw] in both.
 #define PGMI_GEMM_KERNELS_ONLY
 #include "kernels_gemm.hip"
 
@@ -10,58 +10,53 @@
 
 #include "act.h"
 #include "decoder.h"
+#include "tile_f32.h"
 
 namespace pgmi {
 
 namespace {
 
 // ---------------------------------------------------------------- fp32
-constexpr int FT = 64, FK = 16;
+struct F32Args {
+    const float* A;
+    int lda;
+    const uint16_t* W;
+    int ldw, M, N, K;
+    const uint16_t* bias;
+    float* out;
+    int ldo;  // columns; N .. ldo-1 are written as zeros
+    int per;  // 64-deep steps of a K slice, one slab [M][ldo] each
+};
 
-__global__ void __launch_bounds__(256) k_matmul_f32(const float* __restrict__ A, int lda, const uint16_t* __restrict__ W,
-                                                    int ldw, int M, int N, int K, const uint16_t* __restrict__ bias,
-                                                    float* __restrict__ out, int ldo) {
-    __shared__ float As[FK][FT + 4], Bs[FK][FT + 4];
-    const int tid = threadIdx.x, m0 = blockIdx.y * FT, n0 = blockIdx.x * FT;
-    const int tm = (tid >> 4) * 4, tn = (tid & 15) * 4;
-    float acc[4][4] = {};
-    for (int k0 = 0; k0 < K; k0 += FK) {
-#pragma unroll
-        for (int i = 0; i < FT * FK / 256; ++i) {
-            const int e = tid + 256 * i, r = e / FK, k = e % FK;
-            const int m = m0 + r, n = n0 + r, kk = k0 + k;
-            As[k][r] = (m < M && kk < K) ? A[(long)m * lda + kk] : 0.0f;
-            Bs[k][r] = (n < N && kk < K) ? bf2f(W[(long)n * ldw + kk]) : 0.0f;
-        }
-        __syncthreads();
-#pragma unroll
-        for (int k = 0; k < FK; ++k) {
-            float a[4], b[4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) { a[i] = As[k][tm + i]; b[i] = Bs[k][tn + i]; }
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int j = 0; j < 4; ++j) acc[i][j] = fmaf(a[i], b[j], acc[i][j]);
-        }
-        __syncthreads();
-    }
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int m = m0 + tm + i, n = n0 + tn + j;
-            if (m < M && n < ldo) out[(long)m * ldo + n] = n < N ? acc[i][j] + (bias ? bf2f(bias[n]) : 0.0f) : 0.0f;
-        }
+// grid (row tiles x column tiles, K slices), the row tiles of a column tile adjacent.  NB = 2: gate and up columns, silu(gate)
+// up stored.
+template <int WM, int WN, int TM, int TN, int NB>
+__global__ void __launch_bounds__(64 * WM * WN) k_matmul_f32(F32Args a) {
+    constexpr int BM = 16 * WM * TM, BN = 16 * WN * TN;
+    const int n_mt = (a.M + BM - 1) / BM, m0 = blockIdx.x % n_mt * BM, n0 = blockIdx.x / n_mt * BN;
+    const int k0 = blockIdx.y * a.per * 64, k1 = min(a.K, k0 + a.per * 64);
+    float* out = a.out + (long)blockIdx.y * a.M * a.ldo;
+    tile_f32<WM, WN, TM, TN, NB>(
+        a.A, a.lda, a.W, a.ldw, (long)a.N * a.ldw, a.N, a.ldo, n0, k0, k1, [&](int m) { return min(m0 + m, a.M - 1); },
+        [&](int m, int n, float v, float u) {
+            if (m0 + m >= a.M) return;
+            if constexpr (NB == 2) v = siluf_(v) * u;
+            else if (a.bias && n < a.N) v += bf2f(a.bias[n]);
+            out[(long)(m0 + m) * a.ldo + n] = n < a.N ? v : 0.0f;
+        });
 }
 
-// [M][2N] gate|up -> [M][ldo]
-__global__ void k_swiglu_f32(const float* __restrict__ gu, int M, int N, float* __restrict__ out, int ldo) {
-    for (long i = blockIdx.x * 256L + threadIdx.x; i < (long)M * ldo; i += gridDim.x * 256L) {
-        const long m = i / ldo;
-        const int n = (int)(i % ldo);
-        out[i] = n < N ? siluf_(gu[m * 2 * N + n]) * gu[m * 2 * N + N + n] : 0.0f;
-    }
+template <int WM, int WN, int TM, int TN, int NB>
+void run_f32(hipStream_t s, const F32Args& a, int split) {
+    constexpr int BM = 16 * WM * TM, BN = 16 * WN * TN;
+    constexpr size_t lds = tile_f32_lds(BM, BN, NB);
+    static const bool once = [] {
+        return hipFuncSetAttribute(reinterpret_cast<const void*>(&k_matmul_f32<WM, WN, TM, TN, NB>),
+                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) == hipSuccess;
+    }();
+    (void)once;
+    hipLaunchKernelGGL((k_matmul_f32<WM, WN, TM, TN, NB>), dim3((a.M + BM - 1) / BM * ((a.ldo + BN - 1) / BN), split),
+                       dim3(64 * WM * WN), lds, s, a);
 }
 
 // zeros in columns N .. ldo-1 (the GEMM kernels write columns < N only)
@@ -145,12 +140,11 @@ void run_plan(const Job& j) {
         run_p64<EPI, SPLIT>(j);
 }
 
-// K slices for a product whose tiles alone leave CUs idle
-int pick_split(int M, int N, int K, size_t out_bytes) {
+// K slices for a product whose t tiles alone leave CUs idle
+int pick_split(long t, int want, int M, int N, int K, size_t out_bytes) {
     const int nkt = (K + 63) / 64;
-    const long t = tiles(M, N, 64, 64);
     int split = 1;
-    while (t * split < 256 && split < 8 && nkt / (split * 2) >= 4) split *= 2;
+    while (t * split < want && split < 8 && nkt / (split * 2) >= 4) split *= 2;
     while (split > 1 && (size_t)split * M * N * sizeof(float) > out_bytes) split /= 2;
     if (split > 1) {  // every slice non-empty
         const int per = (nkt + split - 1) / split;
@@ -162,24 +156,36 @@ int pick_split(int M, int N, int K, size_t out_bytes) {
 }  // namespace
 
 int matmul_rt(hipStream_t s, Act act, const void* A, int lda, const uint16_t* W, int ldw, int M, int N, int K,
-              RtOut mode, const uint16_t* bias, void* out, int ldo, size_t out_bytes, float* scratch) {
+              RtOut mode, const uint16_t* bias, void* out, int ldo, size_t out_bytes) {
     if (M <= 0 || N <= 0) return 1;
     if (act == ACT_F32) {
-        const float* a = reinterpret_cast<const float*>(A);
-        const bool dual = mode == RT_SWIGLU, plain = mode == RT_F32 || mode == RT_SLABS;
-        const int n = dual ? 2 * N : N;
-        float* o = dual ? scratch : reinterpret_cast<float*>(out);
-        const int ld = dual ? n : plain ? N : ldo;
-        hipLaunchKernelGGL(k_matmul_f32, dim3((ld + FT - 1) / FT, (M + FT - 1) / FT), dim3(256), 0, s, a, lda, W, ldw, M,
-                           n, K, plain ? nullptr : bias, o, ld);
-        if (dual)
-            hipLaunchKernelGGL(k_swiglu_f32, dim3(1024), dim3(256), 0, s, scratch, M, N, reinterpret_cast<float*>(out), ldo);
-        return 1;
+        const bool plain = mode == RT_F32 || mode == RT_SLABS;
+        F32Args f{reinterpret_cast<const float*>(A), lda, W, ldw, M, N, K, plain ? nullptr : bias, reinterpret_cast<float*>(out),
+                  plain ? N : ldo, (K + 63) / 64};
+        // 64 x 128 tiles of 8 waves once they fill the chip, else 32 x 64 tiles of 4 waves, which more workgroups share.
+        // Measured, us: 500 x 1024, K = 4096: 20.9 (4 slices) against 22.1; 500 x 4096, K = 1024: 20.9 / 26.7;
+        // 300 x 1024, K = 1024: 17.2 / 10.4
+        int split = 1;
+        auto cut = [&](int bm, int bn, int want) {
+            const long t = tiles(M, f.ldo, bm, bn);
+            if (mode == RT_SLABS) split = pick_split(t, want, M, N, K, out_bytes);
+            f.per = ((K + 63) / 64 + split - 1) / split;
+            return t * split;
+        };
+        if (cut(64, 128, 256) >= 256) {
+            if (mode == RT_SWIGLU) run_f32<2, 4, 2, 2, 2>(s, f, 1);
+            else run_f32<2, 4, 2, 2, 1>(s, f, split);
+        } else {
+            cut(32, 64, 512);
+            if (mode == RT_SWIGLU) run_f32<1, 4, 2, 1, 2>(s, f, 1);
+            else run_f32<1, 4, 2, 1, 1>(s, f, split);
+        }
+        return split;
     }
     Job j{s, reinterpret_cast<const uint16_t*>(A), lda, W, ldw, M, N, K, {}, nullptr, 1, 0};
     if (mode == RT_F32 || mode == RT_SLABS) {
         j.ws = reinterpret_cast<float*>(out);
-        if (mode == RT_SLABS) j.split = pick_split(M, N, K, out_bytes);
+        if (mode == RT_SLABS) j.split = pick_split(tiles(M, N, 64, 64), 256, M, N, K, out_bytes);
         run_plan<EPI_STORE, true>(j);
         return j.split;
     }

@@ -5,7 +5,7 @@
 //   k_experts         bf16 MFMA, LDS-DMA ring with loader waves: row tiles of one expert's list, gathered by each
 //                     loader lane's own source address, results scattered to the entries' rows
 //   k_experts_8p      the same rows on the 8-phase 256 x 256 tiles of kernels_gemm.hip, for long lists
-//   k_experts_f32     the same product on fp32 FMA tiles
+//   k_experts_f32     the same product of fp32 rows, on tile_f32.h's exact split
 //   k_experts_skinny  few rows: one workgroup per (16 outputs, used expert), MFMA straight from HBM
 #define PGMI_GEMM_KERNELS_ONLY
 #include "kernels_gemm.hip"
@@ -15,6 +15,7 @@
 #include "act.h"
 #include "decoder.h"
 #include "route.h"
+#include "tile_f32.h"
 
 namespace pgmi {
 
@@ -301,50 +302,35 @@ void run_experts_8p(hipStream_t s, const ExpertArgs& a) {
 }
 
 // ---------------------------------------------------------------- fp32
-constexpr int FT = 64, FK = 16;
-
-template <int MODE>
-__global__ void __launch_bounds__(256) k_experts_f32(ExpertArgs a) {
-    constexpr int NB = MODE == EX_SWIGLU ? 2 : 1;
-    __shared__ float As[FK][FT + 4], Bs[NB][FK][FT + 4];
-    __shared__ int ent[FT];
-    const TileAt tl = find_tile(a.cnt, a.experts, FT, (a.ldo + FT - 1) / FT);
+// tile_f32's tiles over an expert's list
+template <int WM, int WN, int TM, int TN, int MODE>
+__global__ void __launch_bounds__(64 * WM * WN) k_experts_f32(ExpertArgs a) {
+    constexpr int BM = 16 * WM * TM, BN = 16 * WN * TN, NB = MODE == EX_SWIGLU ? 2 : 1;
+    const TileAt tl = find_tile(a.cnt, a.experts, BM, (a.ldo + BN - 1) / BN);
     if (tl.e < 0) return;
-    const int tid = threadIdx.x, n0 = tl.nt * FT, tm = (tid >> 4) * 4, tn = (tid & 15) * 4;
-    const uint16_t* We = a.W + tl.e * a.wstride;
-    if (tid < FT) ent[tid] = tl.m0 + tid < tl.cnt ? a.list[(long)tl.e * a.cap + tl.m0 + tid] : -1;
-    __syncthreads();
-    float acc[NB][4][4] = {};
-    for (int k0 = 0; k0 < a.K; k0 += FK) {
-#pragma unroll
-        for (int i = 0; i < FT * FK / 256; ++i) {
-            const int x = tid + 256 * i, r = x / FK, k = x % FK, n = n0 + r, kk = k0 + k;
-            As[k][r] = ent[r] >= 0 && kk < a.K ? reinterpret_cast<const float*>(a.A)[(long)(ent[r] / a.gather) * a.lda + kk]
-                                               : 0.0f;
-#pragma unroll
-            for (int b = 0; b < NB; ++b)
-                Bs[b][k][r] = n < a.N && kk < a.K ? bf2f(We[((long)b * a.N + n) * a.ldw + kk]) : 0.0f;
-        }
-        __syncthreads();
-#pragma unroll
-        for (int k = 0; k < FK; ++k)
-#pragma unroll
-            for (int b = 0; b < NB; ++b)
-#pragma unroll
-                for (int i = 0; i < 4; ++i)
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) acc[b][i][j] = fmaf(As[k][tm + i], Bs[b][k][tn + j], acc[b][i][j]);
-        __syncthreads();
-    }
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int e = ent[tm + i], n = n0 + tn + j;
-            float v = acc[0][i][j];
-            if constexpr (MODE == EX_SWIGLU) v = siluf_(v) * acc[NB - 1][i][j];
-            if (e >= 0 && n < a.ldo) reinterpret_cast<float*>(a.out)[(long)e * a.ldo + n] = n < a.N ? v : 0.0f;
-        }
+    const int* list = a.list + (long)tl.e * a.cap;
+    float* out = reinterpret_cast<float*>(a.out);
+    tile_f32<WM, WN, TM, TN, NB>(
+        reinterpret_cast<const float*>(a.A), a.lda, a.W + tl.e * a.wstride, a.ldw, (long)a.N * a.ldw, a.N, a.ldo, tl.nt * BN, 0,
+        a.K, [&](int m) { return list[min(tl.m0 + m, tl.cnt - 1)] / a.gather; },
+        [&](int m, int n, float v, float u) {
+            if (tl.m0 + m >= tl.cnt) return;
+            if constexpr (MODE == EX_SWIGLU) v = siluf_(v) * u;
+            out[(long)list[tl.m0 + m] * a.ldo + n] = n < a.N ? v : 0.0f;
+        });
+}
+
+template <int WM, int WN, int TM, int TN, int MODE>
+void run_experts_f32(hipStream_t s, const ExpertArgs& a) {
+    constexpr int BM = 16 * WM * TM, BN = 16 * WN * TN;
+    constexpr size_t lds = tile_f32_lds(BM, BN, MODE == EX_SWIGLU ? 2 : 1);
+    static const bool once = [] {
+        return hipFuncSetAttribute(reinterpret_cast<const void*>(&k_experts_f32<WM, WN, TM, TN, MODE>),
+                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) == hipSuccess;
+    }();
+    (void)once;
+    const dim3 grid((unsigned)((max_tiles(a, BM) * ((a.ldo + BN - 1) / BN) + 7) / 8 * 8));
+    hipLaunchKernelGGL((k_experts_f32<WM, WN, TM, TN, MODE>), grid, dim3(64 * WM * WN), lds, s, a);
 }
 
 // ---------------------------------------------------------------- few rows
@@ -436,15 +422,16 @@ void route(hipStream_t s, const RouteArgs& a) {
 }
 
 void experts_rt(hipStream_t s, Act act, ExpertMode mode, const ExpertArgs& a) {
-    if (act == ACT_F32) {
-        const dim3 grid((unsigned)((max_tiles(a, FT) * ((a.ldo + FT - 1) / FT) + 7) / 8 * 8));
-        if (mode == EX_SWIGLU) hipLaunchKernelGGL((k_experts_f32<EX_SWIGLU>), grid, dim3(256), 0, s, a);
-        else hipLaunchKernelGGL((k_experts_f32<EX_STORE>), grid, dim3(256), 0, s, a);
-        return;
-    }
     const int per = a.entries / std::max(1, a.experts);  // rows of an average expert
     auto go = [&](auto mode_c) {
         constexpr int MODE = decltype(mode_c)::value;
+        // fp32: 64 x 128 tiles of 8 waves (120 rows per expert, 512 x 1024: 31.6 us, 4 waves on 64 x 64: 33.8; FMA tiles: 213),
+        // of short lists 32 x 64, whose idle rows cost less
+        if (act == ACT_F32) {
+            if (per > 24) run_experts_f32<2, 4, 2, 2, MODE>(s, a);
+            else run_experts_f32<1, 4, 2, 1, MODE>(s, a);
+            return;
+        }
         const bool p8 = a.K % 64 == 0 && a.K >= 512;
         if (p8 && per > 384) run_experts_8p<8, MODE>(s, a);
         else if (p8 && per > 128) run_experts_8p<6, MODE>(s, a);

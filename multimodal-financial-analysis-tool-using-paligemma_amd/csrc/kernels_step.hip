@@ -2,9 +2,11 @@
 // (up to 16 rows) of any size with the surrounding steps fused (streams' read + grouped norm in front; convolution step, minGRU step, gated
 // activation, streams' update or argmax behind), and the selective-scan step.
 #include <algorithm>
+#include <type_traits>
 
 #include "act.h"
 #include "decoder.h"
+#include "tile_f32.h"
 
 namespace pgmi {
 
@@ -371,10 +373,11 @@ void run_mode(hipStream_t s, GemvRtMode mode, const GemvRtArgs& a) {
 // contract k = 16 lg .. 16 lg + 7 and 16 lg + 8 .. 16 lg + 15 of each lane group -- the activations (straight from
 // L2, B fragments) use the same order.  After the waves' sums meet in LDS, thread (n, b) runs the step's epilogue.
 // GR_F32 with gridDim.y > 1: K is cut over the y workgroups too, out holds their partial slabs [y][B][N].
-template <int MODE>
+template <typename T, int MODE>
 __global__ void __launch_bounds__(256) k_skinny(GemvRtArgs a) {
     constexpr int NM = MODE == GR_GRU ? 3 : MODE == GR_SWIGLU ? 2 : 1;
-    constexpr int U = NM == 1 ? 8 : 4;  // 64-deep steps in flight
+    constexpr bool F32 = std::is_same<T, float>::value;
+    constexpr int U = NM == 1 && !F32 ? 8 : 4;  // 64-deep steps in flight
     __shared__ float sums[4][NM][16][17];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int li = lane & 15, lg = lane >> 4, n0 = blockIdx.x * 16, K = a.K;
@@ -384,14 +387,15 @@ __global__ void __launch_bounds__(256) k_skinny(GemvRtArgs a) {
         const int n = n0 + li < a.N ? n0 + li : a.N - 1;
         wp[m] = a.W + ((long)m * a.N + n) * a.ldw;
     }
-    const uint16_t* xp = reinterpret_cast<const uint16_t*>(a.x) + (long)(li < a.B ? li : a.B - 1) * a.ldx;
+    const T* xp = reinterpret_cast<const T*>(a.x) + (long)(li < a.B ? li : a.B - 1) * a.ldx;
     f32x4 acc[NM];
 #pragma unroll
     for (int m = 0; m < NM; ++m) acc[m] = f32x4{0.f, 0.f, 0.f, 0.f};
     const int nstep = (K + 63) / 64;
     const int per = (nstep + gridDim.y - 1) / gridDim.y, s_end = min(nstep, (int)(blockIdx.y + 1) * per);
     for (int s0 = blockIdx.y * per + wave; s0 < s_end; s0 += 4 * U) {
-        uint4 w[U][NM][2], x[U][2];
+        uint4 w[U][NM][2];
+        typename X8<T>::type x[U][2];
 #pragma unroll
         for (int i = 0; i < U; ++i) {
             const int k = (s0 + 4 * i) * 64 + lg * 16;
@@ -400,16 +404,27 @@ __global__ void __launch_bounds__(256) k_skinny(GemvRtArgs a) {
                 const bool ok = s0 + 4 * i < s_end && k + 8 * h < K;
 #pragma unroll
                 for (int m = 0; m < NM; ++m) w[i][m][h] = ldg16_sel(wp[m] + k + 8 * h, ok, wp[m]);
-                x[i][h] = ldg16_sel(xp + k + 8 * h, ok, xp);
+                if constexpr (F32) ldx(ok ? xp + k + 8 * h : xp, x[i][h]);  // past the end: the weights are zero
+                else x[i][h].q = ldg16_sel(xp + k + 8 * h, ok, xp);
             }
         }
 #pragma unroll
         for (int i = 0; i < U; ++i)
 #pragma unroll
-            for (int h = 0; h < 2; ++h)
+            for (int h = 0; h < 2; ++h) {
+                if constexpr (F32) {  // tile_f32.h's pieces, the smallest first
+                    const F32Pieces q = cut8(x[i][h].a, x[i][h].b);
 #pragma unroll
-                for (int m = 0; m < NM; ++m)
-                    acc[m] = mfma16(__builtin_bit_cast(short8, w[i][m][h]), __builtin_bit_cast(short8, x[i][h]), acc[m]);
+                    for (int p = 2; p >= 0; --p)
+#pragma unroll
+                        for (int m = 0; m < NM; ++m)
+                            acc[m] = mfma16(__builtin_bit_cast(short8, w[i][m][h]), __builtin_bit_cast(short8, q.p[p]), acc[m]);
+                } else {
+#pragma unroll
+                    for (int m = 0; m < NM; ++m)
+                        acc[m] = mfma16(__builtin_bit_cast(short8, w[i][m][h]), __builtin_bit_cast(short8, x[i][h].q), acc[m]);
+                }
+            }
     }
 #pragma unroll
     for (int m = 0; m < NM; ++m)
@@ -422,24 +437,33 @@ __global__ void __launch_bounds__(256) k_skinny(GemvRtArgs a) {
     for (int m = 0; m < NM; ++m)
 #pragma unroll
         for (int q = 0; q < 4; ++q) v[m] += sums[q][m][tid >> 4][b];
+    if constexpr (F32) {
+        // what is not finite (of rows and outputs that there are): the FMA chain over this workgroup's K slice
+        if (b < a.B && n < a.N)
+            for (int m = 0; m < NM; ++m)
+                if (not_finite(v[m]))
+                    v[m] = dot_f32(reinterpret_cast<const float*>(a.x) + (long)b * a.ldx, a.W + ((long)m * a.N + n) * a.ldw,
+                                   blockIdx.y * per * 64, min(K, s_end * 64));
+    }
     if constexpr (MODE == GR_F32) {
         if (b < a.B && n < a.N)
             reinterpret_cast<float*>(a.out)[((long)blockIdx.y * a.B + b) * a.ldo + n] = v[0];
         return;
     }
-    if (b < a.B && n < a.N) step_epilogue<uint16_t, MODE>(a, n, b, v[0], v[1], v[2]);
-    step_pads<uint16_t, MODE>(a);
+    if (b < a.B && n < a.N) step_epilogue<T, MODE>(a, n, b, v[0], v[1], v[2]);
+    step_pads<T, MODE>(a);
 }
 
+template <typename T>
 void run_skinny(hipStream_t s, GemvRtMode mode, const GemvRtArgs& a) {
     const dim3 grid((a.N + 15) / 16), block(256);
     switch (mode) {
-        case GR_ACT: hipLaunchKernelGGL((k_skinny<GR_ACT>), grid, block, 0, s, a); break;
-        case GR_CONV: hipLaunchKernelGGL((k_skinny<GR_CONV>), grid, block, 0, s, a); break;
-        case GR_GRU: hipLaunchKernelGGL((k_skinny<GR_GRU>), grid, block, 0, s, a); break;
-        case GR_SWIGLU: hipLaunchKernelGGL((k_skinny<GR_SWIGLU>), grid, block, 0, s, a); break;
-        case GR_STREAMS: hipLaunchKernelGGL((k_skinny<GR_STREAMS>), grid, block, 0, s, a); break;
-        default: hipLaunchKernelGGL((k_skinny<GR_F32>), dim3(grid.x, a.split < 1 ? 1 : a.split), block, 0, s, a); break;
+        case GR_ACT: hipLaunchKernelGGL((k_skinny<T, GR_ACT>), grid, block, 0, s, a); break;
+        case GR_CONV: hipLaunchKernelGGL((k_skinny<T, GR_CONV>), grid, block, 0, s, a); break;
+        case GR_GRU: hipLaunchKernelGGL((k_skinny<T, GR_GRU>), grid, block, 0, s, a); break;
+        case GR_SWIGLU: hipLaunchKernelGGL((k_skinny<T, GR_SWIGLU>), grid, block, 0, s, a); break;
+        case GR_STREAMS: hipLaunchKernelGGL((k_skinny<T, GR_STREAMS>), grid, block, 0, s, a); break;
+        default: hipLaunchKernelGGL((k_skinny<T, GR_F32>), dim3(grid.x, a.split < 1 ? 1 : a.split), block, 0, s, a); break;
     }
 }
 
@@ -585,10 +609,10 @@ __global__ void __launch_bounds__(256) k_decode_finish(const float* __restrict__
 int gemv_rt_max_batch() { return 16; }
 int gemv_rt_parts() { return 2 * 1024; }
 GemvRtForm gemv_rt_form(int B, Act act, int streams, int width) {
-    // fp32 activations: no MFMA form.  bf16: one row, while every workgroup's own read of the streams stays small;
+    // fp32 activations: two rows.  bf16: one row, while every workgroup's own read of the streams stays small;
     // measured, batch 1, 2 streams: width 1024 0.379 against 0.432 ms per step, 2048 0.802 / 0.818, 4096 0.828 / 0.661
-    if (act == ACT_F32) return B <= 2 ? GF_STREAM : GF_NONE;
-    if (B == 1 && streams * width <= 4096) return GF_STREAM;
+    if (act == ACT_F32 && B <= 2) return GF_STREAM;
+    if (act == ACT_BF16 && B == 1 && streams * width <= 4096) return GF_STREAM;
     return B <= gemv_rt_max_batch() ? GF_SKINNY : GF_NONE;
 }
 
@@ -612,7 +636,8 @@ int gemv_rt_blocks(const GemvRtArgs& a, GemvRtMode mode) {
 }
 
 void gemv_rt(hipStream_t s, Act act, GemvRtMode mode, const GemvRtArgs& a) {
-    if (a.form == GF_SKINNY) run_skinny(s, mode, a);
+    if (a.form == GF_SKINNY && act == ACT_BF16) run_skinny<uint16_t>(s, mode, a);
+    else if (a.form == GF_SKINNY) run_skinny<float>(s, mode, a);
     else if (act == ACT_BF16) run_mode<uint16_t, 1>(s, mode, a);
     else if (a.B <= 1) run_mode<float, 1>(s, mode, a);
     else run_mode<float, 2>(s, mode, a);

@@ -1,0 +1,103 @@
+"""fp32 products on the bf16 matrix units (csrc/tile_f32.h): every form of them against float64 at the edges of its tiles,
+K slices and rows, and values that the exact split does not carry."""
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+import raritar_cases as R
+from decoder_helpers import build, close, tokens
+from oracle import raritar_np
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def eng():
+    return build(R.MECHANISMS["taps_1"], "float32")[0]
+
+
+def product(eng, A, W, N, mode, out):
+    from pgmi import _native as N_
+    M, K = A.shape
+    sp, scratch = ctypes.c_int(), torch.empty((M, 2 * N), device="cuda")
+    N_.check(eng.lib.pgmi_op_matmul(eng.ctx, A.data_ptr(), A.stride(0), W.data_ptr(), W.stride(0), M, N, K, 2, mode, None,
+                                    out.data_ptr(), out.shape[-1], out.numel() * 4, scratch.data_ptr(), ctypes.byref(sp),
+                                    N_.stream_handle(eng.device)))
+    return sp.value
+
+
+# 32 x 64 and 64 x 128 tiles, odd numbers of 64-deep steps, K past where the sums move (1024), one slice and eight
+@pytest.mark.parametrize("M,N,K", [(1, 1, 8), (17, 64, 64), (32, 65, 72), (33, 63, 200), (64, 130, 1032), (65, 4099, 136),
+                                   (513, 4096, 128), (500, 1024, 4160), (200, 8200, 1096)])
+def test_every_mode_against_float64(eng, M, N, K):
+    g = torch.Generator("cuda").manual_seed(M + N + K)
+    A = torch.randn((M, K + 8), device="cuda", generator=g)[:, :K]
+    W = torch.randn((2 * N, K), device="cuda", generator=g).bfloat16()
+    ref = A.double() @ W.double().t()
+    # a K-term fp32 sum: (K / 32 accumulations of 3 pieces + 8 slices) roundings of partial sums of at most sum |a w|
+    bound = (A.double().abs() @ W.double().abs().t()) * 2.0 ** -24 * (3 * min(K, 1024) / 32 + K / 1024 + 10)
+    out = torch.full((M, N), float("nan"), device="cuda")
+    product(eng, A, W, N, 1, out)
+    assert ((out.double() - ref[:, :N]).abs() <= bound[:, :N]).all()
+    slabs = torch.full((8, M, N), float("nan"), device="cuda")
+    sp = product(eng, A, W, N, 2, slabs)
+    assert 1 <= sp <= 8 and ((slabs[:sp].double().sum(0) - ref[:, :N]).abs() <= bound[:, :N]).all()
+    ldo = (N + 7) // 8 * 8
+    out = torch.full((M, ldo), float("nan"), device="cuda")
+    product(eng, A, W, N, 3, out)
+    want = torch.nn.functional.silu(ref[:, :N]) * ref[:, N:]
+    # |d silu| <= 1.1 |d gate|; silu itself to a few ulp
+    tol = 1.1 * bound[:, :N] * (ref[:, N:].abs() + bound[:, N:]) + ref[:, :N].abs() * bound[:, N:] + 1e-6 * want.abs() + 1e-30
+    assert ((out[:, :N].double() - want).abs() <= tol).all() and (out[:, N:] == 0).all()
+
+
+@pytest.mark.parametrize("M,N", [(20, 70), (300, 4096)])
+def test_values_that_are_not_finite_and_the_largest(eng, M, N):
+    """Infinities, not-a-numbers (payload in the low bits only, too) and the largest finite values, in rows and weights, give
+    what the FMA chain gives, and leave the other outputs alone."""
+    K = 200
+    g = torch.Generator("cuda").manual_seed(M)
+    A = torch.randn((M, K), device="cuda", generator=g)
+    W = torch.randn((N, K), device="cuda", generator=g).bfloat16()
+    W[:, 7] = W[:, 7].abs() + 0.5
+    W[:, :2] = torch.tensor([0.0, 1.0], device="cuda").bfloat16()
+    clean = A.double() @ W.double().t()
+    A[1, 7], A[2, 7], A[4, 100] = float("inf"), float("-inf"), float("nan")
+    A[5].view(torch.int32)[9] = 0x7F800001
+    A[6, 7] = 3.4028234663852886e38  # times 0.5 or more: finite or inf, by the weight
+    A[7, 0] = float("inf")  # meets a weight of zero
+    A[8] = 0.0
+    A[9] = 1.0000001
+    W[3, 11] = float("inf")
+    out = torch.empty((M, N), device="cuda")
+    product(eng, A, W, N, 1, out)
+    a, w = A.cpu(), W.float().cpu()
+    chain = torch.zeros((M, N))
+    for k in range(K):
+        chain = chain + a[:, k, None] * w[None, :, k]
+    got = out.cpu()
+    there = torch.ones(M, dtype=torch.bool)
+    there[6] = False  # at the edge of overflow a fused step and this one may part
+    assert torch.equal(torch.isnan(got), torch.isnan(chain))
+    assert torch.equal(got[there][chain[there].isinf()], chain[there][chain[there].isinf()])
+    fin = torch.isfinite(chain)
+    assert ((got - chain).abs()[fin] <= 1e-5 * chain.abs()[fin] + 1e-3).all()
+    ordinary = torch.ones((M, N), dtype=torch.bool)
+    ordinary[1:10], ordinary[:, 3] = False, False
+    assert ((got - clean.cpu()).abs()[ordinary] < 1e-4).all()
+
+
+@pytest.mark.parametrize("rows", [3, 16, 17, 40])
+def test_decode_rows(rows):
+    """One token each: the skinny form (to 16 rows) and the tiles, mixtures of experts included."""
+    cfg = R.MIXED["b"]
+    eng, W = build(cfg, "float32", max_batch=64)
+    seqs = [tokens(cfg, 4, 60 + r) for r in range(rows)]
+    want = [raritar_np.run(cfg, W, s) for s in seqs[:6]]
+    cache = eng.new_cache(rows, 16)
+    slots = [cache.alloc() for _ in seqs]
+    for t in range(4):
+        lg = eng.step(cache, slots, [[s[t]] for s in seqs])
+        close(lg[:6], np.stack([w[t] for w in want]), "float32")
