@@ -16,7 +16,9 @@ void gemv_mf_res_norm(hipStream_t s, const GemvArgs& a, float* ws, const uint16_
 
 template <int B, int KCH, int RPW, int MODE, int WK = 1, int DEPTH = 1, bool EMB = false>
 static void launch_gemv(hipStream_t s, const GemvArgs& a, int max_blocks = 0) {
-    constexpr bool XREG = (MODE != GV_ORES) && B * (KCH / WK) <= 8;
+    // (two rows of the 16,384-wide down projection: 64 registers of activations beside 32 of weights; staged in LDS, their
+    // 64 KiB left two workgroups per CU: 21.9 us, 14.2 in registers, 13.0 with one output per wave and 512 workgroups)
+    constexpr bool XREG = (MODE != GV_ORES) && B * (KCH / WK) <= (WK > 1 ? 16 : 8);
     size_t lds = XREG ? 0 : (size_t)B * KCH * 512 * sizeof(uint16_t);
     static size_t attr = 0;  // largest dynamic LDS size granted so far
     if (lds > attr) {
@@ -77,7 +79,7 @@ void gemv_res(hipStream_t s, int B, int K, const uint16_t* x, const uint16_t* W,
             c.x = x + (long)b0 * K; c.out = h_inout + (long)b0 * N; c.nb = nb;
             // K split in 4 inside the workgroup: 512 workgroups of one row each
             if (nb <= 1) launch_gemv<1, 32, 1, GV_RES, 4>(s, c, 512);
-            else if (nb <= 2) launch_gemv<2, 32, 2, GV_RES, 4>(s, c);
+            else if (nb <= 2) launch_gemv<2, 32, 1, GV_RES, 4>(s, c, 512);
             else launch_gemv<4, 32, 2, GV_RES, 4>(s, c);
         }
     }
@@ -128,7 +130,8 @@ void gemv_geglu(hipStream_t s, int B, const uint16_t* h, const uint16_t* norm_w,
         return;
     }
     if (B <= 1) launch_gemv<1, 4, 1, GV_GEGLU>(s, a, 1024);
-    else L_(2, 4, 2, GV_GEGLU);  // B >= 3 runs on MFMA (above)
+    // two rows: one unit per wave (us: 22.9 on 512 workgroups, 23.6 on 1024, 24.0 on 2048; two units 25.9)
+    else launch_gemv<2, 4, 1, GV_GEGLU>(s, a, 512);  // B >= 3 runs on MFMA (above)
 }
 
 int gemv_logits_blocks() { return 2048; }
