@@ -536,7 +536,7 @@ struct Meta {
         const ChunkInfo* p;
         int n;
         bool multi;  // some sequence has more than one
-    } scan, gru;
+    } scan, gru, conv;
     const int* row_seq;
     const int* want;
     std::map<int, std::pair<const ChunkInfo*, int>> tiles;  // by query heads per key/value head
@@ -566,7 +566,7 @@ int forward_body(pgmi_ctx* x, hipStream_t s, const int64_t* ids, int rows, const
                 CanonArgs c{};
                 c.X = d.X; c.inv = d.inv; c.w = sub.norm; c.w_scalar = d.c.norm_scalar; c.rows = rows; c.D = D;
                 c.taps = d.c.canon_taps; c.cw = w.canon; c.ring = at<float>(state, st[i].ring); c.h = d.h; c.ldh = d.ldh;
-                c.seqs = m.seqs; c.nseq = m.nseq; c.chunks = m.scan.p; c.nchunk = m.scan.n;
+                c.seqs = m.seqs; c.nseq = m.nseq; c.chunks = m.conv.p; c.nchunk = m.conv.n;
                 canon(s, d.act, c);
             }
             pend = {};
@@ -593,7 +593,7 @@ int forward_body(pgmi_ctx* x, hipStream_t s, const int64_t* ids, int rows, const
         if (l.mixer == PGMI_MIXER_MAMBA1) {
             const int C = l.inner, N = l.state, R = l.dt_rank, ldc = r8(C), ldxz = r8(2 * C), ldd = r8(R);
             matmul_rt(s, d.act, d.h, d.ldh, w.in.w, w.in.ldw, rows, 2 * C, w.in.k, RT_ACT, nullptr, d.p0, ldxz, 0);
-            conv_silu(s, d.act, d.p0, ldxz, C, l.conv, w.conv, w.conv_b, m.seqs, m.nseq, m.scan.p, m.scan.n,
+            conv_silu(s, d.act, d.p0, ldxz, C, l.conv, w.conv, w.conv_b, m.seqs, m.nseq, m.conv.p, m.conv.n,
                       at<float>(state, st[i].a), d.p1, ldc);
             const int sp = matmul_rt(s, d.act, d.p1, ldc, w.x.w, w.x.ldw, rows, R + 2 * N, w.x.k, RT_SLABS, nullptr, d.slabs,
                                      0, d.slab_bytes);
@@ -1026,7 +1026,29 @@ int pgmi_decoder_forward(pgmi_ctx* x, const int64_t* ids, int n_seq, const int32
         }
         return c;
     };
-    const Cut scan = cut(rows <= 16384 ? 64 : 256), gru = cut(rows <= 16384 ? 32 : 128);
+    // The recurrences take the longest runs that still give every CU a workgroup: a short step's few runs are otherwise walked
+    // by a few CUs, each row waiting for the one before.  us of the scan's three launches, 64- / 16-row runs: 500 rows of 2,048
+    // channels 86 / 41, 300 rows 69 / 35; where the chip is full short runs only add carries (1,540 rows of 4,096: 98 / 121).
+    auto run_rows = [&](int longest, int width, int per_wg) {  // width channels, per_wg of them per workgroup
+        const long cols = std::max(1, (width + per_wg - 1) / per_wg);
+        int ct = longest;
+        for (const int k : {4, 3, 2, 1}) {  // longest, 3/4, 1/2, 1/4 of it
+            ct = longest * k / 4;
+            long n = 0;
+            for (int r = 0; r < n_seq; ++r) n += (lens[r] + ct - 1) / ct;
+            if (n * cols >= 256) break;
+        }
+        return ct;
+    };
+    int scan_width = 1, gru_width = 1;
+    for (const pgmi_layer_spec& l : d.L) {
+        if (l.mixer == PGMI_MIXER_MAMBA1) scan_width = std::max(scan_width, l.inner);
+        if (l.mixer == PGMI_MIXER_MINGRU) gru_width = std::max(gru_width, l.width);
+    }
+    const bool huge = rows > 16384;
+    const Cut scan = cut(huge ? 256 : run_rows(64, scan_width, 256)), gru = cut(huge ? 128 : run_rows(32, gru_width, 128));
+    // the convolutions carry nothing: 500 rows of 2,048 channels 11.2 us on 64-row runs, 5.9 on 16; 2,048 rows 10.8 / 7.5
+    const Cut conv = cut(huge ? 256 : rows > 2048 ? 32 : 16);
     struct Tiles { int R; size_t o; int n; };
     std::vector<Tiles> tiles;
     for (const pgmi_layer_spec& l : d.L) {
@@ -1064,6 +1086,7 @@ int pgmi_decoder_forward(pgmi_ctx* x, const int64_t* ids, int n_seq, const int32
     meta.nseq = n_seq;
     meta.scan = {reinterpret_cast<const ChunkInfo*>(dm + scan.o), scan.n, scan.multi};
     meta.gru = {reinterpret_cast<const ChunkInfo*>(dm + gru.o), gru.n, gru.multi};
+    meta.conv = {reinterpret_cast<const ChunkInfo*>(dm + conv.o), conv.n, conv.multi};
     meta.row_seq = dm + o_row;
     meta.want = dm + o_want;
     for (const Tiles& t : tiles) meta.tiles[t.R] = {reinterpret_cast<const ChunkInfo*>(dm + t.o), t.n};
