@@ -7,14 +7,17 @@
 // position whose inclusive cumulative mass exceeds a target": target p gives the nucleus
 // cut-off k*, and target r = u * Z (Z = the kept mass, u ~ U[0,1) from the caller) gives the
 // draw, which lands at or before k* because r < Z.  Each is a mass-weighted radix select over
-// the fp32 bit patterns (probabilities are >= 0, so the bit order is the value order): four
-// 8-bit digit levels of 256-bin (count, mass) histograms, walking bins from the top until the
-// running mass crosses the target, then equal probabilities resolved in index order (our tie
-// rule; torch.sort does not define one).  No sort and no materialised cumsum; masses in fp64.
+// the fp32 bit patterns (probabilities are >= 0, so the bit order is the value order): the exponent
+// field by the row's histogram, then three digits of the mantissa over the tokens of that exponent,
+// walking bins from the top until the running mass crosses the target, then equal probabilities
+// resolved in index order (our tie rule; torch.sort does not define one).  No sort and no materialised
+// cumsum; masses in fp64.
 //
-// One 1024-thread workgroup per row; the row's probabilities live in a global scratch row
-// (fp32, L2-resident across the passes).  The draw is a function of u, so it is checkable
-// against the sort-based restatement in oracle/sampling_np.py.
+// Four launches, each a short dependent chain; what bounds a draw is their length and number, not the
+// vocabulary's megabyte.  257,216 logits of a peaked distribution: 42 us as five launches with four digits
+// per select, maxima by LDS atomics (a turn per lane) and a select for the token after the cut-off at every draw, now 20.
+#include <algorithm>
+
 #include "common.h"
 #include "launch.h"
 
@@ -27,33 +30,11 @@ constexpr int kSampleThreads = 1024;
 constexpr double kMassScale = 4611686018427387904.0;  // 2^62
 constexpr double kMassUnit = 1.0 / kMassScale;
 __device__ __forceinline__ unsigned long long mass_q(float v) { return (unsigned long long)((double)v * kMassScale); }
-constexpr int kSampleWaves = kSampleThreads / 64;
 
 __device__ __forceinline__ double wave_sum_d(double v) {
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
     return v;
-}
-
-// block reductions; every thread gets the result (fixed combine order over waves)
-__device__ __forceinline__ float block_max_f(float v, float* red) {
-    v = wave_max(v);
-    __syncthreads();
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
-    __syncthreads();
-    float m = red[0];
-    for (int i = 1; i < kSampleWaves; ++i) m = fmaxf(m, red[i]);
-    return m;
-}
-
-__device__ __forceinline__ double block_sum_d(double v, double* red) {
-    v = wave_sum_d(v);
-    __syncthreads();
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
-    __syncthreads();
-    double s = 0.0;
-    for (int i = 0; i < kSampleWaves; ++i) s += red[i];
-    return s;
 }
 
 struct SelectOut {
@@ -63,28 +44,28 @@ struct SelectOut {
     bool crossed;  // false: target >= the total mass (no crossing)
 };
 
+constexpr int kHeld = 2048;   // candidates that k_tp_select holds in LDS
+constexpr int kRanked = 256;  // and those it orders by comparing each with all
+constexpr int kDigit = 6;     // bits of the mantissa per level: a wave holds a level's bins
+constexpr int kLevels = 4;
 struct SampleSmem {
-    unsigned hcnt[256];
-    unsigned long long hmq[256];
-    double red_d[kSampleWaves];
-    float red_f[kSampleWaves];
-    int sel;
-    double acc;
-    int found;
-    int scan[kSampleThreads];
-    double suf[256 + 4];
+    float val[kHeld];
+    unsigned hcnt[kLevels][64];
+    unsigned long long hmq[kLevels][64];
+    double row_suf[256 + 4];  // the row's suffix masses by exponent
+    int top[4];               // per wave
+    double above;
+    int scan[kSampleThreads / 64];
+    int found, rank;
+    uint32_t key;
 };
 
-// The first bin, walking from the top (bin 255) down, at which `above + (mass of that bin and
-// every bin above it)` exceeds target: a suffix scan over the 256 bins (one per thread of the
-// first 256), then the LARGEST bin whose suffix crosses (suffix sums are monotone up to
-// rounding; taking the largest keeps the answer unique).  Returns the bin (-1: none) and sets
-// *above_out to the mass above the bin.  Every thread of the block must call it.
-__device__ int crossing_bin(const unsigned* cnt, const unsigned long long* mq, double above, double target,
-                            double* suf, int* sh_int, double* sh_d, double* above_out) {
+// suf[t] = mass of bins t .. 255 (mq in fixed point), t < 256: the wave's 64 bins by shuffles, then the higher waves'
+// totals in a fixed order.  Every thread of the block must call it (suf: 260 doubles).
+__device__ __forceinline__ void suffix_masses(const unsigned long long* mq, double* suf) {
     const int t = threadIdx.x, lane = t & 63, w = t >> 6;
     double v = 0.0;
-    if (t < 256) {  // suffix within the wave's 64 bins (bin 64w + lane), by shuffles
+    if (t < 256) {
         v = (double)mq[t] * kMassUnit;
 #pragma unroll
         for (int o = 1; o < 64; o <<= 1) {
@@ -93,19 +74,23 @@ __device__ int crossing_bin(const unsigned* cnt, const unsigned long long* mq, d
         }
         if (lane == 0) suf[256 + w] = v;  // the wave's total
     }
-    if (t == 0) sh_int[0] = -1;
     __syncthreads();
     if (t < 256) {
-        for (int q = w + 1; q < 4; ++q) v += suf[256 + q];  // higher waves' bins, fixed order
+        for (int q = w + 1; q < 4; ++q) v += suf[256 + q];
         suf[t] = v;
-        if (cnt[t] != 0u && above + v > target) atomicMax(sh_int, t);
     }
     __syncthreads();
-    const int d = sh_int[0];
-    if (t == 0) sh_d[0] = d >= 0 ? above + (suf[d] - (double)mq[d] * kMassUnit) : above + suf[0];
+}
+
+// The largest t < 256 of the block's first four waves for which `is` holds, -1 if none: by ballots (a maximum by LDS atomics
+// costs a turn for every lane that takes part).  Two barriers; every thread of the block calls it.
+__device__ __forceinline__ int highest(bool is, int* top) {
+    const unsigned long long m = __ballot(is);
+    const int w = threadIdx.x >> 6;
     __syncthreads();
-    *above_out = sh_d[0];
-    return d;
+    if (w < 4 && (threadIdx.x & 63) == 0) top[w] = m ? 64 * w + 63 - __clzll((long long)m) : -1;
+    __syncthreads();
+    return max(max(top[0], top[1]), max(top[2], top[3]));
 }
 
 __device__ __forceinline__ void hist_add(unsigned* hcnt, unsigned long long* hmq, bool valid, int d, float v) {
@@ -115,31 +100,46 @@ __device__ __forceinline__ void hist_add(unsigned* hcnt, unsigned long long* hmq
     }
 }
 
-// the first position of the descending order whose inclusive cumulative mass exceeds target
-__device__ SelectOut radix_select(const float* __restrict__ p, int V, double target, double above0, SampleSmem& sm) {
-    const int tid = threadIdx.x;
-    uint32_t prefix = 0, pmask = 0;
-    double above = above0;
-    for (int level = 3; level >= 0; --level) {
-        const int shift = level * 8;
-        for (int i = tid; i < 256; i += kSampleThreads) {
-            sm.hcnt[i] = 0u;
-            sm.hmq[i] = 0ull;
-        }
-        __syncthreads();
-        for (int i0 = 0; i0 < V; i0 += kSampleThreads) {  // wave-uniform trip count
-            const int i = i0 + tid;
-            const float v = i < V ? p[i] : 0.f;
+// The first position of the descending order whose inclusive cumulative mass exceeds target, found digit by digit of the
+// mantissa among the candidates of its exponent.  value(i): candidate i of n; used: the row has tokens of exponent threadIdx.x.
+template <typename Value>
+__device__ __forceinline__ SelectOut radix_select(const Value& value, int n, int NT, double target, bool used, SampleSmem& sm) {
+    const int t = threadIdx.x, lane = t & 63;
+    __syncthreads();  // the previous select's readers are done
+    for (int i = t; i < kLevels * 64; i += NT) {  // (behind highest()'s barriers for its users)
+        (&sm.hcnt[0][0])[i] = 0u;
+        (&sm.hmq[0][0])[i] = 0ull;
+    }
+    const int bin = highest(t < 256 && used && sm.row_suf[t & 255] > target, sm.top);
+    if (bin < 0) return SelectOut{0u, sm.row_suf[0], 0, false};
+    uint32_t prefix = (uint32_t)bin << 23, pmask = 0xFF800000u;
+    double above = bin < 255 ? sm.row_suf[bin + 1] : 0.0;
+#pragma unroll 1
+    for (int level = 0; level < kLevels; ++level) {
+        const int shift = max(0, 23 - kDigit * (level + 1)), bits = level + 1 < kLevels ? kDigit : 23 - kDigit * (kLevels - 1);
+        const uint32_t digit = (1u << bits) - 1u;
+#pragma unroll 1
+        for (int i = t; i < n; i += NT) {
+            const float v = value(i);
             const uint32_t k = __float_as_uint(v);
-            hist_add(sm.hcnt, sm.hmq, i < V && (k & pmask) == prefix, (int)((k >> shift) & 255), v);
+            hist_add(sm.hcnt[level], sm.hmq[level], (k & pmask) == prefix, (int)((k >> shift) & digit), v);
         }
         __syncthreads();
-        double a;
-        const int sel = crossing_bin(sm.hcnt, sm.hmq, above, target, sm.suf, &sm.sel, &sm.acc, &a);
-        above = a;
-        if (sel < 0) return SelectOut{0u, above, 0, false};
-        prefix |= (uint32_t)sel << shift;
-        pmask |= 255u << shift;
+        // every wave: mass of bins lane .. 63, then the LARGEST bin whose suffix mass crosses (sums are monotone up to
+        // rounding; taking the largest keeps the answer unique)
+        const unsigned long long own = sm.hmq[level][lane];
+        unsigned long long suf = own;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const unsigned long long x = __shfl_down(suf, o, 64);
+            if (lane + o < 64) suf += x;
+        }
+        const unsigned long long m = __ballot(sm.hcnt[level][lane] != 0u && above + (double)suf * kMassUnit > target);
+        if (!m) return SelectOut{0u, above, 0, false};
+        const int d = 63 - __clzll((long long)m);
+        above += (double)(unsigned long long)__shfl(suf - own, d, 64) * kMassUnit;
+        prefix |= (uint32_t)d << shift;
+        pmask |= digit << shift;
     }
     // tokens equal to the key: the crossing is at the smallest tie rank j with
     // above + (j + 1) * value > target
@@ -154,15 +154,15 @@ __device__ SelectOut radix_select(const float* __restrict__ p, int V, double tar
     return SelectOut{prefix, above, rank, true};
 }
 
-// index of the rank-th token (index order) whose bit pattern equals key; -1 if fewer exist
-__device__ int nth_equal(const float* __restrict__ p, int V, uint32_t key, int rank, SampleSmem& sm) {
-    const int tid = threadIdx.x;
-    const int per = (V + kSampleThreads - 1) / kSampleThreads;  // contiguous slice per thread
-    const int i0 = tid * per, i1 = min(V, i0 + per);
+// place of the rank-th candidate (index order) whose bit pattern equals key; -1 if fewer exist
+template <typename Value>
+__device__ __forceinline__ int nth_equal(const Value& value, int n, int NT, uint32_t key, int rank, SampleSmem& sm) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int per = (n + NT - 1) / NT, i0 = min((int)threadIdx.x * per, n), i1 = min(i0 + per, n);  // contiguous slice per thread
     int c = 0;
-    for (int i = i0; i < i1; ++i) c += (__float_as_uint(p[i]) == key);
+#pragma unroll 1
+    for (int i = i0; i < i1; ++i) c += (__float_as_uint(value(i)) == key);
     // exclusive prefix of the threads' counts: within the wave by shuffles, then wave totals
-    const int lane = tid & 63, wave = tid >> 6;
     int incl = c;
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) {
@@ -171,21 +171,14 @@ __device__ int nth_equal(const float* __restrict__ p, int V, uint32_t key, int r
     }
     __syncthreads();
     if (lane == 63) sm.scan[wave] = incl;
-    if (tid == 0) sm.found = -1;
+    if (threadIdx.x == 0) sm.found = -1;
     __syncthreads();
-    int wbase = 0;
-    for (int w = 0; w < wave; ++w) wbase += sm.scan[w];
-    const int base = wbase + incl - c;
-    if (rank >= base && rank < base + c) {
-        int r = rank - base;
+    int at = incl - c;
+    for (int w = 0; w < wave; ++w) at += sm.scan[w];
+    if (rank >= at && rank < at + c) {
+#pragma unroll 1
         for (int i = i0; i < i1; ++i)
-            if (__float_as_uint(p[i]) == key) {
-                if (r == 0) {
-                    sm.found = i;
-                    break;
-                }
-                --r;
-            }
+            if (__float_as_uint(value(i)) == key && at++ == rank) sm.found = i;
     }
     __syncthreads();
     return sm.found;
@@ -193,22 +186,24 @@ __device__ int nth_equal(const float* __restrict__ p, int V, uint32_t key, int r
 
 // ---------------------------------------------------------------- the multi-kernel pipeline
 // Per row: (1) k_tp_stats, NB blocks: max and sum of exp of z = x / T per slice;
-// (2) k_tp_hist, NB blocks: p = softmax, written once, and per-block histograms of the fp32
-// exponent field (256 bins of count and fp64 mass, no global atomics: block order is the sum
-// order); (3) k_tp_plan, one block: the cut-off bin c1 (where the running mass crosses p) and
-// the highest bin c_hi the draw can reach (r = u Z >= u * mass above c1), so every position the
-// two decisions can land on lies in bins [c1, c_hi], with A_out the mass above c_hi;
-// (4) k_tp_compact, NB blocks: the tokens of bins [c1, c_hi] -> (value, index) in index order;
-// (5) k_tp_select, one block: the two radix selects of the header over the candidates only.
+// (2) k_tp_hist, NB blocks: p = softmax, written once, per-block counts and the row's histogram of the fp32
+// exponent field (256 bins of count and fixed-point mass);
+// (3) k_tp_compact, NB blocks: from that histogram, each for itself, the cut-off bin c1 (where the running mass
+// crosses p) and the highest bin c_hi the draw can reach (r = u Z >= u * mass above c1), so every position the
+// two decisions can land on lies in bins [c1, c_hi]; then the tokens of these bins -> (value, index) in index
+// order;
+// (4) k_tp_select, one block: the two radix selects of the header over the candidates only.
 constexpr int kTpThreads = 256;
+constexpr int kShards = 8;  // copies of the row's histogram: blocks adding to one address wait for each other
+constexpr int kTpHeld = 2048;  // tokens of a slice (tp_blocks) that a block holds in registers
 
 struct TpLayout {
-    size_t p, cv, ci, bm, bs, hc, rc, hm, pre, meta, stride;  // byte offsets within one row's scratch
+    size_t p, cv, ci, bm, bs, hc, hm, meta, stride;  // byte offsets within one row's scratch
 };
 
-__host__ __device__ inline size_t tp_align(size_t x) { return (x + 255) & ~(size_t)255; }
+inline size_t tp_align(size_t x) { return (x + 255) & ~(size_t)255; }
 
-__host__ __device__ inline TpLayout tp_layout(int V, int NB) {
+inline TpLayout tp_layout(int V, int NB) {
     TpLayout L;
     size_t o = 0;
     L.p = o; o = tp_align(o + (size_t)V * 4);
@@ -216,21 +211,20 @@ __host__ __device__ inline TpLayout tp_layout(int V, int NB) {
     L.ci = o; o = tp_align(o + (size_t)V * 4);
     L.bm = o; o = tp_align(o + (size_t)NB * 4);
     L.bs = o; o = tp_align(o + (size_t)NB * 8);
-    L.hc = o; o = tp_align(o + (size_t)NB * 256 * 4);
-    L.rc = o; o = tp_align(o + (size_t)256 * 4);
-    L.hm = o; o = tp_align(o + (size_t)256 * 8);
-    L.pre = o; o = tp_align(o + (size_t)NB * 4);
+    L.hc = o; o = tp_align(o + (size_t)NB * 256 * 2);
+    L.hm = o; o = tp_align(o + (size_t)kShards * 256 * 8);
     L.meta = o; o = tp_align(o + 16 * 8);
-    L.stride = o;
+    // (no less than 1 KiB and 8 bytes per block: the workspace holds the same vocabularies whatever the histograms' layout)
+    L.stride = std::max(o, L.hc + tp_align((size_t)NB * 1024) + 1024 + 2048 + tp_align((size_t)NB * 4) + 256);
     return L;
 }
 
-struct TpMeta {  // one row's plan (k_tp_plan -> k_tp_compact, k_tp_select)
-    double a_out;   // mass of the bins above c_hi
-    double total;   // mass of the row
-    int c1, c_hi;   // candidate bins [c1, c_hi]
+struct TpMeta {  // one row's plan (k_tp_compact -> k_tp_select)
+    double a1;     // mass of the bins above c1
+    double total;  // mass of the row
+    int c1, c_hi;  // candidate bins [c1, c_hi]
     int n_cand;
-    int crossed;    // the cut-off exists (p < total mass)
+    int crossed;   // the cut-off exists (p < total mass)
 };
 
 __device__ __forceinline__ int tp_bin(float v) { return (int)((__float_as_uint(v) >> 23) & 255u); }
@@ -250,16 +244,29 @@ __global__ void __launch_bounds__(kTpThreads) k_tp_stats(const float* __restrict
     uint8_t* base = scratch + (size_t)row * L.stride;
     int i0, i1;
     tp_slice(V, NB, b, i0, i1);
+    // the slice's first kTpHeld tokens stay in registers between the two passes
+    float z[kTpHeld / kTpThreads];
+#pragma unroll
+    for (int k = 0; k < kTpHeld / kTpThreads; ++k) {
+        const int i = i0 + tid + k * kTpThreads;
+        z[k] = xr[i < i1 ? i : i1 - 1] / temperature;
+    }
     float m = -INFINITY;
-    for (int i = i0 + tid; i < i1; i += kTpThreads) m = fmaxf(m, xr[i] / temperature);
+#pragma unroll
+    for (int k = 0; k < kTpHeld / kTpThreads; ++k) m = fmaxf(m, z[k]);
+    for (int i = i0 + tid + kTpHeld; i < i1; i += kTpThreads) m = fmaxf(m, xr[i] / temperature);
     m = wave_max(m);
     if ((tid & 63) == 0) red_f[tid >> 6] = m;
     __syncthreads();
     m = red_f[0];
     for (int w = 1; w < kTpThreads / 64; ++w) m = fmaxf(m, red_f[w]);
     double sum = 0.0;
-    if (m != -INFINITY)
-        for (int i = i0 + tid; i < i1; i += kTpThreads) sum += (double)expf(xr[i] / temperature - m);
+    if (m != -INFINITY) {
+#pragma unroll
+        for (int k = 0; k < kTpHeld / kTpThreads; ++k)
+            if (i0 + tid + k * kTpThreads < i1) sum += (double)expf(z[k] - m);
+        for (int i = i0 + tid + kTpHeld; i < i1; i += kTpThreads) sum += (double)expf(xr[i] / temperature - m);
+    }
     sum = wave_sum_d(sum);
     if ((tid & 63) == 0) red_d[tid >> 6] = sum;
     __syncthreads();
@@ -270,15 +277,13 @@ __global__ void __launch_bounds__(kTpThreads) k_tp_stats(const float* __restrict
         reinterpret_cast<double*>(base + L.bs)[b] = t;
     }
     if (b == 0) {  // the row histogram k_tp_hist accumulates into
-        reinterpret_cast<unsigned*>(base + L.rc)[tid] = 0u;
-        reinterpret_cast<unsigned long long*>(base + L.hm)[tid] = 0ull;
+        for (int q = 0; q < kShards; ++q) reinterpret_cast<unsigned long long*>(base + L.hm)[q * 256 + tid] = 0ull;
     }
 }
 
 __global__ void __launch_bounds__(kTpThreads) k_tp_zero(uint8_t* __restrict__ scratch, TpLayout L) {
     uint8_t* base = scratch + (size_t)blockIdx.x * L.stride;
-    reinterpret_cast<unsigned*>(base + L.rc)[threadIdx.x] = 0u;
-    reinterpret_cast<unsigned long long*>(base + L.hm)[threadIdx.x] = 0ull;
+    for (int q = 0; q < kShards; ++q) reinterpret_cast<unsigned long long*>(base + L.hm)[q * 256 + threadIdx.x] = 0ull;
 }
 
 __global__ void __launch_bounds__(kTpThreads) k_tp_hist(const float* __restrict__ x, int V, float temperature, int NB,
@@ -293,6 +298,14 @@ __global__ void __launch_bounds__(kTpThreads) k_tp_hist(const float* __restrict_
     hmq[tid] = 0ull;
     __shared__ float red_f[kTpThreads / 64];
     __shared__ double red_d[kTpThreads / 64];
+    int i0, i1;
+    tp_slice(V, NB, b, i0, i1);
+    float z[kTpHeld / kTpThreads];  // asked for before the slices' statistics are joined
+#pragma unroll
+    for (int k = 0; k < kTpHeld / kTpThreads; ++k) {
+        const int i = i0 + tid + k * kTpThreads;
+        z[k] = xr[i < i1 ? i : i1 - 1];
+    }
     float m = 0.f, sumf = 1.f;
     if (temperature > 0.f) {  // softmax(x / T): global max, then the slices' sums of exp rescaled to it
         const float* bm = reinterpret_cast<const float*>(base + L.bm);
@@ -315,145 +328,205 @@ __global__ void __launch_bounds__(kTpThreads) k_tp_hist(const float* __restrict_
         sumf = (float)S;
     }
     __syncthreads();
-    int i0, i1;
-    tp_slice(V, NB, b, i0, i1);
-    for (int c0 = i0; c0 < i1; c0 += kTpThreads) {  // block-uniform trip count
-        const int i = c0 + tid;
+    auto token = [&](int i, float x0) {
         float v = 0.f;
         if (i < i1) {
-            v = temperature > 0.f ? expf(xr[i] / temperature - m) / sumf : xr[i];
+            v = temperature > 0.f ? expf(x0 / temperature - m) / sumf : x0;
             if (!(v > 0.f)) v = 0.f;  // negative / NaN probabilities carry no mass
             p[i] = v;
         }
         hist_add(hcnt, hmq, i < i1, tp_bin(v), v);
-    }
+    };
+    // (one body, its tokens through LDS: unrolled it is 6 KiB of code that every CU fetches)
+    __shared__ float held[kTpHeld];
+#pragma unroll
+    for (int k = 0; k < kTpHeld / kTpThreads; ++k) held[tid + k * kTpThreads] = z[k];
+#pragma unroll 1
+    for (int i = i0 + tid; i < i1; i += kTpThreads) token(i, i - i0 < kTpHeld ? held[i - i0] : xr[i]);
     __syncthreads();
-    reinterpret_cast<unsigned*>(base + L.hc)[b * 256 + tid] = hcnt[tid];  // per-block counts (compaction offsets)
-    if (hcnt[tid]) {  // the row histogram: integer atomics, so the sums do not depend on arrival order
-        atomicAdd(reinterpret_cast<unsigned*>(base + L.rc) + tid, hcnt[tid]);
-        atomicAdd(reinterpret_cast<unsigned long long*>(base + L.hm) + tid, hmq[tid]);
-    }
-}
-
-__global__ void __launch_bounds__(256) k_tp_plan(int NB, float top_p, const float* __restrict__ u,
-                                                 uint8_t* __restrict__ scratch, TpLayout L) {
-    __shared__ unsigned cnt[256];
-    __shared__ unsigned long long mq[256];
-    __shared__ int range[2];
-    const int row = blockIdx.x, t = threadIdx.x;
-    uint8_t* base = scratch + (size_t)row * L.stride;
-    const unsigned* hc = reinterpret_cast<const unsigned*>(base + L.hc);
-    cnt[t] = reinterpret_cast<const unsigned*>(base + L.rc)[t];
-    mq[t] = reinterpret_cast<const unsigned long long*>(base + L.hm)[t];
-    __syncthreads();
-    __shared__ double suf[256 + 4];
-    __shared__ int sh_int[1];
-    __shared__ double sh_d[1];
-    double total = 0.0, a1 = 0.0;
-    const double tp = (double)top_p;
-    // lowest non-empty bin and the total mass
-    if (t == 0) sh_int[0] = 256;
-    __syncthreads();
-    if (cnt[t]) atomicMin(sh_int, t);
-    __syncthreads();
-    const int lowest = sh_int[0] < 256 ? sh_int[0] : 0;
-    __syncthreads();
-    int c1 = crossing_bin(cnt, mq, 0.0, tp, suf, sh_int, sh_d, &a1);
-    total = suf[0];
-    __syncthreads();  // suf is rewritten by the next crossing_bin
-    const bool crossed = c1 >= 0;
-    if (!crossed) {  // everything is kept
-        c1 = lowest;
-        a1 = total - (double)mq[lowest] * kMassUnit;
-    }
-    double uu = (double)u[row];
-    if (!(uu >= 0.0)) uu = 0.0;
-    if (uu >= 1.0) uu = 1.0 - 1.0 / 16777216.0;
-    double a_out = 0.0;
-    int chi = crossing_bin(cnt, mq, 0.0, uu * a1, suf, sh_int, sh_d, &a_out);  // r = u Z >= u * a1
-    if (chi < c1) {
-        chi = c1;
-        a_out = a1;
-    }
-    if (t == 0) {
-        range[0] = c1;
-        range[1] = chi;
-        TpMeta M{};
-        M.a_out = a_out;
-        M.total = total;
-        M.c1 = c1;
-        M.c_hi = chi;
-        M.crossed = crossed;
-        *reinterpret_cast<TpMeta*>(base + L.meta) = M;
-    }
-    __syncthreads();
-    // candidate prefix per block (block order = index order)
-    __shared__ unsigned bc[256];
-    for (int q = t; q < NB; q += 256) {
-        unsigned k = 0u;
-        for (int d = range[0]; d <= range[1]; ++d) k += hc[q * 256 + d];
-        bc[q] = k;
-    }
-    __syncthreads();
-    if (t == 0) {
-        unsigned* pre = reinterpret_cast<unsigned*>(base + L.pre);
-        unsigned run = 0u;
-        for (int q = 0; q < NB; ++q) {
-            pre[q] = run;
-            run += bc[q];
+    {  // per-block counts of bins tid and higher (compaction offsets: two reads give any range of bins)
+        __shared__ unsigned wsum[kTpThreads / 64];
+        const int lane = tid & 63, wave = tid >> 6;
+        unsigned n = hcnt[tid];
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const unsigned x = __shfl_down(n, o, 64);
+            if (lane + o < 64) n += x;
         }
-        reinterpret_cast<TpMeta*>(base + L.meta)->n_cand = (int)run;
+        if (lane == 0) wsum[wave] = n;
+        __syncthreads();
+        for (int w = wave + 1; w < kTpThreads / 64; ++w) n += wsum[w];
+        reinterpret_cast<uint16_t*>(base + L.hc)[b * 256 + tid] = (uint16_t)n;
     }
+    if (hmq[tid])  // the row histogram: integer atomics, so the sums do not depend on arrival order
+        atomicAdd(reinterpret_cast<unsigned long long*>(base + L.hm) + b % kShards * 256 + tid, hmq[tid]);
 }
 
-__global__ void __launch_bounds__(kTpThreads) k_tp_compact(int V, int NB, uint8_t* __restrict__ scratch, TpLayout L) {
-    __shared__ unsigned wtot[kTpThreads / 64];
+// bin t of the row's histogram
+__device__ __forceinline__ unsigned long long tp_mass(const uint8_t* base, const TpLayout& L, int t) {
+    unsigned long long m = 0ull;
+#pragma unroll
+    for (int q = 0; q < kShards; ++q) m += reinterpret_cast<const unsigned long long*>(base + L.hm)[q * 256 + t];
+    return m;
+}
+
+__device__ __forceinline__ double tp_uniform(float u) {  // in [0, 1)
+    const double uu = (double)u;
+    if (!(uu >= 0.0)) return 0.0;
+    return uu >= 1.0 ? 1.0 - 1.0 / 16777216.0 : uu;
+}
+
+__global__ void __launch_bounds__(kTpThreads) k_tp_compact(int V, int NB, float top_p, const float* __restrict__ u,
+                                                            uint8_t* __restrict__ scratch, TpLayout L) {
+    __shared__ unsigned long long mq[256];
+    __shared__ double suf[256 + 4];
+    __shared__ int top[4];
+    __shared__ unsigned wtot[kTpThreads / 64][2];
     const int b = blockIdx.x, row = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     uint8_t* base = scratch + (size_t)row * L.stride;
     const float* p = reinterpret_cast<const float*>(base + L.p);
     float* cv = reinterpret_cast<float*>(base + L.cv);
     int* ci = reinterpret_cast<int*>(base + L.ci);
-    const TpMeta M = *reinterpret_cast<const TpMeta*>(base + L.meta);
-    unsigned off = reinterpret_cast<const unsigned*>(base + L.pre)[b];
     int i0, i1;
     tp_slice(V, NB, b, i0, i1);
-    for (int c0 = i0; c0 < i1; c0 += kTpThreads) {  // ordered compaction, 256 tokens per round
-        const int i = c0 + tid;
-        float v = 0.f;
-        bool f = false;
-        if (i < i1) {
-            v = p[i];
-            const int d = tp_bin(v);
-            f = d >= M.c1 && d <= M.c_hi;
+    constexpr int PT = kTpHeld / kTpThreads;  // consecutive tokens of a thread
+    float v[PT];
+    auto load = [&](int c0) {
+#pragma unroll
+        for (int k = 0; k < PT; ++k) {
+            const int i = c0 + tid * PT + k;
+            v[k] = p[i < i1 ? i : i1 - 1];
         }
-        const unsigned long long bal = __ballot(f);
-        const unsigned below = (unsigned)__popcll(bal & ((1ull << lane) - 1ull));
+    };
+    if (i0 < i1) load(i0);  // in flight during the plan
+    mq[tid] = tp_mass(base, L, tid);
+    const bool used = mq[tid] != 0ull;
+    const double uu = tp_uniform(u[row]);
+    __syncthreads();
+    suffix_masses(mq, suf);
+    const int cross = highest(used && suf[tid] > (double)top_p, top);
+    const bool crossed = cross >= 0;
+    int c1 = cross;
+    if (!crossed) {  // everything is kept: from the lowest bin in use
+        const int low = highest(mq[255 - tid] != 0ull, top);
+        c1 = low < 0 ? 0 : 255 - low;
+    }
+    const double a1 = (crossed ? suf[c1] : suf[0]) - (double)mq[c1] * kMassUnit;
+    const int c_hi = max(highest(used && suf[tid] > uu * a1, top), c1);  // r = u Z >= u * a1
+    // this block's place among the candidates (block order = index order), and how many there are
+    const uint16_t* hc = reinterpret_cast<const uint16_t*>(base + L.hc);
+    unsigned before = 0u, all = 0u;
+    for (int q = tid; q < NB; q += kTpThreads) {
+        const unsigned k = hc[q * 256 + c1] - (c_hi < 255 ? hc[q * 256 + c_hi + 1] : 0u);
+        all += k;
+        if (q < b) before += k;
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+        before += __shfl_xor(before, o, 64);
+        all += __shfl_xor(all, o, 64);
+    }
+    if (lane == 0) { wtot[wave][0] = before; wtot[wave][1] = all; }
+    __syncthreads();
+    unsigned off = 0u;
+    all = 0u;
+    for (int w = 0; w < kTpThreads / 64; ++w) {
+        off += wtot[w][0];
+        all += wtot[w][1];
+    }
+    if (b == 0 && tid == 0)
+        *reinterpret_cast<TpMeta*>(base + L.meta) = TpMeta{a1, suf[0], c1, c_hi, (int)all, (int)crossed};
+    for (int c0 = i0; c0 < i1; c0 += kTpHeld) {  // ordered compaction
+        if (c0 > i0) load(c0);
+        unsigned mask = 0u;
+#pragma unroll
+        for (int k = 0; k < PT; ++k) {
+            const int d = tp_bin(v[k]);
+            if (c0 + tid * PT + k < i1 && d >= c1 && d <= c_hi) mask |= 1u << k;
+        }
+        const unsigned n = (unsigned)__popc(mask);
+        unsigned incl = n;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const unsigned x = __shfl_up(incl, o, 64);
+            if (lane >= o) incl += x;
+        }
         __syncthreads();
-        if (lane == 0) wtot[wave] = (unsigned)__popcll(bal);
+        if (lane == 63) wtot[wave][0] = incl;
         __syncthreads();
-        unsigned wo = 0u, all = 0u;
+        unsigned to = off + incl - n;
         for (int w = 0; w < kTpThreads / 64; ++w) {
-            if (w < wave) wo += wtot[w];
-            all += wtot[w];
+            if (w < wave) to += wtot[w][0];
+            off += wtot[w][0];
         }
-        if (f) {
-            cv[off + wo + below] = v;
-            ci[off + wo + below] = i;
-        }
-        off += all;
+#pragma unroll
+        for (int k = 0; k < PT; ++k)
+            if (mask >> k & 1u) {
+                cv[to] = v[k];
+                ci[to++] = c0 + tid * PT + k;
+            }
     }
 }
 
-__global__ void __launch_bounds__(kSampleThreads) k_tp_select(float top_p, const float* __restrict__ u,
+// One select at a time through one loop, its digits through another: a launch starts with an empty instruction cache, and a
+// single workgroup waits for every line of straight code.  Few candidates (the peaked rows) are ordered by comparing each
+// with all, once for both decisions: 5 of them 12.5 us by digits.
+__global__ void __launch_bounds__(kSampleThreads) k_tp_select(int V, float top_p, const float* __restrict__ u,
                                                                uint8_t* __restrict__ scratch, TpLayout L,
                                                                int64_t* __restrict__ out, float* __restrict__ kept_mass) {
     __shared__ SampleSmem sm;
+    __shared__ unsigned long long row_mq[256];
     const int row = blockIdx.x, tid = threadIdx.x;
     uint8_t* base = scratch + (size_t)row * L.stride;
     const float* cv = reinterpret_cast<const float*>(base + L.cv);
     const int* ci = reinterpret_cast<const int*>(base + L.ci);
     const TpMeta M = *reinterpret_cast<const TpMeta*>(base + L.meta);
-    const int n = M.n_cand;
+    const double uu = tp_uniform(u[row]);
+    // the first candidates, before their number is known (cv has V places)
+    const float v0 = cv[min(tid, V - 1)], v1 = cv[min(tid + kSampleThreads, V - 1)];
+    if (tid < 256) row_mq[tid] = tp_mass(base, L, tid);
+    const bool used = tid < 256 && row_mq[tid & 255] != 0ull;
+    static_assert(kHeld == 2 * kSampleThreads, "two held candidates per thread");
+    sm.val[tid] = v0;
+    sm.val[tid + kSampleThreads] = v1;
+    __syncthreads();
+    suffix_masses(row_mq, sm.row_suf);
+    const int n = M.n_cand, NT = n <= kHeld ? 256 : kSampleThreads;
+    if (tid >= NT) return;  // whole waves: the barriers below count those that are left
+    auto value = [&](int i) { return i < kHeld ? sm.val[i] : cv[i]; };
+
+    // ranked: this thread's candidate, the mass of the larger ones, and how many equal ones come before it
+    const bool ranked = n <= kRanked;
+    double larger = 0.0;
+    int ties = 0;
+    if (ranked && tid < n) {
+        unsigned long long q = 0ull;
+#pragma unroll 1
+        for (int j = 0; j < n; ++j) {
+            const float w = sm.val[j];
+            q += w > v0 ? mass_q(w) : 0ull;
+            ties += w == v0 && j < tid;
+        }
+        larger = (M.c_hi < 255 ? sm.row_suf[M.c_hi + 1] : 0.0) + (double)q * kMassUnit;
+    }
+    // first position whose inclusive cumulative mass exceeds target
+    auto select = [&](double target) -> SelectOut {
+        if (!ranked) return radix_select(value, n, NT, target, used, sm);
+        // (one candidate at most: its predecessor's inclusive mass does not exceed it)
+        const bool here = tid < n && larger + (double)(ties + 1) * (double)v0 > target &&
+                          !(larger + (double)ties * (double)v0 > target) && v0 > 0.f;
+        __syncthreads();
+        if (tid == 0) sm.found = 0;
+        __syncthreads();
+        if (here) {
+            sm.key = __float_as_uint(v0);
+            sm.above = larger;
+            sm.rank = ties;
+            sm.found = 1;
+        }
+        __syncthreads();
+        return sm.found ? SelectOut{sm.key, sm.above, sm.rank, true} : SelectOut{0u, 0.0, 0, false};
+    };
 
     // nucleus cut-off.  In exact arithmetic the kept prefix ends at k, the first position whose
     // cumulative mass C exceeds p.  The reference decides in fp32 -- C is torch's CPU cumsum
@@ -461,37 +534,51 @@ __global__ void __launch_bounds__(kSampleThreads) k_tp_select(float top_p, const
     // (:18-19) -- which can drop k or keep positions after it when C lands within an fp32 ulp
     // of p; those boundary positions are re-decided by that formula.
     auto ref_dropped = [&](double C, float v) { return __fsub_rn((float)C, v) > top_p; };
-    double Z = M.total;
-    SelectOut cut{0u, 0.0, 0, false};
-    if (M.crossed) {
-        cut = radix_select(cv, n, (double)top_p, M.a_out, sm);
-        if (cut.crossed) {
-            const float vk = __uint_as_float(cut.key);
-            const double Ck = cut.above + (double)(cut.rank + 1) * (double)vk;
-            if (ref_dropped(Ck, vk)) {
-                Z = Ck - (double)vk;
-            } else {
-                Z = Ck;
-                for (int extra = 0; extra < 4; ++extra) {  // positions after k that fp32 still keeps
-                    const SelectOut nx = radix_select(cv, n, Z, M.a_out, sm);
-                    if (!nx.crossed) break;
-                    const float vn = __uint_as_float(nx.key);
-                    const double Cn = nx.above + (double)(nx.rank + 1) * (double)vn;
-                    if (ref_dropped(Cn, vn)) break;
-                    Z = Cn;
-                }
+    double Z = M.total, Ck = 0.0;
+    SelectOut cut{0u, 0.0, 0, false}, got{0u, 0.0, 0, false};
+    enum { CUT, MORE, DRAW };
+    int extra = 0;
+#pragma unroll 1
+    for (int what = M.crossed ? CUT : DRAW;;) {
+        // DRAW: first position whose inclusive mass exceeds r = u * Z (r < Z, so it is <= k*)
+        got = select(what == CUT ? (double)top_p : what == MORE ? Z : uu * Z);
+        if (what == DRAW) break;
+        const int was = what;
+        what = DRAW;
+        if (got.crossed) {
+            const float v = __uint_as_float(got.key);
+            const double C = got.above + (double)(got.rank + 1) * (double)v;
+            const bool dropped = ref_dropped(C, v);
+            if (was == CUT) {
+                cut = got;
+                Ck = C;
+                Z = dropped ? Ck - (double)v : Ck;
+                // positions after k that fp32 still keeps.  The one after k has fp32(fp32(C) - v) within 2^-23 C of C_k:
+                // when C_k is further than that past p it is dropped, and so is every later one
+                if (!dropped && !(Ck - (double)top_p > 1e-6 * fmax(1.0, M.total))) what = MORE;
+            } else if (!dropped) {
+                Z = C;
+                if (++extra < 4) what = MORE;
             }
-            if (!(Z > 0.0)) Z = Ck;  // a first token alone beyond p is always kept (:19, C_0 - p_0 = 0)
         }
+        if (what == DRAW && cut.crossed && !(Z > 0.0)) Z = Ck;  // a first token alone beyond p is always kept (:19, C_0 - p_0 = 0)
     }
-    // the draw: first position whose inclusive mass exceeds r = u * Z (r < Z, so it is <= k*)
-    double uu = (double)u[row];
-    if (!(uu >= 0.0)) uu = 0.0;
-    if (uu >= 1.0) uu = 1.0 - 1.0 / 16777216.0;
-    const SelectOut pick = radix_select(cv, n, uu * Z, M.a_out, sm);
     int pos = -1;
-    if (pick.crossed) pos = nth_equal(cv, n, pick.key, pick.rank, sm);
-    if (pos < 0 && cut.crossed) pos = nth_equal(cv, n, cut.key, cut.rank, sm);  // rounding at the very end
+#pragma unroll 1
+    for (int k = got.crossed ? 0 : 1; k < 2 && pos < 0; ++k) {  // the cut-off's token: rounding at the very end
+        const SelectOut& q = k == 0 ? got : cut;
+        if (!q.crossed) continue;
+        if (!ranked) {
+            pos = nth_equal(value, n, NT, q.key, q.rank, sm);
+            continue;
+        }
+        __syncthreads();
+        if (tid == 0) sm.found = -1;
+        __syncthreads();
+        if (tid < n && __float_as_uint(v0) == q.key && ties == q.rank) sm.found = tid;
+        __syncthreads();
+        pos = sm.found;
+    }
     if (tid == 0) {
         out[row] = pos >= 0 ? ci[pos] : 0;
         if (kept_mass) kept_mass[row] = (float)Z;
@@ -499,8 +586,8 @@ __global__ void __launch_bounds__(kSampleThreads) k_tp_select(float top_p, const
 }
 
 static int tp_blocks(int V) {
-    const int nb = (V + 2047) / 2048;
-    return nb < 1 ? 1 : (nb > 128 ? 128 : nb);
+    const int nb = (V + 2047) / 2048, least = V / 65535 + 1;  // a block's counts fit 16 bits
+    return std::max(nb < 1 ? 1 : (nb > 128 ? 128 : nb), least);
 }
 
 size_t sample_scratch_bytes(int rows, int V) { return (size_t)rows * tp_layout(V, tp_blocks(V)).stride; }
@@ -515,9 +602,8 @@ void sample_top_p(hipStream_t s, const float* x, int rows, int V, float temperat
     else
         hipLaunchKernelGGL(k_tp_zero, dim3(rows), dim3(kTpThreads), 0, s, sc, L);
     hipLaunchKernelGGL(k_tp_hist, dim3(NB, rows), dim3(kTpThreads), 0, s, x, V, temperature, NB, sc, L);
-    hipLaunchKernelGGL(k_tp_plan, dim3(rows), dim3(256), 0, s, NB, top_p, u, sc, L);
-    hipLaunchKernelGGL(k_tp_compact, dim3(NB, rows), dim3(kTpThreads), 0, s, V, NB, sc, L);
-    hipLaunchKernelGGL(k_tp_select, dim3(rows), dim3(kSampleThreads), 0, s, top_p, u, sc, L, out, kept_mass);
+    hipLaunchKernelGGL(k_tp_compact, dim3(NB, rows), dim3(kTpThreads), 0, s, V, NB, top_p, u, sc, L);
+    hipLaunchKernelGGL(k_tp_select, dim3(rows), dim3(kSampleThreads), 0, s, V, top_p, u, sc, L, out, kept_mass);
 }
 
 }  // namespace pgmi
