@@ -330,6 +330,7 @@ enum GemvRtMode : int {
 };
 struct GemvRtArgs {
     GemvRtForm form;
+    Act act;
     int B, N, K;  // N: outputs (rows of W, or channels); K: padded to 8
     const uint16_t* W;
     int ldw;

@@ -671,7 +671,7 @@ int forward_body(pgmi_ctx* x, hipStream_t s, const int64_t* ids, int rows, const
         const GemvRtForm form = gemv_rt_form(n_want, d.act, 1, 1);
         if (gemv_rt_fits(form, d.head.k, d.act)) {
             GemvRtArgs g{};
-            g.form = form; g.B = n_want; g.N = d.c.vocab; g.K = d.head.k; g.W = d.head.w; g.ldw = d.head.ldw; g.x = h; g.ldx = d.ldh;
+            g.form = form; g.act = d.act; g.B = n_want; g.N = d.c.vocab; g.K = d.head.k; g.W = d.head.w; g.ldw = d.head.ldw; g.x = h; g.ldx = d.ldh;
             g.out = logits; g.ldo = d.c.vocab;
             gemv_rt(s, d.act, GR_F32, g);
         } else {
@@ -728,7 +728,7 @@ int decode_body_rt(pgmi_ctx* x, hipStream_t s, const int64_t* ids, int B, void* 
             have_h = true;
         }
         GemvRtArgs g{};
-        g.form = form; g.B = B; g.N = w.n; g.K = w.k; g.W = w.w; g.ldw = w.ldw; g.S = d.c.streams; g.D = D; g.groups = d.c.norm_groups;
+        g.form = form; g.act = d.act; g.B = B; g.N = w.n; g.K = w.k; g.W = w.w; g.ldw = w.ldw; g.S = d.c.streams; g.D = D; g.groups = d.c.norm_groups;
         g.eps = d.c.norm_eps; g.X = d.X; g.in = sub.in; g.nw = sub.norm; g.slot = d.slot; g.pos = d.pos;
         if (have_h) { g.x = d.h; g.ldx = d.ldh; }
         have_h = false;
@@ -736,7 +736,7 @@ int decode_body_rt(pgmi_ctx* x, hipStream_t s, const int64_t* ids, int B, void* 
     };
     auto row_in = [&](const Lin& w, const void* in, int ldin) {
         GemvRtArgs g{};
-        g.form = form; g.B = B; g.N = w.n; g.K = w.k; g.W = w.w; g.ldw = w.ldw; g.x = in; g.ldx = ldin; g.slot = d.slot; g.pos = d.pos;
+        g.form = form; g.act = d.act; g.B = B; g.N = w.n; g.K = w.k; g.W = w.w; g.ldw = w.ldw; g.x = in; g.ldx = ldin; g.slot = d.slot; g.pos = d.pos;
         return g;
     };
     auto out_proj = [&](const Lin& o, const void* in, int ldin, const Sub& sub) {

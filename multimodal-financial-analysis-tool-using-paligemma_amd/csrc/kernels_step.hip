@@ -332,6 +332,283 @@ __global__ void __launch_bounds__(256) k_gemv_rt(GemvRtArgs a) {
     step_pads<T, MODE>(a);
 }
 
+// ---------------------------------------------------------------- one row of bf16, K a multiple of 512 up to 2048
+// A wave owns a unit's rows whole, the row x of activations in registers.  What bounds it is latency (a unit is one trip to
+// memory) and, in the long products, the stream, so
+//   - x, or the streams it is made of, is asked for before the first weights: the norm runs while they arrive, a quarter of it
+//     in each wave (every wave for itself: 2 streams of 2,048 read four times, 13.2 us where the other form took 12.8);
+//   - a unit's epilogue operands are asked for before the next unit's weights, which would otherwise have to land first
+//     (loads return in order), and the last unit is peeled off so that no branch hides what is in flight.
+// us, the LDS form / this one, 2 streams of 2,048 values: gate|up 27.3 / 21.7, mamba in + convolution 12.8 / 9.3, minGRU
+// 11.2 / 7.9, q|k|v 9.1 / 6.0, output matrix 187 / 158, mamba out 8.4 / 5.8, down 16.6 / 14.4; a step 0.83 / 0.67 ms.
+struct OneIn {  // an epilogue's operands
+    float v[8];
+    uint16_t w[6];
+};
+template <int MODE>
+__device__ __forceinline__ void one_load(const GemvRtArgs& a, int n, int slot, OneIn& e) {
+    n = min(n, a.N - 1);
+    if constexpr (MODE == GR_ACT) {
+        e.w[0] = (a.bias ? a.bias : a.W)[n];
+    } else if constexpr (MODE == GR_CONV) {
+        const int c = min(n, a.C - 1), KT = a.taps_k;
+        const float* tp = a.state + (long)slot * (KT - 1) * a.C + c;
+#pragma unroll
+        for (int j = 0; j < 3; ++j) e.v[j] = (KT > 1 ? tp : a.state)[(long)max(0, min(j, KT - 2)) * a.C];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) e.w[j] = a.cw[(long)c * KT + min(j, KT - 1)];
+        e.w[4] = a.cb[c];
+    } else if constexpr (MODE == GR_GRU) {
+        e.w[0] = a.bias[n];
+        e.w[1] = a.bias[a.N + n];
+        e.v[0] = a.state[(long)slot * a.N + n];
+    } else if constexpr (MODE == GR_STREAMS) {
+#pragma unroll
+        for (int s = 0; s < 4; ++s) e.v[s] = a.X[(long)min(s, a.S - 1) * a.D + n];
+    }
+}
+template <int MODE>
+__device__ __forceinline__ void one_store(const GemvRtArgs& a, int n, float v, float v1, float v2, int slot, bool first, const OneIn& e) {
+    uint16_t* out = reinterpret_cast<uint16_t*>(a.out);
+    if constexpr (MODE == GR_ACT) {
+        out[n] = f2bf(a.bias ? v + bf2f(e.w[0]) : v);
+    } else if constexpr (MODE == GR_LOGITS || MODE == GR_F32) {
+        reinterpret_cast<float*>(a.out)[n] = v;
+    } else if constexpr (MODE == GR_CONV) {
+        if (n >= a.C) {
+            reinterpret_cast<uint16_t*>(a.out2)[n - a.C] = f2bf(v);
+            return;
+        }
+        const int KT = a.taps_k;
+        float* tp = a.state + (long)slot * (KT - 1) * a.C + n;
+        float y = fmaf(bf2f(KT == 4 ? e.w[3] : KT == 3 ? e.w[2] : KT == 2 ? e.w[1] : e.w[0]), v, bf2f(e.w[4]));
+#pragma unroll
+        for (int j = 0; j < 3; ++j)
+            if (j < KT - 1) {
+                const float o = first ? 0.0f : e.v[j];
+                y = fmaf(bf2f(e.w[j]), o, y);
+                if (j > 0) tp[(long)(j - 1) * a.C] = o;
+            }
+        if (KT > 1) tp[(long)(KT - 2) * a.C] = v;
+        out[n] = f2bf(siluf_(y));
+    } else if constexpr (MODE == GR_GRU) {
+        const float z = sigmoidf_(v + bf2f(e.w[0]));
+        const float S = fmaf(1.0f - z, first ? 0.0f : e.v[0], z * gru_candidate(v1 + bf2f(e.w[1])));
+        a.state[(long)slot * a.N + n] = S;
+        out[n] = f2bf(S * siluf_(v2));
+    } else if constexpr (MODE == GR_SWIGLU) {
+        out[n] = f2bf(siluf_(v) * v1);
+    } else {  // GR_STREAMS
+        float* Xr = a.X + n;
+        if (!a.mix) {
+            *Xr = fmaf(a.mult, v, e.v[0]);
+            return;
+        }
+        for (int t = 0; t < a.S; ++t) {
+            float y = bf2f(a.wout[t]) * v;
+#pragma unroll
+            for (int s = 0; s < 4; ++s)
+                if (s < a.S) y = fmaf(bf2f(a.mix[s * a.S + t]), e.v[s], y);
+            Xr[(long)t * a.D] = y;
+        }
+    }
+}
+
+constexpr int one_rows(int mode) { return mode == GR_LOGITS ? 4 : unit_rows(mode); }
+constexpr int one_outs(int mode) { return mode == GR_LOGITS ? 4 : unit_outs(mode); }
+
+// CH: K / 512.  NS: 0: x is a row of activations; else up to NS streams, read and normed here.
+template <int MODE, int CH, int NS>
+__global__ void __launch_bounds__(256) k_gemv_one(GemvRtArgs a) {
+    constexpr int RW = one_rows(MODE), UO = one_outs(MODE);
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int nunit = (a.N + UO - 1) / UO, ustep = gridDim.x * 4, K = a.K;
+    int unit = blockIdx.x * 4 + wave;
+    uint4 w[RW][CH], x[CH], nw;
+    float4 X[NS ? NS : 1][2];
+    // the streams' read and norm are shared out: a wave takes one piece of 512 (of fewer pieces the last one twice)
+    const int piece = min(wave, CH - 1), px = piece * 512 + lane * 8;
+    static_assert(CH <= 4, "a piece per wave");
+    if constexpr (NS == 0) {
+#pragma unroll
+        for (int c = 0; c < CH; ++c) x[c] = ldg16(reinterpret_cast<const uint16_t*>(a.x) + c * 512 + lane * 8);
+    } else {
+#pragma unroll
+        for (int s = 0; s < NS; ++s) {
+            const float* p = a.X + (long)min(s, a.S - 1) * K + px;
+            X[s][0] = *reinterpret_cast<const float4*>(p);
+            X[s][1] = *reinterpret_cast<const float4*>(p + 4);
+        }
+        nw = ldg16(a.nw + px);
+    }
+    auto wload = [&](int u) {
+        u = min(u, nunit - 1);  // a wave without a unit repeats the last one's loads, and stores nothing
+#pragma unroll
+        for (int r = 0; r < RW; ++r) {
+            const uint16_t* p = a.W + (UO == 1 ? (long)r * a.N + u : (long)min(u * UO + r, a.N - 1)) * a.ldw + lane * 8;
+#pragma unroll
+            for (int c = 0; c < CH; ++c) w[r][c] = ldg_nt(p + c * 512);
+        }
+    };
+    wload(unit);
+    asm volatile("" ::: "memory");  // the stream stays ahead of the norm
+    constexpr bool ST = MODE == GR_CONV || MODE == GR_GRU;
+    const int slot = ST ? a.slot[0] : 0;
+    const bool first = ST && a.pos[0] == 0;
+    if constexpr (NS > 0) {
+        __shared__ __attribute__((aligned(16))) uint16_t xs[CH * 512];
+        __shared__ float red[4];
+        float u[8] = {}, q = 0.0f;
+        const int P = K / a.groups;
+#pragma unroll
+        for (int s = 0; s < NS; ++s) {
+            const float f = a.in ? bf2f(a.in[min(s, a.S - 1)]) : 1.0f;
+            const float t[8] = {X[s][0].x, X[s][0].y, X[s][0].z, X[s][0].w, X[s][1].x, X[s][1].y, X[s][1].z, X[s][1].w};
+#pragma unroll
+            for (int i = 0; i < 8; ++i) u[i] = s < a.S ? fmaf(f, t[i], u[i]) : u[i];
+        }
+#pragma unroll
+        for (int i = 0; i < 8; ++i) q = fmaf(u[i], u[i], q);
+        // a group is whole pieces of 512, or a power of two of lanes
+        for (int o = 1; o < 64 && o * 8 < P; o <<= 1) q += __shfl_xor(q, o, 64);
+        if (P > 512) {
+            if (lane == 0 && wave == piece) red[piece] = q;
+            __syncthreads();
+            q = 0.0f;
+            for (int c = piece * 512 / P * (P / 512), e = c + P / 512; c < e; ++c) q += red[c];
+        }
+        const float f = 1.0f / sqrtf(q / (float)P + a.eps);
+        const uint32_t g[4] = {nw.x, nw.y, nw.z, nw.w};
+        uint32_t o[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            o[i] = (uint32_t)f2bf(u[2 * i] * f * __uint_as_float(g[i] << 16)) |
+                   ((uint32_t)f2bf(u[2 * i + 1] * f * __uint_as_float(g[i] & 0xFFFF0000u)) << 16);
+        if (wave == piece) *reinterpret_cast<uint4*>(xs + px) = make_uint4(o[0], o[1], o[2], o[3]);
+        __syncthreads();
+#pragma unroll
+        for (int c = 0; c < CH; ++c) x[c] = *reinterpret_cast<const uint4*>(xs + c * 512 + lane * 8);
+    }
+    float best = -INFINITY;
+    int bi = 0x7fffffff;
+    auto step = [&](auto more) {
+        OneIn e;
+        const int n = unit * UO + (UO > 1 ? min(lane, UO - 1) : 0);
+        one_load<MODE>(a, n, slot, e);
+        float acc[RW];
+#pragma unroll
+        for (int r = 0; r < RW; ++r) {
+            acc[r] = 0.0f;
+#pragma unroll
+            for (int c = 0; c < CH; ++c) acc[r] = dot8(w[r][c], x[c], acc[r]);
+        }
+        if constexpr (decltype(more)::value) wload(unit + ustep);
+#pragma unroll
+        for (int r = 0; r < RW; ++r) acc[r] = wave_sum(acc[r]);
+        float v = acc[0];
+        if constexpr (UO > 1) {
+#pragma unroll
+            for (int r = 1; r < RW; ++r) v = lane == r ? acc[r] : v;
+        }
+        if constexpr (MODE == GR_LOGITS) {
+#pragma unroll
+            for (int r = 0; r < RW; ++r)
+                if (unit * UO + r < a.N && acc[r] > best) { best = acc[r]; bi = unit * UO + r; }
+        }
+        if (lane < UO && n < a.N) one_store<MODE>(a, n, v, acc[RW > 1 ? 1 : 0], acc[RW - 1], slot, first, e);
+        unit += ustep;
+    };
+    while (unit + ustep < nunit) step(std::true_type{});
+    if (unit < nunit) step(std::false_type{});
+    if constexpr (MODE == GR_LOGITS) {
+        __shared__ float sv[4];
+        __shared__ int si[4];
+        if (lane == 0) { sv[wave] = best; si[wave] = bi; }
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            for (int q = 1; q < 4; ++q)
+                if (sv[q] > best || (sv[q] == best && si[q] < bi)) { best = sv[q]; bi = si[q]; }
+            a.pmax[blockIdx.x] = best;
+            a.pidx[blockIdx.x] = bi;
+        }
+    }
+    step_pads<uint16_t, MODE>(a);
+}
+
+// The same for the long rows of the output projections (GR_STREAMS) and small products (GR_F32): the four waves of a workgroup
+// share a row of 2048 CH, one output per turn.
+template <int MODE, int CH>
+__global__ void __launch_bounds__(256) k_gemv_long(GemvRtArgs a) {
+    __shared__ float part[2][4];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int k0 = wave * CH * 512 + lane * 8, N = a.N;
+    int n = blockIdx.x, turn = 0;
+    uint4 w[CH], x[CH];
+#pragma unroll
+    for (int c = 0; c < CH; ++c) x[c] = ldg16(reinterpret_cast<const uint16_t*>(a.x) + k0 + c * 512);
+    auto wload = [&]() {
+        const uint16_t* p = a.W + (long)n * a.ldw + k0;
+#pragma unroll
+        for (int c = 0; c < CH; ++c) w[c] = ldg_nt(p + c * 512);
+    };
+    wload();
+    auto step = [&](auto more) {
+        OneIn e;
+        const int at = n;
+        one_load<MODE>(a, at, 0, e);
+        float acc = 0.0f;
+#pragma unroll
+        for (int c = 0; c < CH; ++c) acc = dot8(w[c], x[c], acc);
+        n += gridDim.x;
+        if constexpr (decltype(more)::value) wload();
+        acc = wave_sum(acc);
+        if (lane == 0) part[turn][wave] = acc;
+        __syncthreads();  // (the sums of two turns back are read before the barrier in between)
+        if (threadIdx.x == 0)
+            one_store<MODE>(a, at, part[turn][0] + part[turn][1] + part[turn][2] + part[turn][3], 0.0f, 0.0f, 0, false, e);
+        turn ^= 1;
+    };
+    while (n + (int)gridDim.x < N) step(std::true_type{});
+    step(std::false_type{});
+}
+
+bool gemv_long_fits(const GemvRtArgs& a, int mode) {
+    return a.form == GF_STREAM && a.B == 1 && a.x && a.S <= 4 && (mode == GR_STREAMS || mode == GR_F32) &&
+           (a.K == 4096 || a.K == 8192 || a.K == 16384);
+}
+template <int MODE>
+void run_long(hipStream_t s, const GemvRtArgs& a) {
+    const dim3 grid(std::min(a.N, a.K >= 16384 ? 512 : 1024)), block(256);
+    if (a.K == 4096) hipLaunchKernelGGL((k_gemv_long<MODE, 2>), grid, block, 0, s, a);
+    else if (a.K == 8192) hipLaunchKernelGGL((k_gemv_long<MODE, 4>), grid, block, 0, s, a);
+    else hipLaunchKernelGGL((k_gemv_long<MODE, 8>), grid, block, 0, s, a);
+}
+
+bool gemv_one_fits(const GemvRtArgs& a, int mode) {
+    if (a.form != GF_STREAM || a.B != 1 || a.K % 512 != 0 || a.K > 2048 || a.S > 4) return false;
+    if (mode == GR_CONV && a.taps_k > 4) return false;
+    if (a.x) return true;
+    const int P = a.K / std::max(1, a.groups);
+    return a.D == a.K && a.groups >= 1 && a.K % a.groups == 0 && (P % 512 == 0 || (512 % P == 0 && P >= 8));
+}
+
+template <int MODE, int CH>
+void run_one_ch(hipStream_t s, const GemvRtArgs& a, int blocks) {
+    if (a.x) hipLaunchKernelGGL((k_gemv_one<MODE, CH, 0>), dim3(blocks), dim3(256), 0, s, a);
+    else if (a.S <= 2) hipLaunchKernelGGL((k_gemv_one<MODE, CH, 2>), dim3(blocks), dim3(256), 0, s, a);
+    else hipLaunchKernelGGL((k_gemv_one<MODE, CH, 4>), dim3(blocks), dim3(256), 0, s, a);
+}
+template <int MODE>
+void run_one(hipStream_t s, const GemvRtArgs& a) {
+    const int blocks = gemv_rt_blocks(a, (GemvRtMode)MODE);
+    switch (a.K / 512) {
+        case 1: run_one_ch<MODE, 1>(s, a, blocks); break;
+        case 2: run_one_ch<MODE, 2>(s, a, blocks); break;
+        case 3: run_one_ch<MODE, 3>(s, a, blocks); break;
+        default: run_one_ch<MODE, 4>(s, a, blocks); break;
+    }
+}
+
 int k_split(const GemvRtArgs& a, int mode) { return mode != GR_LOGITS && a.K >= 4096 ? 4 : 1; }
 
 template <typename T, int NB, int MODE, int WK>
@@ -631,11 +908,32 @@ int gemv_rt_split(GemvRtForm form, int N, int K) {
 }
 
 int gemv_rt_blocks(const GemvRtArgs& a, GemvRtMode mode) {
+    if (a.act == ACT_BF16 && gemv_one_fits(a, mode)) {
+        const int units = (a.N + one_outs(mode) - 1) / one_outs(mode);
+        return std::max(1, std::min((units + 3) / 4, mode == GR_LOGITS ? 2048 : 1024));
+    }
     const int units = (a.N + unit_outs(mode) - 1) / unit_outs(mode), upb = 4 / k_split(a, mode);
     return std::max(1, std::min((units + upb - 1) / upb, 1024));
 }
 
 void gemv_rt(hipStream_t s, Act act, GemvRtMode mode, const GemvRtArgs& a) {
+    if (act == ACT_BF16 && gemv_one_fits(a, mode)) {
+        switch (mode) {
+            case GR_ACT: run_one<GR_ACT>(s, a); break;
+            case GR_CONV: run_one<GR_CONV>(s, a); break;
+            case GR_GRU: run_one<GR_GRU>(s, a); break;
+            case GR_SWIGLU: run_one<GR_SWIGLU>(s, a); break;
+            case GR_STREAMS: run_one<GR_STREAMS>(s, a); break;
+            case GR_LOGITS: run_one<GR_LOGITS>(s, a); break;
+            case GR_F32: run_one<GR_F32>(s, a); break;
+        }
+        return;
+    }
+    if (act == ACT_BF16 && gemv_long_fits(a, mode)) {
+        if (mode == GR_STREAMS) run_long<GR_STREAMS>(s, a);
+        else run_long<GR_F32>(s, a);
+        return;
+    }
     if (a.form == GF_SKINNY && act == ACT_BF16) run_skinny<uint16_t>(s, mode, a);
     else if (a.form == GF_SKINNY) run_skinny<float>(s, mode, a);
     else if (act == ACT_BF16) run_mode<uint16_t, 1>(s, mode, a);
