@@ -731,9 +731,95 @@ __global__ void __launch_bounds__(256) k_skinny(GemvRtArgs a) {
     step_pads<T, MODE>(a);
 }
 
+// The same for bf16 and K up to 2048, the activations held in registers over several groups of 16 outputs per workgroup: what
+// a group moves besides its weights is otherwise as many bytes of activations from L2 (8 rows: the output matrix of 257,216 x
+// 2048 207 us, held 185; gate|up of 16,384 channels 32.0 / 25.7).  The next group's weights are asked for before this one's
+// sums meet, the last group peeled off.  (fp32 rows, three pieces each, would take 200 registers.)
+template <int MODE>
+__global__ void __launch_bounds__(256) k_skinny_held(GemvRtArgs a) {
+    constexpr int NM = MODE == GR_SWIGLU ? 2 : 1, ST = 8;  // 64-deep steps of a wave
+    __shared__ float sums[2][4][NM][16][17];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int li = lane & 15, lg = lane >> 4, K = a.K, ngroup = (a.N + 15) / 16;
+    const uint16_t* xp = reinterpret_cast<const uint16_t*>(a.x) + (long)(li < a.B ? li : a.B - 1) * a.ldx;
+    short8 x[ST][2];
+#pragma unroll
+    for (int i = 0; i < ST; ++i)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const int k = (wave + 4 * i) * 64 + lg * 16 + 8 * h;
+            x[i][h] = __builtin_bit_cast(short8, ldg16_sel(xp + k, k < K, xp));
+        }
+    uint4 w[ST][NM][2];
+    int grp = blockIdx.x, turn = 0;
+    auto wload = [&]() {
+#pragma unroll
+        for (int m = 0; m < NM; ++m) {
+            const uint16_t* p = a.W + ((long)m * a.N + min(grp * 16 + li, a.N - 1)) * a.ldw;
+#pragma unroll
+            for (int i = 0; i < ST; ++i)
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    const int k = (wave + 4 * i) * 64 + lg * 16 + 8 * h;
+                    w[i][m][h] = ldg16(k < K ? p + k : p);  // past the end: the activations are zero
+                }
+        }
+    };
+    wload();
+    auto step = [&](auto more) {
+        const int n0 = grp * 16;
+        f32x4 acc[NM];
+#pragma unroll
+        for (int m = 0; m < NM; ++m) acc[m] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int i = 0; i < ST; ++i)
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+#pragma unroll
+                for (int m = 0; m < NM; ++m) acc[m] = mfma16(__builtin_bit_cast(short8, w[i][m][h]), x[i][h], acc[m]);
+        grp += gridDim.x;
+        if constexpr (decltype(more)::value) wload();
+#pragma unroll
+        for (int m = 0; m < NM; ++m)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) sums[turn][wave][m][4 * lg + r][li] = acc[m][r];
+        __syncthreads();  // (the sums of two turns back are read before the barrier in between)
+        const int b = tid >> 4, n = n0 + (tid & 15);  // consecutive threads store consecutive outputs
+        float v[2] = {0.f, 0.f};
+#pragma unroll
+        for (int m = 0; m < NM; ++m)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) v[m] += sums[turn][q][m][tid & 15][b];
+        turn ^= 1;
+        if (b >= a.B || n >= a.N) return;
+        if (K < 2048) {  // past K a zero has met the row's first weights: formed again where one of them is not finite
+#pragma unroll
+            for (int m = 0; m < NM; ++m)
+                if (not_finite(v[m])) {
+                    const uint16_t* p = a.W + ((long)m * a.N + n) * a.ldw;
+                    v[m] = 0.0f;
+#pragma clang loop unroll(disable)
+                    for (int k = 0; k < K; ++k) v[m] = fmaf(bf2f(reinterpret_cast<const uint16_t*>(a.x)[(long)b * a.ldx + k]), bf2f(p[k]), v[m]);
+                }
+        }
+        if constexpr (MODE == GR_F32) reinterpret_cast<float*>(a.out)[(long)b * a.ldo + n] = v[0];
+        else step_epilogue<uint16_t, MODE>(a, n, b, v[0], v[1], 0.f);
+    };
+    while (grp + (int)gridDim.x < ngroup) step(std::true_type{});
+    step(std::false_type{});
+    step_pads<uint16_t, MODE>(a);
+}
+
 template <typename T>
 void run_skinny(hipStream_t s, GemvRtMode mode, const GemvRtArgs& a) {
     const dim3 grid((a.N + 15) / 16), block(256);
+    constexpr int kHeldBlocks = 512;  // two per CU: 256, 512 and 768 measured equal, 1,024 and more slower
+    if (std::is_same<T, uint16_t>::value && a.K <= 2048 && a.split <= 1 && (int)grid.x > kHeldBlocks &&
+        (mode == GR_F32 || mode == GR_LOGITS || mode == GR_SWIGLU)) {
+        if (mode == GR_SWIGLU) hipLaunchKernelGGL((k_skinny_held<GR_SWIGLU>), dim3(kHeldBlocks), block, 0, s, a);
+        else hipLaunchKernelGGL((k_skinny_held<GR_F32>), dim3(kHeldBlocks), block, 0, s, a);
+        return;
+    }
     switch (mode) {
         case GR_ACT: hipLaunchKernelGGL((k_skinny<T, GR_ACT>), grid, block, 0, s, a); break;
         case GR_CONV: hipLaunchKernelGGL((k_skinny<T, GR_CONV>), grid, block, 0, s, a); break;
