@@ -4,6 +4,7 @@
 //
 //   k_append    norms and rotates the heads of a prefill's rows, writes the key / value rows into the cache
 //   k_wattn     plain form, any size and both activation types: one workgroup per (row, head), online softmax
+//   k_wattn_f   fp32 MFMA form: 16 (position, head) pairs per workgroup, its waves on every fourth 16-key tile
 //   k_wattn_m   bf16 MFMA form: 64 (position, head) pairs per workgroup against 64-key tiles of one key/value head
 //   k_wattn_d   one new token per sequence: keys split over workgroups, partials merged by k_wattn_dc
 //   k_wattn_dm  the same on bf16 MFMA
@@ -214,6 +215,191 @@ __global__ void __launch_bounds__(256) k_wattn(WAttnArgs a) {
     }
     if (h == w.H - 1)
         for (int k = w.H * w.e + tid; k < a.ldo; k += 256) stf(o + k, 0.0f);
+}
+
+// ---------------------------------------------------------------- fp32 MFMA form
+// Products and sums stay fp32 (16x16x4 MFMA, a fused multiply-add per term).  S^T = K Q^T puts a query on lane & 15 and keys
+// 4 (lane >> 4) + r on accumulator r: the B operand of O^T = V^T P^T as it stands, a contraction slot per lane group.  Which
+// slot is which dim or key is free, and which output row is which value column: every load is 16 bytes a lane, straight from
+// the cache into registers.  Bound by the MFMA's rate and by the longest row's chain of tiles, so a tile of 16 pairs (500
+// positions of 8 heads: 250 workgroups) with its keys dealt to four waves, long rows first.  The K of the wave's next tile is
+// asked for between the two products, its V after them.  k_wattn, dims of 128: 500 positions of 8 heads 105 us, 1,024
+// positions 312; here 24 and 58.
+__device__ __forceinline__ f32x4 mfma_f32(float a, float b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
+
+// PAD: heads narrower than D
+template <int D, int SC, bool PAD>
+__global__ void __launch_bounds__(256, D <= 128 ? 2 : 1) k_wattn_f(WAttnArgs a) {
+    constexpr int QC = D / 16, VC = D / 64, PT = kWAttnRows / 16;
+    __shared__ __attribute__((aligned(16))) float part[4][16][68];  // 64 value columns of the waves' sums
+    __shared__ float ms[4][16], ls[4][16];
+    const WAttnHeads& w = a.hd;
+    const int at = a.ntile * PT - 1 - (int)blockIdx.x;  // the later positions of a sequence first
+    const ChunkInfo tl = a.tiles[at / PT];
+    const SeqInfo sq = a.seqs[tl.seq];
+    const int g = blockIdx.y, R = w.H / w.G, nrow = sq.len * R, row0 = tl.rel + at % PT * 16;
+    if (row0 >= nrow) return;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int li = lane & 15, lg = lane >> 4;
+    const int fr = min(row0 + li, nrow - 1), prow = fr / R, h = g * R + fr % R, i = sq.start + prow;
+    const Score<SC> score(a.sc, h);
+    const int window = a.sc.window, keep = a.sc.keep;
+    // positions of the first and last pairs; keys they see: [lo, hi], and the kept ones before them: [0, kept)
+    const int wfirst = sq.start + row0 / R, hi = sq.start + min(row0 + 15, nrow - 1) / R;
+    const int lo = max(0, wfirst - window + 1), kept = min(keep, lo), nh = (kept + 15) / 16, nt = nh + (hi - lo) / 16 + 1;
+    const float* kc = reinterpret_cast<const float*>(a.kc) + ((long)sq.slot * w.G + g) * a.max_tokens * w.dp;
+    const float* vc = reinterpret_cast<const float*>(a.vc) + ((long)sq.slot * w.G + g) * a.max_tokens * w.ep;
+    auto key0 = [&](int t) { return t < nh ? 16 * t : lo + 16 * (t - nh); };
+    auto ld4 = [](const float* p, bool ok, const float* safe) {
+        if constexpr (PAD) return __builtin_bit_cast(f32x4, ldg16_sel(p, ok, safe));
+        else return *reinterpret_cast<const f32x4*>(p);
+    };
+    f32x4 q[QC], k[QC], v[4][VC], o[VC][4];  // v[r][c]: columns 64 c + 4 li .. of key 4 lg + r; o[c][x][r]: column 64 c + 16 lg + 4 r + x
+    const float* qp = reinterpret_cast<const float*>(a.q) + ((long)(sq.off + prow) * w.H + h) * w.dp;
+#pragma unroll
+    for (int c = 0; c < QC; ++c) q[c] = ld4(qp + 16 * c + 4 * lg, 16 * c + 4 * lg < w.dp, qp);
+    auto kload = [&](int t) {
+        const float* p = kc + (long)min(key0(t) + li, hi) * w.dp;
+#pragma unroll
+        for (int c = 0; c < QC; ++c) k[c] = ld4(p + 16 * c + 4 * lg, 16 * c + 4 * lg < w.dp, kc);
+    };
+    auto vload = [&](int t) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const float* p = vc + (long)min(key0(t) + 4 * lg + r, hi) * w.ep;
+#pragma unroll
+            for (int c = 0; c < VC; ++c) v[r][c] = ld4(p + 64 * c + 4 * li, 64 * c + 4 * li < w.ep, vc);
+        }
+    };
+#pragma unroll
+    for (int c = 0; c < VC; ++c)
+#pragma unroll
+        for (int x = 0; x < 4; ++x) o[c][x] = f32x4{0.f, 0.f, 0.f, 0.f};
+    float m = kNone, l = 0.0f;
+    if (wave < nt) {
+        kload(wave);
+        vload(wave);
+    }
+    for (int t = wave; t < nt; t += 4) {
+        const int j0 = key0(t), tn = min(t + 4, nt - 1);
+        f32x4 s = {0.f, 0.f, 0.f, 0.f}, s1 = s;
+#pragma unroll
+        for (int c = 0; c < QC; c += 2)
+#pragma unroll
+            for (int x = 0; x < 4; ++x) {
+                s = mfma_f32(k[c][x], q[c][x], s);
+                s1 = mfma_f32(k[c + 1][x], q[c + 1][x], s1);
+            }
+        kload(tn);
+        __builtin_amdgcn_sched_barrier(0);
+        const bool head = t < nh;  // kept keys: every row sees those before lo
+        const bool whole = head ? j0 + 16 <= kept : j0 + 15 <= wfirst && (hi - j0 < window || j0 + 16 <= keep);
+        const int end = head ? kept : i + 1;
+        auto sees = [&](int j) { return (j < end) & ((i - j < window) | (j < keep)); };
+        float mt = m;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int j = j0 + 4 * lg + r;
+            const float e = score.exact(s[r] + s1[r], (float)(i - j));
+            s[r] = sees(j) ? e : -INFINITY;
+            mt = fmaxf(mt, s[r]);
+        }
+        mt = fmaxf(mt, __shfl_xor(mt, 16, 64));
+        mt = fmaxf(mt, __shfl_xor(mt, 32, 64));
+        const float alpha = exp2f(m - mt);
+        m = mt;
+        l *= alpha;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            s[r] = exp2f(s[r] - m);
+            l += s[r];  // this lane's keys; summed over the lane groups at the end
+        }
+        if (__any(alpha != 1.0f)) {
+#pragma unroll
+            for (int c = 0; c < VC; ++c)
+#pragma unroll
+                for (int x = 0; x < 4; ++x) o[c][x] *= alpha;
+        }
+        float bad = 0.0f;
+        if (!whole) {  // a weight of zero must not meet what is not finite
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+#pragma unroll
+                for (int c = 0; c < VC; ++c)
+#pragma unroll
+                    for (int x = 0; x < 4; ++x) bad = fmaf(v[r][c][x], 0.0f, bad);
+        }
+        if (!__any(bad != bad)) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+#pragma unroll
+                for (int c = 0; c < VC; ++c)
+#pragma unroll
+                    for (int x = 0; x < 4; ++x) o[c][x] = mfma_f32(v[r][c][x], s[r], o[c][x]);
+        } else {
+#pragma clang loop unroll(disable)
+            for (int n = 0; n < 16; ++n) {
+                const int j = j0 + n, from = n / 4 * 16 + li;
+                const float p0 = __shfl(s[0], from, 64), p1 = __shfl(s[1], from, 64), p2 = __shfl(s[2], from, 64), p3 = __shfl(s[3], from, 64);
+                const float p = n & 2 ? n & 1 ? p3 : p2 : n & 1 ? p1 : p0;
+                if (!sees(j)) continue;
+                const float* vp = vc + (long)j * w.ep;
+#pragma unroll
+                for (int c = 0; c < VC; ++c)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        const int col = 64 * c + 16 * lg + 4 * r;
+                        const f32x4 f = ld4(vp + col, col < w.ep, vc);
+                        const bool in = col < w.ep;
+#pragma unroll
+                        for (int x = 0; x < 4; ++x) o[c][x][r] = in ? fmaf(p, f[x], o[c][x][r]) : 0.0f;
+                    }
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        vload(tn);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    l += __shfl_xor(l, 16, 64);
+    l += __shfl_xor(l, 32, 64);
+    if (lg == 0) { ms[wave][li] = m; ls[wave][li] = l; }
+    __syncthreads();
+    const float f = exp2f(m - fmaxf(fmaxf(ms[0][li], ms[1][li]), fmaxf(ms[2][li], ms[3][li])));
+    // a thread per four value columns of a pair
+    const int pr = tid >> 4, of = row0 + pr, oh = g * R + of % R;
+    const float pm = fmaxf(fmaxf(ms[0][pr], ms[1][pr]), fmaxf(ms[2][pr], ms[3][pr]));
+    float sum = 0.0f;
+#pragma unroll
+    for (int x = 0; x < 4; ++x) sum = fmaf(ls[x][pr], exp2f(ms[x][pr] - pm), sum);
+    float* out = reinterpret_cast<float*>(a.o) + (long)(sq.off + of / R) * a.ldo;
+#pragma unroll
+    for (int c = 0; c < VC; ++c) {
+        if (c) __syncthreads();
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+            *reinterpret_cast<f32x4*>(&part[wave][li][16 * lg + 4 * r]) = f32x4{o[c][0][r] * f, o[c][1][r] * f, o[c][2][r] * f, o[c][3][r] * f};
+        __syncthreads();
+        f32x4 t = *reinterpret_cast<const f32x4*>(&part[0][pr][(tid & 15) * 4]);
+#pragma unroll
+        for (int x = 1; x < 4; ++x) t += *reinterpret_cast<const f32x4*>(&part[x][pr][(tid & 15) * 4]);
+        const int col = 64 * c + (tid & 15) * 4;
+        if (of < nrow)
+#pragma unroll
+            for (int x = 0; x < 4; ++x)
+                if (col + x < w.e) out[oh * w.e + col + x] = t[x] / sum;
+    }
+    if (of < nrow && oh == w.H - 1)
+        for (int x = w.H * w.e + (tid & 15); x < a.ldo; x += 16) out[x] = 0.0f;
+}
+
+template <int D>
+void run_f(hipStream_t s, const WAttnArgs& a) {
+    const dim3 grid(a.ntile * (kWAttnRows / 16), a.hd.G);
+    const bool pad = a.hd.dp != D || a.hd.ep != D;
+    if (a.sc.r1 && pad) hipLaunchKernelGGL((k_wattn_f<D, SC_BIAS, true>), grid, dim3(256), 0, s, a);
+    else if (a.sc.r1) hipLaunchKernelGGL((k_wattn_f<D, SC_BIAS, false>), grid, dim3(256), 0, s, a);
+    else if (pad) hipLaunchKernelGGL((k_wattn_f<D, SC_PLAIN, true>), grid, dim3(256), 0, s, a);
+    else hipLaunchKernelGGL((k_wattn_f<D, SC_PLAIN, false>), grid, dim3(256), 0, s, a);
 }
 
 // ---------------------------------------------------------------- bf16 MFMA form
@@ -904,7 +1090,11 @@ void wattn_append(hipStream_t s, Act act, const WAttnArgs& a) {
 void wattn_prefill(hipStream_t s, Act act, const WAttnArgs& a) {
     const int dp = a.hd.dp, ep = a.hd.ep;
     if (act == ACT_F32) {
-        plain_t<float>(s, a);
+        const int n = std::max(dp, ep);
+        if (n > 256) plain_t<float>(s, a);
+        else if (n <= 64) run_f<64>(s, a);
+        else if (n <= 128) run_f<128>(s, a);
+        else run_f<256>(s, a);
     } else if (dp > 256 || ep > 256) {
         plain_t<uint16_t>(s, a);
     } else if (dp <= 64) {
