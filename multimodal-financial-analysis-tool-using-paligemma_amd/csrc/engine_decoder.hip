@@ -2,6 +2,7 @@
 // mixer and an optional feed-forward, around residual streams or one plain residual.  Weight layout, derived
 // tensors, the per-sequence state slab, the ragged forward (prompts and portions of prompts) and the decode step
 // (hipGraph-replayed), over the mechanisms of decoder.h.  A design is its layer list and constants; nothing here names one.
+#include <climits>
 #include <set>
 
 #include "decoder.h"
@@ -1026,14 +1027,29 @@ int pgmi_decoder_forward(pgmi_ctx* x, const int64_t* ids, int n_seq, const int32
         }
         return c;
     };
-    // The recurrences take the longest runs that still give every CU a workgroup: a short step's few runs are otherwise walked
-    // by a few CUs, each row waiting for the one before.  us of the scan's three launches, 64- / 16-row runs: 500 rows of 2,048
-    // channels 86 / 41, 300 rows 69 / 35; where the chip is full short runs only add carries (1,540 rows of 4,096: 98 / 121).
-    auto run_rows = [&](int longest, int width, int per_wg) {  // width channels, per_wg of them per workgroup
-        const long cols = std::max(1, (width + per_wg - 1) / per_wg);
-        int ct = longest;
-        for (const int k : {4, 3, 2, 1}) {  // longest, 3/4, 1/2, 1/4 of it
-            ct = longest * k / 4;
+    // A short step's few runs are walked by a few CUs, each row waiting for the one before; where the chip is full short runs
+    // only add carries.  The scan (workgroups of 256 channels, a wave per SIMD) takes the run length whose rounds of 256
+    // workgroups walk the fewest rows, a workgroup's start costing about 8.  us of its three launches, 64- / 16-row runs: 500
+    // rows of 2,048 channels 86 / 41, 300 rows 69 / 35; 64 rows / this rule: 1,540 rows of
+    // 4,096 channels (50-row runs) 98 / 92.
+    auto scan_rows = [&](int width) {
+        const long cols = std::max(1, (width + 255) / 256);
+        int best = 64;
+        long least = LONG_MAX;
+        for (int ct = 64; ct >= 16; ct -= 2) {
+            long n = 0;
+            for (int r = 0; r < n_seq; ++r) n += (lens[r] + ct - 1) / ct;
+            const long cost = (n * cols + 255) / 256 * (ct + 8);
+            if (cost < least) { least = cost; best = ct; }
+        }
+        return best;
+    };
+    // minGRU: the longest runs, down to 8 rows, that still give every CU a workgroup of 128 channels
+    auto gru_rows = [&](int width) {
+        const long cols = std::max(1, (width + 127) / 128);
+        int ct = 32;
+        for (const int k : {32, 24, 16, 8}) {
+            ct = k;
             long n = 0;
             for (int r = 0; r < n_seq; ++r) n += (lens[r] + ct - 1) / ct;
             if (n * cols >= 256) break;
@@ -1046,7 +1062,7 @@ int pgmi_decoder_forward(pgmi_ctx* x, const int64_t* ids, int n_seq, const int32
         if (l.mixer == PGMI_MIXER_MINGRU) gru_width = std::max(gru_width, l.width);
     }
     const bool huge = rows > 16384;
-    const Cut scan = cut(huge ? 256 : run_rows(64, scan_width, 256)), gru = cut(huge ? 128 : run_rows(32, gru_width, 128));
+    const Cut scan = cut(huge ? 256 : scan_rows(scan_width)), gru = cut(huge ? 128 : gru_rows(gru_width));
     // the convolutions carry nothing: 500 rows of 2,048 channels 11.2 us on 64-row runs, 5.9 on 16; 2,048 rows 10.8 / 7.5
     const Cut conv = cut(huge ? 256 : rows > 2048 ? 32 : 16);
     struct Tiles { int R; size_t o; int n; };
