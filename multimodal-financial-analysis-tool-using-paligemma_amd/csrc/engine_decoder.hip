@@ -1030,8 +1030,7 @@ int pgmi_decoder_forward(pgmi_ctx* x, const int64_t* ids, int n_seq, const int32
     // A short step's few runs are walked by a few CUs, each row waiting for the one before; where the chip is full short runs
     // only add carries.  The scan (workgroups of 256 channels, a wave per SIMD) takes the run length whose rounds of 256
     // workgroups walk the fewest rows, a workgroup's start costing about 8.  us of its three launches, 64- / 16-row runs: 500
-    // rows of 2,048 channels 86 / 41, 300 rows 69 / 35; 64 rows / this rule: 1,540 rows of
-    // 4,096 channels (50-row runs) 98 / 92.
+    // rows of 2,048 channels 86 / 41, 300 rows 69 / 35; 64 rows / this rule: 1,540 rows of 4,096 channels (50-row runs) 98 / 92.
     auto scan_rows = [&](int width) {
         const long cols = std::max(1, (width + 255) / 256);
         int best = 64;
