@@ -188,7 +188,7 @@ __device__ __forceinline__ void gemv_block(const GemvArgs& a, const int blk, con
         // partial rows in one round trip, no LDS staging of the weights, no barrier)
         const int nch = (a.st->kv_len + 1 + kAttnChunk - 1) / kAttnChunk;
         // chunks held in registers (768 keys); longer caches take several passes under a running maximum, each one round trip
-        // to memory: 17 chunks, two rows 23.2 us (one trip per record) -> 13.8
+        // to memory: 17 chunks, two rows 23.2 us (one trip per record) -> 12.0
         constexpr int CMAX = 12;
         const int nitems = a.nb * K / 8;
         for (int e8 = tid; e8 < nitems; e8 += 256) {

@@ -10,7 +10,7 @@ from decoder_helpers import build, tokens
 pytestmark = pytest.mark.gpu
 
 
-# (sequences, tokens each): runs of 64, 48, 32 and 16 rows at these models' widths, and past 16,384 rows of 256
+# (sequences, tokens each): run lengths from 64 rows down to 16 at these models' widths, and past 16,384 rows of 256
 @pytest.mark.parametrize("n,length", [(36, 450), (30, 400), (20, 450), (3, 97), (40, 430)])
 @pytest.mark.parametrize("name", sorted(C.MIXED))
 def test_together_as_alone(name, n, length):
