@@ -39,8 +39,8 @@ __device__ __forceinline__ double wave_sum_d(double v) {
 
 struct SelectOut {
     uint32_t key;  // bit pattern of the probability at the crossing position
-    double above;  // mass of every probability > key
-    int rank;      // the crossing is the rank-th (index order, 0-based) token equal to key
+    double mass;   // inclusive mass at the crossing
+    int rank;      // it is the rank-th (index order, 0-based) token equal to key; ranked candidates: its place among them
     bool crossed;  // false: target >= the total mass (no crossing)
 };
 
@@ -53,11 +53,13 @@ struct SampleSmem {
     unsigned hcnt[kLevels][64];
     unsigned long long hmq[kLevels][64];
     double row_suf[256 + 4];  // the row's suffix masses by exponent
-    int top[4];               // per wave
-    double above;
+    int top[2][4];            // per wave
     int scan[kSampleThreads / 64];
-    int found, rank;
-    uint32_t key;
+    int found;
+    // the ranked candidates in descending order: value, inclusive mass, place
+    float ord_val[kRanked];
+    double ord_mass[kRanked];
+    int ord_at[kRanked];
 };
 
 // suf[t] = mass of bins t .. 255 (mq in fixed point), t < 256: the wave's 64 bins by shuffles, then the higher waves'
@@ -93,6 +95,16 @@ __device__ __forceinline__ int highest(bool is, int* top) {
     return max(max(top[0], top[1]), max(top[2], top[3]));
 }
 
+// The smallest such t, -1 if none; the block is its first four waves.  One barrier: calls in turn take turns with two tops.
+__device__ __forceinline__ int lowest(bool is, int* top) {
+    const unsigned long long m = __ballot(is);
+    const int w = threadIdx.x >> 6;
+    if ((threadIdx.x & 63) == 0) top[w] = m ? 64 * w + __ffsll((long long)m) - 1 : 256;
+    __syncthreads();
+    const int t = min(min(top[0], top[1]), min(top[2], top[3]));
+    return t < 256 ? t : -1;
+}
+
 __device__ __forceinline__ void hist_add(unsigned* hcnt, unsigned long long* hmq, bool valid, int d, float v) {
     if (valid) {
         atomicAdd(&hcnt[d], 1u);
@@ -110,8 +122,8 @@ __device__ __forceinline__ SelectOut radix_select(const Value& value, int n, int
         (&sm.hcnt[0][0])[i] = 0u;
         (&sm.hmq[0][0])[i] = 0ull;
     }
-    const int bin = highest(t < 256 && used && sm.row_suf[t & 255] > target, sm.top);
-    if (bin < 0) return SelectOut{0u, sm.row_suf[0], 0, false};
+    const int bin = highest(t < 256 && used && sm.row_suf[t & 255] > target, sm.top[0]);
+    if (bin < 0) return SelectOut{0u, 0.0, 0, false};
     uint32_t prefix = (uint32_t)bin << 23, pmask = 0xFF800000u;
     double above = bin < 255 ? sm.row_suf[bin + 1] : 0.0;
 #pragma unroll 1
@@ -135,7 +147,7 @@ __device__ __forceinline__ SelectOut radix_select(const Value& value, int n, int
             if (lane + o < 64) suf += x;
         }
         const unsigned long long m = __ballot(sm.hcnt[level][lane] != 0u && above + (double)suf * kMassUnit > target);
-        if (!m) return SelectOut{0u, above, 0, false};
+        if (!m) return SelectOut{0u, 0.0, 0, false};
         const int d = 63 - __clzll((long long)m);
         above += (double)(unsigned long long)__shfl(suf - own, d, 64) * kMassUnit;
         prefix |= (uint32_t)d << shift;
@@ -151,7 +163,7 @@ __device__ __forceinline__ SelectOut radix_select(const Value& value, int n, int
         while (rank > 0 && above + (double)rank * val > target) --rank;
         while (!(above + (double)(rank + 1) * val > target)) ++rank;
     }
-    return SelectOut{prefix, above, rank, true};
+    return SelectOut{prefix, above + (double)(rank + 1) * val, rank, true};
 }
 
 // place of the rank-th candidate (index order) whose bit pattern equals key; -1 if fewer exist
@@ -495,37 +507,42 @@ __global__ void __launch_bounds__(kSampleThreads) k_tp_select(int V, float top_p
     if (tid >= NT) return;  // whole waves: the barriers below count those that are left
     auto value = [&](int i) { return i < kHeld ? sm.val[i] : cv[i]; };
 
-    // ranked: this thread's candidate, the mass of the larger ones, and how many equal ones come before it
+    // ranked: this thread's candidate, the mass of the larger ones, and how many equal ones come before it; then thread t
+    // takes the t-th candidate of the descending order
     const bool ranked = n <= kRanked;
-    double larger = 0.0;
-    int ties = 0;
-    if (ranked && tid < n) {
-        unsigned long long q = 0ull;
-#pragma unroll 1
-        for (int j = 0; j < n; ++j) {
-            const float w = sm.val[j];
-            q += w > v0 ? mass_q(w) : 0ull;
-            ties += w == v0 && j < tid;
+    double mass = 0.0;
+    if (ranked) {
+        if (tid < n) {
+            unsigned long long q = 0ull;
+            int at = 0, ties = 0;
+#pragma unroll 4  // (one at a time each waits for its read: 21.5 us a draw, so 20.1)
+            for (int j = 0; j < n; ++j) {
+                const float w = sm.val[j];
+                q += w > v0 ? mass_q(w) : 0ull;
+                at += w > v0;
+                ties += w == v0 && j < tid;
+            }
+            sm.ord_val[at + ties] = v0;
+            sm.ord_mass[at + ties] = (M.c_hi < 255 ? sm.row_suf[M.c_hi + 1] : 0.0) + (double)q * kMassUnit + (double)(ties + 1) * (double)v0;
+            sm.ord_at[at + ties] = tid;
         }
-        larger = (M.c_hi < 255 ? sm.row_suf[M.c_hi + 1] : 0.0) + (double)q * kMassUnit;
+        __syncthreads();
+        if (tid < n && sm.ord_val[tid] > 0.f) mass = sm.ord_mass[tid];  // (0: cannot be drawn)
     }
-    // first position whose inclusive cumulative mass exceeds target
-    auto select = [&](double target) -> SelectOut {
+    // First position whose inclusive cumulative mass exceeds target.  Ranked: the masses of the larger ones are truncated sums, and
+    // round otherwise than the inclusive ones, so neighbours may both or neither step over a target between them: the first
+    // that is past it counts, and where there must be one, the last that can be drawn.
+    int turn = 0;
+    auto select = [&](double target, bool must) -> SelectOut {
         if (!ranked) return radix_select(value, n, NT, target, used, sm);
-        // (one candidate at most: its predecessor's inclusive mass does not exceed it)
-        const bool here = tid < n && larger + (double)(ties + 1) * (double)v0 > target &&
-                          !(larger + (double)ties * (double)v0 > target) && v0 > 0.f;
-        __syncthreads();
-        if (tid == 0) sm.found = 0;
-        __syncthreads();
-        if (here) {
-            sm.key = __float_as_uint(v0);
-            sm.above = larger;
-            sm.rank = ties;
-            sm.found = 1;
+        int d = lowest(mass > target, sm.top[turn ^= 1]);
+        if (d < 0 && must) {
+            d = n - 1;
+#pragma unroll 1
+            while (d >= 0 && !(sm.ord_val[d] > 0.f)) --d;
         }
-        __syncthreads();
-        return sm.found ? SelectOut{sm.key, sm.above, sm.rank, true} : SelectOut{0u, 0.0, 0, false};
+        if (d < 0) return SelectOut{0u, 0.0, 0, false};
+        return SelectOut{__float_as_uint(sm.ord_val[d]), sm.ord_mass[d], sm.ord_at[d], true};
     };
 
     // nucleus cut-off.  In exact arithmetic the kept prefix ends at k, the first position whose
@@ -541,13 +558,13 @@ __global__ void __launch_bounds__(kSampleThreads) k_tp_select(int V, float top_p
 #pragma unroll 1
     for (int what = M.crossed ? CUT : DRAW;;) {
         // DRAW: first position whose inclusive mass exceeds r = u * Z (r < Z, so it is <= k*)
-        got = select(what == CUT ? (double)top_p : what == MORE ? Z : uu * Z);
+        got = select(what == CUT ? (double)top_p : what == MORE ? Z : uu * Z, what == CUT || (what == DRAW && !cut.crossed));
         if (what == DRAW) break;
         const int was = what;
         what = DRAW;
         if (got.crossed) {
             const float v = __uint_as_float(got.key);
-            const double C = got.above + (double)(got.rank + 1) * (double)v;
+            const double C = got.mass;
             const bool dropped = ref_dropped(C, v);
             if (was == CUT) {
                 cut = got;
@@ -567,17 +584,7 @@ __global__ void __launch_bounds__(kSampleThreads) k_tp_select(int V, float top_p
 #pragma unroll 1
     for (int k = got.crossed ? 0 : 1; k < 2 && pos < 0; ++k) {  // the cut-off's token: rounding at the very end
         const SelectOut& q = k == 0 ? got : cut;
-        if (!q.crossed) continue;
-        if (!ranked) {
-            pos = nth_equal(value, n, NT, q.key, q.rank, sm);
-            continue;
-        }
-        __syncthreads();
-        if (tid == 0) sm.found = -1;
-        __syncthreads();
-        if (tid < n && __float_as_uint(v0) == q.key && ties == q.rank) sm.found = tid;
-        __syncthreads();
-        pos = sm.found;
+        if (q.crossed) pos = ranked ? q.rank : nth_equal(value, n, NT, q.key, q.rank, sm);
     }
     if (tid == 0) {
         out[row] = pos >= 0 ? ci[pos] : 0;
