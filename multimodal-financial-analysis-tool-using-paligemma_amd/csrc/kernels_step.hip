@@ -665,9 +665,10 @@ __global__ void __launch_bounds__(256) k_skinny(GemvRtArgs a) {
         wp[m] = a.W + ((long)m * a.N + n) * a.ldw;
     }
     const T* xp = reinterpret_cast<const T*>(a.x) + (long)(li < a.B ? li : a.B - 1) * a.ldx;
-    f32x4 acc[NM];
+    f32x4 acc[NM], sum[NM];
 #pragma unroll
-    for (int m = 0; m < NM; ++m) acc[m] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int m = 0; m < NM; ++m) sum[m] = acc[m] = f32x4{0.f, 0.f, 0.f, 0.f};
+    int turn = 0;
     const int nstep = (K + 63) / 64;
     const int per = (nstep + gridDim.y - 1) / gridDim.y, s_end = min(nstep, (int)(blockIdx.y + 1) * per);
     for (int s0 = blockIdx.y * per + wave; s0 < s_end; s0 += 4 * U) {
@@ -702,11 +703,18 @@ __global__ void __launch_bounds__(256) k_skinny(GemvRtArgs a) {
                         acc[m] = mfma16(__builtin_bit_cast(short8, w[i][m][h]), __builtin_bit_cast(short8, x[i][h].q), acc[m]);
                 }
             }
+        if (F32 && (++turn & 3) == 0) {  // 1024 of k, as tile_f32 (of K = 16384, positive: 3.6e-6 without, an FMA chain 2.0e-6)
+#pragma unroll
+            for (int m = 0; m < NM; ++m) {
+                sum[m] += acc[m];
+                acc[m] = f32x4{0.f, 0.f, 0.f, 0.f};
+            }
+        }
     }
 #pragma unroll
     for (int m = 0; m < NM; ++m)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) sums[wave][m][4 * lg + r][li] = acc[m][r];
+        for (int r = 0; r < 4; ++r) sums[wave][m][4 * lg + r][li] = F32 ? sum[m][r] + acc[m][r] : acc[m][r];
     __syncthreads();
     const int b = tid & 15, n = n0 + (tid >> 4);
     float v[3] = {0.f, 0.f, 0.f};

@@ -6,9 +6,10 @@ import numpy as np
 import pytest
 import torch
 
+import decoder_cases as C
 import raritar_cases as R
 from decoder_helpers import build, close, tokens
-from oracle import raritar_np
+from oracle import decoder_np, raritar_np
 
 pytestmark = pytest.mark.gpu
 
@@ -101,3 +102,29 @@ def test_decode_rows(rows):
     for t in range(4):
         lg = eng.step(cache, slots, [[s[t]] for s in seqs])
         close(lg[:6], np.stack([w[t] for w in want]), "float32")
+
+
+@pytest.mark.parametrize("B", [3, 16])
+@pytest.mark.parametrize("K", [2048, 8192, 16384])
+def test_long_sums_of_few_rows(K, B):
+    """The output matrix over K positive terms, where sums drift the most: no further from float64 than a chain of fused
+    multiply-adds, which rounds K times."""
+    cfg = C.model([C.gru(8)], width=K, vocab=64, streams=1, groups=1, escale=1.0)
+    W = decoder_np.random_weights(cfg, 3)
+    E = np.random.default_rng(K).random((64, K), dtype=np.float32) * np.float32(0.9) + np.float32(0.1)
+    W["embed"] = (E.view(np.uint32) & np.uint32(0xFFFF0000)).view(np.float32)
+    for n in W:
+        if n.startswith("l0.hc") or "norm" in n:
+            W[n] = np.ones_like(W[n])
+    W["l0.mix.o"] = np.zeros_like(W["l0.mix.o"])  # the residual stays the token's embedding
+    eng, _ = build(cfg, "float32", weights=W, max_batch=16)
+    cache = eng.new_cache(B, 4)
+    got = eng.decode(cache, [cache.alloc() for _ in range(B)], torch.arange(B, device="cuda")).double().cpu().numpy()
+    E = W["embed"].astype(np.float64)
+    h = E[:B] / np.sqrt((E[:B] ** 2).mean(-1, keepdims=True) + cfg["norm"]["eps"])
+    want, chain = h @ E.T, np.zeros((B, 64), np.float32)
+    h = h.astype(np.float32).astype(np.float64)
+    for k in range(K):
+        chain = (chain + h[:, k, None] * E[None, :, k]).astype(np.float32)
+    err = lambda x: np.sqrt(((x - want) ** 2).mean())
+    assert err(got) <= err(chain.astype(np.float64)), (err(got) / want.mean(), err(chain) / want.mean())
