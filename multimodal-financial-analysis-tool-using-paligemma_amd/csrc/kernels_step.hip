@@ -651,7 +651,7 @@ void run_mode(hipStream_t s, GemvRtMode mode, const GemvRtArgs& a) {
 // L2, B fragments) use the same order.  After the waves' sums meet in LDS, thread (n, b) runs the step's epilogue.
 // GR_F32 with gridDim.y > 1: K is cut over the y workgroups too, out holds their partial slabs [y][B][N].
 template <typename T, int MODE>
-__global__ void __launch_bounds__(256) k_skinny(GemvRtArgs a) {
+__global__ void __launch_bounds__(256, sizeof(T) == 4 && MODE != GR_GRU && MODE != GR_SWIGLU ? 4 : 1) k_skinny(GemvRtArgs a) {
     constexpr int NM = MODE == GR_GRU ? 3 : MODE == GR_SWIGLU ? 2 : 1;
     constexpr bool F32 = std::is_same<T, float>::value;
     constexpr int U = NM == 1 && !F32 ? 8 : 4;  // 64-deep steps in flight
@@ -723,12 +723,41 @@ __global__ void __launch_bounds__(256) k_skinny(GemvRtArgs a) {
 #pragma unroll
         for (int q = 0; q < 4; ++q) v[m] += sums[q][m][tid >> 4][b];
     if constexpr (F32) {
-        // what is not finite (of rows and outputs that there are): the FMA chain over this workgroup's K slice
-        if (b < a.B && n < a.N)
-            for (int m = 0; m < NM; ++m)
-                if (not_finite(v[m]))
-                    v[m] = dot_f32(reinterpret_cast<const float*>(a.x) + (long)b * a.ldx, a.W + ((long)m * a.N + n) * a.ldw,
-                                   blockIdx.y * per * 64, min(K, s_end * 64));
+        // what is not finite (of rows and outputs that there are): FMA chains over this workgroup's K slice, as tile_f32
+        __shared__ int flag[4];
+        bool bad = false;
+#pragma unroll
+        for (int m = 0; m < NM; ++m) bad |= b < a.B && n < a.N && not_finite(v[m]);
+        const bool wave_bad = __any(bad);
+        if (lane == 0) flag[wave] = wave_bad;
+        __syncthreads();
+        if (flag[0] | flag[1] | flag[2] | flag[3]) {
+            constexpr int FK = 32, ST = FK + 1;
+            static_assert((1 + NM) * 16 * ST <= 4 * NM * 16 * 17, "the chains' operands fit");
+            float *xs = &sums[0][0][0][0], *ws = xs + 16 * ST;  // [row][k], [matrix and output][k]
+            float c[NM] = {};
+            const int k1 = min(K, s_end * 64);
+#pragma clang loop unroll(disable)
+            for (int k = blockIdx.y * per * 64; k < k1; k += FK) {
+                const int nk = min(FK, k1 - k);
+                __syncthreads();
+#pragma clang loop unroll(disable)
+                for (int i = tid; i < (1 + NM) * 16 * FK; i += 256) {
+                    const int r = i / FK, q = i % FK, kk = k + min(q, nk - 1);
+                    if (r < 16) xs[r * ST + q] = reinterpret_cast<const float*>(a.x)[(long)min(r, a.B - 1) * a.ldx + kk];
+                    else ws[(r - 16) * ST + q] = bf2f(a.W[((long)(r / 16 - 1) * a.N + min(n0 + r % 16, a.N - 1)) * a.ldw + kk]);
+                }
+                __syncthreads();
+#pragma clang loop unroll(disable)
+                for (int q0 = 0; q0 < nk; q0 += 8)  // (K is a multiple of 8)
+#pragma unroll
+                    for (int q = q0; q < q0 + 8; ++q)
+#pragma unroll
+                        for (int m = 0; m < NM; ++m) c[m] = fmaf(xs[b * ST + q], ws[(m * 16 + (tid >> 4)) * ST + q], c[m]);
+            }
+#pragma unroll
+            for (int m = 0; m < NM; ++m) v[m] = not_finite(v[m]) ? c[m] : v[m];
+        }
     }
     if constexpr (MODE == GR_F32) {
         if (b < a.B && n < a.N)
@@ -743,6 +772,7 @@ __global__ void __launch_bounds__(256) k_skinny(GemvRtArgs a) {
 // a group moves besides its weights is otherwise as many bytes of activations from L2 (8 rows: the output matrix of 257,216 x
 // 2048 207 us, held 185; gate|up of 16,384 channels 32.0 / 25.7).  The next group's weights are asked for before this one's
 // sums meet, the last group peeled off.  (fp32 rows, three pieces each, would take 200 registers.)
+__device__ const uint16_t kZeros[8] __attribute__((aligned(16))) = {};  // weights past the end
 template <int MODE>
 __global__ void __launch_bounds__(256) k_skinny_held(GemvRtArgs a) {
     constexpr int NM = MODE == GR_SWIGLU ? 2 : 1, ST = 8;  // 64-deep steps of a wave
@@ -769,7 +799,7 @@ __global__ void __launch_bounds__(256) k_skinny_held(GemvRtArgs a) {
 #pragma unroll
                 for (int h = 0; h < 2; ++h) {
                     const int k = (wave + 4 * i) * 64 + lg * 16 + 8 * h;
-                    w[i][m][h] = ldg16(k < K ? p + k : p);  // past the end: the activations are zero
+                    w[i][m][h] = ldg16(k < K ? p + k : kZeros);
                 }
         }
     };
@@ -800,16 +830,6 @@ __global__ void __launch_bounds__(256) k_skinny_held(GemvRtArgs a) {
             for (int q = 0; q < 4; ++q) v[m] += sums[turn][q][m][tid & 15][b];
         turn ^= 1;
         if (b >= a.B || n >= a.N) return;
-        if (K < 2048) {  // past K a zero has met the row's first weights: formed again where one of them is not finite
-#pragma unroll
-            for (int m = 0; m < NM; ++m)
-                if (not_finite(v[m])) {
-                    const uint16_t* p = a.W + ((long)m * a.N + n) * a.ldw;
-                    v[m] = 0.0f;
-#pragma clang loop unroll(disable)
-                    for (int k = 0; k < K; ++k) v[m] = fmaf(bf2f(reinterpret_cast<const uint16_t*>(a.x)[(long)b * a.ldx + k]), bf2f(p[k]), v[m]);
-                }
-        }
         if constexpr (MODE == GR_F32) reinterpret_cast<float*>(a.out)[(long)b * a.ldo + n] = v[0];
         else step_epilogue<uint16_t, MODE>(a, n, b, v[0], v[1], 0.f);
     };
