@@ -220,6 +220,10 @@ __global__ void __launch_bounds__(256) k_scan(ScanArgs a) {
         A[i] = n < N ? -expf(bf2f(al[i])) * 1.4426950408889634f : 0.0f;
         if (!entry || n >= N) S[i] = 0.0f;
     }
+    // this lane's staged states, as whole vectors: indexed by single states the compiler read them in halves where lanes share a
+    // channel ((C) of 1,540 rows of 2,048 channels of 256 states 709 us, so 410)
+    const f32x4* lB = reinterpret_cast<const f32x4*>(&sB[0][0]) + sub * (NPL / 4);
+    const f32x4* lC = reinterpret_cast<const f32x4*>(&sC[0][0]) + sub * (NPL / 4);
     for (int t0 = 0; t0 < ck.len; t0 += kSub) {
         const int nt = min(kSub, ck.len - t0);
         __syncthreads();
@@ -258,17 +262,17 @@ __global__ void __launch_bounds__(256) k_scan(ScanArgs a) {
                     float y = 0.0f;
 #pragma unroll
                     for (int i = 0; i < NPL; i += 4) {
-                        const float4 B = *reinterpret_cast<const float4*>(&sB[tb + t][n0 + i]);
-                        S[i] = fmaf(__builtin_amdgcn_exp2f(dt[t] * A[i]), S[i], dx * B.x);
-                        S[i + 1] = fmaf(__builtin_amdgcn_exp2f(dt[t] * A[i + 1]), S[i + 1], dx * B.y);
-                        S[i + 2] = fmaf(__builtin_amdgcn_exp2f(dt[t] * A[i + 2]), S[i + 2], dx * B.z);
-                        S[i + 3] = fmaf(__builtin_amdgcn_exp2f(dt[t] * A[i + 3]), S[i + 3], dx * B.w);
+                        const f32x4 B = lB[(tb + t) * (NP / 4) + i / 4];
+                        S[i] = fmaf(__builtin_amdgcn_exp2f(dt[t] * A[i]), S[i], dx * B[0]);
+                        S[i + 1] = fmaf(__builtin_amdgcn_exp2f(dt[t] * A[i + 1]), S[i + 1], dx * B[1]);
+                        S[i + 2] = fmaf(__builtin_amdgcn_exp2f(dt[t] * A[i + 2]), S[i + 2], dx * B[2]);
+                        S[i + 3] = fmaf(__builtin_amdgcn_exp2f(dt[t] * A[i + 3]), S[i + 3], dx * B[3]);
                         if constexpr (PHASE == 1) {
-                            const float4 Cv = *reinterpret_cast<const float4*>(&sC[tb + t][n0 + i]);
-                            y = fmaf(S[i], Cv.x, y);
-                            y = fmaf(S[i + 1], Cv.y, y);
-                            y = fmaf(S[i + 2], Cv.z, y);
-                            y = fmaf(S[i + 3], Cv.w, y);
+                            const f32x4 Cv = lC[(tb + t) * (NP / 4) + i / 4];
+                            y = fmaf(S[i], Cv[0], y);
+                            y = fmaf(S[i + 1], Cv[1], y);
+                            y = fmaf(S[i + 2], Cv[2], y);
+                            y = fmaf(S[i + 3], Cv[3], y);
                         }
                     }
                     if constexpr (PHASE == 1) {

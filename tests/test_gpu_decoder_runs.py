@@ -30,3 +30,20 @@ def test_together_as_alone(name, n, length):
         for got, want in ((together[r], alone[0]), (after[r], nxt[0])):
             rms = want.double().square().mean().sqrt()
             assert torch.isfinite(got).all() and (got - want).double().abs().max() <= 2e-4 * rms
+
+
+def test_time_goes_by_the_states():
+    """1,540 rows of 2,048 channels: 256 states are twice the work of 128, in the same kernel."""
+    times = []
+    for states in (128, 256):
+        eng, _ = build(C.model([C.mamba(2048, states, 8, 4)] * 4, width=64, vocab=64, streams=1, groups=1), "bfloat16")
+        cache = eng.new_cache(1, 2048)
+        slot, toks = cache.alloc(), torch.arange(1540, device="cuda") % 64
+        ev = [torch.cuda.Event(enable_timing=True) for _ in range(9)]
+        for e in ev:
+            cache.length[slot] = 0
+            eng.forward(cache, [slot], toks, [1540])
+            e.record()
+        torch.cuda.synchronize()
+        times.append(min(a.elapsed_time(b) for a, b in zip(ev, ev[1:])))
+    assert times[1] <= 2.5 * times[0]
