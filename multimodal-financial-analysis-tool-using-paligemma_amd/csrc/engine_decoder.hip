@@ -2,10 +2,10 @@
 // mixer and an optional feed-forward, around residual streams or one plain residual.  Weight layout, derived
 // tensors, the per-sequence state slab, the ragged forward (prompts and portions of prompts) and the decode step
 // (hipGraph-replayed), over the mechanisms of decoder.h.  A design is its layer list and constants; nothing here names one.
-#include <climits>
 #include <set>
 
 #include "decoder.h"
+#include "runs.h"
 #include "engine.h"
 
 namespace {
@@ -1027,41 +1027,14 @@ int pgmi_decoder_forward(pgmi_ctx* x, const int64_t* ids, int n_seq, const int32
         }
         return c;
     };
-    // A short step's few runs are walked by a few CUs, each row waiting for the one before; where the chip is full short runs
-    // only add carries.  The scan (workgroups of 256 channels, a wave per SIMD) takes the run length whose rounds of 256
-    // workgroups walk the fewest rows, a workgroup's start costing about 8.  us of its three launches, 64- / 16-row runs: 500
-    // rows of 2,048 channels 86 / 41, 300 rows 69 / 35; 64 rows / this rule: 1,540 rows of 4,096 channels (50-row runs) 98 / 92.
-    auto scan_rows = [&](int width) {
-        const long cols = std::max(1, (width + 255) / 256);
-        int best = 64;
-        long least = LONG_MAX;
-        for (int ct = 64; ct >= 16; ct -= 2) {
-            long n = 0;
-            for (int r = 0; r < n_seq; ++r) n += (lens[r] + ct - 1) / ct;
-            const long cost = (n * cols + 255) / 256 * (ct + 8);
-            if (cost < least) { least = cost; best = ct; }
-        }
-        return best;
-    };
-    // minGRU: the longest runs, down to 8 rows, that still give every CU a workgroup of 128 channels
-    auto gru_rows = [&](int width) {
-        const long cols = std::max(1, (width + 127) / 128);
-        int ct = 32;
-        for (const int k : {32, 24, 16, 8}) {
-            ct = k;
-            long n = 0;
-            for (int r = 0; r < n_seq; ++r) n += (lens[r] + ct - 1) / ct;
-            if (n * cols >= 256) break;
-        }
-        return ct;
-    };
-    int scan_width = 1, gru_width = 1;
+    long scan_cols = 1, gru_cols = 1;
     for (const pgmi_layer_spec& l : d.L) {
-        if (l.mixer == PGMI_MIXER_MAMBA1) scan_width = std::max(scan_width, l.inner);
-        if (l.mixer == PGMI_MIXER_MINGRU) gru_width = std::max(gru_width, l.width);
+        if (l.mixer == PGMI_MIXER_MAMBA1) scan_cols = std::max(scan_cols, scan_columns(l.inner, l.state));
+        if (l.mixer == PGMI_MIXER_MINGRU) gru_cols = std::max(gru_cols, gru_columns(l.width));
     }
     const bool huge = rows > 16384;
-    const Cut scan = cut(huge ? 256 : scan_rows(scan_width)), gru = cut(huge ? 128 : gru_rows(gru_width));
+    const Cut scan = cut(huge ? 256 : scan_run_rows(lens, n_seq, scan_cols)),
+              gru = cut(huge ? 128 : gru_run_rows(lens, n_seq, gru_cols));
     // the convolutions carry nothing: 500 rows of 2,048 channels 11.2 us on 64-row runs, 5.9 on 16; 2,048 rows 10.8 / 7.5
     const Cut conv = cut(huge ? 256 : rows > 2048 ? 32 : 16);
     struct Tiles { int R; size_t o; int n; };

@@ -10,6 +10,7 @@
 
 #include "act.h"
 #include "decoder.h"
+#include "runs.h"
 
 namespace pgmi {
 
@@ -343,12 +344,16 @@ void launch_scan(hipStream_t s, const ScanArgs& a) {
 
 template <typename T>
 void scan_t(hipStream_t s, const ScanArgs& a) {
-    if (a.N <= 8) launch_scan<T, 8, 1>(s, a);
-    else if (a.N <= 16) launch_scan<T, 16, 1>(s, a);
-    else if (a.N <= 32) launch_scan<T, 16, 2>(s, a);
-    else if (a.N <= 64) launch_scan<T, 16, 4>(s, a);
-    else if (a.N <= 128) launch_scan<T, 16, 8>(s, a);
-    else launch_scan<T, 16, 16>(s, a);
+    switch (scan_lanes(a.N)) {
+        case 1:
+            if (a.N <= 8) launch_scan<T, 8, 1>(s, a);
+            else launch_scan<T, 16, 1>(s, a);
+            break;
+        case 2: launch_scan<T, 16, 2>(s, a); break;
+        case 4: launch_scan<T, 16, 4>(s, a); break;
+        case 8: launch_scan<T, 16, 8>(s, a); break;
+        default: launch_scan<T, 16, 16>(s, a); break;
+    }
 }
 
 // ---------------------------------------------------------------- minGRU

@@ -1,0 +1,52 @@
+// runs.h -- how many rows of a sequence one workgroup of a recurrence walks (host code, without HIP).
+//
+// A short step's few runs are walked by a few CUs, each row waiting for the one before; where the chip is full short runs only
+// add carries.
+#pragma once
+#include <algorithm>
+#include <climits>
+#include <cstdint>
+
+namespace pgmi {
+
+constexpr int kRunCUs = 256;
+
+// lanes of a scan workgroup of 256 that share a channel of N states
+constexpr int scan_lanes(int N) { return N <= 16 ? 1 : N <= 32 ? 2 : N <= 64 ? 4 : N <= 128 ? 8 : 16; }
+// What a run of C channels takes of a round of kRunCUs: 256 channels of one lane each, and as much of two and four, which wait on
+// each other's sums and leave room for as many more workgroups; 8 and 16 lanes fill the chip two and four times as fast.
+// Measured, 2,048 channels, us a layer by run lengths 64 / 32 / 16: 500 rows of 64 states 114 / 95 / 93, of 128 144 / 138 / 140, of 256
+// 261 / 267 / 288; 1,540 rows 172 / 171 / 180, 282 / 286 / 308, 655 / 682 / 758.
+constexpr long scan_columns(int C, int N) { return ((long)C + 255) / 256 * std::max(1, scan_lanes(N) / 4); }
+constexpr long gru_columns(int C) { return ((long)C + 127) / 128; }
+
+inline long runs_of(const int32_t* lens, int n_seq, int rows) {
+    long n = 0;
+    for (int r = 0; r < n_seq; ++r) n += (lens[r] + rows - 1) / rows;
+    return n;
+}
+
+// The scan takes the length whose rounds walk the fewest rows, a workgroup's start costing about 8.  us of its three launches,
+// 64- / 16-row runs: 500 rows of 2,048 channels of 16 states 86 / 41, 300 rows 69 / 35; 64 rows / this rule: 1,540 rows of 4,096
+// channels (50-row runs) 98 / 92.  columns: of the layer with the most.
+inline int scan_run_rows(const int32_t* lens, int n_seq, long columns) {
+    int best = 64;
+    long least = LONG_MAX;
+    for (int ct = 64; ct >= 16; ct -= 2) {
+        const long cost = (runs_of(lens, n_seq, ct) * columns + kRunCUs - 1) / kRunCUs * (ct + 8);
+        if (cost < least) { least = cost; best = ct; }
+    }
+    return best;
+}
+
+// minGRU: the longest runs, down to 8 rows, that still give every CU a workgroup of 128 channels
+inline int gru_run_rows(const int32_t* lens, int n_seq, long columns) {
+    int ct = 32;
+    for (const int k : {32, 24, 16, 8}) {
+        ct = k;
+        if (runs_of(lens, n_seq, ct) * columns >= kRunCUs) break;
+    }
+    return ct;
+}
+
+}  // namespace pgmi

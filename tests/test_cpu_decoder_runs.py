@@ -1,0 +1,49 @@
+"""The run lengths of the recurrences (csrc/runs.h), which are host code without HIP: compiled here and asked for steps whose
+best lengths were measured."""
+import os
+import subprocess
+
+import pytest
+
+CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))),
+                    "multimodal-financial-analysis-tool-using-paligemma_amd", "csrc")
+ASK = r"""
+#include <cstdio>
+#include <cstdlib>
+#include <vector>
+#include "runs.h"
+int main(int n, char** v) {  // channels, states, lengths
+    std::vector<int32_t> lens;
+    for (int i = 3; i < n; ++i) lens.push_back(atoi(v[i]));
+    const int C = atoi(v[1]), N = atoi(v[2]);
+    std::printf("%d %d\n", pgmi::scan_run_rows(lens.data(), (int)lens.size(), pgmi::scan_columns(C, N)),
+                pgmi::gru_run_rows(lens.data(), (int)lens.size(), pgmi::gru_columns(C)));
+}
+"""
+
+
+@pytest.fixture(scope="module")
+def ask(tmp_path_factory):
+    at = tmp_path_factory.mktemp("runs")
+    (at / "ask.cpp").write_text(ASK)
+    subprocess.run(["g++", "-std=c++17", "-Wall", "-Werror", "-I", CSRC, str(at / "ask.cpp"), "-o", str(at / "ask")], check=True)
+    return lambda *a: [int(x) for x in subprocess.run([str(at / "ask"), *map(str, a)], check=True, capture_output=True,
+                                                      text=True).stdout.split()]
+
+
+# channels, states, lengths; the shortest and longest run length of those within 4 % of the best measured
+@pytest.mark.parametrize("C,N,lens,least,most", [
+    (2048, 16, [200], 16, 16), (2048, 16, [500], 16, 16), (2048, 16, [1000], 16, 32), (2048, 16, [4000], 32, 64),
+    (4096, 16, [1024, 387, 129], 48, 64), (2048, 32, [500], 16, 16), (2048, 32, [1000], 16, 32), (2048, 32, [4000], 32, 64),
+    (2048, 64, [500], 16, 32), (2048, 64, [1000], 16, 64), (2048, 64, [4000], 32, 64), (4096, 64, [1540], 32, 64),
+    (2048, 128, [200], 16, 24), (2048, 128, [500], 16, 64), (2048, 128, [1540], 48, 64), (2048, 128, [4000], 32, 64),
+    (2048, 256, [500], 60, 64), (2048, 256, [1000], 48, 64), (2048, 256, [1540], 48, 64), (2048, 256, [4000], 48, 64),
+    (2048, 256, [500, 300, 100, 60], 56, 64)])
+def test_scan(ask, C, N, lens, least, most):
+    assert least <= ask(C, N, *lens)[0] <= most
+
+
+@pytest.mark.parametrize("C,lens,rows", [(2048, [1024], 32), (2048, [500], 32), (2048, [370], 24), (2048, [300], 16), (2048, [100], 8), (128, [9000], 32),
+                                         (128, [7000], 24), (128, [100, 3], 8)])
+def test_gru(ask, C, lens, rows):
+    assert ask(C, 16, *lens)[1] == rows
