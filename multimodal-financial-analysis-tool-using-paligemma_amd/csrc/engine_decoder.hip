@@ -58,9 +58,13 @@ struct DecoderState {
     const uint16_t *embed = nullptr, *fnorm = nullptr, *pairs = nullptr;
     Lin head;
     std::vector<void*> derived;  // padded weights, joined biases
-    // workspace of `rows` rows, `chunks` scan chunks and `gchunks` chunks of the gated recurrence
-    int rows = 0, chunks = 0, gchunks = 0;
+    // workspace of `rows` rows
+    int rows = 0;
     void* arena = nullptr;
+    // the recurrences' carries between runs.  A buffer of its own: how many runs a step has does not go by its rows alone, and no
+    // captured step reads it
+    float* carries = nullptr;
+    size_t carry_floats = 0;
     float *X = nullptr, *slabs = nullptr, *dt = nullptr, *bc = nullptr, *cstate = nullptr, *csum = nullptr;
     uint8_t *h = nullptr, *p0 = nullptr, *p1 = nullptr, *p2 = nullptr, *dtl = nullptr;
     // mixture of experts: activations and outputs per entry, choices, weights, gates, lists, counters, used experts
@@ -364,26 +368,23 @@ void decoder_release(pgmi_ctx* x) {
     DecoderState* d = x->dec;
     if (!d) return;
     drop_derived(*d);
-    for (void* p : {d->arena, d->meta, (void*)d->part})
+    for (void* p : {d->arena, d->meta, (void*)d->part, (void*)d->carries})
         if (p) (void)hipFree(p);
     delete d;
     x->dec = nullptr;
 }
 
-// Grow the workspace to these rows and chunks (captured graphs hold its addresses)
-int ensure_workspace(pgmi_ctx* x, int rows, int chunks, int gchunks) {
+// Grow the workspace to these rows (captured graphs hold its addresses)
+int ensure_workspace(pgmi_ctx* x, int rows) {
     DecoderState& d = *x->dec;
-    if (rows <= d.rows && chunks <= d.chunks && gchunks <= d.gchunks) return 0;
-    rows = std::max(rows, d.rows);
-    chunks = std::max(chunks, d.chunks);
-    gchunks = std::max(gchunks, d.gchunks);
+    if (rows <= d.rows) return 0;
     HIPCHK(hipDeviceSynchronize());
     clear_dgraphs(x);
     if (d.arena) (void)hipFree(d.arena);
     d.arena = nullptr;
-    d.rows = d.chunks = d.gchunks = 0;
+    d.rows = 0;
     const int D = d.c.width;
-    int l0 = r8(D), l1 = 8, l2 = 8, ldd = 8, slab_n = D, inner = 1, bcn = 2, cs = 1, cg = 1;
+    int l0 = r8(D), l1 = 8, l2 = 8, ldd = 8, slab_n = D, inner = 1, bcn = 2;
     int lea = 8, top = 0, ne = 0;  // mixtures: expert activations, choices per row, experts
     for (const pgmi_layer_spec& l : d.L) {
         if (l.mixer == PGMI_MIXER_MAMBA1) {
@@ -394,7 +395,6 @@ int ensure_workspace(pgmi_ctx* x, int rows, int chunks, int gchunks) {
             slab_n = std::max(slab_n, l.dt_rank + 2 * l.state);
             inner = std::max(inner, l.inner);
             bcn = std::max(bcn, 2 * l.state);
-            cs = std::max(cs, l.inner * l.state);
         } else if (l.mixer == PGMI_MIXER_ATTENTION) {
             l0 = std::max(l0, r8(qkv_rows(l)));
             l1 = std::max(l1, l.heads * r8(l.dim));
@@ -402,7 +402,6 @@ int ensure_workspace(pgmi_ctx* x, int rows, int chunks, int gchunks) {
         } else {
             l0 = std::max(l0, r8(3 * l.width));
             l2 = std::max(l2, r8(l.width));
-            cg = std::max(cg, l.width);
         }
         l2 = std::max(l2, r8(l.experts ? l.shared_ff : l.ff));
         if (l.experts) {
@@ -419,7 +418,6 @@ int ensure_workspace(pgmi_ctx* x, int rows, int chunks, int gchunks) {
     const size_t sizes[] = {(size_t)rows * d.c.streams * D * 4, (size_t)rows * d.ldh * d.es, (size_t)rows * l0 * d.es,
                             (size_t)rows * l1 * d.es,           (size_t)rows * l2 * d.es,    (size_t)rows * ldd * d.es,
                             d.slab_bytes,                       (size_t)rows * inner * 4,    (size_t)rows * bcn * 4,
-                            std::max((size_t)chunks * cs, (size_t)gchunks * 2 * cg) * 4, (size_t)chunks * inner * 4,
                             ent * lea * d.es, ent * d.ldh * d.es, ent * 4, ent * 4, (size_t)rows * 4, (size_t)rows * 4,
                             (size_t)rows * ne * 4, (size_t)(2 * ne + 2) * 4};
     constexpr int NB = sizeof(sizes) / sizeof(sizes[0]);
@@ -439,20 +437,47 @@ int ensure_workspace(pgmi_ctx* x, int rows, int chunks, int gchunks) {
     d.slabs = reinterpret_cast<float*>(p + off[6]);
     d.dt = reinterpret_cast<float*>(p + off[7]);
     d.bc = reinterpret_cast<float*>(p + off[8]);
-    d.cstate = reinterpret_cast<float*>(p + off[9]);
-    d.csum = reinterpret_cast<float*>(p + off[10]);
-    d.ea = p + off[11]; d.ey = p + off[12];
-    d.esel = reinterpret_cast<int*>(p + off[13]);
-    d.ew = reinterpret_cast<float*>(p + off[14]);
-    d.egate = reinterpret_cast<float*>(p + off[15]);
-    d.inv = reinterpret_cast<float*>(p + off[16]);
-    d.elist = reinterpret_cast<int*>(p + off[17]);
-    d.ecnt = reinterpret_cast<int*>(p + off[18]);
+    d.ea = p + off[9]; d.ey = p + off[10];
+    d.esel = reinterpret_cast<int*>(p + off[11]);
+    d.ew = reinterpret_cast<float*>(p + off[12]);
+    d.egate = reinterpret_cast<float*>(p + off[13]);
+    d.inv = reinterpret_cast<float*>(p + off[14]);
+    d.elist = reinterpret_cast<int*>(p + off[15]);
+    d.ecnt = reinterpret_cast<int*>(p + off[16]);
     d.eactive = d.ecnt + ne;
     d.zero_words = ne + 1;
     d.rows = rows;
-    d.chunks = chunks;
-    d.gchunks = gchunks;
+    return 0;
+}
+
+// The carries of a step with these runs of the scan and of the gated recurrence; grown by half as much again, for steps of other
+// lengths
+int ensure_carries(DecoderState& d, int scan_runs, int gru_runs) {
+    size_t state = 0, sums = 0;
+    for (const pgmi_layer_spec& l : d.L) {
+        if (l.mixer == PGMI_MIXER_MAMBA1) {
+            state = std::max(state, (size_t)scan_runs * l.inner * l.state);
+            sums = std::max(sums, (size_t)scan_runs * l.inner);
+        } else if (l.mixer == PGMI_MIXER_MINGRU) {
+            state = std::max(state, (size_t)gru_runs * 2 * l.width);
+        }
+    }
+    state = (state + 63) / 64 * 64;
+    if (state + sums > d.carry_floats) {
+        HIPCHK(hipDeviceSynchronize());
+        if (d.carries) (void)hipFree(d.carries);
+        d.carries = nullptr;
+        d.carry_floats = 0;
+        const size_t n = state + sums + (state + sums) / 2;
+        if (hipMalloc(reinterpret_cast<void**>(&d.carries), n * 4) != hipSuccess) {
+            (void)hipGetLastError();
+            d.carries = nullptr;
+            return fail(PGMI_E_NOMEM, "carries of " + std::to_string(n * 4) + " bytes");
+        }
+        d.carry_floats = n;
+    }
+    d.cstate = d.carries;
+    d.csum = d.carries + state;
     return 0;
 }
 
@@ -1054,7 +1079,7 @@ int pgmi_decoder_forward(pgmi_ctx* x, const int64_t* ids, int n_seq, const int32
     for (int r = 0; r < n_seq; ++r) m.insert(m.end(), lens[r], r);
     const size_t o_want = m.size();
     m.insert(m.end(), want, want + n_want);
-    if ((rc = ensure_workspace(x, std::max(rows, n_want), scan.n, gru.n))) return rc;
+    if ((rc = ensure_workspace(x, std::max(rows, n_want))) || (rc = ensure_carries(d, scan.n, gru.n))) return rc;
     if (m.size() * 4 > d.meta_bytes) {
         HIPCHK(hipDeviceSynchronize());
         if (d.meta) (void)hipFree(d.meta);
@@ -1095,7 +1120,7 @@ int pgmi_decoder_decode(pgmi_ctx* x, const int64_t* ids, int B, const int32_t* s
         if (positions[b] < 0 || (long)positions[b] + n_steps > max_tokens) return fail(PGMI_E_ARG, "state capacity exceeded");
     HIPCHK(hipSetDevice(x->device));
     hipStream_t s = (hipStream_t)stream;
-    if ((rc = ensure_workspace(x, B, 1, 1))) return rc;
+    if ((rc = ensure_workspace(x, B))) return rc;
     size_t need = 0;
     for (const pgmi_layer_spec& l : d.L)
         if (l.mixer == PGMI_MIXER_ATTENTION)

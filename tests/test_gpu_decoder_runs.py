@@ -47,3 +47,36 @@ def test_time_goes_by_the_states():
         torch.cuda.synchronize()
         times.append(min(a.elapsed_time(b) for a, b in zip(ev, ev[1:])))
     assert times[1] <= 2.5 * times[0]
+
+
+def test_a_shorter_step_of_more_runs_allocates_nothing():
+    """9,081 rows of 4,096 channels go in 142 runs, 8,942 in 160: the workspace of the first holds the second."""
+    eng, _ = build(C.model([C.mamba(4096, 16, 8, 4)], width=64, vocab=64, streams=1, groups=1), "bfloat16")
+    cache = eng.new_cache(1, 9200)
+    slot, toks = cache.alloc(), torch.arange(9081, device="cuda") % 64
+    free = []
+    for n in (9081, 8942):
+        cache.length[slot] = 0
+        eng.forward(cache, [slot], toks[:n], [n])
+        torch.cuda.synchronize()
+        free.append(torch.cuda.mem_get_info()[0])
+    assert free[0] == free[1]
+
+
+def test_captured_steps_outlive_more_runs():
+    """A decode graph, then a packed step of as many rows in more runs, then the graph again: as eager steps."""
+    cfg = C.MIXED["a"]
+    eng, _ = build(cfg, "bfloat16", max_batch=64)
+    out = []
+    for graph in (True, False):
+        cache = eng.new_cache(41, 64)
+        one, logits = cache.alloc(), torch.empty((1, eng.vocab), device="cuda")
+        ids = torch.empty(1, dtype=torch.int64, device="cuda")
+        eng.forward(cache, [one], tokens(cfg, 40, 1), [40])
+        for k in range(6):  # the first eager, the second captured
+            ids.fill_(3 + k)
+            out.append(eng.decode(cache, [one], ids, logits=logits, graph=graph).clone())
+            if k == 2:
+                eng.forward(cache, [cache.alloc() for _ in range(40)], tokens(cfg, 40, 2), [1] * 40)
+    for a, b in zip(out[:6], out[6:]):
+        assert torch.isfinite(a).all() and torch.equal(a, b)
