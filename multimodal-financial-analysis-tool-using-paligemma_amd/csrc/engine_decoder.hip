@@ -1208,7 +1208,8 @@ int pgmi_op_matmul(pgmi_ctx* x, const void* A, int lda, const void* W, int ldw, 
     if (mode == RT_SWIGLU && act == PGMI_DTYPE_F32 && !scratch) return fail(PGMI_E_ARG, "fp32 gate|up needs scratch");
     const int sp = matmul_rt((hipStream_t)stream, act == PGMI_DTYPE_F32 ? ACT_F32 : ACT_BF16, A, lda,
                              reinterpret_cast<const uint16_t*>(W), ldw, M, N, K, (RtOut)mode,
-                             reinterpret_cast<const uint16_t*>(bias), out, ldo, (size_t)std::max<int64_t>(out_bytes, 0));
+                             reinterpret_cast<const uint16_t*>(bias), out, ldo,
+                             split ? (size_t)std::max<int64_t>(out_bytes, 0) : 0);
     if (split) *split = sp;
     LAUNCHCHK();
     return 0;

@@ -19,12 +19,13 @@ def eng():
     return build(R.MECHANISMS["taps_1"], "float32")[0]
 
 
-def product(eng, A, W, N, mode, out):
+def product(eng, A, W, N, mode, out, split=True):
     from pgmi import _native as N_
     M, K = A.shape
     sp, scratch = ctypes.c_int(), torch.empty((M, 2 * N), device="cuda")
-    N_.check(eng.lib.pgmi_op_matmul(eng.ctx, A.data_ptr(), A.stride(0), W.data_ptr(), W.stride(0), M, N, K, 2, mode, None,
-                                    out.data_ptr(), out.shape[-1], out.numel() * 4, scratch.data_ptr(), ctypes.byref(sp),
+    N_.check(eng.lib.pgmi_op_matmul(eng.ctx, A.data_ptr(), A.stride(0), W.data_ptr(), W.stride(0), M, N, K,
+                                    2 if A.dtype is torch.float32 else 0, mode, None, out.data_ptr(), out.shape[-1],
+                                    out.numel() * 4, scratch.data_ptr(), ctypes.byref(sp) if split else None,
                                     N_.stream_handle(eng.device)))
     return sp.value
 
@@ -52,6 +53,20 @@ def test_every_mode_against_float64(eng, M, N, K):
     # |d silu| <= 1.1 |d gate|; silu itself to a few ulp
     tol = 1.1 * bound[:, :N] * (ref[:, N:].abs() + bound[:, N:]) + ref[:, :N].abs() * bound[:, N:] + 1e-6 * want.abs() + 1e-30
     assert ((out[:, :N].double() - want).abs() <= tol).all() and (out[:, N:] == 0).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_slabs_for_a_caller_that_asks_for_no_split(eng, dtype):
+    """One slab, the whole product, though the output has room for more."""
+    g = torch.Generator("cuda").manual_seed(5)
+    A = torch.randn((40, 4096), device="cuda", generator=g).to(dtype)
+    W = torch.randn((64, 4096), device="cuda", generator=g).bfloat16()
+    out = torch.zeros((8, 40, 64), device="cuda")
+    assert product(eng, A, W, 64, 2, out) > 1
+    out.zero_()
+    product(eng, A, W, 64, 2, out, split=False)
+    ref = A.double() @ W.double().t()
+    assert (out[0].double() - ref).norm() <= 1e-5 * ref.norm() and not out[1:].any()
 
 
 @pytest.mark.parametrize("M,N", [(20, 70), (300, 4096)])
