@@ -55,6 +55,15 @@ def test_every_mode_against_float64(eng, M, N, K):
     assert ((out[:, :N].double() - want).abs() <= tol).all() and (out[:, N:] == 0).all()
 
 
+def test_gate_and_up_without_scratch(eng):
+    """Refused for fp32 rows, as include/pgmi.h has it."""
+    from pgmi import _native as N_
+    A, W, out = torch.ones((4, 8), device="cuda"), torch.ones((16, 8), device="cuda").bfloat16(), torch.zeros((4, 8), device="cuda")
+    status = eng.lib.pgmi_op_matmul(eng.ctx, A.data_ptr(), 8, W.data_ptr(), 8, 4, 8, 8, 2, 3, None, out.data_ptr(), 8, 128, None, None,
+                                    N_.stream_handle(eng.device))
+    assert status != 0 and not out.any()
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_slabs_for_a_caller_that_asks_for_no_split(eng, dtype):
     """One slab, the whole product, though the output has room for more."""
