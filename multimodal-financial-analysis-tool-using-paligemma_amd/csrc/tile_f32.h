@@ -18,6 +18,14 @@
 
 namespace pgmi {
 
+// 16 bytes of an operand that may be aligned as single values only (a caller's own view): one load all the same
+template <typename V>
+__device__ __forceinline__ V any16(const void* p) {
+    V v;
+    __builtin_memcpy(&v, p, 16);
+    return v;
+}
+
 // the three pieces of 8 values, as fragments' 16 bytes
 struct F32Pieces { uint4 p[3]; };
 __device__ __forceinline__ uint32_t top_halves(uint32_t lo, uint32_t hi) { return __builtin_amdgcn_perm(hi, lo, 0x07060302u); }
@@ -70,11 +78,11 @@ __device__ __forceinline__ void tile_f32(const float* __restrict__ A, int lda, c
         const int k = k0 + t * 64 + c8 * 8, kk = k < k1 ? k : k0;
 #pragma unroll
         for (int i = 0; i < CA; ++i) {
-            s.a[i][0] = *reinterpret_cast<const float4*>(ap[i] + kk);
-            s.a[i][1] = *reinterpret_cast<const float4*>(ap[i] + kk + 4);
+            s.a[i][0] = any16<float4>(ap[i] + kk);
+            s.a[i][1] = any16<float4>(ap[i] + kk + 4);
         }
 #pragma unroll
-        for (int i = 0; i < CW; ++i) s.w[i] = ldg16(wp[i] + kk);
+        for (int i = 0; i < CW; ++i) s.w[i] = any16<uint4>(wp[i] + kk);
     };
     // 128-byte rows of 8 chunks, chunk c of row r at place c ^ (r & 7): the fragment reads of 16 rows spread over all banks
     auto write = [&](int t, const Step& s) {

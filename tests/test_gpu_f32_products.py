@@ -55,6 +55,19 @@ def test_every_mode_against_float64(eng, M, N, K):
     assert ((out[:, :N].double() - want).abs() <= tol).all() and (out[:, N:] == 0).all()
 
 
+@pytest.mark.parametrize("M,N,K", [(33, 65, 200), (300, 4096, 136)])
+def test_operands_aligned_as_single_values(eng, M, N, K):
+    """Rows that begin 4 bytes, weights that begin 2 bytes past a 16-byte boundary."""
+    g = torch.Generator("cuda").manual_seed(M)
+    A = torch.randn(M * (K + 8) + 1, device="cuda", generator=g)[1:].view(M, K + 8)[:, :K]
+    W = torch.randn(N * K + 1, device="cuda", generator=g).bfloat16()[1:].view(N, K)
+    assert A.data_ptr() % 16 == 4 and W.data_ptr() % 16 == 2
+    out, same = torch.empty((M, N), device="cuda"), torch.empty((M, N), device="cuda")
+    product(eng, A, W, N, 1, out)
+    product(eng, A.clone(memory_format=torch.contiguous_format), W.clone(), N, 1, same)
+    assert torch.equal(out, same)
+
+
 def test_gate_and_up_without_scratch(eng):
     """Refused for fp32 rows, as include/pgmi.h has it."""
     from pgmi import _native as N_
