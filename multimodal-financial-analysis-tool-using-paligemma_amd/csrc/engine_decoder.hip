@@ -61,9 +61,9 @@ struct DecoderState {
     // workspace of `rows` rows
     int rows = 0;
     void* arena = nullptr;
-    // the recurrences' carries between runs.  A buffer of its own: how many runs a step has does not go by its rows alone, and no
-    // captured step reads it
-    float* carries = nullptr;
+    // the recurrences' carries between runs: in the workspace, or, past what it had room for, in a buffer of their own (how many runs
+    // a step has does not go by its rows alone, and no captured step reads them)
+    float *carries = nullptr, *own_carries = nullptr;
     size_t carry_floats = 0;
     float *X = nullptr, *slabs = nullptr, *dt = nullptr, *bc = nullptr, *cstate = nullptr, *csum = nullptr;
     uint8_t *h = nullptr, *p0 = nullptr, *p1 = nullptr, *p2 = nullptr, *dtl = nullptr;
@@ -368,21 +368,59 @@ void decoder_release(pgmi_ctx* x) {
     DecoderState* d = x->dec;
     if (!d) return;
     drop_derived(*d);
-    for (void* p : {d->arena, d->meta, (void*)d->part, (void*)d->carries})
+    for (void* p : {d->arena, d->meta, (void*)d->part, (void*)d->own_carries})
         if (p) (void)hipFree(p);
     delete d;
     x->dec = nullptr;
 }
 
-// Grow the workspace to these rows (captured graphs hold its addresses)
-int ensure_workspace(pgmi_ctx* x, int rows) {
+// floats of a step's carries between these runs of the scan and of the gated recurrence: states, then sums
+struct Carries { size_t state, sums; };
+Carries carries_of(const DecoderState& d, int scan_runs, int gru_runs) {
+    Carries c{0, 0};
+    for (const pgmi_layer_spec& l : d.L) {
+        if (l.mixer == PGMI_MIXER_MAMBA1) {
+            c.state = std::max(c.state, (size_t)scan_runs * l.inner * l.state);
+            c.sums = std::max(c.sums, (size_t)scan_runs * l.inner);
+        } else if (l.mixer == PGMI_MIXER_MINGRU) {
+            c.state = std::max(c.state, (size_t)gru_runs * 2 * l.width);
+        }
+    }
+    c.state = (c.state + 63) / 64 * 64;
+    return c;
+}
+
+// Grow the workspace to these rows (captured graphs hold its addresses) and these carries, by half as much again for steps of other
+// lengths
+int ensure_workspace(pgmi_ctx* x, int rows, size_t carries) {
     DecoderState& d = *x->dec;
-    if (rows <= d.rows) return 0;
+    if (rows <= d.rows) {
+        if (carries <= d.carry_floats) return 0;
+        HIPCHK(hipDeviceSynchronize());
+        if (d.own_carries) (void)hipFree(d.own_carries);
+        d.carries = d.own_carries = nullptr;
+        d.carry_floats = 0;
+        const size_t n = carries + carries / 2;
+        if (hipMalloc(reinterpret_cast<void**>(&d.own_carries), n * 4) != hipSuccess) {
+            (void)hipGetLastError();
+            d.own_carries = nullptr;
+            return fail(PGMI_E_NOMEM, "carries of " + std::to_string(n * 4) + " bytes");
+        }
+        d.carries = d.own_carries;
+        d.carry_floats = n;
+        return 0;
+    }
     HIPCHK(hipDeviceSynchronize());
     clear_dgraphs(x);
     if (d.arena) (void)hipFree(d.arena);
     d.arena = nullptr;
     d.rows = 0;
+    const size_t here = d.own_carries && carries <= d.carry_floats ? 0 : std::max(carries + carries / 2, d.carry_floats);
+    if (here) {
+        if (d.own_carries) (void)hipFree(d.own_carries);
+        d.carries = d.own_carries = nullptr;
+        d.carry_floats = 0;
+    }
     const int D = d.c.width;
     int l0 = r8(D), l1 = 8, l2 = 8, ldd = 8, slab_n = D, inner = 1, bcn = 2;
     int lea = 8, top = 0, ne = 0;  // mixtures: expert activations, choices per row, experts
@@ -419,7 +457,7 @@ int ensure_workspace(pgmi_ctx* x, int rows) {
                             (size_t)rows * l1 * d.es,           (size_t)rows * l2 * d.es,    (size_t)rows * ldd * d.es,
                             d.slab_bytes,                       (size_t)rows * inner * 4,    (size_t)rows * bcn * 4,
                             ent * lea * d.es, ent * d.ldh * d.es, ent * 4, ent * 4, (size_t)rows * 4, (size_t)rows * 4,
-                            (size_t)rows * ne * 4, (size_t)(2 * ne + 2) * 4};
+                            (size_t)rows * ne * 4, (size_t)(2 * ne + 2) * 4, here * 4};
     constexpr int NB = sizeof(sizes) / sizeof(sizes[0]);
     size_t off[NB], total = 0;
     for (int i = 0; i < NB; ++i) {
@@ -444,40 +482,13 @@ int ensure_workspace(pgmi_ctx* x, int rows) {
     d.inv = reinterpret_cast<float*>(p + off[14]);
     d.elist = reinterpret_cast<int*>(p + off[15]);
     d.ecnt = reinterpret_cast<int*>(p + off[16]);
+    if (here) {
+        d.carries = reinterpret_cast<float*>(p + off[17]);
+        d.carry_floats = here;
+    }
     d.eactive = d.ecnt + ne;
     d.zero_words = ne + 1;
     d.rows = rows;
-    return 0;
-}
-
-// The carries of a step with these runs of the scan and of the gated recurrence; grown by half as much again, for steps of other
-// lengths
-int ensure_carries(DecoderState& d, int scan_runs, int gru_runs) {
-    size_t state = 0, sums = 0;
-    for (const pgmi_layer_spec& l : d.L) {
-        if (l.mixer == PGMI_MIXER_MAMBA1) {
-            state = std::max(state, (size_t)scan_runs * l.inner * l.state);
-            sums = std::max(sums, (size_t)scan_runs * l.inner);
-        } else if (l.mixer == PGMI_MIXER_MINGRU) {
-            state = std::max(state, (size_t)gru_runs * 2 * l.width);
-        }
-    }
-    state = (state + 63) / 64 * 64;
-    if (state + sums > d.carry_floats) {
-        HIPCHK(hipDeviceSynchronize());
-        if (d.carries) (void)hipFree(d.carries);
-        d.carries = nullptr;
-        d.carry_floats = 0;
-        const size_t n = state + sums + (state + sums) / 2;
-        if (hipMalloc(reinterpret_cast<void**>(&d.carries), n * 4) != hipSuccess) {
-            (void)hipGetLastError();
-            d.carries = nullptr;
-            return fail(PGMI_E_NOMEM, "carries of " + std::to_string(n * 4) + " bytes");
-        }
-        d.carry_floats = n;
-    }
-    d.cstate = d.carries;
-    d.csum = d.carries + state;
     return 0;
 }
 
@@ -1079,7 +1090,10 @@ int pgmi_decoder_forward(pgmi_ctx* x, const int64_t* ids, int n_seq, const int32
     for (int r = 0; r < n_seq; ++r) m.insert(m.end(), lens[r], r);
     const size_t o_want = m.size();
     m.insert(m.end(), want, want + n_want);
-    if ((rc = ensure_workspace(x, std::max(rows, n_want))) || (rc = ensure_carries(d, scan.n, gru.n))) return rc;
+    const Carries carries = carries_of(d, scan.n, gru.n);
+    if ((rc = ensure_workspace(x, std::max(rows, n_want), carries.state + carries.sums))) return rc;
+    d.cstate = d.carries;
+    d.csum = d.carries + carries.state;
     if (m.size() * 4 > d.meta_bytes) {
         HIPCHK(hipDeviceSynchronize());
         if (d.meta) (void)hipFree(d.meta);
@@ -1120,7 +1134,7 @@ int pgmi_decoder_decode(pgmi_ctx* x, const int64_t* ids, int B, const int32_t* s
         if (positions[b] < 0 || (long)positions[b] + n_steps > max_tokens) return fail(PGMI_E_ARG, "state capacity exceeded");
     HIPCHK(hipSetDevice(x->device));
     hipStream_t s = (hipStream_t)stream;
-    if ((rc = ensure_workspace(x, B))) return rc;
+    if ((rc = ensure_workspace(x, B, 0))) return rc;
     size_t need = 0;
     for (const pgmi_layer_spec& l : d.L)
         if (l.mixer == PGMI_MIXER_ATTENTION)
