@@ -1063,14 +1063,17 @@ int pgmi_decoder_forward(pgmi_ctx* x, const int64_t* ids, int n_seq, const int32
         }
         return c;
     };
-    long scan_cols = 0, gru_cols = 0;  // 0: no such layer, no list
+    long scan_cols = 0, scan_wgs = 0, gru_cols = 0;  // 0: no such layer, no list
     for (const pgmi_layer_spec& l : d.L) {
-        if (l.mixer == PGMI_MIXER_MAMBA1) scan_cols = std::max(scan_cols, scan_columns(l.inner, l.state));
+        if (l.mixer == PGMI_MIXER_MAMBA1) {
+            scan_cols = std::max(scan_cols, scan_columns(l.inner, l.state));
+            scan_wgs = std::max(scan_wgs, scan_workgroups(l.inner, l.state));
+        }
         if (l.mixer == PGMI_MIXER_MINGRU) gru_cols = std::max(gru_cols, gru_columns(l.width));
     }
     const bool huge = rows > 16384;
     Cut scan{0, 0, false}, gru = scan, conv = scan;
-    if (scan_cols) scan = cut(huge ? 256 : scan_run_rows(lens, n_seq, scan_cols));
+    if (scan_cols) scan = cut(huge ? 256 : scan_run_rows(lens, n_seq, scan_cols, scan_wgs));
     if (gru_cols) gru = cut(huge ? 128 : gru_run_rows(lens, n_seq, gru_cols));
     // the convolutions carry nothing: 500 rows of 2,048 channels 11.2 us on 64-row runs, 5.9 on 16; 2,048 rows 10.8 / 7.5
     if (scan_cols || d.c.canon_taps > 0) conv = cut(huge ? 256 : rows > 2048 ? 32 : 16);

@@ -19,6 +19,8 @@ constexpr int scan_lanes(int N) { return N <= 16 ? 1 : N <= 32 ? 2 : N <= 64 ? 4
 // 261 / 267 / 288; 1,540 rows 172 / 171 / 180, 282 / 286 / 308, 655 / 682 / 758.
 constexpr long scan_columns(int C, int N) { return ((long)C + 255) / 256 * std::max(1, scan_lanes(N) / 4); }
 constexpr long gru_columns(int C) { return ((long)C + 127) / 128; }
+// the scan's workgroups for a run of C channels
+constexpr long scan_workgroups(int C, int N) { return ((long)C * scan_lanes(N) + 255) / 256; }
 
 inline long runs_of(const int32_t* lens, int n_seq, int rows) {
     long n = 0;
@@ -26,10 +28,21 @@ inline long runs_of(const int32_t* lens, int n_seq, int rows) {
     return n;
 }
 
+// Sequences that are walked whole take one launch where runs take three, two of them walks: the longest of the sequences if that
+// pays, else 0.  Up to 40 rows it does, and up to 64 where whole sequences fill half the chip; `workgroups` of one run, 0 where
+// only the first counts.  us a layer, whole / in the best runs: 2,048 channels of 16 states, 17 rows 42 / 52, 40 rows 52 / 53, 64 rows 63 /
+// 54; 8 x 64 rows of 4,096 channels 79 / 83, of 2,048 of 64 states 81 / 97, of 512 of 16 states 61 / 54; minGRU of 1,024, 17 rows 17 / 21,
+// 40 rows 22 / 22, 64 rows 27 / 22, 32 x 40 rows 28 / 31.
+inline int whole_rows(const int32_t* lens, int n_seq, long workgroups) {
+    const int most = *std::max_element(lens, lens + n_seq);
+    return most <= 40 || (most <= 64 && n_seq * workgroups >= kRunCUs / 2) ? most : 0;
+}
+
 // The scan takes the length whose rounds walk the fewest rows, a workgroup's start costing about 8.  us of its three launches,
 // 64- / 16-row runs: 500 rows of 2,048 channels of 16 states 86 / 41, 300 rows 69 / 35; 64 rows / this rule: 1,540 rows of 4,096
-// channels (50-row runs) 98 / 92.  columns: of the layer with the most.
-inline int scan_run_rows(const int32_t* lens, int n_seq, long columns) {
+// channels (50-row runs) 98 / 92.  columns, workgroups: of the layer with the most.
+inline int scan_run_rows(const int32_t* lens, int n_seq, long columns, long workgroups) {
+    if (const int whole = whole_rows(lens, n_seq, workgroups)) return whole;
     int best = 64;
     long least = LONG_MAX;
     for (int ct = 64; ct >= 16; ct -= 2) {
@@ -41,6 +54,7 @@ inline int scan_run_rows(const int32_t* lens, int n_seq, long columns) {
 
 // minGRU: the longest runs, down to 8 rows, that still give every CU a workgroup of 128 channels
 inline int gru_run_rows(const int32_t* lens, int n_seq, long columns) {
+    if (const int whole = whole_rows(lens, n_seq, 0)) return whole;
     int ct = 32;
     for (const int k : {32, 24, 16, 8}) {
         ct = k;

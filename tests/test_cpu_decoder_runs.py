@@ -16,7 +16,7 @@ int main(int n, char** v) {  // channels, states, lengths
     std::vector<int32_t> lens;
     for (int i = 3; i < n; ++i) lens.push_back(atoi(v[i]));
     const int C = atoi(v[1]), N = atoi(v[2]);
-    std::printf("%d %d\n", pgmi::scan_run_rows(lens.data(), (int)lens.size(), pgmi::scan_columns(C, N)),
+    std::printf("%d %d\n", pgmi::scan_run_rows(lens.data(), (int)lens.size(), pgmi::scan_columns(C, N), pgmi::scan_workgroups(C, N)),
                 pgmi::gru_run_rows(lens.data(), (int)lens.size(), pgmi::gru_columns(C)));
 }
 """
@@ -38,12 +38,16 @@ def ask(tmp_path_factory):
     (2048, 64, [500], 16, 32), (2048, 64, [1000], 16, 64), (2048, 64, [4000], 32, 64), (4096, 64, [1540], 32, 64),
     (2048, 128, [200], 16, 24), (2048, 128, [500], 16, 64), (2048, 128, [1540], 48, 64), (2048, 128, [4000], 32, 64),
     (2048, 256, [500], 60, 64), (2048, 256, [1000], 48, 64), (2048, 256, [1540], 48, 64), (2048, 256, [4000], 48, 64),
-    (2048, 256, [500, 300, 100, 60], 56, 64)])
+    (2048, 256, [500, 300, 100, 60], 56, 64),
+    # sequences that are walked whole, and just no more
+    (2048, 16, [17], 17, 64), (2048, 16, [32], 32, 64), (2048, 16, [40], 16, 64), (2048, 16, [48], 16, 16), (512, 16, [64] * 8, 16, 16),
+    (4096, 16, [64] * 8, 64, 64), (2048, 64, [64] * 8, 64, 64), (2048, 64, [20] * 8, 20, 64), (4096, 16, [40] * 32, 40, 64), (2048, 16, [1], 1, 64)])
 def test_scan(ask, C, N, lens, least, most):
     assert least <= ask(C, N, *lens)[0] <= most
 
 
-@pytest.mark.parametrize("C,lens,rows", [(2048, [1024], 32), (2048, [500], 32), (2048, [370], 24), (2048, [300], 16), (2048, [100], 8), (128, [9000], 32),
-                                         (128, [7000], 24), (128, [100, 3], 8)])
+@pytest.mark.parametrize("C,lens,rows", [(2048, [1024], 32), (2048, [500], 32), (2048, [370], 24), (2048, [300], 16), (2048, [100], 8), (2048, [41], 8), (2048, [40], 40), (1024, [40] * 32, 40), (300, [17, 3], 17), (128, [9000], 32),
+                                         (128, [7000], 24), (64, [300], 8),
+                                         (128, [100, 3], 8)])
 def test_gru(ask, C, lens, rows):
     assert ask(C, 16, *lens)[1] == rows
