@@ -52,13 +52,16 @@ inline int scan_run_rows(const int32_t* lens, int n_seq, long columns, long work
     return best;
 }
 
-// minGRU: the longest runs, down to 8 rows, that still give every CU a workgroup of 128 channels
+// minGRU: the longest runs, down to 8 rows, that still give every CU a workgroup of 128 channels; of one sequence no more than 84,
+// which the carry walks one after the other (us a layer on runs of 32 / 24 / 16 / 8 rows, 64 channels: 300 rows 30 / 28 / 26 / 24, 700
+// rows 32 / 29 / 27 / 28, 2,000 rows 36 / 35 / 35 / 41, 5,000 rows 50 / 51 / 55 / 76)
 inline int gru_run_rows(const int32_t* lens, int n_seq, long columns) {
     if (const int whole = whole_rows(lens, n_seq, 0)) return whole;
+    const int most = *std::max_element(lens, lens + n_seq);
     int ct = 32;
-    for (const int k : {32, 24, 16, 8}) {
+    for (const int k : {24, 16, 8}) {
+        if (runs_of(lens, n_seq, ct) * columns >= kRunCUs || (most + k - 1) / k > 84) break;
         ct = k;
-        if (runs_of(lens, n_seq, ct) * columns >= kRunCUs) break;
     }
     return ct;
 }

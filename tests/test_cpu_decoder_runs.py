@@ -47,7 +47,7 @@ def test_scan(ask, C, N, lens, least, most):
 
 
 @pytest.mark.parametrize("C,lens,rows", [(2048, [1024], 32), (2048, [500], 32), (2048, [370], 24), (2048, [300], 16), (2048, [100], 8), (2048, [41], 8), (2048, [40], 40), (1024, [40] * 32, 40), (300, [17, 3], 17), (128, [9000], 32),
-                                         (128, [7000], 24), (64, [300], 8),
-                                         (128, [100, 3], 8)])
+                                         (128, [7000], 32), (64, [2000], 24), (64, [700], 16),
+                                         (64, [300], 8), (128, [100, 3], 8)])
 def test_gru(ask, C, lens, rows):
     assert ask(C, 16, *lens)[1] == rows
