@@ -842,8 +842,11 @@ template <typename T>
 void run_skinny(hipStream_t s, GemvRtMode mode, const GemvRtArgs& a) {
     const dim3 grid((a.N + 15) / 16), block(256);
     constexpr int kHeldBlocks = 512;  // two per CU: 256, 512 and 768 measured equal, 1,024 and more slower
-    if (std::is_same<T, uint16_t>::value && a.K <= 2048 && a.split <= 1 && (int)grid.x > kHeldBlocks &&
-        (mode == GR_F32 || mode == GR_LOGITS || mode == GR_SWIGLU)) {
+    // The held form always asks for 2,048 inputs a row, so it pays from a width on, of two matrices with many rows or a greater one.  us
+    // a layer or step, plain / held: gate|up of 16,384 at width 512 32.9 / 35.8 (2 rows), 36.1 / 38.2 (16), at 1,024 47.3 / 48.4 (2),
+    // 57.2 / 54.6 (16), at 1,280 57.4 / 56.1 (2); 65,536 outputs at 256 45.7 / 47.0 (8), at 768 56.2 / 54.5, at 2,048 92.7 / 83.3
+    const bool pays = mode == GR_SWIGLU ? a.K > 1024 || a.B * a.K >= 12288 : (mode == GR_F32 || mode == GR_LOGITS) && a.K > 512;
+    if (std::is_same<T, uint16_t>::value && pays && a.K <= 2048 && a.split <= 1 && (int)grid.x > kHeldBlocks) {
         if (mode == GR_SWIGLU) hipLaunchKernelGGL((k_skinny_held<GR_SWIGLU>), dim3(kHeldBlocks), block, 0, s, a);
         else hipLaunchKernelGGL((k_skinny_held<GR_F32>), dim3(kHeldBlocks), block, 0, s, a);
         return;
