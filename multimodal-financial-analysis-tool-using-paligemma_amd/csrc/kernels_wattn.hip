@@ -770,16 +770,16 @@ __global__ void __launch_bounds__(256) k_wattn_d(WAttnDecodeArgs a) {
 // bf16 MFMA form, 16 query heads of a group per workgroup (grid (split, G * head blocks, B)).  A wave takes 32-key
 // tiles: S^T = K Q^T with the key fragments straight from the cache, then O^T += V^T P^T as k_wattn_m, the values
 // through the wave's own LDS rows; the four waves' running sums meet in LDS.
-// VEC: head sizes that are multiples of 8.
+// VEC: head sizes that are multiples of 8 (up to 64 four waves to a SIMD: 136 registers and three, 16 sequences of 8 heads 143 us for 129).
 template <int DQ, int DV, int SC, bool VEC>
-__global__ void __launch_bounds__(256) k_wattn_dm(WAttnDecodeArgs a) {
+__global__ void __launch_bounds__(256, DQ <= 64 && DV <= 64 && VEC ? 4 : 1) k_wattn_dm(WAttnDecodeArgs a) {
     const WAttnHeads& w = a.hd;
     constexpr int VS = DV + 8;
     __shared__ __attribute__((aligned(16))) uint16_t Vs[4][32 * VS];
     __shared__ float sml[4][16][2];
     __shared__ float2 turned[DQ / 2];  // cos and sin of the rotated pairs
     const int R = w.H / w.G, hb = blockIdx.y / w.G, g = blockIdx.y % w.G, b = blockIdx.z, sp = blockIdx.x;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, li = lane & 15, lg = lane >> 4;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), li = lane & 15, lg = lane >> 4;
     const int slot = a.slot[b], i = a.pos[b];
     const Keys keys(a.sc, i);  // k0, k1, kend, j0 below count the keys this query sees
     const int per = ((keys.n + a.nsplit - 1) / a.nsplit + 127) / 128 * 128;
@@ -801,8 +801,6 @@ __global__ void __launch_bounds__(256) k_wattn_dm(WAttnDecodeArgs a) {
     const bool own = w.own_kv && k1 == keys.n;
     const int kend = own ? k1 - 1 : k1;
     const int h = g * R + r0 + (li < nr ? li : 0);
-    const uint16_t* kn = w.own_kv ? qkv + w.H * w.d + g * w.d : qkv;
-    const uint16_t* vn = w.own_kv ? qkv + (w.H + w.G) * w.d + g * w.e : qkv;
     // first tile's loads, then the query's: all in flight together
     uint4 vr[DV / 16], kr[2][DQ / 32];
     auto gload = [&](int j0) {
@@ -836,23 +834,27 @@ __global__ void __launch_bounds__(256) k_wattn_dm(WAttnDecodeArgs a) {
             }
         }
     };
-    const int dn = w.own_kv ? w.d : 0, en = w.own_kv ? w.e : 0;
     raw(qkv + h * w.d, w.d, qr);
-    raw(kn, dn, knr);
+    // (by the one wave that uses them: every wave asked for them and cut their pads, 40 sequences of 16 heads of 80 53 us a layer, so 49)
+    const bool mine = own && wave == 0;
+    const uint16_t* vn = qkv + (w.H + w.G) * w.d + g * w.e;
+    if (mine) {
+        raw(qkv + w.H * w.d + g * w.d, w.d, knr);
 #pragma unroll
-    for (int c = 0; c < DV / 16; ++c) {
-        const int k = c * 16 + 4 * lg;
-        if constexpr (VEC) {
-            ld4(vn + (k < en ? k : 0), vnr[c]);
+        for (int c = 0; c < DV / 16; ++c) {
+            const int k = c * 16 + 4 * lg;
+            if constexpr (VEC) {
+                ld4(vn + (k < w.e ? k : 0), vnr[c]);
 #pragma unroll
-            for (int r = 0; r < 4; ++r) vnr[c][r] = k < en ? vnr[c][r] : 0.0f;
-        } else {
+                for (int r = 0; r < 4; ++r) vnr[c][r] = k < w.e ? vnr[c][r] : 0.0f;
+            } else {
 #pragma unroll
-            for (int r = 0; r < 4; ++r) vnr[c][r] = k + r < en ? bf2f(vn[k + r]) : 0.0f;
+                for (int r = 0; r < 4; ++r) vnr[c][r] = k + r < w.e ? bf2f(vn[k + r]) : 0.0f;
+            }
         }
     }
     // every head turns by the same angles: a thread per pair, once (by every lane for its own dims, each turn loaded behind its
-    // own check, and the new key and value asked for only then: 8 sequences of 16 heads 13.3 us, now 10.3)
+    // own check, and the new key and value asked for only then: 8 sequences of 16 heads 13.3 us, now 9.8)
     if (tid < w.rot / 2) {
         float s, c;
         angle(w.turns[tid], i, s, c);
@@ -897,7 +899,7 @@ __global__ void __launch_bounds__(256) k_wattn_dm(WAttnDecodeArgs a) {
 #pragma unroll
     for (int c = 0; c < DV / 16; ++c) o[c] = f32x4{0.f, 0.f, 0.f, 0.f};
     float m = SC == SC_CAPPED ? 0.0f : kNone, l = 0.0f;
-    if (own && wave == 0) {
+    if (mine) {
         short8 kf[DQ / 32];
         head_row(knr, kf);
         float dot = 0.0f;
