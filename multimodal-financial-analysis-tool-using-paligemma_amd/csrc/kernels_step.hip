@@ -589,14 +589,16 @@ bool gemv_one_fits(const GemvRtArgs& a, int mode) {
     if (mode == GR_CONV && a.taps_k > 4) return false;
     if (a.x) return true;
     const int P = a.K / std::max(1, a.groups);
-    return a.D == a.K && a.groups >= 1 && a.K % a.groups == 0 && (P % 512 == 0 || (512 % P == 0 && P >= 8));
+    return (a.S <= 2 || a.K <= 1024) && a.D == a.K && a.groups >= 1 && a.K % a.groups == 0 && (P % 512 == 0 || (512 % P == 0 && P >= 8));
 }
 
 template <int MODE, int CH>
 void run_one_ch(hipStream_t s, const GemvRtArgs& a, int blocks) {
-    if (a.x) hipLaunchKernelGGL((k_gemv_one<MODE, CH, 0>), dim3(blocks), dim3(256), 0, s, a);
-    else if (a.S <= 2) hipLaunchKernelGGL((k_gemv_one<MODE, CH, 2>), dim3(blocks), dim3(256), 0, s, a);
-    else hipLaunchKernelGGL((k_gemv_one<MODE, CH, 4>), dim3(blocks), dim3(256), 0, s, a);
+    if (MODE == GR_STREAMS || a.x) hipLaunchKernelGGL((k_gemv_one<MODE, CH, 0>), dim3(blocks), dim3(256), 0, s, a);
+    else if constexpr (MODE != GR_STREAMS) {  // (the update's input is the sublayer's, never the streams)
+        if (CH > 2 || a.S <= 2) hipLaunchKernelGGL((k_gemv_one<MODE, CH, 2>), dim3(blocks), dim3(256), 0, s, a);
+        else if constexpr (CH <= 2) hipLaunchKernelGGL((k_gemv_one<MODE, CH, 4>), dim3(blocks), dim3(256), 0, s, a);
+    }
 }
 template <int MODE>
 void run_one(hipStream_t s, const GemvRtArgs& a) {
@@ -1003,8 +1005,9 @@ __global__ void __launch_bounds__(256) k_decode_finish(const float* __restrict__
 int gemv_rt_max_batch() { return 16; }
 int gemv_rt_parts() { return 2 * 1024; }
 GemvRtForm gemv_rt_form(int B, Act act, int streams, int width) {
-    // fp32 activations: two rows.  bf16: one row, while every workgroup's own read of the streams stays small;
-    // measured, batch 1, 2 streams: width 1024 0.379 against 0.432 ms per step, 2048 0.802 / 0.818, 4096 0.828 / 0.661
+    // fp32 activations: two rows.  bf16: one row, while every workgroup's own read of the streams stays small.  ms a step, this form /
+    // the MFMA form: 2 streams of 1024 0.293 / 0.427, 4 of 1024 0.326 / 0.459, 2 of 2048 0.639 / 0.821, 2 of 4096 0.812 / 0.664.  Streams
+    // times width is not all of it: 3 of 2048 (0.668 / 0.843) and 1 of 4096 (0.770 / 0.656) lie on the side that is slower for them
     if (act == ACT_F32 && B <= 2) return GF_STREAM;
     if (act == ACT_BF16 && B == 1 && streams * width <= 4096) return GF_STREAM;
     return B <= gemv_rt_max_batch() ? GF_SKINNY : GF_NONE;
