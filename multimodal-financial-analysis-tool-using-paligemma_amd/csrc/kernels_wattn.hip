@@ -298,6 +298,7 @@ __global__ void __launch_bounds__(256, D <= 128 ? 2 : 1) k_wattn_f(WAttnArgs a) 
         const bool head = t < nh;  // kept keys: every row sees those before lo
         const bool whole = head ? j0 + 16 <= kept : j0 + 15 <= wfirst && (hi - j0 < window || j0 + 16 <= keep);
         const int end = head ? kept : i + 1;
+        // (& and |: as && and || the compiler branches between the keys)
         auto sees = [&](int j) { return (j < end) & ((i - j < window) | (j < keep)); };
         float mt = m;
 #pragma unroll
