@@ -51,3 +51,11 @@ def test_scan(ask, C, N, lens, least, most):
                                          (64, [300], 8), (128, [100, 3], 8)])
 def test_gru(ask, C, lens, rows):
     assert ask(C, 16, *lens)[1] == rows
+
+
+# the steps of test_gpu_decoder_runs.py, whose layers are all a workgroup wide
+@pytest.mark.parametrize("n,length,scan,gru", [(36, 450, 32, 32), (30, 400, 50, 32), (20, 450, 36, 32), (3, 97, 16, 8), (36, 448, 64, 32),
+                                               (16, 450, 30, 24), (12, 450, 22, 16), (10, 450, 18, 16)])
+@pytest.mark.parametrize("C,N", [(72, 12), (40, 9), (128, 16)])
+def test_steps_of_many_sequences(ask, C, N, n, length, scan, gru):
+    assert ask(C, N, *(length - 7 * (r % 5) for r in range(n))) == [scan, gru]

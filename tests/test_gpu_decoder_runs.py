@@ -10,8 +10,9 @@ from decoder_helpers import build, tokens
 pytestmark = pytest.mark.gpu
 
 
-# (sequences, tokens each): run lengths from 64 rows down to 16 at these models' widths, and past 16,384 rows of 256
-@pytest.mark.parametrize("n,length", [(36, 450), (30, 400), (20, 450), (3, 97), (40, 430)])
+# (sequences, tokens each): runs of the scan of 64, 50, 36, 32, 30, 22, 18 and 16 rows at these models' widths, of minGRU of 32, 24, 16
+# and 8, and past 16,384 rows of 256 and 128
+@pytest.mark.parametrize("n,length", [(36, 450), (30, 400), (20, 450), (3, 97), (40, 430), (36, 448), (16, 450), (12, 450), (10, 450)])
 @pytest.mark.parametrize("name", sorted(C.MIXED))
 def test_together_as_alone(name, n, length):
     cfg = C.MIXED[name]
