@@ -774,10 +774,11 @@ __global__ void __launch_bounds__(256, sizeof(T) == 4 && MODE != GR_GRU && MODE 
 // a group moves besides its weights is otherwise as many bytes of activations from L2 (8 rows: the output matrix of 257,216 x
 // 2048 207 us, held 185; gate|up of 16,384 channels 32.0 / 25.7).  The next group's weights are asked for before this one's
 // sums meet, the last group peeled off.  (fp32 rows, three pieces each, would take 200 registers.)
-__device__ const uint16_t kZeros[8] __attribute__((aligned(16))) = {};  // weights past the end
-template <int MODE>
+// ST: 64-deep steps of a wave, K / 256 rounded up.  PART: K is less than 256 ST; past it the last step loads the row's first weights,
+// made zero where they are used (loads from zeros in memory: gate|up at 2048 26.9 us for 25.1).
+template <int MODE, int ST, bool PART>
 __global__ void __launch_bounds__(256) k_skinny_held(GemvRtArgs a) {
-    constexpr int NM = MODE == GR_SWIGLU ? 2 : 1, ST = 8;  // 64-deep steps of a wave
+    constexpr int NM = MODE == GR_SWIGLU ? 2 : 1;
     __shared__ float sums[2][4][NM][16][17];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int li = lane & 15, lg = lane >> 4, K = a.K, ngroup = (a.N + 15) / 16;
@@ -788,7 +789,7 @@ __global__ void __launch_bounds__(256) k_skinny_held(GemvRtArgs a) {
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
             const int k = (wave + 4 * i) * 64 + lg * 16 + 8 * h;
-            x[i][h] = __builtin_bit_cast(short8, ldg16_sel(xp + k, k < K, xp));
+            x[i][h] = __builtin_bit_cast(short8, ldg16_sel(xp + k, !PART || i + 1 < ST || k < K, xp));
         }
     uint4 w[ST][NM][2];
     int grp = blockIdx.x, turn = 0;
@@ -801,7 +802,7 @@ __global__ void __launch_bounds__(256) k_skinny_held(GemvRtArgs a) {
 #pragma unroll
                 for (int h = 0; h < 2; ++h) {
                     const int k = (wave + 4 * i) * 64 + lg * 16 + 8 * h;
-                    w[i][m][h] = ldg16(k < K ? p + k : kZeros);
+                    w[i][m][h] = ldg16(p + (!PART || i + 1 < ST || k < K ? k : 0));
                 }
         }
     };
@@ -816,7 +817,14 @@ __global__ void __launch_bounds__(256) k_skinny_held(GemvRtArgs a) {
 #pragma unroll
             for (int h = 0; h < 2; ++h)
 #pragma unroll
-                for (int m = 0; m < NM; ++m) acc[m] = mfma16(__builtin_bit_cast(short8, w[i][m][h]), x[i][h], acc[m]);
+                for (int m = 0; m < NM; ++m) {
+                    uint4 q = w[i][m][h];
+                    if (PART && i + 1 == ST) {
+                        const uint32_t keep = (wave + 4 * i) * 64 + lg * 16 + 8 * h < K ? ~0u : 0u;
+                        q = make_uint4(q.x & keep, q.y & keep, q.z & keep, q.w & keep);
+                    }
+                    acc[m] = mfma16(__builtin_bit_cast(short8, q), x[i][h], acc[m]);
+                }
         grp += gridDim.x;
         if constexpr (decltype(more)::value) wload();
 #pragma unroll
@@ -840,17 +848,31 @@ __global__ void __launch_bounds__(256) k_skinny_held(GemvRtArgs a) {
     step_pads<uint16_t, MODE>(a);
 }
 
+template <int ST, bool PART = true>
+void run_held(hipStream_t s, GemvRtMode mode, const GemvRtArgs& a, int blocks) {
+    if (PART && a.K % 256 == 0) return run_held<ST, false>(s, mode, a, blocks);
+    if (mode == GR_SWIGLU) hipLaunchKernelGGL((k_skinny_held<GR_SWIGLU, ST, PART>), dim3(blocks), dim3(256), 0, s, a);
+    else hipLaunchKernelGGL((k_skinny_held<GR_F32, ST, PART>), dim3(blocks), dim3(256), 0, s, a);
+}
+
 template <typename T>
 void run_skinny(hipStream_t s, GemvRtMode mode, const GemvRtArgs& a) {
     const dim3 grid((a.N + 15) / 16), block(256);
     constexpr int kHeldBlocks = 512;  // two per CU: 256, 512 and 768 measured equal, 1,024 and more slower
-    // The held form always asks for 2,048 inputs a row, so it pays from a width on, of two matrices with many rows or a greater one.  us
-    // a layer or step, plain / held: gate|up of 16,384 at width 512 32.9 / 35.8 (2 rows), 36.1 / 38.2 (16), at 1,024 47.3 / 48.4 (2),
-    // 57.2 / 54.6 (16), at 1,280 57.4 / 56.1 (2); 65,536 outputs at 256 45.7 / 47.0 (8), at 768 56.2 / 54.5, at 2,048 92.7 / 83.3
-    const bool pays = mode == GR_SWIGLU ? a.K > 1024 || a.B * a.K >= 12288 : (mode == GR_F32 || mode == GR_LOGITS) && a.K > 512;
+    // The held form pays from 512 inputs on.  us a step of four layers and the output matrix, plain / held: gate|up of 16,384 at width 320
+    // 128 / 129 (2 rows), 135 / 136 (8), at 512 143 / 140 and 149 / 145, at 1,024 188 / 180 and 203 / 188, at 2,048 289 / 270 and 311 /
+    // 285; 65,536 outputs at 512 122 / 117 and 130 / 122, at 1,000 137 / 137 and 143 / 142, at 2,048 181 / 178 and 195 / 186
+    const bool pays = a.K >= 512 && (mode == GR_SWIGLU || mode == GR_F32 || mode == GR_LOGITS);
     if (std::is_same<T, uint16_t>::value && pays && a.K <= 2048 && a.split <= 1 && (int)grid.x > kHeldBlocks) {
-        if (mode == GR_SWIGLU) hipLaunchKernelGGL((k_skinny_held<GR_SWIGLU>), dim3(kHeldBlocks), block, 0, s, a);
-        else hipLaunchKernelGGL((k_skinny_held<GR_F32>), dim3(kHeldBlocks), block, 0, s, a);
+        switch ((a.K + 255) / 256) {
+            case 2: run_held<2>(s, mode, a, kHeldBlocks); break;
+            case 3: run_held<3>(s, mode, a, kHeldBlocks); break;
+            case 4: run_held<4>(s, mode, a, kHeldBlocks); break;
+            case 5: run_held<5>(s, mode, a, kHeldBlocks); break;
+            case 6: run_held<6>(s, mode, a, kHeldBlocks); break;
+            case 7: run_held<7>(s, mode, a, kHeldBlocks); break;
+            default: run_held<8>(s, mode, a, kHeldBlocks); break;
+        }
         return;
     }
     switch (mode) {

@@ -1,6 +1,6 @@
 """Two to sixteen sequences in bf16 where one workgroup walks several groups of outputs (more than 512 of them: the output
-matrix, gate|up), at group edges, widths below and at the held 2,048, one input past them, and on both sides of the widths from
-which it does."""
+matrix, gate|up), at group edges, widths below and at the held 2,048, one input past them, on both sides of the 512 from which it
+does, and with every number of steps, whole and not."""
 import numpy as np
 import pytest
 import torch
@@ -13,12 +13,11 @@ pytestmark = pytest.mark.gpu
 CASES = {
     "8208_outputs": C.model([C.gru(40, ff=8208)], width=72, vocab=8209, streams=2, groups=3),
     "16400_outputs": C.model([C.gru(24, ff=8193)], width=1000, vocab=16400, streams=1, groups=1),
-    "from_520": C.model([C.gru(24, ff=8200)], width=520, vocab=8201, streams=1, groups=1),
-    "to_512": C.model([C.gru(24, ff=8200)], width=512, vocab=8201, streams=1, groups=1),
-    "from_1032": C.model([C.gru(24, ff=8209)], width=1032, vocab=333, streams=1, groups=1),
     "held_2048": C.model([C.gru(16)], width=2048, vocab=9001, streams=2, groups=4),
     "past_2048": C.model([C.gru(16)], width=2056, vocab=8200, streams=2, groups=4),
 }
+CASES.update({f"width_{w}": C.model([C.gru(24, ff=8200)], width=w, vocab=8201, streams=1, groups=1)
+              for w in (504, 512, 520, 768, 1032, 1280, 1400, 1536, 1672, 1792, 2040)})
 
 
 @pytest.mark.parametrize("B", [2, 7, 16])
