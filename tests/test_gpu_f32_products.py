@@ -173,6 +173,25 @@ def test_time_and_values_of_a_step_where_a_weight_is_not_finite(dtype, width, vo
     assert times[1] <= (6 if dtype == "float32" else 2) * times[0], times
 
 
+@pytest.mark.parametrize("part", ["gate", "up", "down"])
+@pytest.mark.parametrize("rows", [40, 300])  # both sizes of tile
+def test_an_expert_whose_weight_is_not_finite(rows, part):
+    """Lost are the rows that chose it (those that another value of the weight changes); the others are the same to the bit."""
+    cfg = R.MECHANISMS["experts_few"]
+    name, toks, logits = f"l0.mlp.e1.{part}", tokens(cfg, rows, 8), []
+    for value in (None, 50.0, np.inf):
+        W = raritar_np.random_weights(cfg, 3)
+        if value is not None:
+            W[name][3, 2] = value
+        eng, _ = build(cfg, "float32", weights=W)
+        cache = eng.new_cache(1, rows)
+        logits.append(eng.step(cache, [cache.alloc()], [toks], want=list(range(rows))).clone())
+    fine, other, broken = logits
+    chose = (fine != other).any(1)
+    assert 0 < int(chose.sum()) < rows
+    assert torch.equal(~broken.isfinite().all(1), chose) and torch.equal(broken[~chose], fine[~chose])
+
+
 @pytest.mark.parametrize("rows", [3, 16, 17, 40])
 def test_decode_rows(rows):
     """One token each: the skinny form (to 16 rows) and the tiles, mixtures of experts included."""
