@@ -173,6 +173,29 @@ def test_time_and_values_of_a_step_where_a_weight_is_not_finite(dtype, width, vo
     assert times[1] <= (6 if dtype == "float32" else 2) * times[0], times
 
 
+@pytest.mark.parametrize("B", [3, 16])
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+def test_a_row_that_is_not_finite(dtype, B):
+    """One sequence's activations, through products whose K is cut over workgroups too: the others are the same to the bit."""
+    cfg = C.model([C.gru(512, ff=8192), C.mamba(1032, 16, 8, 4)], width=264, vocab=300, streams=2, groups=1)
+    W = decoder_np.random_weights(cfg, 3)
+    W["embed"][5], W["embed"][6] = np.inf, np.nan
+    eng, _ = build(cfg, dtype, weights=W, max_batch=16)
+    logits = []
+    for bad in (None, 5, 6):
+        cache, ids = eng.new_cache(B, 4), torch.arange(10, 10 + B, device="cuda")
+        if bad is not None:
+            ids[1] = bad
+        logits.append(eng.decode(cache, [cache.alloc() for _ in range(B)], ids).clone())
+    others = torch.arange(B, device="cuda") != 1
+    columns = torch.ones(300, dtype=torch.bool, device="cuda")
+    columns[5:7] = False  # (the table is the output matrix too)
+    fine = logits[0][others][:, columns]
+    assert fine.isfinite().all()
+    for broken in logits[1:]:
+        assert torch.equal(broken[others][:, columns], fine) and not broken[1].isfinite().any()
+
+
 @pytest.mark.parametrize("part", ["gate", "up", "down"])
 @pytest.mark.parametrize("rows", [40, 300])  # both sizes of tile
 def test_an_expert_whose_weight_is_not_finite(rows, part):
