@@ -214,7 +214,7 @@ def gemm_roofline(eng, rows, iters=36, reps=4):
     token rows.  `iters` launches cycling the layers (cold weights: 18 layers x 134 / 67 MB stream
     past the 256 MiB MALL) are captured into one graph and replayed `reps` times back to back;
     HIP events on the replay stream give the average launch, graph gaps included (an eager
-    ctypes loop is host-bound for a ~20 us kernel: round 3 read 38 us for a 23 us kernel)."""
+    ctypes loop is host-bound for a ~20 us kernel: it read 38 us for a 23 us kernel)."""
     import torch
     from pgmi import _native as N
     t = eng.cfgd

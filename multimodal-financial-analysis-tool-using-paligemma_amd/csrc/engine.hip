@@ -469,7 +469,7 @@ static int lm_body(pgmi_ctx* x, hipStream_t s, const int64_t* ids, const void* i
 // the next layer (k_mf_combine_norm; q|k|v reads dHn unstaged), the post-attention norm from o_proj's 16-column
 // partial sums of squares, applied by gate|up as it loads h (default) -- or each projection stages and
 // normalises its rows itself (pgmi_set_decode_staged_norm,
-// tested by test_batch_rows_teacher_forced_vs_own_reference[8-1]).  Round 4, the unstaged form reading rows
+// tested by test_batch_rows_teacher_forced_vs_own_reference[8-1]).  The unstaged form reading rows
 // normalised by separate passes against the staged form: equal
 // while the weight streams were non-temporal (B = 8 step 1.5449 vs 1.5452 ms); with the default cache policy
 // (kernels_gemv_mfma.hip PGMI_MF_NT) the unstaged form wins, same box: 1.4523 / 1.4550 -> 1.4330 / 1.4320 ms
@@ -493,7 +493,7 @@ static int decode_body(pgmi_ctx* x, hipStream_t s, const int64_t* ids, int B, vo
     else if (!fold) embed_rows(s, ids, B, E, H, normalizer, c.pad_token_id, x->dH);
     // B >= 3 (MFMA projections): every RMSNorm is computed once per row -- the input norm fused into the
     // down projection's combine for the next layer (q|k|v reads dHn unstaged), the post-attention norm's
-    // sums of squares written by o_proj's epilogue (dSS) and applied by gate|up as it loads h.  (Round 5,
+    // sums of squares written by o_proj's epilogue (dSS) and applied by gate|up as it loads h.  (Measured:
     // the input norm the same way -- the down combine writing partials, q|k|v normalising on load: q|k|v
     // 5.97 -> 7.59 us for a combine no shorter, 4.63 -> 4.72 us; with the combine inside the down launch,
     // B = 8 step 1.437 -> 1.446-1.465 ms, same box.)
@@ -604,7 +604,7 @@ struct DevStepIn {
 };
 
 // The fragment-major images of every layer's gate|up, q|k|v, o_proj and down weights that the batched (B >= 3)
-// decode projections read (kernels_gemv_mfma.hip; round 5), (re)built on stream s after a pgmi_prepare.  If the
+// decode projections read (kernels_gemv_mfma.hip), (re)built on stream s after a pgmi_prepare.  If the
 // 3.96 GB (at the 3B shapes) cannot be allocated the batched decode reads the row-major weights instead (the
 // same values in the same lanes: bit-identical results, slower), so the context stays usable.
 static int ensure_mf_image(pgmi_ctx* x, hipStream_t s) {

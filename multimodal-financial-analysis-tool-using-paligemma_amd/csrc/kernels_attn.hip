@@ -1188,20 +1188,20 @@ static size_t attn_full_lds(int head_dim, int Lk) {
 void attention_prefill(hipStream_t s, int head_dim, const AttnArgs& a) {
     int v = g_attn_force;
     if (v < 0) {
-        // measured on MI355X (tools/probes/attn_bench.py, round 1), us per call:
+        // measured on MI355X (tools/probes/attn_bench.py), us per call:
         //   SigLIP 224 (256 rows x 16 heads):  16-row 16.4 | RG2xKSPL4 10.8 | RG4xKSPL2 13.5
         //   SigLIP 448 (1024 x 16):            16-row 153.5 | RG4xKSPL4 32.4 | RG4xKSPL2 36.0
         //   Gemma 224 (288 x 8 heads, MQA):    16-row 21.9 | RG4xKSPL2 26.1 | RG2xKSPL2 26.4
         //   Gemma 448 (1056 x 8):              16-row 159.5 | RG4xKSPL2 61.3 | RG2xKSPL2 122.7
-        // round 3 (same probe, graph-replayed): the one-pass key-split kernel k_attn_fs (variant 9)
+        // same probe, graph-replayed: the one-pass key-split kernel k_attn_fs (variant 9)
         //   Gemma 224 12.2 (full_pre 15.1) | Gemma 448 31.7 (tiled RG4xKSPL2 52.5) | SigLIP 448 24.4 (31.8);
         //   SigLIP 224 stays on k_attn_short at one image (6.7 against 10.6); at 8 images
         //   (tools/probes/plan_sweep.py --batch 8, whole tower) k_attn_fs: tower 4204 -> 3835 us
         const long rows = (long)a.Lq * a.G * a.n_kv * a.B;
         v = head_dim == 256 ? 9 : (a.Lk <= 256 && rows <= 4096) ? 7 : 9;
-        // round 6: Gemma at one 224 px image (288 queries x 8 heads, 288 keys: no key split, 36 workgroups of
+        // Gemma at one 224 px image (288 queries x 8 heads, 288 keys: no key split, 36 workgroups of
         // 4 compute waves) takes 2 compute waves per workgroup, 72 workgroups over the same keys: in situ LM
-        // prefill 2,408.7 -> 2,394.0 us (gpurun_out r6g, variant 82; 1 wave, 81: 2,396.0)
+        // prefill 2,408.7 -> 2,394.0 us (1 wave: 2,396.0)
         if (head_dim == 256 && (a.Lk + 31) / 32 < 16 && (rows + 31) / 32 <= 256) v = 82;
     }
     if ((v == 81 || v == 82) && head_dim == 256) {  // one pass, 1 / 2 compute waves per workgroup, one key range

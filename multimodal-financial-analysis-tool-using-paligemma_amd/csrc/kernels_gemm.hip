@@ -433,7 +433,7 @@ __device__ __forceinline__ void vm_wait_tiles(int n) {
 // sit on one XCD and its L2 serves the panel to all but the first; only panels at a run boundary
 // are fetched by two XCDs.
 //
-// Round 4: when the grid splits into 8 equal blocks of bm row tiles x bn column tiles x bs K slices
+// When the grid splits into 8 equal blocks of bm row tiles x bn column tiles x bs K slices
 // (the host's xcd_block picks the shape that minimises the bytes each XCD must bring into its L2 --
 // bs/S of K x (bm row panels + bn weight panels) -- and passes it as `code`: bm | bn << 6 | bs << 14;
 // bit 30 is k_gemm_w's weight cache policy), XCD x takes block x instead of a run: the batched prefill
@@ -781,7 +781,7 @@ __global__ void __launch_bounds__(64 * (NW + LW), 1) k_gemm_w(const uint16_t* __
     constexpr bool PIPE = !RL && PGMI_GEMM_W_PIPE && TM <= 9 && EPI != EPI_ROPE &&  // (RoPE: its operands spill)
                           2 * (TM + NB * TN) * 4 + NB * TM * TN * 4 <= 200;
     if constexpr (RL) {
-    // In-wave reload (round 6, the RL configurations: one compute wave per SIMD with a wide wave tile, so each
+    // In-wave reload (the RL configurations: one compute wave per SIMD with a wide wave tile, so each
     // fragment read feeds 2 NB TN MFMAs): one set of A fragments, each row tile's reloaded for the next 32-deep
     // step right behind the MFMAs that read it, and two sets of B fragments (the next step's read first), so
     // the step's later rows multiply while the next step's fragments land -- a single wave overlaps its own LDS
@@ -1304,7 +1304,7 @@ enum Cfg : int {
     // 8-phase (k_gemm_8p): 2x4 waves, BN 256 (dual: 128 gate + 128 up), two K-tile buffers
     E256 = 36,     // TM 8: 256 rows
     E192 = 37,     // TM 6: 192 rows
-    // round 6: k_gemm_w's in-wave reload mode (W288w's tiles; bit-identical results)
+    // k_gemm_w's in-wave reload mode (W288w's tiles; bit-identical results)
     R288w = 38,    // 2x4 compute waves, TM 9, BN 128 (dual 64 + 64), 3 slots
     kNumCfg = 39,
 };
@@ -1353,25 +1353,25 @@ static Plan choose(int M, int N, int K, bool dual) {
         const int bn = (dual && c >= P288w) ? bns[c] / 2 : bns[c];
         return {(Cfg)c, bms[c], bn, dual && c < P288w ? 1 : (g_force_split > 0 ? g_force_split : 1)};
     }
-    // Measured on MI355X (tools/gemm_sweep.py; GPU time of graph-replayed calls, round 1): the
+    // Measured on MI355X (tools/gemm_sweep.py; GPU time of graph-replayed calls): the
     // PaliGemma prefill shapes at 224 px (M = 256 vision / 288 text rows) and 448 px (1024 /
     // 1056 rows).  Small GEMMs want every CU busy with little A per CU (64 x 64 tiles, 6-slot
     // ring, no split: the epilogue stays in the GEMM); the dual gate/up and K = 16384 down
     // projections want full-M panels that read each weight byte once.
     struct Entry { int M, N, K; bool dual; Cfg cfg; int split; };
     static const Entry table[] = {
-        // round 2: tools/gemm_sweep.py --cold (every call reads its weights from HBM, as the layer
+        // tools/gemm_sweep.py --cold (every call reads its weights from HBM, as the layer
         // loop does); W* = warp-specialised (k_gemm_w), P*s* = shallow rings
         {288, 2560, 2048, false, W64x64, 1},    // text q|k|v            10.8 us
-        // text rows, round 3 in situ (tools/probes/plan_sweep.py --target lm: the generate loop's whole
+        // text rows, in situ (tools/probes/plan_sweep.py --target lm: the generate loop's whole
         // language-model prefill timed per candidate, split partials reduced by the residual + RMSNorm)
         {288, 2048, 2048, false, W128x128, 4},  // text o_proj           LM -45 us vs W64x64 unsplit
-        {288, 16384, 2048, true, R288w, 1},     // text gate|up (GeGLU)  LM -27 us vs W288w (round 3, W288n); round 6:
+        {288, 16384, 2048, true, R288w, 1},     // text gate|up (GeGLU)  LM -27 us vs W288w (W288n);
                                                 // the in-wave reload form of the same tiles, bit-identical, isolated
-                                                // 47.2 -> 40.5 us (cold), in situ -7 us per LM prefill (gpurun_out r6i)
-        {288, 2048, 16384, false, W288n, 8},    // text down             round 6 in situ: LM -26 / -50 us vs W128x128
-                                                // split 4 on two boxes (gpurun_out r6b / r6e; round 3 had the opposite)
-        // vision rows: round 3, in situ (tools/probes/plan_sweep.py: the whole tower timed per
+                                                // 47.2 -> 40.5 us (cold), in situ -7 us per LM prefill
+        {288, 2048, 16384, false, W288n, 8},    // text down             in situ: LM -26 / -50 us vs W128x128
+                                                // split 4 on two boxes (an earlier build had the opposite)
+        // vision rows: in situ (tools/probes/plan_sweep.py: the whole tower timed per
         // candidate; split-K partials of out_proj / fc2 are reduced by the residual + LayerNorm kernel)
         {256, 3456, 1152, false, P64x64s4, 1},  // vision q|k|v          tower -17 us vs W64x64
         {256, 1152, 1152, false, P64x64s4, 3},  // vision out_proj       tower -38 us vs P32x64s4 unsplit
@@ -1383,7 +1383,7 @@ static Plan choose(int M, int N, int K, bool dual) {
         {1056, 2048, 2048, false, W128x128, 1}, // 448 px text o_proj    19.5 us (P96x64s3 23.9)
         {1056, 16384, 2048, true, E192, 1},     // 448 px gate|up       135.5 us (W352w 149.8); in situ LM 5688 -> 5538 us
         {1056, 2048, 16384, false, E192, 5},    // 448 px down          (W288w split 4 79.1 us); in situ 5688 -> 5539 us;
-                                                // round 4 in situ (profiles/r04_plan_sweeps.txt): split 5 (240 WGs) 5294 -> 5271 us
+                                                // in situ (profiles/r04_plan_sweeps.txt): split 5 (240 WGs) 5294 -> 5271 us
         {1024, 3456, 1152, false, W128x128, 1}, // 448 px vision q|k|v   18.3 us (was 24.6)
         {1024, 1152, 1152, false, P96x64s4, 1}, // 448 px vision out     10.6 us (P32x64s4 13.7)
         {1024, 4304, 1152, false, W288w, 1},    // 448 px vision fc1     25.1 us (exp/rcp GELU; was 29.5)

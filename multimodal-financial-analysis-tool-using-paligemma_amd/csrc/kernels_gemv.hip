@@ -112,7 +112,7 @@ void gemv_o_attn(hipStream_t s, int B, int G, const float* part, int max_chunks,
         return;
     }
     // grid capped so each workgroup's combine prologue is amortised over 8 output rows (256 / 128 / 64
-    // measured in round 4: 952 / 928-939 / 894-899 tok/s, profiles/r04_b1_probes_ab.txt)
+    // measured: 952 / 928-939 / 894-899 tok/s, profiles/r04_b1_probes_ab.txt)
     if (B <= 1) launch_gemv<1, 4, 2, GV_ORES>(s, a, 256);
     else if (B <= 2) launch_gemv<2, 4, 2, GV_ORES>(s, a, 256);
     else if (B <= 4) launch_gemv<4, 4, 1, GV_ORES>(s, a, 256);

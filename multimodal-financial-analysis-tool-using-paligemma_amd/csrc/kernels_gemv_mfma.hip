@@ -878,7 +878,7 @@ void gemv_mf_geglu(hipStream_t s, const GemvArgs& a) {  // K = 2048, gate|up row
     // 1,024 row groups grid-stride, so each stages its 8 normalised rows for two groups; same-box A/B
     // (tools/b8_ab.sh) B = 8 step 1.737 -> 1.681 ms against the one-workgroup-per-CU LDS-DMA ring
     // (k_gemv_ml, 4 waves x 3-deep rings); 256 / 384 / 1,024 workgroups and 2 or 8 K-split waves
-    // measured slower (1.746-2.051 ms); the unstaged form re-swept in round 4 (profiles/r04_gu_blocks_ab.txt:
+    // measured slower (1.746-2.051 ms); the unstaged form swept again (profiles/r04_gu_blocks_ab.txt:
     // 512 best against 384 / 768 / 1,024)
     // (a.ssq: x = h, normalised on load from o_proj's partial sums of squares -- unstaged, norm_w read)
     // a.Wf: the fragment-major weight image (1-KiB lane-linear loads; the decode step passes it)
@@ -919,7 +919,7 @@ void gemv_mf_ores(hipStream_t s, const GemvArgs& a, uint16_t* o) {
 
 int gemv_mf_logits(hipStream_t s, const GemvArgs& a, int max_blocks) {  // K = 2048
     // (the register-streamed form at 512 / 1,024 / 2,048 workgroups measured no faster: 1.741-1.768 ms; again in
-    // round 5 with the peeled loop: B = 8 step 1.283 -> 1.330-1.341 ms, profiles/r05_b8_lm_mf_ab.txt)
+    // with the peeled loop: B = 8 step 1.283 -> 1.330-1.341 ms, profiles/r05_b8_lm_mf_ab.txt)
     const int blocks = ms_blocks(a.n_units, max_blocks < 256 ? max_blocks : 256);
     launch_ml<GV_LOGITS, 1, 2048, 6>(s, a, blocks, 1, nullptr);
     return blocks;

@@ -10,7 +10,7 @@ At every prefill (full_check) the version counters of every parameter the sample
 checked too: the weights engine.prepare() derives tensors from (the text layers' projections -> the
 batched decode's fragment-major images, the patch embedding -> its padded copy) and any parameter that is
 not a slab view (its in-place update never reaches the slab).  A change there re-copies those parameters,
-drops the pending greedy lookahead and re-runs prepare() (round-6 verdict: an in-place update of an
+drops the pending greedy lookahead and re-runs prepare() (an in-place update of an
 unsampled weight left the derived images and a pending lookahead stale).
 """
 from __future__ import annotations

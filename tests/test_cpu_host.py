@@ -227,7 +227,7 @@ def test_ablation_patches_restated_match_reference_semantics():
 
 
 def test_prefill_gemm_shape_labels(tmp_path):
-    """tools/prefill_gemm_shapes.py labels the prefill MLP GEMMs of a kernel trace by template (round 6: the
+    """tools/prefill_gemm_shapes.py labels the prefill MLP GEMMs of a kernel trace by template (the
     M = 288 down runs W288n split 8, its own template, and o_proj W128x128 split 4); a W288w split launch is
     the 8-image down only right after the 8-image gate|up -- the per-shape figures bench.py's in-situ
     prefill_gemm_roofline is checked against."""

@@ -65,7 +65,7 @@ def test_inference_loop_pattern():
 
 def test_in_place_ops_after_materialization_reach_every_read():
     """A real (B, L, V) tensor has one storage: in-place ops on it, or writes through a last-row
-    view, must be seen by later last-row reads (ADVICE r02)."""
+    view, must be seen by later last-row reads."""
     x, full, last, calls = _make()
     x.materialize()
     x.div_(2.0)                                   # tensor method through __getattr__, in place

@@ -47,7 +47,7 @@ def logit_stats(label, ours, ref_bf16, ref_fp32=None):
 STEP_FLOOR_FACTOR = 1.45  # per step: rel-L2 vs reference bf16 <= max(2e-2, 1.45 x the reference's own error)
 MEAN_FLOOR_FACTOR = 1.25  # over the steps: mean <= max(2e-2, 1.25 x the reference's mean error)
 # module-level chains (assert_within_floor: one layer or block against the oracle, base 1e-2) keep the
-# round-4 factor: their floors are a single module's rounding noise, not a whole model's
+# earlier factor: their floors are a single module's rounding noise, not a whole model's
 MODULE_FLOOR_FACTOR = 1.6
 
 
