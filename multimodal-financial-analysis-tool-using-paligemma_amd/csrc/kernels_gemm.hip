@@ -20,6 +20,7 @@
 
 #include "common.h"
 #include "launch.h"
+#include "plan.h"
 
 #include <cstdlib>
 #include <type_traits>
@@ -977,12 +978,12 @@ __global__ void __launch_bounds__(64 * (NW + LW), 1) k_gemm_w(const uint16_t* __
 }
 
 // ---------------------------------------------------------------- 8-phase GEMM (large M)
-// BM x 256 x 64 tiles (BM = 32 TM: 256 at TM 8), one 512-thread workgroup per CU, 8 waves in a
+// BM x 256 x 64 tiles (BM = 32 TM: 64 at TM 2 to 256 at TM 8), one 512-thread workgroup per CU, 8 waves in a
 // 2 (M) x 4 (N) grid, each wave TM x 4 MFMA tiles (TM x 2 gate + TM x 2 up for the dual GeGLU GEMM).
-// A wave's output splits into 4 quadrants (row half qa x column half qb); the LDS image of a K-tile
-// is cut the same way into 4 half-tiles -- A_qa = the qa-th row half of BOTH wave rows, B_qb = the
-// qb-th column half of all 4 wave columns -- so each phase reads exactly one A half and / or one B
-// half.  Two K-tiles per iteration, 8 phases (quadrant order (0,0) (0,1) (1,1) (1,0): every phase
+// A wave's output splits into 4 quadrants (row half qa x column half qb; of an odd TM the first row half has one
+// tile more); the LDS image of a K-tile is cut the same way into 4 half-tiles -- A_qa = the qa-th row half of BOTH
+// wave rows, B_qb = the qb-th column half of all 4 wave columns -- so each phase reads exactly one A half and / or
+// one B half.  Two K-tiles per iteration, 8 phases (quadrant order (0,0) (0,1) (1,1) (1,0): every phase
 // but the first reuses the other operand's fragments from registers), each phase
 //   ds_read its fragments | LDS-DMA one half-tile of a later K-tile | [vmcnt] | s_barrier |
 //   lgkmcnt(0) | 16 MFMAs (setprio 1) | s_barrier
@@ -1004,15 +1005,14 @@ template <int TM, int EPI, bool SPLIT, class G>
 __device__ __forceinline__ void gemm_8p(const uint16_t* __restrict__ A, int lda, const uint16_t* __restrict__ W, int ldw, int M,
                                         int N, int K, int kt_per_split, const EpiArgs& ea, float* __restrict__ ws, long up_off,
                                         int n_mt, int code, G g) {
-    static_assert(TM % 2 == 0, "row halves of whole 16-row tiles");
+    static_assert(TM >= 2 && TM <= 8, "two row halves; 160 KiB of LDS");
     constexpr bool DUAL = epi_dual(EPI);
-    constexpr int H = TM / 2;                 // row tiles per quadrant
+    constexpr int H0 = (TM + 1) / 2, H1 = TM / 2;  // row tiles of the two row halves
     constexpr int BM = 32 * TM;
-    constexpr int HAR = 16 * TM;              // rows of an A half image (H tiles of each wave row)
-    constexpr int HAB = HAR * 128, HBB = 128 * 128;
-    constexpr int PA = HAR / 8, PB = 16;      // 1-KiB pieces per half
-    constexpr int GA = (PA + 7) / 8, GB = PB / 8;
-    constexpr int TB = 2 * HAB + 2 * HBB;     // one K-tile buffer: A0 A1 B0 B1
+    constexpr int AB1 = 32 * H0 * 128, BB0 = BM * 128, HBB = 128 * 128;  // offsets of A1 and B0, bytes of a B half
+    constexpr int PA0 = 4 * H0, PA1 = 4 * H1;      // 1-KiB pieces per A half (H tiles of each wave row)
+    constexpr int GA0 = (PA0 + 7) / 8, GA1 = (PA1 + 7) / 8, GB = 2;  // a wave's LDS-DMA instructions per half
+    constexpr int TB = BB0 + 2 * HBB;              // one K-tile buffer: A0 A1 B0 B1
     extern __shared__ __attribute__((aligned(16))) uint8_t sm8[];
 
     const int tid = threadIdx.x, lane = tid & 63;
@@ -1037,23 +1037,23 @@ __device__ __forceinline__ void gemm_8p(const uint16_t* __restrict__ A, int lda,
     const int nkt = kt1 - kt0;
     if (nkt <= 0) return;
 
-    // per-lane DMA sources (k = 0 of the tile's columns); piece p = wave + 8 i, pieces past the half
-    // repeat an earlier one (same bytes to the same LDS address)
-    const uint16_t* sa[2][GA];
-    int la[GA];
+    // per-lane DMA sources (k = 0 of the tile's columns); piece p = wave + 8 i, pieces past the half repeat an earlier
+    // one (same bytes to the same LDS address: waves that issue one fewer instead, with a wait of their own, took 46 us a
+    // round of 192-row tiles of K = 2048, repeats 43)
+    const uint16_t* sa[2][GA0];
+    int la[2][GA0];
     const uint16_t* sb[2][GB];
     int lb[GB];
     const int prow = lane >> 3, pch = lane & 7;
 #pragma unroll
-    for (int i = 0; i < GA; ++i) {
-        int pc = wave + 8 * i;
-        if (pc >= PA) pc -= PA;
-        la[i] = pc * 1024;
-        const int ir = pc * 8 + prow;
-        const int wr = ir / (8 * TM), r = ir % (8 * TM);
+    for (int i = 0; i < GA0; ++i) {
 #pragma unroll
         for (int qa = 0; qa < 2; ++qa) {
-            int row = m0 + wr * 16 * TM + qa * 8 * TM + r;
+            int pc = wave + 8 * i;
+            while (pc >= (qa ? PA1 : PA0)) pc -= qa ? PA1 : PA0;
+            la[qa][i] = pc * 1024;
+            const int ir = pc * 8 + prow, hr = 16 * (qa ? H1 : H0);  // rows of a wave row in this half
+            int row = m0 + ir / hr * 16 * TM + qa * 16 * H0 + ir % hr;
             row = row < M ? row : M - 1;
             if constexpr (G::kGrouped) row = g.source(row);
             sa[qa][i] = A + (long)row * lda + ((pch ^ (ir & 7)) << 3);
@@ -1083,16 +1083,16 @@ __device__ __forceinline__ void gemm_8p(const uint16_t* __restrict__ A, int lda,
         if constexpr (PGMI_GEMM_DIAG & 2) return;
         kt = kt < kt1 ? kt : kt1 - 1;  // past the range: valid bytes into a buffer never read again
         const int kel = kt * 64;
-        const int base = buf * TB + qa * HAB;
+        const int base = buf * TB + qa * AB1;
 #pragma unroll
-        for (int i = 0; i < GA; ++i)
-            __builtin_amdgcn_global_load_lds(reinterpret_cast<const void*>(sa[qa][i] + kel), PGMI_8P_LDS(base + la[i]), 16, 0, 0);
+        for (int i = 0; i < (qa ? GA1 : GA0); ++i)
+            __builtin_amdgcn_global_load_lds(reinterpret_cast<const void*>(sa[qa][i] + kel), PGMI_8P_LDS(base + la[qa][i]), 16, 0, 0);
     };
     auto stageB = [&](int qb, int kt, int buf) {
         if constexpr (PGMI_GEMM_DIAG & 2) return;
         kt = kt < kt1 ? kt : kt1 - 1;
         const int kel = kt * 64;
-        const int base = buf * TB + 2 * HAB + qb * HBB;
+        const int base = buf * TB + BB0 + qb * HBB;
 #pragma unroll
         for (int i = 0; i < GB; ++i)
             __builtin_amdgcn_global_load_lds(reinterpret_cast<const void*>(sb[qb][i] + kel), PGMI_8P_LDS(base + lb[i]), 16, 0, 0);
@@ -1104,21 +1104,22 @@ __device__ __forceinline__ void gemm_8p(const uint16_t* __restrict__ A, int lda,
     for (int i = 0; i < TM; ++i)
 #pragma unroll
         for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-    short8 fa[H][2], fb[2][2][2];             // fb[qb]: B0's fragments stay live from phase 1 to 4
+    short8 fa[H0][2], fb[2][2][2];            // fb[qb]: B0's fragments stay live from phase 1 to 4
     const int sw = lane & 7;
-    const int arow = (wm * 8 * TM + (lane & 15)) * 128;  // + i * 16 rows
+    const int arow0 = (wm * 16 * H0 + (lane & 15)) * 128, arow1 = (wm * 16 * H1 + (lane & 15)) * 128;  // + i * 16 rows
     const int brow = (wn * 32 + (lane & 15)) * 128;      // + jj * 16 rows
-    auto readA = [&](int qa, int buf) {
-        const uint8_t* b = sm8 + buf * TB + qa * HAB + arow;
+    auto readA = [&](auto qa_c, int buf) {
+        constexpr int QA = decltype(qa_c)::value;
+        const uint8_t* b = sm8 + buf * TB + QA * AB1 + (QA ? arow1 : arow0);
 #pragma unroll
-        for (int i = 0; i < H; ++i)
+        for (int i = 0; i < (QA ? H1 : H0); ++i)
 #pragma unroll
             for (int kk = 0; kk < 2; ++kk)
                 fa[i][kk] = *reinterpret_cast<const short8*>(b + i * 16 * 128 + (((kk * 4 + (lane >> 4)) ^ sw) << 4));
     };
     auto readB = [&](auto qb_c, int buf) {
         constexpr int QB = decltype(qb_c)::value;
-        const uint8_t* b = sm8 + buf * TB + 2 * HAB + QB * HBB + brow;
+        const uint8_t* b = sm8 + buf * TB + BB0 + QB * HBB + brow;
 #pragma unroll
         for (int jj = 0; jj < 2; ++jj)
 #pragma unroll
@@ -1129,7 +1130,7 @@ __device__ __forceinline__ void gemm_8p(const uint16_t* __restrict__ A, int lda,
         constexpr int QA = decltype(qa_c)::value, QB = decltype(qb_c)::value;
         if constexpr (PGMI_GEMM_DIAG & 1) {
 #pragma unroll
-            for (int i = 0; i < H; ++i)
+            for (int i = 0; i < (QA ? H1 : H0); ++i)
 #pragma unroll
                 for (int kk = 0; kk < 2; ++kk) asm volatile("" ::"v"(fa[i][kk]), "v"(fb[QB][0][kk]), "v"(fb[QB][1][kk]));
             return;
@@ -1137,14 +1138,13 @@ __device__ __forceinline__ void gemm_8p(const uint16_t* __restrict__ A, int lda,
 #pragma unroll
         for (int kk = 0; kk < 2; ++kk)
 #pragma unroll
-            for (int i = 0; i < H; ++i)
+            for (int i = 0; i < (QA ? H1 : H0); ++i)
 #pragma unroll
                 for (int jj = 0; jj < 2; ++jj)
-                    acc[QA * H + i][QB * 2 + jj] = mfma16(fa[i][kk], fb[QB][jj][kk], acc[QA * H + i][QB * 2 + jj]);
+                    acc[QA * H0 + i][QB * 2 + jj] = mfma16(fa[i][kk], fb[QB][jj][kk], acc[QA * H0 + i][QB * 2 + jj]);
     };
     using I0 = std::integral_constant<int, 0>;
     using I1 = std::integral_constant<int, 1>;
-    static_assert(GA == GB, "one vmcnt for every half-tile");
 #define PGMI_8P_SB() __builtin_amdgcn_sched_barrier(0)
 #define PGMI_8P_TAIL(QAC, QBC, DO)                                      \
     do {                                                                \
@@ -1157,8 +1157,9 @@ __device__ __forceinline__ void gemm_8p(const uint16_t* __restrict__ A, int lda,
         PGMI_8P_SB();                                                   \
         __builtin_amdgcn_s_barrier();                                   \
     } while (0)
-    // the half-tile the next phase reads was issued four half-tiles (three phases) before this wait
-#define PGMI_8P_VMCNT() asm volatile("s_waitcnt vmcnt(%0)" ::"n"(4 * GA) : "memory")
+    // the half-tile the next phase reads was issued four half-tiles (three phases) before this wait: the four after it,
+    // one of each kind, may be in flight
+#define PGMI_8P_VMCNT() asm volatile("s_waitcnt vmcnt(%0)" ::"n"(GA0 + GA1 + 2 * GB) : "memory")
 
     // Phase p reads (buffer of its K-tile): 1: A0 B0, 2: B1, 3: A1, 4: none (A1 and the kept B0).
     // Wave row 1 runs one barrier behind wave row 0 (one extra s_barrier up front, matched by wave
@@ -1180,15 +1181,15 @@ __device__ __forceinline__ void gemm_8p(const uint16_t* __restrict__ A, int lda,
         const int T = kt0 + t;
         const bool has1 = t + 1 < nkt;
         // ---- K-tile T from buffer 0
-        readA(0, 0); readB(I0{}, 0); PGMI_8P_SB(); stageB(1, T + 1, 1); PGMI_8P_VMCNT(); PGMI_8P_TAIL(I0, I0, true);
+        readA(I0{}, 0); readB(I0{}, 0); PGMI_8P_SB(); stageB(1, T + 1, 1); PGMI_8P_VMCNT(); PGMI_8P_TAIL(I0, I0, true);
         readB(I1{}, 0); PGMI_8P_SB(); stageA(1, T + 1, 1); PGMI_8P_VMCNT();              PGMI_8P_TAIL(I0, I1, true);
-        readA(1, 0); PGMI_8P_SB(); stageA(0, T + 2, 0);                                  PGMI_8P_TAIL(I1, I1, true);
+        readA(I1{}, 0); PGMI_8P_SB(); stageA(0, T + 2, 0);                                  PGMI_8P_TAIL(I1, I1, true);
         PGMI_8P_SB(); stageB(0, T + 2, 0); PGMI_8P_VMCNT();                              PGMI_8P_TAIL(I1, I0, true);
         // ---- K-tile T + 1 from buffer 1 (absent past an odd tile count: the phases keep their
         // barriers and stages, the MFMAs are skipped)
-        readA(0, 1); readB(I0{}, 1); PGMI_8P_SB(); stageB(1, T + 2, 0); PGMI_8P_VMCNT(); PGMI_8P_TAIL(I0, I0, has1);
+        readA(I0{}, 1); readB(I0{}, 1); PGMI_8P_SB(); stageB(1, T + 2, 0); PGMI_8P_VMCNT(); PGMI_8P_TAIL(I0, I0, has1);
         readB(I1{}, 1); PGMI_8P_SB(); stageA(1, T + 2, 0); PGMI_8P_VMCNT();              PGMI_8P_TAIL(I0, I1, has1);
-        readA(1, 1); PGMI_8P_SB(); stageA(0, T + 3, 1);                                  PGMI_8P_TAIL(I1, I1, has1);
+        readA(I1{}, 1); PGMI_8P_SB(); stageA(0, T + 3, 1);                                  PGMI_8P_TAIL(I1, I1, has1);
         PGMI_8P_SB(); stageB(0, T + 3, 1); PGMI_8P_VMCNT();                              PGMI_8P_TAIL(I1, I0, has1);
     }
     if (wm == 0) __builtin_amdgcn_s_barrier();  // the lagging row's last barrier
@@ -1259,179 +1260,6 @@ __global__ void __launch_bounds__(512, 1) k_gemm_8p(const uint16_t* __restrict__
 
 // (PGMI_GEMM_KERNELS_ONLY: the kernel templates alone -- kernels_matmul.hip instantiates its own few)
 #ifndef PGMI_GEMM_KERNELS_ONLY
-// Tile configurations (wave grid, per-wave MFMA tiles).  BM = WGM*TM*16, BN = WGN*TN*16.
-enum Cfg : int {
-    C288x64 = 0,   // 6x1 waves, 3x4 tiles  (text rows: M = 288 = 18 x 16)
-    C288x32 = 1,   // 6x1 waves, 3x2 tiles
-    C256x64 = 2,   // 4x1 waves, 4x4 tiles  (vision rows: M = 256)
-    C256x32 = 3,   // 4x1 waves, 4x2 tiles
-    C128x128 = 4,  // 2x2 waves, 4x4 tiles  (large M)
-    C128x64 = 5,   // 2x2 waves, 4x2 tiles
-    // panel GEMM (k_gemm_p, LDS-DMA ring): BM x BN output columns (dual gate/up: BN/2 columns x 2)
-    P288w = 6,     // TM 9,  BN 128, 3 slots
-    P256w = 7,     // TM 8,  BN 128, 3 slots
-    P352w = 8,     // TM 11, BN 128, 2 slots  (448 px text rows: M = 1056 = 3 x 352)
-    P288n = 9,     // TM 9,  BN 64,  3 slots
-    P256n = 10,    // TM 8,  BN 64,  3 slots
-    P128w = 11,    // TM 4,  BN 128, 3 slots
-    P288t = 12,    // TM 9,  BN 32,  4 slots  (2x2 waves, 1 column fragment each)
-    P256t = 13,    // 4x1 waves, TM 4, BN 32, 4 slots
-    P64x64 = 14,   // TM 2, BN 64,  6 slots   (small GEMMs: every CU busy, little A per CU)
-    P128x64 = 15,  // TM 4, BN 64,  6 slots
-    P64x128 = 16,  // TM 2, BN 128, 6 slots
-    P128x128 = 17, // TM 4, BN 128, 5 slots
-    P64x64d = 18,  // TM 2, BN 64,  10 slots
-    P128x64d = 19, // 4x1 waves, TM 2, BN 64, 6 slots
-    // 8 waves (2 per SIMD: one wave's LDS-DMA issue stalls overlap its partner's MFMAs)
-    Q288w = 20,    // 2x4 waves, TM 9,  BN 128, 3 slots
-    Q352w = 21,    // 2x4 waves, TM 11, BN 128, 2 slots
-    Q256w = 22,    // 2x4 waves, TM 8,  BN 128, 3 slots
-    Q288x256 = 23, // 2x4 waves, TM 9,  BN 256, 2 slots
-    // shallow rings (2-3 workgroups per CU: more k-tiles in flight per CU for the small GEMMs)
-    P64x64s3 = 24, // TM 2, BN 64, 3 slots
-    P64x64s4 = 25, // TM 2, BN 64, 4 slots
-    P32x64s4 = 26, // TM 1, BN 64, 4 slots
-    P64x32s4 = 27, // TM 2, BN 32, 4 slots
-    P96x64s4 = 28, // TM 3, BN 64, 4 slots (M = 288 = 3 x 96)
-    P96x64s3 = 29, // TM 3, BN 64, 3 slots
-    // warp-specialised (k_gemm_w): compute waves + 4 LDS-DMA loader waves
-    W288w = 30,    // 2x4 compute waves, TM 9,  BN 128, 3 slots
-    W288n = 31,    // 2x4 compute waves, TM 9,  BN 64,  3 slots
-    W64x64 = 32,   // 2x2 compute waves, TM 2,  BN 64,  6 slots
-    W352w = 33,    // 2x4 compute waves, TM 11, BN 128, 2 slots
-    W128x128 = 34, // 2x4 compute waves, TM 4,  BN 128, 4 slots
-    W128x64 = 35,  // 2x2 compute waves, TM 4,  BN 64,  5 slots
-    // 8-phase (k_gemm_8p): 2x4 waves, BN 256 (dual: 128 gate + 128 up), two K-tile buffers
-    E256 = 36,     // TM 8: 256 rows
-    E192 = 37,     // TM 6: 192 rows
-    // k_gemm_w's in-wave reload mode (W288w's tiles; bit-identical results)
-    R288w = 38,    // 2x4 compute waves, TM 9, BN 128 (dual 64 + 64), 3 slots
-    kNumCfg = 39,
-};
-static_assert(kNumCfg == kGemmCfgs, "launch.h kGemmCfgs");
-
-struct Plan {
-    Cfg cfg;
-    int bm, bn, split;
-};
-
-static int g_force_cfg = -1, g_force_split = 0;  // tuning override (pgmi_tune_gemm)
-
-void gemm_force_plan(int cfg, int split) {
-    g_force_cfg = cfg;
-    g_force_split = split;
-}
-
-// per-shape plan overrides (tuning hook pgmi_tune_gemm_shape): in-situ sweeps of one GEMM of a
-// forward while the others keep their measured plans
-struct ShapePlan {
-    int M, N, K;
-    bool dual;
-    int cfg, split;
-};
-static ShapePlan g_shape_plans[16];
-static int g_n_shape_plans = 0;
-
-int gemm_force_shape(int M, int N, int K, int dual, int cfg, int split) {
-    for (int i = 0; i < g_n_shape_plans; ++i)
-        if (g_shape_plans[i].M == M && g_shape_plans[i].N == N && g_shape_plans[i].K == K &&
-            g_shape_plans[i].dual == (dual != 0)) {
-            g_shape_plans[i] = g_shape_plans[--g_n_shape_plans];
-            break;
-        }
-    if (cfg < 0) return 0;
-    if (g_n_shape_plans >= 16) return -1;
-    g_shape_plans[g_n_shape_plans++] = {M, N, K, dual != 0, cfg, split < 1 ? 1 : split};
-    return 0;
-}
-
-static Plan choose(int M, int N, int K, bool dual) {
-    if (g_force_cfg >= 0) {
-        static const int bms[] = {288, 288, 256, 256, 128, 128, 288, 256, 352, 288, 256, 128, 288, 256, 64, 128, 64, 128, 64, 128, 288, 352, 256, 288, 64, 64, 32, 64, 96, 96, 288, 288, 64, 352, 128, 128, 256, 192, 288};
-        static const int bns[] = {64, 32, 64, 32, 128, 64, 128, 128, 128, 64, 64, 128, 32, 32, 64, 64, 128, 128, 64, 64, 128, 128, 128, 256, 64, 64, 64, 32, 64, 64, 128, 64, 64, 128, 128, 64, 256, 256, 128};
-        const int c = g_force_cfg;
-        const int bn = (dual && c >= P288w) ? bns[c] / 2 : bns[c];
-        return {(Cfg)c, bms[c], bn, dual && c < P288w ? 1 : (g_force_split > 0 ? g_force_split : 1)};
-    }
-    // Measured on MI355X (tools/gemm_sweep.py; GPU time of graph-replayed calls): the
-    // PaliGemma prefill shapes at 224 px (M = 256 vision / 288 text rows) and 448 px (1024 /
-    // 1056 rows).  Small GEMMs want every CU busy with little A per CU (64 x 64 tiles, 6-slot
-    // ring, no split: the epilogue stays in the GEMM); the dual gate/up and K = 16384 down
-    // projections want full-M panels that read each weight byte once.
-    struct Entry { int M, N, K; bool dual; Cfg cfg; int split; };
-    static const Entry table[] = {
-        // tools/gemm_sweep.py --cold (every call reads its weights from HBM, as the layer
-        // loop does); W* = warp-specialised (k_gemm_w), P*s* = shallow rings
-        {288, 2560, 2048, false, W64x64, 1},    // text q|k|v            10.8 us
-        // text rows, in situ (tools/probes/plan_sweep.py --target lm: the generate loop's whole
-        // language-model prefill timed per candidate, split partials reduced by the residual + RMSNorm)
-        {288, 2048, 2048, false, W128x128, 4},  // text o_proj           LM -45 us vs W64x64 unsplit
-        {288, 16384, 2048, true, R288w, 1},     // text gate|up (GeGLU)  LM -27 us vs W288w (W288n);
-                                                // the in-wave reload form of the same tiles, bit-identical, isolated
-                                                // 47.2 -> 40.5 us (cold), in situ -7 us per LM prefill
-        {288, 2048, 16384, false, W288n, 8},    // text down             in situ: LM -26 / -50 us vs W128x128
-                                                // split 4 on two boxes (an earlier build had the opposite)
-        // vision rows: in situ (tools/probes/plan_sweep.py: the whole tower timed per
-        // candidate; split-K partials of out_proj / fc2 are reduced by the residual + LayerNorm kernel)
-        {256, 3456, 1152, false, P64x64s4, 1},  // vision q|k|v          tower -17 us vs W64x64
-        {256, 1152, 1152, false, P64x64s4, 3},  // vision out_proj       tower -38 us vs P32x64s4 unsplit
-        {256, 4304, 1152, false, P96x64s4, 1},  // vision fc1 (+GELU)    11.0 us (exp/rcp GELU; was 16.4)
-        {256, 1152, 4304, false, P96x64s4, 4},  // vision fc2            tower -19 us vs P64x64s4 split 3
-        {256, 1152, 640, false, P64x32s4, 1},   // patch embedding        5.3 us (was 6.6 on P64x64)
-        {256, 2048, 1152, false, P32x64s4, 1},  // multimodal projector   7.6 us
-        {1056, 2560, 2048, false, W128x128, 1}, // 448 px text q|k|v     21.3 us (P96x64s3 24.0 in the same sweep)
-        {1056, 2048, 2048, false, W128x128, 1}, // 448 px text o_proj    19.5 us (P96x64s3 23.9)
-        {1056, 16384, 2048, true, E192, 1},     // 448 px gate|up       135.5 us (W352w 149.8); in situ LM 5688 -> 5538 us
-        {1056, 2048, 16384, false, E192, 5},    // 448 px down          (W288w split 4 79.1 us); in situ 5688 -> 5539 us;
-                                                // in situ (profiles/r04_plan_sweeps.txt): split 5 (240 WGs) 5294 -> 5271 us
-        {1024, 3456, 1152, false, W128x128, 1}, // 448 px vision q|k|v   18.3 us (was 24.6)
-        {1024, 1152, 1152, false, P96x64s4, 1}, // 448 px vision out     10.6 us (P32x64s4 13.7)
-        {1024, 4304, 1152, false, W288w, 1},    // 448 px vision fc1     25.1 us (exp/rcp GELU; was 29.5)
-        {1024, 1152, 4304, false, W128x128, 3}, // 448 px vision fc2     in situ tower 2965 -> 2904 us vs W288w split 4
-        // 8 images per GPU as one batch (vision 2048 rows, text 2304 rows), cold sweep
-        {2048, 3456, 1152, false, W288w, 1},    // vision q|k|v          31.2 us (was 46.8)
-        {2048, 1152, 1152, false, W128x128, 1}, // vision out_proj       22.3 us (was 31.6)
-        {2048, 4304, 1152, false, W352w, 1},    // vision fc1            48.6 us (was 91.5)
-        {2048, 1152, 4304, false, W288w, 2},    // vision fc2            47.3 us (was 72.2)
-        {2048, 2048, 1152, false, W128x128, 1}, // projector             19.1 us (was 23.8)
-        {2304, 2560, 2048, false, Q256w, 1},    // text q|k|v            in situ LM 9047 -> 8902 us vs W288w + RoPE
-                                                // epilogue (61 us in situ: 160 workgroups); RoPE by k_rope_kv
-        {2304, 2048, 2048, false, W288n, 1},    // text o_proj           35.4 us (was 62.1)
-        {2304, 16384, 2048, true, E256, 1},     // text gate|up         261.8 us (W288w 301.8); in situ LM 10064 -> 9435 us
-        {2304, 2048, 16384, false, W288w, 2},   // text down            153.9 us (was 298.6)
-    };
-    static const int bms[] = {288, 288, 256, 256, 128, 128, 288, 256, 352, 288, 256, 128, 288, 256, 64, 128, 64, 128, 64, 128, 288, 352, 256, 288, 64, 64, 32, 64, 96, 96, 288, 288, 64, 352, 128, 128, 256, 192, 288};
-    static const int bns[] = {64, 32, 64, 32, 128, 64, 128, 128, 128, 64, 64, 128, 32, 32, 64, 64, 128, 128, 64, 64, 128, 128, 128, 256, 64, 64, 64, 32, 64, 64, 128, 64, 64, 128, 128, 64, 256, 256, 128};
-    auto mk = [&](Cfg c, int split) -> Plan { return {c, bms[c], dual ? bns[c] / 2 : bns[c], dual ? 1 : split}; };
-    for (int i = 0; i < g_n_shape_plans; ++i) {
-        const ShapePlan& o = g_shape_plans[i];
-        if (o.M == M && o.N == N && o.K == K && o.dual == dual) return mk((Cfg)o.cfg, o.split);
-    }
-    for (const Entry& e : table)
-        if (e.M == M && e.N == N && e.K == K && e.dual == dual) return mk(e.cfg, e.split);
-    // lock-step decode batches as GEMMs (M <= 16 rows; tools/gemm_sweep.py b8_*
-    // in isolation: gate|up 64x128 tiles 24.2 us, down 64x64 split 8 18.1 us)
-    if (M <= 16) {
-        if (dual) return mk(P64x128, 1);
-        if (K >= 8192) return mk(P64x64, 8);
-    }
-    // other shapes (batched prefill: M = B x 256 / 288 rows; other image sizes)
-    if (dual) return mk(M <= 288 || M >= 2048 ? W288w : W352w, 1);
-    if (K >= 8192) return mk(M <= 288 ? W288n : W288w, M <= 288 ? 8 : M <= 1056 ? 4 : 2);
-    const long t64 = (long)((M + 63) / 64) * ((N + 63) / 64);
-    if (t64 <= 256) return mk(P64x64, 1);
-    const long t128 = (long)((M + 127) / 128) * ((N + 127) / 128);
-    Plan p = mk(P128w, 1);
-    const int nkt = (K + 63) / 64;
-    while (t128 * p.split < 200 && p.split < 4 && nkt / (p.split * 2) >= 4) p.split *= 2;
-    return p;
-}
-
-size_t gemm_ws_bytes(int M, int N, int K) {
-    Plan p = choose(M, N, K, false);
-    return p.split > 1 ? (size_t)p.split * M * N * sizeof(float) : 0;
-}
-
 // host: the XCD block shape for xcd_tile's `code` argument, or 0 for the run order -- used only when
 // it cuts the bytes the 8 XCDs must fetch into their L2s by at least 20 %.  Memoised per launch shape
 // behind a mutex (contexts may be driven from several host threads).
@@ -1697,6 +1525,9 @@ static void launch_pcfg(hipStream_t s, const uint16_t* A, int lda, const uint16_
         case W128x64: launch_w<4, 2, 4, 2, 5, 4, EPI>(s, A, lda, W, ldw, M, N, K, ea, ws, p.split, up_off); break;
         case E256: launch_8p<8, EPI>(s, A, lda, W, ldw, M, N, K, ea, ws, p.split, up_off); break;
         case E192: launch_8p<6, EPI>(s, A, lda, W, ldw, M, N, K, ea, ws, p.split, up_off); break;
+        case E128: launch_8p<4, EPI>(s, A, lda, W, ldw, M, N, K, ea, ws, p.split, up_off); break;
+        case E160: launch_8p<5, EPI>(s, A, lda, W, ldw, M, N, K, ea, ws, p.split, up_off); break;
+        case E224: launch_8p<7, EPI>(s, A, lda, W, ldw, M, N, K, ea, ws, p.split, up_off); break;
         case R288w: launch_w<8, 2, 9, 2, 3, 4, EPI, true>(s, A, lda, W, ldw, M, N, K, ea, ws, p.split, up_off); break;
         default: break;
     }
@@ -1720,8 +1551,8 @@ static void launch_e(hipStream_t s, const uint16_t* A, int lda, const uint16_t* 
 
 int gemm(hipStream_t s, const uint16_t* A, int lda, const uint16_t* W, int ldw, int M, int N, int K, Epi epi,
          const EpiArgs& ea, float* ws, size_t ws_bytes, int up_offset_rows, bool defer) {
-    Plan p = choose(M, N, K, epi == EPI_GEGLU);
-    if ((p.cfg == E256 || p.cfg == E192) && K % 64 != 0) p.cfg = P128w;  // the 8-phase kernel has no K tail
+    Plan p = gemm_plan(M, N, K, epi == EPI_GEGLU, !defer ? AFTER_OWN : epi == EPI_STORE ? AFTER_ROPE : AFTER_NORM, ws_bytes);
+    if ((p.cfg == E256 || p.cfg == E192 || p.cfg >= E128) && K % 64 != 0) p.cfg = P128w;  // the 8-phase kernel has no K tail
     if (p.split > 1 && (size_t)p.split * M * N * sizeof(float) > ws_bytes) p.split = 1;
     if (p.split > 1 && N % 4 != 0) p.split = 1;  // the split-K epilogue works on 4 outputs per thread
     const long up_off = (long)up_offset_rows * ldw;
@@ -1763,9 +1594,9 @@ int gemm(hipStream_t s, const uint16_t* A, int lda, const uint16_t* W, int ldw, 
 }
 
 bool gemm_qkv_rope(hipStream_t s, const uint16_t* A, int lda, const uint16_t* W, int ldw, int M, int N, int K,
-                   const EpiArgs& ea) {
+                   const EpiArgs& ea, size_t ws_bytes) {
     if (N % 256 != 0 || N != (ea.nh + 2 * ea.nkv) * 256) return false;
-    const Plan p = choose(M, N, K, false);
+    const Plan p = gemm_plan(M, N, K, false, AFTER_ROPE, ws_bytes);
     if (p.split != 1) return false;
     // configurations with two 16-column tiles per wave and a tile width dividing 256
 #define P_(wm, tm, st) launch_p<4, wm, tm, 2, st, EPI_ROPE>(s, A, lda, W, ldw, M, N, K, ea, nullptr, 1, 0)

@@ -55,17 +55,16 @@ struct EpiArgs {
 // shape allows it (two 16-column tiles per wave, no split-K); false: nothing launched, the caller
 // runs gemm(EPI_STORE) + rope_kv_append
 bool gemm_qkv_rope(hipStream_t s, const uint16_t* A, int lda, const uint16_t* W, int ldw, int M, int N, int K,
-                   const EpiArgs& ea);
+                   const EpiArgs& ea, size_t ws_bytes);
 int gemm(hipStream_t s, const uint16_t* A, int lda, const uint16_t* W, int ldw, int M, int N, int K,
          Epi epi, const EpiArgs& ea, float* ws, size_t ws_bytes, int up_offset_rows = 0, bool defer = false);
-size_t gemm_ws_bytes(int M, int N, int K);
 void gemm_force_plan(int cfg, int split);  // cfg < 0: automatic
 int gemm_force_shape(int M, int N, int K, int dual, int cfg, int split);  // cfg < 0: remove the override
 // probe: the next GEMM kernel launched takes these events as its own start / stop (hipExtLaunchKernelGGL)
 void gemm_probe_events(hipEvent_t start, hipEvent_t stop);
 // host replica of the panel / 8-phase GEMMs' workgroup -> tile order (CPU test); returns the XCD block code
 int gemm_tile_order(int n_mt, int n_nt, int S, int BM, int BN, int K, int* mt, int* nt, int* z);
-constexpr int kGemmCfgs = 39;              // tile configurations (kernels_gemm.hip Cfg)
+constexpr int kGemmCfgs = 42;              // tile configurations (kernels_gemm.hip Cfg)
 
 // ---------------------------------------------------------------- decode GEMV
 struct StepState {  // device-resident decode step (read by kernels -> graph-replayable)

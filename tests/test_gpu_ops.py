@@ -274,7 +274,7 @@ def test_attention_forced_variant(eng, variant, B, Lq, Lk, H, Hkv, d, scale):
     assert rel_l2(np32(o), _attn_ref(q, k, v, scale)) < 1e-2
 
 
-@pytest.mark.parametrize("cfg", [36, 37])
+@pytest.mark.parametrize("cfg", [36, 37, 39, 40, 41])
 @pytest.mark.parametrize("M,N,K,epi,split", [
     (1056, 512, 2048, "geglu", 1),     # 448 px gate|up shape (rows past 1056: clamped, never stored)
     (300, 384, 1024, "store", 1),      # ragged M, N not a multiple of the tile
@@ -282,7 +282,7 @@ def test_attention_forced_variant(eng, variant, B, Lq, Lk, H, Hkv, d, scale):
     (256, 512, 192, "store", 1),       # 3 K-tiles: an odd tile count (the last iteration's second half idle)
 ])
 def test_gemm_8phase(eng, cfg, M, N, K, epi, split):
-    """The 8-phase large-M GEMM (k_gemm_8p, plans E256 / E192) forced through the tuning hook."""
+    """The 8-phase large-M GEMM (k_gemm_8p, plans E256 / E192 / E128 / E160 / E224) forced through the tuning hook."""
     from pgmi import _native as NN
     from pgmi._native import EPI
     rng = np.random.default_rng(M + N + K + cfg)
@@ -303,3 +303,27 @@ def test_gemm_8phase(eng, cfg, M, N, K, epi, split):
     finally:
         NN.check(eng.lib.pgmi_tune_gemm(-1, 0))
     assert rel_l2(got, ref) < tol
+
+
+@pytest.mark.parametrize("M,N,K,epi", [
+    (17, 2560, 2048, "store"), (33, 200, 72, "bias"), (257, 1152, 1152, "bias_res"), (289, 1001, 2048, "store"),
+    (304, 2048, 4096, "res"), (512, 4304, 1152, "bias_gelu"), (577, 1152, 4304, "bias_res"), (640, 1024, 2048, "geglu"),
+    (783, 2048, 1160, "res"), (1281, 3456, 1152, "bias"), (1540, 520, 2048, "geglu"), (2049, 1152, 1152, "bias_res"),
+])
+def test_gemm_planned_matches_general(eng, M, N, K, epi):
+    """The tiles that the cost rule picks (plan.h: every form up to 288 rows, the 8-phase heights, K tails, rows and columns
+    past the last tile) against the general register-staged tiles, forced through the tuning hook.  Both sum in fp32, in
+    another order, and round to bf16 once per rounding point: they differ by single roundings."""
+    from pgmi import _native as NN
+    from pgmi._native import EPI
+    rng = np.random.default_rng(M + 3 * N + K)
+    A, b, r = bf(rand(rng, M, K)), bf(rand(rng, N)), bf(rand(rng, M, N))
+    Wt = bf(rand(rng, N * (2 if epi == "geglu" else 1), K, scale=1 / np.sqrt(K)))
+    run = lambda: _gemm(eng, A, Wt, EPI.get(epi, 7), bias=b, res=r, geglu=epi == "geglu")  # noqa: E731
+    got = run()
+    NN.check(eng.lib.pgmi_tune_gemm(5, 1))
+    try:
+        ref = run()
+    finally:
+        NN.check(eng.lib.pgmi_tune_gemm(-1, 0))
+    assert rel_l2(got, ref) < 3e-3
