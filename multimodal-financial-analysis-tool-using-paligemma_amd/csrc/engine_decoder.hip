@@ -72,7 +72,13 @@ struct DecoderState {
     float *inv = nullptr, *ew = nullptr, *egate = nullptr;
     int *esel = nullptr, *elist = nullptr, *ecnt = nullptr, *eactive = nullptr;
     int zero_words = 0;  // the counters and the number of used experts
-    size_t slab_bytes = 0;
+    int slab_n = 0;  // columns of the widest product into slabs
+    // room for the K slabs of a step of these rows (not of the largest step so far: a step's sums are cut the same way
+    // whatever ran before it): four of them up to 160 MB, one of any step
+    size_t slab_bytes(int rows) const {
+        const size_t one = (size_t)rows * slab_n * 4;
+        return std::max({one, (size_t)32 << 20, std::min(4 * one, (size_t)160 << 20)});
+    }
     int ldh = 0, ld0 = 0, ld1 = 0, ld2 = 0, ldd = 0;
     // step metadata
     void* meta = nullptr;
@@ -452,10 +458,10 @@ int ensure_workspace(pgmi_ctx* x, int rows, size_t carries) {
     const size_t ent = (size_t)rows * top;
     d.ldh = r8(D);
     d.ld0 = l0; d.ld1 = l1; d.ld2 = l2; d.ldd = ldd;
-    d.slab_bytes = std::max<size_t>((size_t)rows * slab_n * 4, (size_t)32 << 20);
+    d.slab_n = slab_n;
     const size_t sizes[] = {(size_t)rows * d.c.streams * D * 4, (size_t)rows * d.ldh * d.es, (size_t)rows * l0 * d.es,
                             (size_t)rows * l1 * d.es,           (size_t)rows * l2 * d.es,    (size_t)rows * ldd * d.es,
-                            d.slab_bytes,                       (size_t)rows * inner * 4,    (size_t)rows * bcn * 4,
+                            d.slab_bytes(rows),                 (size_t)rows * inner * 4,    (size_t)rows * bcn * 4,
                             ent * lea * d.es, ent * d.ldh * d.es, ent * 4, ent * 4, (size_t)rows * 4, (size_t)rows * 4,
                             (size_t)rows * ne * 4, (size_t)(2 * ne + 2) * 4, here * 4};
     constexpr int NB = sizeof(sizes) / sizeof(sizes[0]);
@@ -619,7 +625,7 @@ int forward_body(pgmi_ctx* x, hipStream_t s, const int64_t* ids, int rows, const
         first = false;
     };
     auto out_proj = [&](const Lin& o, const void* in, int ldin, const Sub& sub) {
-        pend.split = matmul_rt(s, d.act, in, ldin, o.w, o.ldw, rows, D, o.k, RT_SLABS, nullptr, d.slabs, D, d.slab_bytes);
+        pend.split = matmul_rt(s, d.act, in, ldin, o.w, o.ldw, rows, D, o.k, RT_SLABS, nullptr, d.slabs, D, d.slab_bytes(rows));
         pend.y = d.slabs;
         pend.sub = &sub;
     };
@@ -633,7 +639,7 @@ int forward_body(pgmi_ctx* x, hipStream_t s, const int64_t* ids, int rows, const
             conv_silu(s, d.act, d.p0, ldxz, C, l.conv, w.conv, w.conv_b, m.seqs, m.nseq, m.conv.p, m.conv.n,
                       at<float>(state, st[i].a), d.p1, ldc);
             const int sp = matmul_rt(s, d.act, d.p1, ldc, w.x.w, w.x.ldw, rows, R + 2 * N, w.x.k, RT_SLABS, nullptr, d.slabs,
-                                     0, d.slab_bytes);
+                                     0, d.slab_bytes(rows));
             scan_inputs(s, d.act, d.slabs, sp, rows, R, N, d.dtl, ldd, d.bc);
             matmul_rt(s, d.act, d.dtl, ldd, w.dt.w, w.dt.ldw, rows, C, w.dt.k, RT_F32, nullptr, d.dt, C, 0);
             ScanArgs a{};
@@ -667,7 +673,7 @@ int forward_body(pgmi_ctx* x, hipStream_t s, const int64_t* ids, int rows, const
         if (has_ff(l)) read(i, 1, nullptr);
         if (l.experts) {
             const int sp = matmul_rt(s, d.act, d.h, d.ldh, w.router.w, w.router.ldw, rows, w.router.n, w.router.k, RT_SLABS,
-                                     nullptr, d.slabs, 0, d.slab_bytes);
+                                     nullptr, d.slabs, 0, d.slab_bytes(rows));
             route(s, route_args(d, l, w, rows, sp));
             experts_rt(s, d.act, EX_SWIGLU, expert_args(d, l, w, rows, EX_SWIGLU));
             experts_rt(s, d.act, EX_STORE, expert_args(d, l, w, rows, EX_STORE));
@@ -788,7 +794,7 @@ int decode_body_rt(pgmi_ctx* x, hipStream_t s, const int64_t* ids, int B, void* 
             g.X = d.X; g.S = d.c.streams; g.D = D; g.mix = sub.mix; g.wout = sub.out; g.mult = d.c.residual_mult;
             gemv_rt(s, d.act, GR_STREAMS, g);
         } else {
-            pend.split = matmul_rt(s, d.act, in, ldin, o.w, o.ldw, B, D, o.k, RT_SLABS, nullptr, d.slabs, D, d.slab_bytes);
+            pend.split = matmul_rt(s, d.act, in, ldin, o.w, o.ldw, B, D, o.k, RT_SLABS, nullptr, d.slabs, D, d.slab_bytes(B));
             pend.y = d.slabs;
             pend.sub = &sub;
         }
@@ -822,7 +828,7 @@ int decode_body_rt(pgmi_ctx* x, hipStream_t s, const int64_t* ids, int B, void* 
                 a.split = g.split;
             } else {
                 a.split = matmul_rt(s, d.act, d.p1, ldc, w.x.w, w.x.ldw, B, w.x.n, w.x.k, RT_SLABS, nullptr, d.slabs, 0,
-                                    d.slab_bytes);
+                                    d.slab_bytes(B));
             }
             a.slabs = d.slabs; a.Wdt = w.dt.w; a.ldwdt = w.dt.ldw; a.dtb = w.dt_b; a.x = d.p1; a.ldx = ldc; a.A_log = w.A_log;
             a.Dw = w.D; a.state = at<float>(state, st[i].b); a.slot = d.slot; a.pos = d.pos; a.y = d.p2; a.ldy = ldc;
@@ -884,7 +890,7 @@ int decode_body_rt(pgmi_ctx* x, hipStream_t s, const int64_t* ids, int B, void* 
                 gemv_rt(s, d.act, GR_F32, g);
             } else {
                 sp = matmul_rt(s, d.act, d.h, d.ldh, w.router.w, w.router.ldw, B, w.router.n, w.router.k, RT_SLABS, nullptr,
-                               d.slabs, 0, d.slab_bytes);
+                               d.slabs, 0, d.slab_bytes(B));
             }
             route(s, route_args(d, l, w, B, sp));
             experts_rt(s, d.act, EX_SWIGLU, expert_args(d, l, w, B, EX_SWIGLU));
@@ -902,7 +908,7 @@ int decode_body_rt(pgmi_ctx* x, hipStream_t s, const int64_t* ids, int B, void* 
             }
             if (l.experts) {  // the next residual pass scales it by its gate
                 pend.split = matmul_rt(s, d.act, d.p2, r8(ff), w.down.w, w.down.ldw, B, D, w.down.k, RT_SLABS, nullptr, d.slabs, D,
-                                       d.slab_bytes);
+                                       d.slab_bytes(B));
                 pend.y = d.slabs;
             } else {
                 out_proj(w.down, d.p2, r8(ff), w.sub[1]);

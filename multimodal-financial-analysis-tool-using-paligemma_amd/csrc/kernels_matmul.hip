@@ -10,6 +10,7 @@
 
 #include "act.h"
 #include "decoder.h"
+#include "plan.h"
 #include "tile_f32.h"
 
 namespace pgmi {
@@ -92,15 +93,15 @@ struct Job {
     }
 };
 
-// 64 x 64 tiles (dual: 64 x 32 + 32)
-template <int EPI, bool SPLIT>
-void run_p64(const Job& j) {
+// 32 TM x 64 tiles (dual: 32 + 32 columns)
+template <int TM, int EPI, bool SPLIT>
+void run_p(const Job& j) {
     constexpr int NB = epi_dual(EPI) ? 2 : 1, TN = NB == 2 ? 1 : 2, ST = 4;
-    constexpr int BM = 64, BN = 2 * TN * 16;
+    constexpr int BM = 32 * TM, BN = 2 * TN * 16;
     constexpr size_t lds = (size_t)ST * (BM + NB * BN) * 128;
     const int n_mt = (j.M + BM - 1) / BM, n_nt = (j.N + BN - 1) / BN;
-    lds_attr<&k_gemm_p<4, 2, 2, TN, NB, ST, EPI, SPLIT>>(lds);
-    hipLaunchKernelGGL((k_gemm_p<4, 2, 2, TN, NB, ST, EPI, SPLIT>), dim3(n_mt * n_nt, j.split), dim3(256), lds, j.s, j.A,
+    lds_attr<&k_gemm_p<4, 2, TM, TN, NB, ST, EPI, SPLIT>>(lds);
+    hipLaunchKernelGGL((k_gemm_p<4, 2, TM, TN, NB, ST, EPI, SPLIT>), dim3(n_mt * n_nt, j.split), dim3(256), lds, j.s, j.A,
                        j.lda, j.W, j.ldw, j.M, j.N, j.K, j.per(), j.ea, j.ws, j.up, n_mt, 0);
 }
 
@@ -116,28 +117,44 @@ void run_w128(const Job& j) {
                        j.A, j.lda, j.W, j.ldw, j.M, j.N, j.K, j.per(), j.ea, j.ws, j.up, n_mt, n_mt == 1 ? 1 << 30 : 0);
 }
 
-// 256 x 256 tiles, 8 phases (dual: 256 x 128 + 128); K % 64 == 0
-template <int EPI, bool SPLIT>
-void run_e256(const Job& j) {
-    constexpr int BM = 256, BN = epi_dual(EPI) ? 128 : 256;
-    constexpr size_t lds = (size_t)2 * (2 * 16 * 8 * 128 + 2 * 128 * 128);
+// 32 TM x 256 tiles, 8 phases (dual: 128 + 128 columns); K % 64 == 0
+template <int TM, int EPI, bool SPLIT>
+void run_8p(const Job& j) {
+    constexpr int BM = 32 * TM, BN = epi_dual(EPI) ? 128 : 256;
+    constexpr size_t lds = (size_t)2 * (BM * 128 + 2 * 128 * 128);
     const int n_mt = (j.M + BM - 1) / BM, n_nt = (j.N + BN - 1) / BN;
-    lds_attr<&k_gemm_8p<8, EPI, SPLIT>>(lds);
-    hipLaunchKernelGGL((k_gemm_8p<8, EPI, SPLIT>), dim3(n_mt * n_nt, j.split), dim3(512), lds, j.s, j.A, j.lda, j.W, j.ldw,
+    lds_attr<&k_gemm_8p<TM, EPI, SPLIT>>(lds);
+    hipLaunchKernelGGL((k_gemm_8p<TM, EPI, SPLIT>), dim3(n_mt * n_nt, j.split), dim3(512), lds, j.s, j.A, j.lda, j.W, j.ldw,
                        j.M, j.N, j.K, j.per(), j.ea, j.ws, j.up, n_mt, 0);
 }
 
 long tiles(int M, int N, int bm, int bn) { return (long)((M + bm - 1) / bm) * ((N + bn - 1) / bn); }
 
+// The form with the least predicted time (plan.h, whose forms are the same kernels but for the height of their ring).
+// slab_bytes > 0: into slabs, K cut as the form gains from it; the residual's pass then reads every slab, 0.25 us per MB
+// past the first one's.  Before, K slices were counted in 64 x 64 tiles and three tile shapes had fixed borders.  1,540 rows,
+// us before / now: 2048 columns of K = 16384 123 / 97 (three slices), 6144 of 2048 48.3 / 41.0, 2560 of 2048 39.4 / 30.6,
+// 4096 of 128 12.2 / 10.5.
 template <int EPI, bool SPLIT>
-void run_plan(const Job& j) {
-    const int bn2 = epi_dual(EPI) ? 2 : 1;
-    if (j.K % 64 == 0 && j.K >= 1024 && j.M >= 1024 && tiles(j.M, j.N, 256, 256 / bn2) * j.split >= 160)
-        run_e256<EPI, SPLIT>(j);
-    else if (j.N > 192 && tiles(j.M, j.N, 128, 128 / bn2) * j.split >= 128)
-        run_w128<EPI, SPLIT>(j);
-    else
-        run_p64<EPI, SPLIT>(j);
+void run_plan(Job& j, size_t slab_bytes) {
+    const float mb = 4e-6f * (float)j.M * (float)j.N;
+    const TileChoice t = choose_form(j.M, j.N, j.K, epi_dual(EPI), slab_bytes ? 8 : 1, [&](const TileForm& f, int split) {
+        if (f.cfg == R288w || f.cfg == W288n || f.cfg == W64x64 || f.cfg == W128x64) return -1.0f;  // not instantiated here
+        if (split > 1 && (size_t)split * j.M * j.N * sizeof(float) > slab_bytes) return -1.0f;
+        return 0.25f * mb * (float)(split - 1);
+    });
+    j.split = t.split;
+    switch (t.form->cfg) {
+        case P32x64s4: run_p<1, EPI, SPLIT>(j); break;
+        case P96x64s4: run_p<3, EPI, SPLIT>(j); break;
+        case W128x128: run_w128<EPI, SPLIT>(j); break;
+        case E128: run_8p<4, EPI, SPLIT>(j); break;
+        case E160: run_8p<5, EPI, SPLIT>(j); break;
+        case E192: run_8p<6, EPI, SPLIT>(j); break;
+        case E224: run_8p<7, EPI, SPLIT>(j); break;
+        case E256: run_8p<8, EPI, SPLIT>(j); break;
+        default: run_p<2, EPI, SPLIT>(j); break;
+    }
 }
 
 // K slices for a product whose t tiles alone leave CUs idle
@@ -185,8 +202,7 @@ int matmul_rt(hipStream_t s, Act act, const void* A, int lda, const uint16_t* W,
     Job j{s, reinterpret_cast<const uint16_t*>(A), lda, W, ldw, M, N, K, {}, nullptr, 1, 0};
     if (mode == RT_F32 || mode == RT_SLABS) {
         j.ws = reinterpret_cast<float*>(out);
-        if (mode == RT_SLABS) j.split = pick_split(tiles(M, N, 64, 64), 256, M, N, K, out_bytes);
-        run_plan<EPI_STORE, true>(j);
+        run_plan<EPI_STORE, true>(j, mode == RT_SLABS ? out_bytes : 0);
         return j.split;
     }
     j.ea.out = reinterpret_cast<uint16_t*>(out);
@@ -194,11 +210,11 @@ int matmul_rt(hipStream_t s, Act act, const void* A, int lda, const uint16_t* W,
     j.ea.bias = bias;
     if (mode == RT_SWIGLU) {
         j.up = (long)N * ldw;
-        run_plan<EPI_SWIGLU, false>(j);
+        run_plan<EPI_SWIGLU, false>(j, 0);
     } else if (bias) {
-        run_plan<EPI_BIAS, false>(j);
+        run_plan<EPI_BIAS, false>(j, 0);
     } else {
-        run_plan<EPI_STORE, false>(j);
+        run_plan<EPI_STORE, false>(j, 0);
     }
     if (ldo > N && ldo - N < 8)
         hipLaunchKernelGGL(k_zero_cols, dim3(256), dim3(256), 0, s, reinterpret_cast<uint16_t*>(out), M, N, ldo);

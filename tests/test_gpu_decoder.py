@@ -66,6 +66,16 @@ def test_matmul_any_shape(M, N, K, act):
     assert (out[:, N:] == 0).all()
 
 
+@pytest.mark.parametrize("M,N,K", [(40, 2048, 4096), (500, 2561, 2048), (1000, 8190, 1088), (1540, 4096, 128), (1540, 6146, 2048),
+                                   (1537, 8192, 2048), (3000, 4095, 1024), (3000, 2048, 4096), (257, 8192, 2056)])
+def test_matmul_forms(M, N, K):
+    """Sizes at which the least predicted time is each form's in turn (32 and 96 x 64, 128 x 128, 128 to 256 x 256), whole or in
+    K slices, with rows, columns and k past the last tile.  (K <= 4096: K / 32 roundings of a sum of size sqrt(K) add up to
+    about 2^-24 K / sqrt(32), 5 sigma of it over the outputs 2e-7 K on either side; 2e-5 sqrt(K) covers both up to K = 2500
+    and, as partial sums are smaller than the last, 4096.  At 16384, 3.5e-3 stood against 2.6e-3.)"""
+    test_matmul_any_shape(M, N, K, 0)
+
+
 # ---------------------------------------------------------------- mechanisms and whole models
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("name", list(ALL))
