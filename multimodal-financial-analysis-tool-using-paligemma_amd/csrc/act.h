@@ -43,7 +43,7 @@ __device__ __forceinline__ float softplusf_(float x) { return fmaxf(x, 0.0f) + l
 // the same from the hardware exponential and logarithm: a short series where 1 + e would round e away
 __device__ __forceinline__ float softplus_fast(float x) {
     const float e = __expf(-fabsf(x));
-    const float series = e * (1.0f - e * (0.5f - e * (0.33333333f - e * (0.25f - e * 0.2f))));
+    const float series = e * fmaf(e, fmaf(e, fmaf(e, fmaf(e, 0.2f, -0.25f), 0.33333333f), -0.5f), 1.0f);
     return fmaxf(x, 0.0f) + (e < 0.0625f ? series : __logf(1.0f + e));
 }
 template <typename T>

@@ -7,6 +7,7 @@
 // (C) every chunk again from its entry state, writing the outputs; the last chunk leaves the sequence's state.
 // The decay of a chunk is exp(A sum(dt)), so (A) keeps sums of steps and no products.
 #include <algorithm>
+#include <type_traits>
 
 #include "act.h"
 #include "decoder.h"
@@ -134,9 +135,10 @@ constexpr int kPre = 8;   // rows whose step, input and gate are in flight ahead
 // LPC lanes per channel, NPL states per lane (N <= LPC * NPL; states past N are inert: B = C = 0).
 // PHASE 0: (A) zero entry state, no output; 1: (C) / single-chunk walk.
 template <typename T, int NPL, int LPC, int PHASE>
-__global__ void __launch_bounds__(256) k_scan(ScanArgs a) {
+__global__ void __launch_bounds__(256, LPC == 1 ? 2 : LPC == 2 ? 1 : 3) k_scan(ScanArgs a) {
     constexpr int CPB = 256 / LPC;  // channels per workgroup
     constexpr int NP = NPL * LPC;
+    constexpr bool AHEAD = LPC == 1;  // the next row's B | C read under this one's sums (they cost lanes that share a channel a wave)
     __shared__ __attribute__((aligned(16))) float sB[kSub][NP], sC[PHASE ? kSub : 1][PHASE ? NP : 4];
     const ChunkInfo ck = a.chunks[blockIdx.y];
     const bool last = ck.idx + 1 == ck.nch;
@@ -245,7 +247,12 @@ __global__ void __launch_bounds__(256) k_scan(ScanArgs a) {
         }
         __syncthreads();
         if (t0 + kSub < ck.len) hold(t0 + kSub);
-        for (int tb = 0; tb < nt; tb += kPre) {
+        // kPre rows; all of them there: no branch between them, so that the next row's B | C are read under this one's sums.
+        // (A) / (C), us, a branch and reads of its own before each row -> now: 1,540 rows of 4,096 channels of 16 states
+        // 31.0 / 39.4 -> 28.6 / 35.9, 500 rows 15.3 / 19.6 -> 13.2 / 16.2, 2,048 channels of 64 states 54.5 / 76.5 -> 50.7 /
+        // 68.4, of 256 203 / 439 -> 187 / 395.  The step's softplus in its product's epilogue instead: (A) 24, the product
+        // 10.4 -> 18.3, which nothing there covers.
+        auto walk = [&](auto full, int tb) {
             float dt[kPre], x[kPre], g[kPre];
 #pragma unroll
             for (int t = 0; t < kPre; ++t) {
@@ -255,36 +262,58 @@ __global__ void __launch_bounds__(256) k_scan(ScanArgs a) {
                 if constexpr (PHASE == 1) g[t] = siluf_(ldf(&pz[t]));
             }
             if (t0 + tb + kPre < ck.len) fetch(t0 + tb + kPre);
+            f32x4 B[1 + AHEAD][NPL / 4], Cv[1 + AHEAD][PHASE ? NPL / 4 : 1];
+            auto read = [&](int t, int to) {
+#pragma unroll
+                for (int i = 0; i < NPL / 4; ++i) {
+                    B[to][i] = lB[(tb + t) * (NP / 4) + i];
+                    if constexpr (PHASE == 1) Cv[to][i] = lC[(tb + t) * (NP / 4) + i];
+                }
+            };
+            if constexpr (AHEAD) read(0, 0);
 #pragma unroll
             for (int t = 0; t < kPre; ++t) {
-                if (tb + t < nt) {
-                    const float dx = dt[t] * x[t];
-                    dsum += dt[t];
-                    float y = 0.0f;
+                if (!full && tb + t >= nt) break;
+                const int at = AHEAD ? t & 1 : 0;
+                if constexpr (AHEAD) {
+                    if (t + 1 < kPre) read(t + 1, (t + 1) & 1);  // (of a broken block, rows of LDS that are not used)
+                    __builtin_amdgcn_sched_barrier(0);
+                } else {
+                    read(t, 0);
+                }
+                const float dx = dt[t] * x[t];
+                dsum += dt[t];
+                float y0 = 0.0f, y1 = 0.0f;
 #pragma unroll
-                    for (int i = 0; i < NPL; i += 4) {
-                        const f32x4 B = lB[(tb + t) * (NP / 4) + i / 4];
-                        S[i] = fmaf(__builtin_amdgcn_exp2f(dt[t] * A[i]), S[i], dx * B[0]);
-                        S[i + 1] = fmaf(__builtin_amdgcn_exp2f(dt[t] * A[i + 1]), S[i + 1], dx * B[1]);
-                        S[i + 2] = fmaf(__builtin_amdgcn_exp2f(dt[t] * A[i + 2]), S[i + 2], dx * B[2]);
-                        S[i + 3] = fmaf(__builtin_amdgcn_exp2f(dt[t] * A[i + 3]), S[i + 3], dx * B[3]);
-                        if constexpr (PHASE == 1) {
-                            const f32x4 Cv = lC[(tb + t) * (NP / 4) + i / 4];
-                            y = fmaf(S[i], Cv[0], y);
-                            y = fmaf(S[i + 1], Cv[1], y);
-                            y = fmaf(S[i + 2], Cv[2], y);
-                            y = fmaf(S[i + 3], Cv[3], y);
-                        }
+                for (int i = 0; i < NPL; ++i)
+                    S[i] = fmaf(__builtin_amdgcn_exp2f(dt[t] * A[i]), S[i], dx * B[at][i / 4][i % 4]);
+                if constexpr (PHASE == 1) {
+#pragma unroll
+                    for (int i = 0; i < NPL; i += 2) {
+                        y0 = fmaf(S[i], Cv[at][i / 4][i % 4], y0);
+                        y1 = fmaf(S[i + 1], Cv[at][i / 4][i % 4 + 1], y1);
                     }
-                    if constexpr (PHASE == 1) {
+                    float y = y0 + y1;
 #pragma unroll
-                        for (int o = 1; o < LPC; o <<= 1) y += __shfl_xor(y, o, 64);
-                        if (sub == 0 && c < a.ldy)  // columns C .. ldy - 1 are zero
-                            stf(yp + (long)(t0 + tb + t) * a.ldy, ok ? fmaf(Dc, x[t], y) * g[t] : 0.0f);
+                    for (int o = 1; o < LPC; o <<= 1) y += __shfl_xor(y, o, 64);
+                    g[t] *= fmaf(Dc, x[t], y);
+                    asm volatile("" : "+v"(g[t]));  // (else the sum moves into the stores' branch, with every row's states)
+                }
+                if constexpr (AHEAD) __builtin_amdgcn_sched_barrier(0);
+            }
+            if constexpr (PHASE == 1) {
+                if (sub == 0 && c < a.ldy) {  // columns C .. ldy - 1 are zero
+#pragma unroll
+                    for (int t = 0; t < kPre; ++t) {
+                        if (!full && tb + t >= nt) break;
+                        stf(yp + (long)(t0 + tb + t) * a.ldy, ok ? g[t] : 0.0f);
                     }
                 }
             }
-        }
+        };
+        int tb = 0;
+        for (; tb + kPre <= nt; tb += kPre) walk(std::true_type{}, tb);
+        if (tb < nt) walk(std::false_type{}, tb);
     }
     if (!ok) return;
     if (PHASE == 0 && sub == 0) a.csum[(long)blockIdx.y * a.C + c] = dsum;

@@ -94,6 +94,18 @@ def test_layers_and_logits_of_a_prompt(name, dtype):
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("inner,dt_rank,rows", [(1032, 24, 600), (2048, 64, 1301)])
+def test_steps_and_scan_of_many_rows(inner, dt_rank, rows, dtype):
+    """The step sizes' product on the tiles that many rows take (one with columns past the last tile), runs of whole and broken
+    blocks of rows."""
+    cfg = C.model([C.mamba(inner, 16, dt_rank, 4)], width=64, streams=1, groups=1)
+    eng, W = build(cfg, dtype)
+    toks = tokens(cfg, rows, 5)
+    cache = eng.new_cache(1, rows)
+    close(eng.step(cache, [cache.alloc()], [toks], want=range(rows)), O.run(cfg, W, toks), dtype)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("name", list(ALL))
 def test_token_by_token(name, dtype):
     cfg = ALL[name]
