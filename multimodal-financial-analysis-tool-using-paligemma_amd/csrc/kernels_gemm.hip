@@ -1095,10 +1095,12 @@ __global__ void __launch_bounds__(64 * (NW + LW), 1) k_gemm_w(const uint16_t* __
 // G: which rows a tile is made of.  AllRows: consecutive rows of A, the XCD-aware tile order.  A grouped form
 // (G::kGrouped, no split) cuts the tiles out of row lists: tile(BM, BN) finds the workgroup's (false: none left) and
 // sets rows (of its list), m0, nt; weights() its matrix; source(m) the row of A behind list place m, target(m) the row
-// of the output.
+// of the output; first_ktile() the K-tile (modulo their number) that the tile starts with.
 struct AllRows {
     static constexpr bool kGrouped = false;
 };
+
+constexpr size_t lds_8p(int TM) { return (size_t)2 * (32 * TM * 128 + 2 * 128 * 128); }  // two K-tile buffers
 
 template <int TM, int EPI, bool SPLIT, class G>
 __device__ __forceinline__ void gemm_8p(const uint16_t* __restrict__ A, int lda, const uint16_t* __restrict__ W, int ldw, int M,
@@ -1178,10 +1180,17 @@ __device__ __forceinline__ void gemm_8p(const uint16_t* __restrict__ A, int lda,
         }
     }
 #define PGMI_8P_LDS(off) ((__attribute__((address_space(3))) void*)(sm8 + (off)))
+    int skew = 0;
+    if constexpr (G::kGrouped) skew = g.first_ktile() % nkt_total;
+    auto place = [&](int kt) {  // grouped: the walk over K starts at the tile's own place
+        if constexpr (!G::kGrouped) return kt;
+        const int k = kt + skew;
+        return k < nkt_total ? k : k - nkt_total;
+    };
     auto stageA = [&](int qa, int kt, int buf) {
         if constexpr (PGMI_GEMM_DIAG & 2) return;
         kt = kt < kt1 ? kt : kt1 - 1;  // past the range: valid bytes into a buffer never read again
-        const int kel = kt * 64;
+        const int kel = place(kt) * 64;
         const int base = buf * TB + qa * AB1;
 #pragma unroll
         for (int i = 0; i < (qa ? GA1 : GA0); ++i)
@@ -1190,7 +1199,7 @@ __device__ __forceinline__ void gemm_8p(const uint16_t* __restrict__ A, int lda,
     auto stageB = [&](int qb, int kt, int buf) {
         if constexpr (PGMI_GEMM_DIAG & 2) return;
         kt = kt < kt1 ? kt : kt1 - 1;
-        const int kel = kt * 64;
+        const int kel = place(kt) * 64;
         const int base = buf * TB + BB0 + qb * HBB;
 #pragma unroll
         for (int i = 0; i < GB; ++i)
@@ -1569,7 +1578,7 @@ static void launch_8p(hipStream_t s, const uint16_t* A, int lda, const uint16_t*
                       const EpiArgs& ea, float* ws, int split, long up_off) {
     constexpr bool DUAL = epi_dual(EPI);
     constexpr int BM = 32 * TM, BNO = DUAL ? 128 : 256;
-    constexpr size_t lds = (size_t)2 * (2 * 16 * TM * 128 + 2 * 128 * 128);
+    constexpr size_t lds = lds_8p(TM);
     static_assert(lds <= 163840, "LDS exceeds 160 KiB");
     constexpr int EK = EPI < 0 ? EPI_STORE : EPI;
     const int nkt = K / 64;

@@ -273,6 +273,12 @@ struct ExpertRows {
         return e >= 0;
     }
     __device__ __forceinline__ const uint16_t* weights() const { return a.W + e * a.wstride; }
+    // Weight rows of 2,048 or 1,024 columns are 4 or 2 KiB apart, so one K-tile of all of them falls on one of an XCD's 16 cache
+    // channels: tiles in step read cold weights at 4.5 TB/s, tiles three K-tiles apart from each other at 5.9 (rows 128 bytes
+    // further apart 6.0).  Experts' weights are read by one or two row tiles and come from HBM: gate|up of 2,048 rows, top 6
+    // of 60, 152.4 -> 148.2 us, down the same (dense products, whose weights many row tiles share: no change).  A matter of expert
+    // and column tile alone, so that an output's sum does not depend on the step's other rows.
+    __device__ __forceinline__ int first_ktile() const { return 3 * (8 * e + nt); }
     __device__ __forceinline__ int source(int m) const { return list[m] / a.gather; }
     __device__ __forceinline__ int target(int m) const { return list[m]; }
 };

@@ -273,6 +273,22 @@ def test_long_expert_lists(width, mlp, dtype):
     close(feed(eng, cache, cache.alloc(), toks, [333, 40, 100]), want, dtype)
 
 
+@pytest.mark.parametrize("experts,ff,top,rows,pull", [(70, 512, 16, 700, 0.0), (9, 512, 3, 500, 40.0), (4, 640, 1, 600, 40.0),
+                                                      (5, 520, 2, 385, 0.0)])
+def test_expert_lists_of_many_lengths(experts, ff, top, rows, pull):
+    """Mean lists of 129 to 384 rows, whose tiles start K at places of their own: more than 64 experts, one list
+    of every row beside an empty one (by choice corrections that leave the other experts' order, and so its margin, alone),
+    columns past the last tile."""
+    cfg = C.model([C.layer(2, 1, 16, 24, 30, mlp=C.moe(experts, ff, top, 24))], width=512)
+    Wr = R.random_weights(cfg, 17)
+    Wr["l0.mlp.correction"][0] += pull
+    Wr["l0.mlp.correction"][1] -= pull
+    eng, W = build(cfg, "bfloat16", weights=Wr)
+    toks = tokens(cfg, rows, 64)
+    cache = eng.new_cache(1, rows)
+    close(eng.step(cache, [cache.alloc()], [toks], want=range(rows)), R.run(cfg, W, toks), "bfloat16")
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 def test_choice_scores_below_zero_and_unused_experts(dtype):
     """Corrections far below zero: the other groups' experts must not win with a zero; experts nobody chooses."""
