@@ -128,6 +128,7 @@ struct CanonArgs {
     int nseq;
     const ChunkInfo* chunks;
     int nchunk;
+    bool fresh;  // every sequence of the step from its start
 };
 void canon(hipStream_t s, Act act, const CanonArgs& a);
 
@@ -199,7 +200,7 @@ int matmul_rt(hipStream_t s, Act act, const void* A, int lda, const uint16_t* W,
 // ---------------------------------------------------------------- selective scan (Mamba)
 // xz rows [x: C | z: C] (activation type); taps state fp32 [slot][K-1][C]
 void conv_silu(hipStream_t s, Act act, const void* xz, int ldxz, int C, int K, const uint16_t* w, const uint16_t* b,
-               const SeqInfo* seqs, int nseq, const ChunkInfo* chunks, int nchunk, float* taps, void* out,
+               const SeqInfo* seqs, int nseq, const ChunkInfo* chunks, int nchunk, bool fresh, float* taps, void* out,
                int ldo);
 // slabs [split][rows][R + 2N] -> dt_low (activation type, ldd, zero-padded) and B|C fp32 [rows][2N]
 void scan_inputs(hipStream_t s, Act act, const float* slabs, int split, int rows, int R, int N, void* dtl, int ldd,

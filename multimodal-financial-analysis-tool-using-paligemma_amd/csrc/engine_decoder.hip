@@ -580,6 +580,7 @@ struct Meta {
         int n;
         bool multi;  // some sequence has more than one
     } scan, gru, conv;
+    bool fresh;  // every sequence from its start
     const int* row_seq;
     const int* want;
     std::map<int, std::pair<const ChunkInfo*, int>> tiles;  // by query heads per key/value head
@@ -609,7 +610,7 @@ int forward_body(pgmi_ctx* x, hipStream_t s, const int64_t* ids, int rows, const
                 CanonArgs c{};
                 c.X = d.X; c.inv = d.inv; c.w = sub.norm; c.w_scalar = d.c.norm_scalar; c.rows = rows; c.D = D;
                 c.taps = d.c.canon_taps; c.cw = w.canon; c.ring = at<float>(state, st[i].ring); c.h = d.h; c.ldh = d.ldh;
-                c.seqs = m.seqs; c.nseq = m.nseq; c.chunks = m.conv.p; c.nchunk = m.conv.n;
+                c.seqs = m.seqs; c.nseq = m.nseq; c.chunks = m.conv.p; c.nchunk = m.conv.n; c.fresh = m.fresh;
                 canon(s, d.act, c);
             }
             pend = {};
@@ -636,7 +637,7 @@ int forward_body(pgmi_ctx* x, hipStream_t s, const int64_t* ids, int rows, const
         if (l.mixer == PGMI_MIXER_MAMBA1) {
             const int C = l.inner, N = l.state, R = l.dt_rank, ldc = r8(C), ldxz = r8(2 * C), ldd = r8(R);
             matmul_rt(s, d.act, d.h, d.ldh, w.in.w, w.in.ldw, rows, 2 * C, w.in.k, RT_ACT, nullptr, d.p0, ldxz, 0);
-            conv_silu(s, d.act, d.p0, ldxz, C, l.conv, w.conv, w.conv_b, m.seqs, m.nseq, m.conv.p, m.conv.n,
+            conv_silu(s, d.act, d.p0, ldxz, C, l.conv, w.conv, w.conv_b, m.seqs, m.nseq, m.conv.p, m.conv.n, m.fresh,
                       at<float>(state, st[i].a), d.p1, ldc);
             const int sp = matmul_rt(s, d.act, d.p1, ldc, w.x.w, w.x.ldw, rows, R + 2 * N, w.x.k, RT_SLABS, nullptr, d.slabs,
                                      0, d.slab_bytes(rows));
@@ -1121,6 +1122,7 @@ int pgmi_decoder_forward(pgmi_ctx* x, const int64_t* ids, int n_seq, const int32
     Meta meta{};
     meta.seqs = reinterpret_cast<const SeqInfo*>(dm);
     meta.nseq = n_seq;
+    meta.fresh = std::all_of(starts, starts + n_seq, [](int32_t p) { return p == 0; });
     meta.scan = {reinterpret_cast<const ChunkInfo*>(dm + scan.o), scan.n, scan.multi};
     meta.gru = {reinterpret_cast<const ChunkInfo*>(dm + gru.o), gru.n, gru.multi};
     meta.conv = {reinterpret_cast<const ChunkInfo*>(dm + conv.o), conv.n, conv.multi};

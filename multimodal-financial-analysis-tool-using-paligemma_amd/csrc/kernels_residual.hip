@@ -343,7 +343,8 @@ __device__ __forceinline__ float canon_at(const CanonArgs& a, const SeqInfo& q, 
     return p >= 0 ? a.ring[((long)q.slot * a.taps + p % a.taps) * a.D + c] : 0.0f;
 }
 
-// four channels per lane, KT taps in registers, each wave a run of consecutive rows
+// four channels per lane, KT taps in registers, each wave a run of consecutive rows.  a.fresh (every sequence from its start:
+// no wave reads the ring): the wave that ends a sequence leaves its window in the ring, k_canon_keep's launch (4.8 us) goes
 template <typename T, int KT>
 __global__ void __launch_bounds__(256) k_canon(CanonArgs a) {
     const ChunkInfo ck = a.chunks[blockIdx.y];
@@ -392,6 +393,15 @@ __global__ void __launch_bounds__(256) k_canon(CanonArgs a) {
         if (c + 4 == a.D)
             for (int d = a.D; d < a.ldh; ++d) stf(h + (long)(ck.row + r) * a.ldh + d, 0.0f);
     }
+    if (a.fresh && ck.rel + r1 == q.len) {
+#pragma unroll
+        for (int t = 0; t < KT - 1; ++t) {
+            const int p = q.len - (KT - 1) + t;
+            if (p < 0) continue;
+#pragma unroll
+            for (int v = 0; v < 4; ++v) a.ring[((long)q.slot * KT + p % KT) * a.D + c + v] = win[t][v];
+        }
+    }
 }
 
 // any number of taps and channels
@@ -429,7 +439,8 @@ void canon_t(hipStream_t s, const CanonArgs& a) {
     else if (a.D % 4 == 0 && a.taps == 3) hipLaunchKernelGGL((k_canon<T, 3>), grid, dim3(256), 0, s, a);
     else if (a.D % 4 == 0 && a.taps == 2) hipLaunchKernelGGL((k_canon<T, 2>), grid, dim3(256), 0, s, a);
     else hipLaunchKernelGGL((k_canon_any<T>), dim3((a.ldh + 63) / 64, a.nchunk), dim3(256), 0, s, a);
-    if (a.taps > 1)
+    const bool kept = a.fresh && a.D % 4 == 0 && a.taps >= 2 && a.taps <= 4;
+    if (a.taps > 1 && !kept)
         hipLaunchKernelGGL(k_canon_keep, dim3((a.D + 255) / 256, a.nseq * (a.taps - 1)), dim3(256), 0, s, a);
 }
 
