@@ -308,6 +308,7 @@ struct WAttnDecodeArgs {
     const int* pos;
     float* part;
     int nsplit;
+    bool parts_only;  // the splits' partials are left to their reader
 };
 int wattn_decode_splits(int B, int G, const WAttnScore& sc, int max_tokens);
 size_t wattn_decode_floats(int B, int H, int ep, int nsplit);
@@ -360,10 +361,15 @@ struct GemvRtArgs {
     const uint16_t* wout;
     float mult;
     int split;  // GR_F32
+    // GR_STREAMS: x is still an attention's partials (as wattn_decode leaves them: per head `nsplit` of `prs` floats, the last two
+    // maximum and sum, heads of `pe` values); x itself is not read
+    const float* part;
+    int nsplit, prs, pe;
     // GR_LOGITS
     float* pmax;
     int* pidx;
 };
+bool gemv_rt_merges(const GemvRtArgs& a);  // GR_STREAMS takes these partials
 int gemv_rt_max_batch();
 int gemv_rt_parts();  // words of pmax / pidx
 GemvRtForm gemv_rt_form(int B, Act act, int streams, int width);

@@ -783,7 +783,14 @@ int decode_body_rt(pgmi_ctx* x, hipStream_t s, const int64_t* ids, int B, void* 
         g.form = form; g.act = d.act; g.B = B; g.N = w.n; g.K = w.k; g.W = w.w; g.ldw = w.ldw; g.x = in; g.ldx = ldin; g.slot = d.slot; g.pos = d.pos;
         return g;
     };
-    auto out_proj = [&](const Lin& o, const void* in, int ldin, const Sub& sub) {
+    // parts: the input is still the partials of an attention
+    auto out_args = [&](const Lin& o, const void* in, int ldin, const Sub& sub, const WAttnDecodeArgs* parts) {
+        GemvRtArgs g = row_in(o, in, ldin);
+        g.X = d.X; g.S = d.c.streams; g.D = D; g.mix = sub.mix; g.wout = sub.out; g.mult = d.c.residual_mult;
+        if (parts) { g.part = parts->part; g.nsplit = parts->nsplit; g.prs = parts->hd.ep + 2; g.pe = parts->hd.e; }
+        return g;
+    };
+    auto out_proj = [&](const Lin& o, const void* in, int ldin, const Sub& sub, const WAttnDecodeArgs* parts = nullptr) {
         const bool fits = gemv_rt_fits(form, o.k, d.act);
         if (fits && form != GF_STREAM) {  // the next streams pass sums the slabs
             GemvRtArgs g = row_in(o, in, ldin);
@@ -791,9 +798,7 @@ int decode_body_rt(pgmi_ctx* x, hipStream_t s, const int64_t* ids, int B, void* 
             gemv_rt(s, d.act, GR_F32, g);
             pend = {d.slabs, g.split, &sub, {}};
         } else if (fits) {
-            GemvRtArgs g = row_in(o, in, ldin);
-            g.X = d.X; g.S = d.c.streams; g.D = D; g.mix = sub.mix; g.wout = sub.out; g.mult = d.c.residual_mult;
-            gemv_rt(s, d.act, GR_STREAMS, g);
+            gemv_rt(s, d.act, GR_STREAMS, out_args(o, in, ldin, sub, parts));
         } else {
             pend.split = matmul_rt(s, d.act, in, ldin, o.w, o.ldw, B, D, o.k, RT_SLABS, nullptr, d.slabs, D, d.slab_bytes(B));
             pend.y = d.slabs;
@@ -850,8 +855,10 @@ int decode_body_rt(pgmi_ctx* x, hipStream_t s, const int64_t* ids, int B, void* 
             a.qkv = d.p0; a.kc = at<void>(state, st[i].a); a.vc = at<void>(state, st[i].b); a.max_tokens = max_tokens;
             a.o = d.p2; a.B = B; a.slot = d.slot; a.pos = d.pos; a.part = d.part;
             a.nsplit = wattn_decode_splits(B, l.kv_heads, a.sc, max_tokens);
+            a.parts_only = form == GF_STREAM && B == 1 && a.hd.dp <= 256 && a.hd.ep <= 256 && w.o.k == l.heads * l.vdim &&
+                           gemv_rt_fits(form, w.o.k, d.act) && gemv_rt_merges(out_args(w.o, d.p2, a.ldo, w.sub[0], &a));
             wattn_decode(s, d.act, a);
-            out_proj(w.o, d.p2, a.ldo, w.sub[0]);
+            out_proj(w.o, d.p2, a.ldo, w.sub[0], a.parts_only ? &a : nullptr);
         } else {
             const int C = l.width, ldc = r8(C);
             GemvRtArgs g = base(w.sub[0], w.in, fin);

@@ -417,7 +417,9 @@ __device__ __forceinline__ void one_store(const GemvRtArgs& a, int n, float v, f
 constexpr int one_rows(int mode) { return mode == GR_LOGITS ? 4 : unit_rows(mode); }
 constexpr int one_outs(int mode) { return mode == GR_LOGITS ? 4 : unit_outs(mode); }
 
-// CH: K / 512.  NS: 0: x is a row of activations; else up to NS streams, read and normed here.
+// CH: K / 512.  NS: 0: x is a row of activations; NS > 0: up to NS streams, read and normed here; NS < 0: up to -NS partials of
+// every head of an attention, merged here as k_wattn_dc does (a launch of 5.1 us;
+// here 1,024 values of 8 partials take 1.1: 3.3 -> 4.4 us)
 template <int MODE, int CH, int NS>
 __global__ void __launch_bounds__(256) k_gemv_one(GemvRtArgs a) {
     constexpr int RW = one_rows(MODE), UO = one_outs(MODE);
@@ -425,13 +427,24 @@ __global__ void __launch_bounds__(256) k_gemv_one(GemvRtArgs a) {
     const int nunit = (a.N + UO - 1) / UO, ustep = gridDim.x * 4, K = a.K;
     int unit = blockIdx.x * 4 + wave;
     uint4 w[RW][CH], x[CH], nw;
-    float4 X[NS ? NS : 1][2];
+    float4 X[NS > 0 ? NS : 1][2];
+    constexpr int MS = NS < 0 ? -NS : 1;
+    float2 pv[MS][4], ml[MS];
     // the streams' read and norm are shared out: a wave takes one piece of 512 (of fewer pieces the last one twice)
     const int piece = min(wave, CH - 1), px = piece * 512 + lane * 8;
     static_assert(CH <= 4, "a piece per wave");
     if constexpr (NS == 0) {
 #pragma unroll
         for (int c = 0; c < CH; ++c) x[c] = ldg16(reinterpret_cast<const uint16_t*>(a.x) + c * 512 + lane * 8);
+    } else if constexpr (NS < 0) {
+        const float* p = a.part + (long)(px / a.pe) * a.nsplit * a.prs;
+#pragma unroll
+        for (int s = 0; s < MS; ++s) {
+            const float* q = p + (long)min(s, a.nsplit - 1) * a.prs;
+            ml[s] = *reinterpret_cast<const float2*>(q + a.prs - 2);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) pv[s][i] = *reinterpret_cast<const float2*>(q + px % a.pe + 2 * i);
+        }
     } else {
 #pragma unroll
         for (int s = 0; s < NS; ++s) {
@@ -455,6 +468,32 @@ __global__ void __launch_bounds__(256) k_gemv_one(GemvRtArgs a) {
     constexpr bool ST = MODE == GR_CONV || MODE == GR_GRU;
     const int slot = ST ? a.slot[0] : 0;
     const bool first = ST && a.pos[0] == 0;
+    if constexpr (NS < 0) {
+        __shared__ __attribute__((aligned(16))) uint16_t xs[CH * 512];
+        float m = -1e30f, L = 0.0f, t[8] = {};  // an empty split's values were never written: weight 0, not taken
+#pragma unroll
+        for (int s = 0; s < MS; ++s)
+            if (s < a.nsplit && ml[s].y > 0.0f) m = fmaxf(m, ml[s].x);
+#pragma unroll
+        for (int s = 0; s < MS; ++s) {
+            const bool is = s < a.nsplit && ml[s].y > 0.0f;
+            ml[s].x = is ? exp2f(ml[s].x - m) : 0.0f;
+            L += is ? ml[s].y * ml[s].x : 0.0f;
+        }
+#pragma unroll
+        for (int s = 0; s < MS; ++s) {
+            const float w = ml[s].x / L;
+#pragma unroll
+            for (int i = 0; i < 8; ++i) t[i] = w > 0.0f ? fmaf(i & 1 ? pv[s][i / 2].y : pv[s][i / 2].x, w, t[i]) : t[i];
+        }
+        if (wave == piece)
+            *reinterpret_cast<uint4*>(xs + px) =
+                make_uint4(f2bf(t[0]) | (uint32_t)f2bf(t[1]) << 16, f2bf(t[2]) | (uint32_t)f2bf(t[3]) << 16,
+                           f2bf(t[4]) | (uint32_t)f2bf(t[5]) << 16, f2bf(t[6]) | (uint32_t)f2bf(t[7]) << 16);
+        __syncthreads();
+#pragma unroll
+        for (int c = 0; c < CH; ++c) x[c] = *reinterpret_cast<const uint4*>(xs + c * 512 + lane * 8);
+    }
     if constexpr (NS > 0) {
         __shared__ __attribute__((aligned(16))) uint16_t xs[CH * 512];
         __shared__ float red[4];
@@ -594,6 +633,13 @@ bool gemv_one_fits(const GemvRtArgs& a, int mode) {
 
 template <int MODE, int CH>
 void run_one_ch(hipStream_t s, const GemvRtArgs& a, int blocks) {
+    if constexpr (MODE == GR_STREAMS) {
+        if (a.part) {
+            if (a.nsplit <= 8) hipLaunchKernelGGL((k_gemv_one<MODE, CH, -8>), dim3(blocks), dim3(256), 0, s, a);
+            else hipLaunchKernelGGL((k_gemv_one<MODE, CH, -16>), dim3(blocks), dim3(256), 0, s, a);
+            return;
+        }
+    }
     if (MODE == GR_STREAMS || a.x) hipLaunchKernelGGL((k_gemv_one<MODE, CH, 0>), dim3(blocks), dim3(256), 0, s, a);
     else if constexpr (MODE != GR_STREAMS) {  // (the update's input is the sublayer's, never the streams)
         if (CH > 2 || a.S <= 2) hipLaunchKernelGGL((k_gemv_one<MODE, CH, 2>), dim3(blocks), dim3(256), 0, s, a);
@@ -1038,6 +1084,11 @@ GemvRtForm gemv_rt_form(int B, Act act, int streams, int width) {
 bool gemv_rt_fits(GemvRtForm form, int K, Act act) {
     if (form == GF_STREAM) return (size_t)2 * K * (act == ACT_F32 ? 4 : 2) <= 96 * 1024;
     return form == GF_SKINNY;
+}
+
+bool gemv_rt_merges(const GemvRtArgs& a) {
+    return a.act == ACT_BF16 && a.x && gemv_one_fits(a, GR_STREAMS) && a.nsplit <= 16 && a.pe % 8 == 0 && a.K % a.pe == 0 &&
+           a.prs % 2 == 0;
 }
 
 int gemv_rt_split(GemvRtForm form, int N, int K) {

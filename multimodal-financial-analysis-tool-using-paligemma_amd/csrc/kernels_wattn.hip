@@ -1081,7 +1081,7 @@ void run_dm(hipStream_t s, const WAttnDecodeArgs& a) {
     };
     if (w.d % 8 == 0 && w.e % 8 == 0) go(std::true_type{});
     else go(std::false_type{});
-    hipLaunchKernelGGL((k_wattn_dc<uint16_t>), dim3(w.H, a.B), dim3(256), 0, s, a);
+    if (!a.parts_only) hipLaunchKernelGGL((k_wattn_dc<uint16_t>), dim3(w.H, a.B), dim3(256), 0, s, a);
 }
 template <int DQ>
 void run_dmv(hipStream_t s, const WAttnDecodeArgs& a) {

@@ -116,6 +116,19 @@ def test_token_by_token(name, dtype):
     close(got, O.run(cfg, W, toks), dtype)
 
 
+@pytest.mark.parametrize("heads,kv,dim,vdim,window", [(8, 2, 64, 64, 900), (6, 2, 40, 256, 1500), (16, 4, 32, 128, 1990),
+                                                      (128, 1, 16, 8, 300), (4, 4, 24, 128, 2500)])
+def test_one_row_merges_its_attention(heads, kv, dim, vdim, window):
+    """One sequence's steps whose output projection merges the attention's 1 to 16 partials itself (K of 512 to 2048; with 20
+    they keep their launch): empty partials, and windows that leave the first keys behind."""
+    cfg = C.model([C.attn(heads, kv, dim, vdim, window, ff=72), C.attn(heads, kv, dim, vdim, 40)], width=96, streams=2, groups=2)
+    eng, W = build(cfg, "bfloat16")
+    toks = tokens(cfg, 420, 6)
+    cache = eng.new_cache(2, 2600)
+    got = feed(eng, cache, cache.alloc(), toks, [1, 1, 1, 140, 1, 1, 270, 1], graph=True)
+    close(got, O.run(cfg, W, toks), "bfloat16")
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("sizes", [[2], [3], [1, 2, 5, 4], [17, 1, 40], [63, 2], [64], [65, 64], [130, 3]])
 @pytest.mark.parametrize("name", ["mixed_a", "mixed_b"])
