@@ -10,6 +10,7 @@ int gemv_mf_min_batch();
 void gemv_mf_qkv(hipStream_t s, const GemvArgs& a, float* ws);
 void gemv_mf_geglu(hipStream_t s, const GemvArgs& a);
 void gemv_mf_ores(hipStream_t s, const GemvArgs& a, uint16_t* o);
+void attn_combine(hipStream_t s, const GemvArgs& a, uint16_t* o);
 int gemv_mf_logits(hipStream_t s, const GemvArgs& a, int max_blocks);
 void gemv_mf_res(hipStream_t s, const GemvArgs& a, float* ws);
 void gemv_mf_res_norm(hipStream_t s, const GemvArgs& a, float* ws, const uint16_t* norm_w, float eps, uint16_t* hn);
@@ -101,14 +102,23 @@ void gemv_res_norm(hipStream_t s, int B, int K, const uint16_t* x, const uint16_
 }
 
 void gemv_o_attn(hipStream_t s, int B, int G, const float* part, int max_chunks, const StepState* st,
-                 const uint16_t* Wo, int N, uint16_t* h_inout, uint16_t* o_out, float* ssq, const uint16_t* Wf) {
+                 const uint16_t* Wo, int N, uint16_t* h_inout, uint16_t* o, int chunks, float* ssq, const uint16_t* Wf) {
     GemvArgs a{};
     a.x = nullptr; a.norm_w = nullptr; a.W = Wo; a.n_units = N; a.K = G * 256; a.nb = B; a.out = h_inout;
-    a.part = part; a.max_chunks = max_chunks; a.G = G; a.st = st; a.o_out = o_out;
-    if (B >= gemv_mf_min_batch() && o_out) {
+    a.part = part; a.max_chunks = max_chunks; a.G = G; a.st = st;
+    if (B >= gemv_mf_min_batch()) {
         a.ssq = ssq;
         a.Wf = N % 16 == 0 ? Wf : nullptr;
-        gemv_mf_ores(s, a, o_out);
+        gemv_mf_ores(s, a, o);
+        return;
+    }
+    // Every workgroup's prologue combines all heads of all rows: two rows of more chunks than it holds at a time (768 keys)
+    // take it longer than a launch that combines them once.  A step of two sequences, us, prologue / launch: 450 keys 1191 /
+    // 1180, 700 1210 / 1200, 1,056 1274 / 1229, 1,390 1290 / 1227; of one, whose prologue is half as long, 300 1071 / 1115, 1,390
+    // 1133 / 1144.  (Fewer than 13 chunks of two rows: 1166 / 1171.)
+    if (B == 2 && chunks > 12 && a.K == 2048) {
+        attn_combine(s, a, o);
+        gemv_res(s, B, a.K, o, Wo, N, h_inout, nullptr);
         return;
     }
     // grid capped so each workgroup's combine prologue is amortised over 8 output rows (256 / 128 / 64

@@ -899,10 +899,13 @@ void gemv_mf_geglu(hipStream_t s, const GemvArgs& a) {  // K = 2048, gate|up row
     else launch_mf<GV_GEGLU, 2, 512, 4, 1, true>(s, a, 512, 1, nullptr);  // input already normed
 }
 
+void attn_combine(hipStream_t s, const GemvArgs& a, uint16_t* o) {
+    hipLaunchKernelGGL(k_attn_combine, dim3((a.nb * a.K / 8 + 63) / 64), dim3(64), 0, s, a, o, a.K);
+}
+
 // o_proj: combine the attention partials once (-> o, bf16 [nb][K]), then the residual GEMV
 void gemv_mf_ores(hipStream_t s, const GemvArgs& a, uint16_t* o) {
-    const int K = a.K;
-    hipLaunchKernelGGL(k_attn_combine, dim3((a.nb * K / 8 + 63) / 64), dim3(64), 0, s, a, o, K);
+    attn_combine(s, a, o);
     GemvArgs r = a;
     r.x = o;
     r.norm_w = nullptr;
