@@ -145,7 +145,7 @@ constexpr int kPre = 8;   // rows whose step, input and gate are in flight ahead
 // LPC lanes per channel, NPL states per lane (N <= LPC * NPL; states past N are inert: B = C = 0).
 // PHASE 0: (A) zero entry state, no output; 1: (C) / single-chunk walk.
 template <typename T, int NPL, int LPC, int PHASE>
-__global__ void __launch_bounds__(256, LPC == 1 ? 2 : LPC == 2 ? 1 : 3) k_scan(ScanArgs a) {
+__global__ void __launch_bounds__(256, LPC == 1 ? 2 : LPC == 4 || LPC == 8 ? 3 : 1) k_scan(ScanArgs a) {
     constexpr int CPB = 256 / LPC;  // channels per workgroup
     constexpr int NP = NPL * LPC;
     constexpr bool AHEAD = LPC == 1;  // the next row's B | C read under this one's sums (they cost lanes that share a channel a wave)
