@@ -115,7 +115,8 @@ void gemv_o_attn(hipStream_t s, int B, int G, const float* part, int max_chunks,
     // Every workgroup's prologue combines all heads of all rows: two rows of more chunks than it holds at a time (768 keys)
     // take it longer than a launch that combines them once.  A step of two sequences, us, prologue / launch: 450 keys 1191 /
     // 1180, 700 1210 / 1200, 1,056 1274 / 1229, 1,390 1290 / 1227; of one, whose prologue is half as long, 300 1071 / 1115, 1,390
-    // 1133 / 1144.  (Fewer than 13 chunks of two rows: 1166 / 1171.)
+    // 1133 / 1144.  The launched chunks decide, which for a captured step are the cache's capacity: two rows of 250 keys in a
+    // large cache 1166 / 1171.
     if (B == 2 && chunks > 12 && a.K == 2048) {
         attn_combine(s, a, o);
         gemv_res(s, B, a.K, o, Wo, N, h_inout, nullptr);
