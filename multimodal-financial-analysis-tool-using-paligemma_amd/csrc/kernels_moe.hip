@@ -261,8 +261,9 @@ struct ExpertRows {
     static constexpr bool kGrouped = true;
     const ExpertArgs& a;
     const int* list = nullptr;
+    const int apart;
     int e = 0, rows = 0, m0 = 0, nt = 0;
-    __device__ __forceinline__ explicit ExpertRows(const ExpertArgs& x) : a(x) {}
+    __device__ __forceinline__ ExpertRows(const ExpertArgs& x, int k_tiles_apart) : a(x), apart(k_tiles_apart) {}
     __device__ __forceinline__ bool tile(int BM, int BN) {
         const TileAt t = find_tile(a.cnt, a.experts, BM, (a.N + BN - 1) / BN);
         e = t.e;
@@ -278,7 +279,9 @@ struct ExpertRows {
     // further apart 6.0).  Experts' weights are read by one or two row tiles and come from HBM: gate|up of 2,048 rows, top 6
     // of 60, 152.4 -> 148.2 us, down the same (dense products, whose weights many row tiles share: no change).  A matter of expert
     // and column tile alone, so that an output's sum does not depend on the step's other rows.
-    __device__ __forceinline__ int first_ktile() const { return 3 * (8 * e + nt); }
+    // (Long lists on 256-row tiles share their weights too: 4,096 rows of width 4,096, gate|up 840 us from the start, 868 from
+    // places apart, down 451 / 457: apart is 0.)
+    __device__ __forceinline__ int first_ktile() const { return apart * (8 * e + nt); }
     __device__ __forceinline__ int source(int m) const { return list[m] / a.gather; }
     __device__ __forceinline__ int target(int m) const { return list[m]; }
 };
@@ -290,7 +293,7 @@ __global__ void __launch_bounds__(512, 1) k_experts_8p(ExpertArgs a) {
     ea.ldo = a.ldo;
     gemm_8p<TM, MODE == EX_SWIGLU ? EPI_SWIGLU : EPI_STORE, false>(reinterpret_cast<const uint16_t*>(a.A), a.lda, a.W, a.ldw, 0,
                                                                   a.N, a.K, a.K / 64, ea, nullptr, (long)a.N * a.ldw, 0, 0,
-                                                                  ExpertRows(a));
+                                                                  ExpertRows(a, TM < 8 ? 3 : 0));
 }
 
 template <int TM, int MODE>
