@@ -11,6 +11,8 @@
 #pragma once
 #include <stddef.h>
 
+#include <algorithm>
+
 namespace pgmi {
 
 // Tile configurations (wave grid, per-wave MFMA tiles).  BM = WGM*TM*16, BN = WGN*TN*16.
@@ -76,7 +78,7 @@ struct TileForm {
     int cfg;
     int bm, bn;       // rows and columns of a tile (gate and up: bn / 2 of each)
     int per_cu;       // workgroups of one round on a CU
-    bool whole_k;     // needs K % 64 == 0
+    bool whole_k;     // needs K % 64 == 0 and a k-tile
     float c, a, b, lo;
 };
 
@@ -108,8 +110,11 @@ inline long form_tiles(const TileForm& f, int M, int N, bool dual) {
     return (long)((M + f.bm - 1) / f.bm) * ((N + bn - 1) / bn);
 }
 
+// (K = 0, the epilogue of empty sums, is planned as one k-tile)
+inline int k_tiles(int K) { return std::max(1, (K + 63) / 64); }
+
 inline float form_us(const TileForm& f, int M, int N, int K, int split, bool dual) {
-    const int nkt = (K + 63) / 64, per = (nkt + split - 1) / split;
+    const int nkt = k_tiles(K), per = (nkt + split - 1) / split;
     const long t = form_tiles(f, M, N, dual) * ((nkt + per - 1) / per), slots = 256L * f.per_cu;
     const long rest = t % slots;
     const float r = (float)(t / slots) + (rest ? f.lo + (1.0f - f.lo) * (float)rest / (float)slots : 0.0f);
@@ -120,9 +125,9 @@ inline float form_us(const TileForm& f, int M, int N, int K, int split, bool dua
 template <class Extra>
 TileChoice choose_form(int M, int N, int K, bool dual, int max_split, Extra extra) {
     TileChoice best{nullptr, 1, 0.0f};
-    const int nkt = (K + 63) / 64;
+    const int nkt = k_tiles(K);
     for (const TileForm& f : kTileForms) {
-        if (f.whole_k && K % 64 != 0) continue;
+        if (f.whole_k && (K % 64 != 0 || K < 64)) continue;
         for (int s = 1; s <= max_split && (s == 1 || nkt / s >= 4); ++s) {
             if ((nkt + (nkt + s - 1) / s - 1) / ((nkt + s - 1) / s) != s) continue;  // a slice would be empty
             const float x = extra(f, s);

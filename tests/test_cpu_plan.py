@@ -1,0 +1,39 @@
+"""The plans of bf16 products (csrc/plan.h, csrc/gemm_plan.hip), which are host code: compiled here and asked for shapes."""
+import os
+import subprocess
+
+import pytest
+
+CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))),
+                    "multimodal-financial-analysis-tool-using-paligemma_amd", "csrc")
+ASK = r"""
+#include <cstdio>
+#include <cstdlib>
+#include "gemm_plan.hip"
+int main(int n, char** v) {  // M, N, K, dual, what follows (0 .. 2), bytes for slabs
+    if (n != 7) return 2;
+    const pgmi::Plan p = pgmi::gemm_plan(atoi(v[1]), atoi(v[2]), atoi(v[3]), atoi(v[4]), (pgmi::After)atoi(v[5]), atol(v[6]));
+    std::printf("%d %d\n", p.cfg, p.split);
+}
+"""
+EIGHT_PHASE = (36, 37, 39, 40, 41)
+
+
+@pytest.fixture(scope="module")
+def plan(tmp_path_factory):
+    at = tmp_path_factory.mktemp("plan")
+    (at / "ask.cpp").write_text(ASK)
+    rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
+    subprocess.run(["g++", "-std=c++17", "-D__HIP_PLATFORM_AMD__", "-I", os.path.join(rocm, "include"), "-I", CSRC,
+                    str(at / "ask.cpp"), "-o", str(at / "ask")], check=True)
+    return lambda *a: tuple(int(x) for x in subprocess.run([str(at / "ask"), *map(str, a)], check=True, capture_output=True,
+                                                           text=True).stdout.split())
+
+
+@pytest.mark.parametrize("M,N,dual", [(1, 8, 0), (64, 64, 0), (300, 2048, 0), (3000, 4304, 0), (1, 64, 1), (2304, 16384, 1)])
+@pytest.mark.parametrize("after", [0, 1, 2])
+def test_no_k_is_one_slice_of_a_form_that_runs_without_k_tiles(plan, M, N, dual, after):
+    """A product of K = 0 is the epilogue of sums of nothing; the 8-phase kernel, which ends where there is no k-tile, leaves
+    its output unwritten."""
+    cfg, split = plan(M, N, 0, dual, after, 64 << 20)
+    assert split == 1 and cfg not in EIGHT_PHASE

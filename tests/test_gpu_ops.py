@@ -95,6 +95,19 @@ def test_gemm_epilogues(eng, epi):
     assert ulp_frac(got, ref, 1) > 0.98
 
 
+@pytest.mark.parametrize("epi", ["store", "bias", "bias_gelu", "bias_res", "res", "f32", "geglu"])
+@pytest.mark.parametrize("M,N", [(5, 64), (40, 200), (300, 2048), (3000, 264)])
+def test_gemm_of_no_k(eng, M, N, epi):
+    """K = 0: the epilogue of sums of nothing, whatever the rows."""
+    from pgmi._native import EPI
+    rng = np.random.default_rng(M + N)
+    b, r = rand(rng, N), rand(rng, M, N)
+    ref = {"bias": b + 0 * r, "bias_gelu": O.gelu_tanh(b + 0 * r), "bias_res": O.bf16(b + r), "res": r}.get(epi, 0 * r)
+    got = _gemm(eng, bf(np.zeros((M, 0))), bf(np.zeros((N * (2 if epi == "geglu" else 1), 0))), EPI[epi], bias=bf(b), res=bf(r),
+                out_f32=epi == "f32", geglu=epi == "geglu")
+    assert np.abs(got - O.bf16(ref)).max() <= 2.0 ** -7 * np.abs(ref).max()  # one bf16 step, which gelu may turn
+
+
 def test_gemm_geglu(eng):
     rng = np.random.default_rng(9)
     M, N, K = 288, 512, 2048
