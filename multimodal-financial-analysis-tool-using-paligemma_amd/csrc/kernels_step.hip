@@ -476,9 +476,9 @@ __global__ void __launch_bounds__(256) k_gemv_one(GemvRtArgs a) {
             if (s < a.nsplit && ml[s].y > 0.0f) m = fmaxf(m, ml[s].x);
 #pragma unroll
         for (int s = 0; s < MS; ++s) {
-            const bool is = s < a.nsplit && ml[s].y > 0.0f;
-            ml[s].x = is ? exp2f(ml[s].x - m) : 0.0f;
-            L += is ? ml[s].y * ml[s].x : 0.0f;
+            const bool there = s < a.nsplit;
+            ml[s].x = there && ml[s].y > 0.0f ? exp2f(ml[s].x - m) : 0.0f;
+            L += there ? ml[s].y * ml[s].x : 0.0f;  // a sum that is not a number takes the whole head with it (NaN * 0), as there
         }
 #pragma unroll
         for (int s = 0; s < MS; ++s) {

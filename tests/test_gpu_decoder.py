@@ -129,6 +129,26 @@ def test_one_row_merges_its_attention(heads, kv, dim, vdim, window):
     close(got, O.run(cfg, W, toks), "bfloat16")
 
 
+@pytest.mark.parametrize("window,at", [(900, 10), (900, 415), (1990, 300), (100, 400), (2500, 10)])
+def test_one_row_over_a_key_that_is_not_a_number(window, at):
+    """Scores that are not numbers take the heads that meet them out of a step, whichever of the attention's partials they are
+    in (the others' average would look like an answer): 8 and 16 partials merged by the output projection, one, and 20 that
+    keep their launch."""
+    cfg = C.model([C.attn(8, 2, 64, 64, window)], width=96, streams=2, groups=2)
+    W = O.random_weights(cfg, 3)
+    bad = cfg["vocab"] - 1
+    broken = {k: np.array(v) for k, v in W.items()}
+    broken["embed"][bad] = np.nan
+    eng, _ = build(cfg, "bfloat16", weights=broken)
+    toks = [t if t != bad else 0 for t in tokens(cfg, 421, 9)]
+    want = O.run(cfg, O.Weights(dict(W, **{"l0.mix.o": np.zeros_like(W["l0.mix.o"])})), toks)[-1:, :bad]
+    toks[at] = bad
+    cache = eng.new_cache(1, 2600)
+    slot = cache.alloc()
+    eng.step(cache, [slot], [toks[:-1]])
+    close(eng.step(cache, [slot], [toks[-1:]])[:, :bad], want, "bfloat16")
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("sizes", [[2], [3], [1, 2, 5, 4], [17, 1, 40], [63, 2], [64], [65, 64], [130, 3]])
 @pytest.mark.parametrize("name", ["mixed_a", "mixed_b"])
