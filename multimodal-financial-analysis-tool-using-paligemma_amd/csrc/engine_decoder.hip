@@ -7,6 +7,7 @@
 #include "decoder.h"
 #include "runs.h"
 #include "engine.h"
+#include "plan.h"
 
 namespace {
 
@@ -72,13 +73,11 @@ struct DecoderState {
     float *inv = nullptr, *ew = nullptr, *egate = nullptr;
     int *esel = nullptr, *elist = nullptr, *ecnt = nullptr, *eactive = nullptr;
     int zero_words = 0;  // the counters and the number of used experts
-    int slab_n = 0;  // columns of the widest product into slabs
+    int slab_n = 0;         // columns of the widest product into slabs
+    size_t slab_taken = 0;  // what the workspace has for K slabs
     // room for the K slabs of a step of these rows (not of the largest step so far: a step's sums are cut the same way
-    // whatever ran before it): four of them up to 160 MB, one of any step
-    size_t slab_bytes(int rows) const {
-        const size_t one = (size_t)rows * slab_n * 4;
-        return std::max({one, (size_t)32 << 20, std::min(4 * one, (size_t)160 << 20)});
-    }
+    // whatever ran before it; of a workspace that found no room for more than one slab, as that one allows)
+    size_t slab_bytes(int rows) const { return std::min(slab_room(rows, slab_n), slab_taken); }
     int ldh = 0, ld0 = 0, ld1 = 0, ld2 = 0, ldd = 0;
     // step metadata
     void* meta = nullptr;
@@ -459,22 +458,26 @@ int ensure_workspace(pgmi_ctx* x, int rows, size_t carries) {
     d.ldh = r8(D);
     d.ld0 = l0; d.ld1 = l1; d.ld2 = l2; d.ldd = ldd;
     d.slab_n = slab_n;
-    const size_t sizes[] = {(size_t)rows * d.c.streams * D * 4, (size_t)rows * d.ldh * d.es, (size_t)rows * l0 * d.es,
-                            (size_t)rows * l1 * d.es,           (size_t)rows * l2 * d.es,    (size_t)rows * ldd * d.es,
-                            d.slab_bytes(rows),                 (size_t)rows * inner * 4,    (size_t)rows * bcn * 4,
-                            ent * lea * d.es, ent * d.ldh * d.es, ent * 4, ent * 4, (size_t)rows * 4, (size_t)rows * 4,
-                            (size_t)rows * ne * 4, (size_t)(2 * ne + 2) * 4, here * 4};
+    size_t sizes[] = {(size_t)rows * d.c.streams * D * 4, (size_t)rows * d.ldh * d.es, (size_t)rows * l0 * d.es,
+                      (size_t)rows * l1 * d.es,           (size_t)rows * l2 * d.es,    (size_t)rows * ldd * d.es,
+                      0 /* slabs */,                      (size_t)rows * inner * 4,    (size_t)rows * bcn * 4,
+                      ent * lea * d.es, ent * d.ldh * d.es, ent * 4, ent * 4, (size_t)rows * 4, (size_t)rows * 4,
+                      (size_t)rows * ne * 4, (size_t)(2 * ne + 2) * 4, here * 4};
     constexpr int NB = sizeof(sizes) / sizeof(sizes[0]);
     size_t off[NB], total = 0;
-    for (int i = 0; i < NB; ++i) {
-        off[i] = total;
-        total += (sizes[i] + 511) / 256 * 256;
-    }
-    if (hipMalloc(&d.arena, total) != hipSuccess) {
+    d.slab_taken = take_slabs(rows, slab_n, [&](size_t slabs) {
+        sizes[6] = slabs;
+        total = 0;
+        for (int i = 0; i < NB; ++i) {
+            off[i] = total;
+            total += (sizes[i] + 511) / 256 * 256;
+        }
+        if (hipMalloc(&d.arena, total) == hipSuccess) return true;
         (void)hipGetLastError();
         d.arena = nullptr;
-        return fail(PGMI_E_NOMEM, "decoder workspace of " + std::to_string(total) + " bytes");
-    }
+        return false;
+    });
+    if (!d.arena) return fail(PGMI_E_NOMEM, "decoder workspace of " + std::to_string(total) + " bytes");
     uint8_t* p = reinterpret_cast<uint8_t*>(d.arena);
     d.X = reinterpret_cast<float*>(p + off[0]);
     d.h = p + off[1]; d.p0 = p + off[2]; d.p1 = p + off[3]; d.p2 = p + off[4]; d.dtl = p + off[5];

@@ -139,6 +139,20 @@ TileChoice choose_form(int M, int N, int K, bool dual, int max_split, Extra extr
     return best;
 }
 
+// Bytes for the K slabs of a layered decoder's step of these rows, `one` slab of the widest product being rows x n fp32: four of them
+// up to 160 MB, as many as the rule above gains from; at the least one, and 32 MB for steps of few rows.
+inline size_t slab_least(int rows, int n) { return std::max((size_t)rows * n * 4, (size_t)32 << 20); }
+inline size_t slab_room(int rows, int n) {
+    return std::max(slab_least(rows, n), std::min((size_t)rows * n * 16, (size_t)160 << 20));
+}
+// takes the room, or where the device does not have it the least, by alloc(bytes): the bytes taken, 0 if neither is there
+template <class Alloc>
+size_t take_slabs(int rows, int n, Alloc alloc) {
+    const size_t room = slab_room(rows, n), least = slab_least(rows, n);
+    if (alloc(room)) return room;
+    return least < room && alloc(least) ? least : 0;
+}
+
 // what follows a product: its own epilogue (K slices need k_splitk_epi's launch), a residual + norm kernel that reads
 // slabs as readily as rows, or RoPE + KV append (in the epilogue of some forms, else k_rope_kv)
 enum After { AFTER_OWN, AFTER_NORM, AFTER_ROPE };

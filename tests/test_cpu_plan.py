@@ -10,7 +10,13 @@ ASK = r"""
 #include <cstdio>
 #include <cstdlib>
 #include "gemm_plan.hip"
-int main(int n, char** v) {  // M, N, K, dual, what follows (0 .. 2), bytes for slabs
+int main(int n, char** v) {  // M, N, K, dual, what follows (0 .. 2), bytes for slabs; or rows, columns and the device's free bytes
+    if (n == 4) {
+        int tries = 0;
+        const size_t free = atol(v[3]), got = pgmi::take_slabs(atoi(v[1]), atoi(v[2]), [&](size_t b) { return ++tries, b <= free; });
+        std::printf("%zu %d\n", got, tries);
+        return 0;
+    }
     if (n != 7) return 2;
     const pgmi::Plan p = pgmi::gemm_plan(atoi(v[1]), atoi(v[2]), atoi(v[3]), atoi(v[4]), (pgmi::After)atoi(v[5]), atol(v[6]));
     std::printf("%d %d\n", p.cfg, p.split);
@@ -37,3 +43,15 @@ def test_no_k_is_one_slice_of_a_form_that_runs_without_k_tiles(plan, M, N, dual,
     its output unwritten."""
     cfg, split = plan(M, N, 0, dual, after, 64 << 20)
     assert split == 1 and cfg not in EIGHT_PHASE
+
+
+# before slabs were counted in fours, one of them or 32 MB: a device that has just that still takes the step
+@pytest.mark.parametrize("rows,n,room,least", [(1, 2048, 32 << 20, 32 << 20), (1024, 2048, 32 << 20, 32 << 20),
+                                               (1025, 2048, 1025 * 2048 * 16, 32 << 20), (4096, 2048, 4 << 25, 1 << 25),
+                                               (8192, 2048, 160 << 20, 1 << 26), (20480, 2048, 160 << 20, 160 << 20),
+                                               (300000, 4096, 300000 * 4096 * 4, 300000 * 4096 * 4)])
+def test_slabs_that_find_no_room(plan, rows, n, room, least):
+    assert plan(rows, n, room) == (room, 1)
+    assert plan(rows, n, room - 1) == ((least, 2) if least < room else (0, 1))
+    assert plan(rows, n, least) == (least, 1 if least == room else 2)
+    assert plan(rows, n, least - 1) == (0, 1 if least == room else 2)
