@@ -417,7 +417,7 @@ static int lm_body(pgmi_ctx* x, hipStream_t s, const int64_t* ids, const void* i
                 a.mask = x->d_zero; a.mask_b_stride = 0; a.mask_k_stride = 0; a.mask_round = 1;
                 attention_decode(s, a, x->pstep, kv_start + L, x->opart, x->max_chunks);
                 gemv_o_attn(s, B, NH, x->opart, x->max_chunks, x->pstep, TL(x, i, "self_attn.o_proj.weight"), H,
-                            x->lastrows, x->dAO, (kv_start + L + kAttnChunk - 1) / kAttnChunk);
+                            x->lastrows, x->dAO);
             } else {
                 attention_prefill(s, 256, a);
                 gemv_res(s, B, NH * HD, x->dAO, TL(x, i, "self_attn.o_proj.weight"), H, x->lastrows, x->ws);
@@ -521,7 +521,7 @@ static int decode_body(pgmi_ctx* x, hipStream_t s, const int64_t* ids, int B, vo
         }
         attention_decode(s, a, x->step, launch_keys, x->opart, x->max_chunks);
         gemv_o_attn(s, B, NH, x->opart, x->max_chunks, x->step, TL(x, i, "self_attn.o_proj.weight"), H, x->dH,
-                    x->dAO, (launch_keys + kAttnChunk - 1) / kAttnChunk, mf ? x->dSS : nullptr, Lf ? Lf + gu_n + qkv_n : nullptr);
+                    x->dAO, mf ? x->dSS : nullptr, Lf ? Lf + gu_n + qkv_n : nullptr);
         if (mf) {
             // the post-attention RMSNorm: its sums of squares come from o_proj's epilogue (dSS), gate|up
             // normalises h on load (no k_rows_norm pass: B = 8 step -5 us per layer)

@@ -102,7 +102,7 @@ void gemv_res_norm(hipStream_t s, int B, int K, const uint16_t* x, const uint16_
 }
 
 void gemv_o_attn(hipStream_t s, int B, int G, const float* part, int max_chunks, const StepState* st,
-                 const uint16_t* Wo, int N, uint16_t* h_inout, uint16_t* o, int chunks, float* ssq, const uint16_t* Wf) {
+                 const uint16_t* Wo, int N, uint16_t* h_inout, uint16_t* o, float* ssq, const uint16_t* Wf) {
     GemvArgs a{};
     a.x = nullptr; a.norm_w = nullptr; a.W = Wo; a.n_units = N; a.K = G * 256; a.nb = B; a.out = h_inout;
     a.part = part; a.max_chunks = max_chunks; a.G = G; a.st = st;
@@ -112,12 +112,12 @@ void gemv_o_attn(hipStream_t s, int B, int G, const float* part, int max_chunks,
         gemv_mf_ores(s, a, o);
         return;
     }
-    // Every workgroup's prologue combines all heads of all rows: two rows of more chunks than it holds at a time (768 keys)
-    // take it longer than a launch that combines them once.  A step of two sequences, us, prologue / launch: 450 keys 1191 /
-    // 1180, 700 1210 / 1200, 1,056 1274 / 1229, 1,390 1290 / 1227; of one, whose prologue is half as long, 300 1071 / 1115, 1,390
-    // 1133 / 1144.  The launched chunks decide, which for a captured step are the cache's capacity: two rows of 250 keys in a
-    // large cache 1166 / 1171.
-    if (B == 2 && chunks > 12 && a.K == 2048) {
+    // Every workgroup's prologue combines all heads of all rows: for two rows a launch that combines them once is no slower at
+    // any length, and faster from about 300 keys on.  A captured step of two sequences, us, prologue / launch: 58 keys 1136 / 1132,
+    // 250 1169 / 1165, 378 1176 / 1162, 698 1198 / 1177, 762 (a second pass of the prologue) 1236 / 1190, 986 1252 / 1196, 1,338
+    // 1272 / 1203; 100 keys in caches of 256 to 1,408 the same to 1 % faster.  (One row, whose prologue is half as long: 300
+    // keys 1071 / 1115, 1,390 1133 / 1144.)
+    if (B == 2 && a.K == 2048) {
         attn_combine(s, a, o);
         gemv_res(s, B, a.K, o, Wo, N, h_inout, nullptr);
         return;

@@ -100,11 +100,11 @@ void mf_swizzle(hipStream_t s, const uint16_t* W, int rows, int K, uint16_t* out
 void rows_norm(hipStream_t s, const uint16_t* x, const uint16_t* w, float eps, int nb, int K, uint16_t* out);
 // o_proj + residual whose input is the combine of the decode-attention partials (MQA:
 // n_kv = 1, G heads of 256); o [B][G * 256]: room for the combined rows of the forms that combine them in a launch of their
-// own, chunks: of the launched keys.
+// own (two rows and more).
 // ssq (batched MFMA form only, else ignored): each row's 16-column partial sums of squares of the
 // new h, [B][N / 16] -- the next RMSNorm's, read by gemv_geglu
 void gemv_o_attn(hipStream_t s, int B, int G, const float* part, int max_chunks, const StepState* st,
-                 const uint16_t* Wo, int N, uint16_t* h_inout, uint16_t* o, int chunks, float* ssq = nullptr,
+                 const uint16_t* Wo, int N, uint16_t* h_inout, uint16_t* o, float* ssq = nullptr,
                  const uint16_t* Wf = nullptr);
 // fused RMSNorm + gate|up + GeGLU; ssq (B >= gemv_mf_min_batch() only): h's RMSNorm from the
 // partials gemv_o_attn wrote instead of the row pass; Wf (idem): the gate|up weights' fragment-major
