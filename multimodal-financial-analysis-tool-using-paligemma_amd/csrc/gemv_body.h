@@ -58,7 +58,6 @@ struct GemvArgs {
     const float* part;
     int max_chunks;
     int G;
-    uint16_t* o_out;
     // QKV of decode layer 0 (EMB kernels): x is the token's embedding row, bf16(E[id] * normalizer)
     // (modeling_gemma.py:565,368; a pad id gives a zero row), read here instead of from a separate
     // embedding launch; workgroup 0 also stores it to emb_out (the layer's residual h)
@@ -236,7 +235,6 @@ __device__ __forceinline__ void gemv_block(const GemvArgs& a, const int blk, con
 #pragma unroll
             for (int j = 0; j < 8; ++j) ob.v[j] = f2bf(o[j] / S);
             *reinterpret_cast<u16x8*>(xs + b * K + e) = ob;
-            if (a.o_out && blk == 0) *reinterpret_cast<u16x8*>(a.o_out + (long)b * K + e) = ob;
         }
         for (int e8 = tid; e8 < (B - a.nb) * K / 8; e8 += 256)
             *reinterpret_cast<uint4*>(xs + a.nb * K + e8 * 8) = make_uint4(0, 0, 0, 0);

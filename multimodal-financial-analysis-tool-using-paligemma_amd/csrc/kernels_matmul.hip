@@ -121,7 +121,7 @@ void run_w128(const Job& j) {
 template <int TM, int EPI, bool SPLIT>
 void run_8p(const Job& j) {
     constexpr int BM = 32 * TM, BN = epi_dual(EPI) ? 128 : 256;
-    constexpr size_t lds = (size_t)2 * (BM * 128 + 2 * 128 * 128);
+    constexpr size_t lds = lds_8p(TM);
     const int n_mt = (j.M + BM - 1) / BM, n_nt = (j.N + BN - 1) / BN;
     lds_attr<&k_gemm_8p<TM, EPI, SPLIT>>(lds);
     hipLaunchKernelGGL((k_gemm_8p<TM, EPI, SPLIT>), dim3(n_mt * n_nt, j.split), dim3(512), lds, j.s, j.A, j.lda, j.W, j.ldw,

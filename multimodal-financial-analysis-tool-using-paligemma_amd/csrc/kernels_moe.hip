@@ -299,7 +299,7 @@ __global__ void __launch_bounds__(512, 1) k_experts_8p(ExpertArgs a) {
 template <int TM, int MODE>
 void run_experts_8p(hipStream_t s, const ExpertArgs& a) {
     constexpr int BM = 32 * TM, BN = MODE == EX_SWIGLU ? 128 : 256;
-    constexpr size_t lds = (size_t)2 * (2 * 16 * TM * 128 + 2 * 128 * 128);
+    constexpr size_t lds = lds_8p(TM);
     static bool done = false;
     if (!done) {
         (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&k_experts_8p<TM, MODE>),
