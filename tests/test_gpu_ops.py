@@ -11,6 +11,7 @@ import torch
 
 from oracle import paligemma_np as O
 from oracle import weights as W
+from tests_helpers import PLANNED
 
 pytestmark = pytest.mark.gpu
 
@@ -318,13 +319,9 @@ def test_gemm_8phase(eng, cfg, M, N, K, epi, split):
     assert rel_l2(got, ref) < tol
 
 
-@pytest.mark.parametrize("M,N,K,epi", [
-    (17, 2560, 2048, "store"), (33, 200, 72, "bias"), (257, 1152, 1152, "bias_res"), (289, 1001, 2048, "store"),
-    (304, 2048, 4096, "res"), (512, 4304, 1152, "bias_gelu"), (577, 1152, 4304, "bias_res"), (640, 1024, 2048, "geglu"),
-    (783, 2048, 1160, "res"), (1281, 3456, 1152, "bias"), (1540, 520, 2048, "geglu"), (2049, 1152, 1152, "bias_res"),
-])
+@pytest.mark.parametrize("M,N,K,epi", PLANNED)
 def test_gemm_planned_matches_general(eng, M, N, K, epi):
-    """The tiles that the cost rule picks (plan.h: every form up to 288 rows, the 8-phase heights, K tails, rows and columns
+    """The tiles that the cost rule picks (each of plan.h's forms at least once, whole and in K slices, K tails, rows and columns
     past the last tile) against the general register-staged tiles, forced through the tuning hook.  Both sum in fp32, in
     another order, and round to bf16 once per rounding point: they differ by single roundings."""
     from pgmi import _native as NN
@@ -340,3 +337,64 @@ def test_gemm_planned_matches_general(eng, M, N, K, epi):
     finally:
         NN.check(eng.lib.pgmi_tune_gemm(-1, 0))
     assert rel_l2(got, ref) < 3e-3
+
+
+@pytest.mark.parametrize("cfg", [36, 37, 39, 40, 41])
+@pytest.mark.parametrize("N,shift", [(264, 0), (261, 0), (264, 1)])
+def test_gemm_8phase_epilogues(eng, cfg, N, shift):
+    """Every epilogue of whole (unsliced) 8-phase tiles: eight outputs and their operands in 16-byte accesses, and singly where the
+    columns are no multiple of 8 or the addresses no multiple of 16; ragged rows; nothing written beside the output.  (As
+    test_gemm_epilogues: fp32 sums in another order, the same rounding points.)"""
+    from pgmi import _native as NN
+    from pgmi._native import EPI
+    M, K = 301, 320
+    rng = np.random.default_rng(N + cfg)
+    A, Wg, Wu = rand(rng, M, K), rand(rng, N, K, scale=2 / np.sqrt(K)), rand(rng, N, K, scale=2 / np.sqrt(K))
+    b, r = rand(rng, N, scale=0.3), rand(rng, M, N)
+    acc, up = A @ Wg.T, A @ Wu.T
+    want = {"store": O.bf16(acc), "f32": O.bf16(acc), "bias": O.bf16(acc + b), "bias_gelu": O.gelu_tanh(O.bf16(acc + b)),
+            "bias_res": O.bf16(O.bf16(acc + b) + r), "res": O.bf16(O.bf16(acc) + r),
+            "geglu": O.bf16(O.gelu_tanh(O.bf16(acc)) * O.bf16(up))}
+
+    def placed(x):  # `shift` elements past a 16-byte address, between others
+        x = torch.as_tensor(x)
+        flat = torch.full((x.numel() + 16,), 7.0, dtype=x.dtype, device="cuda")
+        flat[8 + shift:8 + shift + x.numel()] = x.flatten()
+        return flat, flat[8 + shift:8 + shift + x.numel()].view(x.shape)
+
+    Ad, Wd = bf(A), bf(np.concatenate([Wg, Wu]))
+    bias, res = placed(bf(b))[1], placed(bf(r))[1]
+    NN.check(eng.lib.pgmi_tune_gemm(cfg, 1))
+    try:
+        for epi, ref in want.items():
+            flat, out = placed(torch.zeros((M, N), dtype=torch.float32 if epi == "f32" else torch.bfloat16))
+            NN.check(eng.lib.pgmi_op_gemm(eng.ctx, Ad.data_ptr(), Wd.data_ptr(), M, N, K, EPI[epi], bias.data_ptr(),
+                                          res.data_ptr(), out.data_ptr(), NN.stream_handle()))
+            torch.cuda.synchronize()
+            assert rel_l2(np32(out), ref) < (5e-3 if epi == "geglu" else 3e-3), epi
+            assert (flat[:8 + shift] == 7.0).all() and (flat[8 + shift + M * N:] == 7.0).all(), epi
+    finally:
+        NN.check(eng.lib.pgmi_tune_gemm(-1, 0))
+
+
+@pytest.mark.parametrize("cfg", [36, 37, 39, 40, 41])
+def test_gemm_8phase_positions(eng, cfg):
+    """The position epilogue of whole 8-phase tiles, rows of several images: the patch embedding at its own sizes."""
+    from pgmi import _native as NN
+    B, C, H, P, D = 2, 3, 196, 14, 264
+    n, k = (H // P) ** 2, C * P * P
+    rng = np.random.default_rng(cfg)
+    px, w = rand(rng, B, C, H, H), rand(rng, D, k, scale=1 / np.sqrt(k))
+    b, pos = rand(rng, D, scale=0.3), rand(rng, n, D)
+    rows = px.reshape(B, C, H // P, P, H // P, P).transpose(0, 2, 4, 1, 3, 5).reshape(B * n, k)
+    want = O.bf16(O.bf16(rows @ w.T + b) + np.tile(pos, (B, 1)))
+    out = torch.empty((B * n, D), dtype=torch.bfloat16, device="cuda")
+    args = [torch.from_numpy(px).cuda(), bf(w), bf(b), bf(pos)]
+    NN.check(eng.lib.pgmi_tune_gemm(cfg, 1))
+    try:
+        NN.check(eng.lib.pgmi_op_patch_embed(eng.ctx, args[0].data_ptr(), 2, B, C, H, P, args[1].data_ptr(), args[2].data_ptr(),
+                                             args[3].data_ptr(), D, out.data_ptr(), NN.stream_handle()))
+        torch.cuda.synchronize()
+    finally:
+        NN.check(eng.lib.pgmi_tune_gemm(-1, 0))
+    assert rel_l2(np32(out), want) < 3e-3

@@ -8,6 +8,21 @@ import numpy as np
 REL_L2_RULE = 2e-2
 
 
+# Products for which the cost rule (csrc/plan.h) picks each of its forms in turn, whole and in K slices, with K tails and rows and
+# columns past the last tile: test_cpu_plan.py holds the list to that, test_gpu_ops.py runs it.
+PLANNED = [
+    (17, 2560, 2048, "store"), (33, 200, 72, "bias"), (257, 1152, 1152, "bias_res"), (289, 1001, 2048, "store"),
+    (304, 2048, 4096, "res"), (512, 4304, 1152, "bias_gelu"), (577, 1152, 4304, "bias_res"), (640, 1024, 2048, "geglu"),
+    (783, 2048, 1160, "res"), (1281, 3456, 1152, "bias"), (1540, 520, 2048, "geglu"), (2049, 1152, 1152, "bias_res"),
+    # the forms that those leave out
+    (33, 3456, 8192, "geglu"), (193, 8200, 72, "geglu"), (601, 2560, 72, "geglu"), (1563, 2560, 2048, "bias_gelu"),
+    (416, 8200, 128, "geglu"), (416, 8200, 512, "geglu"), (601, 8200, 128, "geglu"), (675, 8200, 128, "geglu"),
+    # K slices
+    (17, 200, 4096, "store"), (289, 200, 4304, "bias_res"), (65, 2560, 4304, "res"), (97, 8200, 4096, "bias_gelu"),
+    (161, 8200, 4096, "bias"),
+]
+
+
 def rel_l2(a, b):
     a, b = np.asarray(a, np.float64), np.asarray(b, np.float64)
     return float(np.linalg.norm(a - b) / max(np.linalg.norm(b), 1e-30))
