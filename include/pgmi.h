@@ -230,8 +230,8 @@ int pgmi_prefill_kernel(pgmi_ctx* ctx, int which, int layer, int rows, void* str
 int pgmi_prefill_probe(pgmi_ctx* ctx, int on);
 int pgmi_prefill_probe_times(pgmi_ctx* ctx, float* us, int n);
 /* Tuning hook: force the prefill GEMM tile configuration and split-K factor for subsequent
- * calls (kernels_gemm.hip enum Cfg: 0-5 register-staged tiles, 6-29 LDS-DMA panel tiles, 30-35 warp-specialised panel tiles);
- * cfg < 0 restores the automatic (measured) plan. */
+ * calls (plan.h enum Cfg: 0-5 register-staged tiles, 6-29 LDS-DMA panel tiles, 30-35 and 38 warp-specialised panel tiles, 36,
+ * 37 and 39-41 8-phase tiles); cfg < 0 restores the automatic plan. */
 int pgmi_tune_gemm(int cfg, int split);
 /* Tuning hook: the same for ONE GEMM shape (M x N x K, dual = the gate|up GeGLU form) while every
  * other shape keeps its plan (in-situ sweeps of a whole forward); cfg < 0 removes the override.

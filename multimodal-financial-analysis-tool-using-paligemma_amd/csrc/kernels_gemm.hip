@@ -1674,7 +1674,7 @@ static void launch_e(hipStream_t s, const uint16_t* A, int lda, const uint16_t* 
 int gemm(hipStream_t s, const uint16_t* A, int lda, const uint16_t* W, int ldw, int M, int N, int K, Epi epi,
          const EpiArgs& ea, float* ws, size_t ws_bytes, int up_offset_rows, bool defer) {
     Plan p = gemm_plan(M, N, K, epi == EPI_GEGLU, !defer ? AFTER_OWN : epi == EPI_STORE ? AFTER_ROPE : AFTER_NORM, ws_bytes);
-    if ((p.cfg == E256 || p.cfg == E192 || p.cfg >= E128) && K % 64 != 0) p.cfg = P128w;  // the 8-phase kernel has no K tail
+    if ((p.cfg == E256 || p.cfg == E192 || p.cfg >= E128) && K % 64 != 0) p.cfg = P128w;  // (a forced plan: 8-phase has no K tail)
     if (p.split > 1 && (size_t)p.split * M * N * sizeof(float) > ws_bytes) p.split = 1;
     if (p.split > 1 && N % 4 != 0) p.split = 1;  // the split-K epilogue works on 4 outputs per thread
     const long up_off = (long)up_offset_rows * ldw;
@@ -1720,7 +1720,8 @@ bool gemm_qkv_rope(hipStream_t s, const uint16_t* A, int lda, const uint16_t* W,
     if (N % 256 != 0 || N != (ea.nh + 2 * ea.nkv) * 256) return false;
     const Plan p = gemm_plan(M, N, K, false, AFTER_ROPE, ws_bytes);
     if (p.split != 1) return false;
-    // configurations with two 16-column tiles per wave and a tile width dividing 256
+    // configurations with two 16-column tiles per wave and a tile width dividing 256 (gemm_plan.hip's rope_form, and, for
+    // forced plans, others)
 #define P_(wm, tm, st) launch_p<4, wm, tm, 2, st, EPI_ROPE>(s, A, lda, W, ldw, M, N, K, ea, nullptr, 1, 0)
 #define W_(nw, tm, st) launch_w<nw, 2, tm, 2, st, 4, EPI_ROPE>(s, A, lda, W, ldw, M, N, K, ea, nullptr, 1, 0)
     switch (p.cfg) {

@@ -131,8 +131,9 @@ void run_8p(const Job& j) {
 long tiles(int M, int N, int bm, int bn) { return (long)((M + bm - 1) / bm) * ((N + bn - 1) / bn); }
 
 // The form with the least predicted time (plan.h, whose forms are the same kernels but for the height of their ring).
-// slab_bytes > 0: into slabs, K cut as the form gains from it; the residual's pass then reads every slab, 0.25 us per MB
-// past the first one's.  Before, K slices were counted in 64 x 64 tiles and three tile shapes had fixed borders.  1,540 rows,
+// slab_bytes > 0: into slabs, K cut as the form gains from it; the pass that follows reads every slab, 0.25 us per MB past the
+// first one, which it reads of a whole product too (gemm_plan.hip's readers take bf16 rows where a product is whole, behind
+// fixed work of their own: another price).  Before, K slices were counted in 64 x 64 tiles and three tile shapes had fixed borders.  1,540 rows,
 // us before / now: 2048 columns of K = 16384 123 / 97 (three slices), 6144 of 2048 48.3 / 41.0, 2560 of 2048 39.4 / 30.6,
 // 4096 of 128 12.2 / 10.5.
 template <int EPI, bool SPLIT>

@@ -2,12 +2,17 @@
 //
 // A form's time is c + R (a + b n): n the 64-deep k-tiles of a slice, R the rounds of its workgroups over the chip, of
 // which a round that is not full takes lo + (1 - lo) of its share (the workgroups that are there run faster, not in
-// proportion).  c, a, b and lo (us) were set on MI355X from 11,400 launches with cold weights: M 32 .. 4608 at 27
-// (N, K) of this library's layers, K slices 1 .. 16.  The form chosen is on average 0.9 % slower than the best one
-// measured for its shape, 7 % over the tenth of the shapes where it does worst.
+// proportion).  c, a, b and lo (us) were set on MI355X from launches with cold weights: M 32 .. 4608 at 27 (N, K) of this
+// library's layers, K slices.  tools/plan_fit.py times such launches, holds the constants against them and fits them again;
+// 19,281 of its times are in profiles/gemm_plan_sweep.csv.gz.  Over these the constants are off by 8 % (E128) to 24 % (W64x64)
+// of a time on average, and the form chosen, the price of its slabs included, is 2.2 % (layered decoders) to 3.2 % slower than
+// the best of 702 shapes' measured forms, 16 to 22 % over the tenth of the shapes where it does worst: K of 64 and 128, few
+// tiles of long K, and rows that are no multiple of 128 bytes (K = 4304), whose k-tiles take 1.3 to 1.5 b.
 // What it replaced, plans listed for the shapes of one photo of each size and of eight with one rule for all others:
 // 576 rows, 16384 gate and up columns of K = 2048: 110 us, here 74; 640: 110 / 90; 1280: 190 / 143; 512 rows of q|k|v
 // (3456 columns of K = 1152): 25 / 11; prompts of 2 .. 7 photos 1.21 - 1.33x faster, of one with another text 1.1 - 1.2x.
+// (One listed plan was better: 256 rows, 1152 columns of K = 4304, P96x64s4 in four slices 12.5 us, here P64x64s4 in three
+// 13.3; the tower of one 224 px photo 1,442 -> 1,461 us, the photo's whole call 3,759 -> 3,727.)
 #pragma once
 #include <stddef.h>
 
@@ -15,7 +20,9 @@
 
 namespace pgmi {
 
-// Tile configurations (wave grid, per-wave MFMA tiles).  BM = WGM*TM*16, BN = WGN*TN*16.
+// Tile configurations (wave grid, per-wave MFMA tiles).  BM = WGM*TM*16, BN = WGN*TN*16.  The rule takes those of kTileForms
+// below and, up to 16 rows, P64x64 and P64x128; the others are there for the tuning hooks (pgmi_tune_gemm*), which name a
+// configuration by its number here.
 enum Cfg : int {
     C288x64 = 0,   // 6x1 waves, 3x4 tiles  (text rows: M = 288 = 18 x 16)
     C288x32 = 1,   // 6x1 waves, 3x2 tiles
@@ -121,7 +128,8 @@ inline float form_us(const TileForm& f, int M, int N, int K, int split, bool dua
     return f.c + r * (f.a + f.b * (float)per);
 }
 
-// the least form_us + extra(form, slices) over the forms and slices of at least four k-tiles; extra < 0: not to be taken
+// the least form_us + extra(form, slices) over the forms and slices, of four k-tiles or more on average (the last one takes what
+// is left); extra < 0: not to be taken
 template <class Extra>
 TileChoice choose_form(int M, int N, int K, bool dual, int max_split, Extra extra) {
     TileChoice best{nullptr, 1, 0.0f};
