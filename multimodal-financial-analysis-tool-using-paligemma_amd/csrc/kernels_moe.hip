@@ -277,8 +277,10 @@ struct ExpertRows {
     // Weight rows of 2,048 or 1,024 columns are 4 or 2 KiB apart, so one K-tile of all of them falls on one of an XCD's 16 cache
     // channels: tiles in step read cold weights at 4.5 TB/s, tiles three K-tiles apart from each other at 5.9 (rows 128 bytes
     // further apart 6.0).  Experts' weights are read by one or two row tiles and come from HBM: gate|up of 2,048 rows, top 6
-    // of 60, 152.4 -> 148.2 us, down the same (dense products, whose weights many row tiles share: no change).  A matter of expert
-    // and column tile alone, so that an output's sum does not depend on the step's other rows.
+    // of 60, 152.4 -> 148.2 us, down the same (dense products, whose weights many row tiles share: no change).  The place goes by
+    // the expert and the column tile, not by where a row stands in its list; but these tiles are taken by the step's mean list
+    // (experts_rt: 129 to 384 rows), so past those borders an output's fp32 sum runs in another order, as a dense product's does
+    // with the K slices that its rows bring.
     // (Long lists on 256-row tiles share their weights too: 4,096 rows of width 4,096, gate|up 840 us from the start, 868 from
     // places apart, down 451 / 457: apart is 0.)
     __device__ __forceinline__ int first_ktile() const { return apart * (8 * e + nt); }
