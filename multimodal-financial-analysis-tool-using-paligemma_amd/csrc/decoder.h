@@ -226,6 +226,7 @@ struct ScanArgs {
     const ChunkInfo* chunks;
     int nchunk;
     bool multi;  // some sequence has more than one chunk
+    bool walk;   // whole sequences, a lane per state (9 to 16 of them); chunks, cstate and csum are not read
 };
 int scan_max_state();
 void selective_scan(hipStream_t s, Act act, const ScanArgs& a);

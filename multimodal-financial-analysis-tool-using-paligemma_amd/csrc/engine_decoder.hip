@@ -583,6 +583,7 @@ struct Meta {
         int n;
         bool multi;  // some sequence has more than one
     } scan, gru, conv;
+    ScanStep step;
     bool fresh;  // every sequence from its start
     const int* row_seq;
     const int* want;
@@ -650,7 +651,7 @@ int forward_body(pgmi_ctx* x, hipStream_t s, const int64_t* ids, int rows, const
             a.dt = d.dt; a.dtb = w.dt_b; a.x = d.p1; a.ldx = ldc; a.z = d.p0 + (size_t)C * d.es; a.ldz = ldxz; a.bc = d.bc;
             a.A_log = w.A_log; a.Dw = w.D; a.state = at<float>(state, st[i].b); a.cstate = d.cstate; a.csum = d.csum;
             a.y = d.p2; a.ldy = ldc; a.C = C; a.N = N; a.seqs = m.seqs; a.nseq = m.nseq; a.chunks = m.scan.p;
-            a.nchunk = m.scan.n; a.multi = m.scan.multi;
+            a.nchunk = m.scan.n; a.multi = m.scan.multi; a.walk = scan_walks(m.step, C, N, d.act == ACT_F32);
             selective_scan(s, d.act, a);
             out_proj(w.o, d.p2, ldc, w.sub[0]);
         } else if (l.mixer == PGMI_MIXER_ATTENTION) {
@@ -1090,7 +1091,12 @@ int pgmi_decoder_forward(pgmi_ctx* x, const int64_t* ids, int n_seq, const int32
     }
     const bool huge = rows > 16384;
     Cut scan{0, 0, false}, gru = scan, conv = scan;
-    if (scan_cols) scan = cut(huge ? 256 : scan_run_rows(lens, n_seq, scan_cols, scan_wgs));
+    ScanStep step;
+    if (scan_cols) {
+        const int run = huge ? 256 : scan_run_rows(lens, n_seq, scan_cols, scan_wgs);
+        scan = cut(run);
+        step = scan_step_of(lens, n_seq, run);
+    }
     if (gru_cols) gru = cut(huge ? 128 : gru_run_rows(lens, n_seq, gru_cols));
     // the convolutions carry nothing: 500 rows of 2,048 channels 11.2 us on 64-row runs, 5.9 on 16; 2,048 rows 10.8 / 7.5
     if (scan_cols || d.c.canon_taps > 0) conv = cut(huge ? 256 : rows > 2048 ? 32 : 16);
@@ -1134,6 +1140,7 @@ int pgmi_decoder_forward(pgmi_ctx* x, const int64_t* ids, int n_seq, const int32
     meta.nseq = n_seq;
     meta.fresh = std::all_of(starts, starts + n_seq, [](int32_t p) { return p == 0; });
     meta.scan = {reinterpret_cast<const ChunkInfo*>(dm + scan.o), scan.n, scan.multi};
+    meta.step = step;
     meta.gru = {reinterpret_cast<const ChunkInfo*>(dm + gru.o), gru.n, gru.multi};
     meta.conv = {reinterpret_cast<const ChunkInfo*>(dm + conv.o), conv.n, conv.multi};
     meta.row_seq = dm + o_row;

@@ -6,8 +6,10 @@
 // state and its total decay), (B) one short walk over the chunks that turns these into the chunks' entry states,
 // (C) every chunk again from its entry state, writing the outputs; the last chunk leaves the sequence's state.
 // The decay of a chunk is exp(A sum(dt)), so (A) keeps sums of steps and no products.
+// A scan of 9 to 16 states walks its sequences whole instead, a lane per state, where that is predicted to be faster (scan_walks).
 #include <algorithm>
 #include <type_traits>
+#include <utility>
 
 #include "act.h"
 #include "decoder.h"
@@ -369,6 +371,229 @@ __global__ void __launch_bounds__(256) k_scan_carry(ScanArgs a) {
     }
 }
 
+// ---- sequences walked whole, a lane per state
+// What bounds it: one wave a SIMD has 64 states of one sequence, and issues an instruction every 4.5 to 5.5 clocks (8.4 an exponential)
+// however independent they are; a step is one exponential, two products with a value of the channel (broadcast within the
+// instruction, DPP), an FMA, a product with C and two additions of the sum over the states: 25 ns of the longest sequence's step,
+// 18 of them those instructions'.  So everything else is another four waves' work.  One wave for both: 36 ns; with its loads and
+// stores straight from memory, 16 rows of 4 channels an instruction, 43.  us a layer: see scan_walks.
+constexpr int kWalk = 16;  // channels of a workgroup, lanes of a channel, and rows of a block
+
+// step t's value of a channel's 16 lanes
+template <int t>
+__device__ __forceinline__ float of_step(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x150 + t, 0xF, 0xF, true));
+}
+template <typename F, int... t>
+__device__ __forceinline__ void each_step(const F& f, std::integer_sequence<int, t...>) {
+    (f(std::integral_constant<int, t>{}), ...);
+}
+// lane j of each 16 gets the sum of p[j] over the 16: halves and quarters exchanged by lanes that write only their own part (two
+// additions where a choice and an addition would be three), then the four lanes of a quarter
+__device__ __forceinline__ float sum_of_step(const float (&p)[kWalk], int lane) {
+    float a[8], b[4];
+#define HALF_(k, lo, hi) "v_add_f32_dpp %" #k ", %" #lo ", %" #lo " row_ror:8 row_mask:0xf bank_mask:0x3\n" \
+                         "v_add_f32_dpp %" #k ", %" #hi ", %" #hi " row_ror:8 row_mask:0xf bank_mask:0xc\n"
+#define QUARTER_(k, lo, hi) "v_add_f32_dpp %" #k ", %" #lo ", %" #lo " row_half_mirror row_mask:0xf bank_mask:0x5\n" \
+                            "v_add_f32_dpp %" #k ", %" #hi ", %" #hi " row_half_mirror row_mask:0xf bank_mask:0xa\n"
+    asm("s_nop 1\n" HALF_(0, 8, 16) HALF_(1, 9, 17) HALF_(2, 10, 18) HALF_(3, 11, 19) HALF_(4, 12, 20) HALF_(5, 13, 21)
+        HALF_(6, 14, 22) HALF_(7, 15, 23)
+        : "=&v"(a[0]), "=&v"(a[1]), "=&v"(a[2]), "=&v"(a[3]), "=&v"(a[4]), "=&v"(a[5]), "=&v"(a[6]), "=&v"(a[7])
+        : "v"(p[0]), "v"(p[1]), "v"(p[2]), "v"(p[3]), "v"(p[4]), "v"(p[5]), "v"(p[6]), "v"(p[7]), "v"(p[8]), "v"(p[9]),
+          "v"(p[10]), "v"(p[11]), "v"(p[12]), "v"(p[13]), "v"(p[14]), "v"(p[15]));
+    asm("s_nop 1\n" QUARTER_(0, 4, 8) QUARTER_(1, 5, 9) QUARTER_(2, 6, 10) QUARTER_(3, 7, 11) "s_nop 1\n"
+        : "=&v"(b[0]), "=&v"(b[1]), "=&v"(b[2]), "=&v"(b[3])
+        : "v"(a[0]), "v"(a[1]), "v"(a[2]), "v"(a[3]), "v"(a[4]), "v"(a[5]), "v"(a[6]), "v"(a[7]));
+#undef HALF_
+#undef QUARTER_
+    auto other = [](float v, auto ctrl) {
+        return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), decltype(ctrl)::value, 0xF, 0xF, true));
+    };
+    const bool o1 = lane & 1, o2 = lane & 2;
+    using X1 = std::integral_constant<int, 0xB1>;  // quad_perm 1 0 3 2
+    using X2 = std::integral_constant<int, 0x4E>;  // quad_perm 2 3 0 1
+    const float c0 = (o1 ? b[1] : b[0]) + other(o1 ? b[0] : b[1], X1{}), c1 = (o1 ? b[3] : b[2]) + other(o1 ? b[2] : b[3], X1{});
+    return (o2 ? c1 : c0) + other(o2 ? c0 : c1, X2{});
+}
+
+// Four waves walk 16 channels, four others have the rest: they fetch the rows (asked for 64 rows ahead of their use), form the
+// steps and inputs of the next 64 rows while these are walked, and gate and store the 64 rows before.  V4: such a thread has four
+// channels of one row, else one channel of four rows.  WHOLE: 16 states.
+template <typename T, bool V4, bool WHOLE>
+__global__ void __launch_bounds__(512) k_scan_walk(ScanArgs a) {
+    constexpr int ROWS = 64, LD = ROWS + 4, NB = ROWS / kWalk, CD = kWalk + 4;  // strides of B | C's columns, of a row's channels
+    __shared__ __attribute__((aligned(16))) float sbc[2][2 * kWalk][LD], sdt[2][ROWS][CD], sdx[2][ROWS][CD], sy[2][ROWS][CD];
+    const SeqInfo q = a.seqs[blockIdx.y];
+    // an XCD's workgroups have neighbouring channels, which share the lines of every row
+    const int per = gridDim.x / 8, c0 = ((blockIdx.x % 8) * per + blockIdx.x / 8) * kWalk;
+    const int tid = threadIdx.x & 255, N = a.N, len = q.len, ngr = (len + ROWS - 1) / ROWS;
+    if (c0 >= max(a.C, a.ldy)) return;
+    if (threadIdx.x < 256) {
+        const int lane = tid & 63, j = tid & 15, ch = tid >> 4, c = c0 + ch;
+        const bool mine = c < a.C && j < N;
+        const int cc = min(c, a.C - 1), n = min(j, N - 1);
+        const long at = ((long)q.slot * a.C + cc) * N + n;
+        const float al = bf2f(a.A_log[(long)cc * N + n]), s0 = a.state[at];
+        // dt A in powers of two: exp(dt A) = exp2(dt A log2 e)
+        const float A = j < N ? -expf(al) * 1.4426950408889634f : 0.0f;
+        float S = q.start > 0 && j < N ? s0 : 0.0f;
+        __syncthreads();
+        for (int i = 0; i < ngr; ++i) {
+            const int k = i & 1, nb = min(NB, (len - i * ROWS + kWalk - 1) / kWalk);
+            struct Block { f32x4 B[4], C[4]; float dt, dx; };
+            auto read = [&](int b, Block& o) {
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    o.B[v] = *reinterpret_cast<const f32x4*>(&sbc[k][j][b * kWalk + 4 * v]);
+                    o.C[v] = *reinterpret_cast<const f32x4*>(&sbc[k][kWalk + j][b * kWalk + 4 * v]);
+                }
+                o.dt = sdt[k][b * kWalk + j][ch];  // lane j has row j of the block
+                o.dx = sdx[k][b * kWalk + j][ch];
+            };
+            auto walk = [&](int b, const Block& o) {
+                float e[kWalk], w[kWalk], p[kWalk];
+                each_step([&](auto ti) {  // decays and inputs: none waits for another
+                    constexpr int t = decltype(ti)::value;
+                    e[t] = __builtin_amdgcn_exp2f(of_step<t>(o.dt) * A);
+                    w[t] = of_step<t>(o.dx) * o.B[t / 4][t % 4];
+                }, std::make_integer_sequence<int, kWalk>{});
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int t = 0; t < kWalk; ++t) {
+                    S = fmaf(e[t], S, w[t]);
+                    p[t] = S * o.C[t / 4][t % 4];
+                }
+                sy[k][b * kWalk + j][ch] = sum_of_step(p, lane);
+            };
+            Block o[2];
+            read(0, o[0]);
+            if (nb == NB) {
+#pragma unroll
+                for (int b = 0; b < NB; ++b) {
+                    if (b + 1 < NB) read(b + 1, o[(b + 1) & 1]);
+                    walk(b, o[b & 1]);
+                }
+            } else {
+#pragma clang loop unroll(disable)
+                for (int b = 0; b < nb; ++b) {
+                    if (b) read(b, o[0]);
+                    walk(b, o[0]);
+                }
+            }
+            __syncthreads();
+        }
+        if (mine) a.state[at] = S;
+        return;
+    }
+    typedef T T4 __attribute__((ext_vector_type(4)));
+    const float* __restrict__ dp = a.dt + (long)q.off * a.C;
+    const T* __restrict__ xp = reinterpret_cast<const T*>(a.x) + (long)q.off * a.ldx;
+    const T* __restrict__ zp = reinterpret_cast<const T*>(a.z) + (long)q.off * a.ldz;
+    T* __restrict__ yp = reinterpret_cast<T*>(a.y) + (long)q.off * a.ldy;
+    const float* __restrict__ bc = a.bc + (long)q.off * 2 * N;
+    // element e of a thread: V4: row r0, channel c0 + h0 + e; else row r0 + 16 e, channel c0 + h0
+    const int r0 = V4 ? tid >> 2 : tid >> 4, h0 = V4 ? (tid & 3) * 4 : tid & 15, hc = V4 ? c0 + h0 : min(c0 + h0, a.C - 1);
+    auto row_of = [&](int e) { return V4 ? r0 : r0 + 16 * e; };
+    f32x4 bias, Dc;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        bias[e] = bf2f(a.dtb[V4 ? hc + e : hc]);
+        Dc[e] = bf2f(a.Dw[V4 ? hc + e : hc]);
+    }
+    // B | C: WHOLE: columns 4 (tid % 8) .. of rows tid / 8 and tid / 8 + 32; else column tid % 32 of rows tid / 32 + 8 i
+    const int col = WHOLE ? (tid & 7) * 4 : tid & 31, rb = WHOLE ? tid >> 3 : tid >> 5, cn = col & 15;
+    f32x4 hbc[2], hd;
+    T4 hx, hz;
+    auto hold = [&](int t0) {  // rows past the end repeat the last one (never used)
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+            if constexpr (WHOLE) {
+                hbc[i] = *reinterpret_cast<const f32x4*>(bc + (long)min(t0 + rb + 32 * i, len - 1) * 32 + col);
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    hbc[i][e] = cn < N ? bc[(long)min(t0 + rb + 8 * (4 * i + e), len - 1) * 2 * N + (col < 16 ? cn : N + cn)] : 0.0f;
+            }
+        if constexpr (V4) {
+            const long r = min(t0 + r0, len - 1);
+            hd = *reinterpret_cast<const f32x4*>(dp + r * a.C + hc);
+            hx = *reinterpret_cast<const T4*>(xp + r * a.ldx + hc);
+            hz = *reinterpret_cast<const T4*>(zp + r * a.ldz + hc);
+        } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const long r = min(t0 + row_of(e), len - 1);
+                hd[e] = dp[r * a.C + hc];
+                hx[e] = xp[r * a.ldx + hc];
+                hz[e] = zp[r * a.ldz + hc];
+            }
+        }
+    };
+    struct Gate { f32x4 g, dx; };  // of a row that is being walked: the gate, and what the input adds by itself
+    auto stage = [&](int to, int t0, Gate& gate) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                if constexpr (WHOLE) sbc[to][col + e][rb + 32 * i] = hbc[i][e];
+                else sbc[to][col][rb + 8 * (4 * i + e)] = hbc[i][e];
+        f32x4 dt, dx;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const T xe = hx[e], ze = hz[e];
+            const bool row = t0 + row_of(e) < len;  // no step past the end
+            const float x = ldf(&xe);
+            gate.g[e] = siluf_(ldf(&ze));
+            gate.dx[e] = x;
+            dt[e] = row ? softplus_of<T>(hd[e] + bias[e]) : 0.0f;
+            dx[e] = row ? dt[e] * x : 0.0f;
+        }
+        if constexpr (V4) {
+            *reinterpret_cast<f32x4*>(&sdt[to][r0][h0]) = dt;
+            *reinterpret_cast<f32x4*>(&sdx[to][r0][h0]) = dx;
+        } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                sdt[to][row_of(e)][h0] = dt[e];
+                sdx[to][row_of(e)][h0] = dx[e];
+            }
+        }
+    };
+    auto leave = [&](int from, int t0, const Gate& gate) {
+        T4 o;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const float v = gate.g[e] * fmaf(Dc[e], gate.dx[e], sy[from][row_of(e)][V4 ? h0 + e : h0]);
+            T r;
+            stf(&r, c0 + h0 < a.C ? v : 0.0f);  // columns C .. ldy - 1 are zero
+            o[e] = r;
+        }
+        if constexpr (V4) {
+            if (t0 + r0 < len) *reinterpret_cast<T4*>(yp + (long)(t0 + r0) * a.ldy + hc) = o;
+        } else if (c0 + h0 < a.ldy) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                if (t0 + row_of(e) < len) yp[(long)(t0 + row_of(e)) * a.ldy + c0 + h0] = o[e];
+        }
+    };
+    Gate before, now, next;
+    hold(0);
+    stage(0, 0, now);
+    if (1 < ngr) hold(ROWS);
+    __syncthreads();
+    for (int i = 0; i < ngr; ++i) {
+        if (i > 0) leave(~i & 1, (i - 1) * ROWS, before);
+        if (i + 1 < ngr) {
+            stage(~i & 1, (i + 1) * ROWS, next);
+            if (i + 2 < ngr) hold((i + 2) * ROWS);
+        }
+        before = now;
+        now = next;
+        __syncthreads();
+    }
+    leave(~ngr & 1, (ngr - 1) * ROWS, before);
+}
+
 template <typename T, int NPL, int LPC>
 void launch_scan(hipStream_t s, const ScanArgs& a) {
     const int CPB = 256 / LPC;
@@ -382,7 +607,20 @@ void launch_scan(hipStream_t s, const ScanArgs& a) {
 }
 
 template <typename T>
+void launch_walk(hipStream_t s, const ScanArgs& a) {
+    const dim3 grid(((std::max(a.C, a.ldy) + kWalk - 1) / kWalk + 7) / 8 * 8, a.nseq), blk(512);
+    const uintptr_t at = reinterpret_cast<uintptr_t>(a.dt) | reinterpret_cast<uintptr_t>(a.x) | reinterpret_cast<uintptr_t>(a.z) |
+                         reinterpret_cast<uintptr_t>(a.y);
+    const bool v4 = a.C % kWalk == 0 && a.ldy == a.C && a.ldx % 4 == 0 && a.ldz % 4 == 0 && at % 16 == 0;
+    const bool whole = a.N == 16 && reinterpret_cast<uintptr_t>(a.bc) % 16 == 0;
+    if (v4 && whole) hipLaunchKernelGGL((k_scan_walk<T, true, true>), grid, blk, 0, s, a);
+    else if (v4) hipLaunchKernelGGL((k_scan_walk<T, true, false>), grid, blk, 0, s, a);
+    else hipLaunchKernelGGL((k_scan_walk<T, false, false>), grid, blk, 0, s, a);
+}
+
+template <typename T>
 void scan_t(hipStream_t s, const ScanArgs& a) {
+    if (a.walk) return launch_walk<T>(s, a);
     switch (scan_lanes(a.N)) {
         case 1:
             if (a.N <= 8) launch_scan<T, 8, 1>(s, a);

@@ -52,6 +52,44 @@ inline int scan_run_rows(const int32_t* lens, int n_seq, long columns, long work
     return best;
 }
 
+// A step as the scan sees it: its sequences, and the runs that they would be cut into
+struct ScanStep {
+    int n_seq = 0, longest = 0, run_rows = 0, most_runs = 0;  // most_runs: of one sequence
+    long rows = 0, padded = 0, runs = 0;                      // padded: every sequence's rows in whole blocks of 16
+};
+inline ScanStep scan_step_of(const int32_t* lens, int n_seq, int run_rows) {
+    ScanStep s;
+    s.n_seq = n_seq;
+    s.run_rows = run_rows;
+    for (int r = 0; r < n_seq; ++r) {
+        const int n = (lens[r] + run_rows - 1) / run_rows;
+        s.longest = std::max(s.longest, (int)lens[r]);
+        s.most_runs = std::max(s.most_runs, n);
+        s.rows += lens[r];
+        s.padded += (lens[r] + 15) / 16 * 16;
+        s.runs += n;
+    }
+    return s;
+}
+// Whether a layer walks its sequences with a lane per state (k_scan_walk: every exponential once, one launch) rather than in runs
+// with a lane per channel (k_scan: twice, three launches): by the predicted time, in us.  A walk takes what its longest sequence
+// takes alone, or what the chip takes for all of them (a CU's share of the workgroups, each with its start and its steps); runs take
+// their launches, the rows' traffic, the rounds of rows walked one after the other and the carries.  The constants are fitted to 196
+// steps of 64 to 8,192 channels and 33 to 4,096 rows: the rule loses 0.1 % of the better form on average, 8 % at most.  us a
+// layer, runs / walk: 1,024 + 387 + 129 rows of 4,096 channels 70.0 / 37.1, 512 rows 33.7 / 15.7, 8 x 512 rows 145 / 87, 500 rows of
+// 2,048 fp32 channels 32.3 / 20.6; 4,096 rows of 2,048 channels 83 / 113, 64 x 33 rows of 4,096 50 / 103.
+inline bool scan_walks(const ScanStep& s, int C, int N, bool f32) {
+    if (N <= 8 || N > 16) return false;
+    const double per_cu = (C + 15) / 16 / (double)kRunCUs;
+    const double walk = (f32 ? 5 : 3) + std::max((f32 ? 0.033 : 0.024) * s.longest,
+                                                 per_cu * (0.5 * s.n_seq + (f32 ? 0.029 : 0.023) * (double)s.padded));
+    const double rounds = (double)((s.runs * ((C + 255) / 256) + kRunCUs - 1) / kRunCUs);
+    const double runs = s.most_runs == 1 ? 10 + rounds * s.run_rows * (f32 ? 0.44 : 0.3)
+                                         : (f32 ? 18.9 + 8.5e-6 * C * (double)s.rows : 17.6 + 7.1e-6 * C * (double)s.rows) +
+                                               rounds * (s.run_rows + 8) * (f32 ? 0.21 : 0.048) + 0.093 * s.most_runs;
+    return walk < runs;
+}
+
 // minGRU: the longest runs, down to 8 rows, that still give every CU a workgroup of 128 channels; of one sequence no more than 84,
 // which the carry walks one after the other (us a layer on runs of 32 / 24 / 16 / 8 rows, 64 channels: 300 rows 30 / 28 / 26 / 24, 700
 // rows 32 / 29 / 27 / 28, 2,000 rows 36 / 35 / 35 / 41, 5,000 rows 50 / 51 / 55 / 76)

@@ -59,3 +59,38 @@ def test_gru(ask, C, lens, rows):
 @pytest.mark.parametrize("C,N", [(72, 12), (40, 9), (128, 16)])
 def test_steps_of_many_sequences(ask, C, N, n, length, scan, gru):
     assert ask(C, N, *(length - 7 * (r % 5) for r in range(n))) == [scan, gru]
+
+
+WALKS = r"""
+#include <cstdio>
+#include <cstdlib>
+#include <vector>
+#include "runs.h"
+int main(int n, char** v) {  // channels, states, lengths
+    std::vector<int32_t> lens;
+    for (int i = 3; i < n; ++i) lens.push_back(atoi(v[i]));
+    const int C = atoi(v[1]), N = atoi(v[2]), k = (int)lens.size();
+    const int run = pgmi::scan_run_rows(lens.data(), k, pgmi::scan_columns(C, N), pgmi::scan_workgroups(C, N));
+    const pgmi::ScanStep s = pgmi::scan_step_of(lens.data(), k, run);
+    std::printf("%d %d\n", (int)pgmi::scan_walks(s, C, N, false), (int)pgmi::scan_walks(s, C, N, true));
+}
+"""
+
+
+@pytest.fixture(scope="module")
+def walks(tmp_path_factory):
+    at = tmp_path_factory.mktemp("walks")
+    (at / "ask.cpp").write_text(WALKS)
+    subprocess.run(["g++", "-std=c++17", "-Wall", "-Werror", "-I", CSRC, str(at / "ask.cpp"), "-o", str(at / "ask")], check=True)
+    return lambda *a: [int(x) for x in subprocess.run([str(at / "ask"), *map(str, a)], check=True, capture_output=True,
+                                                      text=True).stdout.split()]
+
+
+# whole sequences with a lane per state (bf16, fp32) where that was the faster form by more than the rule's error
+@pytest.mark.parametrize("C,N,lens,bf16,f32", [
+    (4096, 16, [1024, 387, 129], 1, 1), (4096, 16, [1540], 1, 1), (4096, 16, [512] * 8, 1, 1), (4096, 16, [4096], 1, 1),
+    (2048, 16, [500], 1, 1), (2048, 16, [1000], 1, 1), (2048, 16, [4096], 0, 0), (1024, 16, [3000], 0, 0), (512, 16, [700], 1, 1),
+    (64, 16, [1500], 0, 0), (64, 16, [300], 1, 1), (4096, 16, [33] * 64, 0, 0), (8192, 16, [64] * 32, 0, 0), (1024, 16, [64] * 32, 1, 1),
+    (72, 12, [70, 33, 5], 1, 1), (72, 8, [70, 33, 5], 0, 0), (72, 17, [70, 33, 5], 0, 0), (2048, 64, [500], 0, 0), (64, 9, [1], 1, 1)])
+def test_scan_walks(walks, C, N, lens, bf16, f32):
+    assert walks(C, N, *lens) == [bf16, f32]

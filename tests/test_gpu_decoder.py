@@ -106,6 +106,35 @@ def test_steps_and_scan_of_many_rows(inner, dt_rank, rows, dtype):
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("inner,states", [(16, 16), (48, 9), (64, 12), (72, 16), (40, 13)])
+def test_scan_of_sequences_walked_whole(inner, states, dtype):
+    """Sequences that end just before, on and just after a block of 16 and a stage of 64 rows, of channels that are and are not whole
+    vectors and workgroups, then the next portions from the states that were left."""
+    cfg = C.model([C.mamba(inner, states, 8, 4)], width=64, streams=1, groups=1)
+    eng, W = build(cfg, dtype)
+    first, then = [1, 15, 16, 17, 63, 64, 65, 129, 190], [65, 1, 128, 16, 2, 64, 63, 17, 3]
+    seqs = [tokens(cfg, a + b, 40 + r) for r, (a, b) in enumerate(zip(first, then))]
+    cache = eng.new_cache(len(seqs), 256)
+    slots = [cache.alloc() for _ in seqs]
+    a = eng.forward(cache, slots, [t for s, n in zip(seqs, first) for t in s[:n]], first, want=range(sum(first))).clone()
+    b = eng.forward(cache, slots, [t for s, n in zip(seqs, first) for t in s[n:]], then, want=range(sum(then))).clone()
+    for r, s in enumerate(seqs):
+        i, j = sum(first[:r]), sum(then[:r])
+        close(torch.cat([a[i:i + first[r]], b[j:j + then[r]]]), O.run(cfg, W, s), dtype)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_scan_in_runs_as_walked(dtype):
+    """2,300 rows of few channels go in runs; in portions of 230 they are walked."""
+    cfg = C.model([C.mamba(64, 16, 8, 4)], width=64, streams=1, groups=1)
+    eng, _ = build(cfg, dtype)
+    toks = tokens(cfg, 2300, 9)
+    cache = eng.new_cache(2, 2304)
+    whole = eng.forward(cache, [cache.alloc()], toks, [len(toks)], want=range(len(toks))).clone()
+    close(feed(eng, cache, cache.alloc(), toks, [230]), whole.double().cpu().numpy(), dtype)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("name", list(ALL))
 def test_token_by_token(name, dtype):
     cfg = ALL[name]
