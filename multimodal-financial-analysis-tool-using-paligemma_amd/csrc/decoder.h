@@ -287,6 +287,7 @@ struct WAttnArgs {
     const int* row_seq;  // [rows]
     const ChunkInfo* tiles;
     int ntile;
+    bool teams;  // bf16: two teams of four waves a tile, which take its key tiles in turn (wattn_teams)
 };
 void wattn_append(hipStream_t s, Act act, const WAttnArgs& a);
 constexpr int kWAttnRows = 64;  // (position, query head of the group) pairs per prefill tile: ChunkInfo.rel of `tiles`

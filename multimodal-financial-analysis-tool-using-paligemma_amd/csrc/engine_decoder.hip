@@ -584,6 +584,7 @@ struct Meta {
         bool multi;  // some sequence has more than one
     } scan, gru, conv;
     ScanStep step;
+    const int32_t *starts, *lens;  // on the host
     bool fresh;  // every sequence from its start
     const int* row_seq;
     const int* want;
@@ -663,6 +664,7 @@ int forward_body(pgmi_ctx* x, hipStream_t s, const int64_t* ids, int rows, const
             a.max_tokens = max_tokens; a.o = d.p2; a.rows = rows; a.seqs = m.seqs; a.nseq = m.nseq; a.row_seq = m.row_seq;
             const auto& t = m.tiles.at(l.heads / l.kv_heads);
             a.tiles = t.first; a.ntile = t.second;
+            a.teams = wattn_teams(m.starts, m.lens, m.nseq, l.heads, l.kv_heads, l.window, l.keep_first);
             wattn_append(s, d.act, a);
             wattn_prefill(s, d.act, a);
             out_proj(w.o, d.p2, a.ldo, w.sub[0]);
@@ -1141,6 +1143,8 @@ int pgmi_decoder_forward(pgmi_ctx* x, const int64_t* ids, int n_seq, const int32
     meta.fresh = std::all_of(starts, starts + n_seq, [](int32_t p) { return p == 0; });
     meta.scan = {reinterpret_cast<const ChunkInfo*>(dm + scan.o), scan.n, scan.multi};
     meta.step = step;
+    meta.starts = starts;
+    meta.lens = lens;
     meta.gru = {reinterpret_cast<const ChunkInfo*>(dm + gru.o), gru.n, gru.multi};
     meta.conv = {reinterpret_cast<const ChunkInfo*>(dm + conv.o), conv.n, conv.multi};
     meta.row_seq = dm + o_row;

@@ -411,20 +411,28 @@ void run_f(hipStream_t s, const WAttnArgs& a) {
 // two 16-key tiles, exactly the 8 weights its B fragment of O^T = V^T P^T needs (the contraction order is free:
 // slot 8g + i is key 4g + i of the first tile for i < 4, of the second for i >= 4).  V^T fragments are
 // transposed LDS reads of the row-major V tile.
-template <int DQ, int DV, int SC>
-__global__ void __launch_bounds__(256) k_wattn_m(WAttnArgs a) {
+// Bound, where the chip is full, by LDS (a tile's K and V are read by each of its four waves, 128 KB, and V in halves) and by the
+// score's vector operations; where it is not, by the longest tile's chain of barriers, LDS reads, two products and what is between
+// them, which two teams halve (wattn_teams).  us, 1,300 + 511 + 235 + 2 rows of 16 heads of 128, capped scores: 51.3 before; sums in
+// VGPRs, loads and masks without a branch each 46.2; two teams 39.6.  32 rows a wave, which halves the LDS reads, beat this only for
+// one sequence of 4,096 rows (64 against 77) and lost 20 to 40 % below 1,000.
+constexpr size_t wattn_m_lds(int DQ, int DV, int teams) { return (size_t)teams * 64 * (DQ + 8 + DV + 8) * 2; }
+template <int DQ, int DV, int SC, int TEAMS, bool PAD>
+__global__ void __launch_bounds__(256 * TEAMS) k_wattn_m(WAttnArgs a) {
     const WAttnHeads& w = a.hd;
     constexpr int KT = 64;                 // keys per tile
     constexpr int KS = DQ + 8, VS = DV + 8;  // LDS row strides (elements)
     constexpr int KQ = KT * DQ / 8 / 256, VQ = KT * DV / 8 / 256;  // 16-byte pieces per thread
-    __shared__ __attribute__((aligned(16))) uint16_t Ks[KT * KS];
-    __shared__ __attribute__((aligned(16))) uint16_t Vs[KT * VS];
+    extern __shared__ __attribute__((aligned(16))) uint8_t smem_wattn[];
+    const int team = TEAMS == 1 ? 0 : __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 8);
+    uint16_t* Ks = reinterpret_cast<uint16_t*>(smem_wattn + (size_t)team * wattn_m_lds(DQ, DV, 1));
+    uint16_t* Vs = Ks + KT * KS;
     const int g = blockIdx.y, R = w.H / w.G;
     // later positions see more keys: every other key/value head backwards, so that a CU's two workgroups are not both long
     // (2,048 rows in sequences up to 1,300: 53.0 us, so 47.3)
     const ChunkInfo tl = a.tiles[g & 1 ? a.ntile - 1 - (int)blockIdx.x : blockIdx.x];
     const SeqInfo sq = a.seqs[tl.seq];
-    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int tid = threadIdx.x & 255, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int li = lane & 15, lg = lane >> 4;
     const int nrow = sq.len * R;
     // this lane's query row
@@ -433,13 +441,16 @@ __global__ void __launch_bounds__(256) k_wattn_m(WAttnArgs a) {
     const int frc = ok ? fr : nrow - 1;
     const int prow = frc / R, hh = frc % R, h = g * R + hh;
     const int i = sq.start + prow;
+    auto ld = [](const uint16_t* p, bool in, const uint16_t* safe) {  // (the choice is a branch around every load)
+        if constexpr (PAD) return ldg16_sel(p, in, safe);
+        else return ldg16(p);
+    };
     const uint16_t* qp = reinterpret_cast<const uint16_t*>(a.q) + ((long)(sq.off + prow) * w.H + h) * w.dp;
     short8 qf[DQ / 32];
 #pragma unroll
     for (int c = 0; c < DQ / 32; ++c) {
         const int k = c * 32 + 8 * lg;
-        const uint4 v = ldg16_sel(qp + k, k < w.dp, qp);
-        qf[c] = __builtin_bit_cast(short8, v);
+        qf[c] = __builtin_bit_cast(short8, ld(qp + k, k < w.dp, qp));
     }
     const Score<SC> score(a.sc, h);
     const float r1 = score.r1, r2 = score.r2, c1 = score.c1;
@@ -463,20 +474,21 @@ __global__ void __launch_bounds__(256) k_wattn_m(WAttnArgs a) {
         for (int x = 0; x < KQ; ++x) {
             const int e = tid + 256 * x, r = e / (DQ / 8), k = (e % (DQ / 8)) * 8;
             const int j = min(j0 + r, hi);
-            kr[x] = ldg16_sel(kc + (long)j * w.dp + k, k < w.dp, kc);
+            kr[x] = ld(kc + (long)j * w.dp + k, k < w.dp, kc);
         }
 #pragma unroll
         for (int x = 0; x < VQ; ++x) {
             const int e = tid + 256 * x, r = e / (DV / 8), k = (e % (DV / 8)) * 8;
             const int j = min(j0 + r, hi);
-            vr[x] = ldg16_sel(vc + (long)j * w.ep + k, k < w.ep, vc);
+            vr[x] = ld(vc + (long)j * w.ep + k, k < w.ep, vc);
         }
     };
-    auto next = [&](int j0) { return j0 < kept && j0 + KT >= kept ? lo : j0 + KT; };  // kept keys end before lo
-    const int first = kept > 0 ? 0 : lo;
-    gload(first);
-    for (int j0 = first, jn; j0 <= hi; j0 = jn) {
-        jn = next(j0);
+    // tile t: the kept keys' first, then the window's; a team takes every TEAMS-th
+    const int nh = (kept + KT - 1) / KT, nt = nh + (hi - lo) / KT + 1;
+    auto key0 = [&](int t) { return t < nh ? KT * t : lo + KT * (t - nh); };
+    if (team < nt) gload(key0(team));
+    for (int t0 = 0; t0 < nt; t0 += TEAMS) {
+        const int t = t0 + team, j0 = key0(t);
         __syncthreads();  // the previous tile's reads are done
 #pragma unroll
         for (int x = 0; x < KQ; ++x) {
@@ -489,19 +501,20 @@ __global__ void __launch_bounds__(256) k_wattn_m(WAttnArgs a) {
             *reinterpret_cast<uint4*>(Vs + r * VS + k) = vr[x];
         }
         __syncthreads();
-        if (jn <= hi) gload(jn);
-        if (j0 > wlast || (j0 + KT <= wfirst - window + 1 && j0 >= keep)) continue;  // no row of this wave sees the tile
+        if (t + TEAMS < nt) gload(key0(t + TEAMS));
+        if (t >= nt || j0 > wlast || (j0 + KT <= wfirst - window + 1 && j0 >= keep)) continue;  // no row of this wave sees the tile
         f32x4 st[4];
 #pragma unroll
-        for (int t = 0; t < 4; ++t) {
-            st[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int n = 0; n < 4; ++n) {
+            st[n] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int c = 0; c < DQ / 32; ++c) {
-                const short8 kf = *reinterpret_cast<const short8*>(Ks + (t * 16 + li) * KS + c * 32 + 8 * lg);
-                st[t] = mfma16(kf, qf[c], st[t]);
+                const short8 kf = *reinterpret_cast<const short8*>(Ks + (n * 16 + li) * KS + c * 32 + 8 * lg);
+                st[n] = mfma16(kf, qf[c], st[n]);
             }
         }
-        const bool head = j0 < kept;  // kept keys: every row sees those before lo
+        const bool head = t < nh;  // kept keys: every row sees those before lo
+        const int end = head ? kept : i + 1;
         float mt = m;
         // 1 + r2 (i - j) for key j0 + 4 lg, less r2 per key after it
         const float x0 = fmaf(r2, (float)(i - j0 - 4 * lg), 1.0f);
@@ -511,26 +524,26 @@ __global__ void __launch_bounds__(256) k_wattn_m(WAttnArgs a) {
         };
         if (head ? j0 + KT <= kept : j0 + KT - 1 <= wfirst && (wlast - j0 < window || j0 + KT <= keep)) {  // no mask
 #pragma unroll
-            for (int t = 0; t < 4; ++t)
+            for (int n = 0; n < 4; ++n)
 #pragma unroll
-                for (int r = 0; r < 4; ++r) st[t][r] = value(st[t][r], t * 16 + r);
+                for (int r = 0; r < 4; ++r) st[n][r] = value(st[n][r], n * 16 + r);
         } else {
 #pragma unroll
-            for (int t = 0; t < 4; ++t)
+            for (int n = 0; n < 4; ++n)
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
-                    const int j = j0 + t * 16 + 4 * lg + r, dist = i - j;
-                    const bool see = head ? j < kept : dist >= 0 && (dist < window || j < keep);
-                    const float s = value(st[t][r], t * 16 + r);
-                    st[t][r] = see ? s : -INFINITY;
+                    const int j = j0 + n * 16 + 4 * lg + r;
+                    const bool see = (j < end) & ((i - j < window) | (j < keep));  // (as && and || branches between the keys)
+                    const float s = value(st[n][r], n * 16 + r);
+                    st[n][r] = see ? s : -INFINITY;
                 }
         }
         float alpha = 1.0f;
         if constexpr (SC != SC_CAPPED) {
 #pragma unroll
-            for (int t = 0; t < 4; ++t)
+            for (int n = 0; n < 4; ++n)
 #pragma unroll
-                for (int r = 0; r < 4; ++r) mt = fmaxf(mt, st[t][r]);
+                for (int r = 0; r < 4; ++r) mt = fmaxf(mt, st[n][r]);
             mt = fmaxf(mt, __shfl_xor(mt, 16, 64));
             mt = fmaxf(mt, __shfl_xor(mt, 32, 64));
             alpha = __builtin_amdgcn_exp2f(m - mt);
@@ -538,11 +551,11 @@ __global__ void __launch_bounds__(256) k_wattn_m(WAttnArgs a) {
         }
         float ls = 0.0f;
 #pragma unroll
-        for (int t = 0; t < 4; ++t)
+        for (int n = 0; n < 4; ++n)
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                st[t][r] = __builtin_amdgcn_exp2f(SC == SC_CAPPED ? st[t][r] : st[t][r] - m);
-                ls += st[t][r];
+                st[n][r] = __builtin_amdgcn_exp2f(SC == SC_CAPPED ? st[n][r] : st[n][r] - m);
+                ls += st[n][r];
             }
         l = l * alpha + ls;  // this lane's keys; summed over the lane groups at the end
         if (SC != SC_CAPPED && __any(alpha != 1.0f)) {
@@ -569,6 +582,28 @@ __global__ void __launch_bounds__(256) k_wattn_m(WAttnArgs a) {
             }
         }
     }
+    if constexpr (TEAMS == 2) {  // the other team's sums, in its lanes' places
+        f32x4* at = reinterpret_cast<f32x4*>(smem_wattn) + tid;
+        float* ml = reinterpret_cast<float*>(at + (DV / 16) * 256 - tid) + tid;
+        __syncthreads();  // the last tiles' reads are done
+        if (team) {
+#pragma unroll
+            for (int c = 0; c < DV / 16; ++c) at[c * 256] = o[c];
+            ml[0] = m;
+            ml[256] = l;
+        }
+        __syncthreads();
+        if (team) return;
+        const float m2 = ml[0], mt = fmaxf(m, m2);
+        const float f1 = SC == SC_CAPPED ? 1.0f : __builtin_amdgcn_exp2f(m - mt), f2 = SC == SC_CAPPED ? 1.0f : __builtin_amdgcn_exp2f(m2 - mt);
+        l = l * f1 + ml[256] * f2;
+#pragma unroll
+        for (int c = 0; c < DV / 16; ++c) {
+            const f32x4 o2 = at[c * 256];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) o[c][r] = o[c][r] * f1 + o2[r] * f2;
+        }
+    }
     l += __shfl_xor(l, 16, 64);
     l += __shfl_xor(l, 32, 64);
     if (!ok) return;
@@ -588,13 +623,29 @@ __global__ void __launch_bounds__(256) k_wattn_m(WAttnArgs a) {
 // the score mode of a layer on the hardware's transcendentals
 int score_mode(const WAttnScore& sc) { return sc.r1 ? SC_BIAS : sc.cap > 0.0f && sc.cap <= kCapFixed ? SC_CAPPED : SC_PLAIN; }
 
+template <int DQ, int DV, int SC, int TEAMS, bool PAD>
+void run_mt(hipStream_t s, const WAttnArgs& a) {
+    constexpr size_t lds = wattn_m_lds(DQ, DV, TEAMS);
+    static_assert(TEAMS == 1 || (size_t)256 * (DV + 8) <= lds, "the other team's sums fit");
+    static const bool once = [] {
+        return hipFuncSetAttribute(reinterpret_cast<const void*>(&k_wattn_m<DQ, DV, SC, TEAMS, PAD>),
+                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) == hipSuccess;
+    }();
+    (void)once;
+    hipLaunchKernelGGL((k_wattn_m<DQ, DV, SC, TEAMS, PAD>), dim3(a.ntile, a.hd.G), dim3(256 * TEAMS), lds, s, a);
+}
+template <int DQ, int DV, int SC>
+void run_ms(hipStream_t s, const WAttnArgs& a) {
+    const bool pad = a.hd.dp != DQ || a.hd.ep != DV;
+    if (a.teams) pad ? run_mt<DQ, DV, SC, 2, true>(s, a) : run_mt<DQ, DV, SC, 2, false>(s, a);
+    else pad ? run_mt<DQ, DV, SC, 1, true>(s, a) : run_mt<DQ, DV, SC, 1, false>(s, a);
+}
 template <int DQ, int DV>
 void run_m(hipStream_t s, const WAttnArgs& a) {
-    const dim3 grid(a.ntile, a.hd.G);
     const int mode = score_mode(a.sc);
-    if (mode == SC_BIAS) hipLaunchKernelGGL((k_wattn_m<DQ, DV, SC_BIAS>), grid, dim3(256), 0, s, a);
-    else if (mode == SC_CAPPED) hipLaunchKernelGGL((k_wattn_m<DQ, DV, SC_CAPPED>), grid, dim3(256), 0, s, a);
-    else hipLaunchKernelGGL((k_wattn_m<DQ, DV, SC_PLAIN>), grid, dim3(256), 0, s, a);
+    if (mode == SC_BIAS) run_ms<DQ, DV, SC_BIAS>(s, a);
+    else if (mode == SC_CAPPED) run_ms<DQ, DV, SC_CAPPED>(s, a);
+    else run_ms<DQ, DV, SC_PLAIN>(s, a);
 }
 template <int DQ>
 void run_mv(hipStream_t s, const WAttnArgs& a) {

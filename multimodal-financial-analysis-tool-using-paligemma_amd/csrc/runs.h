@@ -1,4 +1,5 @@
-// runs.h -- how many rows of a sequence one workgroup of a recurrence walks (host code, without HIP).
+// runs.h -- how many rows of a sequence one workgroup of a recurrence walks, and who walks an attention's keys (host code, without
+// HIP).
 //
 // A short step's few runs are walked by a few CUs, each row waiting for the one before; where the chip is full short runs only
 // add carries.
@@ -102,6 +103,23 @@ inline int gru_run_rows(const int32_t* lens, int n_seq, long columns) {
         ct = k;
     }
     return ct;
+}
+
+// Whether a prompt's attention gives each tile of 64 (position, head) pairs to two teams of four waves, which take its 64-key tiles in
+// turn, rather than to one: where the longest tile's chain is what the step waits for, and not the sum of all tiles over the chip (the
+// second team's sums cost LDS and a merge).  us, one team / two, 16 heads of 128 in 2 groups, window 1,024: 1,300 + 511 + 235 + 2 rows
+// 46.2 / 39.6, 1,024 + 387 + 129 rows with distance bias 34.4 / 31.5, 1,300 rows 33.4 / 25.7, 1,540 rows 35.5 / 32.9, 500 rows of 8
+// heads 18.2 / 15.8; 2 x 1,024 rows 35.0 / 39.6, 2,048 rows 45.8 / 48.5, 8 x 512 rows 44.4 / 47.1, 32 x 64 rows 12.5 / 16.1.
+inline bool wattn_teams(const int32_t* starts, const int32_t* lens, int n_seq, int heads, int groups, int window, int keep) {
+    const double most = (double)window + keep, R = heads / groups;
+    auto keys = [&](double n) { return n <= most ? n * (n + 1) / 2 : most * (most + 1) / 2 + (n - most) * most; };  // of positions 0 .. n - 1
+    double work = 0, longest = 0;  // 64-key tiles
+    for (int r = 0; r < n_seq; ++r) {
+        const double end = (double)starts[r] + lens[r];
+        work += groups * R * ((keys(end) - keys(starts[r])) / 4096 + 0.5 * lens[r] / 64);
+        longest = std::max(longest, std::min(end, most) / 64);
+    }
+    return longest > 2 && longest * kRunCUs >= work;
 }
 
 }  // namespace pgmi

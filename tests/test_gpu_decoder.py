@@ -145,6 +145,24 @@ def test_token_by_token(name, dtype):
     close(got, O.run(cfg, W, toks), dtype)
 
 
+@pytest.mark.parametrize("heads,kv,dim,vdim,window", [(8, 2, 64, 64, 900), (6, 3, 24, 36, 150), (4, 1, 128, 128, 192),
+                                                      (2, 1, 256, 256, 700), (4, 2, 96, 128, 129), (3, 3, 40, 200, 300)])
+@pytest.mark.parametrize("lens", [[129], [192, 1], [257, 64, 130], [321]])
+def test_attention_of_two_teams(heads, kv, dim, vdim, window, lens):
+    """Tiles of an odd and an even number of key tiles, a team without one, windows that leave keys behind, padded and whole heads;
+    then portions over the keys that are there."""
+    cfg = C.model([C.attn(heads, kv, dim, vdim, window)], width=72, streams=1, groups=1)
+    eng, W = build(cfg, "bfloat16")
+    seqs = [tokens(cfg, n + 200, 60 + r) for r, n in enumerate(lens)]
+    cache = eng.new_cache(len(lens), 640)
+    slots = [cache.alloc() for _ in lens]
+    a = eng.forward(cache, slots, [t for s, n in zip(seqs, lens) for t in s[:n]], lens, want=range(sum(lens))).clone()
+    b = eng.forward(cache, slots, [t for s, n in zip(seqs, lens) for t in s[n:]], [200] * len(lens), want=range(200 * len(lens))).clone()
+    for r, (s, n) in enumerate(zip(seqs, lens)):
+        i = sum(lens[:r])
+        close(torch.cat([a[i:i + n], b[200 * r:200 * (r + 1)]]), O.run(cfg, W, s), "bfloat16")
+
+
 @pytest.mark.parametrize("heads,kv,dim,vdim,window", [(8, 2, 64, 64, 900), (6, 2, 40, 256, 1500), (16, 4, 32, 128, 1990),
                                                       (128, 1, 16, 8, 300), (4, 4, 24, 128, 2500)])
 def test_one_row_merges_its_attention(heads, kv, dim, vdim, window):
