@@ -73,6 +73,13 @@ __device__ __forceinline__ uint4 ldg16(const void* p) {
     return *reinterpret_cast<const uint4*>(p);
 }
 
+// The same as one vector for fragments that are carried around a loop: hipcc reads a uint4 as four words, joins them again, and has
+// then lost three of them to another register's use (few-row experts' weights, ROCm 7.2; its IR was right, its assembly not)
+__device__ __forceinline__ uint4 ldv16(const void* p) {
+    const u32x4 v = *reinterpret_cast<const u32x4*>(p);
+    return make_uint4(v.x, v.y, v.z, v.w);
+}
+
 // 16-B load whose lane may be out of range: the load is ALWAYS issued (from `safe` when !ok) and
 // the value zeroed afterwards -- a conditional load (ok ? load : 0) makes hipcc branch around the
 // load and wait vmcnt(0) for it, one dependent round trip per element (cdna_hip_programming.md

@@ -443,7 +443,7 @@ __global__ void __launch_bounds__(256 * TEAMS) k_wattn_m(WAttnArgs a) {
     const int i = sq.start + prow;
     auto ld = [](const uint16_t* p, bool in, const uint16_t* safe) {  // (the choice is a branch around every load)
         if constexpr (PAD) return ldg16_sel(p, in, safe);
-        else return ldg16(p);
+        else return ldv16(p);
     };
     const uint16_t* qp = reinterpret_cast<const uint16_t*>(a.q) + ((long)(sq.off + prow) * w.H + h) * w.dp;
     short8 qf[DQ / 32];
@@ -823,9 +823,18 @@ __global__ void __launch_bounds__(256) k_wattn_d(WAttnDecodeArgs a) {
 // tiles: S^T = K Q^T with the key fragments straight from the cache, then O^T += V^T P^T as k_wattn_m, the values
 // through the wave's own LDS rows; the four waves' running sums meet in LDS.
 // VEC: head sizes that are multiples of 8 (up to 64 four waves to a SIMD: 136 registers and three, 16 sequences of 8 heads 143 us for 129).
-template <int DQ, int DV, int SC, bool VEC>
-__global__ void __launch_bounds__(256, DQ <= 64 && DV <= 64 && VEC ? 4 : 1) k_wattn_dm(WAttnDecodeArgs a) {
+// how a head lies: of odd sizes; of whole vectors, padded to DQ and DV; DQ and DV themselves (15.1 KB of code for those, 12.4 where
+// nothing is chosen: one row over 1,000 keys 9.1 -> 7.2 us, 8 rows over up to 1,411 10.0 -> 8.5)
+enum { ODD, VECTORS, WHOLE };
+template <int DQ, int DV, int SC, int HEADS>
+__global__ void __launch_bounds__(256, DQ <= 64 && DV <= 64 && HEADS != ODD ? 4 : 1) k_wattn_dm(WAttnDecodeArgs a) {
     const WAttnHeads& w = a.hd;
+    constexpr bool VEC = HEADS != ODD, FULL = HEADS == WHOLE;
+    const int dp = FULL ? DQ : w.dp, ep = FULL ? DV : w.ep, qd = FULL ? DQ : w.d, ve = FULL ? DV : w.e;
+    auto ld = [](const uint16_t* p, bool in, const uint16_t* safe) {  // (the choice is a branch around every load)
+        if constexpr (FULL) return ldv16(p);
+        else return ldg16_sel(p, in, safe);
+    };
     constexpr int VS = DV + 8;
     __shared__ __attribute__((aligned(16))) uint16_t Vs[4][32 * VS];
     __shared__ float sml[4][16][2];
@@ -837,17 +846,17 @@ __global__ void __launch_bounds__(256, DQ <= 64 && DV <= 64 && VEC ? 4 : 1) k_wa
     const int per = ((keys.n + a.nsplit - 1) / a.nsplit + 127) / 128 * 128;
     const int k0 = sp * per, k1 = min(keys.n, k0 + per);
     const uint16_t* qkv = reinterpret_cast<const uint16_t*>(a.qkv) + (long)b * a.ldqkv;
-    const int r0 = hb * 16, nr = min(16, R - r0), rs = w.ep + 2;
+    const int r0 = hb * 16, nr = min(16, R - r0), rs = ep + 2;
     float* part = a.part + (((long)b * w.H + g * R + r0) * a.nsplit + sp) * rs;
     if (k0 >= k1) {
         if (tid < nr) {
-            part[(long)tid * a.nsplit * rs + w.ep] = kNone;
-            part[(long)tid * a.nsplit * rs + w.ep + 1] = 0.0f;
+            part[(long)tid * a.nsplit * rs + ep] = kNone;
+            part[(long)tid * a.nsplit * rs + ep + 1] = 0.0f;
         }
         return;
     }
-    uint16_t* kc = reinterpret_cast<uint16_t*>(a.kc) + ((long)slot * w.G + g) * a.max_tokens * w.dp;
-    uint16_t* vc = reinterpret_cast<uint16_t*>(a.vc) + ((long)slot * w.G + g) * a.max_tokens * w.ep;
+    uint16_t* kc = reinterpret_cast<uint16_t*>(a.kc) + ((long)slot * w.G + g) * a.max_tokens * dp;
+    uint16_t* vc = reinterpret_cast<uint16_t*>(a.vc) + ((long)slot * w.G + g) * a.max_tokens * ep;
     // A new key (position i) never passes through the cache here: its score and value come from its qkv row, in
     // wave 0 of the last split, which also writes its cache rows.  Cached keys end at kend.
     const bool own = w.own_kv && k1 == keys.n;
@@ -859,14 +868,14 @@ __global__ void __launch_bounds__(256, DQ <= 64 && DV <= 64 && VEC ? 4 : 1) k_wa
         const int jm = max(kend - 1, 0);
 #pragma unroll
         for (int t = 0; t < 2; ++t) {
-            const uint16_t* p = kc + (long)keys.at(min(j0 + t * 16 + li, jm)) * w.dp;
+            const uint16_t* p = kc + (long)keys.at(min(j0 + t * 16 + li, jm)) * dp;
 #pragma unroll
-            for (int c = 0; c < DQ / 32; ++c) kr[t][c] = ldg16_sel(p + c * 32 + 8 * lg, c * 32 + 8 * lg < w.dp, p);
+            for (int c = 0; c < DQ / 32; ++c) kr[t][c] = ld(p + c * 32 + 8 * lg, c * 32 + 8 * lg < dp, p);
         }
 #pragma unroll
         for (int x = 0; x < DV / 16; ++x) {
             const int e = lane + 64 * x, r = e / (DV / 8), k = (e % (DV / 8)) * 8;
-            vr[x] = ldg16_sel(vc + (long)keys.at(min(j0 + r, jm)) * w.ep + k, k < w.ep, vc);
+            vr[x] = ld(vc + (long)keys.at(min(j0 + r, jm)) * ep + k, k < ep, vc);
         }
     };
     if (k0 + wave * 32 < kend) gload(k0 + wave * 32);
@@ -886,22 +895,22 @@ __global__ void __launch_bounds__(256, DQ <= 64 && DV <= 64 && VEC ? 4 : 1) k_wa
             }
         }
     };
-    raw(qkv + h * w.d, w.d, qr);
+    raw(qkv + h * qd, qd, qr);
     // (by the one wave that uses them: every wave asked for them and cut their pads, 40 sequences of 16 heads of 80 53 us a layer, so 49)
     const bool mine = own && wave == 0;
-    const uint16_t* vn = qkv + (w.H + w.G) * w.d + g * w.e;
+    const uint16_t* vn = qkv + (w.H + w.G) * qd + g * ve;
     if (mine) {
-        raw(qkv + w.H * w.d + g * w.d, w.d, knr);
+        raw(qkv + w.H * qd + g * qd, qd, knr);
 #pragma unroll
         for (int c = 0; c < DV / 16; ++c) {
             const int k = c * 16 + 4 * lg;
             if constexpr (VEC) {
-                ld4(vn + (k < w.e ? k : 0), vnr[c]);
+                ld4(vn + (k < ve ? k : 0), vnr[c]);
 #pragma unroll
-                for (int r = 0; r < 4; ++r) vnr[c][r] = k < w.e ? vnr[c][r] : 0.0f;
+                for (int r = 0; r < 4; ++r) vnr[c][r] = k < ve ? vnr[c][r] : 0.0f;
             } else {
 #pragma unroll
-                for (int r = 0; r < 4; ++r) vnr[c][r] = k + r < w.e ? bf2f(vn[k + r]) : 0.0f;
+                for (int r = 0; r < 4; ++r) vnr[c][r] = k + r < ve ? bf2f(vn[k + r]) : 0.0f;
             }
         }
     }
@@ -924,7 +933,7 @@ __global__ void __launch_bounds__(256, DQ <= 64 && DV <= 64 && VEC ? 4 : 1) k_wa
                 for (int v = 0; v < 8; ++v) ss = fmaf(q[c][v], q[c][v], ss);
             ss += __shfl_xor(ss, 16, 64);
             ss += __shfl_xor(ss, 32, 64);
-            inv = 1.0f / sqrtf(ss / (float)w.d + w.eps);
+            inv = 1.0f / sqrtf(ss / (float)qd + w.eps);
         }
 #pragma unroll
         for (int c = 0; c < DQ / 32; ++c) {
@@ -978,7 +987,7 @@ __global__ void __launch_bounds__(256, DQ <= 64 && DV <= 64 && VEC ? 4 : 1) k_wa
         if (w.v_norm) {
             vss += __shfl_xor(vss, 16, 64);
             vss += __shfl_xor(vss, 32, 64);
-            vinv = 1.0f / sqrtf(vss / (float)w.e + w.eps);
+            vinv = 1.0f / sqrtf(vss / (float)ve + w.eps);
         }
 #pragma unroll
         for (int c = 0; c < DV / 16; ++c)
@@ -987,9 +996,9 @@ __global__ void __launch_bounds__(256, DQ <= 64 && DV <= 64 && VEC ? 4 : 1) k_wa
         if (li == 0) {
 #pragma unroll
             for (int c = 0; c < DQ / 32; ++c)
-                if (c * 32 + 8 * lg < w.dp) *reinterpret_cast<short8*>(kc + (long)i * w.dp + c * 32 + 8 * lg) = kf[c];
+                if (c * 32 + 8 * lg < dp) *reinterpret_cast<short8*>(kc + (long)i * dp + c * 32 + 8 * lg) = kf[c];
         }
-        for (int k = lane; k < w.ep; k += 64) vc[(long)i * w.ep + k] = k < w.e ? f2bf(bf2f(vn[k]) * vinv) : 0;
+        for (int k = lane; k < ep; k += 64) vc[(long)i * ep + k] = k < ve ? f2bf(bf2f(vn[k]) * vinv) : 0;
     }
     for (int j0 = k0 + wave * 32; j0 < kend; j0 += 128) {
         f32x4 st[2];
@@ -1063,8 +1072,8 @@ __global__ void __launch_bounds__(256, DQ <= 64 && DV <= 64 && VEC ? 4 : 1) k_wa
         *reinterpret_cast<float4*>(os + (wave * 16 + li) * OS + c * 16 + 4 * lg) =
             make_float4(o[c][0] * f, o[c][1] * f, o[c][2] * f, o[c][3] * f);
     __syncthreads();
-    for (int e = tid; e < nr * w.ep; e += 256) {
-        const int r = e / w.ep, c = e % w.ep;
+    for (int e = tid; e < nr * ep; e += 256) {
+        const int r = e / ep, c = e % ep;
         float t = 0.0f;
 #pragma unroll
         for (int w = 0; w < 4; ++w) t += os[(w * 16 + r) * OS + c];
@@ -1076,8 +1085,8 @@ __global__ void __launch_bounds__(256, DQ <= 64 && DV <= 64 && VEC ? 4 : 1) k_wa
         for (int w = 0; w < 4; ++w) mm = fmaxf(mm, sml[w][tid][0]);
 #pragma unroll
         for (int w = 0; w < 4; ++w) ll += sml[w][tid][1] * __builtin_amdgcn_exp2f(sml[w][tid][0] - mm);
-        part[(long)tid * a.nsplit * rs + w.ep] = mm;
-        part[(long)tid * a.nsplit * rs + w.ep + 1] = ll;
+        part[(long)tid * a.nsplit * rs + ep] = mm;
+        part[(long)tid * a.nsplit * rs + ep + 1] = ll;
     }
 }
 
@@ -1124,14 +1133,15 @@ void run_dm(hipStream_t s, const WAttnDecodeArgs& a) {
     const WAttnHeads& w = a.hd;
     const dim3 grid(a.nsplit, w.G * ((w.H / w.G + 15) / 16), a.B);
     const int mode = score_mode(a.sc);
-    auto go = [&](auto vec) {
-        constexpr bool VEC = decltype(vec)::value;
-        if (mode == SC_BIAS) hipLaunchKernelGGL((k_wattn_dm<DQ, DV, SC_BIAS, VEC>), grid, dim3(256), 0, s, a);
-        else if (mode == SC_CAPPED) hipLaunchKernelGGL((k_wattn_dm<DQ, DV, SC_CAPPED, VEC>), grid, dim3(256), 0, s, a);
-        else hipLaunchKernelGGL((k_wattn_dm<DQ, DV, SC_PLAIN, VEC>), grid, dim3(256), 0, s, a);
+    auto go = [&](auto heads) {
+        constexpr int HEADS = decltype(heads)::value;
+        if (mode == SC_BIAS) hipLaunchKernelGGL((k_wattn_dm<DQ, DV, SC_BIAS, HEADS>), grid, dim3(256), 0, s, a);
+        else if (mode == SC_CAPPED) hipLaunchKernelGGL((k_wattn_dm<DQ, DV, SC_CAPPED, HEADS>), grid, dim3(256), 0, s, a);
+        else hipLaunchKernelGGL((k_wattn_dm<DQ, DV, SC_PLAIN, HEADS>), grid, dim3(256), 0, s, a);
     };
-    if (w.d % 8 == 0 && w.e % 8 == 0) go(std::true_type{});
-    else go(std::false_type{});
+    if (w.d == DQ && w.e == DV) go(std::integral_constant<int, WHOLE>{});
+    else if (w.d % 8 == 0 && w.e % 8 == 0) go(std::integral_constant<int, VECTORS>{});
+    else go(std::integral_constant<int, ODD>{});
     if (!a.parts_only) hipLaunchKernelGGL((k_wattn_dc<uint16_t>), dim3(w.H, a.B), dim3(256), 0, s, a);
 }
 template <int DQ>
