@@ -82,6 +82,26 @@ def test_unequal_batch_then_decoding(lens, dtype):
         close(lg, np.stack([want[r][lens[r] + t] for r in live]), dtype)
 
 
+@pytest.mark.parametrize("width,ff,shared,dim", [(1024, 512, 1024, 64), (2048, 1024, 512, 128), (1024, 1024, 1536, 256),
+                                                 (2048, 256, 2048, 128)])
+@pytest.mark.parametrize("rows", [1, 2, 7, 16])
+def test_steps_of_whole_turns(width, ff, shared, dim, rows):
+    """Few-row expert products whose K is whole turns of 1, 2, 4 or 8 steps of the waves (or, for one of the two, is not), and heads
+    that fill their width, of one row and of several."""
+    cfg = C.model([C.layer(4, 2, dim, dim, 90, keep=3, rot=32, mlp=C.moe(5, ff, 2, shared, identity=1, groups=(2, 1))),
+                   C.layer(4, 2, dim, dim, 20, rot=32, kv_from=0)], width=width, vocab=101)
+    eng, W = build(cfg, "bfloat16")
+    lens = [3 + 9 * r for r in range(rows)]
+    seqs = [tokens(cfg, n + 3, 80 + r) for r, n in enumerate(lens)]
+    cache = eng.new_cache(rows, 160)
+    slots = [cache.alloc() for _ in lens]
+    eng.forward(cache, slots, [t for s, n in zip(seqs, lens) for t in s[:n]], lens)
+    want = [R.run(cfg, W, s) for s in seqs]
+    for t in range(3):
+        lg = eng.step(cache, slots, [[s[n + t]] for s, n in zip(seqs, lens)])
+        close(lg, np.stack([w[n + t] for w, n in zip(want, lens)]), "bfloat16")
+
+
 def test_mixed_portions_and_single_tokens_in_one_step():
     cfg = C.MIXED["b"]
     eng, W = build(cfg, "float32")
