@@ -791,7 +791,7 @@ __global__ void __launch_bounds__(256) k_attn_short(AttnArgs a) {
 // pulling ~1.6 MB through its CU (~30 GB/s per CU: the kernel is bound by that intake, MFMA busy
 // < 0.1).  Here a workgroup owns QB = NW x 16 query rows (MQA: the G heads of a KV head are rows of
 // the same tiles) and one of `ns` contiguous key ranges; K and V reach LDS by LDS-DMA into an
-// ST-slot ring filled by LW loader waves (counted vmcnt, one raw s_barrier per 32-key tile); the NW
+// ST-slot ring filled by LW loader waves (counted vmcnt, one raw s_barrier per tile of TK keys); the NW
 // compute waves run S^T = K Q^T, an online softmax and P.V on MFMA.  Each workgroup writes its
 // unnormalised O (fp32) and its per-row (max, sum) to scratch; k_attn_fs_combine merges the key
 // ranges in a fixed order (ns == 1: the workgroup normalises and stores bf16 itself).
@@ -805,14 +805,14 @@ __global__ void __launch_bounds__(256) k_attn_short(AttnArgs a) {
 // swizzle is applied to each lane's SOURCE address (the LDS-DMA destination is lane-linear); chunks
 // past the head dim (HD 72) load a copy of chunk 0 (finite; multiplied by Q's zeroed k range, or
 // feeding output columns that are never stored).
-template <int HD>
+template <int HD, int TK>
 struct FSInfo {
     static constexpr int KS = (HD + 31) / 32;        // 32-deep k-steps of K.Q
     static constexpr int CT = (HD + 15) / 16;        // 16-wide output tiles of P.V
     static constexpr int CH = (HD + 7) / 8;          // 16-B chunks of a head row in HBM
     static constexpr int CR = HD <= 128 ? 16 : 32;   // 16-B chunks of an LDS row
     static constexpr int ROWB = CR * 16;
-    static constexpr int TILEB = 32 * ROWB;          // one 32-key K (or V) image
+    static constexpr int TILEB = TK * ROWB;          // one tile's K (or V) image
     static constexpr int SLOTB = 2 * TILEB;          // ring slot: K image, then V image
     static constexpr int PCS = SLOTB / 1024;         // 1-KiB LDS-DMA pieces per slot
     static_assert(CR >= 4 * KS && CR >= 2 * CT && CR >= 16, "LDS row holds every k-step and tile");
@@ -834,19 +834,19 @@ __device__ __forceinline__ void fs_vm_wait(int n) {  // s_waitcnt vmcnt(G * min(
 
 // grid (row blocks, n_kv * ns, B); key range sp = blockIdx.y % ns covers tiles [sp * tps, (sp + 1) * tps)
 // P2: scale is a power of two (Gemma: 1/16), so bf16(bf16(x) * scale) = bf16(x) * scale (one rounding)
-template <int HD, int NW, int LW, int ST, bool P2>
+template <int HD, int NW, int LW, int ST, bool P2, int TK>
 __global__ void __launch_bounds__(64 * (NW + LW), 1) k_attn_fs(AttnArgs a, int ns, int tps) {
-    using I = FSInfo<HD>;
+    using I = FSInfo<HD, TK>;
     constexpr int KS = I::KS, CT = I::CT, CH = I::CH, CR = I::CR, ROWB = I::ROWB, TILEB = I::TILEB;
     constexpr int SLOTB = I::SLOTB, PCS = I::PCS, GPW = PCS / LW;
-    constexpr int QB = NW * 16;
+    constexpr int QB = NW * 16, KB = TK / 16;  // keys in blocks of 16
     static_assert(PCS % LW == 0, "whole pieces per loader wave");
     extern __shared__ __attribute__((aligned(16))) uint8_t fs_sm[];
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int b = blockIdx.z, kvh = blockIdx.y / ns, sp = blockIdx.y % ns;
-    const int nt = (a.Lk + 31) / 32;
+    const int nt = (a.Lk + TK - 1) / TK;
     const int t0 = sp * tps;
     const int t1 = t0 + tps < nt ? t0 + tps : nt;
     const int ntl = t1 > t0 ? t1 - t0 : 0;
@@ -873,7 +873,7 @@ __global__ void __launch_bounds__(64 * (NW + LW), 1) k_attn_fs(AttnArgs a, int n
         auto issue = [&](int t, int slot) {
 #pragma unroll
             for (int i = 0; i < GPW; ++i) {
-                int key = t * 32 + prow[i];
+                int key = t * TK + prow[i];
                 key = key < a.Lk ? key : a.Lk - 1;  // rows past the keys: a valid row, masked (s = -inf)
                 const uint16_t* src =
                     (pv[i] ? vbase + (long)key * a.v_row_stride : kbase + (long)key * a.k_row_stride) + pch[i] * 8;
@@ -924,14 +924,14 @@ __global__ void __launch_bounds__(64 * (NW + LW), 1) k_attn_fs(AttnArgs a, int n
     const int vsw = (vr0 & 7) << 1;
     // S^T = K Q^T of the tile in `sl`: lane holds keys 16 kt + 4 g + j of query li; even / odd
     // k-steps accumulate in two chains
-    auto scores = [&](int sl, f32x4 (&ac)[2][2]) {
+    auto scores = [&](int sl, f32x4 (&ac)[KB][2]) {
         const uint8_t* kb = fs_sm + sl * SLOTB;
 #pragma unroll
-        for (int kt = 0; kt < 2; ++kt) ac[kt][0] = ac[kt][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int kt = 0; kt < KB; ++kt) ac[kt][0] = ac[kt][1] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int kk = 0; kk < KS; ++kk)
 #pragma unroll
-            for (int kt = 0; kt < 2; ++kt) {
+            for (int kt = 0; kt < KB; ++kt) {
                 const int r = kt * 16 + li;
                 const short8 kf = *reinterpret_cast<const short8*>(kb + r * ROWB + (((kk * 4 + g) ^ (r & 15)) << 4));
                 ac[kt][kk & 1] = mfma16(kf, qf[kk], ac[kt][kk & 1]);
@@ -939,24 +939,24 @@ __global__ void __launch_bounds__(64 * (NW + LW), 1) k_attn_fs(AttnArgs a, int n
     };
     // s = bf16(bf16(k.q) * scale), keys past Lk masked (the last tile only: wave-uniform branch);
     // returns the tile's max of row li
-    auto finish = [&](int t, const f32x4 (&ac)[2][2], float (&sv)[2][4]) -> float {
+    auto finish = [&](int t, const f32x4 (&ac)[KB][2], float (&sv)[KB][4]) -> float {
         float mx = -INFINITY;
 #pragma unroll
-        for (int kt = 0; kt < 2; ++kt)
+        for (int kt = 0; kt < KB; ++kt)
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 const float x = rbf(ac[kt][0][j] + ac[kt][1][j]);
                 sv[kt][j] = P2 ? x * a.scale : rbf(x * a.scale);
             }
-        if (t * 32 + 32 > a.Lk) {
+        if (t * TK + TK > a.Lk) {
 #pragma unroll
-            for (int kt = 0; kt < 2; ++kt)
+            for (int kt = 0; kt < KB; ++kt)
 #pragma unroll
                 for (int j = 0; j < 4; ++j)
-                    if (t * 32 + kt * 16 + 4 * g + j >= a.Lk) sv[kt][j] = -INFINITY;
+                    if (t * TK + kt * 16 + 4 * g + j >= a.Lk) sv[kt][j] = -INFINITY;
         }
 #pragma unroll
-        for (int kt = 0; kt < 2; ++kt)
+        for (int kt = 0; kt < KB; ++kt)
 #pragma unroll
             for (int j = 0; j < 4; ++j) mx = fmaxf(mx, sv[kt][j]);
         mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
@@ -964,10 +964,10 @@ __global__ void __launch_bounds__(64 * (NW + LW), 1) k_attn_fs(AttnArgs a, int n
     };
     // one tile ahead: iteration it multiplies K of tile it + 1 while it runs the softmax and P.V of
     // tile it (the two are independent, so the MFMAs of one overlap the VALU of the other)
-    float s[2][4], tm = -INFINITY;
+    float s[KB][4], tm = -INFINITY;
     if (ntl > 0) {
         __builtin_amdgcn_s_barrier();  // barrier 0: tiles 0 and 1 landed
-        f32x4 ac[2][2];
+        f32x4 ac[KB][2];
         scores(0, ac);
         tm = finish(t0, ac, s);
     }
@@ -978,7 +978,7 @@ __global__ void __launch_bounds__(64 * (NW + LW), 1) k_attn_fs(AttnArgs a, int n
             __builtin_amdgcn_s_barrier();                         // tiles it and it + 1 in the ring
         }
         const int nslot = slot + 1 == ST ? 0 : slot + 1;
-        f32x4 acn[2][2];
+        f32x4 acn[KB][2];
         scores(nslot, acn);  // tile it + 1 (past the last tile: stale LDS, never used)
         // deferred running max: raised (and O, l rescaled) only when a row's tile max passes it by
         // kFsDefer; wave-uniform branch
@@ -994,24 +994,27 @@ __global__ void __launch_bounds__(64 * (NW + LW), 1) k_attn_fs(AttnArgs a, int n
             }
             m = mn;
         }
-        short8 pa;
+        short8 pa[TK / 32];
 #pragma unroll
-        for (int kt = 0; kt < 2; ++kt)
+        for (int kt = 0; kt < KB; ++kt)
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 const float e = fa_exp(s[kt][j] - m);  // masked: exp(-inf) = 0
                 l += e;
-                pa[kt * 4 + j] = (short)f2bf(e);
+                pa[kt / 2][kt % 2 * 4 + j] = (short)f2bf(e);
             }
         const uint8_t* vb = fs_sm + slot * SLOTB + TILEB;
 #pragma unroll
         for (int c = 0; c < CT; ++c) {
             const int cidx = 2 * c + ((li & 3) >> 1);
-            const uint8_t* pl = vb + vr0 * ROWB + ((cidx ^ vsw) << 4) + (li & 1) * 8;
-            const s4v lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s4v*)pl);
-            const s4v hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s4v*)(pl + 16 * ROWB));
-            const short8 vv = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-            o[c] = mfma16(pa, vv, o[c]);
+#pragma unroll
+            for (int u = 0; u < TK / 32; ++u) {
+                const uint8_t* pl = vb + (u * 32 + vr0) * ROWB + ((cidx ^ vsw) << 4) + (li & 1) * 8;
+                const s4v lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s4v*)pl);
+                const s4v hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s4v*)(pl + 16 * ROWB));
+                const short8 vv = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+                o[c] = mfma16(pa[u], vv, o[c]);
+            }
         }
         tm = finish(t0 + it + 1, acn, s);
         slot = nslot;
@@ -1096,46 +1099,47 @@ __global__ void __launch_bounds__(256) k_attn_fs_combine(AttnArgs a, int ns) {
 // workgroups runs in two rounds: split the keys (2, 4, ...) only while the grid stays within one
 // round and every range keeps >= 16 tiles (shorter ranges lose more to the combine than they gain);
 // scratch for the partials or the split is dropped
-static int fs_splits(const AttnArgs& a, int HD, int QB, int want) {
-    const int nrows = a.Lq * a.G, nt = (a.Lk + 31) / 32;
+static int fs_splits(const AttnArgs& a, int HD, int QB, int TK, int want) {
+    const int nrows = a.Lq * a.G, nt = (a.Lk + TK - 1) / TK;
     const long blocks = (long)(nrows + QB - 1) / QB * a.n_kv * a.B;
     int ns = 1;
     if (want > 0) ns = want;
     else
-        while (blocks * ns * 2 <= 256 && nt / (ns * 2) >= 16) ns *= 2;
+        while (blocks * ns * 2 <= 256 && nt / (ns * 2) >= 512 / TK) ns *= 2;
     if (ns > nt) ns = nt;
     while (ns > 1 && (!a.ws || (long)a.B * a.n_kv * ns * nrows * (HD + 2) > a.ws_floats)) ns >>= 1;
     return ns < 1 ? 1 : ns;
 }
 
-template <int HD, int NW, int LW, int ST, bool P2>
+template <int HD, int NW, int LW, int ST, bool P2, int TK>
 static void launch_fs_t(hipStream_t s, const AttnArgs& a, int ns, int tps, dim3 grid) {
-    constexpr size_t lds = (size_t)ST * FSInfo<HD>::SLOTB;
+    constexpr size_t lds = (size_t)ST * FSInfo<HD, TK>::SLOTB;
     static_assert(lds <= 160 * 1024, "LDS");
     static bool attr = false;
     if (!attr) {
-        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&k_attn_fs<HD, NW, LW, ST, P2>),
+        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&k_attn_fs<HD, NW, LW, ST, P2, TK>),
                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         attr = true;
     }
-    hipLaunchKernelGGL((k_attn_fs<HD, NW, LW, ST, P2>), grid, dim3(64 * (NW + LW)), lds, s, a, ns, tps);
+    hipLaunchKernelGGL((k_attn_fs<HD, NW, LW, ST, P2, TK>), grid, dim3(64 * (NW + LW)), lds, s, a, ns, tps);
 }
 
 template <int HD, int NWQ = 0>
 static void launch_fs(hipStream_t s, const AttnArgs& a, int want_ns) {
     // head dim 256: 4 compute waves (their registers fit 2 waves per SIMD with the loaders, not 3) and a
-    // 5-slot ring (160 KiB); head dim 72: 8 compute waves, 8 slots.  NWQ > 0: that many compute waves (fewer
+    // 5-slot ring (160 KiB) of 32-key tiles; head dim 72: 8 compute waves, 4 slots of 64-key tiles, whose barriers and row maxima
+    // are half as many (of 32 keys in 8 slots a 448 px photo's prefill 0.5 % slower; 5 slots: the same).  NWQ > 0: that many compute waves (fewer
     // query rows per workgroup, more workgroups over the same keys: probe variants 81 / 82)
-    constexpr int NW = NWQ > 0 ? NWQ : HD == 256 ? 4 : 8, LW = 4, ST = HD == 256 ? 5 : 8;
-    const int nrows = a.Lq * a.G, nt = (a.Lk + 31) / 32;
-    int ns = fs_splits(a, HD, NW * 16, want_ns);
+    constexpr int NW = NWQ > 0 ? NWQ : HD == 256 ? 4 : 8, LW = 4, TK = HD == 256 ? 32 : 64, ST = HD == 256 ? 5 : 4;
+    const int nrows = a.Lq * a.G, nt = (a.Lk + TK - 1) / TK;
+    int ns = fs_splits(a, HD, NW * 16, TK, want_ns);
     const int tps = (nt + ns - 1) / ns;
     ns = (nt + tps - 1) / tps;  // no empty range
     dim3 grid((nrows + NW * 16 - 1) / (NW * 16), a.n_kv * ns, a.B);
     int e2 = 0;
     const bool p2 = std::frexp(a.scale, &e2) == 0.5f;
-    if (p2) launch_fs_t<HD, NW, LW, ST, true>(s, a, ns, tps, grid);
-    else launch_fs_t<HD, NW, LW, ST, false>(s, a, ns, tps, grid);
+    if (p2) launch_fs_t<HD, NW, LW, ST, true, TK>(s, a, ns, tps, grid);
+    else launch_fs_t<HD, NW, LW, ST, false, TK>(s, a, ns, tps, grid);
     if (ns > 1) {
         const long n8 = (long)a.B * a.n_kv * nrows * (HD / 8);
         hipLaunchKernelGGL(k_attn_fs_combine<HD>, dim3((unsigned)((n8 + 255) / 256)), dim3(256), 0, s, a, ns);
@@ -1211,7 +1215,10 @@ void attention_prefill(hipStream_t s, int head_dim, const AttnArgs& a) {
     }
     if (v == 9 || v == 91 || v == 92 || v == 94) {  // one pass, keys split over workgroups (auto / 1 / 2 / 4 ranges)
         const int want = v == 9 ? 0 : v - 90;
-        if (head_dim == 256) launch_fs<256>(s, a, want);
+        // past 256 workgroups of 64 rows (one a CU), 128 rows each: eight 288-token prompts 288 workgroups, in two rounds, so 144
+        // (with the towers' longer tiles, eight photos' prefill 12,446 -> 12,354 us)
+        if (head_dim == 256 && (long)(a.Lq * a.G + 63) / 64 * a.n_kv * a.B > 256) launch_fs<256, 8>(s, a, want);
+        else if (head_dim == 256) launch_fs<256>(s, a, want);
         else launch_fs<72>(s, a, want);
         return;
     }
