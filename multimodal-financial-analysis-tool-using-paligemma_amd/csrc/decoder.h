@@ -246,6 +246,7 @@ struct GruArgs {
     const ChunkInfo* chunks;
     int nchunk;
     bool multi;
+    bool walk;  // whole sequences, as the scan's; chunks and cstate are not read
 };
 void mingru_scan(hipStream_t s, Act act, const GruArgs& a);
 

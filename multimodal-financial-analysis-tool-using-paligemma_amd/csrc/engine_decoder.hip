@@ -583,7 +583,7 @@ struct Meta {
         int n;
         bool multi;  // some sequence has more than one
     } scan, gru, conv;
-    ScanStep step;
+    ScanStep step, gru_step;  // the sequences in scan's and in gru's runs
     const int32_t *starts, *lens;  // on the host
     bool fresh;  // every sequence from its start
     const int* row_seq;
@@ -674,6 +674,7 @@ int forward_body(pgmi_ctx* x, hipStream_t s, const int64_t* ids, int rows, const
             GruArgs a{};
             a.zug = d.p0; a.ld = ldz; a.state = at<float>(state, st[i].a); a.cstate = d.cstate; a.y = d.p2; a.ldy = ldc;
             a.C = C; a.seqs = m.seqs; a.nseq = m.nseq; a.chunks = m.gru.p; a.nchunk = m.gru.n; a.multi = m.gru.multi;
+            a.walk = gru_walks(m.gru_step, C, d.act == ACT_F32);
             mingru_scan(s, d.act, a);
             out_proj(w.o, d.p2, ldc, w.sub[0]);
         }
@@ -1093,13 +1094,17 @@ int pgmi_decoder_forward(pgmi_ctx* x, const int64_t* ids, int n_seq, const int32
     }
     const bool huge = rows > 16384;
     Cut scan{0, 0, false}, gru = scan, conv = scan;
-    ScanStep step;
+    ScanStep step, gru_step;
     if (scan_cols) {
         const int run = huge ? 256 : scan_run_rows(lens, n_seq, scan_cols, scan_wgs);
         scan = cut(run);
         step = scan_step_of(lens, n_seq, run);
     }
-    if (gru_cols) gru = cut(huge ? 128 : gru_run_rows(lens, n_seq, gru_cols));
+    if (gru_cols) {
+        const int run = huge ? 128 : gru_run_rows(lens, n_seq, gru_cols);
+        gru = cut(run);
+        gru_step = scan_step_of(lens, n_seq, run);
+    }
     // the convolutions carry nothing: 500 rows of 2,048 channels 11.2 us on 64-row runs, 5.9 on 16; 2,048 rows 10.8 / 7.5
     if (scan_cols || d.c.canon_taps > 0) conv = cut(huge ? 256 : rows > 2048 ? 32 : 16);
     struct Tiles { int R; size_t o; int n; };
@@ -1143,6 +1148,7 @@ int pgmi_decoder_forward(pgmi_ctx* x, const int64_t* ids, int n_seq, const int32
     meta.fresh = std::all_of(starts, starts + n_seq, [](int32_t p) { return p == 0; });
     meta.scan = {reinterpret_cast<const ChunkInfo*>(dm + scan.o), scan.n, scan.multi};
     meta.step = step;
+    meta.gru_step = gru_step;
     meta.starts = starts;
     meta.lens = lens;
     meta.gru = {reinterpret_cast<const ChunkInfo*>(dm + gru.o), gru.n, gru.multi};

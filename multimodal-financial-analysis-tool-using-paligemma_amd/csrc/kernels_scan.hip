@@ -739,6 +739,139 @@ __global__ void __launch_bounds__(64) k_gru_carry(GruArgs a) {
     }
 }
 
+// ---- sequences walked whole: one wave has 16 channels' states, eight others the rest
+// A step of the walk is one FMA behind the step before; the gates, candidates and outputs of 128 rows are formed around it, ahead of it
+// and after it, as in k_scan_walk.  V4: a thread of the eight waves has four channels of one row, else one channel of four rows.
+// Bound by those waves' three sigmoids a value, two waves a SIMD: 8 ns a row of the longest sequence (four waves and 64 rows 18, rows held
+// one group ahead or two alike).  us a layer, three launches of runs / this: 1,024 + 387 + 129 rows of 2,048 channels 21.6 / 13.5, 500
+// rows of 1,024 fp32 channels 14.7 / 7.7; the line between them: gru_walks.
+template <typename T, bool V4>
+__global__ void __launch_bounds__(576) k_gru_walk(GruArgs a) {
+    constexpr int ROWS = 128, LD = ROWS + 4;
+    __shared__ __attribute__((aligned(16))) float sa[2][kWalk][LD], sb[2][kWalk][LD], ss[2][kWalk][LD];  // keep, add, states
+    const SeqInfo q = a.seqs[blockIdx.y];
+    // an XCD's workgroups have neighbouring channels, which share the lines of every row
+    const int per = gridDim.x / 8, c0 = ((blockIdx.x % 8) * per + blockIdx.x / 8) * kWalk;
+    const int len = q.len, ngr = (len + ROWS - 1) / ROWS;
+    if (c0 >= max(a.C, a.ldy)) return;
+    if (threadIdx.x >= 512) {
+        const int ch = threadIdx.x & 15, c = c0 + ch;
+        const bool mine = threadIdx.x < 512 + kWalk && c < a.C;
+        float* st = a.state + (long)q.slot * a.C + min(c, a.C - 1);
+        float S = q.start > 0 ? *st : 0.0f;
+        __syncthreads();
+        for (int i = 0; i < ngr; ++i) {
+            const int k = i & 1;
+            if (mine) {
+                // 32 rows' operands before their chain, so that it waits for no read but the first
+#pragma unroll
+                for (int h = 0; h < ROWS; h += 32) {  // rows past the end keep the state
+                    if (h >= len - i * ROWS) break;
+                    f32x4 va[8], vb[8];
+#pragma unroll
+                    for (int r = 0; r < 8; ++r) {
+                        va[r] = *reinterpret_cast<const f32x4*>(&sa[k][ch][h + 4 * r]);
+                        vb[r] = *reinterpret_cast<const f32x4*>(&sb[k][ch][h + 4 * r]);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                    for (int r = 0; r < 8; ++r) {
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) vb[r][e] = S = fmaf(va[r][e], S, vb[r][e]);
+                        *reinterpret_cast<f32x4*>(&ss[k][ch][h + 4 * r]) = vb[r];
+                    }
+                }
+            }
+            __syncthreads();
+        }
+        if (mine) *st = S;
+        return;
+    }
+    typedef T T4 __attribute__((ext_vector_type(4)));
+    const int tid = threadIdx.x;
+    const T* __restrict__ zp = reinterpret_cast<const T*>(a.zug) + (long)q.off * a.ld;
+    T* __restrict__ yp = reinterpret_cast<T*>(a.y) + (long)q.off * a.ldy;
+    // element e of a thread: V4: row r0, channel c0 + h0 + e; else row r0 + e, channel c0 + h0; 16 rows a wave
+    const int r0 = V4 ? tid >> 2 : (tid >> 4) * 4, w0 = (tid >> 6) * 16, h0 = V4 ? (tid & 3) * 4 : tid & 15, hc = V4 ? c0 + h0 : min(c0 + h0, a.C - 1);
+    auto row_of = [&](int e) { return V4 ? r0 : r0 + e; };
+    struct Held { T4 z, u, g; };
+    auto hold = [&](int t0, Held& h) {  // rows past the end repeat the last one (never used)
+        if constexpr (V4) {
+            const T* r = zp + (long)min(t0 + r0, len - 1) * a.ld + hc;
+            h.z = *reinterpret_cast<const T4*>(r);
+            h.u = *reinterpret_cast<const T4*>(r + a.C);
+            h.g = *reinterpret_cast<const T4*>(r + 2 * a.C);
+        } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const T* r = zp + (long)min(t0 + row_of(e), len - 1) * a.ld + hc;
+                h.z[e] = r[0];
+                h.u[e] = r[a.C];
+                h.g[e] = r[2 * a.C];
+            }
+        }
+    };
+    auto stage = [&](int to, int t0, const Held& h, f32x4& gate) {
+        if (w0 >= (len - t0 + 31 & ~31)) return;  // the walker stops there
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const T ze = h.z[e], ue = h.u[e], ge = h.g[e];
+            const bool row = t0 + row_of(e) < len;
+            const float zz = sigmoidf_(ldf(&ze));
+            const int ch = V4 ? h0 + e : h0;
+            sa[to][ch][row_of(e)] = row ? 1.0f - zz : 1.0f;
+            sb[to][ch][row_of(e)] = row ? zz * gru_candidate(ldf(&ue)) : 0.0f;
+            gate[e] = siluf_(ldf(&ge));
+        }
+    };
+    auto leave = [&](int from, int t0, const f32x4& gate) {
+        T4 o;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            T r;
+            stf(&r, c0 + h0 < a.C ? ss[from][V4 ? h0 + e : h0][row_of(e)] * gate[e] : 0.0f);  // columns C .. ldy - 1 are zero
+            o[e] = r;
+        }
+        if constexpr (V4) {
+            if (t0 + r0 < len) *reinterpret_cast<T4*>(yp + (long)(t0 + r0) * a.ldy + hc) = o;
+        } else if (c0 + h0 < a.ldy) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                if (t0 + row_of(e) < len) yp[(long)(t0 + row_of(e)) * a.ldy + c0 + h0] = o[e];
+        }
+    };
+    f32x4 before{}, now{}, next{};
+    Held even, odd;  // two groups of rows on their way
+    auto turn = [&](int i, Held& h) {  // h: group i + 1
+        if (i > 0) leave(~i & 1, (i - 1) * ROWS, before);
+        if (i + 1 < ngr) {
+            stage(~i & 1, (i + 1) * ROWS, h, next);
+            if (i + 3 < ngr) hold((i + 3) * ROWS, h);
+        }
+        before = now;
+        now = next;
+        __syncthreads();
+    };
+    hold(0, even);
+    if (1 < ngr) hold(ROWS, odd);
+    stage(0, 0, even, now);
+    if (2 < ngr) hold(2 * ROWS, even);
+    __syncthreads();
+    for (int i = 0; i < ngr; i += 2) {
+        turn(i, odd);
+        if (i + 1 < ngr) turn(i + 1, even);
+    }
+    leave(~ngr & 1, (ngr - 1) * ROWS, before);
+}
+
+template <typename T>
+void launch_gru_walk(hipStream_t s, const GruArgs& a) {
+    const dim3 grid(((std::max(a.C, a.ldy) + kWalk - 1) / kWalk + 7) / 8 * 8, a.nseq), blk(576);
+    const uintptr_t at = reinterpret_cast<uintptr_t>(a.zug) | reinterpret_cast<uintptr_t>(a.y);
+    if (a.C % kWalk == 0 && a.ldy == a.C && a.ld % 4 == 0 && at % 16 == 0) hipLaunchKernelGGL((k_gru_walk<T, true>), grid, blk, 0, s, a);
+    else hipLaunchKernelGGL((k_gru_walk<T, false>), grid, blk, 0, s, a);
+}
+
 template <typename T, int V>
 void gru_v(hipStream_t s, const GruArgs& a) {
     const int cols = std::max(a.C, V == 1 ? a.ldy : a.C);
@@ -752,6 +885,7 @@ void gru_v(hipStream_t s, const GruArgs& a) {
 
 template <typename T>
 void gru_t(hipStream_t s, const GruArgs& a) {
+    if (a.walk) return launch_gru_walk<T>(s, a);
     if (a.C % 8 == 0 && a.ld % 8 == 0) gru_v<T, 2>(s, a);
     else gru_v<T, 1>(s, a);
 }

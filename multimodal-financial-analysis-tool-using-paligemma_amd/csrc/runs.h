@@ -105,6 +105,18 @@ inline int gru_run_rows(const int32_t* lens, int n_seq, long columns) {
     return ct;
 }
 
+// Whether a minGRU layer walks its sequences whole (k_gru_walk, one launch) rather than in the runs above: as scan_walks, by the
+// predicted time in us, fitted to 180 steps of 44 to 4,096 channels and 17 to 4,096 rows; it loses 1.1 % of the better form on average,
+// mostly at 64 x 33 rows of 256 channels (9 instead of 7).  us a layer, runs / walk: 1,024 + 387 + 129 rows of 2,048 channels 21.6 / 13.5,
+// 500 rows of 1,024 fp32 channels 14.7 / 7.7, 60 rows of 2,048 10.9 / 5.6, 8 x 512 rows 29.8 / 25.1; 64 x 33 rows 11.0 / 40, 4,096
+// rows of 1,024 channels 30 / 38.
+inline bool gru_walks(const ScanStep& s, int C, bool f32) {
+    const double per_cu = (C + 15) / 16 / (double)kRunCUs, traffic = (f32 ? 3.4e-6 : 1.65e-6) * C * (double)s.rows;
+    const double walk = 4.5 + std::max(0.008 * s.longest, per_cu * (0.5 * s.n_seq + (f32 ? 0.0135 : 0.0095) * (double)s.padded));
+    const double runs = traffic + (s.most_runs == 1 ? 3.6 + 0.11 * s.run_rows : 8.2 + 0.21 * s.run_rows + 0.07 * s.most_runs);
+    return walk < runs;
+}
+
 // Whether a prompt's attention gives each tile of 64 (position, head) pairs to two teams of four waves, which take its 64-key tiles in
 // turn, rather than to one: where the longest tile's chain is what the step waits for, and not the sum of all tiles over the chip (the
 // second team's sums cost LDS and a merge).  us, one team / two, 16 heads of 128 in 2 groups, window 1,024: 1,300 + 511 + 235 + 2 rows

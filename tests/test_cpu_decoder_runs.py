@@ -94,3 +94,36 @@ def walks(tmp_path_factory):
     (72, 12, [70, 33, 5], 1, 1), (72, 8, [70, 33, 5], 0, 0), (72, 17, [70, 33, 5], 0, 0), (2048, 64, [500], 0, 0), (64, 9, [1], 1, 1)])
 def test_scan_walks(walks, C, N, lens, bf16, f32):
     assert walks(C, N, *lens) == [bf16, f32]
+
+
+GRU_WALKS = r"""
+#include <cstdio>
+#include <cstdlib>
+#include <vector>
+#include "runs.h"
+int main(int n, char** v) {  // channels, lengths
+    std::vector<int32_t> lens;
+    for (int i = 2; i < n; ++i) lens.push_back(atoi(v[i]));
+    const int C = atoi(v[1]), k = (int)lens.size();
+    const pgmi::ScanStep s = pgmi::scan_step_of(lens.data(), k, pgmi::gru_run_rows(lens.data(), k, (C + 127) / 128));
+    std::printf("%d %d\n", (int)pgmi::gru_walks(s, C, false), (int)pgmi::gru_walks(s, C, true));
+}
+"""
+
+
+@pytest.fixture(scope="module")
+def gru_walks(tmp_path_factory):
+    at = tmp_path_factory.mktemp("gru_walks")
+    (at / "ask.cpp").write_text(GRU_WALKS)
+    subprocess.run(["g++", "-std=c++17", "-Wall", "-Werror", "-I", CSRC, str(at / "ask.cpp"), "-o", str(at / "ask")], check=True)
+    return lambda *a: [int(x) for x in subprocess.run([str(at / "ask"), *map(str, a)], check=True, capture_output=True,
+                                                      text=True).stdout.split()]
+
+
+# minGRU's sequences walked whole (bf16, fp32) where that was the faster form by more than the rule's error
+@pytest.mark.parametrize("C,lens,bf16,f32", [
+    (2048, [1024, 387, 129], 1, 1), (1024, [500], 1, 1), (2048, [60], 1, 1), (4096, [1000], 1, 1), (2048, [1000] * 4, 1, 1),
+    (1024, [512] * 8, 1, 1), (256, [64] * 32, 1, 1), (44, [300], 1, 1), (1024, [33] * 64, 0, 0), (4096, [33] * 64, 0, 0),
+    (4096, [64] * 32, 0, 0), (64, [4096], 0, 0), (256, [4096], 0, 0), (44, [2000], 0, 0)])
+def test_gru_walks(gru_walks, C, lens, bf16, f32):
+    assert gru_walks(C, *lens) == [bf16, f32]

@@ -135,6 +135,35 @@ def test_scan_in_runs_as_walked(dtype):
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("width", [16, 48, 56, 13])
+def test_gru_of_sequences_walked_whole(width, dtype):
+    """Sequences that end just before, on and just after a wave's 16 rows, the walker's 32 and a stage's 128, of one to four stages,
+    of channels that are and are not whole vectors and workgroups, then the next portions from the states that were left."""
+    cfg = C.model([C.gru(width)], width=64, streams=1, groups=1)
+    eng, W = build(cfg, dtype)
+    first, then = [1, 15, 17, 32, 33, 127, 128, 129, 256, 257, 400], [129, 1, 128, 16, 31, 64, 33, 17, 3, 270, 2]
+    seqs = [tokens(cfg, a + b, 60 + r) for r, (a, b) in enumerate(zip(first, then))]
+    cache = eng.new_cache(len(seqs), 640)
+    slots = [cache.alloc() for _ in seqs]
+    a = eng.forward(cache, slots, [t for s, n in zip(seqs, first) for t in s[:n]], first, want=range(sum(first))).clone()
+    b = eng.forward(cache, slots, [t for s, n in zip(seqs, first) for t in s[n:]], then, want=range(sum(then))).clone()
+    for r, s in enumerate(seqs):
+        i, j = sum(first[:r]), sum(then[:r])
+        close(torch.cat([a[i:i + first[r]], b[j:j + then[r]]]), O.run(cfg, W, s), dtype)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_gru_in_runs_as_walked(dtype):
+    """4,100 rows of few channels go in runs; in portions of 410 they are walked."""
+    cfg = C.model([C.gru(64)], width=64, streams=1, groups=1)
+    eng, _ = build(cfg, dtype)
+    toks = tokens(cfg, 4100, 9)
+    cache = eng.new_cache(2, 4112)
+    whole = eng.forward(cache, [cache.alloc()], toks, [len(toks)], want=range(len(toks))).clone()
+    close(feed(eng, cache, cache.alloc(), toks, [410]), whole.double().cpu().numpy(), dtype)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("name", list(ALL))
 def test_token_by_token(name, dtype):
     cfg = ALL[name]
