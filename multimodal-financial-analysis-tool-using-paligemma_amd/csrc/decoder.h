@@ -291,7 +291,7 @@ struct WAttnArgs {
     bool teams;  // bf16: two teams of four waves a tile, which take its key tiles in turn (wattn_teams)
 };
 void wattn_append(hipStream_t s, Act act, const WAttnArgs& a);
-constexpr int kWAttnRows = 64;  // (position, query head of the group) pairs per prefill tile: ChunkInfo.rel of `tiles`
+constexpr int kWAttnRows = 64;  // (position, query head of the group) pairs per prefill tile: ChunkInfo.rel of `tiles`, fewest keys first (attn_tiles)
 void wattn_prefill(hipStream_t s, Act act, const WAttnArgs& a);
 
 // one new token per sequence: row b of qkv (activation type [B][ldqkv], biases added) is position pos[b] of slot[b]; appends

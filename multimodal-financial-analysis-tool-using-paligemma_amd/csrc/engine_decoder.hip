@@ -1114,9 +1114,11 @@ int pgmi_decoder_forward(pgmi_ctx* x, const int64_t* ids, int n_seq, const int32
         const int R = l.heads / l.kv_heads;
         if (std::any_of(tiles.begin(), tiles.end(), [&](const Tiles& t) { return t.R == R; })) continue;
         Tiles t{R, m.size(), 0};
-        for (int r = 0; r < n_seq; ++r) {
+        for (int r = 0; r < n_seq; ++r)
             if ((long)lens[r] * R > INT32_MAX - kWAttnRows) return fail(PGMI_E_ARG, "too many tokens in one step");
-            for (int f = 0; f < lens[r] * R; f += kWAttnRows, ++t.n) put({r, 0, kWAttnRows, f, 0, 0});
+        for (const AttnTile& k : attn_tiles(starts, lens, n_seq, R, kWAttnRows)) {
+            put({k.seq, 0, kWAttnRows, k.first, 0, 0});
+            ++t.n;
         }
         tiles.push_back(t);
     }

@@ -230,6 +230,16 @@ __global__ void __launch_bounds__(256) k_wattn(WAttnArgs a) {
 // positions 312; here 24 and 58.
 __device__ __forceinline__ f32x4 mfma_f32(float a, float b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
 
+// The piece of work, of n pieces with the longest first, that this workgroup takes.  Workgroups b and b + 256 share a CU from the start,
+// later ones come as others end: the longest 256 backwards, so that the second of a CU is the shorter the longer its first is, and
+// the longest are alone where n < 512.  A group's neighbours are other key/value heads' equal pieces.  us, pieces by sequence
+// and head, so this: fp32, 8 heads of 128 in 2 groups, 700 rows 39.9 / 31.9, 1,024 rows 68.9 / 45.0, 1,024 + 387 + 129 rows 72.4 / 53.2;
+// bf16, 16 heads, 1,024 + 387 + 129 rows 32.0 / 25.8, 1,411 + 700 + 510 + 256 + 90 rows 51.6 / 47.0.
+__device__ __forceinline__ int piece() {
+    const int n = gridDim.x * gridDim.y, b = blockIdx.x + gridDim.x * blockIdx.y;
+    return n > 256 && b < 256 ? 255 - b : b;
+}
+
 // PAD: heads narrower than D
 template <int D, int SC, bool PAD>
 __global__ void __launch_bounds__(256, D <= 128 ? 2 : 1) k_wattn_f(WAttnArgs a) {
@@ -237,10 +247,10 @@ __global__ void __launch_bounds__(256, D <= 128 ? 2 : 1) k_wattn_f(WAttnArgs a) 
     __shared__ __attribute__((aligned(16))) float part[4][16][68];  // 64 value columns of the waves' sums
     __shared__ float ms[4][16], ls[4][16];
     const WAttnHeads& w = a.hd;
-    const int at = a.ntile * PT - 1 - (int)blockIdx.x;  // the later positions of a sequence first
+    const int pc = piece(), g = pc % w.G, at = a.ntile * PT - 1 - pc / w.G;  // the later positions first
     const ChunkInfo tl = a.tiles[at / PT];
     const SeqInfo sq = a.seqs[tl.seq];
-    const int g = blockIdx.y, R = w.H / w.G, nrow = sq.len * R, row0 = tl.rel + at % PT * 16;
+    const int R = w.H / w.G, nrow = sq.len * R, row0 = tl.rel + at % PT * 16;
     if (row0 >= nrow) return;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int li = lane & 15, lg = lane >> 4;
@@ -427,10 +437,11 @@ __global__ void __launch_bounds__(256 * TEAMS) k_wattn_m(WAttnArgs a) {
     const int team = TEAMS == 1 ? 0 : __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 8);
     uint16_t* Ks = reinterpret_cast<uint16_t*>(smem_wattn + (size_t)team * wattn_m_lds(DQ, DV, 1));
     uint16_t* Vs = Ks + KT * KS;
-    const int g = blockIdx.y, R = w.H / w.G;
-    // later positions see more keys: every other key/value head backwards, so that a CU's two workgroups are not both long
-    // (2,048 rows in sequences up to 1,300: 53.0 us, so 47.3)
-    const ChunkInfo tl = a.tiles[g & 1 ? a.ntile - 1 - (int)blockIdx.x : blockIdx.x];
+    const int R = w.H / w.G;
+    // One sequence: every other key/value head backwards, so that a CU's two workgroups are not both long (2,048 rows 48.3 us, as
+    // pieces 49.8); several: pieces
+    const int pc = piece(), g = a.nseq > 1 ? pc % w.G : blockIdx.y;
+    const ChunkInfo tl = a.tiles[a.nseq > 1 ? a.ntile - 1 - pc / w.G : g & 1 ? a.ntile - 1 - (int)blockIdx.x : blockIdx.x];
     const SeqInfo sq = a.seqs[tl.seq];
     const int tid = threadIdx.x & 255, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int li = lane & 15, lg = lane >> 4;

@@ -1,5 +1,5 @@
-// runs.h -- how many rows of a sequence one workgroup of a recurrence walks, and who walks an attention's keys (host code, without
-// HIP).
+// runs.h -- how many rows of a sequence one workgroup of a recurrence walks, who walks an attention's keys and in which order its tiles
+// are listed (host code, without HIP).
 //
 // A short step's few runs are walked by a few CUs, each row waiting for the one before; where the chip is full short runs only
 // add carries.
@@ -7,6 +7,7 @@
 #include <algorithm>
 #include <climits>
 #include <cstdint>
+#include <vector>
 
 namespace pgmi {
 
@@ -115,6 +116,30 @@ inline bool gru_walks(const ScanStep& s, int C, bool f32) {
     const double walk = 4.5 + std::max(0.008 * s.longest, per_cu * (0.5 * s.n_seq + (f32 ? 0.0135 : 0.0095) * (double)s.padded));
     const double runs = traffic + (s.most_runs == 1 ? 3.6 + 0.11 * s.run_rows : 8.2 + 0.21 * s.run_rows + 0.07 * s.most_runs);
     return walk < runs;
+}
+
+// The tiles of a prompt's attention, `rows` (position, head) pairs of one sequence each: by the 64 keys that the last position's fall in,
+// so fewest keys first whatever the window, then by sequence.
+struct AttnTile { int seq, first; };
+inline std::vector<AttnTile> attn_tiles(const int32_t* starts, const int32_t* lens, int n_seq, int R, int rows) {
+    std::vector<AttnTile> t;
+    std::vector<int> end;
+    long lo = LONG_MAX, hi = 0;
+    for (int r = 0; r < n_seq; ++r)
+        for (int f = 0, n = lens[r] * R; f < n; f += rows) {
+            end.push_back(starts[r] / 64 + (starts[r] % 64 + (std::min((long)f + rows, (long)n) - 1) / R) / 64);
+            lo = std::min(lo, (long)end.back());
+            hi = std::max(hi, (long)end.back());
+            t.push_back({r, f});
+            if (n - f <= rows) break;
+        }
+    if (n_seq == 1) return t;
+    std::vector<int> at(hi - lo + 2);
+    for (const int e : end) ++at[e - lo + 1];
+    for (size_t k = 1; k < at.size(); ++k) at[k] += at[k - 1];
+    std::vector<AttnTile> sorted(t.size());
+    for (size_t k = 0; k < t.size(); ++k) sorted[at[end[k] - lo]++] = t[k];
+    return sorted;
 }
 
 // Whether a prompt's attention gives each tile of 64 (position, head) pairs to two teams of four waves, which take its 64-key tiles in

@@ -127,3 +127,38 @@ def gru_walks(tmp_path_factory):
     (4096, [64] * 32, 0, 0), (64, [4096], 0, 0), (256, [4096], 0, 0), (44, [2000], 0, 0)])
 def test_gru_walks(gru_walks, C, lens, bf16, f32):
     assert gru_walks(C, *lens) == [bf16, f32]
+
+
+TILES = r"""
+#include <cstdio>
+#include <cstdlib>
+#include "runs.h"
+int main(int n, char** v) {  // heads per key/value head, starts and lengths in turn
+    std::vector<int32_t> starts, lens;
+    for (int i = 2; i < n; i += 2) {
+        starts.push_back(atoi(v[i]));
+        lens.push_back(atoi(v[i + 1]));
+    }
+    for (const pgmi::AttnTile& t : pgmi::attn_tiles(starts.data(), lens.data(), (int)lens.size(), atoi(v[1]), 64)) std::printf("%d %d\n", t.seq, t.first);
+}
+"""
+
+
+@pytest.fixture(scope="module")
+def attn_tiles(tmp_path_factory):
+    at = tmp_path_factory.mktemp("attn_tiles")
+    (at / "ask.cpp").write_text(TILES)
+    subprocess.run(["g++", "-std=c++17", "-Wall", "-Werror", "-I", CSRC, str(at / "ask.cpp"), "-o", str(at / "ask")], check=True)
+    return lambda *a: [tuple(map(int, x.split())) for x in subprocess.run([str(at / "ask"), *map(str, a)], check=True, capture_output=True,
+                                                                          text=True).stdout.splitlines()]
+
+
+@pytest.mark.parametrize("R", [1, 3, 8])
+@pytest.mark.parametrize("seqs", [[(0, 500)], [(7, 1)], [(0, 1024), (0, 387), (0, 129)], [(900, 63), (0, 64), (64, 65), (63, 1), (5, 900)],
+                                  [(2147480000, 640), (0, 640)]])
+def test_attn_tiles(attn_tiles, R, seqs):
+    """Every tile once, in the order of the 64 keys its last position falls in."""
+    got = attn_tiles(R, *(x for s in seqs for x in s))
+    assert sorted(got) == [(r, f) for r, (_, n) in enumerate(seqs) for f in range(0, n * R, 64)]
+    end = [(seqs[r][0] + (min(f + 64, seqs[r][1] * R) - 1) // R) // 64 for r, f in got]
+    assert end == sorted(end)

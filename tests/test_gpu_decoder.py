@@ -164,6 +164,23 @@ def test_gru_in_runs_as_walked(dtype):
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("heads,kv", [(8, 8), (12, 4), (6, 1)])
+@pytest.mark.parametrize("lens", [[700, 33, 900, 129, 500], [64, 1, 65]])
+def test_attention_of_several_prompts(lens, heads, kv, dtype):
+    """More pieces than CUs and fewer, in the order of their keys, as each sequence's alone."""
+    cfg = C.model([C.attn(heads, kv, 16, 16, 300)], width=64, streams=1, groups=1)
+    eng, _ = build(cfg, dtype)
+    seqs = [tokens(cfg, n, 70 + r) for r, n in enumerate(lens)]
+    cache = eng.new_cache(len(lens) + 1, 1024)
+    got = eng.forward(cache, [cache.alloc() for _ in lens], [t for s in seqs for t in s], lens, want=range(sum(lens))).clone()
+    for r, s in enumerate(seqs):
+        alone = cache.alloc()
+        one = eng.forward(cache, [alone], s, [len(s)], want=range(len(s)))
+        cache.free(alone)
+        close(got[sum(lens[:r]):sum(lens[:r + 1])], one.double().cpu().numpy(), dtype)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("name", list(ALL))
 def test_token_by_token(name, dtype):
     cfg = ALL[name]
