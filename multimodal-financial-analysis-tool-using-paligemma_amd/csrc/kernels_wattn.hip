@@ -227,7 +227,7 @@ __global__ void __launch_bounds__(256) k_wattn(WAttnArgs a) {
 // the cache into registers.  Bound by the MFMA's rate and by the longest row's chain of tiles, so a tile of 16 pairs (500
 // positions of 8 heads: 250 workgroups) with its keys dealt to four waves, long rows first.  The K of the wave's next tile is
 // asked for between the two products, its V after them.  k_wattn, dims of 128: 500 positions of 8 heads 105 us, 1,024
-// positions 312; here 24 and 58.
+// positions 312; here 24 and 45.
 __device__ __forceinline__ f32x4 mfma_f32(float a, float b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
 
 // The piece of work, of n pieces with the longest first, that this workgroup takes.  Workgroups b and b + 256 share a CU from the start,
@@ -424,7 +424,7 @@ void run_f(hipStream_t s, const WAttnArgs& a) {
 // Bound, where the chip is full, by LDS (a tile's K and V are read by each of its four waves, 128 KB, and V in halves) and by the
 // score's vector operations; where it is not, by the longest tile's chain of barriers, LDS reads, two products and what is between
 // them, which two teams halve (wattn_teams).  us, 1,300 + 511 + 235 + 2 rows of 16 heads of 128, capped scores: 51.3 before; sums in
-// VGPRs, loads and masks without a branch each 46.2; two teams 39.6.  32 rows a wave, which halves the LDS reads, beat this only for
+// VGPRs, loads and masks without a branch each 46.2; two teams 39.6, tiles in the order of their keys 33.0.  32 rows a wave, which halves the LDS reads, beat this only for
 // one sequence of 4,096 rows (64 against 77) and lost 20 to 40 % below 1,000.
 constexpr size_t wattn_m_lds(int DQ, int DV, int teams) { return (size_t)teams * 64 * (DQ + 8 + DV + 8) * 2; }
 template <int DQ, int DV, int SC, int TEAMS, bool PAD>

@@ -144,9 +144,10 @@ inline std::vector<AttnTile> attn_tiles(const int32_t* starts, const int32_t* le
 
 // Whether a prompt's attention gives each tile of 64 (position, head) pairs to two teams of four waves, which take its 64-key tiles in
 // turn, rather than to one: where the longest tile's chain is what the step waits for, and not the sum of all tiles over the chip (the
-// second team's sums cost LDS and a merge).  us, one team / two, 16 heads of 128 in 2 groups, window 1,024: 1,300 + 511 + 235 + 2 rows
-// 46.2 / 39.6, 1,024 + 387 + 129 rows with distance bias 34.4 / 31.5, 1,300 rows 33.4 / 25.7, 1,540 rows 35.5 / 32.9, 500 rows of 8
-// heads 18.2 / 15.8; 2 x 1,024 rows 35.0 / 39.6, 2,048 rows 45.8 / 48.5, 8 x 512 rows 44.4 / 47.1, 32 x 64 rows 12.5 / 16.1.
+// second team's sums cost LDS and a merge).  us, one team / two, 16 heads of 128 in 2 groups, window 1,024, distance bias, tiles
+// in the order above: 1,300 + 511 + 235 + 2 rows 37.3 / 37.2, 1,024 + 387 + 129 rows 32.5 / 26.2, 1,300 rows 33.1 / 27.0, 600 + 500 rows
+// 21.6 / 18.3, 500 rows of 8 heads 18.1 / 15.5; 2,048 rows 44.1 / 48.2, 8 x 512 rows 37.3 / 46.5, 32 x 64 rows 13.0 / 17.0, 1,411 + 700 +
+// 510 + 256 + 90 rows 38.1 / 45.6.  Of 19 such steps it misses 1,540 rows (36.2 / 33.0) and 4 x 300 (14.6 / 17.6).
 inline bool wattn_teams(const int32_t* starts, const int32_t* lens, int n_seq, int heads, int groups, int window, int keep) {
     const double most = (double)window + keep, R = heads / groups;
     auto keys = [&](double n) { return n <= most ? n * (n + 1) / 2 : most * (most + 1) / 2 + (n - most) * most; };  // of positions 0 .. n - 1
