@@ -439,7 +439,7 @@ __global__ void __launch_bounds__(512) k_scan_walk(ScanArgs a) {
         float S = q.start > 0 && j < N ? s0 : 0.0f;
         __syncthreads();
         for (int i = 0; i < ngr; ++i) {
-            const int k = i & 1, nb = min(NB, (len - i * ROWS + kWalk - 1) / kWalk);
+            const int k = i & 1, rows = min(ROWS, len - i * ROWS);
             struct Block { f32x4 B[4], C[4]; float dt, dx; };
             auto read = [&](int b, Block& o) {
 #pragma unroll
@@ -450,7 +450,9 @@ __global__ void __launch_bounds__(512) k_scan_walk(ScanArgs a) {
                 o.dt = sdt[k][b * kWalk + j][ch];  // lane j has row j of the block
                 o.dx = sdx[k][b * kWalk + j][ch];
             };
-            auto walk = [&](int b, const Block& o) {
+            // n: rows of the block; those past the sequence's end leave the state (their step of 0 does not where A is -inf, nor does
+            // their input of 0 where the last row's B, which they repeat, is not finite)
+            auto walk = [&](auto full, int b, int n, const Block& o) {
                 float e[kWalk], w[kWalk], p[kWalk];
                 each_step([&](auto ti) {  // decays and inputs: none waits for another
                     constexpr int t = decltype(ti)::value;
@@ -460,24 +462,26 @@ __global__ void __launch_bounds__(512) k_scan_walk(ScanArgs a) {
                 __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
                 for (int t = 0; t < kWalk; ++t) {
-                    S = fmaf(e[t], S, w[t]);
+                    const float next = fmaf(e[t], S, w[t]);
+                    S = full || t < n ? next : S;
                     p[t] = S * o.C[t / 4][t % 4];
                 }
                 sy[k][b * kWalk + j][ch] = sum_of_step(p, lane);
             };
             Block o[2];
             read(0, o[0]);
-            if (nb == NB) {
+            if (rows > ROWS - kWalk) {
 #pragma unroll
                 for (int b = 0; b < NB; ++b) {
                     if (b + 1 < NB) read(b + 1, o[(b + 1) & 1]);
-                    walk(b, o[b & 1]);
+                    if (b + 1 < NB || rows == ROWS) walk(std::true_type{}, b, kWalk, o[b & 1]);
+                    else walk(std::false_type{}, b, rows - b * kWalk, o[b & 1]);
                 }
             } else {
 #pragma clang loop unroll(disable)
-                for (int b = 0; b < nb; ++b) {
+                for (int b = 0; b * kWalk < rows; ++b) {
                     if (b) read(b, o[0]);
-                    walk(b, o[0]);
+                    walk(std::false_type{}, b, rows - b * kWalk, o[0]);
                 }
             }
             __syncthreads();

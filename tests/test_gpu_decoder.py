@@ -11,7 +11,7 @@ import pytest
 import torch
 
 import decoder_cases as C
-from decoder_helpers import DTYPES, REPO, TOL, build, close, feed, rel, save, tokens
+from decoder_helpers import DTYPES, REPO, TOL, build, close, feed, oracle, rel, save, tokens
 from oracle import decoder_np as O
 
 pytestmark = pytest.mark.gpu
@@ -121,6 +121,57 @@ def test_scan_of_sequences_walked_whole(inner, states, dtype):
     for r, s in enumerate(seqs):
         i, j = sum(first[:r]), sum(then[:r])
         close(torch.cat([a[i:i + first[r]], b[j:j + then[r]]]), O.run(cfg, W, s), dtype)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("states", [9, 16])
+def test_scan_of_states_that_do_not_last(states, dtype):
+    """A_log = 90, whose decay per step of 1 is not finite in fp32: such a state keeps its last input alone, whether or not the
+    sequence ends with a block of 16 or a stage of 64 rows, and the next portions and single tokens go on from it."""
+    cfg = C.model([C.mamba(48, states, 8, 4)], width=64, streams=1, groups=1)
+    weights = oracle(cfg).random_weights(cfg, 3)
+    name = next(n for n in weights if n.endswith("mix.A_log"))
+    weights[name] = weights[name].copy()
+    weights[name][::3, ::2] = 90.0
+    eng, W = build(cfg, dtype, weights=weights)
+    first, then = [1, 15, 16, 17, 63, 64, 65, 130], [20, 1, 16, 3, 64, 65, 2, 15]
+    seqs = [tokens(cfg, a + b + 2, 90 + r) for r, (a, b) in enumerate(zip(first, then))]
+    cache = eng.new_cache(len(seqs), 256)
+    slots = [cache.alloc() for _ in seqs]
+    a = eng.forward(cache, slots, [t for s, n in zip(seqs, first) for t in s[:n]], first, want=range(sum(first))).clone()
+    b = eng.forward(cache, slots, [t for s, n, m in zip(seqs, first, then) for t in s[n:n + m]], then, want=range(sum(then))).clone()
+    c = [eng.step(cache, slots, [[s[k]] for s in seqs]).clone() for k in (-2, -1)]
+    for r, s in enumerate(seqs):
+        i, j = sum(first[:r]), sum(then[:r])
+        close(torch.cat([a[i:i + first[r]], b[j:j + then[r]], c[0][r:r + 1], c[1][r:r + 1]]), O.run(cfg, W, s), dtype)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("mixer", ["mamba", "gru"])
+def test_walked_sequences_beside_one_that_is_not_finite(mixer, dtype):
+    """A token whose embedding is not a number, last or in the middle of its sequence: what comes before it and the other sequences
+    are what they are without it, what comes after it is no number."""
+    cfg = C.model([C.mamba(48, 16, 8, 4) if mixer == "mamba" else C.gru(48)], width=64, streams=1, groups=1)
+    weights = oracle(cfg).random_weights(cfg, 3)
+    weights["embed"] = weights["embed"].copy()
+    weights["embed"][5] = np.nan
+    eng, _ = build(cfg, dtype, weights=weights)
+    lens, bad = [33, 70, 129, 20], {1: 69, 3: 7}
+    seqs = [[t + 1 if t == 5 else t for t in tokens(cfg, n + 9, 95 + r)] for r, n in enumerate(lens)]
+    got = []
+    for planted in (False, True):
+        cache = eng.new_cache(len(lens), 160)
+        slots = [cache.alloc() for _ in lens]
+        now = [[5 if planted and bad.get(r) == i else t for i, t in enumerate(s)] for r, s in enumerate(seqs)]
+        a = eng.forward(cache, slots, [t for s, n in zip(now, lens) for t in s[:n]], lens, want=range(sum(lens))).clone()
+        b = eng.forward(cache, slots, [t for s, n in zip(now, lens) for t in s[n:]], [9] * len(lens), want=range(9 * len(lens))).clone()
+        got.append([torch.cat([a[sum(lens[:r]):sum(lens[:r + 1])], b[9 * r:9 * r + 9]]) for r in range(len(lens))])
+    for r in range(len(lens)):
+        sound = bad.get(r, lens[r] + 9)
+        finite = torch.isfinite(got[0][r]).all(0)  # (the tied output matrix has the token's row too)
+        assert int(finite.sum()) == cfg["vocab"] - 1
+        assert torch.equal(got[0][r][:sound, finite], got[1][r][:sound, finite])
+        assert torch.isnan(got[1][r][sound:]).all()
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
