@@ -1126,10 +1126,11 @@ static void launch_fs_t(hipStream_t s, const AttnArgs& a, int ns, int tps, dim3 
 
 template <int HD, int NWQ = 0>
 static void launch_fs(hipStream_t s, const AttnArgs& a, int want_ns) {
-    // head dim 256: 4 compute waves (their registers fit 2 waves per SIMD with the loaders, not 3) and a
-    // 5-slot ring (160 KiB) of 32-key tiles; head dim 72: 8 compute waves, 4 slots of 64-key tiles, whose barriers and row maxima
-    // are half as many (of 32 keys in 8 slots a 448 px photo's prefill 0.5 % slower; 5 slots: the same).  NWQ > 0: that many compute waves (fewer
-    // query rows per workgroup, more workgroups over the same keys: probe variants 81 / 82)
+    // head dim 256: 4 compute waves (181 registers: with the loaders 2 waves per SIMD) and a 5-slot ring (160 KiB) of 32-key tiles;
+    // 8 compute waves fit too, 3 waves per SIMD of 168 registers, 4 of which are spilled (20 bytes of scratch a lane).  Head dim 72: 8
+    // compute waves, 4 slots of 64-key tiles, whose barriers and row maxima are half as many as of 32 keys in 8 slots (us, 32 / 64
+    // keys: 1,024 rows and keys of 16 heads 22.8 / 21.4, of four images 57.4 / 51.2, 256 of eight 14.5 / 14.1).
+    // NWQ > 0: that many compute waves
     constexpr int NW = NWQ > 0 ? NWQ : HD == 256 ? 4 : 8, LW = 4, TK = HD == 256 ? 32 : 64, ST = HD == 256 ? 5 : 4;
     const int nrows = a.Lq * a.G, nt = (a.Lk + TK - 1) / TK;
     int ns = fs_splits(a, HD, NW * 16, TK, want_ns);
@@ -1215,9 +1216,11 @@ void attention_prefill(hipStream_t s, int head_dim, const AttnArgs& a) {
     }
     if (v == 9 || v == 91 || v == 92 || v == 94) {  // one pass, keys split over workgroups (auto / 1 / 2 / 4 ranges)
         const int want = v == 9 ? 0 : v - 90;
-        // past 256 workgroups of 64 rows (one a CU), 128 rows each: eight 288-token prompts 288 workgroups, in two rounds, so 144
-        // (with the towers' longer tiles, eight photos' prefill 12,446 -> 12,354 us)
-        if (head_dim == 256 && (long)(a.Lq * a.G + 63) / 64 * a.n_kv * a.B > 256) launch_fs<256, 8>(s, a, want);
+        // A workgroup has a CU to itself.  128 rows take 1.55 to 1.7 times the time of 64, so they are taken where the rounds of the
+        // chip are fewer by more than that.  us, 64 / 128 rows: 8 x 288 rows 25.1 / 19.9 (2 rounds, 1), 2 x 1,056 60.5 / 48.8, 6 x 1,056
+        // 118 / 98 (4, 2), 8 x 1,056 148 / 145 (5, 3); 4 x 1,056 89 / 97 (3, 2), 16 x 288 36.7 / 37.8, 8 x 256 19.5 / 28.1 (1, 1)
+        auto rounds = [&](int rows) { return ((long)(a.Lq * a.G + rows - 1) / rows * a.n_kv * a.B + 255) / 256; };
+        if (head_dim == 256 && 8 * rounds(128) < 5 * rounds(64)) launch_fs<256, 8>(s, a, want);
         else if (head_dim == 256) launch_fs<256>(s, a, want);
         else launch_fs<72>(s, a, want);
         return;

@@ -288,6 +288,18 @@ def test_attention_forced_variant(eng, variant, B, Lq, Lk, H, Hkv, d, scale):
     assert rel_l2(np32(o), _attn_ref(q, k, v, scale)) < 1e-2
 
 
+@pytest.mark.parametrize("variant", [-1, 9, 92, 94])
+@pytest.mark.parametrize("B,Lq,Lk,H,Hkv,d,scale", [
+    # 128 rows a workgroup, where those of 64 would take the chip twice: rows past the last 128, keys inside the last 32, one key
+    (8, 288, 288, 8, 1, 256, 1 / 16), (8, 301, 301, 8, 1, 256, 1 / 16), (9, 257, 290, 8, 1, 256, 0.07), (3, 700, 1000, 8, 1, 256, 1 / 16),
+    (5, 900, 33, 4, 1, 256, 1 / 16), (4, 300, 1, 16, 2, 256, 0.07),
+    # three rounds of 64 rows or two of 128: 64
+    (16, 288, 65, 8, 1, 256, 1 / 16)])
+def test_attention_of_rows_and_keys_past_the_tiles(eng, variant, B, Lq, Lk, H, Hkv, d, scale):
+    """The one-pass kernel's forms at their edges, keys whole and in forced ranges."""
+    test_attention_forced_variant(eng, variant, B, Lq, Lk, H, Hkv, d, scale)
+
+
 @pytest.mark.parametrize("cfg", [36, 37, 39, 40, 41])
 @pytest.mark.parametrize("M,N,K,epi,split", [
     (1056, 512, 2048, "geglu", 1),     # 448 px gate|up shape (rows past 1056: clamped, never stored)
