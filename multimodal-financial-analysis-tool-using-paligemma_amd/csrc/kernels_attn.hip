@@ -1124,14 +1124,14 @@ static void launch_fs_t(hipStream_t s, const AttnArgs& a, int ns, int tps, dim3 
     hipLaunchKernelGGL((k_attn_fs<HD, NW, LW, ST, P2, TK>), grid, dim3(64 * (NW + LW)), lds, s, a, ns, tps);
 }
 
-template <int HD, int NWQ = 0>
+template <int HD, int NWQ = 0, int TKQ = 0>
 static void launch_fs(hipStream_t s, const AttnArgs& a, int want_ns) {
     // head dim 256: 4 compute waves (181 registers: with the loaders 2 waves per SIMD) and a 5-slot ring (160 KiB) of 32-key tiles;
     // 8 compute waves fit too, 3 waves per SIMD of 168 registers, 4 of which are spilled (20 bytes of scratch a lane).  Head dim 72: 8
     // compute waves, 4 slots of 64-key tiles, whose barriers and row maxima are half as many as of 32 keys in 8 slots (us, 32 / 64
     // keys: 1,024 rows and keys of 16 heads 22.8 / 21.4, of four images 57.4 / 51.2, 256 of eight 14.5 / 14.1).
-    // NWQ > 0: that many compute waves
-    constexpr int NW = NWQ > 0 ? NWQ : HD == 256 ? 4 : 8, LW = 4, TK = HD == 256 ? 32 : 64, ST = HD == 256 ? 5 : 4;
+    // NWQ > 0: that many compute waves; TKQ > 0: tiles of that many keys, in as much LDS
+    constexpr int NW = NWQ > 0 ? NWQ : HD == 256 ? 4 : 8, LW = 4, TK = TKQ > 0 ? TKQ : HD == 256 ? 32 : 64, ST = HD == 256 ? 5 : 256 / TK;
     const int nrows = a.Lq * a.G, nt = (a.Lk + TK - 1) / TK;
     int ns = fs_splits(a, HD, NW * 16, TK, want_ns);
     const int tps = (nt + ns - 1) / ns;
@@ -1222,6 +1222,9 @@ void attention_prefill(hipStream_t s, int head_dim, const AttnArgs& a) {
         auto rounds = [&](int rows) { return ((long)(a.Lq * a.G + rows - 1) / rows * a.n_kv * a.B + 255) / 256; };
         if (head_dim == 256 && 8 * rounds(128) < 5 * rounds(64)) launch_fs<256, 8>(s, a, want);
         else if (head_dim == 256) launch_fs<256>(s, a, want);
+        // few keys whose last 64 would be at most half full: tiles of 32 (us, 32 / 64: 8 x 65 keys 6.8 / 7.6, 96 7.3 / 8.3, 160 11.1 /
+        // 12.1, 193 13.7 / 14.0; the same from 257)
+        else if (a.Lk < 224 && (a.Lk + 31) / 32 % 2) launch_fs<72, 0, 32>(s, a, want);
         else launch_fs<72>(s, a, want);
         return;
     }

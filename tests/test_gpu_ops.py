@@ -294,7 +294,11 @@ def test_attention_forced_variant(eng, variant, B, Lq, Lk, H, Hkv, d, scale):
     (8, 288, 288, 8, 1, 256, 1 / 16), (8, 301, 301, 8, 1, 256, 1 / 16), (9, 257, 290, 8, 1, 256, 0.07), (3, 700, 1000, 8, 1, 256, 1 / 16),
     (5, 900, 33, 4, 1, 256, 1 / 16), (4, 300, 1, 16, 2, 256, 0.07),
     # three rounds of 64 rows or two of 128: 64
-    (16, 288, 65, 8, 1, 256, 1 / 16)])
+    (16, 288, 65, 8, 1, 256, 1 / 16),
+    # tiles of 64 keys with 1, 32, 33 and 63 in the last, and of 32
+    (2, 130, 65, 16, 16, 72, 72 ** -0.5), (4, 65, 127, 16, 16, 72, 72 ** -0.5), (8, 100, 128, 16, 16, 72, 0.125), (8, 40, 129, 16, 16, 72, 72 ** -0.5),
+    (8, 64, 160, 16, 16, 72, 72 ** -0.5), (8, 64, 161, 16, 4, 72, 0.125), (6, 64, 193, 16, 16, 72, 72 ** -0.5), (6, 64, 223, 16, 16, 72, 72 ** -0.5),
+    (6, 64, 224, 16, 16, 72, 72 ** -0.5), (6, 64, 225, 16, 16, 72, 72 ** -0.5), (1, 257, 257, 16, 16, 72, 72 ** -0.5), (1, 300, 319, 16, 16, 72, 72 ** -0.5)])
 def test_attention_of_rows_and_keys_past_the_tiles(eng, variant, B, Lq, Lk, H, Hkv, d, scale):
     """The one-pass kernel's forms at their edges, keys whole and in forced ranges."""
     test_attention_forced_variant(eng, variant, B, Lq, Lk, H, Hkv, d, scale)
