@@ -664,7 +664,7 @@ int forward_body(pgmi_ctx* x, hipStream_t s, const int64_t* ids, int rows, const
             a.max_tokens = max_tokens; a.o = d.p2; a.rows = rows; a.seqs = m.seqs; a.nseq = m.nseq; a.row_seq = m.row_seq;
             const auto& t = m.tiles.at(l.heads / l.kv_heads);
             a.tiles = t.first; a.ntile = t.second;
-            a.teams = wattn_teams(m.starts, m.lens, m.nseq, l.heads, l.kv_heads, l.window, l.keep_first);
+            a.teams = wattn_teams(m.starts, m.lens, m.nseq, l.heads, l.kv_heads, l.dim, l.vdim, l.window, l.keep_first);
             wattn_append(s, d.act, a);
             wattn_prefill(s, d.act, a);
             out_proj(w.o, d.p2, a.ldo, w.sub[0]);

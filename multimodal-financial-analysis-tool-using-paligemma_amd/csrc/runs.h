@@ -6,6 +6,7 @@
 #pragma once
 #include <algorithm>
 #include <climits>
+#include <cmath>
 #include <cstdint>
 #include <vector>
 
@@ -143,21 +144,28 @@ inline std::vector<AttnTile> attn_tiles(const int32_t* starts, const int32_t* le
 }
 
 // Whether a prompt's attention gives each tile of 64 (position, head) pairs to two teams of four waves, which take its 64-key tiles in
-// turn, rather than to one: where the longest tile's chain is what the step waits for, and not the sum of all tiles over the chip (the
-// second team's sums cost LDS and a merge).  us, one team / two, 16 heads of 128 in 2 groups, window 1,024, distance bias, tiles
-// in the order above: 1,300 + 511 + 235 + 2 rows 37.3 / 37.2, 1,024 + 387 + 129 rows 32.5 / 26.2, 1,300 rows 33.1 / 27.0, 600 + 500 rows
-// 21.6 / 18.3, 500 rows of 8 heads 18.1 / 15.5; 2,048 rows 44.1 / 48.2, 8 x 512 rows 37.3 / 46.5, 32 x 64 rows 13.0 / 17.0, 1,411 + 700 +
-// 510 + 256 + 90 rows 38.1 / 45.6.  Of 19 such steps it misses 1,540 rows (36.2 / 33.0) and 4 x 300 (14.6 / 17.6).
-inline bool wattn_teams(const int32_t* starts, const int32_t* lens, int n_seq, int heads, int groups, int window, int keep) {
+// turn, rather than to one: by the predicted time, in us of heads of 128 (narrower and wider ones take a like share more or less of every
+// term).  A step takes what its longest tile's chain takes, or what the chip takes for all tiles and keys; two teams halve the chain,
+// but fill a CU (heads of up to 64: half of it), so that tiles past 256 (512) wait for others to end.  Fitted to 627 steps of 1 to 16
+// sequences, 60 to 5,000 rows, heads of 32 to 256, windows of 256 to 4,096: the rule loses 0.3 % of the better form on average, 12 % at
+// most.  us, one team / two, 16 heads of 128 in 2 groups, window 1,024, distance bias: 1,024 + 387 + 129 rows 31.3 / 25.7, 500 rows 18.5 /
+// 16.0, 600 + 500 rows 21.6 / 18.7; 4 x 300 rows 14.5 / 17.5, 8 x 512 rows 37.1 / 46.4, 2,048 rows 46.5 / 50.3; 4 x 130 rows of 32 heads
+// in 8 groups 12.8 / 16.9; heads of 64, 2 x 1,000 rows 23.3 / 19.8.
+inline bool wattn_teams(const int32_t* starts, const int32_t* lens, int n_seq, int heads, int groups, int dim, int vdim, int window, int keep) {
     const double most = (double)window + keep, R = heads / groups;
-    auto keys = [&](double n) { return n <= most ? n * (n + 1) / 2 : most * (most + 1) / 2 + (n - most) * most; };  // of positions 0 .. n - 1
-    double work = 0, longest = 0;  // 64-key tiles
+    auto pairs = [&](double n) { return n <= most ? n * (n + 1) / 2 : most * (most + 1) / 2 + (n - most) * most; };  // of positions 0 .. n - 1
+    double tiles = 0, keys = 0, longest = 0;  // the last two in tiles of 64
     for (int r = 0; r < n_seq; ++r) {
         const double end = (double)starts[r] + lens[r];
-        work += groups * R * ((keys(end) - keys(starts[r])) / 4096 + 0.5 * lens[r] / 64);
-        longest = std::max(longest, std::min(end, most) / 64);
+        tiles += groups * std::ceil(lens[r] * R / 64);
+        keys += groups * R * ((pairs(end) - pairs(starts[r])) / 4096 + 0.5 * lens[r] / 64);
+        longest = std::max(longest, std::ceil(std::min(end, most) / 64) + (end > most));
     }
-    return longest > 2 && longest * kRunCUs >= work;
+    const bool half = dim <= 64 && vdim <= 64;
+    const double one = std::max(6.5 + 1.6 * longest, (2 * tiles + 1.45 * keys) / kRunCUs);
+    const double two = std::max(std::max(7.5 + 2.2 * std::ceil(longest / 2), tiles > (half ? 2 : 1) * kRunCUs ? 2 * (7.5 + 2.2) : 0.0),
+                                ((half ? 4.8 : 7.3) * tiles + 1.25 * keys) / kRunCUs);
+    return two < one;
 }
 
 }  // namespace pgmi

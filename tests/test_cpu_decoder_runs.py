@@ -22,13 +22,19 @@ int main(int n, char** v) {  // channels, states, lengths
 """
 
 
+def compiled(tmp_path_factory, name, source):
+    """The program, as a function of its arguments: the whole numbers of each line that it prints."""
+    at = tmp_path_factory.mktemp(name)
+    (at / "ask.cpp").write_text(source)
+    subprocess.run(["g++", "-std=c++17", "-Wall", "-Werror", "-I", CSRC, str(at / "ask.cpp"), "-o", str(at / "ask")], check=True)
+    return lambda *a: [[int(x) for x in line.split()] for line in subprocess.run([str(at / "ask"), *map(str, a)], check=True, capture_output=True,
+                                                                                 text=True).stdout.splitlines()]
+
+
 @pytest.fixture(scope="module")
 def ask(tmp_path_factory):
-    at = tmp_path_factory.mktemp("runs")
-    (at / "ask.cpp").write_text(ASK)
-    subprocess.run(["g++", "-std=c++17", "-Wall", "-Werror", "-I", CSRC, str(at / "ask.cpp"), "-o", str(at / "ask")], check=True)
-    return lambda *a: [int(x) for x in subprocess.run([str(at / "ask"), *map(str, a)], check=True, capture_output=True,
-                                                      text=True).stdout.split()]
+    run = compiled(tmp_path_factory, "runs", ASK)
+    return lambda *a: run(*a)[0]
 
 
 # channels, states, lengths; the shortest and longest run length of those within 4 % of the best measured
@@ -79,11 +85,8 @@ int main(int n, char** v) {  // channels, states, lengths
 
 @pytest.fixture(scope="module")
 def walks(tmp_path_factory):
-    at = tmp_path_factory.mktemp("walks")
-    (at / "ask.cpp").write_text(WALKS)
-    subprocess.run(["g++", "-std=c++17", "-Wall", "-Werror", "-I", CSRC, str(at / "ask.cpp"), "-o", str(at / "ask")], check=True)
-    return lambda *a: [int(x) for x in subprocess.run([str(at / "ask"), *map(str, a)], check=True, capture_output=True,
-                                                      text=True).stdout.split()]
+    run = compiled(tmp_path_factory, "walks", WALKS)
+    return lambda *a: run(*a)[0]
 
 
 # whole sequences with a lane per state (bf16, fp32) where that was the faster form by more than the rule's error
@@ -113,11 +116,8 @@ int main(int n, char** v) {  // channels, lengths
 
 @pytest.fixture(scope="module")
 def gru_walks(tmp_path_factory):
-    at = tmp_path_factory.mktemp("gru_walks")
-    (at / "ask.cpp").write_text(GRU_WALKS)
-    subprocess.run(["g++", "-std=c++17", "-Wall", "-Werror", "-I", CSRC, str(at / "ask.cpp"), "-o", str(at / "ask")], check=True)
-    return lambda *a: [int(x) for x in subprocess.run([str(at / "ask"), *map(str, a)], check=True, capture_output=True,
-                                                      text=True).stdout.split()]
+    run = compiled(tmp_path_factory, "gru_walks", GRU_WALKS)
+    return lambda *a: run(*a)[0]
 
 
 # minGRU's sequences walked whole (bf16, fp32) where that was the faster form by more than the rule's error
@@ -146,11 +146,8 @@ int main(int n, char** v) {  // heads per key/value head, starts and lengths in 
 
 @pytest.fixture(scope="module")
 def attn_tiles(tmp_path_factory):
-    at = tmp_path_factory.mktemp("attn_tiles")
-    (at / "ask.cpp").write_text(TILES)
-    subprocess.run(["g++", "-std=c++17", "-Wall", "-Werror", "-I", CSRC, str(at / "ask.cpp"), "-o", str(at / "ask")], check=True)
-    return lambda *a: [tuple(map(int, x.split())) for x in subprocess.run([str(at / "ask"), *map(str, a)], check=True, capture_output=True,
-                                                                          text=True).stdout.splitlines()]
+    run = compiled(tmp_path_factory, "attn_tiles", TILES)
+    return lambda *a: [tuple(line) for line in run(*a)]
 
 
 @pytest.mark.parametrize("R", [1, 3, 8])
@@ -162,3 +159,40 @@ def test_attn_tiles(attn_tiles, R, seqs):
     assert sorted(got) == [(r, f) for r, (_, n) in enumerate(seqs) for f in range(0, n * R, 64)]
     end = [(seqs[r][0] + (min(f + 64, seqs[r][1] * R) - 1) // R) // 64 for r, f in got]
     assert end == sorted(end)
+
+
+TEAMS = r"""
+#include <cstdio>
+#include <cstdlib>
+#include "runs.h"
+int main(int n, char** v) {  // heads, key/value heads, width, window, kept, starts and lengths in turn
+    std::vector<int32_t> starts, lens;
+    for (int i = 6; i < n; i += 2) {
+        starts.push_back(atoi(v[i]));
+        lens.push_back(atoi(v[i + 1]));
+    }
+    std::printf("%d\n", (int)pgmi::wattn_teams(starts.data(), lens.data(), (int)lens.size(), atoi(v[1]), atoi(v[2]), atoi(v[3]), atoi(v[3]), atoi(v[4]),
+                                               atoi(v[5])));
+}
+"""
+
+
+@pytest.fixture(scope="module")
+def teams(tmp_path_factory):
+    return compiled(tmp_path_factory, "teams", TEAMS)
+
+
+# steps whose better form was measured to be so by more than the rule's error
+@pytest.mark.parametrize("H,G,d,window,keep,lens,two", [
+    (16, 2, 128, 1024, 0, [1024, 387, 129], 1), (16, 2, 128, 1024, 0, [500], 1), (16, 2, 128, 1024, 16, [600, 500], 1),
+    (8, 2, 128, 1024, 0, [2048], 1), (16, 2, 64, 1024, 0, [1000] * 2, 1), (16, 2, 256, 1024, 0, [500], 1), (8, 8, 256, 1024, 0, [400] * 3, 1),
+    (8, 2, 128, 1024, 0, [1411, 700, 510, 256, 90], 1),
+    (16, 2, 128, 1024, 0, [300] * 4, 0), (32, 8, 128, 1024, 0, [130] * 4, 0), (16, 2, 128, 256, 0, [600, 500], 0), (16, 2, 128, 1024, 0, [512] * 8, 0),
+    (16, 2, 128, 1024, 0, [4096], 0), (16, 2, 256, 1024, 0, [300] * 4, 0), (16, 2, 128, 256, 0, [1540], 0), (32, 8, 128, 1024, 0, [1024, 387, 129], 0),
+    (16, 2, 64, 1024, 0, [512] * 8, 0), (16, 2, 128, 1024, 0, [60], 0)])
+def test_teams(teams, H, G, d, window, keep, lens, two):
+    assert teams(H, G, d, window, keep, *(x for n in lens for x in (0, n))) == [[two]]
+
+
+def test_teams_of_huge_steps(teams):
+    assert teams(8, 1, 128, 2147483647, 2147483647, 2147480000, 640) in ([[0]], [[1]])
