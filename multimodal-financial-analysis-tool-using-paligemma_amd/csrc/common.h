@@ -69,13 +69,9 @@ __device__ __forceinline__ uint4 ldg_nt(const void* p) {
     return make_uint4(v.x, v.y, v.z, v.w);
 }
 
+// Read as one vector: of a uint4 read word by word, joined again for a matrix instruction and carried around a loop, hipcc (ROCm 7.2)
+// has given words to another value while they were needed (few-row experts' weights: its IR was right, its registers not)
 __device__ __forceinline__ uint4 ldg16(const void* p) {
-    return *reinterpret_cast<const uint4*>(p);
-}
-
-// The same as one vector for fragments that are carried around a loop: hipcc reads a uint4 as four words, joins them again, and has
-// then lost three of them to another register's use (few-row experts' weights, ROCm 7.2; its IR was right, its assembly not)
-__device__ __forceinline__ uint4 ldv16(const void* p) {
     const u32x4 v = *reinterpret_cast<const u32x4*>(p);
     return make_uint4(v.x, v.y, v.z, v.w);
 }

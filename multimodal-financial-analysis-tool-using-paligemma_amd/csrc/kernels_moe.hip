@@ -366,7 +366,7 @@ __global__ void __launch_bounds__(256) k_experts_skinny(ExpertArgs a) {
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int li = lane & 15, lg = lane >> 4;
     auto ld = [](const uint16_t* p, bool in, const uint16_t* safe) {
-        if constexpr (WHOLE) return ldv16(p);
+        if constexpr (WHOLE) return ldg16(p);
         else return ldg16_sel(p, in, safe);
     };
     const uint16_t* wp[NM];

@@ -454,7 +454,7 @@ __global__ void __launch_bounds__(256 * TEAMS) k_wattn_m(WAttnArgs a) {
     const int i = sq.start + prow;
     auto ld = [](const uint16_t* p, bool in, const uint16_t* safe) {  // (the choice is a branch around every load)
         if constexpr (PAD) return ldg16_sel(p, in, safe);
-        else return ldv16(p);
+        else return ldg16(p);
     };
     const uint16_t* qp = reinterpret_cast<const uint16_t*>(a.q) + ((long)(sq.off + prow) * w.H + h) * w.dp;
     short8 qf[DQ / 32];
@@ -843,7 +843,7 @@ __global__ void __launch_bounds__(256, DQ <= 64 && DV <= 64 && HEADS != ODD ? 4 
     constexpr bool VEC = HEADS != ODD, FULL = HEADS == WHOLE;
     const int dp = FULL ? DQ : w.dp, ep = FULL ? DV : w.ep, qd = FULL ? DQ : w.d, ve = FULL ? DV : w.e;
     auto ld = [](const uint16_t* p, bool in, const uint16_t* safe) {  // (the choice is a branch around every load)
-        if constexpr (FULL) return ldv16(p);
+        if constexpr (FULL) return ldg16(p);
         else return ldg16_sel(p, in, safe);
     };
     constexpr int VS = DV + 8;
