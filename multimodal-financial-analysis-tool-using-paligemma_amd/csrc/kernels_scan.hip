@@ -416,12 +416,27 @@ __device__ __forceinline__ float sum_of_step(const float (&p)[kWalk], int lane) 
     return (o2 ? c1 : c0) + other(o2 ? c0 : c1, X2{});
 }
 
+__device__ __forceinline__ float sum_of_lanes(float v) {  // of a channel's 16
+    auto turned = [](float x, auto by) {
+        return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x120 + decltype(by)::value, 0xF, 0xF, true));
+    };
+    v += turned(v, std::integral_constant<int, 8>{});
+    v += turned(v, std::integral_constant<int, 4>{});
+    v += turned(v, std::integral_constant<int, 2>{});
+    return v + turned(v, std::integral_constant<int, 1>{});
+}
+
 // Four waves walk 16 channels, four others have the rest: they fetch the rows (asked for 64 rows ahead of their use), form the
 // steps and inputs of the next 64 rows while these are walked, and gate and store the 64 rows before.  V4: such a thread has four
 // channels of one row, else one channel of four rows.  WHOLE: 16 states.
 template <typename T, bool V4, bool WHOLE>
 __global__ void __launch_bounds__(512) k_scan_walk(ScanArgs a) {
     constexpr int ROWS = 64, LD = ROWS + 4, NB = ROWS / kWalk, CD = kWalk + 4;  // strides of B | C's columns, of a row's channels
+    // fp32: the state goes from block to block by one decay over the sum of the block's steps, as it does from run to run.  Error against
+    // 64 bits, 500 rows of 2,048 channels, outputs / state: runs 1.10e-7 / 1.02e-7, step by step 1.20e-7 / 1.25e-7, so 1.10e-7 /
+    // 0.98e-7 (a 500-token prompt 0.6 % longer).  bf16 rows round 10,000 times as much: 40 prompts' and steps' error 1.001 +- 0.006 of
+    // that of runs.
+    constexpr bool LEAP = sizeof(T) == 4;
     __shared__ __attribute__((aligned(16))) float sbc[2][2 * kWalk][LD], sdt[2][ROWS][CD], sdx[2][ROWS][CD], sy[2][ROWS][CD];
     const SeqInfo q = a.seqs[blockIdx.y];
     // an XCD's workgroups have neighbouring channels, which share the lines of every row
@@ -460,13 +475,17 @@ __global__ void __launch_bounds__(512) k_scan_walk(ScanArgs a) {
                     w[t] = of_step<t>(o.dx) * o.B[t / 4][t % 4];
                 }, std::make_integer_sequence<int, kWalk>{});
                 __builtin_amdgcn_sched_barrier(0);
+                const float entry = S;
+                float own = 0.0f;  // the block's state from its own inputs
 #pragma unroll
                 for (int t = 0; t < kWalk; ++t) {
-                    const float next = fmaf(e[t], S, w[t]);
-                    S = full || t < n ? next : S;
+                    const bool there = full || t < n;
+                    S = there ? fmaf(e[t], S, w[t]) : S;
+                    if constexpr (LEAP) own = there ? fmaf(e[t], own, w[t]) : own;
                     p[t] = S * o.C[t / 4][t % 4];
                 }
                 sy[k][b * kWalk + j][ch] = sum_of_step(p, lane);
+                if constexpr (LEAP) S = fmaf(__builtin_amdgcn_exp2f(sum_of_lanes(o.dt) * A), entry, own);
             };
             Block o[2];
             read(0, o[0]);

@@ -78,13 +78,14 @@ inline ScanStep scan_step_of(const int32_t* lens, int n_seq, int run_rows) {
 // with a lane per channel (k_scan: twice, three launches): by the predicted time, in us.  A walk takes what its longest sequence
 // takes alone, or what the chip takes for all of them (a CU's share of the workgroups, each with its start and its steps); runs take
 // their launches, the rows' traffic, the rounds of rows walked one after the other and the carries.  The constants are fitted to 196
-// steps of 64 to 8,192 channels and 33 to 4,096 rows: the rule loses 0.1 % of the better form on average, 8 % at most.  us a
+// steps of 64 to 8,192 channels and 33 to 4,096 rows: the rule loses 0.2 % of the better form on average, 22 % at most (runs kept for 700
+// fp32 rows of 64 channels), and no walk that it takes is slower than runs by more than 1.3 %.  us a
 // layer, runs / walk: 1,024 + 387 + 129 rows of 4,096 channels 70.0 / 37.1, 512 rows 33.7 / 15.7, 8 x 512 rows 145 / 87, 500 rows of
-// 2,048 fp32 channels 32.3 / 20.6; 4,096 rows of 2,048 channels 83 / 113, 64 x 33 rows of 4,096 50 / 103.
+// 2,048 fp32 channels 31.3 / 21.1; 4,096 rows of 2,048 channels 83 / 113, 64 x 33 rows of 4,096 50 / 116.
 inline bool scan_walks(const ScanStep& s, int C, int N, bool f32) {
     if (N <= 8 || N > 16) return false;
     const double per_cu = (C + 15) / 16 / (double)kRunCUs;
-    const double walk = (f32 ? 5 : 3) + std::max((f32 ? 0.033 : 0.024) * s.longest,
+    const double walk = (f32 ? 5 : 3) + std::max((f32 ? 0.035 : 0.024) * s.longest,
                                                  per_cu * (0.5 * s.n_seq + (f32 ? 0.029 : 0.023) * (double)s.padded));
     const double rounds = (double)((s.runs * ((C + 255) / 256) + kRunCUs - 1) / kRunCUs);
     const double runs = s.most_runs == 1 ? 10 + rounds * s.run_rows * (f32 ? 0.44 : 0.3)
