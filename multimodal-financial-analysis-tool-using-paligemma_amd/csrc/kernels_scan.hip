@@ -763,11 +763,22 @@ __global__ void __launch_bounds__(64) k_gru_carry(GruArgs a) {
 }
 
 // ---- sequences walked whole: one wave has 16 channels' states, eight others the rest
-// A step of the walk is one FMA behind the step before; the gates, candidates and outputs of 128 rows are formed around it, ahead of it
-// and after it, as in k_scan_walk.  V4: a thread of the eight waves has four channels of one row, else one channel of four rows.
-// Bound by those waves' three sigmoids a value, two waves a SIMD: 8 ns a row of the longest sequence (four waves and 64 rows 18, rows held
-// one group ahead or two alike).  us a layer, three launches of runs / this: 1,024 + 387 + 129 rows of 2,048 channels 21.6 / 13.5, 500
-// rows of 1,024 fp32 channels 14.7 / 7.7; the line between them: gru_walks.
+// The gates, candidates and outputs of 128 rows are formed around the walk, ahead of it and after it, as in k_scan_walk.  V4: a thread of
+// the eight waves has four channels of one row, else one channel of four rows.
+// The walking wave takes 32 rows at a time, as runs of 8 side by side: what each leaves by itself and keeps, the state before each from
+// these, then its rows.  Row after row instead, the roundings of a whole sequence add up: error against 64 bits, 500 fp32 rows, gates of
+// sigmoid(-4), outputs / state, of that of three launches over runs 1.08 / 1.13, as it is now 0.99 / 1.00.
+// Bound by the other waves' three sigmoids a value, two waves a SIMD: 8 ns a row of the longest sequence (four waves and 64 rows 18, rows held
+// one group ahead or two alike).  us a layer, three launches of runs / this: 1,024 + 387 + 129 rows of 2,048 channels 21.7 / 12.6, 500
+// rows of 1,024 fp32 channels 14.7 / 6.8; the line between them: gru_walks.
+
+// v of lanes 0 .. 15, 16 .. 31, 32 .. 47 and 48 .. 63, in all four
+__device__ __forceinline__ void of_parts(float v, float (&o)[4]) {
+    const unsigned u = __float_as_uint(v);
+    const auto a = __builtin_amdgcn_permlane16_swap(u, u, false, false);  // of the even parts, of the odd ones
+    const auto b = __builtin_amdgcn_permlane32_swap(a[0], a[0], false, false), c = __builtin_amdgcn_permlane32_swap(a[1], a[1], false, false);
+    o[0] = __uint_as_float(b[0]), o[1] = __uint_as_float(c[0]), o[2] = __uint_as_float(b[1]), o[3] = __uint_as_float(c[1]);
+}
 template <typename T, bool V4>
 __global__ void __launch_bounds__(576) k_gru_walk(GruArgs a) {
     constexpr int ROWS = 128, LD = ROWS + 4;
@@ -778,36 +789,66 @@ __global__ void __launch_bounds__(576) k_gru_walk(GruArgs a) {
     const int len = q.len, ngr = (len + ROWS - 1) / ROWS;
     if (c0 >= max(a.C, a.ldy)) return;
     if (threadIdx.x >= 512) {
-        const int ch = threadIdx.x & 15, c = c0 + ch;
-        const bool mine = threadIdx.x < 512 + kWalk && c < a.C;
+        // 8 of 32 rows each: lanes 0 .. 15 the first, 16 .. 31 the next, ..
+        const int ch = threadIdx.x & 15, part = (threadIdx.x & 63) >> 4, c = c0 + ch;
+        const bool mine = c < a.C;
         float* st = a.state + (long)q.slot * a.C + min(c, a.C - 1);
         float S = q.start > 0 ? *st : 0.0f;
         __syncthreads();
         for (int i = 0; i < ngr; ++i) {
-            const int k = i & 1;
-            if (mine) {
-                // 32 rows' operands before their chain, so that it waits for no read but the first
+            const int k = i & 1, rows = len - i * ROWS;
+            struct Piece { f32x4 a[2], b[2]; float own, kept; };  // what 8 rows leave of no state, and keep of one
+            auto read = [&](int h, Piece& w) {
 #pragma unroll
-                for (int h = 0; h < ROWS; h += 32) {  // rows past the end keep the state
-                    if (h >= len - i * ROWS) break;
-                    f32x4 va[8], vb[8];
+                for (int r = 0; r < 2; ++r) {
+                    w.a[r] = *reinterpret_cast<const f32x4*>(&sa[k][ch][h + 8 * part + 4 * r]);
+                    w.b[r] = *reinterpret_cast<const f32x4*>(&sb[k][ch][h + 8 * part + 4 * r]);
+                }
+            };
+            auto sum = [&](Piece& w) {
+                w.own = 0.0f, w.kept = 1.0f;
 #pragma unroll
-                    for (int r = 0; r < 8; ++r) {
-                        va[r] = *reinterpret_cast<const f32x4*>(&sa[k][ch][h + 4 * r]);
-                        vb[r] = *reinterpret_cast<const f32x4*>(&sb[k][ch][h + 4 * r]);
-                    }
-                    __builtin_amdgcn_sched_barrier(0);
+                for (int r = 0; r < 8; ++r) {
+                    w.own = fmaf(w.a[r / 4][r % 4], w.own, w.b[r / 4][r % 4]);
+                    w.kept *= w.a[r / 4][r % 4];
+                }
+            };
+            auto walk = [&](int h, Piece& w) {
+                float o[4], f[4], e = S;
+                of_parts(w.own, o);
+                of_parts(w.kept, f);
 #pragma unroll
-                    for (int r = 0; r < 8; ++r) {
+                for (int n = 0; n < 4; ++n) {
+                    if (part == n) e = S;
+                    S = fmaf(f[n], S, o[n]);
+                }
+                const int at = h + 8 * part;
 #pragma unroll
-                        for (int e = 0; e < 4; ++e) vb[r][e] = S = fmaf(va[r][e], S, vb[r][e]);
-                        *reinterpret_cast<f32x4*>(&ss[k][ch][h + 4 * r]) = vb[r];
-                    }
+                for (int r = 0; r < 2; ++r) {
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) w.b[r][v] = e = fmaf(w.a[r][v], e, w.b[r][v]);
+                    *reinterpret_cast<f32x4*>(&ss[k][ch][at + 4 * r]) = w.b[r];
+                }
+                if (mine && at < rows && at + 8 >= rows) *st = e;  // the sequence's last row
+            };
+            Piece w[ROWS / 32];
+            if (rows > ROWS - 32) {
+#pragma unroll
+                for (int n = 0; n < ROWS / 32; ++n) read(32 * n, w[n]);
+#pragma unroll
+                for (int n = 0; n < ROWS / 32; ++n) sum(w[n]);
+#pragma unroll
+                for (int n = 0; n < ROWS / 32; ++n) walk(32 * n, w[n]);
+            } else {
+#pragma clang loop unroll(disable)
+                for (int h = 0; h < rows; h += 32) {  // rows past the end keep the state
+                    read(h, w[0]);
+                    sum(w[0]);
+                    walk(h, w[0]);
                 }
             }
             __syncthreads();
         }
-        if (mine) *st = S;
         return;
     }
     typedef T T4 __attribute__((ext_vector_type(4)));

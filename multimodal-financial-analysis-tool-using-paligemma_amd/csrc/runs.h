@@ -109,10 +109,10 @@ inline int gru_run_rows(const int32_t* lens, int n_seq, long columns) {
 }
 
 // Whether a minGRU layer walks its sequences whole (k_gru_walk, one launch) rather than in the runs above: as scan_walks, by the
-// predicted time in us, fitted to 180 steps of 44 to 4,096 channels and 17 to 4,096 rows; it loses 1.1 % of the better form on average,
-// mostly at 64 x 33 rows of 256 channels (9 instead of 7).  us a layer, runs / walk: 1,024 + 387 + 129 rows of 2,048 channels 21.6 / 13.5,
-// 500 rows of 1,024 fp32 channels 14.7 / 7.7, 60 rows of 2,048 10.9 / 5.6, 8 x 512 rows 29.8 / 25.1; 64 x 33 rows 11.0 / 40, 4,096
-// rows of 1,024 channels 30 / 38.
+// predicted time in us, fitted to 180 steps of 44 to 4,096 channels and 17 to 4,096 rows.  It leans to the runs: it loses 1.8 % of the
+// better form on average, up to 37 % where runs are kept for 2,000 rows of up to 256 channels, and 12 % at most where a walk is taken
+// (4,096 fp32 rows of 2,048 channels).  us a layer, runs / walk: 1,024 + 387 + 129 rows of 2,048 channels 21.7 / 12.6, 500 rows of 1,024 fp32
+// channels 14.7 / 6.8, 60 rows of 2,048 11.0 / 5.7, 8 x 512 rows 30.1 / 22.5; 64 x 33 rows 10.9 / 40, 4,096 rows of 1,024 channels 30 / 34.
 inline bool gru_walks(const ScanStep& s, int C, bool f32) {
     const double per_cu = (C + 15) / 16 / (double)kRunCUs, traffic = (f32 ? 3.4e-6 : 1.65e-6) * C * (double)s.rows;
     const double walk = 4.5 + std::max(0.008 * s.longest, per_cu * (0.5 * s.n_seq + (f32 ? 0.0135 : 0.0095) * (double)s.padded));

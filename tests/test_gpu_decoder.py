@@ -174,11 +174,11 @@ def test_walked_sequences_beside_one_that_is_not_finite(mixer, dtype):
         assert torch.isnan(got[1][r][sound:]).all()
 
 
-@pytest.mark.parametrize("mixer,width,rows,seed,most", [("mamba", 512, 700, 3, 5.5e-7)])
+@pytest.mark.parametrize("mixer,width,rows,seed,most", [("mamba", 512, 700, 3, 5.5e-7), ("gru", 512, 900, 4, 1.3e-6)])
 def test_walked_states_that_last(mixer, width, rows, seed, most):
     """fp32 states that last for hundreds of rows, whose roundings add up: the error of the last 100 rows' logits, rms, mean over the
-    rows.  Scan: 3.6e-7 in runs and as it is walked, of which 3.4e-7 are the products around it; 7.8e-7 step by step.  The bound lies
-    half way."""
+    rows.  Scan: 3.6e-7 in runs and as it is walked, of which 3.4e-7 are the products around it; 7.8e-7 step by step.  minGRU: 8.5e-7 as
+    it is walked, 1.7e-6 row by row.  The bounds lie half way."""
     cfg = C.model([C.mamba(width, 16, 8, 4) if mixer == "mamba" else C.gru(width)], width=64, streams=1, groups=1)
     weights = oracle(cfg).random_weights(cfg, seed)
     for name in weights:
