@@ -96,8 +96,7 @@ def test_layers_and_logits_of_a_prompt(name, dtype):
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("inner,dt_rank,rows", [(1032, 24, 600), (2048, 64, 1301)])
 def test_steps_and_scan_of_many_rows(inner, dt_rank, rows, dtype):
-    """The step sizes' product on the tiles that many rows take (one with columns past the last tile), runs of whole and broken
-    blocks of rows."""
+    """The step sizes' product on the tiles that many rows take (one with columns past the last tile), and their scan."""
     cfg = C.model([C.mamba(inner, 16, dt_rank, 4)], width=64, streams=1, groups=1)
     eng, W = build(cfg, dtype)
     toks = tokens(cfg, rows, 5)
@@ -195,9 +194,10 @@ def test_walked_states_that_last(mixer, width, rows, seed, most):
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
-def test_scan_in_runs_as_walked(dtype):
-    """2,300 rows of few channels go in runs; in portions of 230 they are walked."""
-    cfg = C.model([C.mamba(64, 16, 8, 4)], width=64, streams=1, groups=1)
+@pytest.mark.parametrize("inner", [64, 1032])
+def test_scan_in_runs_as_walked(inner, dtype):
+    """2,300 rows of few channels go in runs, with whole and broken blocks of rows; in portions of 230 they are walked."""
+    cfg = C.model([C.mamba(inner, 16, 8, 4)], width=64, streams=1, groups=1)
     eng, _ = build(cfg, dtype)
     toks = tokens(cfg, 2300, 9)
     cache = eng.new_cache(2, 2304)

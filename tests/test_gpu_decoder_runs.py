@@ -1,5 +1,5 @@
 """The recurrences' run lengths (rows one workgroup walks) follow the step's size: sequences read together, in steps large enough
-for each run length, against the same sequences alone, whose runs are the shortest."""
+for each run length, against the same sequences alone, whose runs are the shortest or which are walked whole."""
 import numpy as np
 import pytest
 import torch
@@ -10,12 +10,18 @@ from decoder_helpers import build, tokens
 pytestmark = pytest.mark.gpu
 
 
-# (sequences, tokens each): runs of the scan of 64, 50, 36, 32, 30, 22, 18 and 16 rows at these models' widths, of minGRU of 32, 24, 16
-# and 8, and past 16,384 rows of 256 and 128
+# The scans of MIXED have 9 to 16 states, and these steps walk their sequences whole, as they do minGRU's; those of other numbers of states
+# go in runs.
+MODELS = {**C.MIXED, "runs": C.model([C.mamba(72, 8, 6, 3), C.gru(44), C.attn(6, 3, 24, 36, 40, ff=100), C.mamba(40, 20, 3, 5, ff=28)],
+                                     width=84, streams=2, groups=3, vocab=211)}
+
+
+# (sequences, tokens each): runs of the scan of 64, 50, 36, 32, 30, 22, 18 and 16 rows at these models' widths, and past 16,384 rows of
+# 256
 @pytest.mark.parametrize("n,length", [(36, 450), (30, 400), (20, 450), (3, 97), (40, 430), (36, 448), (16, 450), (12, 450), (10, 450)])
-@pytest.mark.parametrize("name", sorted(C.MIXED))
+@pytest.mark.parametrize("name", sorted(MODELS))
 def test_together_as_alone(name, n, length):
-    cfg = C.MIXED[name]
+    cfg = MODELS[name]
     eng, _ = build(cfg, "float32", max_batch=64)
     lens = [length - 7 * (r % 5) for r in range(n)]
     seqs = [tokens(cfg, k + 1, 200 + r) for r, k in enumerate(lens)]
@@ -50,9 +56,11 @@ def test_time_goes_by_the_states():
     assert times[1] <= 2.5 * times[0]
 
 
-def test_a_shorter_step_of_more_runs_allocates_nothing():
-    """9,081 rows of 4,096 channels go in 142 runs, 8,942 in 160: the workspace of the first holds the second."""
-    eng, _ = build(C.model([C.mamba(4096, 16, 8, 4)], width=64, vocab=64, streams=1, groups=1), "bfloat16")
+@pytest.mark.parametrize("states", [8, 16])
+def test_a_shorter_step_of_more_runs_allocates_nothing(states):
+    """9,081 rows of 4,096 channels of 8 states go in 142 runs, 8,942 in 160: the workspace of the first holds the second.  (Of 16 states
+    both are walked whole and carry nothing.)"""
+    eng, _ = build(C.model([C.mamba(4096, states, 8, 4)], width=64, vocab=64, streams=1, groups=1), "bfloat16")
     cache = eng.new_cache(1, 9200)
     slot, toks = cache.alloc(), torch.arange(9081, device="cuda") % 64
     free = []
@@ -64,9 +72,10 @@ def test_a_shorter_step_of_more_runs_allocates_nothing():
     assert free[0] == free[1]
 
 
-def test_captured_steps_outlive_more_runs():
-    """A decode graph, then a packed step of as many rows in more runs, then the graph again: as eager steps."""
-    cfg = C.MIXED["a"]
+@pytest.mark.parametrize("name", ["a", "runs"])
+def test_captured_steps_outlive_more_runs(name):
+    """A decode graph, then a packed step of as many rows in more runs (of "a", walked whole), then the graph again: as eager steps."""
+    cfg = MODELS[name]
     eng, _ = build(cfg, "bfloat16", max_batch=64)
     out = []
     for graph in (True, False):
