@@ -1095,16 +1095,15 @@ int pgmi_decoder_forward(pgmi_ctx* x, const int64_t* ids, int n_seq, const int32
     const bool huge = rows > 16384;
     Cut scan{0, 0, false}, gru = scan, conv = scan;
     ScanStep step, gru_step;
-    if (scan_cols) {
-        const int run = huge ? 256 : scan_run_rows(lens, n_seq, scan_cols, scan_wgs);
-        scan = cut(run);
-        step = scan_step_of(lens, n_seq, run);
+    if (scan_cols) step = scan_step_of(lens, n_seq, huge ? 256 : scan_run_rows(lens, n_seq, scan_cols, scan_wgs));
+    if (gru_cols) gru_step = scan_step_of(lens, n_seq, huge ? 128 : gru_run_rows(lens, n_seq, gru_cols));
+    bool scan_runs = false, gru_runs = false;  // layers that walk their sequences read no runs
+    for (const pgmi_layer_spec& l : d.L) {
+        scan_runs |= l.mixer == PGMI_MIXER_MAMBA1 && !scan_walks(step, l.inner, l.state, d.act == ACT_F32);
+        gru_runs |= l.mixer == PGMI_MIXER_MINGRU && !gru_walks(gru_step, l.width, d.act == ACT_F32);
     }
-    if (gru_cols) {
-        const int run = huge ? 128 : gru_run_rows(lens, n_seq, gru_cols);
-        gru = cut(run);
-        gru_step = scan_step_of(lens, n_seq, run);
-    }
+    if (scan_runs) scan = cut(step.run_rows);
+    if (gru_runs) gru = cut(gru_step.run_rows);
     // the convolutions carry nothing: 500 rows of 2,048 channels 11.2 us on 64-row runs, 5.9 on 16; 2,048 rows 10.8 / 7.5
     if (scan_cols || d.c.canon_taps > 0) conv = cut(huge ? 256 : rows > 2048 ? 32 : 16);
     struct Tiles { int R; size_t o; int n; };
