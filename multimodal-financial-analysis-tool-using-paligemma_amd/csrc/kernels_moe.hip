@@ -466,6 +466,8 @@ void experts_skinny(hipStream_t s, ExpertMode mode, const ExpertArgs& a) {
     const dim3 grid((n + 15) / 16, 1 + (a.B == 1 ? a.entries : std::min(a.experts, a.entries)));
     // one row has too few workgroups to cover the memory's latency with four steps: 25.0 -> 20.5 us (width 2048, 6 + 1
     // experts); with more rows, or the shorter rows of the down product, eight are slower
+    // (K of 512 times an odd number, two steps whole instead of four chosen: a step of eight rows over experts of 512 of the 1,024-wide
+    // model 498 us for 504, of one row 349 for 350)
     auto whole = [&](int steps) { return a.K % (256 * steps) == 0 && (!a.Wsh || a.Ksh % (256 * steps) == 0); };
 #define SKINNY_(mode, u, w) hipLaunchKernelGGL((k_experts_skinny<mode, u, w>), grid, dim3(256), 0, s, a)
     if (mode == EX_SWIGLU) {

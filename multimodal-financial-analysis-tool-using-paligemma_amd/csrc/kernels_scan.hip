@@ -372,11 +372,12 @@ __global__ void __launch_bounds__(256) k_scan_carry(ScanArgs a) {
 }
 
 // ---- sequences walked whole, a lane per state
-// What bounds it: one wave a SIMD has 64 states of one sequence, and issues an instruction every 4.5 to 5.5 clocks (8.4 an exponential)
-// however independent they are; a step is one exponential, two products with a value of the channel (broadcast within the
-// instruction, DPP), an FMA, a product with C and two additions of the sum over the states: 25 ns of the longest sequence's step,
-// 18 of them those instructions'.  So everything else is another four waves' work.  One wave for both: 36 ns; with its loads and
-// stores straight from memory, 16 rows of 4 channels an instruction, 43.  us a layer: see scan_walks.
+// Bound by the vector units: an instruction of 64 lanes takes a SIMD of 16 four clocks (measured 4.5 to 5.5, an exponential 8.4), so that
+// walking waves which share a SIMD gain nothing: a step takes a CU's share of all rows, or its longest sequence's where that is
+// longer.  It is one exponential, two products with a value of the channel (broadcast within the instruction, DPP), an FMA (fp32:
+// two), a product with C and two additions of the sum over the states: 24 ns a row (fp32 35), 18 of them those instructions'.  So
+// everything else is another four waves' work.  One wave for both: 36 ns; with its loads and stores straight from memory, 16 rows
+// of 4 channels an instruction, 43.  us a layer: see scan_walks.
 constexpr int kWalk = 16;  // channels of a workgroup, lanes of a channel, and rows of a block
 
 // step t's value of a channel's 16 lanes
@@ -779,6 +780,7 @@ __device__ __forceinline__ void of_parts(float v, float (&o)[4]) {
     const auto b = __builtin_amdgcn_permlane32_swap(a[0], a[0], false, false), c = __builtin_amdgcn_permlane32_swap(a[1], a[1], false, false);
     o[0] = __uint_as_float(b[0]), o[1] = __uint_as_float(c[0]), o[2] = __uint_as_float(b[1]), o[3] = __uint_as_float(c[1]);
 }
+
 template <typename T, bool V4>
 __global__ void __launch_bounds__(576) k_gru_walk(GruArgs a) {
     constexpr int ROWS = 128, LD = ROWS + 4;
