@@ -3,9 +3,9 @@
  *
  * This is the drop-in boundary below the reference's Python API
  * (PaliGemmaForConditionalGeneration / SiglipVisionModel / GemmaForCausalLM / KVCache in
- * /root/reference/modeling_gemma.py and modeling_siglip.py).  The reference itself has no
+ * modeling_gemma.py and modeling_siglip.py).  The reference itself has no
  * FFI -- it is pure PyTorch -- so each entry point names the reference function whose body it
- * replaces; INTEGRATION.md shows the ctypes binding a maintainer would add.
+ * replaces.
  *
  * Conventions
  *   - plain C, every call returns 0 on success or a negative PGMI_E* code; the message of the
@@ -62,7 +62,7 @@ int pgmi_create(int device, const pgmi_config* cfg, pgmi_ctx** out);
 int pgmi_destroy(pgmi_ctx* ctx);
 
 /* ---- weights: one bf16 slab in caller-owned device memory, laid out by the library.
- * Tensor names and shapes are the reference state-dict keys (SURVEY.md sec.3.5); lm_head is
+ * Tensor names and shapes are the reference state-dict keys; lm_head is
  * tied to embed_tokens (modeling_gemma.py:396-397) and has no slot of its own. */
 int64_t pgmi_weights_bytes(const pgmi_ctx* ctx);
 int pgmi_weight_count(const pgmi_ctx* ctx);
@@ -73,7 +73,7 @@ int pgmi_bind_weights(pgmi_ctx* ctx, void* dev_slab);
  * (and converts to bf16) from host or device memory into the slab. */
 int pgmi_load_weight(pgmi_ctx* ctx, const char* name, const void* src, int src_dtype, int src_on_device,
                      void* stream);
-/* Native safetensors reader (SURVEY.md sec.8f rank 3; replaces the safe_open / accelerate
+/* Native safetensors reader (replaces the safe_open / accelerate
  * shard loop of utils.py:19-44 and ablation_study_fixed.py:304-332): one *.safetensors file is
  * memory-mapped and every tensor whose name is a slab weight is shape-checked, converted to bf16
  * (BF16 copied, F32/F16 rounded to nearest even on the device) and written into the slab.
@@ -173,13 +173,13 @@ int pgmi_set_decode_staged_norm(pgmi_ctx* ctx, int on);
 /* lm_head + .float() of GemmaForCausalLM (modeling_gemma.py:417-418) over final-normed hidden
  * rows: logits (device fp32 [rows][vocab]) = fp32(bf16(normed . E^T)) with the tied embedding E.
  * Together with pgmi_lm_final_hidden this materialises the prefill's all-row logits on demand
- * after a last-row-only pgmi_lm_forward (SURVEY.md sec.7 hard part 3: lazy logits). */
+ * after a last-row-only pgmi_lm_forward (lazy logits). */
 int pgmi_lm_head(pgmi_ctx* ctx, const void* normed, int rows, float* logits, void* stream);
 /* Copies the final RMSNorm output (GemmaModel.norm, modeling_gemma.py:379) of the B*L rows of the
  * last pgmi_lm_forward (bf16 [rows][hidden], row-major) into `out` (device memory). */
 int pgmi_lm_final_hidden(pgmi_ctx* ctx, void* out, int rows, void* stream);
 
-/* ---- replicas (SURVEY.md sec.8e): the load-time weight broadcast over RCCL (xGMI).  The
+/* ---- replicas: the load-time weight broadcast over RCCL (xGMI).  The
  * reference has no multi-GPU path (accelerate placement only, utils.py:27-38).  One process per
  * GPU: the root calls pgmi_comm_unique_id, ships the PGMI_COMM_ID_BYTES bytes to every rank (any
  * channel), each rank calls pgmi_comm_init, then pgmi_broadcast_weights copies the root's whole

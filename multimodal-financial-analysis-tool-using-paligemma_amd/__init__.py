@@ -2,7 +2,7 @@
 
 Put this directory on sys.path to use it as a drop-in for the reference's modules:
 ``import modeling_gemma, modeling_siglip, processing_paligemma, utils`` resolve to the
-MI355X-native implementations here (see INTEGRATION.md).
+MI355X-native implementations here.
 """
 import os as _os
 import sys as _sys

@@ -8,7 +8,7 @@
 // prologue of the o_proj GEMV that consumes o (gemv_body.h, GV_ORES).
 // P.V runs on MFMA from bf16 e = exp(s - m_c) (the reference rounds the normalised p to bf16,
 // modeling_gemma.py:273,277; here the unnormalised chunk-local e is rounded, the fp32 sum l_c
-// normalises at the combine: same rounding granularity, documented in DESIGN.md).
+// normalises at the combine: same rounding granularity).
 #include "common.h"
 #include "launch.h"
 

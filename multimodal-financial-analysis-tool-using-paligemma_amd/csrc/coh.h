@@ -1,6 +1,6 @@
 // coh.h -- coherent (write-through / L2-bypassing) loads and stores for cross-workgroup hand-offs
 // inside one launch (gfx950, 8 XCDs with private L2s): relaxed agent-scope atomic stores and loads,
-// no fences (cdna_hip_programming.md sec.6 Guideline 16, form R1).  Used by the lm_head's folded
+// no fences.  Used by the lm_head's folded
 // argmax: each workgroup publishes its partial write-through, counts its arrival, and the last
 // one to arrive reads every partial coherently (no workgroup ever waits on another).
 #pragma once

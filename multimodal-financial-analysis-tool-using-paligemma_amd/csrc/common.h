@@ -2,7 +2,7 @@
 //
 // bf16 is carried as raw uint16 bit patterns; all arithmetic is fp32 with an
 // explicit round-to-nearest-even back to bf16 exactly where the reference's bf16
-// PyTorch modules round ("rounding points").
+// PyTorch modules round (their bf16 outputs).
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -78,8 +78,7 @@ __device__ __forceinline__ uint4 ldg16(const void* p) {
 
 // 16-B load whose lane may be out of range: the load is ALWAYS issued (from `safe` when !ok) and
 // the value zeroed afterwards -- a conditional load (ok ? load : 0) makes hipcc branch around the
-// load and wait vmcnt(0) for it, one dependent round trip per element (cdna_hip_programming.md
-// sec.5 "Projection GEMM at M = 256", trap (c))
+// load and wait vmcnt(0) for it, one dependent round trip per element
 __device__ __forceinline__ uint4 ldg16_sel(const void* p, bool ok, const void* safe) {
     const uint4 v = *reinterpret_cast<const uint4*>(ok ? p : safe);
     return ok ? v : make_uint4(0, 0, 0, 0);

@@ -1,7 +1,7 @@
 // engine.hip -- the PaliGemma family of libpgmi: weight layout, workspaces, forward orchestration, hipGraph
 // decode, and its extern "C" entry points of include/pgmi.h.
 //
-// Orchestration restates the reference's call stacks (SURVEY.md sec.3.2/3.3):
+// Orchestration restates the reference's call stacks:
 //   vision   SiglipVisionTransformer.forward   modeling_siglip.py:236-244
 //   lm       GemmaModel/GemmaForCausalLM        modeling_gemma.py:357-427
 //   decode   one inference.py loop iteration    inference.py:56-78

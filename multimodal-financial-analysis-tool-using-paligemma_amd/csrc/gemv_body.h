@@ -1,7 +1,7 @@
 #pragma once
 // gemv_body.h -- KV-cached decode projections (batch B <= 8 rows), gfx950.
 //
-// Decode at batch 1 streams ~5.02 GB of weights per token (SURVEY.md sec.8d), so every
+// Decode at batch 1 streams ~5.02 GB of weights per token, so every
 // projection of GemmaDecoderLayer (modeling_gemma.py:307-338) is one HBM-bound pass over
 // its nn.Linear weight [N][K] (K contiguous, used as stored):
 //   - each wave owns RPW "units" (1 row, or a row pair: RoPE's (d, d+128) or GeGLU's

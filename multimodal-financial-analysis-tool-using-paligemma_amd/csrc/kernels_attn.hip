@@ -798,7 +798,7 @@ __global__ void __launch_bounds__(256) k_attn_short(AttnArgs a) {
 // Rounding: s = bf16(bf16(k.q) * scale) as the reference; p is rounded to bf16 as exp(s - m) with m
 // the workgroup's running row max (deferred: raised only when a tile's max passes it by kFsDefer,
 // e <= e^8 in between) and normalised in fp32 at the end, where the reference rounds the globally
-// normalised p -- the flash-decoding deviation of the decode step (DESIGN.md sec.5).
+// normalised p -- the flash-decoding deviation of the decode step.
 // LDS images (rows of CR 16-B chunks): K chunk c of key row r at chunk c ^ (r & 15) (conflict-free
 // ds_read_b128 of 16 rows x one 16-B k slice); V chunk c at chunk c ^ ((r & 7) << 1) (the
 // ds_read_b64_tr_b16 reads of 8 rows x 32 B per half-wave hit 8 distinct 32-B bank groups).  The

@@ -1087,9 +1087,8 @@ __global__ void __launch_bounds__(64 * (NW + LW), 1) k_gemm_w(const uint16_t* __
 //   ds_read its fragments | LDS-DMA one half-tile of a later K-tile | [vmcnt] | s_barrier |
 //   lgkmcnt(0) | 16 MFMAs (setprio 1) | s_barrier
 // with the two wave rows staggered by one barrier (ping-pong: one wave of each SIMD in its MFMA
-// cluster while the other reads and stages) and four half-tiles in flight across every barrier:
-// cdna_hip_programming.md's 256^2 8-phase template, restated for this LDS image, with B0's
-// fragments kept in registers across the tile (one fewer fragment read per K-tile).
+// cluster while the other reads and stages) and four half-tiles in flight across every barrier; B0's
+// fragments stay in registers across the tile (one fewer fragment read per K-tile).
 // LDS rows are 128 B with the 16-B chunk XOR-swizzled by (row & 7) on the DMA's source address.
 //
 // G: which rows a tile is made of.  AllRows: consecutive rows of A, the XCD-aware tile order.  A grouped form

@@ -1,5 +1,4 @@
-// kernels_gemv_mfma.hip -- decode projections for 2..16 sequences in lock-step (
-// 8 images per GPU), on MFMA.
+// kernels_gemv_mfma.hip -- decode projections for 2..16 sequences in lock-step (8 images per GPU), on MFMA.
 //
 // At batch 1 a decode projection is one HBM pass with v_dot2 (gemv_body.h).  At batch B the
 // same pass owes B dot products per weight byte; on v_dot2 that turns the pass VALU-bound (B = 8:

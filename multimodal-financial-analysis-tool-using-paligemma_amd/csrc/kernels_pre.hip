@@ -1,4 +1,4 @@
-// kernels_pre.hip -- image preprocessing on the GPU (SURVEY.md sec.8f rank 2):
+// kernels_pre.hip -- image preprocessing on the GPU:
 // processing_paligemma.py:13-18,40-49 = PIL Image.resize(BICUBIC) -> x/255 -> (x-0.5)/0.5 -> CHW.
 //
 // PIL's resample (libImaging/Resample.c; restated in oracle/resize_np.py) is reproduced

@@ -1,5 +1,5 @@
 // kernels_sample.hip -- temperature softmax + top-p (nucleus) sampling on the device
-// (inference.py:15-24 _sample_top_p, with the softmax(logits / T) of :65), SURVEY.md sec.8f rank 4.
+// (inference.py:15-24 _sample_top_p, with the softmax(logits / T) of :65).
 //
 // The reference sorts all 257,216 probabilities, takes the cumulative sum, zeroes every entry
 // whose preceding mass already exceeds p, renormalises and draws with torch.multinomial.  The

@@ -1,7 +1,7 @@
 """Drop-in for the reference's modeling_gemma.py (Gemma decoder, KV cache, PaliGemma), MI355X-native.
 
 Same classes, constructor signatures, attributes and state-dict names as
-/root/reference/modeling_gemma.py, so the reference's inference.py / utils.py /
+modeling_gemma.py, so the reference's inference.py / utils.py /
 ablation_study_fixed.py drive it unchanged.  The forwards of the three boundary modules run in
 libpgmi (include/pgmi.h):
 

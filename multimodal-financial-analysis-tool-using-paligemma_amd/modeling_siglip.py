@@ -1,7 +1,7 @@
 """Drop-in for the reference's modeling_siglip.py (SigLIP vision tower), MI355X-native.
 
 The module tree, constructor signatures and state-dict names are the reference's
-(/root/reference/modeling_siglip.py:7-255), so checkpoints load unchanged.  The forward of
+(modeling_siglip.py:7-255), so checkpoints load unchanged.  The forward of
 SiglipVisionModel runs the whole tower in libpgmi (pgmi_vision: im2col+MFMA patch embedding,
 27 x [LayerNorm, fused QKV GEMM, MHA, out-proj+residual, LayerNorm, fc1+GELU, fc2+residual],
 post-LayerNorm; csrc/engine.hip).  The per-layer submodules (embeddings, attention, MLP, encoder

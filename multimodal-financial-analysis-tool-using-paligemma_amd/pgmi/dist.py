@@ -1,4 +1,4 @@
-"""Multi-GPU: one process per GPU, independent replicas (SURVEY.md sec.8e).
+"""Multi-GPU: one process per GPU, independent replicas.
 
 The path does not exchange data per token: images are sharded across ranks and every rank
 runs its own full replica.  The only collective is the load-time broadcast of the packed

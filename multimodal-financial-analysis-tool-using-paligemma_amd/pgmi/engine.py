@@ -100,7 +100,7 @@ class EngineBase:
         self.prepared = False
 
     def load_safetensors(self, path: str, strict: bool = True) -> int:
-        """Native safetensors loading into the slab (pgmi_load_safetensors; SURVEY.md sec.8f rank 3).
+        """Native safetensors loading into the slab (pgmi_load_safetensors).
         `path` is a *.safetensors file or a directory of shards.  With strict, every slab weight
         must come from the files.  Returns the number of tensors loaded."""
         import glob
@@ -152,7 +152,7 @@ class EngineBase:
     def sample_top_p(self, x: torch.Tensor, top_p: float, temperature: Optional[float] = None,
                      u: Optional[torch.Tensor] = None, generator: Optional[torch.Generator] = None,
                      return_kept_mass: bool = False):
-        """Nucleus sampling on the device (inference.py:15-24; SURVEY.md sec.8f rank 4).
+        """Nucleus sampling on the device (inference.py:15-24).
         x (..., V) fp32: logits when `temperature` > 0 (softmax(x / T) of inference.py:65 is
         fused), else probabilities (the reference _sample_top_p's input).  u: uniforms in [0, 1)
         per row (default: torch.rand on the device with `generator`).  Returns int64 (rows,)."""
@@ -492,7 +492,7 @@ class Engine(EngineBase):
                  kv: torch.Tensor = None, do_sample: bool = False, temperature: float = 0.8, top_p: float = 0.9,
                  generator: Optional[torch.Generator] = None, eos_token_id: Optional[int] = None,
                  pad_token_id: Optional[int] = None, sync_every: int = 16, return_lengths: bool = False):
-        """Batched generation (SURVEY.md sec.8f rank 1): prefill, then n_tokens-1 decode steps
+        """Batched generation: prefill, then n_tokens-1 decode steps
         with the next token picked on the device -- greedy argmax, or with do_sample the
         temperature + top-p draw of inference.py:64-66 -- and no host sync per token.
         Positions follow inference.py's semantics (first decode position = L + 1,

@@ -1,4 +1,4 @@
-"""Prefill logits computed lazily (SURVEY.md sec.7 hard part 3).
+"""Prefill logits computed lazily.
 
 The reference's GemmaForCausalLM returns logits for EVERY prefill position: (B, L, 257216) fp32,
 288 x 257216 x 4 B = 296 MB and a 303 GFLOP GEMM at 224 px (modeling_gemma.py:417-418), while

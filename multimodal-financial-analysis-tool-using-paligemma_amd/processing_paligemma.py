@@ -1,11 +1,11 @@
 """Drop-in for the reference's processing_paligemma.py (image preprocessing + prompt glue).
 
-Same functions, constants and PaliGemmaProcessor API as /root/reference/processing_paligemma.py
+Same functions, constants and PaliGemmaProcessor API as processing_paligemma.py
 (:1-117): BICUBIC resize (PIL), x/255, (x - 0.5)/0.5, HWC -> CHW, and the
 "<image>" * N + bos + prompt + "\\n" prompt layout; tests/test_cpu_host.py pins it to the
 reference's own outputs on the committed COCO images.  `process_images_gpu` (and
 PaliGemmaProcessor(..., engine=...)) runs the same steps on the MI355X through libpgmi
-(pgmi_preprocess: PIL-exact resample, SURVEY.md sec.8f rank 2; tests/test_gpu_preprocess.py).
+(pgmi_preprocess: PIL-exact resample; tests/test_gpu_preprocess.py).
 """
 from __future__ import annotations
 

@@ -1,6 +1,6 @@
 """Drop-in for the reference's utils.py: load_hf_model(model_path, device) -> (model, tokenizer).
 
-Replaces the reference's full random init + accelerate dispatch (/root/reference/utils.py:6-46)
+Replaces the reference's full random init + accelerate dispatch (utils.py:6-46)
 with: config.json -> PaliGemmaConfig, the module tree built on the meta device (no 3B random
 init), safetensors read straight into bf16 device parameters, non-persistent buffers
 recomputed, weights tied (utils.py:44).  There is no "load without weights" fallback: a missing

@@ -2,7 +2,7 @@
 
 CPU restatement (numpy, float32 arithmetic with explicit bf16 rounding) of the
 reference's PaliGemma inference path.  It rounds to bf16 exactly where the
-reference's bf16 modules do (SURVEY.md sec.8a "rounding points" column), so it
+reference's bf16 modules do, so it
 is the checker for the HIP path.  Only tests/, __graft_entry__.smoke() and
 bench.py's cpu_baseline leg may use it; the product never imports it.
 
@@ -322,7 +322,7 @@ def paligemma_prefill(P, cfg, input_ids, pixel_values, taps=None, all_logits=Tru
 def paligemma_decode(P, cfg, next_ids, kv, mask_len):
     """One decode step with inference.py semantics: input_ids (B,1), attention_mask has
     `mask_len` ones, position = cumsum(mask)[-1] = mask_len (modeling_gemma.py:516-528),
-    which after prefill of L tokens is L+1 (the position-id gap, SURVEY.md sec.0)."""
+    which after prefill of L tokens is L+1 (the position-id gap)."""
     ids = np.asarray(next_ids).reshape(-1, 1)
     emb = merge(P, cfg, None, ids)
     pos = np.full((ids.shape[0], 1), mask_len, dtype=np.int64)

@@ -6,8 +6,8 @@ reference modules in the survey container) and the HIP path all run on the same
 deterministic synthetic weights produced by ``wgen.c``.
 
 State-dict names/shapes follow the reference module tree
-(/root/reference/modeling_gemma.py:440-456,
-/root/reference/modeling_siglip.py:36-255).
+(modeling_gemma.py:440-456,
+modeling_siglip.py:36-255).
 """
 from __future__ import annotations
 
@@ -22,7 +22,7 @@ _HERE = os.path.dirname(os.path.abspath(__file__))
 _LIB = os.path.join(_HERE, "libwgen.so")
 
 # HF google/paligemma-3b-pt-224 config.json, as consumed by PaliGemmaConfig
-# (/root/reference/modeling_gemma.py:74-105).
+# (modeling_gemma.py:74-105).
 FULL_224 = {
     "vision_config": {
         "hidden_size": 1152, "intermediate_size": 4304, "num_hidden_layers": 27,
@@ -122,7 +122,7 @@ GAINS = {"embed": 0.02, "pos_embed": 0.1, "proj": 2.0, "qk": 3.0, "o_down": 8.0}
 def init_policy(name: str, shape: tuple) -> "tuple[float, float]":
     """(scale, offset) of the synthetic init: w = bf16(offset + U[-1,1) * scale).
 
-    gain/sqrt(fan_in) for projections (SURVEY.md sec.8c item 1); norms get small
+    gain/sqrt(fan_in) for projections; norms get small
     random deviations so the (1 + w) RMSNorm path (modeling_gemma.py:119) and the
     LayerNorm affine are exercised."""
     g = GAINS

@@ -3,7 +3,7 @@
  *
  * Deterministic synthetic-weight generator shared by the oracle, the golden
  * fixture script and the parity tests.  PaliGemma weights/tokenizer are not
- * available offline (SURVEY.md sec.7 "hard parts" 8), so parity is defined on
+ * available offline, so parity is defined on
  * synthetic weights that every party can regenerate bit-exactly:
  *
  *   key   = splitmix64(seed ^ fnv1a64(state_dict_name))
