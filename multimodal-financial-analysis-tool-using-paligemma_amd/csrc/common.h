@@ -78,7 +78,8 @@ __device__ __forceinline__ uint4 ldg16(const void* p) {
 
 // 16-B load whose lane may be out of range: the load is ALWAYS issued (from `safe` when !ok) and
 // the value zeroed afterwards -- a conditional load (ok ? load : 0) makes hipcc branch around the
-// load and wait vmcnt(0) for it, one dependent round trip per element
+// load and wait vmcnt(0) for it, one dependent round trip per element.  Its words are read and chosen one by one, unlike ldg16's (as
+// one vector residual + router spills 18 registers); in the disassembly of its users no matrix instruction's words are overwritten
 __device__ __forceinline__ uint4 ldg16_sel(const void* p, bool ok, const void* safe) {
     const uint4 v = *reinterpret_cast<const uint4*>(ok ? p : safe);
     return ok ? v : make_uint4(0, 0, 0, 0);
