@@ -79,13 +79,15 @@ inline ScanStep scan_step_of(const int32_t* lens, int n_seq, int run_rows) {
 // takes alone, or what the chip takes for all of them (a CU's share of the workgroups, each with its start and its steps); runs take
 // their launches, the rows' traffic, the rounds of rows walked one after the other and the carries.  The constants are fitted to 196
 // steps of 64 to 8,192 channels and 33 to 4,096 rows: the rule loses 0.2 % of the better form on average, 22 % at most (runs kept for 700
-// fp32 rows of 64 channels), and no walk that it takes is slower than runs by more than 1.3 %.  us a
-// layer, runs / walk: 1,024 + 387 + 129 rows of 4,096 channels 70.0 / 37.1, 512 rows 33.7 / 15.7, 8 x 512 rows 145 / 87, 500 rows of
-// 2,048 fp32 channels 31.3 / 21.1; 4,096 rows of 2,048 channels 83 / 113, 64 x 33 rows of 4,096 50 / 116.
+// fp32 rows of 64 channels), and no walk that it takes is slower than runs by more than 1.3 %
+// (nor by more than 3 % of 144 steps of other channels and 9 to 15 states).  us a layer, runs / walk: 1,024 + 387 + 129 rows of 4,096 channels
+// 70.5 / 38.1, 512 rows 34.0 / 16.5, 8 x 512 rows 145 / 89, 500 rows of 2,048 fp32 channels 31.3 / 21.1; 4,096 rows of 2,048 channels
+// 83 / 113, 64 x 33 rows of 4,096 50 / 116, 1,000 rows of 1,000 channels of 12 states 32.8 / 38.7 (1,024 of 16: 31 / 27).
 inline bool scan_walks(const ScanStep& s, int C, int N, bool f32) {
     if (N <= 8 || N > 16) return false;
     const double per_cu = (C + 15) / 16 / (double)kRunCUs;
-    const double walk = (f32 ? 5 : 3) + std::max((f32 ? 0.035 : 0.024) * s.longest,
+    const int odd = (C % 16 != 0) + (N != 16);  // single elements: channels that are no whole workgroups, states that are no 16
+    const double walk = (f32 ? 5 : 3) + std::max((f32 ? 0.035 + 0.0035 * odd : 0.024 + 0.006 * odd) * s.longest,
                                                  per_cu * (0.5 * s.n_seq + (f32 ? 0.029 : 0.023) * (double)s.padded));
     const double rounds = (double)((s.runs * ((C + 255) / 256) + kRunCUs - 1) / kRunCUs);
     const double runs = s.most_runs == 1 ? 10 + rounds * s.run_rows * (f32 ? 0.44 : 0.3)
@@ -109,13 +111,14 @@ inline int gru_run_rows(const int32_t* lens, int n_seq, long columns) {
 }
 
 // Whether a minGRU layer walks its sequences whole (k_gru_walk, one launch) rather than in the runs above: as scan_walks, by the
-// predicted time in us, fitted to 180 steps of 44 to 4,096 channels and 17 to 4,096 rows.  It leans to the runs: it loses 1.8 % of the
+// predicted time in us, fitted to 180 steps of 44 to 4,096 channels and 17 to 4,096 rows.  It leans to the runs: it loses 2.1 % of the
 // better form on average, up to 37 % where runs are kept for 2,000 rows of up to 256 channels, and 12 % at most where a walk is taken
 // (4,096 fp32 rows of 2,048 channels).  us a layer, runs / walk: 1,024 + 387 + 129 rows of 2,048 channels 21.7 / 12.6, 500 rows of 1,024 fp32
 // channels 14.7 / 6.8, 60 rows of 2,048 11.0 / 5.7, 8 x 512 rows 30.1 / 22.5; 64 x 33 rows 10.9 / 40, 4,096 rows of 1,024 channels 30 / 34.
 inline bool gru_walks(const ScanStep& s, int C, bool f32) {
     const double per_cu = (C + 15) / 16 / (double)kRunCUs, traffic = (f32 ? 3.4e-6 : 1.65e-6) * C * (double)s.rows;
-    const double walk = 4.5 + std::max(0.008 * s.longest, per_cu * (0.5 * s.n_seq + (f32 ? 0.0135 : 0.0095) * (double)s.padded));
+    const double row = C % 16 == 0 ? 0.008 : f32 ? 0.011 : 0.0135;  // (channels that are no whole workgroups: single elements)
+    const double walk = 4.5 + std::max(row * s.longest, per_cu * (0.5 * s.n_seq + (f32 ? 0.0135 : 0.0095) * (double)s.padded));
     const double runs = traffic + (s.most_runs == 1 ? 3.6 + 0.11 * s.run_rows : 8.2 + 0.21 * s.run_rows + 0.07 * s.most_runs);
     return walk < runs;
 }

@@ -94,6 +94,7 @@ def walks(tmp_path_factory):
     (4096, 16, [1024, 387, 129], 1, 1), (4096, 16, [1540], 1, 1), (4096, 16, [512] * 8, 1, 1), (4096, 16, [4096], 1, 1),
     (2048, 16, [500], 1, 1), (2048, 16, [1000], 1, 1), (2048, 16, [4096], 0, 0), (1024, 16, [3000], 0, 0), (512, 16, [700], 1, 1),
     (64, 16, [1500], 0, 0), (64, 16, [300], 1, 1), (4096, 16, [33] * 64, 0, 0), (8192, 16, [64] * 32, 0, 0), (1024, 16, [64] * 32, 1, 1),
+    (1000, 12, [1000], 0, 0), (520, 10, [1000], 0, 0), (264, 16, [1000] * 2, 0, 0), (1000, 12, [300], 1, 1), (4096, 9, [1000], 1, 1),
     (72, 12, [70, 33, 5], 1, 1), (72, 8, [70, 33, 5], 0, 0), (72, 17, [70, 33, 5], 0, 0), (2048, 64, [500], 0, 0), (64, 9, [1], 1, 1)])
 def test_scan_walks(walks, C, N, lens, bf16, f32):
     assert walks(C, N, *lens) == [bf16, f32]
@@ -124,7 +125,7 @@ def gru_walks(tmp_path_factory):
 @pytest.mark.parametrize("C,lens,bf16,f32", [
     (2048, [1024, 387, 129], 1, 1), (1024, [500], 1, 1), (2048, [60], 1, 1), (4096, [1000], 1, 1), (2048, [1000] * 4, 1, 1),
     (1024, [512] * 8, 1, 1), (256, [64] * 32, 1, 1), (44, [300], 1, 1), (1024, [33] * 64, 0, 0), (4096, [33] * 64, 0, 0),
-    (4096, [64] * 32, 0, 0), (64, [4096], 0, 0), (256, [4096], 0, 0), (44, [2000], 0, 0)])
+    (4096, [64] * 32, 0, 0), (300, [2000], 0, 0), (4088, [1000], 1, 1), (64, [4096], 0, 0), (256, [4096], 0, 0), (44, [2000], 0, 0)])
 def test_gru_walks(gru_walks, C, lens, bf16, f32):
     assert gru_walks(C, *lens) == [bf16, f32]
 
