@@ -53,7 +53,7 @@ struct GraphKey {
     int kv_batch, kv_max;
     float* logits;
     int64_t* next;
-    const int64_t* ids;  // the ids buffer the graph reads (the context's staging copy, or in place)
+    const int64_t* ids;  // the ids that the graph reads: those it feeds back in place (null: the launch in front of it reads them)
     bool emb;            // the step's input is the staged embedding rows (pgmi_decode_embeds), not ids
     int masked;          // 0: no mask (a zero word), 1: staged bf16 mask (sum rounded), 2: staged fp32 mask
     int n_steps;         // decode steps captured back to back (pgmi_decode_steps; 1 otherwise)
@@ -64,6 +64,9 @@ struct GraphKey {
                         o.tokens);
     }
 };
+
+// a decode step, its first launch (the only one that reads its token ids), or all but that
+enum StepPart { STEP_ALL, STEP_HEAD, STEP_REST };
 
 struct GraphEntry {
     int seen = 0;
@@ -119,7 +122,6 @@ struct pgmi_ctx {
     int max_chunks;
     StepState* step;
     StepState* pstep;  // the generate-loop prefill's last-row attention (flash-decoding over the prompt's keys)
-    int64_t* d_ids;
     uint16_t* d_emb;             // staged input rows of pgmi_decode_embeds ([max_batch][hidden] bf16)
     float* d_mask;               // staged additive decode mask ([max_batch][max_kv] fp32, pgmi_decode_embeds_dev)
     float* d_zero;               // one zero word: the "no mask" mask of the decode attention

@@ -186,7 +186,6 @@ int paligemma_prepare(pgmi_ctx* x) {
         if ((rc = dalloc_t(x, &x->pstep, 1))) return rc;
         if ((rc = dalloc_t(x, &x->amax_v, (size_t)argmax_scratch_parts()))) return rc;
         if ((rc = dalloc_t(x, &x->amax_i, (size_t)argmax_scratch_parts()))) return rc;
-        if ((rc = dalloc_t(x, &x->d_ids, (size_t)B))) return rc;
         if ((rc = dalloc_t(x, &x->d_emb, (size_t)B * H))) return rc;
         if ((rc = dalloc_t(x, &x->d_mask, (size_t)B * c.max_kv))) return rc;
         if ((rc = dalloc_t(x, &x->d_zero, 64))) return rc;
@@ -487,7 +486,7 @@ static bool mf_staged(const pgmi_ctx* x) { return x->mf_staged > 0; }
 
 static int decode_body(pgmi_ctx* x, hipStream_t s, const int64_t* ids, int B, void* kv, int kv_batch, int kv_max,
                        int launch_keys, float* logits, int64_t* next_ids, const uint16_t* embeds = nullptr,
-                       int masked = 0, int64_t* hist = nullptr) {
+                       int masked = 0, int64_t* hist = nullptr, StepPart part = STEP_ALL) {
     const pgmi_config& c = x->c;
     const int H = c.t_hidden, NH = c.t_heads, NKV = c.t_kv_heads, HD = c.t_head_dim;
     const float eps = c.t_rms_eps;
@@ -499,8 +498,10 @@ static int decode_body(pgmi_ctx* x, hipStream_t s, const int64_t* ids, int B, vo
     const bool fold = !embeds && gemv_qkv_folds_embed(B) && c.t_layers > 0;
     const EmbedFold emb{ids, E, normalizer, c.pad_token_id, x->dH};
     // given input rows (a caller's merge, pgmi_decode_embeds): h = rows x bf16(sqrt(hidden)) (modeling_gemma.py:367-368)
+    const bool rest = part == STEP_REST;
     if (embeds) scale_rows(s, embeds, (long)B * H, normalizer, x->dH);
-    else if (!fold) embed_rows(s, ids, B, E, H, normalizer, c.pad_token_id, x->dH);
+    else if (!fold && !rest) embed_rows(s, ids, B, E, H, normalizer, c.pad_token_id, x->dH);
+    if (!fold && part == STEP_HEAD) return 0;
     // B >= 3 (MFMA projections): every RMSNorm is computed once per row -- the input norm fused into the
     // down projection's combine for the next layer (q|k|v reads dHn unstaged), the post-attention norm's
     // sums of squares written by o_proj's epilogue (dSS) and applied by gate|up as it loads h.  (Measured:
@@ -515,9 +516,11 @@ static int decode_body(pgmi_ctx* x, hipStream_t s, const int64_t* ids, int B, vo
         // fragment-major weight images of this layer (prepare's mf_swizzle), when built: gate|up, q|k|v, o_proj
         const uint16_t* Lf = x->mfw ? x->mfw + x->mfw_layer * i : nullptr;
         const size_t gu_n = (size_t)2 * c.t_intermediate * H, qkv_n = (size_t)(NH + 2 * NKV) * HD * H;
-        gemv_qkv(s, B, NH, NKV, mf ? x->dHn : x->dH, mf ? nullptr : TL(x, i, "input_layernorm.weight"), eps,
-                 TL(x, i, "self_attn.q_proj.weight"), x->cosT, x->sinT, c.t_max_pos, x->step, x->dQ, Kc, Vc, kvb, x->ws,
-                 (fold && i == 0) ? &emb : nullptr, Lf ? Lf + gu_n : nullptr);
+        if (!(fold && rest && i == 0))
+            gemv_qkv(s, B, NH, NKV, mf ? x->dHn : x->dH, mf ? nullptr : TL(x, i, "input_layernorm.weight"), eps,
+                     TL(x, i, "self_attn.q_proj.weight"), x->cosT, x->sinT, c.t_max_pos, x->step, x->dQ, Kc, Vc, kvb, x->ws,
+                     (fold && i == 0) ? &emb : nullptr, Lf ? Lf + gu_n : nullptr);
+        if (part == STEP_HEAD) return 0;
         AttnArgs a{};
         a.q = x->dQ; a.q_b_stride = (long)NH * HD; a.q_row_stride = NH * HD; a.q_head_stride = HD;
         a.k = Kc; a.k_b_stride = kvb; a.k_row_stride = (int)kvd; a.k_head_stride = HD;
@@ -687,11 +690,12 @@ static int decode_step(pgmi_ctx* x, const int64_t* ids, const void* embeds, int 
     // n_steps greedy steps back to back: step t > 0 reads the argmax step t - 1 wrote (next_ids, or the
     // context's d_next when the caller passes none); step t's token also goes to tokens[t][B] when given
     int64_t* fb = next_ids ? next_ids : x->d_next;
-    auto body = [&](hipStream_t st, const int64_t* first, int keys0, bool grow) -> int {
+    auto body = [&](hipStream_t st, const int64_t* first, int keys0, bool grow, StepPart part = STEP_ALL) -> int {
         for (int t = 0; t < n_steps; ++t) {
             const int r = decode_body(x, st, t == 0 ? first : fb, B, kv, kv_batch, kv_max, grow ? keys0 + t : keys0,
-                                      logits, next_ids, erows, masked, tokens ? tokens + (long)t * B : nullptr);
-            if (r) return r;
+                                      logits, next_ids, erows, masked, tokens ? tokens + (long)t * B : nullptr,
+                                      t == 0 ? part : STEP_ALL);
+            if (r || part == STEP_HEAD) return r;
         }
         return 0;
     };
@@ -701,19 +705,16 @@ static int decode_step(pgmi_ctx* x, const int64_t* ids, const void* embeds, int 
         advanced();
         return 0;
     }
-    // in-place feedback (next_ids == ids: the step reads its tokens first and writes the next
-    // ones last) needs no staging copy; other callers' ids are staged into the context's buffer
-    const int64_t* gids = ids;
-    if (!embeds && ids != next_ids) {
-        HIPCHK(hipMemcpyAsync(x->d_ids, ids, (size_t)B * sizeof(int64_t), hipMemcpyDeviceToDevice, s));
-        gids = x->d_ids;
-    }
-    if (embeds) gids = nullptr;
+    // in-place feedback (next_ids == ids: the step reads its tokens first and writes the next ones last) is read by the
+    // graph; other callers' ids by the step's first launch in front of it, so that the graph holds no address of them
+    // and nothing copies them (a copy is a launch more: 4.5 us)
+    const bool head = !embeds && ids != next_ids && c.t_layers > 0;
+    const int64_t* gids = embeds || head ? nullptr : ids;
     GraphKey key{B, kv, kv_batch, kv_max, logits, next_ids, gids, embeds != nullptr, masked, n_steps, tokens};
     GraphEntry& ge = x->graphs[key];
     if (!ge.exec) {
         if (ge.seen++ == 0) {  // first call with this key: run eagerly (sets kernel attributes)
-            if ((rc = body(s, gids, kv_max, false))) return rc;
+            if ((rc = body(s, ids, kv_max, false))) return rc;
             LAUNCHCHK();
             advanced();
             return 0;
@@ -721,12 +722,13 @@ static int decode_step(pgmi_ctx* x, const int64_t* ids, const void* embeds, int 
         HIPCHK(hipStreamSynchronize(s));
         hipGraph_t g;
         HIPCHK(hipStreamBeginCapture(x->cap_stream, hipStreamCaptureModeThreadLocal));
-        rc = body(x->cap_stream, gids, kv_max, false);
+        rc = body(x->cap_stream, gids, kv_max, false, head ? STEP_REST : STEP_ALL);
         HIPCHK(hipStreamEndCapture(x->cap_stream, &g));
         if (rc) return rc;
         HIPCHK(hipGraphInstantiate(&ge.exec, g, nullptr, nullptr, 0));
         (void)hipGraphDestroy(g);
     }
+    if (head && (rc = body(s, ids, kv_max, false, STEP_HEAD))) return rc;
     HIPCHK(hipGraphLaunch(ge.exec, s));
     LAUNCHCHK();
     advanced();

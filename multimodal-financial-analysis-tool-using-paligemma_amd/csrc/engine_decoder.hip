@@ -89,7 +89,7 @@ struct DecoderState {
     size_t part_floats = 0;
     float* pmax = nullptr;
     int* pidx = nullptr;
-    int64_t *d_ids = nullptr, *d_next = nullptr;
+    int64_t* d_next = nullptr;
     std::vector<int> known_slot, known_pos;  // what slot / pos hold once the enqueued steps have run (empty: unknown)
 };
 
@@ -357,7 +357,6 @@ int decoder_prepare(pgmi_ctx* x) {
         if ((rc = dalloc_t(x, &x->amax_i, (size_t)argmax_scratch_parts()))) return rc;
         if ((rc = dalloc_t(x, &d.slot, (size_t)B))) return rc;
         if ((rc = dalloc_t(x, &d.pos, (size_t)B))) return rc;
-        if ((rc = dalloc_t(x, &d.d_ids, (size_t)B))) return rc;
         if ((rc = dalloc_t(x, &d.d_next, (size_t)B))) return rc;
         if ((rc = dalloc_t(x, &d.pmax, (size_t)gemv_rt_parts()))) return rc;
         if ((rc = dalloc_t(x, &d.pidx, (size_t)gemv_rt_parts()))) return rc;
@@ -734,18 +733,20 @@ int forward_body(pgmi_ctx* x, hipStream_t s, const int64_t* ids, int rows, const
     return 0;
 }
 
+// part: the whole step, its first launch (the only one that reads ids), or all but that
 int decode_body_rt(pgmi_ctx* x, hipStream_t s, const int64_t* ids, int B, void* state, int n_slots, int max_tokens,
-                   float* logits, int64_t* next, int64_t* hist) {
+                   float* logits, int64_t* next, int64_t* hist, StepPart part) {
     DecoderState& d = *x->dec;
     const int D = d.c.width, V = d.c.vocab;
     const StateMap sm = state_layout(d, n_slots, max_tokens);
     const std::vector<StateAt>& st = sm.at;
     const bool plain = d.c.plain_residual;
-    if (!plain) {  // the embedding rows into every stream, and the first sublayer's input
+    if (!plain && part != STEP_REST) {  // the embedding rows into every stream, and the first sublayer's input
         StreamsArgs a = streams_args(d, B);
         a.ids = ids; a.in = d.W[0].sub[0].in; a.w = d.W[0].sub[0].norm;
         streams_norm(s, d.act, a);
     }
+    if (!plain && part == STEP_HEAD) return 0;
     const GemvRtForm form = gemv_rt_form(B, d.act, d.c.streams, D);
     bool have_h = !plain;  // d.h holds the coming sublayer's input
     bool first = true;     // plain residual: X is not made yet
@@ -763,7 +764,7 @@ int decode_body_rt(pgmi_ctx* x, hipStream_t s, const int64_t* ids, int B, void* 
         }
         if (!end && q == 0 && d.L[i].experts) { a.zero = d.ecnt; a.nzero = d.zero_words; }
         if (router) residual_route(s, a, d.W[i].router.w, d.W[i].router.ldw, *router);
-        else residual_norm(s, d.act, a);
+        else if (!first || part != STEP_REST) residual_norm(s, d.act, a);
         pend = {};
         first = false;
         have_h = true;
@@ -817,6 +818,7 @@ int decode_body_rt(pgmi_ctx* x, hipStream_t s, const int64_t* ids, int B, void* 
         const LayerW& w = d.W[i];
         const bool fin = gemv_rt_fits(form, w.in.k, d.act);
         read(i, 0);
+        if (part == STEP_HEAD) return 0;
         if (l.mixer == PGMI_MIXER_MAMBA1) {
             const int C = l.inner, N = l.state, R = l.dt_rank, ldc = r8(C);
             float* taps = at<float>(state, st[i].a);
@@ -938,14 +940,15 @@ int decode_body_rt(pgmi_ctx* x, hipStream_t s, const int64_t* ids, int B, void* 
     if (fl) {
         g.out = logits; g.ldo = V; g.pmax = d.pmax; g.pidx = d.pidx;
         gemv_rt(s, d.act, GR_LOGITS, g);
-        const int parts = form == GF_STREAM ? gemv_rt_blocks(g, GR_LOGITS) : 0;
-        if (!parts) argmax_rows(s, logits, B, V, x->amax_v, x->amax_i, next);
-        decode_finish(s, B, d.pmax, d.pidx, parts, next, hist, d.pos);
+        if (form == GF_STREAM) {
+            decode_finish(s, B, d.pmax, d.pidx, gemv_rt_blocks(g, GR_LOGITS), next, hist, d.pos);
+            return 0;
+        }
     } else {
         matmul_rt(s, d.act, d.h, d.ldh, d.head.w, d.head.ldw, B, V, d.head.k, RT_F32, nullptr, logits, V, 0);
-        argmax_rows(s, logits, B, V, x->amax_v, x->amax_i, next);
-        decode_finish(s, B, nullptr, nullptr, 0, next, hist, d.pos);
     }
+    const int parts = argmax_parts(s, logits, B, V, x->amax_v, x->amax_i, next);
+    decode_finish(s, B, x->amax_v, x->amax_i, parts, next, hist, d.pos);
     return 0;
 }
 
@@ -1205,11 +1208,11 @@ int pgmi_decoder_decode(pgmi_ctx* x, const int64_t* ids, int B, const int32_t* s
         for (int& p : d.known_pos) p += n_steps;
     };
     int64_t* nx = next_ids ? next_ids : d.d_next;
-    auto body = [&](hipStream_t st, const int64_t* first) -> int {
+    auto body = [&](hipStream_t st, const int64_t* first, StepPart part = STEP_ALL) -> int {
         for (int t = 0; t < n_steps; ++t) {
             const int r = decode_body_rt(x, st, t == 0 ? first : nx, B, state, n_slots, max_tokens, logits, nx,
-                                         tokens ? tokens + (long)t * B : nullptr);
-            if (r) return r;
+                                         tokens ? tokens + (long)t * B : nullptr, t == 0 ? part : STEP_ALL);
+            if (r || part == STEP_HEAD) return r;
         }
         return 0;
     };
@@ -1219,16 +1222,14 @@ int pgmi_decoder_decode(pgmi_ctx* x, const int64_t* ids, int B, const int32_t* s
         advanced();
         return 0;
     }
-    const int64_t* gids = ids;
-    if (ids != next_ids) {  // a stable address for the graph
-        HIPCHK(hipMemcpyAsync(d.d_ids, ids, (size_t)B * sizeof(int64_t), hipMemcpyDeviceToDevice, s));
-        gids = d.d_ids;
-    }
-    GraphKey key{B, state, n_slots, max_tokens, logits, next_ids, gids, false, 0, n_steps, tokens};
+    // ids fed back in place are read by the graph; others by the step's first launch in front of it, so that the graph holds no
+    // address of them and nothing copies them (a copy is a launch more: 4 us)
+    const bool in_place = ids == next_ids;
+    GraphKey key{B, state, n_slots, max_tokens, logits, next_ids, in_place ? ids : nullptr, false, 0, n_steps, tokens};
     GraphEntry& ge = x->graphs[key];
     if (!ge.exec) {
         if (ge.seen++ == 0) {  // first call with this key: run eagerly (sets kernel attributes)
-            if ((rc = body(s, gids))) return rc;
+            if ((rc = body(s, ids))) return rc;
             LAUNCHCHK();
             advanced();
             return 0;
@@ -1236,7 +1237,7 @@ int pgmi_decoder_decode(pgmi_ctx* x, const int64_t* ids, int B, const int32_t* s
         HIPCHK(hipStreamSynchronize(s));
         hipGraph_t g;
         HIPCHK(hipStreamBeginCapture(x->cap_stream, hipStreamCaptureModeThreadLocal));
-        rc = body(x->cap_stream, gids);
+        rc = body(x->cap_stream, in_place ? ids : nullptr, in_place ? STEP_ALL : STEP_REST);
         HIPCHK(hipStreamEndCapture(x->cap_stream, &g));
         if (rc) {
             (void)hipGraphDestroy(g);
@@ -1245,6 +1246,7 @@ int pgmi_decoder_decode(pgmi_ctx* x, const int64_t* ids, int B, const int32_t* s
         HIPCHK(hipGraphInstantiate(&ge.exec, g, nullptr, nullptr, 0));
         (void)hipGraphDestroy(g);
     }
+    if (!in_place && (rc = body(s, ids, STEP_HEAD))) return rc;
     HIPCHK(hipGraphLaunch(ge.exec, s));
     LAUNCHCHK();
     advanced();

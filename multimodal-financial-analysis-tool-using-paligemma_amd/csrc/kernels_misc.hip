@@ -619,13 +619,18 @@ __global__ void k_argmax_part(const float* __restrict__ x, int V, int slice, flo
 
 int argmax_scratch_parts() { return 1024; }
 
-void argmax_rows(hipStream_t s, const float* x, int rows, int V, float* pmax, int* pidx, int64_t* out) {
+int argmax_parts(hipStream_t s, const float* x, int rows, int V, float* pmax, int* pidx, int64_t* out) {
     int nb = rows >= argmax_scratch_parts() ? 1 : argmax_scratch_parts() / rows;
     nb = std::max(1, std::min(nb, std::min(128, (V + 2047) / 2048)));
     const int slice = ((V + nb - 1) / nb + 3) & ~3;
     nb = (V + slice - 1) / slice;
     hipLaunchKernelGGL(k_argmax_part, dim3(nb, rows), dim3(256), 0, s, x, V, slice, pmax, pidx, out);
-    if (nb > 1) hipLaunchKernelGGL(k_argmax_finish, dim3(rows), dim3(256), 0, s, pmax, pidx, nb, out, nullptr, nullptr);
+    return nb > 1 ? nb : 0;
+}
+
+void argmax_rows(hipStream_t s, const float* x, int rows, int V, float* pmax, int* pidx, int64_t* out) {
+    const int nb = argmax_parts(s, x, rows, V, pmax, pidx, out);
+    if (nb) hipLaunchKernelGGL(k_argmax_finish, dim3(rows), dim3(256), 0, s, pmax, pidx, nb, out, nullptr, nullptr);
 }
 
 // ---------------------------------------------------------------- synthetic weights (bench / tests)

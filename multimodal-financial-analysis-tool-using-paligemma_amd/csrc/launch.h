@@ -125,6 +125,8 @@ void argmax_finish(hipStream_t s, int B, const float* pmax, const int* pidx, int
                    StepState* adv = nullptr, int64_t* hist = nullptr);
 int argmax_scratch_parts();
 void argmax_rows(hipStream_t s, const float* x, int rows, int V, float* pmax, int* pidx, int64_t* out);
+// its first launch alone: the partials per row that are left to join, 0 if out is written
+int argmax_parts(hipStream_t s, const float* x, int rows, int V, float* pmax, int* pidx, int64_t* out);
 void eos_update(hipStream_t s, int64_t* next, int* finished, int B, int64_t eos, int64_t pad, int* n_alive);
 
 // ---------------------------------------------------------------- attention
