@@ -41,17 +41,82 @@ __device__ __forceinline__ float gelu_tanh(float x) {
     return x * __builtin_amdgcn_rcpf(1.0f + e);
 }
 
-__device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+// Values joined across lanes by the vector unit's own lane moves (DPP within 16 lanes, the row swaps past them): a step is one or two
+// instructions.  By ds_bpermute (what __shfl_xor becomes) it is a round trip through LDS of some 100 cycles, six of them for a
+// wave's sum, which nothing hides in a kernel of a few us (a small model's step 296 -> 280 us, a reply 1,071 -> 1,050).  op is
+// commutative, so the tree is the butterfly's and its results are __shfl_xor's to the bit.
+template <int CTRL, typename T>
+__device__ __forceinline__ T lane_move(T v) {
+    return __builtin_bit_cast(T, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xF, 0xF, true));
+}
+constexpr int kDppXor1 = 0xB1, kDppXor2 = 0x4E, kDppHalfMirror = 0x141, kDppRor4 = 0x124, kDppRor8 = 0x128;
+// with lane ^ 16, with lane ^ 32: the swapped pair is (the lower row's, the upper row's) in both rows
+template <typename T, typename Op>
+__device__ __forceinline__ T join_xor16(T v, Op op) {
+    const unsigned u = __builtin_bit_cast(unsigned, v);
+    const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+    return op(__builtin_bit_cast(T, (unsigned)r[0]), __builtin_bit_cast(T, (unsigned)r[1]));
+}
+template <typename T, typename Op>
+__device__ __forceinline__ T join_xor32(T v, Op op) {
+    const unsigned u = __builtin_bit_cast(unsigned, v);
+    const auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+    return op(__builtin_bit_cast(T, (unsigned)r[0]), __builtin_bit_cast(T, (unsigned)r[1]));
+}
+// all 64 lanes, from lane ^ 32 down to lane ^ 1 (behind ^ 8 a row's halves are alike: a turn by 4 is ^ 4)
+template <typename T, typename Op>
+__device__ __forceinline__ T wave_join(T v, Op op) {
+    v = join_xor16(join_xor32(v, op), op);
+    v = op(v, lane_move<kDppRor8>(v));
+    v = op(v, lane_move<kDppRor4>(v));
+    v = op(v, lane_move<kDppXor2>(v));
+    return op(v, lane_move<kDppXor1>(v));
+}
+// groups of N lanes (a power of two), from lane ^ 1 up to lane ^ N / 2 (behind ^ 2 four lanes are alike: a mirrored half row is ^ 4)
+template <int N, typename T, typename Op>
+__device__ __forceinline__ T lanes_join(T v, Op op) {
+    if constexpr (N > 1) v = op(v, lane_move<kDppXor1>(v));
+    if constexpr (N > 2) v = op(v, lane_move<kDppXor2>(v));
+    if constexpr (N > 4) v = op(v, lane_move<kDppHalfMirror>(v));
+    if constexpr (N > 8) v = op(v, lane_move<kDppRor8>(v));
+    if constexpr (N > 16) v = join_xor16(v, op);
+    if constexpr (N > 32) v = join_xor32(v, op);
     return v;
 }
+// groups of n lanes, n a power of two known to the whole wave
+template <typename T, typename Op>
+__device__ __forceinline__ T lanes_join_n(T v, int n, Op op) {
+    if (n > 1) v = op(v, lane_move<kDppXor1>(v));
+    if (n > 2) v = op(v, lane_move<kDppXor2>(v));
+    if (n > 4) v = op(v, lane_move<kDppHalfMirror>(v));
+    if (n > 8) v = op(v, lane_move<kDppRor8>(v));
+    if (n > 16) v = join_xor16(v, op);
+    if (n > 32) v = join_xor32(v, op);
+    return v;
+}
+// inclusive sums over the wave's lanes (lanes that a move finds nothing for add 0)
+__device__ __forceinline__ int wave_scan(int v) {
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xF, 0xF, false);  // the lane before, in a row of 16
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xF, 0xF, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xF, 0xF, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xF, 0xF, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xA, 0xF, false);  // a row's last lane to the next row: rows 1 and 3
+    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xC, 0xF, false);  // lane 31 to rows 2 and 3
+    return v;
+}
+struct SumOp {
+    template <typename T>
+    __device__ __forceinline__ T operator()(T a, T b) const { return a + b; }
+};
+struct MaxOp {
+    __device__ __forceinline__ float operator()(float a, float b) const { return fmaxf(a, b); }
+};
 
-__device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
-    return v;
-}
+__device__ __forceinline__ float wave_sum(float v) { return wave_join(v, SumOp{}); }
+__device__ __forceinline__ float wave_max(float v) { return wave_join(v, MaxOp{}); }
+// over the 4 lanes of one place in a row of 16: ^ 16, then ^ 32
+__device__ __forceinline__ float rows_sum(float v) { return join_xor32(join_xor16(v, SumOp{}), SumOp{}); }
+__device__ __forceinline__ float rows_max(float v) { return join_xor32(join_xor16(v, MaxOp{}), MaxOp{}); }
 
 // 8 bf16 (16 B) dot 8 bf16 with fp32 accumulation via v_dot2_f32_bf16
 __device__ __forceinline__ float dot8(const uint4 a, const uint4 b, float acc) {

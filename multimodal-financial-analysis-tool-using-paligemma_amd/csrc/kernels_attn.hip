@@ -289,9 +289,7 @@ __global__ void __launch_bounds__(256) k_attn_full_pre(AttnArgs a) {
         for (int j = 1; j < MAXT; ++j) mx[r] = fmaxf(mx[r], sc[j][r]);
     }
 #pragma unroll
-    for (int o = 1; o < 16; o <<= 1)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) mx[r] = fmaxf(mx[r], __shfl_xor(mx[r], o, 64));
+    for (int r = 0; r < 4; ++r) mx[r] = lanes_join<16>(mx[r], MaxOp{});
     if (li == 0) {
 #pragma unroll
         for (int r = 0; r < 4; ++r) red[wave * 16 + 4 * g + r] = mx[r];
@@ -309,9 +307,7 @@ __global__ void __launch_bounds__(256) k_attn_full_pre(AttnArgs a) {
         }
     }
 #pragma unroll
-    for (int o = 1; o < 16; o <<= 1)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) sm[r] += __shfl_xor(sm[r], o, 64);
+    for (int r = 0; r < 4; ++r) sm[r] = lanes_join<16>(sm[r], SumOp{});
     if (li == 0) {
 #pragma unroll
         for (int r = 0; r < 4; ++r) red[64 + wave * 16 + 4 * g + r] = sm[r];
@@ -717,8 +713,7 @@ __global__ void __launch_bounds__(256) k_attn_short(AttnArgs a) {
         }
     }
     // ---- exact softmax statistics: lane groups g, then the 4 waves in a fixed order
-    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    mx = rows_max(mx);
     if (g == 0) red[0][wave][li] = mx;
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's V DMAs landed (visible after the barrier)
     __syncthreads();
@@ -731,8 +726,7 @@ __global__ void __launch_bounds__(256) k_attn_short(AttnArgs a) {
             sc[t][r] = sc[t][r] == -INFINITY ? 0.f : fa_exp(sc[t][r] - M);
             sm += sc[t][r];
         }
-    sm += __shfl_xor(sm, 16, 64);
-    sm += __shfl_xor(sm, 32, 64);
+    sm = rows_sum(sm);
     if (g == 0) red[1][wave][li] = sm;
     __syncthreads();
     const float invl = 1.0f / (((red[1][0][li] + red[1][1][li]) + red[1][2][li]) + red[1][3][li]);

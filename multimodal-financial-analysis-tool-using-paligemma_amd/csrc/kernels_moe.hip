@@ -71,10 +71,7 @@ __device__ __forceinline__ TileAt find_tile(const int* cnt, int experts, int BM,
     int total = 0;
     for (int e0 = 0; e0 < experts; e0 += 64) {
         const int c = e0 + lane < experts ? cnt[e0 + lane] : 0;
-        int t = (c + BM - 1) / BM;
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) t += __shfl_xor(t, o, 64);
-        total += t;
+        total += wave_join((c + BM - 1) / BM, SumOp{});
     }
     total *= n_nt;
     const int lin = blockIdx.x, x = lin & 7, j = lin >> 3, q = total >> 3, r = total & 7;
@@ -83,12 +80,7 @@ __device__ __forceinline__ TileAt find_tile(const int* cnt, int experts, int BM,
     for (int e0 = 0; e0 < experts; e0 += 64) {
         const int c = e0 + lane < experts ? cnt[e0 + lane] : 0;
         const int t = (c + BM - 1) / BM * n_nt;
-        int s = t;  // inclusive sum
-#pragma unroll
-        for (int o = 1; o < 64; o <<= 1) {
-            const int u = __shfl_up(s, o, 64);
-            if (lane >= o) s += u;
-        }
+        const int s = wave_scan(t);
         const unsigned long long in = __ballot(idx < s);
         if (in) {
             const int w = __builtin_amdgcn_readfirstlane(__ffsll((long long)in) - 1);

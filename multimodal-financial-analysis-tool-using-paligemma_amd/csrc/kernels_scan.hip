@@ -306,8 +306,7 @@ __global__ void __launch_bounds__(256, LPC == 1 ? 2 : LPC == 4 || LPC == 8 ? 3 :
                         y1 = fmaf(S[i + 1], Cv[at][i / 4][i % 4 + 1], y1);
                     }
                     float y = y0 + y1;
-#pragma unroll
-                    for (int o = 1; o < LPC; o <<= 1) y += __shfl_xor(y, o, 64);
+                    y = lanes_join<LPC>(y, SumOp{});
                     g[t] *= fmaf(Dc, x[t], y);
                     asm volatile("" : "+v"(g[t]));  // (else the sum moves into the stores' branch, with every row's states)
                 }

@@ -509,7 +509,7 @@ __global__ void __launch_bounds__(256) k_gemv_one(GemvRtArgs a) {
 #pragma unroll
         for (int i = 0; i < 8; ++i) q = fmaf(u[i], u[i], q);
         // a group is whole pieces of 512, or a power of two of lanes
-        for (int o = 1; o < 64 && o * 8 < P; o <<= 1) q += __shfl_xor(q, o, 64);
+        q = lanes_join_n(q, P / 8, SumOp{});
         if (P > 512) {
             if (lane == 0 && wave == piece) red[piece] = q;
             __syncthreads();
@@ -982,8 +982,7 @@ __global__ void __launch_bounds__(256) k_scan_step(ScanStepArgs a) {
         for (int v = 0; v < 8; ++v)
             if (r + v < a.R) dt = fmaf(w[v], sm[r + v], dt);
     }
-#pragma unroll
-    for (int o = 1; o < LPC; o <<= 1) dt += __shfl_xor(dt, o, 64);
+    dt = lanes_join<LPC>(dt, SumOp{});
     dt = softplusf_(dt + bf2f(a.dtb[cc]));
     const float x = ldf(reinterpret_cast<const T*>(a.x) + (long)b * a.ldx + cc);
     const float dx = dt * x;
@@ -998,8 +997,7 @@ __global__ void __launch_bounds__(256) k_scan_step(ScanStepArgs a) {
         if (ok) st[n] = S;
         y = fmaf(S, Cv[n], y);
     }
-#pragma unroll
-    for (int o = 1; o < LPC; o <<= 1) y += __shfl_xor(y, o, 64);
+    y = lanes_join<LPC>(y, SumOp{});
     if (sub == 0 && c < a.ldy) {
         y = fmaf(bf2f(a.Dw[cc]), x, y);
         stf(reinterpret_cast<T*>(a.y) + (long)b * a.ldy + c,

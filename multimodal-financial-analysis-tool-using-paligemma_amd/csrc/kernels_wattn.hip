@@ -121,8 +121,7 @@ __global__ void __launch_bounds__(256) k_append(WAttnArgs a) {
             ss = fmaf(v, v, ss);
         }
     }
-#pragma unroll
-    for (int o = 1; o < LPH; o <<= 1) ss += __shfl_xor(ss, o, 64);
+    ss = lanes_join<LPH>(ss, SumOp{});
     const float inv = norm ? 1.0f / sqrtf(ss / (float)n + w.eps) : 1.0f;
     if (head >= NH) return;
     for (int i = sub * V; i < np; i += LPH * V) {
@@ -318,8 +317,7 @@ __global__ void __launch_bounds__(256, D <= 128 ? 2 : 1) k_wattn_f(WAttnArgs a) 
             s[r] = sees(j) ? e : -INFINITY;
             mt = fmaxf(mt, s[r]);
         }
-        mt = fmaxf(mt, __shfl_xor(mt, 16, 64));
-        mt = fmaxf(mt, __shfl_xor(mt, 32, 64));
+        mt = rows_max(mt);
         const float alpha = exp2f(m - mt);
         m = mt;
         l *= alpha;
@@ -374,8 +372,7 @@ __global__ void __launch_bounds__(256, D <= 128 ? 2 : 1) k_wattn_f(WAttnArgs a) 
         vload(tn);
         __builtin_amdgcn_sched_barrier(0);
     }
-    l += __shfl_xor(l, 16, 64);
-    l += __shfl_xor(l, 32, 64);
+    l = rows_sum(l);
     if (lg == 0) { ms[wave][li] = m; ls[wave][li] = l; }
     __syncthreads();
     const float f = exp2f(m - fmaxf(fmaxf(ms[0][li], ms[1][li]), fmaxf(ms[2][li], ms[3][li])));
@@ -555,8 +552,7 @@ __global__ void __launch_bounds__(256 * TEAMS) k_wattn_m(WAttnArgs a) {
             for (int n = 0; n < 4; ++n)
 #pragma unroll
                 for (int r = 0; r < 4; ++r) mt = fmaxf(mt, st[n][r]);
-            mt = fmaxf(mt, __shfl_xor(mt, 16, 64));
-            mt = fmaxf(mt, __shfl_xor(mt, 32, 64));
+            mt = rows_max(mt);
             alpha = __builtin_amdgcn_exp2f(m - mt);
             m = mt;
         }
@@ -615,8 +611,7 @@ __global__ void __launch_bounds__(256 * TEAMS) k_wattn_m(WAttnArgs a) {
             for (int r = 0; r < 4; ++r) o[c][r] = o[c][r] * f1 + o2[r] * f2;
         }
     }
-    l += __shfl_xor(l, 16, 64);
-    l += __shfl_xor(l, 32, 64);
+    l = rows_sum(l);
     if (!ok) return;
     const float inv = 1.0f / l;
     uint16_t* op = reinterpret_cast<uint16_t*>(a.o) + (long)(sq.off + prow) * a.ldo + h * w.e;
@@ -761,9 +756,8 @@ __global__ void __launch_bounds__(256) k_wattn_d(WAttnDecodeArgs a) {
                             for (int v = 0; v < 8; ++v) dot[r] = fmaf(q[v], kv[v], dot[r]);
                         }
                     }
-                for (int o = 1; o < LPK; o <<= 1)
 #pragma unroll
-                    for (int r = 0; r < RB; ++r) dot[r] += __shfl_xor(dot[r], o, 64);
+                for (int r = 0; r < RB; ++r) dot[r] = lanes_join_n(dot[r], LPK, SumOp{});
                 if (kl == 0) {
 #pragma unroll
                     for (int r = 0; r < RB; ++r) {
@@ -942,8 +936,7 @@ __global__ void __launch_bounds__(256, DQ <= 64 && DV <= 64 && HEADS != ODD ? 4 
             for (int c = 0; c < DQ / 32; ++c)
 #pragma unroll
                 for (int v = 0; v < 8; ++v) ss = fmaf(q[c][v], q[c][v], ss);
-            ss += __shfl_xor(ss, 16, 64);
-            ss += __shfl_xor(ss, 32, 64);
+            ss = rows_sum(ss);
             inv = 1.0f / sqrtf(ss / (float)qd + w.eps);
         }
 #pragma unroll
@@ -979,8 +972,7 @@ __global__ void __launch_bounds__(256, DQ <= 64 && DV <= 64 && HEADS != ODD ? 4 
         for (int c = 0; c < DQ / 32; ++c)
 #pragma unroll
             for (int v = 0; v < 8; ++v) dot = fmaf(bf2f((uint16_t)qf[c][v]), bf2f((uint16_t)kf[c][v]), dot);
-        dot += __shfl_xor(dot, 16, 64);
-        dot += __shfl_xor(dot, 32, 64);
+        dot = rows_sum(dot);
         const float s = score.fast(dot, 0.0f);
         float p = 1.0f;
         if constexpr (SC == SC_CAPPED) p = __builtin_amdgcn_exp2f(s);
@@ -996,8 +988,7 @@ __global__ void __launch_bounds__(256, DQ <= 64 && DV <= 64 && HEADS != ODD ? 4 
             }
         float vinv = 1.0f;
         if (w.v_norm) {
-            vss += __shfl_xor(vss, 16, 64);
-            vss += __shfl_xor(vss, 32, 64);
+            vss = rows_sum(vss);
             vinv = 1.0f / sqrtf(vss / (float)ve + w.eps);
         }
 #pragma unroll
@@ -1031,8 +1022,7 @@ __global__ void __launch_bounds__(256, DQ <= 64 && DV <= 64 && HEADS != ODD ? 4 
             }
         float alpha = 1.0f;
         if constexpr (SC != SC_CAPPED) {
-            mt = fmaxf(mt, __shfl_xor(mt, 16, 64));
-            mt = fmaxf(mt, __shfl_xor(mt, 32, 64));
+            mt = rows_max(mt);
             alpha = __builtin_amdgcn_exp2f(m - mt);
             m = mt;
             l *= alpha;
@@ -1067,8 +1057,7 @@ __global__ void __launch_bounds__(256, DQ <= 64 && DV <= 64 && HEADS != ODD ? 4 
         }
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     }
-    l += __shfl_xor(l, 16, 64);
-    l += __shfl_xor(l, 32, 64);
+    l = rows_sum(l);
     if (lg == 0) { sml[wave][li][0] = m; sml[wave][li][1] = l; }
     __syncthreads();
     float M = kNone;
