@@ -828,8 +828,11 @@ __device__ __forceinline__ void fs_vm_wait(int n) {  // s_waitcnt vmcnt(G * min(
 
 // grid (row blocks, n_kv * ns, B); key range sp = blockIdx.y % ns covers tiles [sp * tps, (sp + 1) * tps)
 // P2: scale is a power of two (Gemma: 1/16), so bf16(bf16(x) * scale) = bf16(x) * scale (one rounding)
+// (a workgroup has its CU's LDS to itself: registers for more waves than its own would buy nothing, and taken from the tile in flight
+// they cost 8 us of 34 for 1,056 rows and keys of 8 heads)
 template <int HD, int NW, int LW, int ST, bool P2, int TK>
-__global__ void __launch_bounds__(64 * (NW + LW), 1) k_attn_fs(AttnArgs a, int ns, int tps) {
+__global__ void __launch_bounds__(64 * (NW + LW)) __attribute__((amdgpu_waves_per_eu((NW + LW + 3) / 4, (NW + LW + 3) / 4)))
+k_attn_fs(AttnArgs a, int ns, int tps) {
     using I = FSInfo<HD, TK>;
     constexpr int KS = I::KS, CT = I::CT, CH = I::CH, CR = I::CR, ROWB = I::ROWB, TILEB = I::TILEB;
     constexpr int SLOTB = I::SLOTB, PCS = I::PCS, GPW = PCS / LW;
@@ -916,32 +919,33 @@ __global__ void __launch_bounds__(64 * (NW + LW), 1) k_attn_fs(AttnArgs a, int n
     // P.V operand: lane reads rows vr0 (lo) and vr0 + 16 (hi), columns 16c + 4 (li & 3) .. + 3
     const int vr0 = 4 * g + (li >> 2);
     const int vsw = (vr0 & 7) << 1;
-    // S^T = K Q^T of the tile in `sl`: lane holds keys 16 kt + 4 g + j of query li; even / odd
-    // k-steps accumulate in two chains
-    auto scores = [&](int sl, f32x4 (&ac)[KB][2]) {
-        const uint8_t* kb = fs_sm + sl * SLOTB;
-#pragma unroll
-        for (int kt = 0; kt < KB; ++kt) ac[kt][0] = ac[kt][1] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int kk = 0; kk < KS; ++kk)
-#pragma unroll
-            for (int kt = 0; kt < KB; ++kt) {
-                const int r = kt * 16 + li;
-                const short8 kf = *reinterpret_cast<const short8*>(kb + r * ROWB + (((kk * 4 + g) ^ (r & 15)) << 4));
-                ac[kt][kk & 1] = mfma16(kf, qf[kk], ac[kt][kk & 1]);
-            }
+    // S^T = K Q^T of a tile: lane holds keys 16 kt + 4 g + j of query li; even / odd k-steps accumulate in two chains
+    constexpr int NQ = KS * KB, NS = KB * 4, UV = TK / 32, NV = CT * UV;  // multiplications, a lane's scores
+    short8 kf[NQ], vf[NV];
+    auto kread = [&](int sl, int f) {
+        const int kk = f / KB, r = f % KB * 16 + li;
+        kf[f] = *reinterpret_cast<const short8*>(fs_sm + sl * SLOTB + r * ROWB + (((kk * 4 + g) ^ (r & 15)) << 4));
     };
-    // s = bf16(bf16(k.q) * scale), keys past Lk masked (the last tile only: wave-uniform branch);
-    // returns the tile's max of row li
-    auto finish = [&](int t, const f32x4 (&ac)[KB][2], float (&sv)[KB][4]) -> float {
+    auto vread = [&](int sl, int v) {
+        const int c = v / UV, u = v % UV, cidx = 2 * c + ((li & 3) >> 1);
+        const uint8_t* pl = fs_sm + sl * SLOTB + TILEB + (u * 32 + vr0) * ROWB + ((cidx ^ vsw) << 4) + (li & 1) * 8;
+        const s4v lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s4v*)pl);
+        const s4v hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s4v*)(pl + 16 * ROWB));
+        vf[v] = short8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+    };
+    auto kmul = [&](int f, f32x4 (&ac)[KB][2]) {
+        const int kk = f / KB, kt = f % KB;
+        ac[kt][kk & 1] = mfma16(kf[f], qf[kk], kk < 2 ? f32x4{0.f, 0.f, 0.f, 0.f} : ac[kt][kk & 1]);
+    };
+    // s = bf16(bf16(k.q) * scale)
+    auto score = [&](const f32x4 (&ac)[KB][2], int i, float (&sv)[KB][4]) {
+        const int kt = i / 4, j = i % 4;
+        const float x = rbf(KS > 1 ? ac[kt][0][j] + ac[kt][1][j] : ac[kt][0][j]);
+        sv[kt][j] = P2 ? x * a.scale : rbf(x * a.scale);
+    };
+    // keys past Lk masked (the last tile only: wave-uniform branch); the tile's max of row li
+    auto tile_max = [&](int t, float (&sv)[KB][4]) -> float {
         float mx = -INFINITY;
-#pragma unroll
-        for (int kt = 0; kt < KB; ++kt)
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const float x = rbf(ac[kt][0][j] + ac[kt][1][j]);
-                sv[kt][j] = P2 ? x * a.scale : rbf(x * a.scale);
-            }
         if (t * TK + TK > a.Lk) {
 #pragma unroll
             for (int kt = 0; kt < KB; ++kt)
@@ -953,17 +957,24 @@ __global__ void __launch_bounds__(64 * (NW + LW), 1) k_attn_fs(AttnArgs a, int n
         for (int kt = 0; kt < KB; ++kt)
 #pragma unroll
             for (int j = 0; j < 4; ++j) mx = fmaxf(mx, sv[kt][j]);
-        mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-        return fmaxf(mx, __shfl_xor(mx, 32, 64));
+        return rows_max(mx);
     };
-    // one tile ahead: iteration it multiplies K of tile it + 1 while it runs the softmax and P.V of
-    // tile it (the two are independent, so the MFMAs of one overlap the VALU of the other)
+    // One tile ahead: iteration it multiplies K of tile it + 1 while it runs the softmax of tile it, and V of tile it while it
+    // rounds the scores of it + 1.  A wave has its SIMD alone or shares it with one more, so what it waits for nobody fills:
+    // a fragment is read AH multiplications before its own (left to the compiler, two: each multiplication waited out an LDS
+    // read, 1,056 rows and keys of 8 heads 33.2 us, so 29.6), and the exponentials go between the multiplications.
+    constexpr int AH = NW + LW <= 8 ? 8 : HD > 128 ? 0 : 6;
     float s[KB][4], tm = -INFINITY;
     if (ntl > 0) {
         __builtin_amdgcn_s_barrier();  // barrier 0: tiles 0 and 1 landed
         f32x4 ac[KB][2];
-        scores(0, ac);
-        tm = finish(t0, ac, s);
+#pragma unroll
+        for (int f = 0; f < NQ; ++f) kread(0, f);
+#pragma unroll
+        for (int f = 0; f < NQ; ++f) kmul(f, ac);
+#pragma unroll
+        for (int i = 0; i < NS; ++i) score(ac, i, s);
+        tm = tile_max(t0, s);
     }
     int slot = 0;
     for (int it = 0; it < ntl; ++it) {
@@ -972,8 +983,6 @@ __global__ void __launch_bounds__(64 * (NW + LW), 1) k_attn_fs(AttnArgs a, int n
             __builtin_amdgcn_s_barrier();                         // tiles it and it + 1 in the ring
         }
         const int nslot = slot + 1 == ST ? 0 : slot + 1;
-        f32x4 acn[KB][2];
-        scores(nslot, acn);  // tile it + 1 (past the last tile: stale LDS, never used)
         // deferred running max: raised (and O, l rescaled) only when a row's tile max passes it by
         // kFsDefer; wave-uniform branch
         if (__ballot(tm > m + kFsDefer)) {
@@ -988,34 +997,37 @@ __global__ void __launch_bounds__(64 * (NW + LW), 1) k_attn_fs(AttnArgs a, int n
             }
             m = mn;
         }
-        short8 pa[TK / 32];
+        f32x4 acn[KB][2];  // K of tile it + 1 (past the last tile: stale LDS, never used)
+        short8 pa[UV];
 #pragma unroll
-        for (int kt = 0; kt < KB; ++kt)
+        for (int f = 0; f < AH && f < NQ; ++f) kread(nslot, f);
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
+        for (int f = 0; f < NQ; ++f) {
+            if (f + AH < NQ) kread(nslot, f + AH);
+            else if (f + AH - NQ < NV) vread(slot, f + AH - NQ);
+            kmul(f, acn);
+#pragma unroll
+            for (int i = f * NS / NQ; i < (f + 1) * NS / NQ; ++i) {
+                const int kt = i / 4, j = i % 4;
                 const float e = fa_exp(s[kt][j] - m);  // masked: exp(-inf) = 0
                 l += e;
                 pa[kt / 2][kt % 2 * 4 + j] = (short)f2bf(e);
             }
-        const uint8_t* vb = fs_sm + slot * SLOTB + TILEB;
-#pragma unroll
-        for (int c = 0; c < CT; ++c) {
-            const int cidx = 2 * c + ((li & 3) >> 1);
-#pragma unroll
-            for (int u = 0; u < TK / 32; ++u) {
-                const uint8_t* pl = vb + (u * 32 + vr0) * ROWB + ((cidx ^ vsw) << 4) + (li & 1) * 8;
-                const s4v lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s4v*)pl);
-                const s4v hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s4v*)(pl + 16 * ROWB));
-                const short8 vv = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-                o[c] = mfma16(pa[u], vv, o[c]);
-            }
+            if constexpr (AH > 0) __builtin_amdgcn_sched_barrier(0);
         }
-        tm = finish(t0 + it + 1, acn, s);
+#pragma unroll
+        for (int v = 0; v < NV; ++v) {
+            if (v + AH < NV) vread(slot, v + AH);
+            o[v / UV] = mfma16(pa[v % UV], vf[v], o[v / UV]);
+#pragma unroll
+            for (int i = v * NS / NV; i < (v + 1) * NS / NV; ++i) score(acn, i, s);
+            if constexpr (AH > 0) __builtin_amdgcn_sched_barrier(0);
+        }
+        tm = tile_max(t0 + it + 1, s);
         slot = nslot;
     }
     // row sums: the 4 lane groups of query li, in a fixed order
-    l += __shfl_xor(l, 16, 64);
-    l += __shfl_xor(l, 32, 64);
+    l = rows_sum(l);
     if (ns == 1) {
         const float inv = 1.0f / l;
         uint16_t* orow[4];
@@ -1120,8 +1132,9 @@ static void launch_fs_t(hipStream_t s, const AttnArgs& a, int ns, int tps, dim3 
 
 template <int HD, int NWQ = 0, int TKQ = 0>
 static void launch_fs(hipStream_t s, const AttnArgs& a, int want_ns) {
-    // head dim 256: 4 compute waves (181 registers: with the loaders 2 waves per SIMD) and a 5-slot ring (160 KiB) of 32-key tiles;
-    // 8 compute waves fit too, 3 waves per SIMD of 168 registers, 4 of which are spilled (20 bytes of scratch a lane).  Head dim 72: 8
+    // head dim 256: 4 compute waves (205 registers: with the loaders 2 waves per SIMD) and a 5-slot ring (160 KiB) of 32-key tiles;
+    // 8 compute waves fit too, 3 waves per SIMD of 168 registers, 2 or 3 of which are spilled (16 bytes of scratch a lane; with
+    // fragments read ahead 16, 2 x 1,056 rows 46 -> 61 us).  Head dim 72: 8
     // compute waves, 4 slots of 64-key tiles, whose barriers and row maxima are half as many as of 32 keys in 8 slots (us, 32 / 64
     // keys: 1,024 rows and keys of 16 heads 22.8 / 21.4, of four images 57.4 / 51.2, 256 of eight 14.5 / 14.1).
     // NWQ > 0: that many compute waves; TKQ > 0: tiles of that many keys, in as much LDS
