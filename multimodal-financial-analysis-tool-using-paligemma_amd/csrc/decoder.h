@@ -181,6 +181,7 @@ struct ExpertArgs {
     int ldash, B;
     void* outsh;
     int ldosh;
+    bool dotsh;  // (set by the launcher)
 };
 void experts_rt(hipStream_t s, Act act, ExpertMode mode, const ExpertArgs& a);
 // the same for up to kRouteRows rows of bf16 activations, the shared expert included (EX_STORE: its output is fp32)

@@ -342,7 +342,74 @@ void run_experts_f32(hipStream_t s, const ExpertArgs& a) {
 // U: 64-deep steps a wave has in flight.  WHOLE: K of the experts and of the shared one is a multiple of the 256 U of a turn of the
 // waves, and no load is chosen (ldg16_sel's choice becomes a branch around every load): 8 rows, 48 experts of 1,024 and a shared one
 // of 4,096, width 2,048, gate|up 61.6 -> 57.7 us, down 29.5 -> 28.7.  Eight steps in flight for them too: a step of 8 rows 3 % slower.
-template <int MODE, int U, bool WHOLE>
+// CH > 0 (K of the experts is 512 CH): up to four rows are taken by dot products, each wave whole weight rows as one stream of 1-KiB
+// pieces, as a reply's projections do.  As a matrix instruction's operand 16 rows are read 64 bytes at a time, at 5.3 TB/s, and
+// most of the products are of rows that are not there.  us a step of the 2,048-wide model, of 1, 2, 4, 8 and 16 rows: 742, 905, 1,025, 1,270
+// and 1,495, so 704, 826, 942, 1,150 and 1,354 (up to two rows: 708, 828, 939, 1,157, 1,375; cached weights: 8 rows 1,222).
+template <int MODE, int CH, int R, bool SHARED>
+__device__ __forceinline__ void experts_dot(const ExpertArgs& a, const uint16_t* W, const int* list) {
+    const int N = SHARED ? a.Nsh : a.N, ldw = SHARED ? a.ldwsh : a.ldw;
+    constexpr int NM = MODE == EX_SWIGLU ? 2 : 1, P = NM * CH >= 8 ? 1 : 8 / (NM * CH);  // outputs a turn: 8 pieces in flight
+    const int lane = threadIdx.x & 63, nu = N / P, ustep = gridDim.x * 4;
+    int u = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (u >= nu) return;
+    uint4 w[P][NM][CH], x[R][CH];
+    auto wload = [&](int at) {
+#pragma unroll
+        for (int p = 0; p < P; ++p)
+#pragma unroll
+            for (int q = 0; q < NM; ++q) {
+                const uint16_t* wp = W + ((long)q * N + at * P + p) * ldw + lane * 8;
+#pragma unroll
+                for (int c = 0; c < CH; ++c) w[p][q][c] = ldg_nt(wp + c * 512);
+            }
+    };
+    wload(u);
+    long o[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const int entry = SHARED ? r : list[r];
+        o[r] = (long)entry * (SHARED ? a.ldosh : a.ldo);
+        const uint16_t* xp = reinterpret_cast<const uint16_t*>(SHARED ? a.Ash : a.A) + (SHARED ? (long)r * a.ldash : (long)(entry / a.gather) * a.lda) + lane * 8;
+#pragma unroll
+        for (int c = 0; c < CH; ++c) x[r][c] = ldg16(xp + c * 512);
+    }
+    auto step = [&](auto more) {
+        float acc[P][NM][R];
+#pragma unroll
+        for (int p = 0; p < P; ++p)
+#pragma unroll
+            for (int q = 0; q < NM; ++q)
+#pragma unroll
+                for (int r = 0; r < R; ++r) {
+                    acc[p][q][r] = 0.0f;
+#pragma unroll
+                    for (int c = 0; c < CH; ++c) acc[p][q][r] = dot8(w[p][q][c], x[r][c], acc[p][q][r]);
+                }
+        const int n = u * P;
+        u += ustep;
+        if constexpr (decltype(more)::value) wload(u);
+        float v[R];  // lane p: output n + p
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            float g = 0.0f, h = 0.0f;
+#pragma unroll
+            for (int p = 0; p < P; ++p) {
+                const float s0 = wave_sum(acc[p][0][r]), s1 = NM > 1 ? wave_sum(acc[p][NM - 1][r]) : 0.0f;
+                g = lane == p ? s0 : g;
+                h = lane == p ? s1 : h;
+            }
+            v[r] = MODE == EX_SWIGLU ? siluf_(g) * h : g;
+        }
+        if (lane < P)
+#pragma unroll
+            for (int r = 0; r < R; ++r) reinterpret_cast<uint16_t*>(SHARED ? a.outsh : a.out)[o[r] + n + lane] = f2bf(v[r]);
+    };
+    while (u + ustep < nu) step(std::true_type{});
+    step(std::false_type{});
+}
+
+template <int MODE, int U, bool WHOLE, int CH>
 __global__ void __launch_bounds__(256) k_experts_skinny(ExpertArgs a) {
     constexpr int NM = MODE == EX_SWIGLU ? 2 : 1;
     __shared__ float sums[4][NM][16][17];
@@ -352,9 +419,22 @@ __global__ void __launch_bounds__(256) k_experts_skinny(ExpertArgs a) {
     if (e < 0) return;
     const int N = shared ? a.Nsh : a.N, K = shared ? a.Ksh : a.K, ldw = shared ? a.ldwsh : a.ldw, n0 = blockIdx.x * 16;
     const int ldo = shared ? a.ldosh : a.ldo;
-    if (n0 >= ldo) return;
     const uint16_t* W = shared ? a.Wsh : a.W + e * a.wstride;
     const int* list = a.list + (long)e * a.cap;
+    if constexpr (CH > 0)
+        if (!shared) {
+            const int rows = a.B == 1 ? 1 : a.cnt[e];
+            if (rows == 1) return experts_dot<MODE, CH, 1, false>(a, W, list);
+            if (rows == 2) return experts_dot<MODE, CH, 2, false>(a, W, list);
+            if (rows == 3) return experts_dot<MODE, CH, 3, false>(a, W, list);
+            if (rows == 4) return experts_dot<MODE, CH, 4, false>(a, W, list);
+        } else if (MODE == EX_SWIGLU && a.dotsh) {
+            if (a.B == 1) return experts_dot<MODE, CH, 1, true>(a, W, list);
+            if (a.B == 2) return experts_dot<MODE, CH, 2, true>(a, W, list);
+            if (a.B == 3) return experts_dot<MODE, CH, 3, true>(a, W, list);
+            if (a.B == 4) return experts_dot<MODE, CH, 4, true>(a, W, list);
+        }
+    if (n0 >= ldo) return;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int li = lane & 15, lg = lane >> 4;
     auto ld = [](const uint16_t* p, bool in, const uint16_t* safe) {
@@ -452,7 +532,8 @@ void experts_rt(hipStream_t s, Act act, ExpertMode mode, const ExpertArgs& a) {
     else go(std::integral_constant<int, EX_STORE>{});
 }
 
-void experts_skinny(hipStream_t s, ExpertMode mode, const ExpertArgs& a) {
+void experts_skinny(hipStream_t s, ExpertMode mode, const ExpertArgs& args) {
+    ExpertArgs a = args;
     const int n = std::max(a.ldo, a.Wsh ? a.ldosh : 0);
     // one row lists its choices by place, identities included
     const dim3 grid((n + 15) / 16, 1 + (a.B == 1 ? a.entries : std::min(a.experts, a.entries)));
@@ -461,17 +542,31 @@ void experts_skinny(hipStream_t s, ExpertMode mode, const ExpertArgs& a) {
     // (K of 512 times an odd number, two steps whole instead of four chosen: a step of eight rows over experts of 512 of the 1,024-wide
     // model 498 us for 504, of one row 349 for 350)
     auto whole = [&](int steps) { return a.K % (256 * steps) == 0 && (!a.Wsh || a.Ksh % (256 * steps) == 0); };
-#define SKINNY_(mode, u, w) hipLaunchKernelGGL((k_experts_skinny<mode, u, w>), grid, dim3(256), 0, s, a)
-    if (mode == EX_SWIGLU) {
-        if (a.B == 1 && whole(8)) SKINNY_(EX_SWIGLU, 8, true);
-        else if (whole(4)) SKINNY_(EX_SWIGLU, 4, true);
-        else if (a.B == 1) SKINNY_(EX_SWIGLU, 8, false);
-        else SKINNY_(EX_SWIGLU, 4, false);
-    } else {
-        if (whole(4)) SKINNY_(EX_STORE, 4, true);
-        else if (whole(2)) SKINNY_(EX_STORE, 2, true);
-        else SKINNY_(EX_STORE, 4, false);
+    // dot products: rows of whole 1-KiB pieces, as many outputs as a turn takes, no columns to clear; of the shared expert where it is
+    // the same kind of product (its down product has fp32 outputs and rows of its own length)
+    const int ch = a.K % 512 == 0 && a.ldo == a.N ? a.K / 512 : 0, turn = std::max(1, 8 / (std::max(1, ch) * (mode == EX_SWIGLU ? 2 : 1)));
+    const int dots = (ch == 1 || ch == 2 || ch == 4 || ch == 8) && a.N % turn == 0 ? ch : 0;
+    a.dotsh = mode == EX_SWIGLU && a.Ksh == a.K && a.ldosh == a.Nsh && a.Nsh % turn == 0;
+#define SKINNY_(mode, u, w, c) hipLaunchKernelGGL((k_experts_skinny<mode, u, w, c>), grid, dim3(256), 0, s, a)
+#define DOTS_(mode, u)                              \
+    switch (dots) {                                 \
+        case 1: SKINNY_(mode, u, true, 1); break;   \
+        case 2: SKINNY_(mode, u, true, 2); break;   \
+        case 4: SKINNY_(mode, u, true, 4); break;   \
+        case 8: SKINNY_(mode, u, true, 8); break;   \
+        default: SKINNY_(mode, u, true, 0); break;  \
     }
+    if (mode == EX_SWIGLU) {
+        if (a.B == 1 && whole(8)) { DOTS_(EX_SWIGLU, 8) }
+        else if (whole(4)) { DOTS_(EX_SWIGLU, 4) }
+        else if (a.B == 1) SKINNY_(EX_SWIGLU, 8, false, 0);
+        else SKINNY_(EX_SWIGLU, 4, false, 0);
+    } else {
+        if (whole(4)) { DOTS_(EX_STORE, 4) }
+        else if (whole(2)) { DOTS_(EX_STORE, 2) }
+        else SKINNY_(EX_STORE, 4, false, 0);
+    }
+#undef DOTS_
 #undef SKINNY_
 }
 
