@@ -436,61 +436,113 @@ __global__ void __launch_bounds__(256) k_experts_skinny(ExpertArgs a) {
         }
     if (n0 >= ldo) return;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int li = lane & 15, lg = lane >> 4;
-    auto ld = [](const uint16_t* p, bool in, const uint16_t* safe) {
-        if constexpr (WHOLE) return ldg16(p);
-        else return ldg16_sel(p, in, safe);
-    };
-    const uint16_t* wp[NM];
-#pragma unroll
-    for (int q = 0; q < NM; ++q) wp[q] = W + ((long)q * N + min(n0 + li, N - 1)) * ldw;
-    f32x4 acc[NM];
-#pragma unroll
-    for (int q = 0; q < NM; ++q) acc[q] = f32x4{0.f, 0.f, 0.f, 0.f};
-    const int nstep = (K + 63) / 64;
-    uint4 w[U][NM][2];
-    auto wload = [&](int s0) {
-#pragma unroll
-        for (int i = 0; i < U; ++i) {
-            const int k = (s0 + 4 * i) * 64 + lg * 16;
-#pragma unroll
-            for (int h = 0; h < 2; ++h)
-#pragma unroll
-                for (int q = 0; q < NM; ++q) w[i][q][h] = ld(wp[q] + k + 8 * h, k + 8 * h < K, wp[q]);
-        }
-    };
-    wload(wave);  // in flight while the rows are looked up
+    const int li = lane & 15, lg = lane >> 4, nstep = (K + 63) / 64;
+    const int b = tid >> 4, n = n0 + (tid & 15);  // consecutive threads store consecutive outputs
     const int cnt = shared ? a.B : a.cnt[e];
-    const int m = min(li, cnt - 1), row = shared ? m : list[m] / a.gather;
-    const uint16_t* xp = reinterpret_cast<const uint16_t*>(shared ? a.Ash : a.A) + (long)row * (shared ? a.ldash : a.lda);
-    for (int s0 = wave; s0 < nstep; s0 += 4 * U) {
-        uint4 x[U][2];
+    const uint16_t* A = reinterpret_cast<const uint16_t*>(shared ? a.Ash : a.A);
+    const int lda = shared ? a.ldash : a.lda;
+    float v[2] = {0.f, 0.f};
+    if (WHOLE && cnt <= 8) {  // by whole lines, as k_skinny_lines: 8 outputs and two halves of a step are the 16 weight rows
+        const int k0 = wave * 64 + (li >> 3) * 32 + lg * 8;
+        const uint16_t* wp[NM][2];
+        f32x4 acc[NM][2];
 #pragma unroll
-        for (int i = 0; i < U; ++i) {
-            const int k = (s0 + 4 * i) * 64 + lg * 16;
+        for (int q = 0; q < NM; ++q)
 #pragma unroll
-            for (int h = 0; h < 2; ++h) x[i][h] = ld(xp + k + 8 * h, k + 8 * h < K, xp);
-        }
+            for (int h = 0; h < 2; ++h) {
+                wp[q][h] = W + ((long)q * N + min(n0 + 8 * h + (li & 7), N - 1)) * ldw + k0;
+                acc[q][h] = f32x4{0.f, 0.f, 0.f, 0.f};
+            }
+        uint4 w[U][NM][2];
+        auto wload = [&](int s0) {
 #pragma unroll
-        for (int i = 0; i < U; ++i)
-#pragma unroll
-            for (int h = 0; h < 2; ++h)
+            for (int i = 0; i < U; ++i)
 #pragma unroll
                 for (int q = 0; q < NM; ++q)
-                    acc[q] = mfma16(__builtin_bit_cast(short8, w[i][q][h]), __builtin_bit_cast(short8, x[i][h]), acc[q]);
-        if (s0 + 4 * U < nstep) wload(s0 + 4 * U);
+#pragma unroll
+                    for (int h = 0; h < 2; ++h) w[i][q][h] = ldg_nt(wp[q][h] + (s0 + 4 * i) * 64);
+        };
+        wload(0);  // in flight while the rows are looked up
+        const int m = min(li & 7, cnt - 1);
+        const uint16_t* xp = A + (long)(shared ? m : list[m] / a.gather) * lda + k0;
+        for (int s0 = 0; s0 < nstep; s0 += 4 * U) {
+            uint4 x[U];
+#pragma unroll
+            for (int i = 0; i < U; ++i) x[i] = ldg16(xp + (s0 + 4 * i) * 64);
+#pragma unroll
+            for (int i = 0; i < U; ++i)
+#pragma unroll
+                for (int q = 0; q < NM; ++q)
+#pragma unroll
+                    for (int h = 0; h < 2; ++h)
+                        acc[q][h] = mfma16(__builtin_bit_cast(short8, w[i][q][h]), __builtin_bit_cast(short8, x[i]), acc[q][h]);
+            if (s0 + 4 * U < nstep) wload(s0 + 4 * U);
+        }
+        if ((lg >> 1) == (li >> 3))
+#pragma unroll
+            for (int q = 0; q < NM; ++q)
+#pragma unroll
+                for (int h = 0; h < 2; ++h)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) sums[wave][q][8 * h + 4 * (lg & 1) + r][li] = acc[q][h][r];
+        __syncthreads();
+        if (b < 8)
+#pragma unroll
+            for (int q = 0; q < NM; ++q)
+#pragma unroll
+                for (int u = 0; u < 4; ++u) v[q] += sums[u][q][tid & 15][b] + sums[u][q][tid & 15][b + 8];
+    } else {
+        auto ld = [](const uint16_t* p, bool in, const uint16_t* safe) {
+            if constexpr (WHOLE) return ldg16(p);
+            else return ldg16_sel(p, in, safe);
+        };
+        const uint16_t* wp[NM];
+#pragma unroll
+        for (int q = 0; q < NM; ++q) wp[q] = W + ((long)q * N + min(n0 + li, N - 1)) * ldw;
+        f32x4 acc[NM];
+#pragma unroll
+        for (int q = 0; q < NM; ++q) acc[q] = f32x4{0.f, 0.f, 0.f, 0.f};
+        uint4 w[U][NM][2];
+        auto wload = [&](int s0) {
+#pragma unroll
+            for (int i = 0; i < U; ++i) {
+                const int k = (s0 + 4 * i) * 64 + lg * 16;
+#pragma unroll
+                for (int h = 0; h < 2; ++h)
+#pragma unroll
+                    for (int q = 0; q < NM; ++q) w[i][q][h] = ld(wp[q] + k + 8 * h, k + 8 * h < K, wp[q]);
+            }
+        };
+        wload(wave);  // in flight while the rows are looked up
+        const int m = min(li, cnt - 1), row = shared ? m : list[m] / a.gather;
+        const uint16_t* xp = A + (long)row * lda;
+        for (int s0 = wave; s0 < nstep; s0 += 4 * U) {
+            uint4 x[U][2];
+#pragma unroll
+            for (int i = 0; i < U; ++i) {
+                const int k = (s0 + 4 * i) * 64 + lg * 16;
+#pragma unroll
+                for (int h = 0; h < 2; ++h) x[i][h] = ld(xp + k + 8 * h, k + 8 * h < K, xp);
+            }
+#pragma unroll
+            for (int i = 0; i < U; ++i)
+#pragma unroll
+                for (int h = 0; h < 2; ++h)
+#pragma unroll
+                    for (int q = 0; q < NM; ++q)
+                        acc[q] = mfma16(__builtin_bit_cast(short8, w[i][q][h]), __builtin_bit_cast(short8, x[i][h]), acc[q]);
+            if (s0 + 4 * U < nstep) wload(s0 + 4 * U);
+        }
+#pragma unroll
+        for (int q = 0; q < NM; ++q)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) sums[wave][q][4 * lg + r][li] = acc[q][r];
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < NM; ++q)
+#pragma unroll
+            for (int u = 0; u < 4; ++u) v[q] += sums[u][q][tid & 15][b];
     }
-#pragma unroll
-    for (int q = 0; q < NM; ++q)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) sums[wave][q][4 * lg + r][li] = acc[q][r];
-    __syncthreads();
-    const int b = tid >> 4, n = n0 + (tid & 15);  // consecutive threads store consecutive outputs
-    float v[2] = {0.f, 0.f};
-#pragma unroll
-    for (int q = 0; q < NM; ++q)
-#pragma unroll
-        for (int u = 0; u < 4; ++u) v[q] += sums[u][q][tid & 15][b];
     if (b >= cnt || n >= ldo) return;
     if constexpr (MODE == EX_SWIGLU) v[0] = siluf_(v[0]) * v[1];
     if (n >= N) v[0] = 0.0f;

@@ -698,7 +698,8 @@ void run_mode(hipStream_t s, GemvRtMode mode, const GemvRtArgs& a) {
 // contract k = 16 lg .. 16 lg + 7 and 16 lg + 8 .. 16 lg + 15 of each lane group -- the activations (straight from
 // L2, B fragments) use the same order.  After the waves' sums meet in LDS, thread (n, b) runs the step's epilogue.
 // GR_F32 with gridDim.y > 1: K is cut over the y workgroups too, out holds their partial slabs [y][B][N].
-template <typename T, int MODE>
+// LU > 0: by whole lines (k_skinny_lines), up to 8 rows, a wave's steps of a slice being whole turns of LU.
+template <typename T, int MODE, int LU = 0>
 __global__ void __launch_bounds__(256, sizeof(T) == 4 && MODE != GR_GRU && MODE != GR_SWIGLU ? 4 : 1) k_skinny(GemvRtArgs a) {
     constexpr int NM = MODE == GR_GRU ? 3 : MODE == GR_SWIGLU ? 2 : 1;
     constexpr bool F32 = std::is_same<T, float>::value;
@@ -706,70 +707,114 @@ __global__ void __launch_bounds__(256, sizeof(T) == 4 && MODE != GR_GRU && MODE 
     __shared__ float sums[4][NM][16][17];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int li = lane & 15, lg = lane >> 4, n0 = blockIdx.x * 16, K = a.K;
-    const uint16_t* wp[NM];
+    float v[3] = {0.f, 0.f, 0.f};
+    const int b = tid & 15, n = n0 + (tid >> 4);
+    const int nstep = (K + 63) / 64, per = (nstep + gridDim.y - 1) / gridDim.y, s_end = min(nstep, (int)(blockIdx.y + 1) * per);
+    if constexpr (LU > 0) {
+        const int k0 = wave * 64 + (li >> 3) * 32 + lg * 8;  // this lane's 8 of the wave's first step
+        const uint16_t* xp = reinterpret_cast<const uint16_t*>(a.x) + (long)min(li & 7, a.B - 1) * a.ldx + k0;
+        const uint16_t* wp[NM][2];
+        f32x4 acc[NM][2];
 #pragma unroll
-    for (int m = 0; m < NM; ++m) {
-        const int n = n0 + li < a.N ? n0 + li : a.N - 1;
-        wp[m] = a.W + ((long)m * a.N + n) * a.ldw;
-    }
-    const T* xp = reinterpret_cast<const T*>(a.x) + (long)(li < a.B ? li : a.B - 1) * a.ldx;
-    f32x4 acc[NM], sum[NM];
-#pragma unroll
-    for (int m = 0; m < NM; ++m) sum[m] = acc[m] = f32x4{0.f, 0.f, 0.f, 0.f};
-    int turn = 0;
-    const int nstep = (K + 63) / 64;
-    const int per = (nstep + gridDim.y - 1) / gridDim.y, s_end = min(nstep, (int)(blockIdx.y + 1) * per);
-    for (int s0 = blockIdx.y * per + wave; s0 < s_end; s0 += 4 * U) {
-        uint4 w[U][NM][2];
-        typename X8<T>::type x[U][2];
-#pragma unroll
-        for (int i = 0; i < U; ++i) {
-            const int k = (s0 + 4 * i) * 64 + lg * 16;
+        for (int m = 0; m < NM; ++m)
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
-                const bool ok = s0 + 4 * i < s_end && k + 8 * h < K;
-#pragma unroll
-                for (int m = 0; m < NM; ++m) w[i][m][h] = ldg16_sel(wp[m] + k + 8 * h, ok, wp[m]);
-                if constexpr (F32) ldx(ok ? xp + k + 8 * h : xp, x[i][h]);  // past the end: the weights are zero
-                else x[i][h].q = ldg16_sel(xp + k + 8 * h, ok, xp);
+                wp[m][h] = a.W + ((long)m * a.N + min(n0 + h * 8 + (li & 7), a.N - 1)) * a.ldw + k0;
+                acc[m][h] = f32x4{0.f, 0.f, 0.f, 0.f};
             }
+        for (int s0 = blockIdx.y * per; s0 < s_end; s0 += 4 * LU) {
+            uint4 w[LU][NM][2], x[LU];
+#pragma unroll
+            for (int i = 0; i < LU; ++i) {
+#pragma unroll
+                for (int m = 0; m < NM; ++m)
+#pragma unroll
+                    for (int h = 0; h < 2; ++h) w[i][m][h] = ldg_nt(wp[m][h] + (s0 + 4 * i) * 64);
+                x[i] = ldg16(xp + (s0 + 4 * i) * 64);
+            }
+#pragma unroll
+            for (int i = 0; i < LU; ++i)
+#pragma unroll
+                for (int m = 0; m < NM; ++m)
+#pragma unroll
+                    for (int h = 0; h < 2; ++h)
+                        acc[m][h] = mfma16(__builtin_bit_cast(short8, w[i][m][h]), __builtin_bit_cast(short8, x[i]), acc[m][h]);
         }
+        if ((lg >> 1) == (li >> 3))
 #pragma unroll
-        for (int i = 0; i < U; ++i)
+            for (int m = 0; m < NM; ++m)
 #pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                if constexpr (F32) {  // tile_f32.h's pieces, the smallest first
-                    const F32Pieces q = cut8(x[i][h].a, x[i][h].b);
+                for (int h = 0; h < 2; ++h)
 #pragma unroll
-                    for (int p = 2; p >= 0; --p)
+                    for (int r = 0; r < 4; ++r) sums[wave][m][8 * h + 4 * (lg & 1) + r][li] = acc[m][h][r];
+        __syncthreads();
+        if (b < 8)
 #pragma unroll
-                        for (int m = 0; m < NM; ++m)
-                            acc[m] = mfma16(__builtin_bit_cast(short8, w[i][m][h]), __builtin_bit_cast(short8, q.p[p]), acc[m]);
-                } else {
+            for (int m = 0; m < NM; ++m)
 #pragma unroll
-                    for (int m = 0; m < NM; ++m)
-                        acc[m] = mfma16(__builtin_bit_cast(short8, w[i][m][h]), __builtin_bit_cast(short8, x[i][h].q), acc[m]);
+                for (int q = 0; q < 4; ++q) v[m] += sums[q][m][tid >> 4][b] + sums[q][m][tid >> 4][b + 8];
+    } else {
+        const uint16_t* wp[NM];
+#pragma unroll
+        for (int m = 0; m < NM; ++m) {
+            const int n = n0 + li < a.N ? n0 + li : a.N - 1;
+            wp[m] = a.W + ((long)m * a.N + n) * a.ldw;
+        }
+        const T* xp = reinterpret_cast<const T*>(a.x) + (long)(li < a.B ? li : a.B - 1) * a.ldx;
+        f32x4 acc[NM], sum[NM];
+#pragma unroll
+        for (int m = 0; m < NM; ++m) sum[m] = acc[m] = f32x4{0.f, 0.f, 0.f, 0.f};
+        int turn = 0;
+        for (int s0 = blockIdx.y * per + wave; s0 < s_end; s0 += 4 * U) {
+            uint4 w[U][NM][2];
+            typename X8<T>::type x[U][2];
+#pragma unroll
+            for (int i = 0; i < U; ++i) {
+                const int k = (s0 + 4 * i) * 64 + lg * 16;
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    const bool ok = s0 + 4 * i < s_end && k + 8 * h < K;
+#pragma unroll
+                    for (int m = 0; m < NM; ++m) w[i][m][h] = ldg16_sel(wp[m] + k + 8 * h, ok, wp[m]);
+                    if constexpr (F32) ldx(ok ? xp + k + 8 * h : xp, x[i][h]);  // past the end: the weights are zero
+                    else x[i][h].q = ldg16_sel(xp + k + 8 * h, ok, xp);
                 }
             }
-        if (F32 && (++turn & 3) == 0) {  // 1024 of k, as tile_f32 (of K = 16384, positive: 3.6e-6 without, an FMA chain 2.0e-6)
 #pragma unroll
-            for (int m = 0; m < NM; ++m) {
-                sum[m] += acc[m];
-                acc[m] = f32x4{0.f, 0.f, 0.f, 0.f};
+            for (int i = 0; i < U; ++i)
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    if constexpr (F32) {  // tile_f32.h's pieces, the smallest first
+                        const F32Pieces q = cut8(x[i][h].a, x[i][h].b);
+#pragma unroll
+                        for (int p = 2; p >= 0; --p)
+#pragma unroll
+                            for (int m = 0; m < NM; ++m)
+                                acc[m] = mfma16(__builtin_bit_cast(short8, w[i][m][h]), __builtin_bit_cast(short8, q.p[p]), acc[m]);
+                    } else {
+#pragma unroll
+                        for (int m = 0; m < NM; ++m)
+                            acc[m] = mfma16(__builtin_bit_cast(short8, w[i][m][h]), __builtin_bit_cast(short8, x[i][h].q), acc[m]);
+                    }
+                }
+            if (F32 && (++turn & 3) == 0) {  // 1024 of k, as tile_f32 (of K = 16384, positive: 3.6e-6 without, an FMA chain 2.0e-6)
+#pragma unroll
+                for (int m = 0; m < NM; ++m) {
+                    sum[m] += acc[m];
+                    acc[m] = f32x4{0.f, 0.f, 0.f, 0.f};
+                }
             }
         }
+#pragma unroll
+        for (int m = 0; m < NM; ++m)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) sums[wave][m][4 * lg + r][li] = F32 ? sum[m][r] + acc[m][r] : acc[m][r];
+        __syncthreads();
+#pragma unroll
+        for (int m = 0; m < NM; ++m)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) v[m] += sums[q][m][tid >> 4][b];
     }
-#pragma unroll
-    for (int m = 0; m < NM; ++m)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) sums[wave][m][4 * lg + r][li] = F32 ? sum[m][r] + acc[m][r] : acc[m][r];
-    __syncthreads();
-    const int b = tid & 15, n = n0 + (tid >> 4);
-    float v[3] = {0.f, 0.f, 0.f};
-#pragma unroll
-    for (int m = 0; m < NM; ++m)
-#pragma unroll
-        for (int q = 0; q < 4; ++q) v[m] += sums[q][m][tid >> 4][b];
     if constexpr (F32) {
         // what is not finite (of rows and outputs that there are): FMA chains over this workgroup's K slice, as tile_f32
         __shared__ int flag[4];
@@ -894,6 +939,80 @@ __global__ void __launch_bounds__(256) k_skinny_held(GemvRtArgs a) {
     step_pads<uint16_t, MODE>(a);
 }
 
+// The same for up to 8 rows and K of 256 ST, by whole lines: 8 outputs and two halves of each 64-deep step are the 16 rows of one
+// matrix operand, the 8 rows of activations and the same halves the 16 of the other, so a load instruction reads 8 rows by 128
+// bytes, each line once and by one instruction (16 rows by half of a line, twice, need the cache between them, and are slower
+// uncached).  Of the product's quarters the two of unlike halves are not used, the two others added.  8 rows, output matrix of 257,216 x
+// 2,048 182 -> 172 us, 3 rows 187 -> 158; 256 to 1,280 workgroups measured equal.
+template <int MODE, int ST>
+__global__ void __launch_bounds__(256) k_skinny_lines(GemvRtArgs a) {
+    constexpr int NM = MODE == GR_SWIGLU ? 2 : 1;
+    __shared__ float sums[2][4][NM][16][17];  // [.][wave][matrix][output][half and row]
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int li = lane & 15, lg = lane >> 4, ngroup = (a.N + 15) / 16;
+    const int k0 = wave * 64 + (li >> 3) * 32 + lg * 8;  // this lane's 8 of the wave's first step
+    const uint16_t* xp = reinterpret_cast<const uint16_t*>(a.x) + (long)min(li & 7, a.B - 1) * a.ldx + k0;
+    short8 x[ST];
+#pragma unroll
+    for (int i = 0; i < ST; ++i) x[i] = __builtin_bit_cast(short8, ldg16(xp + i * 256));
+    uint4 w[NM][2][ST];
+    int grp = blockIdx.x, turn = 0;
+    auto wload = [&]() {
+#pragma unroll
+        for (int m = 0; m < NM; ++m)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const uint16_t* p = a.W + ((long)m * a.N + min(grp * 16 + h * 8 + (li & 7), a.N - 1)) * a.ldw + k0;
+#pragma unroll
+                for (int i = 0; i < ST; ++i) w[m][h][i] = ldg_nt(p + i * 256);
+            }
+    };
+    wload();
+    auto step = [&](auto more) {
+        const int n0 = grp * 16;
+        f32x4 acc[NM][2];
+#pragma unroll
+        for (int m = 0; m < NM; ++m)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                acc[m][h] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int i = 0; i < ST; ++i) acc[m][h] = mfma16(__builtin_bit_cast(short8, w[m][h][i]), x[i], acc[m][h]);
+            }
+        grp += gridDim.x;
+        if constexpr (decltype(more)::value) wload();
+        // lane: products of operand rows 4 lg .. (output % 8, half lg / 2) with column li (row % 8, half li / 8)
+        if ((lg >> 1) == (li >> 3))
+#pragma unroll
+            for (int m = 0; m < NM; ++m)
+#pragma unroll
+                for (int h = 0; h < 2; ++h)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) sums[turn][wave][m][8 * h + 4 * (lg & 1) + r][li] = acc[m][h][r];
+        __syncthreads();  // (the sums of two turns back are read before the barrier in between)
+        const int b = tid >> 4, n = n0 + (tid & 15);  // consecutive threads store consecutive outputs
+        float v[2] = {0.f, 0.f};
+        if (b < 8)
+#pragma unroll
+            for (int m = 0; m < NM; ++m)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) v[m] += sums[turn][q][m][tid & 15][b] + sums[turn][q][m][tid & 15][b + 8];
+        turn ^= 1;
+        if (b >= a.B || n >= a.N) return;
+        if constexpr (MODE == GR_F32) reinterpret_cast<float*>(a.out)[(long)b * a.ldo + n] = v[0];
+        else step_epilogue<uint16_t, MODE>(a, n, b, v[0], v[1], 0.f);
+    };
+    while (grp + (int)gridDim.x < ngroup) step(std::true_type{});
+    step(std::false_type{});
+    step_pads<uint16_t, MODE>(a);
+}
+
+template <int ST>
+void run_lines(hipStream_t s, GemvRtMode mode, const GemvRtArgs& a, int blocks) {
+    if (mode == GR_SWIGLU) hipLaunchKernelGGL((k_skinny_lines<GR_SWIGLU, ST>), dim3(blocks), dim3(256), 0, s, a);
+    else hipLaunchKernelGGL((k_skinny_lines<GR_F32, ST>), dim3(blocks), dim3(256), 0, s, a);
+}
+
 template <int ST, bool PART = true>
 void run_held(hipStream_t s, GemvRtMode mode, const GemvRtArgs& a, int blocks) {
     if (PART && a.K % 256 == 0) return run_held<ST, false>(s, mode, a, blocks);
@@ -910,6 +1029,17 @@ void run_skinny(hipStream_t s, GemvRtMode mode, const GemvRtArgs& a) {
     // 285; 65,536 outputs at 512 122 / 117 and 130 / 122, at 1,000 137 / 137 and 143 / 142, at 2,048 181 / 178 and 195 / 186
     const bool pays = a.K >= 512 && (mode == GR_SWIGLU || mode == GR_F32 || mode == GR_LOGITS);
     if (std::is_same<T, uint16_t>::value && pays && a.K <= 2048 && a.split <= 1 && (int)grid.x > kHeldBlocks) {
+        if (a.B <= 8 && a.K % 256 == 0) {
+            switch (a.K / 256) {
+                case 2: run_lines<2>(s, mode, a, kHeldBlocks); return;
+                case 3: run_lines<3>(s, mode, a, kHeldBlocks); return;
+                case 4: run_lines<4>(s, mode, a, kHeldBlocks); return;
+                case 5: run_lines<5>(s, mode, a, kHeldBlocks); return;
+                case 6: run_lines<6>(s, mode, a, kHeldBlocks); return;
+                case 7: run_lines<7>(s, mode, a, kHeldBlocks); return;
+                default: run_lines<8>(s, mode, a, kHeldBlocks); return;
+            }
+        }
         switch ((a.K + 255) / 256) {
             case 2: run_held<2>(s, mode, a, kHeldBlocks); break;
             case 3: run_held<3>(s, mode, a, kHeldBlocks); break;
@@ -921,13 +1051,32 @@ void run_skinny(hipStream_t s, GemvRtMode mode, const GemvRtArgs& a) {
         }
         return;
     }
+    // By whole lines: turns of 8 steps a wave (of several matrices 4), of short rows fewer.  us a step of the 2,048-wide streams model,
+    // 2 and 8 rows: 801 -> 761, 867 -> 816.  Matrices under 4 MB, whose time is not their bytes', as before (1,536 outputs of
+    // K = 1,024: a step of 8 layers 408 -> 411)
+    int turn = 0;
+    const int nm = mode == GR_GRU ? 3 : mode == GR_SWIGLU ? 2 : 1;
+    if (std::is_same<T, uint16_t>::value && a.B <= 8 && a.K % (64 * std::max(1, a.split)) == 0 && (long)nm * a.N * a.K >= 2 << 20) {
+        const int steps = a.K / 64 / std::max(1, a.split);  // of a slice, dealt to four waves
+        for (int u = nm > 1 ? 4 : 8; u >= 2 && !turn; u /= 2)
+            if (steps % (4 * u) == 0) turn = u;
+    }
+    auto go = [&](auto mode_c, dim3 g) {
+        constexpr int MODE = decltype(mode_c)::value;
+        if constexpr (std::is_same<T, uint16_t>::value) {
+            if (turn == 8) { hipLaunchKernelGGL((k_skinny<T, MODE, 8>), g, block, 0, s, a); return; }
+            if (turn == 4) { hipLaunchKernelGGL((k_skinny<T, MODE, 4>), g, block, 0, s, a); return; }
+            if (turn == 2) { hipLaunchKernelGGL((k_skinny<T, MODE, 2>), g, block, 0, s, a); return; }
+        }
+        hipLaunchKernelGGL((k_skinny<T, MODE>), g, block, 0, s, a);
+    };
     switch (mode) {
-        case GR_ACT: hipLaunchKernelGGL((k_skinny<T, GR_ACT>), grid, block, 0, s, a); break;
-        case GR_CONV: hipLaunchKernelGGL((k_skinny<T, GR_CONV>), grid, block, 0, s, a); break;
-        case GR_GRU: hipLaunchKernelGGL((k_skinny<T, GR_GRU>), grid, block, 0, s, a); break;
-        case GR_SWIGLU: hipLaunchKernelGGL((k_skinny<T, GR_SWIGLU>), grid, block, 0, s, a); break;
-        case GR_STREAMS: hipLaunchKernelGGL((k_skinny<T, GR_STREAMS>), grid, block, 0, s, a); break;
-        default: hipLaunchKernelGGL((k_skinny<T, GR_F32>), dim3(grid.x, a.split < 1 ? 1 : a.split), block, 0, s, a); break;
+        case GR_ACT: go(std::integral_constant<int, GR_ACT>{}, grid); break;
+        case GR_CONV: go(std::integral_constant<int, GR_CONV>{}, grid); break;
+        case GR_GRU: go(std::integral_constant<int, GR_GRU>{}, grid); break;
+        case GR_SWIGLU: go(std::integral_constant<int, GR_SWIGLU>{}, grid); break;
+        case GR_STREAMS: go(std::integral_constant<int, GR_STREAMS>{}, grid); break;
+        default: go(std::integral_constant<int, GR_F32>{}, dim3(grid.x, a.split < 1 ? 1 : a.split)); break;
     }
 }
 
