@@ -509,6 +509,7 @@ static int decode_body(pgmi_ctx* x, hipStream_t s, const int64_t* ids, int B, vo
     // 5.97 -> 7.59 us for a combine no shorter, 4.63 -> 4.72 us; with the combine inside the down launch,
     // B = 8 step 1.437 -> 1.446-1.465 ms, same box.)
     const bool mf = B >= gemv_mf_min_batch() && !mf_staged(x);
+    const uint16_t* fnorm = W(x, "language_model.model.norm.weight");
     if (mf && c.t_layers > 0) rows_norm(s, x->dH, TL(x, 0, "input_layernorm.weight"), eps, B, H, x->dHn);
     for (int i = 0; i < c.t_layers; ++i) {
         uint16_t* Kc = kvp + ((long)(i * 2 + 0) * kv_batch) * kvb;
@@ -541,7 +542,7 @@ static int decode_body(pgmi_ctx* x, hipStream_t s, const int64_t* ids, int B, vo
             gemv_geglu(s, B, x->dH, TL(x, i, "post_attention_layernorm.weight"), eps, TL(x, i, "mlp.gate_proj.weight"),
                        c.t_intermediate, x->dACT, x->dSS, Lf);
             gemv_res_norm(s, B, c.t_intermediate, x->dACT, TL(x, i, "mlp.down_proj.weight"), H, x->dH, x->ws,
-                          i + 1 < c.t_layers ? TL(x, i + 1, "input_layernorm.weight") : nullptr, eps, x->dHn,
+                          i + 1 < c.t_layers ? TL(x, i + 1, "input_layernorm.weight") : fnorm, eps, x->dHn,
                           Lf ? Lf + gu_n + qkv_n + (size_t)H * NH * HD : nullptr);
             continue;
         }
@@ -553,7 +554,8 @@ static int decode_body(pgmi_ctx* x, hipStream_t s, const int64_t* ids, int B, vo
     int64_t* nx = next_ids ? next_ids : x->d_next;
     // the step's last work also advances the device step state (pgmi_decode skips its host-side
     // set when the next call continues the sequence): lm_head's last workgroup, or argmax_finish
-    if (!gemv_logits(s, B, x->dH, W(x, "language_model.model.norm.weight"), eps, E, c.t_vocab, logits, x->pmax,
+    const bool normed = mf && c.t_layers > 0;  // by the last layer's combine
+    if (!gemv_logits(s, B, normed ? x->dHn : x->dH, normed ? nullptr : fnorm, eps, E, c.t_vocab, logits, x->pmax,
                      x->pidx, &nparts, x->lm_done, nx, x->step, hist))
         argmax_finish(s, B, x->pmax, x->pidx, nparts, nx, x->step, hist);
     return 0;

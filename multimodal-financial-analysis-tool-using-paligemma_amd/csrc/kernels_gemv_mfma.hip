@@ -16,6 +16,7 @@
 //     fused in, or read from global (o_proj's and down_proj's inputs);
 //   - epilogues and rounding points exactly as gemv_body.h (RoPE + KV append, GeGLU, residual,
 //     fp32 logits + per-workgroup first-max argmax partials).
+#include <algorithm>
 #include <cstdlib>
 
 #include "gemv_body.h"
@@ -732,6 +733,76 @@ __global__ void k_mf_combine(const float* __restrict__ ws, int KS, int nb, int N
     h[i] = f2bf(rbf(s) + bf2f(h[i]));
 }
 
+// The tied output matrix over normalised rows (a.x), up to 8 of them, K = 2048: 8 outputs and two halves of each 64-deep step are the
+// 16 rows of one matrix operand, the rows and the same halves the 16 of the other, so a load instruction reads 8 weight rows by
+// 128 bytes and a line is read once, straight into registers; of the product's quarters the two of like halves are added.
+// Bound by the stream: 257,216 outputs, 8 rows, 176 us through the LDS-DMA ring (k_gemv_ml, 256 bytes of a row at a time), so 163.
+__global__ void __launch_bounds__(256) k_logits_lines(GemvArgs a) {
+    constexpr int ST = 8;  // 64-deep steps of a wave: the four waves split K
+    __shared__ float sums[2][4][16][17];
+    __shared__ float bv[8][16];
+    __shared__ int bi[8][16];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int li = lane & 15, lg = lane >> 4, N = a.n_units, ngroup = (N + 15) / 16;
+    const int k0 = wave * 64 + (li >> 3) * 32 + lg * 8;  // this lane's 8 of the wave's first step
+    const uint16_t* xp = a.x + (long)min(li & 7, a.nb - 1) * 2048 + k0;
+    short8 x[ST];
+#pragma unroll
+    for (int i = 0; i < ST; ++i) x[i] = __builtin_bit_cast(short8, ldg16(xp + i * 256));
+    uint4 w[2][ST];
+    int grp = blockIdx.x, turn = 0;
+    auto wload = [&]() {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const uint16_t* p = a.W + (long)min(grp * 16 + h * 8 + (li & 7), N - 1) * 2048 + k0;
+#pragma unroll
+            for (int i = 0; i < ST; ++i) w[h][i] = ldg_nt(p + i * 256);
+        }
+    };
+    wload();
+    const int b = tid >> 4, nn = tid & 15;
+    float best = -INFINITY;
+    int besti = 0x7fffffff;
+    auto step = [&](auto more) {
+        const int n = grp * 16 + nn;
+        f32x4 acc[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+        for (int i = 0; i < ST; ++i)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) acc[h] = mfma16(__builtin_bit_cast(short8, w[h][i]), x[i], acc[h]);
+        grp += gridDim.x;
+        if constexpr (decltype(more)::value) wload();
+        // lane: products of operand rows 4 lg .. (output % 8, half lg / 2) with column li (row % 8, half li / 8)
+        if ((lg >> 1) == (li >> 3))
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) sums[turn][wave][8 * h + 4 * (lg & 1) + r][li] = acc[h][r];
+        __syncthreads();  // (the sums of two turns back are read before the barrier in between)
+        if (b < a.nb && n < N) {
+            float v = 0.f;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) v += sums[turn][q][nn][b] + sums[turn][q][nn][b + 8];
+            v = rbf(v);
+            a.logits[(long)b * N + n] = v;
+            if (v > best) { best = v; besti = n; }
+        }
+        turn ^= 1;
+    };
+    while (grp + (int)gridDim.x < ngroup) step(std::true_type{});
+    step(std::false_type{});
+    if (b < 8) { bv[b][nn] = best; bi[b][nn] = besti; }
+    __syncthreads();
+    if (tid < a.nb) {
+        float m = bv[tid][0];
+        int mi = bi[tid][0];
+        for (int q = 1; q < 16; ++q)
+            if (bv[tid][q] > m || (bv[tid][q] == m && bi[tid][q] < mi)) { m = bv[tid][q]; mi = bi[tid][q]; }
+        a.pmax[(long)tid * gridDim.x + blockIdx.x] = m;
+        a.pidx[(long)tid * gridDim.x + blockIdx.x] = mi;
+    }
+}
+
 // One workgroup per batch row: RMSNorm (modeling_gemma.py:114-120) of x -> out, the rows the
 // unstaged batched projections read.  Every thread's chunks are loaded before the reduction.
 __global__ void __launch_bounds__(256) k_rows_norm(const uint16_t* __restrict__ x, const uint16_t* __restrict__ w,
@@ -920,6 +991,11 @@ void gemv_mf_ores(hipStream_t s, const GemvArgs& a, uint16_t* o) {
 int gemv_mf_logits(hipStream_t s, const GemvArgs& a, int max_blocks) {  // K = 2048
     // (the register-streamed form at 512 / 1,024 / 2,048 workgroups measured no faster: 1.741-1.768 ms; again in
     // with the peeled loop: B = 8 step 1.283 -> 1.330-1.341 ms, profiles/r05_b8_lm_mf_ab.txt)
+    if (!a.norm_w && a.nb <= 8 && a.K == 2048) {  // rows normalised already
+        const int blocks = std::min({groups_of(a.n_units), max_blocks, 512});
+        hipLaunchKernelGGL(k_logits_lines, dim3(blocks), dim3(256), 0, s, a);
+        return blocks;
+    }
     const int blocks = ms_blocks(a.n_units, max_blocks < 256 ? max_blocks : 256);
     launch_ml<GV_LOGITS, 1, 2048, 6>(s, a, blocks, 1, nullptr);
     return blocks;
