@@ -39,10 +39,14 @@ __global__ void __launch_bounds__(64 * WM * WN) k_matmul_f32(F32Args a) {
     float* out = a.out + (long)blockIdx.y * a.M * a.ldo;
     tile_f32<WM, WN, TM, TN, NB>(
         a.A, a.lda, a.W, a.ldw, (long)a.N * a.ldw, a.N, a.ldo, n0, k0, k1, [&](int m) { return min(m0 + m, a.M - 1); },
-        [&](int m, int n, float v, float u) {
+        [&](int n) {
+            if constexpr (NB == 2) return 0.0f;
+            else return a.bias ? bf2f(a.bias[min(n, a.N - 1)]) : 0.0f;
+        },
+        [&](int m, int n, float v, float u, float b) {
             if (m0 + m >= a.M) return;
             if constexpr (NB == 2) v = siluf_(v) * u;
-            else if (a.bias && n < a.N) v += bf2f(a.bias[n]);
+            else if (a.bias) v += b;
             out[(long)(m0 + m) * a.ldo + n] = n < a.N ? v : 0.0f;
         });
 }

@@ -316,7 +316,8 @@ __global__ void __launch_bounds__(64 * WM * WN) k_experts_f32(ExpertArgs a) {
     tile_f32<WM, WN, TM, TN, NB>(
         reinterpret_cast<const float*>(a.A), a.lda, a.W + tl.e * a.wstride, a.ldw, (long)a.N * a.ldw, a.N, a.ldo, tl.nt * BN, 0,
         a.K, [&](int m) { return list[min(tl.m0 + m, tl.cnt - 1)] / a.gather; },
-        [&](int m, int n, float v, float u) {
+        [](int) { return 0.0f; },
+        [&](int m, int n, float v, float u, float) {
             if (tl.m0 + m >= tl.cnt) return;
             if constexpr (MODE == EX_SWIGLU) v = siluf_(v) * u;
             out[(long)list[tl.m0 + m] * a.ldo + n] = n < a.N ? v : 0.0f;

@@ -52,11 +52,11 @@ constexpr size_t tile_f32_lds(int BM, int BN, int NB) { return (size_t)2 * (3 * 
 
 // One tile: rows [0, BM) of the caller's (source(m): the A row of tile row m, always a readable one), columns n0 .. n0 + BN
 // of W and, with NB = 2, the same columns `up` elements further on; k in [k0, k1), both multiples of 8.  WM x WN waves of
-// TM x TN 16 x 16 blocks.  put(m, n, v, v_up) gets every element of the tile with n < ncol; columns past N hold the last
+// TM x TN 16 x 16 blocks.  put(m, n, v, v_up, bias(n)) gets every element of the tile with n < ncol; columns past N hold the last
 // column's values.  A row past the caller's own is dropped by put.
-template <int WM, int WN, int TM, int TN, int NB, typename Source, typename Put>
+template <int WM, int WN, int TM, int TN, int NB, typename Source, typename Bias, typename Put>
 __device__ __forceinline__ void tile_f32(const float* __restrict__ A, int lda, const uint16_t* __restrict__ W, int ldw, long up,
-                                         int N, int ncol, int n0, int k0, int k1, const Source& source, const Put& put) {
+                                         int N, int ncol, int n0, int k0, int k1, const Source& source, const Bias& bias, const Put& put) {
     constexpr int NT = 64 * WM * WN, BM = 16 * WM * TM, BN = 16 * WN * TN;
     constexpr int CA = BM * 8 / NT, CW = NB * BN * 8 / NT;  // 8-element chunks that a thread moves per step
     static_assert(CA * NT == BM * 8 && CW * NT == NB * BN * 8, "whole chunks");
@@ -73,6 +73,11 @@ __device__ __forceinline__ void tile_f32(const float* __restrict__ A, int lda, c
         const int r = (tid + NT * i) >> 3;
         wp[i] = W + (NB == 2 ? (r / BN) * up : 0L) + (long)min(n0 + r % BN, N - 1) * ldw;
     }
+    // ahead of the steps: asked for where it is added, each output waits for its own load, and for the store of the one before
+    // (500 rows, 3,072 and 1,536 outputs of K = 1,024: 21.9 and 16.0 us, so 20.7 and 15.1)
+    float bv[TN];
+#pragma unroll
+    for (int j = 0; j < TN; ++j) bv[j] = bias(n0 + (wn * TN + j) * 16 + (lane & 15));
     struct Step { float4 a[CA][2]; uint4 w[CW]; };
     auto load = [&](int t, Step& s) {  // a chunk at or past k1 is read at k0 instead, and its weights are zero
         const int k = k0 + t * 64 + c8 * 8, kk = k < k1 ? k : k0;
@@ -247,7 +252,7 @@ __device__ __forceinline__ void tile_f32(const float* __restrict__ A, int lda, c
             const int n = n0 + (wn * TN + j) * 16 + li;
 #pragma unroll
             for (int r = 0; r < 4; ++r)
-                if (n < ncol) put((wm * TM + i) * 16 + lg * 4 + r, n, sum[0][i][j][r], sum[NB - 1][i][j][r]);
+                if (n < ncol) put((wm * TM + i) * 16 + lg * 4 + r, n, sum[0][i][j][r], sum[NB - 1][i][j][r], bv[j]);
         }
 }
 
