@@ -45,23 +45,46 @@ __device__ __forceinline__ float gelu_tanh(float x) {
 // instructions.  By ds_bpermute (what __shfl_xor becomes) it is a round trip through LDS of some 100 cycles, six of them for a
 // wave's sum, which nothing hides in a kernel of a few us (a small model's step 296 -> 280 us, a reply 1,071 -> 1,050).  op is
 // commutative, so the tree is the butterfly's and its results are __shfl_xor's to the bit.
+// (8-byte values: both halves.)
+typedef int i32x2 __attribute__((ext_vector_type(2)));
 template <int CTRL, typename T>
 __device__ __forceinline__ T lane_move(T v) {
-    return __builtin_bit_cast(T, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xF, 0xF, true));
+    if constexpr (sizeof(T) == 8) {
+        i32x2 h = __builtin_bit_cast(i32x2, v);
+        h.x = lane_move<CTRL>((int)h.x);
+        h.y = lane_move<CTRL>((int)h.y);
+        return __builtin_bit_cast(T, h);
+    } else {
+        return __builtin_bit_cast(T, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xF, 0xF, true));
+    }
 }
 constexpr int kDppXor1 = 0xB1, kDppXor2 = 0x4E, kDppHalfMirror = 0x141, kDppRor4 = 0x124, kDppRor8 = 0x128;
 // with lane ^ 16, with lane ^ 32: the swapped pair is (the lower row's, the upper row's) in both rows
 template <typename T, typename Op>
 __device__ __forceinline__ T join_xor16(T v, Op op) {
-    const unsigned u = __builtin_bit_cast(unsigned, v);
-    const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
-    return op(__builtin_bit_cast(T, (unsigned)r[0]), __builtin_bit_cast(T, (unsigned)r[1]));
+    if constexpr (sizeof(T) == 8) {
+        const i32x2 u = __builtin_bit_cast(i32x2, v);
+        const auto x = __builtin_amdgcn_permlane16_swap((unsigned)u.x, (unsigned)u.x, false, false);
+        const auto y = __builtin_amdgcn_permlane16_swap((unsigned)u.y, (unsigned)u.y, false, false);
+        return op(__builtin_bit_cast(T, i32x2{(int)x[0], (int)y[0]}), __builtin_bit_cast(T, i32x2{(int)x[1], (int)y[1]}));
+    } else {
+        const unsigned u = __builtin_bit_cast(unsigned, v);
+        const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+        return op(__builtin_bit_cast(T, (unsigned)r[0]), __builtin_bit_cast(T, (unsigned)r[1]));
+    }
 }
 template <typename T, typename Op>
 __device__ __forceinline__ T join_xor32(T v, Op op) {
-    const unsigned u = __builtin_bit_cast(unsigned, v);
-    const auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
-    return op(__builtin_bit_cast(T, (unsigned)r[0]), __builtin_bit_cast(T, (unsigned)r[1]));
+    if constexpr (sizeof(T) == 8) {
+        const i32x2 u = __builtin_bit_cast(i32x2, v);
+        const auto x = __builtin_amdgcn_permlane32_swap((unsigned)u.x, (unsigned)u.x, false, false);
+        const auto y = __builtin_amdgcn_permlane32_swap((unsigned)u.y, (unsigned)u.y, false, false);
+        return op(__builtin_bit_cast(T, i32x2{(int)x[0], (int)y[0]}), __builtin_bit_cast(T, i32x2{(int)x[1], (int)y[1]}));
+    } else {
+        const unsigned u = __builtin_bit_cast(unsigned, v);
+        const auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+        return op(__builtin_bit_cast(T, (unsigned)r[0]), __builtin_bit_cast(T, (unsigned)r[1]));
+    }
 }
 // all 64 lanes, from lane ^ 32 down to lane ^ 1 (behind ^ 8 a row's halves are alike: a turn by 4 is ^ 4)
 template <typename T, typename Op>
@@ -95,13 +118,23 @@ __device__ __forceinline__ T lanes_join_n(T v, int n, Op op) {
     return v;
 }
 // inclusive sums over the wave's lanes (lanes that a move finds nothing for add 0)
-__device__ __forceinline__ int wave_scan(int v) {
-    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xF, 0xF, false);  // the lane before, in a row of 16
-    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xF, 0xF, false);
-    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xF, 0xF, false);
-    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xF, 0xF, false);
-    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xA, 0xF, false);  // a row's last lane to the next row: rows 1 and 3
-    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xC, 0xF, false);  // lane 31 to rows 2 and 3
+template <int CTRL, int ROWS, typename T>
+__device__ __forceinline__ T lane_before(T v) {
+    if constexpr (sizeof(T) == 8) {
+        const i32x2 h = __builtin_bit_cast(i32x2, v);
+        return __builtin_bit_cast(T, i32x2{lane_before<CTRL, ROWS>((int)h.x), lane_before<CTRL, ROWS>((int)h.y)});
+    } else {
+        return __builtin_bit_cast(T, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, ROWS, 0xF, false));
+    }
+}
+template <typename T>
+__device__ __forceinline__ T wave_scan(T v) {
+    v += lane_before<0x111, 0xF>(v);  // the lane before, in a row of 16
+    v += lane_before<0x112, 0xF>(v);
+    v += lane_before<0x114, 0xF>(v);
+    v += lane_before<0x118, 0xF>(v);
+    v += lane_before<0x142, 0xA>(v);  // a row's last lane to the next row: rows 1 and 3
+    v += lane_before<0x143, 0xC>(v);  // lane 31 to rows 2 and 3
     return v;
 }
 struct SumOp {

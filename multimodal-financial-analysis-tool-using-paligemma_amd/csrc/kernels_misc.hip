@@ -148,14 +148,8 @@ __global__ void __launch_bounds__(1024) k_image_scan(const int64_t* __restrict__
     for (int base = 0; base < n; base += 1024) {
         const int i = base + threadIdx.x;
         const int f = (i < n && ids[i] == image_token) ? 1 : 0;
-        // inclusive scan within the wave
-        int v = f;
         const int l = threadIdx.x & 63, w = threadIdx.x >> 6;
-#pragma unroll
-        for (int o = 1; o < 64; o <<= 1) {
-            int t = __shfl_up(v, o, 64);
-            if (l >= o) v += t;
-        }
+        const int v = wave_scan(f);
         if (l == 63) warp_tot[w] = v;
         __syncthreads();
         int pre = carry;

@@ -15,7 +15,8 @@
 //
 // Four launches, each a short dependent chain; what bounds a draw is their length and number, not the
 // vocabulary's megabyte.  257,216 logits of a peaked distribution: 42 us as five launches with four digits
-// per select, maxima by LDS atomics (a turn per lane) and a select for the token after the cut-off at every draw, now 20.
+// per select, maxima by LDS atomics (a turn per lane) and a select for the token after the cut-off at every draw, later 21.2, 19.6 since
+// the masses of bins and the places of candidates are scanned by the vector unit's lane moves (common.h) and not through LDS.
 #include <algorithm>
 
 #include "common.h"
@@ -30,12 +31,6 @@ constexpr int kSampleThreads = 1024;
 constexpr double kMassScale = 4611686018427387904.0;  // 2^62
 constexpr double kMassUnit = 1.0 / kMassScale;
 __device__ __forceinline__ unsigned long long mass_q(float v) { return (unsigned long long)((double)v * kMassScale); }
-
-__device__ __forceinline__ double wave_sum_d(double v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-    return v;
-}
 
 struct SelectOut {
     uint32_t key;  // bit pattern of the probability at the crossing position
@@ -62,24 +57,19 @@ struct SampleSmem {
     int ord_at[kRanked];
 };
 
-// suf[t] = mass of bins t .. 255 (mq in fixed point), t < 256: the wave's 64 bins by shuffles, then the higher waves'
-// totals in a fixed order.  Every thread of the block must call it (suf: 260 doubles).
+// suf[t] = mass of bins t .. 255 (mq in fixed point), t < 256: a wave scans its 64 bins from the highest down, then the higher
+// waves' totals in a fixed order.  Every thread of the block must call it (suf: 260 doubles).
 __device__ __forceinline__ void suffix_masses(const unsigned long long* mq, double* suf) {
-    const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+    const int t = threadIdx.x, w = t >> 6, bin = t ^ 63;
     double v = 0.0;
     if (t < 256) {
-        v = (double)mq[t] * kMassUnit;
-#pragma unroll
-        for (int o = 1; o < 64; o <<= 1) {
-            const double x = __shfl_down(v, o, 64);
-            if (lane + o < 64) v += x;
-        }
-        if (lane == 0) suf[256 + w] = v;  // the wave's total
+        v = wave_scan((double)mq[bin] * kMassUnit);
+        if ((t & 63) == 63) suf[256 + w] = v;  // the wave's total
     }
     __syncthreads();
     if (t < 256) {
         for (int q = w + 1; q < 4; ++q) v += suf[256 + q];
-        suf[t] = v;
+        suf[bin] = v;
     }
     __syncthreads();
 }
@@ -137,19 +127,13 @@ __device__ __forceinline__ SelectOut radix_select(const Value& value, int n, int
             hist_add(sm.hcnt[level], sm.hmq[level], (k & pmask) == prefix, (int)((k >> shift) & digit), v);
         }
         __syncthreads();
-        // every wave: mass of bins lane .. 63, then the LARGEST bin whose suffix mass crosses (sums are monotone up to
-        // rounding; taking the largest keeps the answer unique)
-        const unsigned long long own = sm.hmq[level][lane];
-        unsigned long long suf = own;
-#pragma unroll
-        for (int o = 1; o < 64; o <<= 1) {
-            const unsigned long long x = __shfl_down(suf, o, 64);
-            if (lane + o < 64) suf += x;
-        }
-        const unsigned long long m = __ballot(sm.hcnt[level][lane] != 0u && above + (double)suf * kMassUnit > target);
+        // every wave, its lanes from the highest bin down: mass of the bin and those above, then the LARGEST bin whose mass
+        // crosses (sums are monotone up to rounding; taking the largest keeps the answer unique)
+        const unsigned long long own = sm.hmq[level][63 - lane], suf = wave_scan(own);
+        const unsigned long long m = __ballot(sm.hcnt[level][63 - lane] != 0u && above + (double)suf * kMassUnit > target);
         if (!m) return SelectOut{0u, 0.0, 0, false};
-        const int d = 63 - __clzll((long long)m);
-        above += (double)(unsigned long long)__shfl(suf - own, d, 64) * kMassUnit;
+        const int at = __ffsll((long long)m) - 1, d = 63 - at;
+        above += (double)(unsigned long long)__shfl(suf - own, at, 64) * kMassUnit;
         prefix |= (uint32_t)d << shift;
         pmask |= digit << shift;
     }
@@ -174,13 +158,8 @@ __device__ __forceinline__ int nth_equal(const Value& value, int n, int NT, uint
     int c = 0;
 #pragma unroll 1
     for (int i = i0; i < i1; ++i) c += (__float_as_uint(value(i)) == key);
-    // exclusive prefix of the threads' counts: within the wave by shuffles, then wave totals
-    int incl = c;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-        const int v = __shfl_up(incl, o, 64);
-        if (lane >= o) incl += v;
-    }
+    // exclusive prefix of the threads' counts: within the wave, then wave totals
+    const int incl = wave_scan(c);
     __syncthreads();
     if (lane == 63) sm.scan[wave] = incl;
     if (threadIdx.x == 0) sm.found = -1;
@@ -279,7 +258,7 @@ __global__ void __launch_bounds__(kTpThreads) k_tp_stats(const float* __restrict
             if (i0 + tid + k * kTpThreads < i1) sum += (double)expf(z[k] - m);
         for (int i = i0 + tid + kTpHeld; i < i1; i += kTpThreads) sum += (double)expf(xr[i] / temperature - m);
     }
-    sum = wave_sum_d(sum);
+    sum = wave_join(sum, SumOp{});
     if ((tid & 63) == 0) red_d[tid >> 6] = sum;
     __syncthreads();
     if (tid == 0) {
@@ -332,7 +311,7 @@ __global__ void __launch_bounds__(kTpThreads) k_tp_hist(const float* __restrict_
         double S = 0.0;
         for (int q = tid; q < NB; q += kTpThreads)
             if (bm[q] != -INFINITY) S += bs[q] * exp((double)bm[q] - (double)m);
-        S = wave_sum_d(S);  // a fixed reduction tree: the same sum every run
+        S = wave_join(S, SumOp{});  // a fixed reduction tree: the same sum every run
         if ((tid & 63) == 0) red_d[tid >> 6] = S;
         __syncthreads();
         S = 0.0;
@@ -358,17 +337,12 @@ __global__ void __launch_bounds__(kTpThreads) k_tp_hist(const float* __restrict_
     __syncthreads();
     {  // per-block counts of bins tid and higher (compaction offsets: two reads give any range of bins)
         __shared__ unsigned wsum[kTpThreads / 64];
-        const int lane = tid & 63, wave = tid >> 6;
-        unsigned n = hcnt[tid];
-#pragma unroll
-        for (int o = 1; o < 64; o <<= 1) {
-            const unsigned x = __shfl_down(n, o, 64);
-            if (lane + o < 64) n += x;
-        }
-        if (lane == 0) wsum[wave] = n;
+        const int wave = tid >> 6, bin = tid ^ 63;  // (a wave's lanes from its highest bin down)
+        unsigned n = wave_scan(hcnt[bin]);
+        if ((tid & 63) == 63) wsum[wave] = n;
         __syncthreads();
         for (int w = wave + 1; w < kTpThreads / 64; ++w) n += wsum[w];
-        reinterpret_cast<uint16_t*>(base + L.hc)[b * 256 + tid] = (uint16_t)n;
+        reinterpret_cast<uint16_t*>(base + L.hc)[b * 256 + bin] = (uint16_t)n;
     }
     if (hmq[tid])  // the row histogram: integer atomics, so the sums do not depend on arrival order
         atomicAdd(reinterpret_cast<unsigned long long*>(base + L.hm) + b % kShards * 256 + tid, hmq[tid]);
@@ -433,11 +407,8 @@ __global__ void __launch_bounds__(kTpThreads) k_tp_compact(int V, int NB, float 
         all += k;
         if (q < b) before += k;
     }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-        before += __shfl_xor(before, o, 64);
-        all += __shfl_xor(all, o, 64);
-    }
+    before = wave_join(before, SumOp{});
+    all = wave_join(all, SumOp{});
     if (lane == 0) { wtot[wave][0] = before; wtot[wave][1] = all; }
     __syncthreads();
     unsigned off = 0u;
@@ -457,12 +428,7 @@ __global__ void __launch_bounds__(kTpThreads) k_tp_compact(int V, int NB, float 
             if (c0 + tid * PT + k < i1 && d >= c1 && d <= c_hi) mask |= 1u << k;
         }
         const unsigned n = (unsigned)__popc(mask);
-        unsigned incl = n;
-#pragma unroll
-        for (int o = 1; o < 64; o <<= 1) {
-            const unsigned x = __shfl_up(incl, o, 64);
-            if (lane >= o) incl += x;
-        }
+        const unsigned incl = wave_scan(n);
         __syncthreads();
         if (lane == 63) wtot[wave][0] = incl;
         __syncthreads();
