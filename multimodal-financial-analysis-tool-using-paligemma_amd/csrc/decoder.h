@@ -257,8 +257,8 @@ void mingru_scan(hipStream_t s, Act act, const GruArgs& a);
 // activation type, dp / ep = d / e rounded up to 8 with zero pads.
 struct WAttnHeads {
     int H, G, d, e, dp, ep;
-    bool own_kv;
-    bool qk_norm, v_norm;  // heads over their root mean square
+    int own_kv;           // truth values in words: a byte of the arguments is a vector load, and a wait for it
+    int qk_norm, v_norm;  // heads over their root mean square
     float eps;
     const double* turns;   // [rot / 2] turns per position of the pairs (2i, 2i + 1) of q and k
     int rot;               // rotated leading dims, 0: none

@@ -40,54 +40,125 @@ constexpr int unit_rows(int mode) { return mode == GR_GRU ? 3 : 2; }
 // outputs a unit covers (plain modes: two rows; GRU, SwiGLU: one channel)
 constexpr int unit_outs(int mode) { return mode == GR_GRU || mode == GR_SWIGLU ? 1 : 2; }
 
-// The step that follows a projection, for output n of row b (v: its sum over K; GR_GRU: v = z, v1 = u, v2 = g;
-// GR_SWIGLU: v = gate, v1 = up).  Every (n, b) is handled by one thread.
-template <typename T, int MODE>
-__device__ __forceinline__ void step_epilogue(const GemvRtArgs& a, int n, int b, float v, float v1, float v2) {
+// The step that follows a projection.  Its operands are asked for ahead of the sums: read where they are used, in turn and each behind
+// its own wait, they were most of a small projection's time (a step of the 1,024-wide
+// streams model, these and the scan's and attention's below: 280 -> 249 us).
+struct StepIn {  // of output n of row b
+    int slot, pos;
+    float v[8];     // the state, or the streams
+    uint16_t w[5];  // bias, or taps
+};
+// the streams' coefficients (up to 8 streams), a lane each: in[s], out[t] and mix[s S + t]
+struct StepMix {
+    int in, out, mix;
+};
+template <int MODE, bool IN>
+__device__ __forceinline__ StepMix step_mix(const GemvRtArgs& a) {
+    StepMix m{};
+    const int lane = threadIdx.x & 63;
+    if constexpr (IN) m.in = (a.in ? a.in : a.nw)[min(lane, a.S - 1)];
+    if constexpr (MODE == GR_STREAMS) {
+        m.out = (a.mix ? a.wout : a.W)[a.mix ? min(lane, a.S - 1) : 0];
+        m.mix = (a.mix ? a.mix : a.W)[a.mix ? min(lane, a.S * a.S - 1) : 0];
+    }
+    return m;
+}
+__device__ __forceinline__ float of_lane(int bf, int lane) { return __uint_as_float((unsigned)__builtin_amdgcn_readlane(bf, lane) << 16); }
+
+// (the slot and position by lanes, also where all have the same: a scalar load would be waited for with the arguments, before
+// anything else is asked for)
+template <int MODE>
+__device__ __forceinline__ void step_slot(const GemvRtArgs& a, int b, StepIn& e) {
+    if constexpr (MODE == GR_CONV || MODE == GR_GRU) {
+        e.slot = a.slot[b];
+        e.pos = a.pos[b];
+    }
+}
+// n and b past the last ones: the last ones'.  MS: streams at most
+template <int MODE, int MS>
+__device__ __forceinline__ void step_load(const GemvRtArgs& a, int n, int b, StepIn& e) {
+    n = min(n, a.N - 1);
     if constexpr (MODE == GR_ACT) {
-        if (a.bias) v += bf2f(a.bias[n]);
-        stf(reinterpret_cast<T*>(a.out) + (long)b * a.ldo + n, v);
+        e.w[0] = (a.bias ? a.bias : a.W)[n];
+    } else if constexpr (MODE == GR_CONV) {
+        const int c = min(n, a.C - 1), KT = a.taps_k;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) e.w[j] = a.cw[(long)c * KT + min(j, KT - 1)];
+        e.w[4] = a.cb[c];
+    } else if constexpr (MODE == GR_GRU) {
+        e.w[0] = a.bias[n];
+        e.w[1] = a.bias[a.N + n];
+    } else if constexpr (MODE == GR_STREAMS) {
+        const float* p = a.X + (long)min(b, a.B - 1) * a.S * a.D + n;
+#pragma unroll
+        for (int s = 0; s < 2; ++s) e.v[s] = p[(long)min(s, a.S - 1) * a.D];
+        if (a.S > 2)
+#pragma unroll
+            for (int s = 2; s < MS; ++s) e.v[s] = p[(long)min(s, a.S - 1) * a.D];
+    }
+}
+// what is found by the slot
+template <int MODE>
+__device__ __forceinline__ void step_state(const GemvRtArgs& a, int n, StepIn& e) {
+    if constexpr (MODE == GR_CONV) {
+        const int KT = a.taps_k;
+        const float* tp = a.state + (long)e.slot * (KT - 1) * a.C + min(n, a.C - 1);
+#pragma unroll
+        for (int j = 0; j < 3; ++j) e.v[j] = (KT > 1 ? tp : a.state)[(long)max(0, min(j, KT - 2)) * a.C];
+    } else if constexpr (MODE == GR_GRU) {
+        e.v[0] = a.state[(long)e.slot * a.N + min(n, a.N - 1)];
+    }
+}
+// output n of row b, both there (v: its sum over K; GR_GRU: v = z, v1 = u, v2 = g; GR_SWIGLU: v = gate, v1 = up).  Every (n, b) is
+// handled by one thread.
+template <typename T, int MODE, int MS>
+__device__ __forceinline__ void step_store(const GemvRtArgs& a, int n, int b, float v, float v1, float v2, const StepIn& e,
+                                           const StepMix& m) {
+    T* out = reinterpret_cast<T*>(a.out) + (long)b * a.ldo + n;
+    if constexpr (MODE == GR_ACT) {
+        stf(out, a.bias ? v + bf2f(e.w[0]) : v);
     } else if constexpr (MODE == GR_LOGITS || MODE == GR_F32) {
         reinterpret_cast<float*>(a.out)[(long)b * a.ldo + n] = v;
     } else if constexpr (MODE == GR_CONV) {
-        if (n < a.C) {
-            const int KT = a.taps_k;
-            float* tp = a.state + (long)a.slot[b] * (KT - 1) * a.C + n;
-            const bool first = a.pos[b] == 0;
-            const uint16_t* cw = a.cw + (long)n * KT;
-            float y = fmaf(bf2f(cw[KT - 1]), v, bf2f(a.cb[n]));
-            for (int j = 0; j < KT - 1; ++j) {
-                const float o = first ? 0.0f : tp[(long)j * a.C];
-                y = fmaf(bf2f(cw[j]), o, y);
-                if (j > 0) tp[(long)(j - 1) * a.C] = o;
-            }
-            if (KT > 1) tp[(long)(KT - 2) * a.C] = v;
-            stf(reinterpret_cast<T*>(a.out) + (long)b * a.ldo + n, siluf_(y));
-        } else {
+        if (n >= a.C) {
             stf(reinterpret_cast<T*>(a.out2) + (long)b * a.ldo2 + n - a.C, v);
+            return;
         }
+        const int KT = a.taps_k;
+        const uint16_t* cw = a.cw + (long)n * KT;
+        float* tp = a.state + (long)e.slot * (KT - 1) * a.C + n;
+        const uint16_t w0 = e.w[0], w1 = e.w[1], w2 = e.w[2], w3 = e.w[3];  // (a choice among an array's places keeps it in memory)
+        const uint16_t last = KT == 4 ? w3 : KT == 3 ? w2 : KT == 2 ? w1 : w0;
+        float y = fmaf(bf2f(KT > 4 ? cw[KT - 1] : last), v, bf2f(e.w[4]));
+        auto tap = [&](int j, uint16_t w, float was) {
+            const float o = e.pos == 0 ? 0.0f : was;
+            y = fmaf(bf2f(w), o, y);
+            if (j > 0) tp[(long)(j - 1) * a.C] = o;
+        };
+#pragma unroll
+        for (int j = 0; j < 3; ++j)
+            if (j < KT - 1) tap(j, e.w[j], e.v[j]);
+        for (int j = 3; j < KT - 1; ++j) tap(j, cw[j], tp[(long)j * a.C]);
+        if (KT > 1) tp[(long)(KT - 2) * a.C] = v;
+        stf(out, siluf_(y));
     } else if constexpr (MODE == GR_GRU) {
-        const float z = sigmoidf_(v + bf2f(a.bias[n]));
-        float* st = a.state + (long)a.slot[b] * a.N + n;
-        const float S = fmaf(1.0f - z, a.pos[b] > 0 ? *st : 0.0f, z * gru_candidate(v1 + bf2f(a.bias[a.N + n])));
-        *st = S;
-        stf(reinterpret_cast<T*>(a.out) + (long)b * a.ldo + n, S * siluf_(v2));
+        const float z = sigmoidf_(v + bf2f(e.w[0]));
+        const float S = fmaf(1.0f - z, e.pos > 0 ? e.v[0] : 0.0f, z * gru_candidate(v1 + bf2f(e.w[1])));
+        a.state[(long)e.slot * a.N + n] = S;
+        stf(out, S * siluf_(v2));
     } else if constexpr (MODE == GR_SWIGLU) {
-        stf(reinterpret_cast<T*>(a.out) + (long)b * a.ldo + n, siluf_(v) * v1);
+        stf(out, siluf_(v) * v1);
     } else {  // GR_STREAMS: the whole column of streams at once
         float* Xr = a.X + (long)b * a.S * a.D + n;
         if (!a.mix) {
-            *Xr = fmaf(a.mult, v, *Xr);
+            *Xr = fmaf(a.mult, v, e.v[0]);
             return;
         }
-        float x[8];
-#pragma unroll
-        for (int s = 0; s < 8; ++s) x[s] = s < a.S ? Xr[(long)s * a.D] : 0.0f;
         for (int t = 0; t < a.S; ++t) {
-            float y = bf2f(a.wout[t]) * v;
+            float y = of_lane(m.out, t) * v;
 #pragma unroll
-            for (int s = 0; s < 8; ++s)
-                if (s < a.S) y = fmaf(bf2f(a.mix[s * a.S + t]), x[s], y);
+            for (int s = 0; s < MS; ++s)
+                if (s < a.S) y = fmaf(of_lane(m.mix, s * a.S + t), e.v[s], y);
             Xr[(long)t * a.D] = y;
         }
     }
@@ -147,6 +218,11 @@ __global__ void __launch_bounds__(256) k_gemv_rt(GemvRtArgs a) {
         }
     };
     wload(w[0], unit, 0);  // in flight during the prologue
+    // lane (r, b) of the unit's first wave finishes output r of row b
+    const int lr = lane / NB, lb = lane % NB;
+    StepIn e;
+    step_slot<MODE>(a, min(lb, a.B - 1), e);
+    const StepMix mix = step_mix<MODE, false>(a);
     if constexpr (XG) {
         xload(0, 0);
     } else {
@@ -261,6 +337,10 @@ __global__ void __launch_bounds__(256) k_gemv_rt(GemvRtArgs a) {
                 mac(1, k0 + KB);
             }
         }
+        const int n = unit * UO + min(lr, UO - 1);
+        step_load<MODE, 8>(a, n, lb, e);
+        step_state<MODE>(a, n, e);
+        asm volatile("" ::: "memory");
         if (u0 + ustep < nunit) {
             wload(w[0], unit + ustep, 0);
             xload(0, 0);
@@ -293,12 +373,10 @@ __global__ void __launch_bounds__(256) k_gemv_rt(GemvRtArgs a) {
             for (int r = 0; r < RW; ++r)
 #pragma unroll
                 for (int b = 0; b < NB; ++b) {
-                    const int n = unit * 2 + r;
-                    if (n < a.N && acc[r][b] > best[b]) { best[b] = acc[r][b]; bi[b] = n; }
+                    const int o = unit * 2 + r;
+                    if (o < a.N && acc[r][b] > best[b]) { best[b] = acc[r][b]; bi[b] = o; }
                 }
         }
-        // lane (r, b) of the unit's first wave finishes output r of row b
-        const int lr = lane / NB, lb = lane % NB;
         float v = 0.0f, v1 = 0.0f, v2 = 0.0f;
 #pragma unroll
         for (int b = 0; b < NB; ++b) {
@@ -310,8 +388,7 @@ __global__ void __launch_bounds__(256) k_gemv_rt(GemvRtArgs a) {
                     if (lr == r && lb == b) v = acc[r][b];
             }
         }
-        const int n = unit * UO + lr;
-        if (kw == 0 && lr < UO && lb < a.B && n < a.N) step_epilogue<T, MODE>(a, n, lb, v, v1, v2);
+        if (kw == 0 && lr < UO && lb < a.B && n < a.N) step_store<T, MODE, 8>(a, n, lb, v, v1, v2, e, mix);
     }
     if constexpr (MODE == GR_LOGITS) {
         __shared__ float sv[4][NB];
@@ -338,82 +415,12 @@ __global__ void __launch_bounds__(256) k_gemv_rt(GemvRtArgs a) {
 //   - x, or the streams it is made of, is asked for before the first weights: the norm runs while they arrive, a quarter of it
 //     in each wave (every wave for itself: 2 streams of 2,048 read four times, 13.2 us where the other form took 12.8);
 //   - a unit's epilogue operands are asked for before the next unit's weights, which would otherwise have to land first
-//     (loads return in order), and the last unit is peeled off so that no branch hides what is in flight.
+//     (loads return in order), the first unit's behind its weights, and the last unit is peeled off so that no branch hides what
+//     is in flight;
+//   - the streams' few coefficients come before everything else, a lane each (behind the weights, they held up the norm until those
+//     were there).
 // us, the LDS form / this one, 2 streams of 2,048 values: gate|up 27.3 / 21.7, mamba in + convolution 12.8 / 9.3, minGRU
 // 11.2 / 7.9, q|k|v 9.1 / 6.0, output matrix 187 / 158, mamba out 8.4 / 5.8, down 16.6 / 14.4; a step 0.83 / 0.67 ms.
-struct OneIn {  // an epilogue's operands
-    float v[8];
-    uint16_t w[6];
-};
-template <int MODE>
-__device__ __forceinline__ void one_load(const GemvRtArgs& a, int n, int slot, OneIn& e) {
-    n = min(n, a.N - 1);
-    if constexpr (MODE == GR_ACT) {
-        e.w[0] = (a.bias ? a.bias : a.W)[n];
-    } else if constexpr (MODE == GR_CONV) {
-        const int c = min(n, a.C - 1), KT = a.taps_k;
-        const float* tp = a.state + (long)slot * (KT - 1) * a.C + c;
-#pragma unroll
-        for (int j = 0; j < 3; ++j) e.v[j] = (KT > 1 ? tp : a.state)[(long)max(0, min(j, KT - 2)) * a.C];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) e.w[j] = a.cw[(long)c * KT + min(j, KT - 1)];
-        e.w[4] = a.cb[c];
-    } else if constexpr (MODE == GR_GRU) {
-        e.w[0] = a.bias[n];
-        e.w[1] = a.bias[a.N + n];
-        e.v[0] = a.state[(long)slot * a.N + n];
-    } else if constexpr (MODE == GR_STREAMS) {
-#pragma unroll
-        for (int s = 0; s < 4; ++s) e.v[s] = a.X[(long)min(s, a.S - 1) * a.D + n];
-    }
-}
-template <int MODE>
-__device__ __forceinline__ void one_store(const GemvRtArgs& a, int n, float v, float v1, float v2, int slot, bool first, const OneIn& e) {
-    uint16_t* out = reinterpret_cast<uint16_t*>(a.out);
-    if constexpr (MODE == GR_ACT) {
-        out[n] = f2bf(a.bias ? v + bf2f(e.w[0]) : v);
-    } else if constexpr (MODE == GR_LOGITS || MODE == GR_F32) {
-        reinterpret_cast<float*>(a.out)[n] = v;
-    } else if constexpr (MODE == GR_CONV) {
-        if (n >= a.C) {
-            reinterpret_cast<uint16_t*>(a.out2)[n - a.C] = f2bf(v);
-            return;
-        }
-        const int KT = a.taps_k;
-        float* tp = a.state + (long)slot * (KT - 1) * a.C + n;
-        float y = fmaf(bf2f(KT == 4 ? e.w[3] : KT == 3 ? e.w[2] : KT == 2 ? e.w[1] : e.w[0]), v, bf2f(e.w[4]));
-#pragma unroll
-        for (int j = 0; j < 3; ++j)
-            if (j < KT - 1) {
-                const float o = first ? 0.0f : e.v[j];
-                y = fmaf(bf2f(e.w[j]), o, y);
-                if (j > 0) tp[(long)(j - 1) * a.C] = o;
-            }
-        if (KT > 1) tp[(long)(KT - 2) * a.C] = v;
-        out[n] = f2bf(siluf_(y));
-    } else if constexpr (MODE == GR_GRU) {
-        const float z = sigmoidf_(v + bf2f(e.w[0]));
-        const float S = fmaf(1.0f - z, first ? 0.0f : e.v[0], z * gru_candidate(v1 + bf2f(e.w[1])));
-        a.state[(long)slot * a.N + n] = S;
-        out[n] = f2bf(S * siluf_(v2));
-    } else if constexpr (MODE == GR_SWIGLU) {
-        out[n] = f2bf(siluf_(v) * v1);
-    } else {  // GR_STREAMS
-        float* Xr = a.X + n;
-        if (!a.mix) {
-            *Xr = fmaf(a.mult, v, e.v[0]);
-            return;
-        }
-        for (int t = 0; t < a.S; ++t) {
-            float y = bf2f(a.wout[t]) * v;
-#pragma unroll
-            for (int s = 0; s < 4; ++s)
-                if (s < a.S) y = fmaf(bf2f(a.mix[s * a.S + t]), e.v[s], y);
-            Xr[(long)t * a.D] = y;
-        }
-    }
-}
-
 constexpr int one_rows(int mode) { return mode == GR_LOGITS ? 4 : unit_rows(mode); }
 constexpr int one_outs(int mode) { return mode == GR_LOGITS ? 4 : unit_outs(mode); }
 
@@ -433,6 +440,9 @@ __global__ void __launch_bounds__(256) k_gemv_one(GemvRtArgs a) {
     // the streams' read and norm are shared out: a wave takes one piece of 512 (of fewer pieces the last one twice)
     const int piece = min(wave, CH - 1), px = piece * 512 + lane * 8;
     static_assert(CH <= 4, "a piece per wave");
+    StepIn e;
+    step_slot<MODE>(a, min(lane, a.B - 1), e);
+    const StepMix mix = step_mix<MODE, (NS > 0)>(a);
     if constexpr (NS == 0) {
 #pragma unroll
         for (int c = 0; c < CH; ++c) x[c] = ldg16(reinterpret_cast<const uint16_t*>(a.x) + c * 512 + lane * 8);
@@ -463,11 +473,14 @@ __global__ void __launch_bounds__(256) k_gemv_one(GemvRtArgs a) {
             for (int c = 0; c < CH; ++c) w[r][c] = ldg_nt(p + c * 512);
         }
     };
+    auto output = [&](int u) { return u * UO + (UO > 1 ? min(lane, UO - 1) : 0); };
+    auto operands = [&](int u) {
+        step_load<MODE, 4>(a, output(u), 0, e);
+        step_state<MODE>(a, output(u), e);
+    };
     wload(unit);
-    asm volatile("" ::: "memory");  // the stream stays ahead of the norm
-    constexpr bool ST = MODE == GR_CONV || MODE == GR_GRU;
-    const int slot = ST ? a.slot[0] : 0;
-    const bool first = ST && a.pos[0] == 0;
+    operands(unit);
+    asm volatile("" ::: "memory");  // the stream, and what its epilogue reads, stay ahead of the norm
     if constexpr (NS < 0) {
         __shared__ __attribute__((aligned(16))) uint16_t xs[CH * 512];
         float m = -1e30f, L = 0.0f, t[8] = {};  // an empty split's values were never written: weight 0, not taken
@@ -501,7 +514,7 @@ __global__ void __launch_bounds__(256) k_gemv_one(GemvRtArgs a) {
         const int P = K / a.groups;
 #pragma unroll
         for (int s = 0; s < NS; ++s) {
-            const float f = a.in ? bf2f(a.in[min(s, a.S - 1)]) : 1.0f;
+            const float f = a.in ? of_lane(mix.in, min(s, a.S - 1)) : 1.0f;
             const float t[8] = {X[s][0].x, X[s][0].y, X[s][0].z, X[s][0].w, X[s][1].x, X[s][1].y, X[s][1].z, X[s][1].w};
 #pragma unroll
             for (int i = 0; i < 8; ++i) u[i] = s < a.S ? fmaf(f, t[i], u[i]) : u[i];
@@ -531,9 +544,8 @@ __global__ void __launch_bounds__(256) k_gemv_one(GemvRtArgs a) {
     float best = -INFINITY;
     int bi = 0x7fffffff;
     auto step = [&](auto more) {
-        OneIn e;
-        const int n = unit * UO + (UO > 1 ? min(lane, UO - 1) : 0);
-        one_load<MODE>(a, n, slot, e);
+        const int n = output(unit);
+        const StepIn now = e;
         float acc[RW];
 #pragma unroll
         for (int r = 0; r < RW; ++r) {
@@ -541,7 +553,11 @@ __global__ void __launch_bounds__(256) k_gemv_one(GemvRtArgs a) {
 #pragma unroll
             for (int c = 0; c < CH; ++c) acc[r] = dot8(w[r][c], x[c], acc[r]);
         }
-        if constexpr (decltype(more)::value) wload(unit + ustep);
+        if constexpr (decltype(more)::value) {
+            operands(unit + ustep);
+            wload(unit + ustep);
+            asm volatile("" ::: "memory");
+        }
 #pragma unroll
         for (int r = 0; r < RW; ++r) acc[r] = wave_sum(acc[r]);
         float v = acc[0];
@@ -554,7 +570,7 @@ __global__ void __launch_bounds__(256) k_gemv_one(GemvRtArgs a) {
             for (int r = 0; r < RW; ++r)
                 if (unit * UO + r < a.N && acc[r] > best) { best = acc[r]; bi = unit * UO + r; }
         }
-        if (lane < UO && n < a.N) one_store<MODE>(a, n, v, acc[RW > 1 ? 1 : 0], acc[RW - 1], slot, first, e);
+        if (lane < UO && n < a.N) step_store<uint16_t, MODE, 4>(a, n, 0, v, acc[RW > 1 ? 1 : 0], acc[RW - 1], now, mix);
         unit += ustep;
     };
     while (unit + ustep < nunit) step(std::true_type{});
@@ -583,6 +599,7 @@ __global__ void __launch_bounds__(256) k_gemv_long(GemvRtArgs a) {
     const int k0 = wave * CH * 512 + lane * 8, N = a.N;
     int n = blockIdx.x, turn = 0;
     uint4 w[CH], x[CH];
+    const StepMix mix = step_mix<MODE, false>(a);
 #pragma unroll
     for (int c = 0; c < CH; ++c) x[c] = ldg16(reinterpret_cast<const uint16_t*>(a.x) + k0 + c * 512);
     auto wload = [&]() {
@@ -591,20 +608,26 @@ __global__ void __launch_bounds__(256) k_gemv_long(GemvRtArgs a) {
         for (int c = 0; c < CH; ++c) w[c] = ldg_nt(p + c * 512);
     };
     wload();
+    StepIn e;
+    step_load<MODE, 4>(a, n, 0, e);
+    asm volatile("" ::: "memory");
     auto step = [&](auto more) {
-        OneIn e;
+        const StepIn now = e;
         const int at = n;
-        one_load<MODE>(a, at, 0, e);
         float acc = 0.0f;
 #pragma unroll
         for (int c = 0; c < CH; ++c) acc = dot8(w[c], x[c], acc);
         n += gridDim.x;
-        if constexpr (decltype(more)::value) wload();
+        if constexpr (decltype(more)::value) {
+            step_load<MODE, 4>(a, n, 0, e);
+            wload();
+            asm volatile("" ::: "memory");
+        }
         acc = wave_sum(acc);
         if (lane == 0) part[turn][wave] = acc;
         __syncthreads();  // (the sums of two turns back are read before the barrier in between)
         if (threadIdx.x == 0)
-            one_store<MODE>(a, at, part[turn][0] + part[turn][1] + part[turn][2] + part[turn][3], 0.0f, 0.0f, 0, false, e);
+            step_store<uint16_t, MODE, 4>(a, at, 0, part[turn][0] + part[turn][1] + part[turn][2] + part[turn][3], 0.0f, 0.0f, now, mix);
         turn ^= 1;
     };
     while (n + (int)gridDim.x < N) step(std::true_type{});
@@ -710,6 +733,11 @@ __global__ void __launch_bounds__(256, sizeof(T) == 4 && MODE != GR_GRU && MODE 
     float v[3] = {0.f, 0.f, 0.f};
     const int b = tid & 15, n = n0 + (tid >> 4);
     const int nstep = (K + 63) / 64, per = (nstep + gridDim.y - 1) / gridDim.y, s_end = min(nstep, (int)(blockIdx.y + 1) * per);
+    StepIn e;
+    step_slot<MODE>(a, min(b, a.B - 1), e);
+    if constexpr (!F32) step_load<MODE, 8>(a, n, b, e);  // (fp32: 128 registers are all in use)
+    const StepMix mix = step_mix<MODE, false>(a);
+    asm volatile("" ::: "memory");
     if constexpr (LU > 0) {
         const int k0 = wave * 64 + (li >> 3) * 32 + lg * 8;  // this lane's 8 of the wave's first step
         const uint16_t* xp = reinterpret_cast<const uint16_t*>(a.x) + (long)min(li & 7, a.B - 1) * a.ldx + k0;
@@ -732,6 +760,7 @@ __global__ void __launch_bounds__(256, sizeof(T) == 4 && MODE != GR_GRU && MODE 
                     for (int h = 0; h < 2; ++h) w[i][m][h] = ldg_nt(wp[m][h] + (s0 + 4 * i) * 64);
                 x[i] = ldg16(xp + (s0 + 4 * i) * 64);
             }
+            __builtin_amdgcn_sched_barrier(0);  // all in flight: left to itself the compiler keeps six
 #pragma unroll
             for (int i = 0; i < LU; ++i)
 #pragma unroll
@@ -740,6 +769,8 @@ __global__ void __launch_bounds__(256, sizeof(T) == 4 && MODE != GR_GRU && MODE 
                     for (int h = 0; h < 2; ++h)
                         acc[m][h] = mfma16(__builtin_bit_cast(short8, w[i][m][h]), __builtin_bit_cast(short8, x[i]), acc[m][h]);
         }
+        step_state<MODE>(a, n, e);
+        asm volatile("" ::: "memory");
         if ((lg >> 1) == (li >> 3))
 #pragma unroll
             for (int m = 0; m < NM; ++m)
@@ -805,6 +836,9 @@ __global__ void __launch_bounds__(256, sizeof(T) == 4 && MODE != GR_GRU && MODE 
                 }
             }
         }
+        if constexpr (F32) step_load<MODE, 8>(a, n, b, e);
+        step_state<MODE>(a, n, e);
+        asm volatile("" ::: "memory");
 #pragma unroll
         for (int m = 0; m < NM; ++m)
 #pragma unroll
@@ -857,7 +891,7 @@ __global__ void __launch_bounds__(256, sizeof(T) == 4 && MODE != GR_GRU && MODE 
             reinterpret_cast<float*>(a.out)[((long)blockIdx.y * a.B + b) * a.ldo + n] = v[0];
         return;
     }
-    if (b < a.B && n < a.N) step_epilogue<T, MODE>(a, n, b, v[0], v[1], v[2]);
+    if (b < a.B && n < a.N) step_store<T, MODE, 8>(a, n, b, v[0], v[1], v[2], e, mix);
     step_pads<T, MODE>(a);
 }
 
@@ -932,7 +966,7 @@ __global__ void __launch_bounds__(256) k_skinny_held(GemvRtArgs a) {
         turn ^= 1;
         if (b >= a.B || n >= a.N) return;
         if constexpr (MODE == GR_F32) reinterpret_cast<float*>(a.out)[(long)b * a.ldo + n] = v[0];
-        else step_epilogue<uint16_t, MODE>(a, n, b, v[0], v[1], 0.f);
+        else step_store<uint16_t, MODE, 8>(a, n, b, v[0], v[1], 0.f, StepIn{}, StepMix{});
     };
     while (grp + (int)gridDim.x < ngroup) step(std::true_type{});
     step(std::false_type{});
@@ -1000,7 +1034,7 @@ __global__ void __launch_bounds__(256) k_skinny_lines(GemvRtArgs a) {
         turn ^= 1;
         if (b >= a.B || n >= a.N) return;
         if constexpr (MODE == GR_F32) reinterpret_cast<float*>(a.out)[(long)b * a.ldo + n] = v[0];
-        else step_epilogue<uint16_t, MODE>(a, n, b, v[0], v[1], 0.f);
+        else step_store<uint16_t, MODE, 8>(a, n, b, v[0], v[1], 0.f, StepIn{}, StepMix{});
     };
     while (grp + (int)gridDim.x < ngroup) step(std::true_type{});
     step(std::false_type{});
@@ -1106,57 +1140,96 @@ __global__ void __launch_bounds__(256) k_conv_step(const T* __restrict__ xz, int
 }
 
 // ---------------------------------------------------------------- selective-scan step
-// LPC lanes per channel: they share the dt dot product over R and hold the channel's states
+// LPC lanes per channel: they share the dt dot product over R and hold the channel's states.  What bounds it is latency: everything
+// that does not hang on the projection's sums (the first AHEAD pieces of a channel's row of Wdt, the first AHEAD states of a lane
+// and their A) is asked for together, ahead of them; read where it is used it was eight trips to memory, one behind the other (2,048
+// channels of 16 states: 4.1 -> 3.2 us)
 template <typename T, int LPC>
 __global__ void __launch_bounds__(256) k_scan_step(ScanStepArgs a) {
-    extern __shared__ float sm[];  // [R + 2N] of this sequence
-    constexpr int CPB = 256 / LPC;
+    extern __shared__ __attribute__((aligned(16))) float sm[];  // [R + 2N] of this sequence, read to whole 8 of R
+    constexpr int CPB = 256 / LPC, AHEAD = 2, SLABS = 4;
     const int b = blockIdx.y, tid = threadIdx.x, sub = tid % LPC;
     const int M = a.R + 2 * a.N;
-    for (int i = tid; i < M; i += 256) {
-        float v = 0.0f;
-        for (int z = 0; z < a.split; ++z) v += a.slabs[((long)z * a.B + b) * M + i];
-        sm[i] = v;
-    }
-    __syncthreads();
     const int c = blockIdx.x * CPB + tid / LPC;
     const bool ok = c < a.C;
     const int cc = ok ? c : a.C - 1;
-    float dt = 0.0f;
-    const uint16_t* wd = a.Wdt + (long)cc * a.ldwdt;
-    for (int r = sub * 8; r < a.R; r += LPC * 8) {  // rows of Wdt are 16-byte aligned, zero past R
-        float w[8];
-        ld8(wd + r, w);
+    int row = b;
+    asm volatile("" : "+v"(row));  // (by vector loads: scalar ones would be waited for with the arguments)
+    const int slot = a.slot[row], pos = a.pos[row];
+    const uint16_t* wd = a.Wdt + (long)cc * a.ldwdt;  // rows of Wdt are 16-byte aligned, zero past R
+    const uint16_t* Al = a.A_log + (long)cc * a.N;
+    float part[SLABS];  // the sums' first slabs
+    const float* slab = a.slabs + (long)b * M + min(tid, M - 1);
 #pragma unroll
-        for (int v = 0; v < 8; ++v)
-            if (r + v < a.R) dt = fmaf(w[v], sm[r + v], dt);
+    for (int z = 0; z < SLABS; ++z) part[z] = slab[(long)min(z, a.split - 1) * a.B * M];
+    uint4 wq[AHEAD];
+    uint16_t aq[AHEAD];
+    float sq[AHEAD];
+#pragma unroll
+    for (int q = 0; q < AHEAD; ++q) {
+        const int r = (q * LPC + sub) * 8;
+        wq[q] = ldg16(wd + (r < a.R ? r : 0));
+        aq[q] = Al[min(q * LPC + sub, a.N - 1)];
     }
-    dt = lanes_join<LPC>(dt, SumOp{});
-    dt = softplusf_(dt + bf2f(a.dtb[cc]));
+    const uint16_t dtb = a.dtb[cc], Dw = a.Dw[cc];
     const float x = ldf(reinterpret_cast<const T*>(a.x) + (long)b * a.ldx + cc);
+    const float gate = ldf(reinterpret_cast<const T*>(a.z) + (long)b * a.ldz + cc);
+    float* st = a.state + ((long)slot * a.C + cc) * a.N;
+#pragma unroll
+    for (int q = 0; q < AHEAD; ++q) sq[q] = st[min(q * LPC + sub, a.N - 1)];
+    asm volatile("" ::: "memory");
+    for (int i = tid; i < M; i += 256) {
+        float v = 0.0f;
+        if (i == tid) {
+#pragma unroll
+            for (int z = 0; z < SLABS; ++z) v += z < a.split ? part[z] : 0.0f;
+        }
+        for (int z = i == tid ? SLABS : 0; z < a.split; ++z) v += a.slabs[((long)z * a.B + b) * M + i];
+        sm[i] = v;
+    }
+    __syncthreads();
+    float dt = 0.0f;
+    auto dot = [&](const uint4 w, int r) {
+        const uint32_t h[4] = {w.x, w.y, w.z, w.w};
+        const float* p = sm + (r < a.R ? r : 0);
+        const f32x4 lo = *reinterpret_cast<const f32x4*>(p), hi = *reinterpret_cast<const f32x4*>(p + 4);
+#pragma unroll
+        for (int v = 0; v < 8; ++v) {
+            const float f = fmaf(__uint_as_float(v & 1 ? h[v / 2] & 0xFFFF0000u : h[v / 2] << 16), v < 4 ? lo[v % 4] : hi[v % 4], dt);
+            dt = r + v < a.R ? f : dt;
+        }
+    };
+#pragma unroll
+    for (int q = 0; q < AHEAD; ++q) dot(wq[q], (q * LPC + sub) * 8);
+    for (int r = (AHEAD * LPC + sub) * 8; r < a.R; r += LPC * 8) dot(ldg16(wd + r), r);
+    dt = lanes_join<LPC>(dt, SumOp{});
+    dt = softplusf_(dt + bf2f(dtb));
     const float dx = dt * x;
-    const bool first = a.pos[b] == 0;
-    float* st = a.state + ((long)a.slot[b] * a.C + cc) * a.N;
     const float* B = sm + a.R;
     const float* Cv = B + a.N;
     float y = 0.0f;
-    for (int n = sub; n < a.N; n += LPC) {
-        const float A = -expf(bf2f(a.A_log[(long)cc * a.N + n])) * 1.4426950408889634f;
-        const float S = fmaf(__builtin_amdgcn_exp2f(dt * A), first ? 0.0f : st[n], dx * B[n]);
-        if (ok) st[n] = S;
-        y = fmaf(S, Cv[n], y);
+    auto state = [&](int n, uint16_t al, float old, float bn, float cn) {
+        const float A = -expf(bf2f(al)) * 1.4426950408889634f;
+        const float S = fmaf(__builtin_amdgcn_exp2f(dt * A), pos == 0 ? 0.0f : old, dx * bn);
+        if (ok && n < a.N) st[n] = S;
+        y = n < a.N ? fmaf(S, cn, y) : y;
+    };
+#pragma unroll
+    for (int q = 0; q < AHEAD; ++q) {
+        const int n = q * LPC + sub, in = min(n, a.N - 1);
+        state(n, aq[q], sq[q], B[in], Cv[in]);
     }
+    for (int n = AHEAD * LPC + sub; n < a.N; n += LPC) state(n, Al[n], st[n], B[n], Cv[n]);
     y = lanes_join<LPC>(y, SumOp{});
     if (sub == 0 && c < a.ldy) {
-        y = fmaf(bf2f(a.Dw[cc]), x, y);
-        stf(reinterpret_cast<T*>(a.y) + (long)b * a.ldy + c,
-            ok ? y * siluf_(ldf(reinterpret_cast<const T*>(a.z) + (long)b * a.ldz + cc)) : 0.0f);
+        y = fmaf(bf2f(Dw), x, y);
+        stf(reinterpret_cast<T*>(a.y) + (long)b * a.ldy + c, ok ? y * siluf_(gate) : 0.0f);
     }
 }
 
 template <typename T>
 void scan_step_t(hipStream_t s, const ScanStepArgs& a) {
-    const size_t lds = (size_t)(a.R + 2 * a.N) * sizeof(float);
+    const size_t lds = (size_t)((a.R + 7) / 8 * 8 + 2 * a.N) * sizeof(float);
     const int cols = std::max(a.C, a.ldy);
     if (a.N <= 16) hipLaunchKernelGGL((k_scan_step<T, 8>), dim3((cols + 31) / 32, a.B), dim3(256), lds, s, a);
     else hipLaunchKernelGGL((k_scan_step<T, 16>), dim3((cols + 15) / 16, a.B), dim3(256), lds, s, a);

@@ -843,7 +843,7 @@ __global__ void __launch_bounds__(256, DQ <= 64 && DV <= 64 && HEADS != ODD ? 4 
     constexpr int VS = DV + 8;
     __shared__ __attribute__((aligned(16))) uint16_t Vs[4][32 * VS];
     __shared__ float sml[4][16][2];
-    __shared__ float2 turned[DQ / 2];  // cos and sin of the rotated pairs
+    __shared__ __attribute__((aligned(16))) float2 turned[DQ / 2];  // cos and sin of the rotated pairs
     const int R = w.H / w.G, hb = blockIdx.y / w.G, g = blockIdx.y % w.G, b = blockIdx.z, sp = blockIdx.x;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), li = lane & 15, lg = lane >> 4;
     const int slot = a.slot[b], i = a.pos[b];
@@ -867,7 +867,12 @@ __global__ void __launch_bounds__(256, DQ <= 64 && DV <= 64 && HEADS != ODD ? 4 
     const bool own = w.own_kv && k1 == keys.n;
     const int kend = own ? k1 - 1 : k1;
     const int h = g * R + r0 + (li < nr ? li : 0);
-    // first tile's loads, then the query's: all in flight together
+    // the scores' and angles' few operands (each asked for where it was used, a trip to memory behind all others: 8 heads
+    // at 1,000 keys 8.3 us, so 6.4), the first
+    // tile's loads, then the query's: all in flight together
+    const Score<SC> score(a.sc, h);
+    const double turn = w.rot > 0 ? w.turns[min(tid, w.rot / 2 - 1)] : 0.0;
+    asm volatile("" ::: "memory");
     uint4 vr[DV / 16], kr[2][DQ / 32];
     auto gload = [&](int j0) {
         const int jm = max(kend - 1, 0);
@@ -923,7 +928,7 @@ __global__ void __launch_bounds__(256, DQ <= 64 && DV <= 64 && HEADS != ODD ? 4 
     // own check, and the new key and value asked for only then: 8 sequences of 16 heads 13.3 us, now 9.8)
     if (tid < w.rot / 2) {
         float s, c;
-        angle(w.turns[tid], i, s, c);
+        angle(turn, i, s, c);
         turned[tid] = make_float2(c, s);
     }
     if (w.rot > 0) __syncthreads();
@@ -939,27 +944,33 @@ __global__ void __launch_bounds__(256, DQ <= 64 && DV <= 64 && HEADS != ODD ? 4 
             ss = rows_sum(ss);
             inv = 1.0f / sqrtf(ss / (float)qd + w.eps);
         }
+        auto put = [&](auto turns) {
+            float2 r[DQ / 32][4];  // (all asked for at once; past the rotated pairs whatever is there, and not taken)
+            if constexpr (decltype(turns)::value)
 #pragma unroll
-        for (int c = 0; c < DQ / 32; ++c) {
-            const bool any = c * 32 < w.rot;
+                for (int c = 0; c < DQ / 32; ++c)
 #pragma unroll
-            for (int v = 0; v < 8; v += 2) {
-                float x = q[c][v] * inv, y = q[c][v + 1] * inv;
-                if (any) {
-                    const int k = c * 32 + 8 * lg + v;
-                    const float2 r = turned[k / 2];
-                    const float u = x * r.x - y * r.y, z = y * r.x + x * r.y;
-                    x = k < w.rot ? u : x;
-                    y = k < w.rot ? z : y;
+                    for (int v = 0; v < 4; ++v) r[c][v] = turned[c * 16 + 4 * lg + v];
+#pragma unroll
+            for (int c = 0; c < DQ / 32; ++c)
+#pragma unroll
+                for (int v = 0; v < 8; v += 2) {
+                    float x = q[c][v] * inv, y = q[c][v + 1] * inv;
+                    if constexpr (decltype(turns)::value) {
+                        const float u = x * r[c][v / 2].x - y * r[c][v / 2].y, z = y * r[c][v / 2].x + x * r[c][v / 2].y;
+                        const bool in = c * 32 + 8 * lg + v < w.rot;
+                        x = in ? u : x;
+                        y = in ? z : y;
+                    }
+                    f[c][v] = (short)f2bf(x);
+                    f[c][v + 1] = (short)f2bf(y);
                 }
-                f[c][v] = (short)f2bf(x);
-                f[c][v + 1] = (short)f2bf(y);
-            }
-        }
+        };
+        if (w.rot > 0) put(std::true_type{});
+        else put(std::false_type{});
     };
     short8 qf[DQ / 32];
     head_row(qr, qf);
-    const Score<SC> score(a.sc, h);
     f32x4 o[DV / 16];
 #pragma unroll
     for (int c = 0; c < DV / 16; ++c) o[c] = f32x4{0.f, 0.f, 0.f, 0.f};
