@@ -1101,14 +1101,25 @@ __global__ void __launch_bounds__(256, DQ <= 64 && DV <= 64 && HEADS != ODD ? 4 
     }
 }
 
-// merge a head's partials: grid (H, B), nsplit <= 64
+// merge a head's partials: grid (H, B), nsplit <= 64.  A thread's values of the first AHEAD splits are asked for ahead of their weights,
+// also an empty split's, which were never written and are not taken (each behind its weight: 9 trips to memory, 8 sequences of 16 heads 5.2 us, now 4.8)
 template <typename T>
 __global__ void __launch_bounds__(256) k_wattn_dc(WAttnDecodeArgs a) {
     __shared__ float wt[64];
-    const int h = blockIdx.x, b = blockIdx.y, rs = a.hd.ep + 2, n = a.nsplit, lane = threadIdx.x & 63;
+    constexpr int AHEAD = 16;
+    const int h = blockIdx.x, b = blockIdx.y, rs = a.hd.ep + 2, n = a.nsplit, lane = threadIdx.x & 63, E = a.hd.e;
     const float* p = a.part + ((long)b * a.hd.H + h) * n * rs;
+    const float* pl = p + (long)min(lane, n - 1) * rs + a.hd.ep;
+    const float ml = pl[0], ll = pl[1];
+    float q[AHEAD];
+    auto load = [&](int c, int s0) {
+#pragma unroll
+        for (int s = 0; s < AHEAD; ++s) q[s] = p[(long)min(s0 + s, n - 1) * rs + min(c, E - 1)];
+    };
+    load(threadIdx.x, 0);
+    asm volatile("" ::: "memory");
     {
-        const float m = lane < n ? p[(long)lane * rs + a.hd.ep] : kNone, l = lane < n ? p[(long)lane * rs + a.hd.ep + 1] : 0.0f;
+        const float m = lane < n ? ml : kNone, l = lane < n ? ll : 0.0f;
         const float M = wave_max(l > 0.0f ? m : kNone);
         const float w = l > 0.0f ? exp2f(m - M) : 0.0f;
         const float L = wave_sum(l * w);
@@ -1116,16 +1127,20 @@ __global__ void __launch_bounds__(256) k_wattn_dc(WAttnDecodeArgs a) {
     }
     __syncthreads();
     T* o = reinterpret_cast<T*>(a.o) + (long)b * a.ldo;
-    for (int c = threadIdx.x; c < a.hd.e; c += 256) {
+    for (int c = threadIdx.x; c < E; c += 256) {
         float t = 0.0f;
-        // an empty split's values were never written: weight 0, not read
-#pragma unroll 8
-        for (int s = 0; s < n; ++s)
-            if (wt[s] > 0.0f) t = fmaf(p[(long)s * rs + c], wt[s], t);
-        stf(o + h * a.hd.e + c, t);
+        for (int s0 = 0; s0 < n; s0 += AHEAD) {
+            if (s0 > 0 || c >= 256) load(c, s0);
+#pragma unroll
+            for (int s = 0; s < AHEAD; ++s) {
+                const float w = s0 + s < n ? wt[s0 + s] : 0.0f;
+                t = w > 0.0f ? fmaf(q[s], w, t) : t;
+            }
+        }
+        stf(o + h * E + c, t);
     }
     if (h == a.hd.H - 1)
-        for (int k = a.hd.H * a.hd.e + threadIdx.x; k < a.ldo; k += 256) stf(o + k, 0.0f);
+        for (int k = a.hd.H * E + threadIdx.x; k < a.ldo; k += 256) stf(o + k, 0.0f);
 }
 
 template <typename T, int RB, int SC>
