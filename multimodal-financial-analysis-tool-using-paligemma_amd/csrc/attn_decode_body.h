@@ -45,13 +45,6 @@ __device__ __forceinline__ void attn_decode_block(const AttnArgs& a, const StepS
     float (*stat)[16] = reinterpret_cast<float (*)[16]>(lds + DVH * DVS * 2 + 16 * (DCH + 4) * 4 + 16 * DPS * 2);
 
     const uint16_t* vb = a.v + b * a.v_b_stride + kvh * a.v_head_stride;
-    uint4 vr[DCH * 32 / 256];
-#pragma unroll
-    for (int i = 0; i < DCH * 32 / 256; ++i) {
-        const int e = tid + 256 * i, r = e >> 5, c = e & 31;
-        // rows past the cache read the last row instead: their e is 0 (finite data times 0)
-        vr[i] = ldg16(vb + (long)(r < nk ? t0 + r : Lk - 1) * a.v_row_stride + 8 * c);
-    }
     const int qi = lane & 15;
     const bool qvalid = qi < a.G;
     const uint16_t* qrow = a.q + b * a.q_b_stride + (kvh * a.G + (qvalid ? qi : 0)) * a.q_head_stride;
@@ -67,6 +60,16 @@ __device__ __forceinline__ void attn_decode_block(const AttnArgs& a, const StepS
 
 #pragma unroll
     for (int kk = 0; kk < 8; ++kk) qf[kk] = frag256(qrow, kk, lane);
+    uint4 vr[DCH * 32 / 256];
+#pragma unroll
+    for (int i = 0; i < DCH * 32 / 256; ++i) {
+        const int e = tid + 256 * i, r = e >> 5, c = e & 31;
+        // rows past the cache read the last row instead: their e is 0 (finite data times 0)
+        vr[i] = ldg16(vb + (long)(r < nk ? t0 + r : Lk - 1) * a.v_row_stride + 8 * c);
+    }
+    // all in flight together, what the scores wait for first (the mask's word sank to its use: a trip to memory of its own)
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
 
     // ---- scores (MFMA): wave w -> keys t0 + 16w + (lane & 15)
     {

@@ -166,17 +166,53 @@ __device__ __forceinline__ void gemv_block(const GemvArgs& a, const int blk, con
     // the weight flight (measured: the streaming modes lose a little by it -- same-box A/B,
     // tools/probes/decode_kernels.py -- and keep the weights-first order)
     constexpr bool XFIRST = MODE == GV_QKV;
+    // Epilogue operands of a group (residual h, RoPE cos / sin) as they lie in memory, queued behind its weights and ahead of all
+    // that waits: read where they are used they were a trip to memory of their own behind the sums (with
+    // the attention's mask, 18 layers: a step 1,052 -> 1,046 us, of two rows 1,173 -> 1,167)
+    int kv_len = 0, pos = 0;
+    if constexpr (MODE == GV_QKV) {
+        int at = 0;
+        asm volatile("" : "+v"(at));  // (vector loads: scalar ones would be waited for with the arguments)
+        kv_len = a.st[at].kv_len;
+        pos = a.st[at].position;
+    }
+    uint16_t pre[RPW][B][2];
+    auto load_pre = [&](int base) {
+        const int at = min(max(pos, 0), a.max_pos - 1);  // (modeling_gemma.py:163-165)
+#pragma unroll
+        for (int i = 0; i < RPW; ++i) {
+            const int u = base + i < bend ? base + i : bend - 1;
+#pragma unroll
+            for (int b = 0; b < B; ++b) {
+                const int bq = b < a.nb ? b : a.nb - 1;
+                if constexpr (MODE == GV_RES || MODE == GV_ORES) {
+                    pre[i][b][0] = ldxh<false>(a.out + (long)bq * a.n_units + u);
+                } else if constexpr (MODE == GV_QKV) {
+                    pre[i][b][0] = a.cosT[(long)at * 128 + (u & 127)];
+                    pre[i][b][1] = a.sinT[(long)at * 128 + (u & 127)];
+                }
+            }
+        }
+    };
     if constexpr (XFIRST) {
         load_x();
         // unconditional (issue clamps the unit): a branch around the stream would make the
         // compiler's in-order vmcnt model drain it before the activation can be used
         issue(S0{}, ub);
         if constexpr (DEPTH == 2) issue(S1{}, ub + stride);
+        __builtin_amdgcn_sched_barrier(0);  // (the position is waited for behind the stream's loads)
+        load_pre(ub);
         asm volatile("" ::: "memory");  // keep the weight stream ahead of the norm (no sinking past it)
     } else {
         issue(S0{}, ub);
         if constexpr (DEPTH == 2) issue(S1{}, ub + stride);
         load_x();
+    }
+    int nch = 0;
+    if constexpr (MODE == GV_ORES) {
+        nch = (a.st->kv_len + 1 + kAttnChunk - 1) / kAttnChunk;
+        load_pre(ub);
+        asm volatile("" ::: "memory");
     }
 
     if constexpr (MODE == GV_ORES) {
@@ -185,7 +221,6 @@ __device__ __forceinline__ void gemv_block(const GemvArgs& a, const int blk, con
         // a fixed order (the flash-decoding combine of k_attn_decode's partials)
         // every thread combines its own 8 outputs from the chunk records directly (stats and
         // partial rows in one round trip, no LDS staging of the weights, no barrier)
-        const int nch = (a.st->kv_len + 1 + kAttnChunk - 1) / kAttnChunk;
         // chunks held in registers (768 keys); longer caches take several passes under a running maximum, each one round trip
         // to memory: 17 chunks, two rows 23.2 us (one trip per record) -> 12.0
         constexpr int CMAX = 12;
@@ -330,13 +365,6 @@ __device__ __forceinline__ void gemv_block(const GemvArgs& a, const int blk, con
         __syncthreads();
     }
 
-    int kv_len = 0, pos = 0;
-    if constexpr (MODE == GV_QKV) {
-        kv_len = a.st->kv_len;
-        pos = a.st->position;
-        if (pos < 0) pos = 0;
-        if (pos > a.max_pos - 1) pos = a.max_pos - 1;  // clamp (modeling_gemma.py:163-165)
-    }
     float best[B];
     int besti[B];
 #pragma unroll
@@ -349,22 +377,17 @@ __device__ __forceinline__ void gemv_block(const GemvArgs& a, const int blk, con
     auto step = [&](auto slot, auto issue_next) {
         constexpr int SL = decltype(slot)::value;
         constexpr bool ISSUE = decltype(issue_next)::value;
-        // epilogue operands of this group (residual h, RoPE cos/sin), queued behind its weights
-        float pre[RPW][B][2];
+        // (o_proj's and q|k|v's groups: the first one's are there, the next one's go out ahead of its weights; down_proj's, whose
+        // stream the loads would wait for, with its sums)
+        if constexpr (MODE == GV_RES) load_pre(ub);
+        uint16_t now[RPW][B][2];
 #pragma unroll
-        for (int i = 0; i < RPW; ++i) {
-            const int u = ub + i < bend ? ub + i : bend - 1;
+        for (int i = 0; i < RPW; ++i)
 #pragma unroll
             for (int b = 0; b < B; ++b) {
-                const int bq = b < a.nb ? b : a.nb - 1;
-                if constexpr (MODE == GV_RES || MODE == GV_ORES) {
-                    pre[i][b][0] = bf2f(ldxh<false>(a.out + (long)bq * a.n_units + u));
-                } else if constexpr (MODE == GV_QKV) {
-                    pre[i][b][0] = bf2f(a.cosT[(long)pos * 128 + (u & 127)]);
-                    pre[i][b][1] = bf2f(a.sinT[(long)pos * 128 + (u & 127)]);
-                }
+                now[i][b][0] = pre[i][b][0];
+                now[i][b][1] = pre[i][b][1];
             }
-        }
         float acc[RPW][NR][B];
 #pragma unroll
         for (int i = 0; i < RPW; ++i)
@@ -390,6 +413,7 @@ __device__ __forceinline__ void gemv_block(const GemvArgs& a, const int blk, con
         bb += stride;
         // the stream of group +DEPTH starts before this group's epilogue, into the freed set
         if constexpr (ISSUE) {
+            if constexpr (MODE == GV_ORES || MODE == GV_QKV) load_pre(ub);
             if constexpr (DEPTH == 1) issue(slot, ub + (DEPTH - 1) * stride);
             else if (ub + (DEPTH - 1) * stride < bend) issue(slot, ub + (DEPTH - 1) * stride);
         }
@@ -435,7 +459,7 @@ __device__ __forceinline__ void gemv_block(const GemvArgs& a, const int blk, con
                 if (b >= a.nb) break;
                 if constexpr (MODE == GV_RES || MODE == GV_ORES) {
                     if (lane == 0) {
-                        stxh<false>(a.out + (long)b * a.n_units + u, f2bf(rbf(acc[i][0][b]) + pre[i][b][0]));
+                        stxh<false>(a.out + (long)b * a.n_units + u, f2bf(rbf(acc[i][0][b]) + bf2f(now[i][b][0])));
                     }
                 } else if constexpr (MODE == GV_GEGLU) {
                     if (lane == 0) {
@@ -452,8 +476,8 @@ __device__ __forceinline__ void gemv_block(const GemvArgs& a, const int blk, con
                         const float x0 = rbf(acc[i][0][b]), x1 = rbf(acc[i][1][b]);
                         const int nh = a.I;
                         if (hh < nh + a.nkv) {
-                            const float c = pre[i][b][0];
-                            const float sn = pre[i][b][1];
+                            const float c = bf2f(now[i][b][0]);
+                            const float sn = bf2f(now[i][b][1]);
                             const uint16_t o0 = f2bf(rbf(x0 * c) + rbf(-x1 * sn));
                             const uint16_t o1 = f2bf(rbf(x1 * c) + rbf(x0 * sn));
                             uint16_t* dst;
