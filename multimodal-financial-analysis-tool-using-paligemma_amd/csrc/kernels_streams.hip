@@ -142,8 +142,12 @@ __global__ void __launch_bounds__(NT) k_streams(StreamsArgs a) {
     for (int d = tid; d < a.ldh; d += NT) stf(h + d, d < D ? u_[d] * inv[d / P] * bf2f(a.w[d]) : 0.0f);
 }
 
+__device__ __forceinline__ float of_lane(int bf, int lane) { return __uint_as_float((unsigned)__builtin_amdgcn_readlane(bf, lane) << 16); }
+
 // The same for widths whose groups are whole numbers of 256 elements (D <= 8192): PC pieces of 4 elements per thread,
-// every load of the row issued before the first is used, one barrier.
+// every load of the row issued before the first is used, one barrier.  The coefficients come a lane each, before all else, and the
+// update's slabs four at a time: one by one where they were used, each was a trip to memory (500 fp32
+// rows of 1,024 6.1 -> 5.5 us, 1,540 rows of 2,048, up to three slabs, 17.3 -> 13.9).
 template <typename T, int SM, int PC>
 __global__ void __launch_bounds__(1024) k_streams_v(StreamsArgs a) {
     __shared__ float red[32];
@@ -151,55 +155,82 @@ __global__ void __launch_bounds__(1024) k_streams_v(StreamsArgs a) {
     const int S = a.S, D = a.D, P = D / a.groups;
     const int row = a.rows_idx ? a.rows_idx[blockIdx.x] : blockIdx.x;
     float* Xr = a.X + (long)row * S * D;
-    float x[PC][SM][4], y[PC][4], u[PC][4];
+    constexpr int YB = 4;  // slabs in flight
+    float x[PC][SM][4], y[PC][4], u[PC][4], q[YB][PC][4];
     ushort4 nw[PC];
+    const uint16_t* any = reinterpret_cast<const uint16_t*>(Xr);  // what is not there: read from here, not used
+    const int cin = (a.in ? a.in : any)[min(lane, S - 1)], cout = (a.mix ? a.out : any)[min(lane, S - 1)];
+    const int cmix = (a.mix ? a.mix : any)[min(lane, S * S - 1)];
     const uint16_t* er = nullptr;
     if (a.ids) {
         long id = a.ids[row];
         id = id < 0 ? 0 : (id >= a.vocab ? a.vocab - 1 : id);
         er = a.E + id * D;
     }
+    const bool update = !er && a.mix;
+    const int ylast = a.mix ? max(a.ysplit - 1, 0) : 0;
+    const float* yr = a.mix && a.ysplit > 0 ? a.y + (long)row * D : Xr;
+    auto yload = [&](int z0) {
 #pragma unroll
-    for (int i = 0; i < PC; ++i) {
-        const int d = (i * NTV + tid) * 4;
-        const bool ok = d < D;
-        const int dd = ok ? d : 0;
-        nw[i] = a.h ? *reinterpret_cast<const ushort4*>(a.w + dd) : make_ushort4(0, 0, 0, 0);
-#pragma unroll
-        for (int v = 0; v < 4; ++v) y[i][v] = 0.0f;
-        if (er) {
-            float e[4];
-            ld4(er + dd, e);
-#pragma unroll
-            for (int s = 0; s < SM; ++s)
-#pragma unroll
-                for (int v = 0; v < 4; ++v) x[i][s][v] = ok && s < S ? e[v] * a.escale : 0.0f;
-        } else {
-#pragma unroll
-            for (int s = 0; s < SM; ++s) {
-                if (s < S) ld4(Xr + (long)s * D + dd, x[i][s]);
-                else x[i][s][0] = x[i][s][1] = x[i][s][2] = x[i][s][3] = 0.0f;
-            }
-        }
-    }
-    if (!er && a.mix) {
-#pragma unroll 4
-        for (int z = 0; z < a.ysplit; ++z) {
+        for (int j = 0; j < YB; ++j)
 #pragma unroll
             for (int i = 0; i < PC; ++i) {
                 const int d = (i * NTV + tid) * 4;
-                float q[4];
-                ld4(a.y + (long)z * a.ystride + (long)row * D + (d < D ? d : 0), q);
-#pragma unroll
-                for (int v = 0; v < 4; ++v) y[i][v] += q[v];
+                ld4(yr + (long)min(z0 + j, ylast) * a.ystride + (d < D ? d : 0), q[j][i]);
             }
+    };
+#pragma unroll
+    for (int i = 0; i < PC; ++i) {
+        const int d = (i * NTV + tid) * 4;
+        nw[i] = *reinterpret_cast<const ushort4*>((a.h ? a.w : any) + (d < D ? d : 0));
+#pragma unroll
+        for (int v = 0; v < 4; ++v) y[i][v] = 0.0f;
+    }
+    if (er) {
+#pragma unroll
+        for (int i = 0; i < PC; ++i) {
+            const int d = (i * NTV + tid) * 4;
+            const bool ok = d < D;
+            float e[4];
+            ld4(er + (ok ? d : 0), e);
+#pragma unroll
+            for (int s = 0; s < SM; ++s)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) x[i][s][v] = ok ? e[v] * a.escale : 0.0f;
+        }
+    } else {  // (no branch among these: what is loaded would be moved, and waited for, where paths meet)
+#pragma unroll
+        for (int i = 0; i < PC; ++i) {
+            const int d = (i * NTV + tid) * 4;
+#pragma unroll
+            for (int s = 0; s < SM; ++s) ld4(Xr + (long)min(s, S - 1) * D + (d < D ? d : 0), x[i][s]);
+        }
+        yload(0);
+        __builtin_amdgcn_sched_barrier(0);
+        asm volatile("" ::: "memory");
+    }
+#pragma unroll
+    for (int i = 0; i < PC; ++i)
+#pragma unroll
+        for (int s = 1; s < SM; ++s)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) x[i][s][v] = s < S ? x[i][s][v] : 0.0f;
+    if (update) {
+        for (int z0 = 0; z0 < a.ysplit; z0 += YB) {
+            if (z0 > 0) yload(z0);
+#pragma unroll
+            for (int j = 0; j < YB; ++j)
+#pragma unroll
+                for (int i = 0; i < PC; ++i)
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) y[i][v] = z0 + j < a.ysplit ? y[i][v] + q[j][i][v] : y[i][v];
         }
         float m[SM][SM], o[SM];
 #pragma unroll
         for (int t = 0; t < SM; ++t) {
-            o[t] = t < S ? bf2f(a.out[t]) : 0.0f;
+            o[t] = t < S ? of_lane(cout, t) : 0.0f;
 #pragma unroll
-            for (int s = 0; s < SM; ++s) m[s][t] = s < S && t < S ? bf2f(a.mix[s * S + t]) : 0.0f;
+            for (int s = 0; s < SM; ++s) m[s][t] = s < S && t < S ? of_lane(cmix, s * S + t) : 0.0f;
         }
 #pragma unroll
         for (int i = 0; i < PC; ++i)
@@ -218,7 +249,7 @@ __global__ void __launch_bounds__(1024) k_streams_v(StreamsArgs a) {
     }
     float c[SM];
 #pragma unroll
-    for (int s = 0; s < SM; ++s) c[s] = s < S ? (a.in ? bf2f(a.in[s]) : 1.0f) : 0.0f;
+    for (int s = 0; s < SM; ++s) c[s] = s < S ? (a.in ? of_lane(cin, s) : 1.0f) : 0.0f;
 #pragma unroll
     for (int i = 0; i < PC; ++i) {
         const int d = (i * NTV + tid) * 4;
