@@ -16,7 +16,8 @@
 // Four launches, each a short dependent chain; what bounds a draw is their length and number, not the
 // vocabulary's megabyte.  257,216 logits of a peaked distribution: 42 us as five launches with four digits
 // per select, maxima by LDS atomics (a turn per lane) and a select for the token after the cut-off at every draw, later 21.2, 19.6 since
-// the masses of bins and the places of candidates are scanned by the vector unit's lane moves (common.h) and not through LDS.
+// the masses of bins and the places of candidates are scanned by the vector unit's lane moves (common.h) and not through LDS, 18.7 with
+// the slices' statistics and the candidates' tokens asked for ahead.
 #include <algorithm>
 
 #include "common.h"
@@ -55,6 +56,7 @@ struct SampleSmem {
     float ord_val[kRanked];
     double ord_mass[kRanked];
     int ord_at[kRanked];
+    int token[kRanked];  // of the first candidates
 };
 
 // suf[t] = mass of bins t .. 255 (mq in fixed point), t < 256: a wave scans its 64 bins from the highest down, then the higher
@@ -68,7 +70,9 @@ __device__ __forceinline__ void suffix_masses(const unsigned long long* mq, doub
     }
     __syncthreads();
     if (t < 256) {
-        for (int q = w + 1; q < 4; ++q) v += suf[256 + q];
+        const double total[4] = {0.0, suf[257], suf[258], suf[259]};  // (read together)
+#pragma unroll
+        for (int q = 1; q < 4; ++q) v = q > w ? v + total[q] : v;
         suf[bin] = v;
     }
     __syncthreads();
@@ -301,15 +305,18 @@ __global__ void __launch_bounds__(kTpThreads) k_tp_hist(const float* __restrict_
     if (temperature > 0.f) {  // softmax(x / T): global max, then the slices' sums of exp rescaled to it
         const float* bm = reinterpret_cast<const float*>(base + L.bm);
         const double* bs = reinterpret_cast<const double*>(base + L.bs);
-        float mq = -INFINITY;
-        for (int q = tid; q < NB; q += kTpThreads) mq = fmaxf(mq, bm[q]);
+        // (a thread's first slice asked for at once: the maximum, again behind the barrier, and the sum behind it were three trips)
+        const float m0 = bm[min(tid, NB - 1)];
+        const double s0 = bs[min(tid, NB - 1)];
+        float mq = tid < NB ? m0 : -INFINITY;
+        for (int q = tid + kTpThreads; q < NB; q += kTpThreads) mq = fmaxf(mq, bm[q]);
         mq = wave_max(mq);
         if ((tid & 63) == 0) red_f[tid >> 6] = mq;
         __syncthreads();
         m = red_f[0];
         for (int w = 1; w < kTpThreads / 64; ++w) m = fmaxf(m, red_f[w]);
-        double S = 0.0;
-        for (int q = tid; q < NB; q += kTpThreads)
+        double S = tid < NB && m0 != -INFINITY ? s0 * exp((double)m0 - (double)m) : 0.0;
+        for (int q = tid + kTpThreads; q < NB; q += kTpThreads)
             if (bm[q] != -INFINITY) S += bs[q] * exp((double)bm[q] - (double)m);
         S = wave_join(S, SumOp{});  // a fixed reduction tree: the same sum every run
         if ((tid & 63) == 0) red_d[tid >> 6] = S;
@@ -462,11 +469,13 @@ __global__ void __launch_bounds__(kSampleThreads) k_tp_select(int V, float top_p
     const double uu = tp_uniform(u[row]);
     // the first candidates, before their number is known (cv has V places)
     const float v0 = cv[min(tid, V - 1)], v1 = cv[min(tid + kSampleThreads, V - 1)];
+    const int token0 = ci[min(tid, V - 1)];
     if (tid < 256) row_mq[tid] = tp_mass(base, L, tid);
     const bool used = tid < 256 && row_mq[tid & 255] != 0ull;
     static_assert(kHeld == 2 * kSampleThreads, "two held candidates per thread");
     sm.val[tid] = v0;
     sm.val[tid + kSampleThreads] = v1;
+    if (tid < kRanked) sm.token[tid] = token0;
     __syncthreads();
     suffix_masses(row_mq, sm.row_suf);
     const int n = M.n_cand, NT = n <= kHeld ? 256 : kSampleThreads;
@@ -553,7 +562,7 @@ __global__ void __launch_bounds__(kSampleThreads) k_tp_select(int V, float top_p
         if (q.crossed) pos = ranked ? q.rank : nth_equal(value, n, NT, q.key, q.rank, sm);
     }
     if (tid == 0) {
-        out[row] = pos >= 0 ? ci[pos] : 0;
+        out[row] = pos < 0 ? 0 : pos < kRanked ? sm.token[pos] : ci[pos];
         if (kept_mass) kept_mass[row] = (float)Z;
     }
 }
