@@ -95,8 +95,7 @@ struct pgmi_ctx {
     // derived
     uint16_t* patch_w = nullptr;  // [v_hidden][kpad]
     int kpad = 0;
-    uint16_t* fc2_w = nullptr;    // [v_layers][v_hidden][ipad], where v_intermediate is no multiple of 64
-    int ipad = 0;                 // v_intermediate rounded up to 64: the row pitch of vH
+    int ipad = 0;  // v_intermediate rounded up to 64: the row pitch of vH
     uint16_t* cosT = nullptr;
     uint16_t* sinT = nullptr;
     // text prefill workspace (rows = max_batch*max_seq)

@@ -160,13 +160,12 @@ int paligemma_prepare(pgmi_ctx* x) {
         if ((rc = dalloc_t(x, &x->vT, RV * c.v_hidden))) return rc;
         if ((rc = dalloc_t(x, &x->vQKV, RV * 3 * c.v_hidden))) return rc;
         if ((rc = dalloc_t(x, &x->vAO, RV * c.v_hidden))) return rc;
-        // fc2's rows are whole 128-byte lines (K = 4304: 8,608 bytes), their last columns zeros on both sides: a k-tile of rows that
-        // straddle lines takes 1.3 to 1.5 times one that does not, and the 8-phase forms need whole k-tiles (a 224 px photo's call
-        // 3,823 -> 3,748 us, a 448 px photo's 8,214 -> 8,087, eight photos' 12,389 -> 12,289)
+        // fc1's output rows start on 128-byte lines (K = 4304: 8,608 bytes otherwise, and a k-tile's piece of a row straddles two; a
+        // 224 px photo's call 3,786 -> 3,741 us, a 448 px photo's 7,977 -> 7,924, eight photos' 12,368 -> 12,253).  fc2's weights
+        // are read where they are, at their own pitch: a copy with rows of 4,352 gave 3,715, 7,888 and 12,253, and a write to
+        // the slab behind prepare did not reach it.
         x->ipad = (c.v_intermediate + 63) / 64 * 64;
         if ((rc = dalloc_t(x, &x->vH, RV * x->ipad))) return rc;
-        HIPCHK(hipMemset(x->vH, 0, RV * x->ipad * 2));  // (columns past v_intermediate stay zero: fc1 writes none of them)
-        if (x->ipad != c.v_intermediate && (rc = dalloc_t(x, &x->fc2_w, (size_t)c.v_layers * c.v_hidden * x->ipad))) return rc;
         if ((rc = dalloc_t(x, &x->vP, RV * x->kpad))) return rc;
         x->ws_bytes = (size_t)64 << 20;
         if ((rc = dalloc(x, reinterpret_cast<void**>(&x->ws), x->ws_bytes))) return rc;
@@ -198,10 +197,6 @@ int paligemma_prepare(pgmi_ctx* x) {
     // derived tensors
     pad_rows(nullptr, W(x, "vision_tower.vision_model.embeddings.patch_embedding.weight"), c.v_hidden,
              c.v_channels * c.v_patch * c.v_patch, x->kpad, x->patch_w);
-    if (x->fc2_w)
-        for (int i = 0; i < c.v_layers; ++i)
-            pad_rows(nullptr, VL(x, i, "mlp.fc2.weight"), c.v_hidden, c.v_intermediate, x->ipad,
-                     x->fc2_w + (size_t)i * c.v_hidden * x->ipad);
     LAUNCHCHK();
     // the batched decode's fragment-major weight images: built by the first decode step with B >= 3 after this
     // call (ensure_mf_image), not here -- a context that never decodes a batch (the drop-in's single-sequence
@@ -286,8 +281,8 @@ static int vision_body(pgmi_ctx* x, hipStream_t s, const void* pixels, int dtype
         gemm(s, x->vT, D, VL(x, i, "mlp.fc1.weight"), D, rows, Iv, D, EPI_BIAS_GELU, f1, x->ws, x->ws_bytes);
         EpiArgs f2{};
         f2.bias = VL(x, i, "mlp.fc2.bias"); f2.res = x->vX; f2.ldr = D; f2.out = x->vX; f2.ldo = D;
-        const int sp = gemm(s, x->vH, Ip, x->fc2_w ? x->fc2_w + (size_t)i * D * Ip : VL(x, i, "mlp.fc2.weight"), Ip, rows, D, Ip,
-                            EPI_BIAS_RES, f2, x->ws, x->ws_bytes, 0, true);
+        const int sp = gemm(s, x->vH, Ip, VL(x, i, "mlp.fc2.weight"), Iv, rows, D, Iv, EPI_BIAS_RES, f2, x->ws,
+                            x->ws_bytes, 0, true);
         splitk_res_norm(s, x->ws, sp, f2.bias, x->vX,
                         last ? W(x, "vision_tower.vision_model.post_layernorm.weight") : VL(x, i + 1, "layer_norm1.weight"),
                         last ? W(x, "vision_tower.vision_model.post_layernorm.bias") : VL(x, i + 1, "layer_norm1.bias"),

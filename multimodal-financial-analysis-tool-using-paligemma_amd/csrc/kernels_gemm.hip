@@ -507,7 +507,7 @@ __global__ void k_splitk_epi(const float* __restrict__ ws, int S, int M, int N, 
 // (counted vmcnt, raw s_barrier).  LDS rows are 128 B with the 16-B chunk index XOR-ed by
 // (row & 7): the swizzle is applied to each lane's SOURCE address (LDS-DMA destinations are
 // lane-linear), and the matching XOR on the ds_read_b128 fragment reads makes them
-// bank-conflict free.  K tails (K % 64) read a zero block.
+// bank-conflict free.  K tails (K % 64, e.g. SigLIP fc2 K = 4304) read a zero block.
 // Waves form a 2 x 2 grid; wave (wm, wn) owns TM x TN (x NB) 16x16 MFMA tiles.
 static __device__ __attribute__((aligned(16))) uint4 g_zero_chunk[1] = {{0u, 0u, 0u, 0u}};
 

@@ -200,6 +200,31 @@ def test_inplace_update_of_unsampled_weight_rebinds(gold):
     del fresh
 
 
+@pytest.mark.parametrize("write", ["op", "data", "slab"])
+@torch.no_grad()
+def test_inplace_update_of_the_towers_fc2_is_seen(gold, write):
+    """The tower reads its fc2 weights where they are: a write to one that the binding's sample does not hold reaches the
+    next call, whether it counts as a version (an op), does not (`p.data`, as merged adapters write) or passes the module
+    by (the engine's view)."""
+    m = _model(W.small_config())
+    px = _inputs(gold)[1]
+    for _ in range(3):  # eager, captured, replayed
+        before = m.vision_tower(px).clone()
+    eng = m.__dict__["_pgmi_bound"].engine
+    sampled = {id(p) for p in m.__dict__["_pgmi_bound"].sample}
+    name, p = next((n, p) for n, p in m.named_parameters() if n.endswith("mlp.fc2.weight") and id(p) not in sampled)
+    assert p.shape[1] % 64, p.shape
+    {"op": p, "data": p.data, "slab": eng.views[name]}[write].mul_(0.5)
+    got = m.vision_tower(px)
+    assert m.__dict__["_pgmi_bound"].engine is eng, "the sample saw it"
+    fresh = _model(W.small_config())
+    fresh.load_state_dict(m.state_dict())
+    fresh.tie_weights()
+    want = fresh.vision_tower(px)
+    assert not torch.equal(want, before), name
+    assert torch.equal(got, want), (name, (got.float() - want.float()).abs().max().item())
+
+
 @torch.no_grad()
 def test_dropped_model_releases_engine_without_gc(gold):
     """A model dropped after lookahead decode steps frees its engine (context, weight slab, workspaces) at

@@ -1,5 +1,5 @@
-"""The vision tower at widths of the feed-forward that are whole k-tiles of 64 (fc2 reads its weights where they are) and that
-are not (fc2 reads rows padded with zeros), several batches, and once more after the weights changed."""
+"""The vision tower at widths of the feed-forward that are whole k-tiles of 64 and that are not (fc1's output rows are further apart
+than they are long), several batches, and once more after the weights changed."""
 import numpy as np
 import pytest
 import torch
@@ -18,7 +18,7 @@ def test_tower_feed_forward_widths(ff):
     eng = Engine(cfg, max_batch=2, max_seq=320, max_kv=320)
     rng = np.random.default_rng(ff)
     px = O.bf16(rng.uniform(-1, 1, (2, 3, 224, 224)).astype(np.float32))
-    for seed in (5, 6):  # the second load must reach fc2's padded rows
+    for seed in (5, 6):  # the second load must reach fc2
         eng.fill_synthetic(seed, W.init_policy)
         eng.prepare()
         want = O.siglip_vision(W.synthetic_state_dict_f32(cfg, seed), cfg, px)
