@@ -137,6 +137,9 @@ __device__ __forceinline__ T wave_scan(T v) {
     v += lane_before<0x143, 0xC>(v);  // lane 31 to rows 2 and 3
     return v;
 }
+// a bf16 that lane `lane` of the wave holds in an int, in every lane.  That lane has to be on: behind a branch it was not in, the register
+// that it is read from may not be the one it was written to
+__device__ __forceinline__ float of_lane(int bf, int lane) { return __uint_as_float((unsigned)__builtin_amdgcn_readlane(bf, lane) << 16); }
 struct SumOp {
     template <typename T>
     __device__ __forceinline__ T operator()(T a, T b) const { return a + b; }

@@ -63,7 +63,6 @@ __device__ __forceinline__ StepMix step_mix(const GemvRtArgs& a) {
     }
     return m;
 }
-__device__ __forceinline__ float of_lane(int bf, int lane) { return __uint_as_float((unsigned)__builtin_amdgcn_readlane(bf, lane) << 16); }
 
 // (the slot and position by lanes, also where all have the same: a scalar load would be waited for with the arguments, before
 // anything else is asked for)
@@ -109,11 +108,28 @@ __device__ __forceinline__ void step_state(const GemvRtArgs& a, int n, StepIn& e
         e.v[0] = a.state[(long)e.slot * a.N + min(n, a.N - 1)];
     }
 }
-// output n of row b, both there (v: its sum over K; GR_GRU: v = z, v1 = u, v2 = g; GR_SWIGLU: v = gate, v1 = up).  Every (n, b) is
-// handled by one thread.
+// output n of row b (v: its sum over K; GR_GRU: v = z, v1 = u, v2 = g; GR_SWIGLU: v = gate, v1 = up), `mine` where both are there and
+// this thread's: every (n, b) is handled by one thread.  Called by whole waves: the streams' coefficients are read from the lanes that
+// hold them, which a branch around the call would have switched off.
 template <typename T, int MODE, int MS>
-__device__ __forceinline__ void step_store(const GemvRtArgs& a, int n, int b, float v, float v1, float v2, const StepIn& e,
+__device__ __forceinline__ void step_store(const GemvRtArgs& a, bool mine, int n, int b, float v, float v1, float v2, const StepIn& e,
                                            const StepMix& m) {
+    if constexpr (MODE == GR_STREAMS) {  // the whole column of streams at once
+        float* Xr = a.X + (long)b * a.S * a.D + n;
+        if (!a.mix) {
+            if (mine) *Xr = fmaf(a.mult, v, e.v[0]);
+            return;
+        }
+        for (int t = 0; t < a.S; ++t) {
+            float y = of_lane(m.out, t) * v;
+#pragma unroll
+            for (int s = 0; s < MS; ++s)
+                if (s < a.S) y = fmaf(of_lane(m.mix, s * a.S + t), e.v[s], y);
+            if (mine) Xr[(long)t * a.D] = y;
+        }
+        return;
+    }
+    if (!mine) return;
     T* out = reinterpret_cast<T*>(a.out) + (long)b * a.ldo + n;
     if constexpr (MODE == GR_ACT) {
         stf(out, a.bias ? v + bf2f(e.w[0]) : v);
@@ -148,19 +164,6 @@ __device__ __forceinline__ void step_store(const GemvRtArgs& a, int n, int b, fl
         stf(out, S * siluf_(v2));
     } else if constexpr (MODE == GR_SWIGLU) {
         stf(out, siluf_(v) * v1);
-    } else {  // GR_STREAMS: the whole column of streams at once
-        float* Xr = a.X + (long)b * a.S * a.D + n;
-        if (!a.mix) {
-            *Xr = fmaf(a.mult, v, e.v[0]);
-            return;
-        }
-        for (int t = 0; t < a.S; ++t) {
-            float y = of_lane(m.out, t) * v;
-#pragma unroll
-            for (int s = 0; s < MS; ++s)
-                if (s < a.S) y = fmaf(of_lane(m.mix, s * a.S + t), e.v[s], y);
-            Xr[(long)t * a.D] = y;
-        }
     }
 }
 
@@ -388,7 +391,7 @@ __global__ void __launch_bounds__(256) k_gemv_rt(GemvRtArgs a) {
                     if (lr == r && lb == b) v = acc[r][b];
             }
         }
-        if (kw == 0 && lr < UO && lb < a.B && n < a.N) step_store<T, MODE, 8>(a, n, lb, v, v1, v2, e, mix);
+        if (kw == 0) step_store<T, MODE, 8>(a, lr < UO && lb < a.B && n < a.N, n, lb, v, v1, v2, e, mix);
     }
     if constexpr (MODE == GR_LOGITS) {
         __shared__ float sv[4][NB];
@@ -570,7 +573,7 @@ __global__ void __launch_bounds__(256) k_gemv_one(GemvRtArgs a) {
             for (int r = 0; r < RW; ++r)
                 if (unit * UO + r < a.N && acc[r] > best) { best = acc[r]; bi = unit * UO + r; }
         }
-        if (lane < UO && n < a.N) step_store<uint16_t, MODE, 4>(a, n, 0, v, acc[RW > 1 ? 1 : 0], acc[RW - 1], now, mix);
+        step_store<uint16_t, MODE, 4>(a, lane < UO && n < a.N, n, 0, v, acc[RW > 1 ? 1 : 0], acc[RW - 1], now, mix);
         unit += ustep;
     };
     while (unit + ustep < nunit) step(std::true_type{});
@@ -626,8 +629,8 @@ __global__ void __launch_bounds__(256) k_gemv_long(GemvRtArgs a) {
         acc = wave_sum(acc);
         if (lane == 0) part[turn][wave] = acc;
         __syncthreads();  // (the sums of two turns back are read before the barrier in between)
-        if (threadIdx.x == 0)
-            step_store<uint16_t, MODE, 4>(a, at, 0, part[turn][0] + part[turn][1] + part[turn][2] + part[turn][3], 0.0f, 0.0f, now, mix);
+        if (wave == 0)
+            step_store<uint16_t, MODE, 4>(a, lane == 0, at, 0, part[turn][0] + part[turn][1] + part[turn][2] + part[turn][3], 0.0f, 0.0f, now, mix);
         turn ^= 1;
     };
     while (n + (int)gridDim.x < N) step(std::true_type{});
@@ -891,7 +894,7 @@ __global__ void __launch_bounds__(256, sizeof(T) == 4 && MODE != GR_GRU && MODE 
             reinterpret_cast<float*>(a.out)[((long)blockIdx.y * a.B + b) * a.ldo + n] = v[0];
         return;
     }
-    if (b < a.B && n < a.N) step_store<T, MODE, 8>(a, n, b, v[0], v[1], v[2], e, mix);
+    step_store<T, MODE, 8>(a, b < a.B && n < a.N, n, b, v[0], v[1], v[2], e, mix);
     step_pads<T, MODE>(a);
 }
 
@@ -966,7 +969,7 @@ __global__ void __launch_bounds__(256) k_skinny_held(GemvRtArgs a) {
         turn ^= 1;
         if (b >= a.B || n >= a.N) return;
         if constexpr (MODE == GR_F32) reinterpret_cast<float*>(a.out)[(long)b * a.ldo + n] = v[0];
-        else step_store<uint16_t, MODE, 8>(a, n, b, v[0], v[1], 0.f, StepIn{}, StepMix{});
+        else step_store<uint16_t, MODE, 8>(a, true, n, b, v[0], v[1], 0.f, StepIn{}, StepMix{});
     };
     while (grp + (int)gridDim.x < ngroup) step(std::true_type{});
     step(std::false_type{});
@@ -1034,7 +1037,7 @@ __global__ void __launch_bounds__(256) k_skinny_lines(GemvRtArgs a) {
         turn ^= 1;
         if (b >= a.B || n >= a.N) return;
         if constexpr (MODE == GR_F32) reinterpret_cast<float*>(a.out)[(long)b * a.ldo + n] = v[0];
-        else step_store<uint16_t, MODE, 8>(a, n, b, v[0], v[1], 0.f, StepIn{}, StepMix{});
+        else step_store<uint16_t, MODE, 8>(a, true, n, b, v[0], v[1], 0.f, StepIn{}, StepMix{});
     };
     while (grp + (int)gridDim.x < ngroup) step(std::true_type{});
     step(std::false_type{});

@@ -142,8 +142,6 @@ __global__ void __launch_bounds__(NT) k_streams(StreamsArgs a) {
     for (int d = tid; d < a.ldh; d += NT) stf(h + d, d < D ? u_[d] * inv[d / P] * bf2f(a.w[d]) : 0.0f);
 }
 
-__device__ __forceinline__ float of_lane(int bf, int lane) { return __uint_as_float((unsigned)__builtin_amdgcn_readlane(bf, lane) << 16); }
-
 // The same for widths whose groups are whole numbers of 256 elements (D <= 8192): PC pieces of 4 elements per thread,
 // every load of the row issued before the first is used, one barrier.  The coefficients come a lane each, before all else, and the
 // update's slabs four at a time: one by one where they were used, each was a trip to memory (500 fp32
