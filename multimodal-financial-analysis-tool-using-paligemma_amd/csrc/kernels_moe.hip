@@ -600,27 +600,32 @@ void experts_skinny(hipStream_t s, ExpertMode mode, const ExpertArgs& args) {
     const int ch = a.K % 512 == 0 && a.ldo == a.N ? a.K / 512 : 0, turn = std::max(1, 8 / (std::max(1, ch) * (mode == EX_SWIGLU ? 2 : 1)));
     const int dots = (ch == 1 || ch == 2 || ch == 4 || ch == 8) && a.N % turn == 0 ? ch : 0;
     a.dotsh = mode == EX_SWIGLU && a.Ksh == a.K && a.ldosh == a.Nsh && a.Nsh % turn == 0;
-#define SKINNY_(mode, u, w, c) hipLaunchKernelGGL((k_experts_skinny<mode, u, w, c>), grid, dim3(256), 0, s, a)
-#define DOTS_(mode, u)                              \
-    switch (dots) {                                 \
-        case 1: SKINNY_(mode, u, true, 1); break;   \
-        case 2: SKINNY_(mode, u, true, 2); break;   \
-        case 4: SKINNY_(mode, u, true, 4); break;   \
-        case 8: SKINNY_(mode, u, true, 8); break;   \
-        default: SKINNY_(mode, u, true, 0); break;  \
-    }
+    auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(256), 0, s, a); };
+    auto go = [&](auto mode_c, auto u_c) {  // whole turns of U steps
+        constexpr int MODE = decltype(mode_c)::value, U = decltype(u_c)::value;
+        auto dot = [&](auto ch_c) {
+            constexpr int CH = decltype(ch_c)::value;
+            if constexpr (2 * CH % U == 0)
+                if (dots == CH) { launch(k_experts_skinny<MODE, U, true, CH>); return true; }
+            return false;
+        };
+        using std::integral_constant;
+        if (!dot(integral_constant<int, 1>{}) && !dot(integral_constant<int, 2>{}) && !dot(integral_constant<int, 4>{}) &&
+            !dot(integral_constant<int, 8>{}))
+            launch(k_experts_skinny<MODE, U, true, 0>);
+    };
+    constexpr std::integral_constant<int, EX_SWIGLU> up;
+    constexpr std::integral_constant<int, EX_STORE> down;
     if (mode == EX_SWIGLU) {
-        if (a.B == 1 && whole(8)) { DOTS_(EX_SWIGLU, 8) }
-        else if (whole(4)) { DOTS_(EX_SWIGLU, 4) }
-        else if (a.B == 1) SKINNY_(EX_SWIGLU, 8, false, 0);
-        else SKINNY_(EX_SWIGLU, 4, false, 0);
+        if (a.B == 1 && whole(8)) go(up, std::integral_constant<int, 8>{});
+        else if (whole(4)) go(up, std::integral_constant<int, 4>{});
+        else if (a.B == 1) launch(k_experts_skinny<EX_SWIGLU, 8, false, 0>);
+        else launch(k_experts_skinny<EX_SWIGLU, 4, false, 0>);
     } else {
-        if (whole(4)) { DOTS_(EX_STORE, 4) }
-        else if (whole(2)) { DOTS_(EX_STORE, 2) }
-        else SKINNY_(EX_STORE, 4, false, 0);
+        if (whole(4)) go(down, std::integral_constant<int, 4>{});
+        else if (whole(2)) go(down, std::integral_constant<int, 2>{});
+        else launch(k_experts_skinny<EX_STORE, 4, false, 0>);
     }
-#undef DOTS_
-#undef SKINNY_
 }
 
 }  // namespace pgmi

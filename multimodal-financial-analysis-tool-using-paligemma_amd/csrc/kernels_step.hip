@@ -2,6 +2,7 @@
 // (up to 16 rows) of any size with the surrounding steps fused (streams' read + grouped norm in front; convolution step, minGRU step, gated
 // activation, streams' update or argmax behind), and the selective-scan step.
 #include <algorithm>
+#include <cassert>
 #include <type_traits>
 
 #include "act.h"
@@ -739,7 +740,6 @@ __global__ void __launch_bounds__(256, sizeof(T) == 4 && MODE != GR_GRU && MODE 
     StepIn e;
     step_slot<MODE>(a, min(b, a.B - 1), e);
     if constexpr (!F32) step_load<MODE, 8>(a, n, b, e);  // (fp32: 128 registers are all in use)
-    const StepMix mix = step_mix<MODE, false>(a);
     asm volatile("" ::: "memory");
     if constexpr (LU > 0) {
         const int k0 = wave * 64 + (li >> 3) * 32 + lg * 8;  // this lane's 8 of the wave's first step
@@ -894,7 +894,7 @@ __global__ void __launch_bounds__(256, sizeof(T) == 4 && MODE != GR_GRU && MODE 
             reinterpret_cast<float*>(a.out)[((long)blockIdx.y * a.B + b) * a.ldo + n] = v[0];
         return;
     }
-    step_store<T, MODE, 8>(a, b < a.B && n < a.N, n, b, v[0], v[1], v[2], e, mix);
+    step_store<T, MODE, 8>(a, b < a.B && n < a.N, n, b, v[0], v[1], v[2], e, StepMix{});
     step_pads<T, MODE>(a);
 }
 
@@ -1101,18 +1101,19 @@ void run_skinny(hipStream_t s, GemvRtMode mode, const GemvRtArgs& a) {
     auto go = [&](auto mode_c, dim3 g) {
         constexpr int MODE = decltype(mode_c)::value;
         if constexpr (std::is_same<T, uint16_t>::value) {
-            if (turn == 8) { hipLaunchKernelGGL((k_skinny<T, MODE, 8>), g, block, 0, s, a); return; }
+            if constexpr (MODE != GR_GRU && MODE != GR_SWIGLU)
+                if (turn == 8) { hipLaunchKernelGGL((k_skinny<T, MODE, 8>), g, block, 0, s, a); return; }
             if (turn == 4) { hipLaunchKernelGGL((k_skinny<T, MODE, 4>), g, block, 0, s, a); return; }
             if (turn == 2) { hipLaunchKernelGGL((k_skinny<T, MODE, 2>), g, block, 0, s, a); return; }
         }
         hipLaunchKernelGGL((k_skinny<T, MODE>), g, block, 0, s, a);
     };
+    assert(mode != GR_STREAMS);  // output projections in this form leave slabs (GR_F32), which the next streams pass joins
     switch (mode) {
         case GR_ACT: go(std::integral_constant<int, GR_ACT>{}, grid); break;
         case GR_CONV: go(std::integral_constant<int, GR_CONV>{}, grid); break;
         case GR_GRU: go(std::integral_constant<int, GR_GRU>{}, grid); break;
         case GR_SWIGLU: go(std::integral_constant<int, GR_SWIGLU>{}, grid); break;
-        case GR_STREAMS: go(std::integral_constant<int, GR_STREAMS>{}, grid); break;
         default: go(std::integral_constant<int, GR_F32>{}, dim3(grid.x, a.split < 1 ? 1 : a.split)); break;
     }
 }
