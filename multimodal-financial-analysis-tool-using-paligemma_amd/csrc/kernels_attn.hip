@@ -1223,11 +1223,14 @@ void attention_prefill(hipStream_t s, int head_dim, const AttnArgs& a) {
     }
     if (v == 9 || v == 91 || v == 92 || v == 94) {  // one pass, keys split over workgroups (auto / 1 / 2 / 4 ranges)
         const int want = v == 9 ? 0 : v - 90;
-        // A workgroup has a CU to itself.  128 rows take 1.55 to 1.7 times the time of 64, so they are taken where the rounds of the
-        // chip are fewer by more than that.  us, 64 / 128 rows: 8 x 288 rows 25.1 / 19.9 (2 rounds, 1), 2 x 1,056 60.5 / 48.8, 6 x 1,056
-        // 118 / 98 (4, 2), 8 x 1,056 148 / 145 (5, 3); 4 x 1,056 89 / 97 (3, 2), 16 x 288 36.7 / 37.8, 8 x 256 19.5 / 28.1 (1, 1)
+        // A workgroup has a CU to itself.  128 rows take 1.4 to 1.5 times the time of 64 in one round of the chip, 1.6 in several and, of
+        // many keys, whose tiles then are all of it, 1.7; they are taken where the rounds are fewer by more than that.  us, 64 / 128
+        // rows: 8 x 288 rows 23.2 / 19.1 (2 rounds, 1), 2 x 1,056 53.1 / 44.2, 6 x 1,056 104.5 / 89.9 (4, 2), 12 x 1,056 182.6 / 178.7
+        // (7, 4); 4 x 1,056 79.1 / 88.2 (3, 2), 16 x 288 33.5 / 35.6, 8 x 256 12.1 / 17.0 (1, 1).  5 rounds and 3 are the close call:
+        // 30 x 288 55.7 / 54.9, 24 x 384 65.6 / 65.0, 18 x 512 and 12 x 768 alike, 10 x 900 118.5 / 121.1, 8 x 1,056 132.1 / 133.8,
+        // 7 x 1,280 155.4 / 157.8
         auto rounds = [&](int rows) { return ((long)(a.Lq * a.G + rows - 1) / rows * a.n_kv * a.B + 255) / 256; };
-        if (head_dim == 256 && 8 * rounds(128) < 5 * rounds(64)) launch_fs<256, 8>(s, a, want);
+        if (head_dim == 256 && (a.Lk > 832 ? 17 : 16) * rounds(128) < 10 * rounds(64)) launch_fs<256, 8>(s, a, want);
         else if (head_dim == 256) launch_fs<256>(s, a, want);
         // few keys whose last 64 would be at most half full: tiles of 32 (us, 32 / 64: 8 x 65 keys 6.8 / 7.6, 96 7.3 / 8.3, 160 11.1 /
         // 12.1, 193 13.7 / 14.0; the same from 257)
