@@ -1133,7 +1133,7 @@ static void launch_fs_t(hipStream_t s, const AttnArgs& a, int ns, int tps, dim3 
 template <int HD, int NWQ = 0, int TKQ = 0>
 static void launch_fs(hipStream_t s, const AttnArgs& a, int want_ns) {
     // head dim 256: 4 compute waves (205 registers: with the loaders 2 waves per SIMD) and a 5-slot ring (160 KiB) of 32-key tiles;
-    // 8 compute waves fit too, 3 waves per SIMD of 168 registers, 2 or 3 of which are spilled (16 bytes of scratch a lane; with
+    // 8 compute waves fit too, 3 waves per SIMD of 168 registers, 2 or 3 of which are spilled (12 or 16 bytes of scratch a lane; with
     // fragments read ahead 16, 2 x 1,056 rows 46 -> 61 us).  Head dim 72: 8
     // compute waves, 4 slots of 64-key tiles, whose barriers and row maxima are half as many as of 32 keys in 8 slots (us, 32 / 64
     // keys: 1,024 rows and keys of 16 heads 22.8 / 21.4, of four images 57.4 / 51.2, 256 of eight 14.5 / 14.1).

@@ -736,7 +736,7 @@ __global__ void k_mf_combine(const float* __restrict__ ws, int KS, int nb, int N
 // The tied output matrix over normalised rows (a.x), up to 8 of them, K = 2048: 8 outputs and two halves of each 64-deep step are the
 // 16 rows of one matrix operand, the rows and the same halves the 16 of the other, so a load instruction reads 8 weight rows by
 // 128 bytes and a line is read once, straight into registers; of the product's quarters the two of like halves are added.
-// Bound by the stream: 257,216 outputs, 8 rows, 176 us through the LDS-DMA ring (k_gemv_ml, 256 bytes of a row at a time), so 163.
+// Bound by the stream: 257,216 outputs, 8 rows, 176 us through the LDS-DMA ring (k_gemv_ml, 256 bytes of a row at a time), so 170.
 __global__ void __launch_bounds__(256) k_logits_lines(GemvArgs a) {
     constexpr int ST = 8;  // 64-deep steps of a wave: the four waves split K
     __shared__ float sums[2][4][16][17];

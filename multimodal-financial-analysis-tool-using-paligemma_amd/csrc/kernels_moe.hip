@@ -345,8 +345,11 @@ void run_experts_f32(hipStream_t s, const ExpertArgs& a) {
 // of 4,096, width 2,048, gate|up 61.6 -> 57.7 us, down 29.5 -> 28.7.  Eight steps in flight for them too: a step of 8 rows 3 % slower.
 // CH > 0 (K of the experts is 512 CH): up to four rows are taken by dot products, each wave whole weight rows as one stream of 1-KiB
 // pieces, as a reply's projections do.  As a matrix instruction's operand 16 rows are read 64 bytes at a time, at 5.3 TB/s, and
-// most of the products are of rows that are not there.  us a step of the 2,048-wide model, of 1, 2, 4, 8 and 16 rows: 742, 905, 1,025, 1,270
-// and 1,495, so 704, 826, 942, 1,150 and 1,354 (up to two rows: 708, 828, 939, 1,157, 1,375; cached weights: 8 rows 1,222).
+// most of the products are of rows that are not there.  us a step of the 2,048-wide model, of 1, 2, 3, 4, 8 and 16 rows of 512 tokens,
+// without and with: 640 / 600, 751 / 711, 819 / 779, 887 / 843, 1,051 / 1,007, 1,404 / 1,343.  (In the tree that it was made in, 8 rows
+// 1,270 and 1,150, up to two rows only 1,157, cached weights 1,222.)  A product's error against 64 bits is the smaller one: K = 2,048
+// 7.4e-8 of its root mean square, by matrix instructions 1.3e-7.  CH 1, 2, 4 and 8 are the widths and feed-forwards of 512 to 4,096
+// that the framework is measured at; other numbers of pieces, a form each, were not and keep the matrix instruction.
 template <int MODE, int CH, int R, bool SHARED>
 __device__ __forceinline__ void experts_dot(const ExpertArgs& a, const uint16_t* W, const int* list) {
     const int N = SHARED ? a.Nsh : a.N, ldw = SHARED ? a.ldwsh : a.ldw;

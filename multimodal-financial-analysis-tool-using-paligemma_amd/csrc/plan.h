@@ -7,7 +7,8 @@
 // 19,281 of its times are in profiles/gemm_plan_sweep.csv.gz.  Over these the constants are off by 8 % (E128) to 24 % (W64x64)
 // of a time on average, and the form chosen, the price of its slabs included, is 2.2 % (layered decoders) to 3.2 % slower than
 // the best of 702 shapes' measured forms, 16 to 22 % over the tenth of the shapes where it does worst: K of 64 and 128, few
-// tiles of long K, and rows that are no multiple of 128 bytes (K = 4304), whose k-tiles take 1.3 to 1.5 b.
+// tiles of long K, and rows that are no multiple of 128 bytes (K = 4304), whose k-tiles take 1.3 to 1.5 b where those of both
+// operands are (the vision tower's activations lie 4,352 apart).
 // What it replaced, plans listed for the shapes of one photo of each size and of eight with one rule for all others:
 // 576 rows, 16384 gate and up columns of K = 2048: 110 us, here 74; 640: 110 / 90; 1280: 190 / 143; 512 rows of q|k|v
 // (3456 columns of K = 1152): 25 / 11; prompts of 2 .. 7 photos 1.21 - 1.33x faster, of one with another text 1.1 - 1.2x.
